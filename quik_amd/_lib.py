@@ -88,6 +88,24 @@ def load():
     return _lib
 
 
+_front = None
+
+
+def front():
+    """The native host front end (csrc/front.cpp); like the library it loads, there is no fallback when it is missing."""
+    global _front
+    if _front is None:
+        load()
+        try:
+            from . import _front as module
+        except ImportError as e:
+            raise RuntimeError(
+                f"{_HERE}/_front.so cannot be loaded ({e}): build it with `make -C quik_amd/csrc` (or "
+                "__graft_entry__.build())") from e
+        _front = module
+    return _front
+
+
 def check(status: int, op: str):
     if status != 0:
         lib = load()

@@ -144,6 +144,9 @@ def quantize(src: torch.Tensor, int_indices: torch.Tensor, fp_indices: torch.Ten
 
     dst: uint8 [M, K/2] (bits=4, low nibble = even element) or int8 [M, K]; meta: [2M]
     interleaved (scale, zero) in src's dtype; fp_x[r, j] = src[r, fp_indices[j]]."""
+    out = L.front().quantize(src, int_indices, fp_indices, bits)
+    if out is not None:
+        return out
     _check_bits(bits)
     L.check_cuda_contiguous("quantize", src=src)
     L.check_cuda_contiguous("quantize", int_indices=int_indices)
@@ -159,6 +162,9 @@ def dequantize(x: torch.Tensor, meta: torch.Tensor, scale_col: torch.Tensor, wRe
     """out = dtype(f32(x) * (s_row * s_col) + ((zero + 2^(bits-1) * s_row) * wReduced + y)).
 
     x int32 [M, N]; meta [2M]; scale_col with size(0) == N; wReduced with size(1) == N; y [M, N]."""
+    out = L.front().dequantize(x, meta, scale_col, wReduced, y, bits)
+    if out is not None:
+        return out
     L.check_cuda_contiguous("dequantize", x=x, meta=meta, scale_col=scale_col, y=y)
     L.check_cuda_contiguous("dequantize", wReduced=wReduced.contiguous())
     _check_bits(bits)
@@ -230,6 +236,10 @@ def _fused_operands(op, A, B, bits):
 
 
 def _fused_dequantize(op, bits, A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y):
+    if zero_row is not None:
+        out = L.front().fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits)
+        if out is not None:
+            return out
     L.check_cuda_contiguous(op, A=A, B=B, scale_row=scale_row, scale_col=scale_col, zero_row=zero_row,
                             w_reduced=w_reduced, y=y)
     M, N, K = _fused_operands(op, A, B, bits)

@@ -27,6 +27,8 @@ from . import _lib as L
 from . import asymmetric, matmul, symmetric
 from ._lib import device_guard
 
+_front = None     # the native front end; set when the first plan is made (only plans lead into it)
+
 __all__ = ["MixedQLinear", "SharedQuantizedInput", "FusedMixedQLinearGroup", "Linear4bit", "Linear8bit", "pack_to_i4",
            "two_compl"]
 
@@ -49,6 +51,9 @@ class _PerObjectCache(dict):
 
     def __deepcopy__(self, memo):
         return _PerObjectCache()
+
+    def __reduce__(self):
+        return _PerObjectCache, ()
 
 
 class SharedQuantizedInput:
@@ -75,17 +80,18 @@ class SharedQuantizedInput:
         self._fused = None      # the concatenated layer (built by the first call), or False: this group cannot be fused
         self._fused_key = None
         self._outs = None       # column views of the group's result, one per member, until the last member was called
+        self._fast = None       # the group's plan for the native front end (csrc/front.cpp), made by a round that ran fused
 
     def __getstate__(self):     # (weak references and device tensors of a forward in flight do not travel)
         state = dict(self.__dict__)
-        state.update(_members=[], _fused=None, _fused_key=None, _outs=None, qint_x=None, fp_x=None, qscale_x=None,
+        state.update(_members=[], _fused=None, _fused_key=None, _outs=None, _fast=None, qint_x=None, fp_x=None, qscale_x=None,
                      meta=None, x6=None, cur_group_elem=0)
         return state
 
     def register(self, module):
         self._members = [r for r in self._members if r() is not None and r() is not module]
         self._members.append(weakref.ref(module))
-        self._fused = None
+        self._fused = self._fast = None
 
     def finish(self):
         self.cur_group_elem += 1
@@ -165,11 +171,29 @@ class SharedQuantizedInput:
                 return None
             mods = [r() for r in self._members]
             self._outs = {id(m): o for m, o in zip(mods, whole.split(self._split, dim=-1))}
+            self._make_fast(mods, fused)
         if self._outs is None or id(member) not in self._outs:
             return None
         out = self._outs[id(member)]
         self.finish()
         return out
+
+    def _make_fast(self, mods, fused):
+        """Hand the round just served by Python to the native front end: later rounds on unchanged members go through
+        `_front.group_forward`, which every member finds under its own "fast" entry."""
+        inner = fused._descs.get("fast")
+        if inner is None or inner[1] is not None or not all(type(m).fuse_shared_groups for m in mods):
+            return
+        names = _BUFFER_NAMES
+        plan = _front.group(weakref.ref(self), fused, inner[0],
+                               tuple((r, id(m), m.out_features, names) for r, m in zip(self._members, mods)))
+        self._fast = plan
+        if plan is not None:
+            for i, m in enumerate(mods):
+                m._descs["fast"] = (plan, i)
+
+
+_BUFFER_NAMES = ("int_weight", "weights_scales", "int_indices", "fp_indices", "reduced_w", "fp_weight", "bias")
 
 
 def _concatenate_layers(layers):
@@ -254,6 +278,18 @@ class MixedQLinear(torch.nn.Module):
         self._descs = _PerObjectCache()
         if shared_input is not None and hasattr(shared_input, "register"):
             shared_input.register(self)
+
+    def __setattr__(self, name, value):
+        # anything set on the module (a switch, a buffer) is read again by the next forward: the native front end's
+        # plans (csrc/front.cpp) go.  (`mid_event` is read by the plan itself.)
+        if name != "mid_event":
+            state = self.__dict__
+            if "_descs" in state:
+                state["_descs"].pop("fast", None)
+                shared = state.get("shared_input")
+                if shared is not None and getattr(shared, "_fast", None) is not None:
+                    shared._fast = None
+        super().__setattr__(name, value)
 
     def _apply(self, fn, recurse=True):
         """`.to()` / `.half()` / `.bfloat16()` convert the floating-point buffers; `dtype` (a plain attribute in the
@@ -431,7 +467,26 @@ class MixedQLinear(torch.nn.Module):
             mid, self.mid_event = self.mid_event.cuda_event, None
         L.check(lib.quik_layer_forward(ctypes.byref(desc), x2.data_ptr(), rows, ws.data_ptr(), nbytes, L.ptr(sk),
                                        sk_bytes, out.data_ptr(), mid, L.stream()), "MixedQLinear.forward")
+        self._make_fast(tiled, x2.device)
         return out
+
+    def _make_fast(self, tiled, device):
+        """A plan for the native front end (csrc/front.cpp) from the descriptors this forward used: later calls on the
+        unchanged module are one crossing into C++, which makes the same checks, allocations and library call."""
+        if L.load() is not L._lib or type(self).mid_event is not None or self.mid_event is not None:
+            return        # (a substituted binding, a class-wide profiling hook: the Python path serves those)
+        row, til = self._descs.get(False), self._descs.get(True)
+        if (til if tiled else row) is None:
+            return        # transient_tiled_copy: the operand is repacked by every call
+        min_rows = self.six_bit_min_rows if self.bits == 4 else self.tile8_min_rows
+        global _front
+        _front = L.front()
+        plan = _front.plan(self, _BUFFER_NAMES, bytes(row[1]) if row is not None else None,
+                              bytes(til[1]) if til is not None else None,
+                              min_rows if self._six_bit_ok(max(min_rows, 1)) else 2 ** 62, device.index,
+                              self.dtype == torch.bfloat16, device, matmul._splitk_workspace, (row, til))
+        if plan is not None:
+            self._descs["fast"] = (plan, None)
 
     def _quantize_input(self, x, shared_input):
         if self.symmetric and x.dtype == torch.float16 and x.data_ptr() % 16 == 0 and self._streams_flag():
@@ -455,12 +510,20 @@ class MixedQLinear(torch.nn.Module):
                 x, self._column_map(), self.int_features_num, self.fp_features_num, self.bits)
 
     def forward(self, x):
+        fast = self._descs.get("fast")
+        if fast is not None:
+            plan, index = fast
+            out = _front.forward(plan, self, x) if index is None else _front.group_forward(plan, index, self, x)
+            if out is not None:
+                return out
         if self.int_features_num <= 0:
             return torch.nn.functional.linear(x, self.fp_weight, self.bias)
         if not x.is_cuda:
             raise RuntimeError("MixedQLinear.forward needs a tensor on the GPU; there is no CPU path")
         lead = x.shape[:-1] if x.dim() == 3 else (1, x.shape[0])
         x2 = x.reshape(-1, x.shape[-1])
+        if x2.shape[1] != self.in_features:
+            raise RuntimeError(f"MixedQLinear.forward: expected {self.in_features} input features but got {x2.shape[1]}")
         if not x2.is_contiguous():
             x2 = x2.contiguous()
         if self.fused and (self.shared_input is None or self.shared_input.group_size == 1):

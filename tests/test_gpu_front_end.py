@@ -1,0 +1,104 @@
+"""The native front end (csrc/front.cpp) behind MixedQLinear.forward and the stand-alone operations.
+
+A repeated forward runs through a plan made by the first one; whatever the plan was made from may change between two
+calls (a buffer written in place or replaced, a switch of the module or of its class, the input's form), and the
+next call has to see it.  Every check compares bits with a module built afresh in the changed state.
+"""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def _module(seed, N, n_in, F, bits, shared=None, bias=False):
+    from quik_amd.qlinear import MixedQLinear
+    rng = np.random.default_rng(seed)
+    fi = torch.from_numpy(np.sort(np.random.default_rng(1).permutation(n_in)[:F]))
+    s_w = torch.from_numpy(rng.uniform(0.001, 0.01, (N, 1)).astype(np.float16))
+    lo, hi = (-8, 8) if bits == 4 else (-127, 128)
+    W = torch.from_numpy((rng.integers(lo, hi, (N, n_in)) * s_w.float().numpy()).astype(np.float16))
+    lin = torch.nn.Linear(n_in, N, bias=bias, dtype=torch.float16)
+    return MixedQLinear.from_float(lin, W, s_w, shared, fi, bits=bits).to(DEV)
+
+
+def _same(a, b):
+    return torch.equal(a.view(torch.int16), b.view(torch.int16))
+
+
+def _planned(mod):
+    return "fast" in mod._descs
+
+
+@pytest.mark.parametrize("rows", [1, 2, 3, 32, 33, 70])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_a_planned_forward_sees_every_change(rows, bits):
+    from quik_amd.qlinear import MixedQLinear
+    N, n_in, F = 264, 1024 + 64, 64
+    mod = _module(0, N, n_in, F, bits, bias=True)
+    x = torch.randn(rows, n_in, generator=torch.Generator().manual_seed(rows)).half().to(DEV)
+    first = mod(x)
+    assert _planned(mod)
+    assert _same(mod(x), first) and mod(x).shape == (1, rows, N)
+    assert mod(x[None]).shape == (1, rows, N)
+    # a form the plan does not take: a view with other strides, another type of tensor
+    wide = torch.zeros(rows, 2 * n_in, dtype=torch.float16, device=DEV)
+    wide[:, :n_in] = x
+    assert _same(mod(wide[:, :n_in]), first)
+    assert _same(mod(torch.nn.Parameter(x, requires_grad=False)), first)
+    with pytest.raises(RuntimeError):
+        mod(x[:, :-1].contiguous())
+    # in place, replaced, and back
+    other = _module(7, N, n_in, F, bits, bias=True)
+    mod.load_state_dict(other.state_dict())
+    want = other(x)
+    assert not _same(want, first)
+    assert _same(mod(x), want) and _same(mod(x), want)
+    mod.bias = None
+    no_bias = _module(7, N, n_in, F, bits)
+    assert _same(mod(x), no_bias(x)) and _same(mod(x), no_bias(x))
+    mod.weights_scales.data = mod.weights_scales.data * 2      # (a new address, no new version of the old tensor)
+    no_bias.weights_scales.mul_(2)
+    assert _same(mod(x), no_bias(x))
+    # switches of the module and of the class
+    mod.six_bit_path = False
+    assert _same(mod(x), no_bias(x)) or rows <= 32
+    keep = MixedQLinear.six_bit_min_rows
+    calls = []
+    real = MixedQLinear._forward_one_call
+    try:
+        MixedQLinear._forward_one_call = lambda self, x2: calls.append(1) or real(self, x2)
+        mod(x)
+        assert calls == [1]
+    finally:
+        MixedQLinear._forward_one_call = real
+    assert MixedQLinear.six_bit_min_rows == keep
+
+
+@pytest.mark.parametrize("rows", [1, 40])
+def test_a_planned_group_sees_every_change(rows):
+    from quik_amd.qlinear import SharedQuantizedInput
+    n_in, F, sizes = 1024 + 64, 64, (256, 64, 64)
+    shared = SharedQuantizedInput(3)
+    mods = [_module(i, n, n_in, F, 4, shared) for i, n in enumerate(sizes)]
+    alone = [_module(i, n, n_in, F, 4) for i, n in enumerate(sizes)]
+    x = torch.randn(rows, n_in, generator=torch.Generator().manual_seed(3)).half().to(DEV)
+    for _ in range(3):
+        for m, a in zip(mods, alone):
+            assert _same(m(x), a(x))
+        assert shared._fast is not None and shared.cur_group_elem == 0 and shared._outs is None
+    for order in ((2, 0, 1), (1, 2, 0)):                     # any call order
+        for i in order:
+            assert _same(mods[i](x[None]), alone[i](x[None]))
+    for m, a in zip(mods, alone):                            # one member's scales change in place
+        m.weights_scales.mul_(2)
+        a.weights_scales.mul_(2)
+    for _ in range(2):
+        for m, a in zip(mods, alone):
+            assert _same(m(x), a(x))
+    outs = [mods[0](x)]                                      # a switch set in the middle of a round
+    mods[1].fuse_shared_groups = True
+    outs += [mods[1](x), mods[2](x)]
+    assert all(_same(o, a(x)) for o, a in zip(outs, alone))
+    assert shared.cur_group_elem == 0
