@@ -64,6 +64,14 @@ int quik_asym_quantize(const void *x, int dtype, int64_t rows, int64_t cols,
                        const void *colmap, int64_t num_int, int64_t num_fp, int bits,
                        void *dst, void *meta, void *fp_x, void *stream);
 
+/* The same operation straight from the two index lists, for callers that hold no column map: a map of the sections
+ * this operation reads is built into colmap_workspace (quik_colmap_bytes(cols, num_int, num_fp) bytes, 256-byte
+ * aligned, free again behind the call on the stream) and used once; it must not be given to another entry point. */
+int quik_asym_quantize_indexed(const void *x, int dtype, int64_t rows, int64_t cols,
+                               const int64_t *int_indices, int64_t num_int,
+                               const int64_t *fp_indices, int64_t num_fp, int bits,
+                               void *colmap_workspace, void *dst, void *meta, void *fp_x, void *stream);
+
 /* quik.asymmetric.find_meta(src, bits) -> meta [2*rows]; fp16 only, all columns.
  * replaces findMaxMinMetaCUDA, src/asymmetric/asymmetric.cu:320-338. */
 int quik_asym_find_meta(const void *x, int64_t rows, int64_t cols, int bits,

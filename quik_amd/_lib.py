@@ -21,6 +21,7 @@ SIGNATURES = {
     "quik_colmap_bytes": (_i64, [_i64, _i64, _i64]),
     "quik_colmap_build": (_int, [_vp, _i64, _vp, _i64, _i64, _vp, _vp]),
     "quik_asym_quantize": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _i64, _int, _vp, _vp, _vp, _vp]),
+    "quik_asym_quantize_indexed": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _vp, _i64, _int, _vp, _vp, _vp, _vp, _vp]),
     "quik_asym_find_meta": (_int, [_vp, _i64, _i64, _int, _vp, _vp]),
     "quik_asym_quantize_old": (_int, [_vp, _vp, _i64, _i64, _int, _vp, _vp]),
     "quik_asym_dequantize": (_int, [_vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _int, _vp, _vp]),

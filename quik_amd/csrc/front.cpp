@@ -387,11 +387,9 @@ PyObject *py_quantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
     const c10::DataPtr cm = c10::hip::HIPCachingAllocator::get()->allocate(static_cast<size_t>(quik_colmap_bytes(cols, num_int, num_fp)));
     at::Tensor dst = bits == 4 ? new_empty({rows, num_int / 2}, at::kByte, dev) : new_empty({rows, num_int}, at::kChar, dev);
     at::Tensor meta = new_empty({2 * rows}, src->scalar_type(), dev), fp_x = new_empty({rows, num_fp}, src->scalar_type(), dev);
-    int rc = quik_colmap_build(static_cast<const int64_t *>(ptr(*ii)), num_int, static_cast<const int64_t *>(ptr(*fi)), num_fp,
-                               cols, cm.get(), st);
-    if (rc == QUIK_OK)
-      rc = quik_asym_quantize(ptr(*src), dt, rows, cols, cm.get(), num_int, num_fp, static_cast<int>(bits), out_ptr(dst),
-                              out_ptr(meta), out_ptr(fp_x), st);
+    const int rc = quik_asym_quantize_indexed(ptr(*src), dt, rows, cols, static_cast<const int64_t *>(ptr(*ii)), num_int,
+                                              static_cast<const int64_t *>(ptr(*fi)), num_fp, static_cast<int>(bits), cm.get(),
+                                              out_ptr(dst), out_ptr(meta), out_ptr(fp_x), st);
     if (rc != QUIK_OK) return fail("quantize", rc);
     return triple(std::move(dst), std::move(meta), std::move(fp_x));
   });
