@@ -1,0 +1,355 @@
+// Fused layer GEMM on tile-ordered operands for problems of few tiles: every wave streams its own share of K straight
+// from memory into the MFMA operand registers.
+//
+// What bounds the ring kernels (gemm_fp6.h, gemm_tile8.h) on few and narrow tiles is the step itself: a 128x64 tile has
+// two MFMAs per wave and k-step, 64 cycles of work between two barriers, an LDS round trip and a wait for copies
+// (measured 250 .. 300 cycles a step; 13824 columns at 128 rows: 16 us for 53 MB of weights).  The operand buffers hold
+// each fragment as one contiguous kilobyte (fp6_format.h), so a wave can load fragments directly, and nothing has to be
+// shared inside the workgroup if the waves split K instead of the tile: each of the four waves computes the WHOLE tile
+// over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of loads in flight.
+// The traffic between a CU and its L2 is that of a ring kernel with the same tile.  Afterwards the waves add their
+// integer sums through LDS (exact, so in any order), each ending up with the blocks it owns, convert them, run the
+// outlier steps on them in the same order as the ring kernels and store: the same output bits.
+//
+// Workgroups may share a tile's K further (SplitK, as in gemm_fp6.h): when the tiles are fewer than the CUs.
+#pragma once
+#include <type_traits>
+
+#include "gemm_tile8.h"
+
+#define QUIK_INLINE __attribute__((always_inline))
+
+namespace quik {
+
+// SIX: 6-bit operands (Fused6Args), else int8 (Fused8Args: the same fields)
+template <bool SIX_, int MI_, int NI_, int SETS_>
+struct DirectCfg {
+  static constexpr bool SIX = SIX_;
+  static constexpr int MI = MI_, NI = NI_, SETS = SETS_, NF = MI + NI;
+  static constexpr int WAVES = 4, kThreads = 64 * WAVES;
+  static constexpr int BM = 32 * MI, BN = 32 * NI;
+  static constexpr int UNIT = SIX ? 3072 : 2048;
+  static constexpr int PHASES = MI * NI > WAVES ? MI * NI / WAVES : 1;  // blocks a wave owns
+  static_assert((MI == 4 && NI == 2) || (MI == 2 && (NI == 2 || NI == 1)), "supported tiles");
+  static constexpr int kOutlierSets = 8;
+  static constexpr int RED_BYTES = WAVES * (WAVES - 1) * 4096;
+  static constexpr int OUT_STRIDE = BN * 2 + 16;
+  static constexpr int VEC_OFF = RED_BYTES > BM * OUT_STRIDE ? RED_BYTES : BM * OUT_STRIDE;
+  static constexpr int SMEM = VEC_OFF + (4 * BN + 3 * BM) * 4;
+  // block (mi, ni) owned by wave w in phase p; waves without one (64x32 tiles have two blocks) own nothing
+  static constexpr int own_mi(int w, int) { return MI == 4 ? w : w & 1; }
+  static constexpr int own_ni(int w, int p) { return MI == 4 ? p : w >> 1; }
+  static constexpr bool owns(int w) { return MI == 4 || (w >> 1) < NI; }
+};
+
+// One step's fragments of a wave.  6-bit: head in dwords 0 .. 3, tail in 4 and 5, as the MFMA takes it.  (Kept as whole
+// operand vectors: with heads and tails in arrays of their own the compiler merges neighbouring elements into one
+// wider access, cannot split the arrays into registers any more and puts them into scratch memory.)
+template <class D>
+struct DirectFrag {
+  std::conditional_t<D::SIX, v8i, v4i> f[D::NF];
+};
+
+template <class D, bool BF16, bool SPLITK, class Args>
+__device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8_t *smem, int split, int tile_id,
+                                            const SplitK *sk) {
+  constexpr int MI = D::MI, NI = D::NI, SETS = D::SETS, NF = D::NF, WAVES = D::WAVES, UNIT = D::UNIT;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int m0 = tm * D::BM, n0 = tn * D::BN;
+  int64_t x_blocks, w_blocks, block_bytes, x_sums = 0, w_sums = 0;
+  int steps, fsteps;
+  if constexpr (D::SIX) {
+    const Fp6Layout lx = fp6_layout(p.M, p.K, p.F), lw = fp6_layout(p.N_total, p.K, p.F);
+    x_blocks = lx.blocks, w_blocks = lw.blocks, block_bytes = lx.block_bytes;
+    x_sums = lx.sums_off, w_sums = lw.sums_off;
+    steps = static_cast<int>(lx.steps), fsteps = static_cast<int>(lx.fsteps);
+  } else {
+    const Tile8Layout lx = tile8_layout(p.M, p.K, p.F), lw = tile8_layout(p.N_total, p.K, p.F);
+    x_blocks = lx.blocks, w_blocks = lw.blocks, block_bytes = lx.block_bytes;
+    steps = static_cast<int>(lx.steps), fsteps = static_cast<int>(lx.fsteps);
+  }
+
+  // sources: one scalar base per 64-row block; a 32-row fragment is half a block (blocks past the matrix: any valid
+  // one, results never stored)
+  const int r = lane & 31, h = lane >> 5;
+  const uint32_t head_off = r * 32 + ((h ^ ((r >> 3) & 1)) << 4), tail_off = 2048 + h * 512 + r * 8;
+  const int wrow = p.n_first + n0, whalf = (wrow >> 5) & 1;  // (whalf: single-fragment tiles may start inside a block)
+  auto block = [&](int64_t b, int64_t blocks) { return (b < blocks ? b : blocks - 1) * block_bytes; };
+  const uint8_t *base[MI / 2 + (NI + 1) / 2];
+#pragma unroll
+  for (int b = 0; b < MI / 2; ++b) base[b] = p.xbuf + block(m0 / 64 + b, x_blocks);
+#pragma unroll
+  for (int b = 0; b < (NI + 1) / 2; ++b) base[MI / 2 + b] = p.wbuf + block(wrow / 64 + b, w_blocks);
+  auto load_step = [&](DirectFrag<D> &f, int64_t step) QUIK_INLINE {
+    // (opaque per step: the lane offsets stay 32-bit offsets to a scalar base, instead of being folded into a 64-bit
+    // vector address per fragment that every step then has to advance)
+    uint32_t ho = head_off, to = tail_off;
+    asm volatile("" : "+v"(ho), "+v"(to));
+    static_for<NF>([&](auto J) QUIK_INLINE {
+      constexpr int j = J, jj = j < MI ? j : j - MI, b = j < MI ? j / 2 : MI / 2 + jj / 2;
+      const int half = j < MI || NI > 1 ? jj & 1 : whalf;
+      const v4i head = *reinterpret_cast<const v4i *>(base[b] + step * UNIT + half * 1024 + ho);
+      if constexpr (D::SIX) {
+        const v2i tail = *reinterpret_cast<const v2i *>(base[b] + step * UNIT + half * 256 + to);
+        f.f[j] = v8i{head.x, head.y, head.z, head.w, tail.x, tail.y, 0, 0};
+      } else {
+        f.f[j] = head;
+      }
+    });
+  };
+
+  int k0 = 0, k1 = steps;
+  if constexpr (SPLITK) {
+    k0 = split * sk->per;
+    k1 = k0 + sk->per < steps ? k0 + sk->per : steps;
+  }
+  // this wave's steps: k0 + wave, k0 + wave + WAVES, ...
+  const int mine = k1 - k0 > wave ? (k1 - k0 - wave + WAVES - 1) / WAVES : 0;
+  auto at = [&](int i) { return static_cast<int64_t>(k0 + wave + i * WAVES); };
+  // per-row and per-column scalars of this thread: requested first, unconditionally (a load under a branch would make
+  // the waits of everything around it waits for all loads), used after the main loop
+  const int vi = threadIdx.x;
+  const int64_t vn = n0 + vi % D::BN < p.N ? n0 + vi % D::BN : p.N - 1, vm = m0 + vi % D::BM < p.M ? m0 + vi % D::BM : p.M - 1;
+  const bool asym = p.w_red != nullptr;  // asymmetric: meta holds (scale, zero) pairs; symmetric: one scale per row, no zero term
+  const uint16_t v_sc = p.s_col[vn], v_wr = (asym ? p.w_red : p.s_col)[vn], v_bs = (p.bias ? p.bias : p.s_col)[vn];
+  const uint16_t v_sr = p.meta[asym ? 2 * vm : vm], v_zr = p.meta[asym ? 2 * vm + 1 : vm];
+  int v_cs = 0, v_rs = 0;
+  if constexpr (D::SIX) {
+    v_cs = reinterpret_cast<const int32_t *>(p.wbuf + w_sums)[p.n_first + vn];
+    v_rs = reinterpret_cast<const int32_t *>(p.xbuf + x_sums)[vm];
+  }
+
+  DirectFrag<D> set[SETS];
+  const int last_step = k1 > 0 ? k1 - 1 : 0;
+  static_for<SETS>([&](auto S) QUIK_INLINE { load_step(set[S], at(S) < last_step ? at(S) : last_step); });
+
+  v16f acc[MI][NI];  // fp32 sums (SIX) or int32 bit patterns
+#pragma unroll
+  for (int mi = 0; mi < MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < NI; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0.0f;
+  auto multiply = [&](const DirectFrag<D> &f) QUIK_INLINE {
+    static_for<MI * NI>([&](auto I) QUIK_INLINE {
+      constexpr int mi = I % MI, ni = I / MI;
+      if constexpr (D::SIX) {
+        acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.f[MI + ni], f.f[mi], acc[mi][ni], 2, 2, 0, 0, 0, 0);
+      } else {
+        FragOps<kInt8>::mma(f.f[mi], f.f[MI + ni], acc[mi][ni]);
+      }
+    });
+  };
+  {
+    int it = 0;
+    for (; it + 2 * SETS <= mine; it += SETS) {
+      static_for<SETS>([&](auto S) QUIK_INLINE {
+        multiply(set[S]);
+        load_step(set[S], at(it + SETS + S));
+        __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
+      });
+    }
+    static_for<SETS>([&](auto S) QUIK_INLINE {
+      if (it + S < mine) multiply(set[S]);
+      if (it + SETS + S < mine) load_step(set[S], at(it + SETS + S));
+    });
+    static_for<SETS>([&](auto S) QUIK_INLINE {
+      if (it + SETS + S < mine) multiply(set[S]);
+    });
+  }
+
+  float *const scol = reinterpret_cast<float *>(smem + D::VEC_OFF), *const wred = scol + D::BN, *const bias = wred + D::BN,
+               *const colc = bias + D::BN, *const srow = colc + D::BN, *const zs = srow + D::BM, *const rowc = zs + D::BM;
+  if (vi < D::BN) {
+    scol[vi] = to_f32<BF16>(v_sc);
+    wred[vi] = asym ? to_f32<BF16>(v_wr) : 0.0f;
+    bias[vi] = p.bias ? to_f32<BF16>(v_bs) : 0.0f;
+    colc[vi] = static_cast<float>(v_cs) * -0.125f;
+  }
+  if (vi < D::BM) {
+    const float s = to_f32<BF16>(v_sr);
+    srow[vi] = s;
+    zs[vi] = asym ? to_f32<BF16>(v_zr) + (D::SIX ? 8.0f : 128.0f) * s : 0.0f;
+    rowc[vi] = static_cast<float>(8 * v_rs - 64 * p.K);
+  }  // (visible behind the exchange's barrier)
+
+  // the first outlier steps of the blocks this wave will own are requested in front of the exchange
+  constexpr int PH = D::PHASES, OS = D::kOutlierSets;
+  v4i ox[OS], ow[OS][PH];
+  const int omi = D::own_mi(wave, 0);
+  auto load_outlier = [&](auto S, int t) QUIK_INLINE {
+    constexpr int s = S;
+    const int64_t step = steps + t;
+    ox[s] = *reinterpret_cast<const v4i *>(p.xbuf + block((m0 + 32 * omi) / 64, x_blocks) + step * UNIT + (omi & 1) * 1024 + head_off);
+#pragma unroll
+    for (int q = 0; q < PH; ++q) {
+      const int row = wrow + 32 * (D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0);
+      ow[s][q] = *reinterpret_cast<const v4i *>(p.wbuf + block(row / 64, w_blocks) + step * UNIT + ((row >> 5) & 1) * 1024 + head_off);
+    }
+  };
+  const bool outliers = fsteps > 0 && !SPLITK;
+  if (outliers) static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, S < fsteps ? S : fsteps - 1); });
+
+  // exchange: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the three it finds
+  v16f own[PH] = {};
+  auto add = [](float a, int b) {
+    return D::SIX ? a + __int_as_float(b) : __int_as_float(__float_as_int(a) + b);
+  };
+  static_for<PH>([&](auto Q) QUIK_INLINE {
+    constexpr int q = Q;
+    if constexpr (q > 0) __syncthreads();  // the slots are free again
+    static_for<WAVES>([&](auto O) QUIK_INLINE {
+      constexpr int o = O;
+      if constexpr (D::owns(o)) {
+        const v16f &b = acc[D::own_mi(o, q)][D::own_ni(o, q)];
+        if (o == wave) {
+          own[q] = b;
+        } else {
+          uint8_t *slot = smem + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
+        }
+      }
+    });
+    __syncthreads();
+    if (D::owns(wave)) {
+#pragma unroll
+      for (int s = 0; s < WAVES - 1; ++s) {
+        const uint8_t *slot = smem + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) own[q][4 * g + e] = add(own[q][4 * g + e], t[e]);
+        }
+      }
+    }
+  });
+
+  if constexpr (SPLITK) {
+    // the same between the workgroups of a tile, through memory (see splitk_combine in gemm_fp6.h): partial sums
+    // [tile][split][wave][phase][group of 4][lane][4]
+    constexpr int kPer = WAVES * PH * 1024;
+    int32_t *part = sk->partials + int64_t(tile_id) * sk->splits * kPer + wave * PH * 1024 + lane * 4;
+    if (D::owns(wave)) {
+#pragma unroll
+      for (int q = 0; q < PH; ++q)
+#pragma unroll
+        for (int g = 0; g < 4; ++g)
+          splitk_store4(part + int64_t(split) * kPer + q * 1024 + g * 256,
+                        v4i{__float_as_int(own[q][4 * g]), __float_as_int(own[q][4 * g + 1]),
+                            __float_as_int(own[q][4 * g + 2]), __float_as_int(own[q][4 * g + 3])});
+    }
+    splitk_stores_done();
+    __syncthreads();
+    int *last_s = reinterpret_cast<int *>(smem);
+    if (threadIdx.x == 0) {
+      const uint32_t before = __hip_atomic_fetch_add(sk->counters + tile_id, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      *last_s = before == static_cast<uint32_t>(sk->splits - 1);
+    }
+    __syncthreads();
+    const bool last = *last_s != 0;
+    if (!last) return;
+    if (fsteps > 0) static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, S < fsteps ? S : fsteps - 1); });
+    if (D::owns(wave)) {
+      for (int o = 0; o < sk->splits; ++o) {
+        if (o == split) continue;
+        const int32_t *theirs = part + int64_t(o) * kPer;
+        v4i t[8];
+        splitk_load4<256>(theirs, t);
+        if constexpr (PH == 2) splitk_load4<256>(theirs + 1024, t + 4);
+#pragma unroll
+        for (int q = 0; q < PH; ++q)
+#pragma unroll
+          for (int g = 0; g < 4; ++g)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) own[q][4 * g + e] = add(own[q][4 * g + e], t[4 * q + g][e]);
+      }
+    }
+    if (threadIdx.x == 0) __hip_atomic_store(sk->counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+
+  // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned blocks
+  if (D::owns(wave)) {
+    const float rs = srow[32 * omi + r], rz = zs[32 * omi + r], rc = D::SIX ? rowc[32 * omi + r] : 0.0f;
+#pragma unroll
+    for (int q = 0; q < PH; ++q) {
+      const int ni = D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int c = ni * 32 + acc_col(g, lane);
+        const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
+                     bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
+        const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
+                    ccv[4] = {cc.x, cc.y, cc.z, cc.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const float raw = own[q][4 * g + e];
+          const float iacc = D::SIX ? __builtin_fmaf(raw + ccv[e], 64.0f, -rc)  // exact: integers below 2^24
+                                    : static_cast<float>(__float_as_int(raw));
+          own[q][4 * g + e] = __builtin_fmaf(iacc, rs * scv[e], __builtin_fmaf(rz, wrv[e], bsv[e]));
+        }
+      }
+    }
+    for (int t0 = 0; t0 < fsteps; t0 += OS) {
+      const bool more = t0 + OS < fsteps;
+      static_for<OS>([&](auto S) QUIK_INLINE {
+        if (t0 + S < fsteps) {
+          static_for<PH>([&](auto Q) QUIK_INLINE { FragOps<BF16 ? kBF16 : kF16>::mma(ox[S], ow[S][Q], own[Q]); });
+        }
+        if (more) load_outlier(S, t0 + OS + S < fsteps ? t0 + OS + S : fsteps - 1);
+      });
+    }
+  }
+  __syncthreads();  // every wave has read its slots: the area becomes the output tile
+  if (D::owns(wave)) {
+#pragma unroll
+    for (int q = 0; q < PH; ++q) {
+      const int ni = D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0;
+#pragma unroll
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (ni * 32 + acc_col(g, lane)) * 2) =
+            make_uint2(pack2_from_f32<BF16>(own[q][4 * g], own[q][4 * g + 1]),
+                       pack2_from_f32<BF16>(own[q][4 * g + 2], own[q][4 * g + 3]));
+    }
+  }
+  __syncthreads();
+  const bool vec = (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
+  constexpr int kPieces = D::BN / 8;  // 16-byte pieces of a row
+#pragma unroll
+  for (int i = threadIdx.x; i < D::BM * kPieces; i += D::kThreads) {
+    const int row = i / kPieces, col = (i % kPieces) * 8;
+    if (m0 + row >= p.M || n0 + col >= p.N) continue;
+    const v4i piece = *reinterpret_cast<const v4i *>(smem + row * D::OUT_STRIDE + col * 2);
+    uint16_t *dst = p.out + int64_t(m0 + row) * p.ldo + n0 + col;
+    if (vec && n0 + col + 8 <= p.N) {
+      __builtin_nontemporal_store(piece, reinterpret_cast<v4i *>(dst));
+    } else {
+      uint16_t tmp[8];
+      __builtin_memcpy(tmp, &piece, 16);
+#pragma unroll
+      for (int e = 0; e < 8; ++e)
+        if (n0 + col + e < p.N) dst[e] = tmp[e];
+    }
+  }
+}
+
+// OCC: workgroups per CU the registers are budgeted for (1: 512 per lane, 2: 256)
+template <class D, bool BF16, int OCC, class Args>
+__global__ __launch_bounds__(D::kThreads, OCC) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  int tm, tn;
+  if (!tile_of_block<D::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
+  direct_tile<D, BF16, false>(p, tm, tn, smem, 0, 0, nullptr);
+}
+template <class D, bool BF16, int OCC, class Args>
+__global__ __launch_bounds__(D::kThreads, OCC) void gemm_direct_splitk_kernel(Args p, int tiles_m, int tiles_n, SplitK sk) {
+  extern __shared__ __align__(16) uint8_t smem[];
+  int tm, tn;
+  const int split = blockIdx.x / sk.grid_tiles;
+  if (!tile_of_block<D::BM>(blockIdx.x - split * sk.grid_tiles, tiles_m, tiles_n, tm, tn)) return;
+  direct_tile<D, BF16, true>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
+}
+
+}  // namespace quik

@@ -428,16 +428,25 @@ __device__ __forceinline__ void run_mainloop(const uint8_t *__restrict__ X, int6
 }
 
 // Workgroup id -> tile.  Hardware deals consecutive workgroup ids round-robin to the 8 XCDs;
-// ids congruent mod 8 therefore share an L2.  Give each XCD a contiguous run of tiles, with M
-// fastest, so concurrently resident tiles of an XCD share W rows and cover all of X.
+// ids congruent mod 8 therefore share an L2.  Give each XCD a contiguous run of tiles.  The run goes through bands of
+// kBandRows token rows, M fastest inside a band: the 32 (or 64) tiles an XCD has in flight then form a block of about as
+// many rows as columns, and what the XCD has to fetch past its 4 MB L2 per k-step, their rows plus their columns, is
+// smallest.  (With M fastest over ALL rows, 8192 rows are 32 tiles of one column each: 8448 operand rows per k-step
+// instead of 3072.  6-bit GEMM 8192 x 28672 x 8192: 1057 -> 919 us, int8 8192 x 8192 x 28672: 1494 -> 1417 us, 2048 rows
+// of 28672 x 8192: 256 -> 247 us; up to 1024 rows nothing changes.)
 // `bid` is the workgroup's index inside its launch region; regions start at multiples of 8.
+constexpr int kBandRows = 1024;
+template <int BM>
 __device__ __forceinline__ bool tile_of_block(int bid, int tiles_m, int tiles_n, int &tm, int &tn) {
+  constexpr int kBand = kBandRows / BM;
   const int total = tiles_m * tiles_n;
   const int per_xcd = (total + 7) / 8;
   const int logical = (bid % 8) * per_xcd + bid / 8;
   if (logical >= total) return false;
-  tm = logical % tiles_m;
-  tn = logical / tiles_m;
+  const int first = logical / (kBand * tiles_n) * kBand, local = logical - first * tiles_n;
+  const int rows = tiles_m - first < kBand ? tiles_m - first : kBand;
+  tm = first + local % rows;
+  tn = local / rows;
   return true;
 }
 
@@ -625,7 +634,7 @@ template <class C, int MODE>
 __global__ __launch_bounds__(C::kThreads) void gemm_i32_kernel(I32Args a, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  if (!tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
+  if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   i32_tile<C, MODE>(a, tm, tn, smem);
 }
 
@@ -710,7 +719,7 @@ template <class C, int MODE, bool ASYM>
 __global__ __launch_bounds__(C::kThreads) void gemm_chain_kernel(I32Args a, ChainArgs e, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  if (!tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
+  if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   chain_tile<C, MODE, ASYM>(a, e, tm, tn, smem);
 }
 
@@ -722,19 +731,20 @@ __global__ __launch_bounds__(C::kThreads) void gemm_chain_kernel(I32Args a, Chai
 struct SplitGrid {
   int tiles_m, tiles_n_wide, tiles_n_tail, lead, wide_blocks;
   // returns 0: no tile, 1: wide tile, 2: tail tile
+  template <int BM>
   __device__ __forceinline__ int locate(int bid, int &tm, int &tn) const {
-    if (bid >= lead && bid < lead + wide_blocks) return tile_of_block(bid - lead, tiles_m, tiles_n_wide, tm, tn) ? 1 : 0;
+    if (bid >= lead && bid < lead + wide_blocks) return tile_of_block<BM>(bid - lead, tiles_m, tiles_n_wide, tm, tn) ? 1 : 0;
     const int local = bid < lead ? bid : bid - wide_blocks;
-    return tile_of_block(local, tiles_m, tiles_n_tail, tm, tn) ? 2 : 0;
+    return tile_of_block<BM>(local, tiles_m, tiles_n_tail, tm, tn) ? 2 : 0;
   }
 };
 
 template <class CW, class CT, int MODE>
 __global__ __launch_bounds__(CW::kThreads) void gemm_i32_split_kernel(I32Args wide, I32Args tail, SplitGrid grid) {
-  static_assert(CW::kThreads == CT::kThreads, "one block size");
+  static_assert(CW::kThreads == CT::kThreads && CW::BM == CT::BM, "one block size, one tile height");
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  const int kind = grid.locate(blockIdx.x, tm, tn);
+  const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
   if (kind == 1) {
     i32_tile<CW, MODE>(wide, tm, tn, smem);
   } else if (kind == 2) {
@@ -907,7 +917,7 @@ template <class C, int MODE, bool BF16>
 __global__ __launch_bounds__(C::kThreads) void gemm_fused_kernel(FusedArgs p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  if (!tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
+  if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   fused_tile<C, MODE, BF16>(p, tm, tn, smem);
 }
 
@@ -915,10 +925,10 @@ __global__ __launch_bounds__(C::kThreads) void gemm_fused_kernel(FusedArgs p, in
 template <class CW, class CT, int MODE, bool BF16>
 __global__ __launch_bounds__(CW::kThreads) void gemm_fused_split_kernel(FusedArgs wide, FusedArgs tail,
                                                                         SplitGrid grid) {
-  static_assert(CW::kThreads == CT::kThreads, "one block size");
+  static_assert(CW::kThreads == CT::kThreads && CW::BM == CT::BM, "one block size, one tile height");
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  const int kind = grid.locate(blockIdx.x, tm, tn);
+  const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
   if (kind == 1) {
     fused_tile<CW, MODE, BF16>(wide, tm, tn, smem);
   } else if (kind == 2) {

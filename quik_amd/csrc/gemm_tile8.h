@@ -385,7 +385,7 @@ template <class C, bool BF16>
 __global__ __launch_bounds__(C::kThreads) void gemm_fused8t_kernel(Fused8Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  if (!tile_of_block(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
+  if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   fused8t_tile<C, BF16>(p, tm, tn, smem);
 }
 
@@ -397,7 +397,7 @@ __global__ __launch_bounds__(C::kThreads) void gemm_fused8t_splitk_kernel(Fused8
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int split = blockIdx.x / sk.grid_tiles;
-  if (!tile_of_block(blockIdx.x - split * sk.grid_tiles, tiles_m, tiles_n, tm, tn)) return;
+  if (!tile_of_block<C::BM>(blockIdx.x - split * sk.grid_tiles, tiles_m, tiles_n, tm, tn)) return;
   fused8t_tile<C, BF16, true>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
 }
 
@@ -405,10 +405,10 @@ __global__ __launch_bounds__(C::kThreads) void gemm_fused8t_splitk_kernel(Fused8
 template <class CW, class CT, bool BF16>
 __global__ __launch_bounds__(CW::kThreads) void gemm_fused8t_split_kernel(Fused8Args wide, Fused8Args tail,
                                                                           SplitGrid grid) {
-  static_assert(CW::kThreads == CT::kThreads, "one block size");
+  static_assert(CW::kThreads == CT::kThreads && CW::BM == CT::BM, "one block size, one tile height");
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
-  const int kind = grid.locate(blockIdx.x, tm, tn);
+  const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
   if (kind == 1) {
     fused8t_tile<CW, BF16>(wide, tm, tn, smem);
   } else if (kind == 2) {
