@@ -39,7 +39,7 @@ struct PyRef {  // owned reference
   ~PyRef() { Py_XDECREF(p); }
 };
 
-PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_finish;
+PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_finish, *s_workspaces, *s_split_k;
 
 // A class keeps its version tag until one of its attributes (or of its bases') is set: methods and class-wide
 // switches are as they were when the plan was made.
@@ -175,15 +175,31 @@ bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &
   int64_t sk_bytes = 0;
   PyRef sk_tensor;
   if (tiled && quik_splitk_workspace_bytes(rows, l.out_features, l.num_int, l.bits) > 0) {
-    PyObject *r = PyObject_CallFunction(p.splitk_fn.p, "OLLLi", p.device_obj.p, static_cast<long long>(rows),
-                                        static_cast<long long>(l.out_features), static_cast<long long>(l.num_int),
-                                        static_cast<int>(l.bits));
-    if (!r) return false;
-    sk_tensor.p = r;
-    PyObject *t = PyTuple_GET_ITEM(r, 0);
-    if (t != Py_None) {
-      sk = const_cast<void *>(data_of(THPVariable_Unpack(t)));
-      sk_bytes = PyLong_AsLongLong(PyTuple_GET_ITEM(r, 1));
+    // the stream's workspace as matmul._splitk_workspace keeps it, or that function where there is none yet
+    PyObject *globals = PyFunction_GetGlobals(p.splitk_fn.p), *known = PyDict_GetItemWithError(globals, s_workspaces);
+    hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
+    const c10::hip::HIPStream cur = c10::hip::getCurrentHIPStream(p.device);
+    if (known && PyDict_GetItemWithError(globals, s_split_k) == Py_True &&
+        hipStreamIsCapturing(cur.stream(), &capture) == hipSuccess && capture == hipStreamCaptureStatusNone) {
+      PyRef key;
+      key.p = Py_BuildValue("(iK)", static_cast<int>(p.device), reinterpret_cast<unsigned long long>(cur.stream()));
+      if (!key.p) return false;
+      if (PyObject *t = PyDict_GetItemWithError(known, key.p); t && THPVariable_CheckExact(t)) {
+        sk = const_cast<void *>(data_of(THPVariable_Unpack(t)));
+        sk_bytes = THPVariable_Unpack(t).numel();
+      }
+    }
+    if (!sk) {
+      PyObject *r = PyObject_CallFunction(p.splitk_fn.p, "OLLLi", p.device_obj.p, static_cast<long long>(rows),
+                                          static_cast<long long>(l.out_features), static_cast<long long>(l.num_int),
+                                          static_cast<int>(l.bits));
+      if (!r) return false;
+      sk_tensor.p = r;
+      PyObject *t = PyTuple_GET_ITEM(r, 0);
+      if (t != Py_None) {
+        sk = const_cast<void *>(data_of(THPVariable_Unpack(t)));
+        sk_bytes = PyLong_AsLongLong(PyTuple_GET_ITEM(r, 1));
+      }
     }
   }
   try {
@@ -506,5 +522,7 @@ PyMODINIT_FUNC PyInit__front() {
   s_fast = PyUnicode_InternFromString("_fast");
   s_fused = PyUnicode_InternFromString("_fused");
   s_finish = PyUnicode_InternFromString("finish");
+  s_workspaces = PyUnicode_InternFromString("_splitk_workspaces");
+  s_split_k = PyUnicode_InternFromString("split_k");
   return PyModule_Create(&kModule);
 }

@@ -10,6 +10,7 @@
 #ifndef GEMV_MAX_ROWS
 #define GEMV_MAX_ROWS 2
 #endif
+#include "gemm_direct.h"
 #include "gemm_tile8.h"
 #include "gemm_kernels.h"
 
@@ -479,12 +480,78 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
   return check_launch();
 }
 
+// Register-streaming kernel (gemm_direct.h) or ring kernel, for problems below the 256-row tiles.  Both are priced in ns:
+// a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (45 .. 50 per cycle, whichever kernel asks),
+// never less than the weights at 5.5 TB/s, and for a K split the exchange (its partial sums cross memory: 16 KB per
+// workgroup here, 64 KB in the ring kernel).  Constants fitted to 21 shapes of 40 .. 2048 rows and 1024 .. 28672 columns,
+// both widths; the choice was right on all of them to within 0.5 us.
+struct DirectPlan {
+  int bn, splits;  // tile width (64 or 32; 0: ring kernel), workgroups per tile
+  int64_t bytes;   // workspace of the split
+};
+DirectPlan plan_direct(int64_t M, int64_t N, int64_t K, int bits, int64_t workspace_bytes) {
+  const DirectPlan ring{0, 1, 0};
+  if (make_plan6(M, N, 1).kind != Plan::kMid) return ring;
+  const int64_t steps = bits == 4 ? K / 64 : K / 32, unit = bits == 4 ? 3072 : 2048, cus = num_cus();
+  const int64_t stream = N * steps * unit / 64 * 10 / 55000;
+  auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
+  auto busiest = [&](int64_t groups, int64_t per, int64_t step_bytes) {
+    const int64_t ns = up(groups, cus) * per * step_bytes / 103;
+    return ns > stream ? ns : stream;
+  };
+  const int64_t tiles128 = up(M, 128) * up(N, 128);
+  const SplitPlan sp = plan_splitk(M, N, steps, bits == 4 ? kSplitMinSteps6 : kSplitMinSteps8, 1, bits == 4 ? 3 : 2);
+  int64_t best = sp.splits > 1 && workspace_bytes >= sp.bytes ? 10000 + 1500 * sp.splits + busiest(tiles128 * sp.splits, sp.per, 4 * unit)
+                 : bits == 4 && tiles128 * 8 <= cus * 5        ? 5800 + busiest(up(M, 128) * up(N, 64), steps, 3 * unit)
+                                                               : 5800 + busiest(tiles128, steps, 4 * unit);
+  DirectPlan plan = ring;
+  for (const int bn : {64, 32}) {
+    const int64_t tiles = up(M, 64) * up(N, bn);
+    for (const int splits : {1, 2, 4}) {
+      const int64_t bytes = splits > 1 ? kSplitCounterBytes + tiles * splits * DirectCfg<true, 2, 2, 4>::PARTIAL_BYTES : 0;
+      if (splits > 1 && (tiles * 4 > kSplitCounterBytes || bytes > workspace_bytes || up(steps, splits) * (splits - 1) >= steps)) continue;
+      const int64_t ns = 6300 + (splits > 1 ? 1500 + 500 * splits : 0) + busiest(tiles * splits, up(steps, splits), unit + unit * bn / 64);
+      if (ns < best) best = ns, plan = {bn, splits, bytes};
+    }
+  }
+  return plan;
+}
+
+template <class D, bool BF16, class Args>
+int launch_direct(const Args &p, int splits, void *workspace, hipStream_t st) {
+  int tiles_m, tiles_n;
+  const int grid = grid_of<D>(p.M, p.N, tiles_m, tiles_n);
+  if (splits > 1) {
+    const int steps = p.K / (D::SIX ? 64 : 32);
+    SplitK sk{splits, (steps + splits - 1) / splits, grid, static_cast<uint32_t *>(workspace),
+              reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace) + kSplitCounterBytes)};
+    auto kern = gemm_direct_splitk_kernel<D, BF16, Args>;
+    if (int rc = prepare(kern, D::SMEM)) return rc;
+    hipLaunchKernelGGL(kern, dim3(grid * splits), dim3(D::kThreads), D::SMEM, st, p, tiles_m, tiles_n, sk);
+    return splitk_launch_status(workspace, st);
+  }
+  auto kern = gemm_direct_kernel<D, BF16, Args>;
+  if (int rc = prepare(kern, D::SMEM)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(D::kThreads), D::SMEM, st, p, tiles_m, tiles_n);
+  return check_launch();
+}
+// kChainNotHandled: the ring kernels serve this call.  SETS: as many steps in flight as registers allow with two
+// workgroups per CU; more measured no better
+template <bool SIX, bool BF16, class Args>
+int run_direct(const Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
+  const DirectPlan d = plan_direct(p.M, p.N, p.K, SIX ? 4 : 8, workspace ? workspace_bytes : 0);
+  if (d.bn == 64) return launch_direct<DirectCfg<SIX, 2, 2, SIX ? 4 : 6>, BF16>(p, d.splits, workspace, st);
+  if (d.bn == 32) return launch_direct<DirectCfg<SIX, 2, 1, SIX ? 8 : 10>, BF16>(p, d.splits, workspace, st);
+  return kChainNotHandled;
+}
+
 // The 6-bit matrix-core path (gemm_fp6.h): 256x256 tiles alone (eight waves), 256x256 + 256x128 tiles in one
 // launch (four waves), or 128x128 tiles.
 template <bool BF16>
 int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
   // any row count: up to 32 rows the weight-streaming kernel on the packed nibbles reads a third fewer bytes, and
   // callers that keep both weight copies route such calls there
+  if (const int rc = run_direct<true, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
   const Plan plan = make_plan6(p.M, p.N, 1);
   if (plan.kind == Plan::kSplit && plan.n_wide >= p.N) return launch_fused6<CfgL8, BF16>(p, st);
   if (plan.kind != Plan::kSplit) {
@@ -538,6 +605,7 @@ int launch_fused8t_split(const Fused8Args &wide, const Fused8Args &tail, hipStre
 // W8A8 on tile-ordered operands (gemm_tile8.h): same plan and tile shapes as the 6-bit path.
 template <bool BF16>
 int run_fused8t(const Fused8Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
+  if (const int rc = run_direct<false, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
   const Plan plan = make_plan6(p.M, p.N, 1);  // any row count: with few rows this path competes with the weight-streaming kernel
   if (plan.kind != Plan::kSplit) {
     const SplitPlan sp = plan_splitk(p.M, p.N, p.K / 32, kSplitMinSteps8, 1, 2);
@@ -707,7 +775,12 @@ extern "C" int quik_mixed_linear_fwd(const void *qx, const void *qw, const void 
 extern "C" int64_t quik_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits) {
   if (M <= 0 || N <= 0 || K <= 0 || (bits != 4 && bits != 8)) return 0;
   if (bits == 4 ? K % 128 != 0 : K % 64 != 0) return 0;
-  return (bits == 4 ? plan_splitk(M, N, K / 64, kSplitMinSteps6, 1, 3) : plan_splitk(M, N, K / 32, kSplitMinSteps8, 1, 2)).bytes;
+  // whichever kernel a call with that much workspace takes; a shape the ring kernels would split keeps its workspace
+  // even where the register-streaming kernel then does without
+  const int64_t ring = (bits == 4 ? plan_splitk(M, N, K / 64, kSplitMinSteps6, 1, 3)
+                                  : plan_splitk(M, N, K / 32, kSplitMinSteps8, 1, 2)).bytes;
+  const int64_t direct = plan_direct(M, N, K, bits, kSplitCounterBytes + int64_t(kMaxCUs) * 128 * 128 * 4).bytes;
+  return ring > direct ? ring : direct;
 }
 
 extern "C" int quik_mixed_linear_fwd_fp6(const void *x6, const void *w6, const void *meta, const void *s_col,

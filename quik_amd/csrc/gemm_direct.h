@@ -6,12 +6,17 @@
 // (measured 250 .. 300 cycles a step; 13824 columns at 128 rows: 16 us for 53 MB of weights).  The operand buffers hold
 // each fragment as one contiguous kilobyte (fp6_format.h), so a wave can load fragments directly, and nothing has to be
 // shared inside the workgroup if the waves split K instead of the tile: each of the four waves computes the WHOLE tile
-// over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of loads in flight.
-// The traffic between a CU and its L2 is that of a ring kernel with the same tile.  Afterwards the waves add their
+// (64x64 or 64x32) over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of
+// loads in flight.  What bounds it is the rate at which a CU takes in operands, 45 .. 50 bytes per cycle (a ring kernel
+// with the same tile moves the same bytes).  Afterwards the waves add their
 // integer sums through LDS (exact, so in any order), each ending up with the blocks it owns, convert them, run the
 // outlier steps on them in the same order as the ring kernels and store: the same output bits.
 //
 // Workgroups may share a tile's K further (SplitK, as in gemm_fp6.h): when the tiles are fewer than the CUs.
+//
+// Measured against the ring kernels (GEMM launch in a graph, us): W4A4 64 x 8192 x 7936 22.7 -> 12.6, 64 x 10240 x 7936
+// 23.0 -> 14.9, 128 x 8192 x 7936 23.4 -> 14.4, 40 x 4096 x 3840 11.9 -> 8.5, 256 x 4096 x 3840 12.1 -> 9.8,
+// 512 x 1024 x 3968 9.9 -> 7.7; W8A8 64 x 5120 x 13568 27.1 -> 18.0, 64 x 4096 x 10752 26.6 -> 13.9.
 #pragma once
 #include <type_traits>
 
@@ -29,17 +34,18 @@ struct DirectCfg {
   static constexpr int WAVES = 4, kThreads = 64 * WAVES;
   static constexpr int BM = 32 * MI, BN = 32 * NI;
   static constexpr int UNIT = SIX ? 3072 : 2048;
-  static constexpr int PHASES = MI * NI > WAVES ? MI * NI / WAVES : 1;  // blocks a wave owns
-  static_assert((MI == 4 && NI == 2) || (MI == 2 && (NI == 2 || NI == 1)), "supported tiles");
-  static constexpr int kOutlierSets = 8;
+  // (larger tiles, 128x64 and 64x128, were slower at every shape tried: their exchange and outlier steps take 2 us more)
+  static_assert(MI == 2 && (NI == 2 || NI == 1), "supported tiles");
+  static constexpr int kOutlierSets = 16;  // outlier steps in flight: all of them for 256 columns
   static constexpr int RED_BYTES = WAVES * (WAVES - 1) * 4096;
+  static constexpr int PARTIAL_BYTES = WAVES * 4096;  // a workgroup's partial sums (SplitK)
   static constexpr int OUT_STRIDE = BN * 2 + 16;
   static constexpr int VEC_OFF = RED_BYTES > BM * OUT_STRIDE ? RED_BYTES : BM * OUT_STRIDE;
   static constexpr int SMEM = VEC_OFF + (4 * BN + 3 * BM) * 4;
-  // block (mi, ni) owned by wave w in phase p; waves without one (64x32 tiles have two blocks) own nothing
-  static constexpr int own_mi(int w, int) { return MI == 4 ? w : w & 1; }
-  static constexpr int own_ni(int w, int p) { return MI == 4 ? p : w >> 1; }
-  static constexpr bool owns(int w) { return MI == 4 || (w >> 1) < NI; }
+  // the 32x32 block (mi, ni) that wave w owns after the exchange; 64x32 tiles have two blocks, waves 2 and 3 none
+  static constexpr int own_mi(int w) { return w & 1; }
+  static constexpr int own_ni(int w) { return w >> 1; }
+  static constexpr bool owns(int w) { return own_ni(w) < NI; }
 };
 
 // One step's fragments of a wave.  6-bit: head in dwords 0 .. 3, tail in 4 and 5, as the MFMA takes it.  (Kept as whole
@@ -170,76 +176,69 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     const float s = to_f32<BF16>(v_sr);
     srow[vi] = s;
     zs[vi] = asym ? to_f32<BF16>(v_zr) + (D::SIX ? 8.0f : 128.0f) * s : 0.0f;
-    rowc[vi] = static_cast<float>(8 * v_rs - 64 * p.K);
+    rowc[vi] = D::SIX ? static_cast<float>(8 * v_rs - 64 * p.K) : 0.0f;
   }  // (visible behind the exchange's barrier)
 
-  // the first outlier steps of the blocks this wave will own are requested in front of the exchange
-  constexpr int PH = D::PHASES, OS = D::kOutlierSets;
-  v4i ox[OS], ow[OS][PH];
-  const int omi = D::own_mi(wave, 0);
+  // the first outlier steps of the block this wave will own are requested in front of the exchange
+  constexpr int OS = D::kOutlierSets;
+  v4i ox[OS], ow[OS];
+  const int omi = D::own_mi(wave), oni = D::owns(wave) ? D::own_ni(wave) : 0;
+  const uint8_t *const ox_base = p.xbuf + block(m0 / 64, x_blocks) + omi * 1024;
+  const uint8_t *const ow_base = p.wbuf + block((wrow + 32 * oni) / 64, w_blocks) + (((wrow + 32 * oni) >> 5) & 1) * 1024;
   auto load_outlier = [&](auto S, int t) QUIK_INLINE {
-    constexpr int s = S;
     const int64_t step = steps + t;
-    ox[s] = *reinterpret_cast<const v4i *>(p.xbuf + block((m0 + 32 * omi) / 64, x_blocks) + step * UNIT + (omi & 1) * 1024 + head_off);
-#pragma unroll
-    for (int q = 0; q < PH; ++q) {
-      const int row = wrow + 32 * (D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0);
-      ow[s][q] = *reinterpret_cast<const v4i *>(p.wbuf + block(row / 64, w_blocks) + step * UNIT + ((row >> 5) & 1) * 1024 + head_off);
-    }
+    ox[S] = *reinterpret_cast<const v4i *>(ox_base + step * UNIT + head_off);
+    ow[S] = *reinterpret_cast<const v4i *>(ow_base + step * UNIT + head_off);
   };
-  const bool outliers = fsteps > 0 && !SPLITK;
-  if (outliers) static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, S < fsteps ? S : fsteps - 1); });
+  auto load_outliers = [&](int t0) QUIK_INLINE {
+    static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, t0 + S < fsteps ? t0 + S : fsteps - 1); });
+  };
+  if (!SPLITK && fsteps > 0) load_outliers(0);
 
   // exchange: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the three it finds
-  v16f own[PH] = {};
-  auto add = [](float a, int b) {
+  v16f own = {};
+  auto add = [](float a, int b) QUIK_INLINE {
     return D::SIX ? a + __int_as_float(b) : __int_as_float(__float_as_int(a) + b);
   };
-  static_for<PH>([&](auto Q) QUIK_INLINE {
-    constexpr int q = Q;
-    if constexpr (q > 0) __syncthreads();  // the slots are free again
-    static_for<WAVES>([&](auto O) QUIK_INLINE {
-      constexpr int o = O;
-      if constexpr (D::owns(o)) {
-        const v16f &b = acc[D::own_mi(o, q)][D::own_ni(o, q)];
-        if (o == wave) {
-          own[q] = b;
-        } else {
-          uint8_t *slot = smem + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
+  static_for<WAVES>([&](auto O) QUIK_INLINE {
+    constexpr int o = O;
+    if constexpr (D::owns(o)) {
+      const v16f &b = acc[D::own_mi(o)][D::own_ni(o)];
+      if (o == wave) {
+        own = b;
+      } else {
+        uint8_t *slot = smem + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
-        }
-      }
-    });
-    __syncthreads();
-    if (D::owns(wave)) {
-#pragma unroll
-      for (int s = 0; s < WAVES - 1; ++s) {
-        const uint8_t *slot = smem + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
-#pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) own[q][4 * g + e] = add(own[q][4 * g + e], t[e]);
-        }
+        for (int g = 0; g < 4; ++g)
+          *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
       }
     }
   });
+  __syncthreads();
+  if (D::owns(wave)) {
+#pragma unroll
+    for (int s = 0; s < WAVES - 1; ++s) {
+      const uint8_t *slot = smem + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) own[4 * g + e] = add(own[4 * g + e], t[e]);
+      }
+    }
+  }
 
   if constexpr (SPLITK) {
     // the same between the workgroups of a tile, through memory (see splitk_combine in gemm_fp6.h): partial sums
-    // [tile][split][wave][phase][group of 4][lane][4]
-    constexpr int kPer = WAVES * PH * 1024;
-    int32_t *part = sk->partials + int64_t(tile_id) * sk->splits * kPer + wave * PH * 1024 + lane * 4;
+    // [tile][split][wave][group of 4][lane][4]
+    constexpr int kPer = D::PARTIAL_BYTES / 4;
+    int32_t *part = sk->partials + int64_t(tile_id) * sk->splits * kPer + wave * 1024 + lane * 4;
     if (D::owns(wave)) {
 #pragma unroll
-      for (int q = 0; q < PH; ++q)
-#pragma unroll
-        for (int g = 0; g < 4; ++g)
-          splitk_store4(part + int64_t(split) * kPer + q * 1024 + g * 256,
-                        v4i{__float_as_int(own[q][4 * g]), __float_as_int(own[q][4 * g + 1]),
-                            __float_as_int(own[q][4 * g + 2]), __float_as_int(own[q][4 * g + 3])});
+      for (int g = 0; g < 4; ++g)
+        splitk_store4(part + int64_t(split) * kPer + g * 256,
+                      v4i{__float_as_int(own[4 * g]), __float_as_int(own[4 * g + 1]), __float_as_int(own[4 * g + 2]),
+                          __float_as_int(own[4 * g + 3])});
     }
     splitk_stores_done();
     __syncthreads();
@@ -249,55 +248,44 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
       *last_s = before == static_cast<uint32_t>(sk->splits - 1);
     }
     __syncthreads();
-    const bool last = *last_s != 0;
-    if (!last) return;
-    if (fsteps > 0) static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, S < fsteps ? S : fsteps - 1); });
+    if (*last_s == 0) return;
+    if (fsteps > 0) load_outliers(0);
     if (D::owns(wave)) {
       for (int o = 0; o < sk->splits; ++o) {
         if (o == split) continue;
-        const int32_t *theirs = part + int64_t(o) * kPer;
-        v4i t[8];
-        splitk_load4<256>(theirs, t);
-        if constexpr (PH == 2) splitk_load4<256>(theirs + 1024, t + 4);
+        v4i t[4];
+        splitk_load4<256>(part + int64_t(o) * kPer, t);
 #pragma unroll
-        for (int q = 0; q < PH; ++q)
+        for (int g = 0; g < 4; ++g)
 #pragma unroll
-          for (int g = 0; g < 4; ++g)
-#pragma unroll
-            for (int e = 0; e < 4; ++e) own[q][4 * g + e] = add(own[q][4 * g + e], t[4 * q + g][e]);
+          for (int e = 0; e < 4; ++e) own[4 * g + e] = add(own[4 * g + e], t[g][e]);
       }
     }
     if (threadIdx.x == 0) __hip_atomic_store(sk->counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned blocks
+  // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned block
   if (D::owns(wave)) {
-    const float rs = srow[32 * omi + r], rz = zs[32 * omi + r], rc = D::SIX ? rowc[32 * omi + r] : 0.0f;
+    const float rs = srow[32 * omi + r], rz = zs[32 * omi + r], rc = rowc[32 * omi + r];
 #pragma unroll
-    for (int q = 0; q < PH; ++q) {
-      const int ni = D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0;
+    for (int g = 0; g < 4; ++g) {
+      const int c = oni * 32 + acc_col(g, lane);
+      const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
+                   bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
+      const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
+                  ccv[4] = {cc.x, cc.y, cc.z, cc.w};
 #pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const int c = ni * 32 + acc_col(g, lane);
-        const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
-                     bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
-        const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
-                    ccv[4] = {cc.x, cc.y, cc.z, cc.w};
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          const float raw = own[q][4 * g + e];
-          const float iacc = D::SIX ? __builtin_fmaf(raw + ccv[e], 64.0f, -rc)  // exact: integers below 2^24
-                                    : static_cast<float>(__float_as_int(raw));
-          own[q][4 * g + e] = __builtin_fmaf(iacc, rs * scv[e], __builtin_fmaf(rz, wrv[e], bsv[e]));
-        }
+      for (int e = 0; e < 4; ++e) {
+        const float raw = own[4 * g + e];
+        const float iacc = D::SIX ? __builtin_fmaf(raw + ccv[e], 64.0f, -rc)  // exact: integers below 2^24
+                                  : static_cast<float>(__float_as_int(raw));
+        own[4 * g + e] = __builtin_fmaf(iacc, rs * scv[e], __builtin_fmaf(rz, wrv[e], bsv[e]));
       }
     }
     for (int t0 = 0; t0 < fsteps; t0 += OS) {
       const bool more = t0 + OS < fsteps;
       static_for<OS>([&](auto S) QUIK_INLINE {
-        if (t0 + S < fsteps) {
-          static_for<PH>([&](auto Q) QUIK_INLINE { FragOps<BF16 ? kBF16 : kF16>::mma(ox[S], ow[S][Q], own[Q]); });
-        }
+        if (t0 + S < fsteps) FragOps<BF16 ? kBF16 : kF16>::mma(ox[S], ow[S], own);
         if (more) load_outlier(S, t0 + OS + S < fsteps ? t0 + OS + S : fsteps - 1);
       });
     }
@@ -305,14 +293,9 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   __syncthreads();  // every wave has read its slots: the area becomes the output tile
   if (D::owns(wave)) {
 #pragma unroll
-    for (int q = 0; q < PH; ++q) {
-      const int ni = D::MI == 4 ? q : NI > 1 ? wave >> 1 : 0;
-#pragma unroll
-      for (int g = 0; g < 4; ++g)
-        *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (ni * 32 + acc_col(g, lane)) * 2) =
-            make_uint2(pack2_from_f32<BF16>(own[q][4 * g], own[q][4 * g + 1]),
-                       pack2_from_f32<BF16>(own[q][4 * g + 2], own[q][4 * g + 3]));
-    }
+    for (int g = 0; g < 4; ++g)
+      *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (oni * 32 + acc_col(g, lane)) * 2) =
+          make_uint2(pack2_from_f32<BF16>(own[4 * g], own[4 * g + 1]), pack2_from_f32<BF16>(own[4 * g + 2], own[4 * g + 3]));
   }
   __syncthreads();
   const bool vec = (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
@@ -335,16 +318,15 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   }
 }
 
-// OCC: workgroups per CU the registers are budgeted for (1: 512 per lane, 2: 256)
-template <class D, bool BF16, int OCC, class Args>
-__global__ __launch_bounds__(D::kThreads, OCC) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
+template <class D, bool BF16, class Args>
+__global__ __launch_bounds__(D::kThreads, 2) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_of_block<D::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   direct_tile<D, BF16, false>(p, tm, tn, smem, 0, 0, nullptr);
 }
-template <class D, bool BF16, int OCC, class Args>
-__global__ __launch_bounds__(D::kThreads, OCC) void gemm_direct_splitk_kernel(Args p, int tiles_m, int tiles_n, SplitK sk) {
+template <class D, bool BF16, class Args>
+__global__ __launch_bounds__(D::kThreads, 2) void gemm_direct_splitk_kernel(Args p, int tiles_m, int tiles_n, SplitK sk) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int split = blockIdx.x / sk.grid_tiles;

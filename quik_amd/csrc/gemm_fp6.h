@@ -459,6 +459,17 @@ __device__ __forceinline__ void splitk_load8(const int32_t *p, v4i *r) {
       : "memory");
 }
 
+template <int STRIDE>
+__device__ __forceinline__ void splitk_load4(const int32_t *p, v4i *r) {
+  asm volatile(
+      "global_load_dwordx4 %0, %4, off sc1\n\tglobal_load_dwordx4 %1, %5, off sc1\n\t"
+      "global_load_dwordx4 %2, %6, off sc1\n\tglobal_load_dwordx4 %3, %7, off sc1\n\t"
+      "s_waitcnt vmcnt(0)"
+      : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+      : "v"(p), "v"(p + STRIDE), "v"(p + 2 * STRIDE), "v"(p + 3 * STRIDE)
+      : "memory");
+}
+
 // Adds a tile's raw accumulators over the splits (see SplitK).  Returns false in every workgroup but the one that
 // arrived last; there `acc` holds the whole-K sums (INT: int32 bit patterns, else fp32) and the ring is idle.
 template <class C, bool INT>
