@@ -257,7 +257,7 @@ int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *m
  *                   quik_colmap_streaming returned for it
  *   int_weight [out, num_int/2] u8 or [out, num_int] i8; weights_scales [out]; reduced_w [out] (NULL when
  *   symmetric); fp_weight [out, num_fp] (NULL when num_fp == 0); bias [out] or NULL
- *   tiled_weight    quik_fp6_pack_weight (bits 4) / quik_tile8_pack_weight (bits 8) buffer, or NULL
+ *   tiled_weight    quik_layer_pack_weight (or quik_fp6_pack_weight / quik_tile8_pack_weight) buffer, or NULL
  *   tiled_min_rows  33 is what MixedQLinear uses.  With 1 every call takes the tile-ordered path and reads
  *                   only tiled_weight: int_weight and fp_weight may then be NULL, i.e. the layer can live
  *                   with ONE copy of its weights (0.75 byte per int4 weight, 1 per int8 weight) at the price
@@ -274,6 +274,14 @@ typedef struct quik_layer {
   int32_t colmap_streams, tiled_min_rows, reserved;
   const void *colmap, *int_weight, *weights_scales, *reduced_w, *fp_weight, *bias, *tiled_weight;
 } quik_layer;
+/* tiled_weight for a layer whose integer columns are no multiple of 128 (4 bits; then of 32) or 64 (8 bits; of 16):
+ * the buffer of quik_fp6_pack_weight / quik_tile8_pack_weight with the last k-steps filled up with zeros, for
+ * quik_layer_forward only (identical to theirs where those take the shape).  colmap: 4 bits only.
+ * quik_layer_weight_bytes returns 0 for a shape the tile-ordered path does not take. */
+int64_t quik_layer_weight_bytes(int64_t N, int64_t K, int64_t F, int bits);
+int quik_layer_pack_weight(const void *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, int bits,
+                           const void *colmap, void *out, void *stream);
+
 int64_t quik_layer_workspace_bytes(const quik_layer *layer, int64_t rows);
 int quik_layer_forward(const quik_layer *layer, const void *x, int64_t rows, void *workspace,
                        int64_t workspace_bytes, void *splitk_workspace, int64_t splitk_bytes, void *out,

@@ -47,6 +47,8 @@ SIGNATURES = {
                                             _vp]),
     "quik_mixed_linear_fwd_tile8_ws": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _i64,
                                               _vp]),
+    "quik_layer_weight_bytes": (_i64, [_i64, _i64, _i64, _int]),
+    "quik_layer_pack_weight": (_int, [_vp, _vp, _i64, _i64, _i64, _int, _vp, _vp, _vp]),
     "quik_layer_workspace_bytes": (_i64, [_vp, _i64]),
     "quik_layer_forward": (_int, [_vp, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _vp, _vp]),
     "quik_layer_set_one_launch": (None, [_int]),

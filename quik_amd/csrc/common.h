@@ -39,6 +39,26 @@ int gemv_forward_one_launch(const void *x, int dtype, int64_t rows, int64_t cols
                             const void *fp_w, const void *bias, int64_t N, void *out, float sym_divisor,
                             hipStream_t st);
 
+// The tile-ordered steps of a layer forward, for any number of integer columns that fills whole fragments (4 bits: a
+// multiple of kLayerK4, 8 bits: of kLayerK8).  The exported functions of the same steps (quik_asym_quantize_fp6, ...) ask
+// for whole pairs of k-steps, 128 / 64 columns, and pass that as `k_multiple`.
+constexpr int64_t kLayerK4 = 32, kLayerK8 = 16;
+int64_t fp6_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple);
+int64_t tile8_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple);
+int asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
+                      int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple);
+int asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
+                        int64_t num_fp, void *out8, void *meta, void *stream, int64_t k_multiple);
+int sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp,
+                        int bits, float divisor, int tiled, void *dst, void *scale, void *fp_x, void *stream,
+                        int64_t k_multiple);
+int mixed_linear_fp6(const void *x6, const void *w6, const void *meta, const void *s_col, const void *w_reduced,
+                     const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
+                     void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);
+int mixed_linear_tile8(const void *x8, const void *w8, const void *meta, const void *s_col, const void *w_reduced,
+                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
+                       void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);
+
 // gemm.hip: integer GEMM + the fp16-arithmetic epilogue of the reference's fused ops in one launch (zero_row ==
 // NULL: symmetric form).  Returns kChainNotHandled for shapes it leaves to the two-launch path.
 constexpr int kChainNotHandled = 1;

@@ -32,6 +32,11 @@ __global__ __launch_bounds__(kThreads) void pack_weight_kernel(const uint8_t *__
   __syncthreads();
   int sum = 0;
   for (int64_t f = threadIdx.x; f < frags_per_row; f += kThreads) {
+    if (f >= K / 32) {  // positions past the integer columns: levels of 0
+      const uint32_t zero[6] = {};
+      fp6_store_fragment(out, l, row, f, zero);
+      continue;
+    }
     uint32_t b[8];
 #pragma unroll
     for (int i = 0; i < 8; ++i) {
@@ -61,28 +66,18 @@ __global__ __launch_bounds__(kThreads) void pack_weight8_kernel(const uint8_t *_
                                                                 int64_t K, int64_t F, uint8_t *__restrict__ out) {
   const Tile8Layout l = tile8_layout(rows, K, F);
   const int64_t row = blockIdx.x;
-  for (int64_t c = threadIdx.x; c < K / 16; c += kThreads)
+  for (int64_t c = threadIdx.x; c < 2 * l.steps; c += kThreads)  // (zeros past the integer columns)
     *reinterpret_cast<uint4 *>(out + tile8_offset(l, row, c >> 1, static_cast<int>(c & 1))) =
-        *reinterpret_cast<const uint4 *>(qw + row * K + c * 16);
+        c < K / 16 ? *reinterpret_cast<const uint4 *>(qw + row * K + c * 16) : make_uint4(0, 0, 0, 0);
   for (int64_t c = threadIdx.x; c < F / 8; c += kThreads)
     *reinterpret_cast<uint4 *>(out + tile8_offset(l, row, l.steps + (c >> 1), static_cast<int>(c & 1))) =
         *reinterpret_cast<const uint4 *>(fp_w + row * F + c * 8);
 }
 
-}  // namespace
-}  // namespace quik
-
-using namespace quik;
-
-extern "C" int64_t quik_tile8_operand_bytes(int64_t rows, int64_t K, int64_t F) {
-  if (rows <= 0 || K <= 0 || K % 64 != 0 || F < 0 || F % 32 != 0) return 0;
-  return tile8_layout(rows, K, F).bytes;
-}
-
-extern "C" int quik_tile8_pack_weight(const int8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, void *out,
-                                      void *stream) {
+int tile8_pack_weight(const int8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, void *out, void *stream,
+                      int64_t k_multiple) {
   if (N <= 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
-  if (K % 64 != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
+  if (K % k_multiple != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
   if (!qw || !out || (F > 0 && !fp_w)) return QUIK_ERR_NULL;
   if (reinterpret_cast<uintptr_t>(qw) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 256 != 0 ||
       reinterpret_cast<uintptr_t>(fp_w) % 16 != 0)
@@ -94,15 +89,10 @@ extern "C" int quik_tile8_pack_weight(const int8_t *qw, const void *fp_w, int64_
   return check_launch();
 }
 
-extern "C" int64_t quik_fp6_operand_bytes(int64_t rows, int64_t K, int64_t F) {
-  if (rows <= 0 || K <= 0 || K % 128 != 0 || K > 74496 || F < 0 || F % 32 != 0) return 0;
-  return fp6_layout(rows, K, F).bytes;
-}
-
-extern "C" int quik_fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F,
-                                    const void *colmap, void *out, void *stream) {
+int fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, const void *colmap, void *out,
+                    void *stream, int64_t k_multiple) {
   if (N <= 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
-  if (K % 128 != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
+  if (K % k_multiple != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
   if (!qw || !out || !colmap || (F > 0 && !fp_w)) return QUIK_ERR_NULL;
   if (reinterpret_cast<uintptr_t>(qw) % 16 != 0 || reinterpret_cast<uintptr_t>(out) % 256 != 0 ||
       reinterpret_cast<uintptr_t>(fp_w) % 16 != 0 || reinterpret_cast<uintptr_t>(colmap) % 16 != 0)
@@ -116,4 +106,44 @@ extern "C" int quik_fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t
                      reinterpret_cast<const uint16_t *>(cm + cl.off_kperm),
                      reinterpret_cast<const uint32_t *>(cm + cl.off_flags), N, K, F, static_cast<uint8_t *>(out));
   return check_launch();
+}
+
+}  // namespace
+
+int64_t tile8_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple) {
+  if (rows <= 0 || K <= 0 || K % k_multiple != 0 || F < 0 || F % 32 != 0) return 0;
+  return tile8_layout(rows, K, F).bytes;
+}
+
+int64_t fp6_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple) {
+  if (rows <= 0 || K <= 0 || K % k_multiple != 0 || K > 74496 || F < 0 || F % 32 != 0) return 0;
+  return fp6_layout(rows, K, F).bytes;
+}
+}  // namespace quik
+
+using namespace quik;
+
+extern "C" int64_t quik_tile8_operand_bytes(int64_t rows, int64_t K, int64_t F) { return tile8_operand_bytes(rows, K, F, 64); }
+
+extern "C" int64_t quik_fp6_operand_bytes(int64_t rows, int64_t K, int64_t F) { return fp6_operand_bytes(rows, K, F, 128); }
+
+extern "C" int quik_tile8_pack_weight(const int8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, void *out,
+                                      void *stream) {
+  return tile8_pack_weight(qw, fp_w, N, K, F, out, stream, 64);
+}
+
+extern "C" int quik_fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F,
+                                    const void *colmap, void *out, void *stream) {
+  return fp6_pack_weight(qw, fp_w, N, K, F, colmap, out, stream, 128);
+}
+
+extern "C" int64_t quik_layer_weight_bytes(int64_t N, int64_t K, int64_t F, int bits) {
+  return bits == 4 ? fp6_operand_bytes(N, K, F, kLayerK4) : bits == 8 ? tile8_operand_bytes(N, K, F, kLayerK8) : 0;
+}
+
+extern "C" int quik_layer_pack_weight(const void *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, int bits,
+                                      const void *colmap, void *out, void *stream) {
+  if (bits == 4) return fp6_pack_weight(static_cast<const uint8_t *>(qw), fp_w, N, K, F, colmap, out, stream, kLayerK4);
+  if (bits == 8) return tile8_pack_weight(static_cast<const int8_t *>(qw), fp_w, N, K, F, out, stream, kLayerK8);
+  return QUIK_ERR_BITS;
 }

@@ -23,6 +23,9 @@
 // A block's units are contiguous: K / 64 integer steps, then F / 16 outlier steps, so the GEMM walks one
 // pointer per block through all its steps.  The buffer ends with one int32 per row: the sum of the row's
 // levels.
+// Integer columns that are no multiple of 128 (int8: 64): the steps are rounded up to an even number and the positions
+// past K are zero in the weights (levels of 0, not codes of 0), so that what stands there in the activations, which is
+// never written, does not matter: any 6-bit pattern is a finite number.  The level sums are those of the K columns.
 // Rows of the last block beyond the matrix are never written; any bit pattern is a finite E2M3
 // or half value times results that are never stored.
 #pragma once
@@ -36,7 +39,7 @@ struct Fp6Layout {
 __host__ __device__ inline Fp6Layout fp6_layout(int64_t rows, int64_t K, int64_t F) {
   Fp6Layout l;
   l.blocks = (rows + 63) / 64;
-  l.steps = K / 64;
+  l.steps = (K + 127) / 128 * 2;
   l.fsteps = F / 16;
   l.block_bytes = (l.steps + l.fsteps) * 3072;
   l.sums_off = l.blocks * l.block_bytes;
@@ -64,7 +67,7 @@ struct Tile8Layout {
 __host__ __device__ inline Tile8Layout tile8_layout(int64_t rows, int64_t K, int64_t F) {
   Tile8Layout l;
   l.blocks = (rows + 63) / 64;
-  l.steps = K / 32;
+  l.steps = (K + 63) / 64 * 2;
   l.fsteps = F / 16;
   l.block_bytes = (l.steps + l.fsteps) * 2048;
   l.bytes = l.blocks * l.block_bytes;

@@ -396,6 +396,8 @@ Plan make_plan6(int64_t M, int64_t N, int64_t min_rows) {
 // followed by the partial accumulators.
 constexpr int64_t kSplitCounterBytes = 4096;
 constexpr int64_t kSplitMinSteps8 = 32, kSplitMinSteps6 = 32;  // at least 1024 (int8) / 2048 (6-bit) elements of K per workgroup
+// integer k-steps of an operand buffer (fp6_layout, tile8_layout)
+int64_t tile_steps(int64_t K, int bits) { return bits == 4 ? (K + 127) / 128 * 2 : (K + 63) / 64 * 2; }
 struct SplitPlan {
   int splits, per;
   int64_t bytes;
@@ -492,7 +494,7 @@ struct DirectPlan {
 DirectPlan plan_direct(int64_t M, int64_t N, int64_t K, int bits, int64_t workspace_bytes) {
   const DirectPlan ring{0, 1, 0};
   if (make_plan6(M, N, 1).kind != Plan::kMid) return ring;
-  const int64_t steps = bits == 4 ? K / 64 : K / 32, unit = bits == 4 ? 3072 : 2048, cus = num_cus();
+  const int64_t steps = tile_steps(K, bits), unit = bits == 4 ? 3072 : 2048, cus = num_cus();
   const int64_t stream = N * steps * unit / 64 * 10 / 55000;
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto busiest = [&](int64_t groups, int64_t per, int64_t step_bytes) {
@@ -522,7 +524,7 @@ int launch_direct(const Args &p, int splits, void *workspace, hipStream_t st) {
   int tiles_m, tiles_n;
   const int grid = grid_of<D>(p.M, p.N, tiles_m, tiles_n);
   if (splits > 1) {
-    const int steps = p.K / (D::SIX ? 64 : 32);
+    const int steps = static_cast<int>(tile_steps(p.K, D::SIX ? 4 : 8));
     SplitK sk{splits, (steps + splits - 1) / splits, grid, static_cast<uint32_t *>(workspace),
               reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace) + kSplitCounterBytes)};
     auto kern = gemm_direct_splitk_kernel<D, BF16, Args>;
@@ -555,7 +557,7 @@ int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t wor
   const Plan plan = make_plan6(p.M, p.N, 1);
   if (plan.kind == Plan::kSplit && plan.n_wide >= p.N) return launch_fused6<CfgL8, BF16>(p, st);
   if (plan.kind != Plan::kSplit) {
-    const SplitPlan sp = plan_splitk(p.M, p.N, p.K / 64, kSplitMinSteps6, 1, 3);
+    const SplitPlan sp = plan_splitk(p.M, p.N, tile_steps(p.K, 4), kSplitMinSteps6, 1, 3);
     if (sp.splits > 1 && workspace && workspace_bytes >= sp.bytes) return launch_fused6_splitk<BF16>(p, sp, workspace, st);
     // too few 128x128 tiles for the CUs and no K split (it takes three workgroups per tile to pay): 128x64 tiles
     const int64_t mid_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128);
@@ -608,7 +610,7 @@ int run_fused8t(const Fused8Args &p, hipStream_t st, void *workspace, int64_t wo
   if (const int rc = run_direct<false, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
   const Plan plan = make_plan6(p.M, p.N, 1);  // any row count: with few rows this path competes with the weight-streaming kernel
   if (plan.kind != Plan::kSplit) {
-    const SplitPlan sp = plan_splitk(p.M, p.N, p.K / 32, kSplitMinSteps8, 1, 2);
+    const SplitPlan sp = plan_splitk(p.M, p.N, tile_steps(p.K, 8), kSplitMinSteps8, 1, 2);
     if (sp.splits > 1 && workspace && workspace_bytes >= sp.bytes) return launch_fused8t_splitk<BF16>(p, sp, workspace, st);
     return launch_fused8t<CfgM, BF16>(p, st);
   }
@@ -774,11 +776,11 @@ extern "C" int quik_mixed_linear_fwd(const void *qx, const void *qw, const void 
 
 extern "C" int64_t quik_splitk_workspace_bytes(int64_t M, int64_t N, int64_t K, int bits) {
   if (M <= 0 || N <= 0 || K <= 0 || (bits != 4 && bits != 8)) return 0;
-  if (bits == 4 ? K % 128 != 0 : K % 64 != 0) return 0;
+  if (bits == 4 ? K % kLayerK4 != 0 : K % kLayerK8 != 0) return 0;
   // whichever kernel a call with that much workspace takes; a shape the ring kernels would split keeps its workspace
   // even where the register-streaming kernel then does without
-  const int64_t ring = (bits == 4 ? plan_splitk(M, N, K / 64, kSplitMinSteps6, 1, 3)
-                                  : plan_splitk(M, N, K / 32, kSplitMinSteps8, 1, 2)).bytes;
+  const int64_t ring = (bits == 4 ? plan_splitk(M, N, tile_steps(K, 4), kSplitMinSteps6, 1, 3)
+                                  : plan_splitk(M, N, tile_steps(K, 8), kSplitMinSteps8, 1, 2)).bytes;
   const int64_t direct = plan_direct(M, N, K, bits, kSplitCounterBytes + int64_t(kMaxCUs) * 128 * 128 * 4).bytes;
   return ring > direct ? ring : direct;
 }
@@ -789,15 +791,14 @@ extern "C" int quik_mixed_linear_fwd_fp6(const void *x6, const void *w6, const v
   return quik_mixed_linear_fwd_fp6_ws(x6, w6, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, nullptr, 0, stream);
 }
 
-extern "C" int quik_mixed_linear_fwd_fp6_ws(const void *x6, const void *w6, const void *meta, const void *s_col,
-                                            const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
-                                            int64_t K, int64_t F, void *out, void *workspace,
-                                            int64_t workspace_bytes, void *stream) {
+int quik::mixed_linear_fp6(const void *x6, const void *w6, const void *meta, const void *s_col, const void *w_reduced,
+                           const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
+                           void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (M < 0 || N < 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
   if (M == 0 || N == 0) return QUIK_OK;
   if (!x6 || !w6 || !meta || !s_col || !out) return QUIK_ERR_NULL;  // w_reduced == NULL: symmetric activations
-  if (K % 128 != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
+  if (K % k_multiple != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
   auto misaligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 256 != 0; };
   if (misaligned(x6) || misaligned(w6)) return QUIK_ERR_ALIGN;
   if (M > (1 << 30) || N > (1 << 30) || K > 74496) return QUIK_ERR_RANGE;  // 225 K < 2^24: the fp32 sums stay exact
@@ -822,21 +823,27 @@ extern "C" int quik_mixed_linear_fwd_fp6_ws(const void *x6, const void *w6, cons
                            : run_fused6<true>(p, st, workspace, workspace_bytes);
 }
 
+extern "C" int quik_mixed_linear_fwd_fp6_ws(const void *x6, const void *w6, const void *meta, const void *s_col,
+                                            const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
+                                            int64_t K, int64_t F, void *out, void *workspace,
+                                            int64_t workspace_bytes, void *stream) {
+  return mixed_linear_fp6(x6, w6, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, workspace, workspace_bytes, stream, 128);
+}
+
 extern "C" int quik_mixed_linear_fwd_tile8(const void *x8, const void *w8, const void *meta, const void *s_col,
                                            const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
                                            int64_t K, int64_t F, void *out, void *stream) {
   return quik_mixed_linear_fwd_tile8_ws(x8, w8, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, nullptr, 0, stream);
 }
 
-extern "C" int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *meta, const void *s_col,
-                                              const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
-                                              int64_t K, int64_t F, void *out, void *workspace,
-                                              int64_t workspace_bytes, void *stream) {
+int quik::mixed_linear_tile8(const void *x8, const void *w8, const void *meta, const void *s_col, const void *w_reduced,
+                             const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
+                             void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (M < 0 || N < 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
   if (M == 0 || N == 0) return QUIK_OK;
   if (!x8 || !w8 || !meta || !s_col || !out) return QUIK_ERR_NULL;  // w_reduced == NULL: symmetric activations
-  if (K % 64 != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
+  if (K % k_multiple != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
   auto misaligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 256 != 0; };
   if (misaligned(x8) || misaligned(w8)) return QUIK_ERR_ALIGN;
   if (M > (1 << 30) || N > (1 << 30) || K > (1 << 24)) return QUIK_ERR_RANGE;
@@ -859,6 +866,13 @@ extern "C" int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, co
   if (workspace && reinterpret_cast<uintptr_t>(workspace) % 16 != 0) return QUIK_ERR_ALIGN;
   return dtype == QUIK_F16 ? run_fused8t<false>(p, st, workspace, workspace_bytes)
                            : run_fused8t<true>(p, st, workspace, workspace_bytes);
+}
+
+extern "C" int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *meta, const void *s_col,
+                                              const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
+                                              int64_t K, int64_t F, void *out, void *workspace,
+                                              int64_t workspace_bytes, void *stream) {
+  return mixed_linear_tile8(x8, w8, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, workspace, workspace_bytes, stream, 64);
 }
 
 // ---- the entry point that allocates nothing ------------------------------------------------------------------

@@ -31,8 +31,8 @@ bool layer_valid(const quik_layer *l) {
 bool use_tiled(const quik_layer *l, int64_t rows) {
   if (!l->tiled_weight || rows < l->tiled_min_rows || !l->colmap_streams) return false;
   if (l->symmetric && l->dtype != QUIK_F16) return false;
-  return (l->bits == 4 ? quik_fp6_operand_bytes(rows, l->num_int, l->num_fp)
-                       : quik_tile8_operand_bytes(rows, l->num_int, l->num_fp)) > 0;
+  return (l->bits == 4 ? fp6_operand_bytes(rows, l->num_int, l->num_fp, kLayerK4)
+                       : tile8_operand_bytes(rows, l->num_int, l->num_fp, kLayerK8)) > 0;
 }
 
 LayerPlan plan_layer(const quik_layer *l, int64_t rows) {
@@ -40,8 +40,8 @@ LayerPlan plan_layer(const quik_layer *l, int64_t rows) {
   p.tiled = use_tiled(l, rows);
   const int64_t meta_bytes = align256((l->symmetric ? 1 : 2) * rows * 2);
   if (p.tiled) {
-    const int64_t qb = l->bits == 4 ? quik_fp6_operand_bytes(rows, l->num_int, l->num_fp)
-                                    : quik_tile8_operand_bytes(rows, l->num_int, l->num_fp);
+    const int64_t qb = l->bits == 4 ? fp6_operand_bytes(rows, l->num_int, l->num_fp, kLayerK4)
+                                    : tile8_operand_bytes(rows, l->num_int, l->num_fp, kLayerK8);
     p.off_q = 0;
     p.off_meta = align256(qb);
     p.off_fp = p.off_meta + meta_bytes;
@@ -102,14 +102,14 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
   }
   if (l.symmetric) {
     if (l.dtype != QUIK_F16 || !l.colmap_streams) return QUIK_ERR_DTYPE;  // the caller's op sequence serves these
-    if (int rc = quik_sym_quantize_mapped(x, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, l.sym_divisor,
-                                          p.tiled ? 1 : 0, q, meta, fp_x, stream))
+    if (int rc = sym_quantize_mapped(x, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, l.sym_divisor,
+                                     p.tiled ? 1 : 0, q, meta, fp_x, stream, l.bits == 4 ? kLayerK4 : kLayerK8))
       return rc;
   } else if (p.tiled) {
-    if (int rc = l.bits == 4 ? quik_asym_quantize_fp6(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, q,
-                                                      meta, stream)
-                             : quik_asym_quantize_tile8(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp,
-                                                        q, meta, stream))
+    if (int rc = l.bits == 4 ? asym_quantize_fp6(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, q,
+                                                      meta, stream, kLayerK4)
+                             : asym_quantize_tile8(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp,
+                                                        q, meta, stream, kLayerK8))
       return rc;
   } else {
     if (int rc = quik_asym_quantize(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, q, meta, fp_x,
@@ -124,12 +124,12 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
     }
   }
   if (p.tiled) {
-    return l.bits == 4 ? quik_mixed_linear_fwd_fp6_ws(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
+    return l.bits == 4 ? mixed_linear_fp6(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
                                                       rows, l.out_features, l.num_int, l.num_fp, out, splitk_workspace,
-                                                      splitk_bytes, stream)
-                       : quik_mixed_linear_fwd_tile8_ws(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
+                                                      splitk_bytes, stream, kLayerK4)
+                       : mixed_linear_tile8(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
                                                         rows, l.out_features, l.num_int, l.num_fp, out,
-                                                        splitk_workspace, splitk_bytes, stream);
+                                                        splitk_workspace, splitk_bytes, stream, kLayerK8);
   }
   return quik_mixed_linear_fwd(q, l.int_weight, meta, l.weights_scales, w_red, fp_x, l.fp_weight, l.bias, l.dtype, rows,
                                l.out_features, l.num_int, l.num_fp, l.bits, out, stream);

@@ -370,7 +370,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t *__restrict__ x, int6
                                             float sym_divisor = 1.0f) {
   // vec_out: 0 byte-wise output, 1 16-byte output,
   // 3 (8 bits only): dst is an int8 operand buffer in tile order for gemm_tile8.h, which also takes the outlier
-  // values (fp_x is not written); needs num_int % 64 == 0 and num_fp % 32 == 0
+  // values (fp_x is not written); needs num_int % 16 == 0 and num_fp % 32 == 0
   // (the 6-bit operand buffers of gemm_fp6.h are written by quantize_fp6_wave_kernel below)
   const Tile8Layout l8 = tile8_layout(rows, num_int, num_fp);
   const bool to8 = BITS == 8 && vec_out == 3;
@@ -832,6 +832,7 @@ __global__ __launch_bounds__(kRingThreads) void quantize_tile8_ring_kernel(
   // units (colmap.h): consecutive columns are 16 consecutive staged bytes from the unit's first column on ("plain");
   // the others are gathered byte by byte, one unit per lane of the first `ngather` lanes
   const int nu_int = static_cast<int>(num_int >> 4), nu = nu_int + static_cast<int>(num_fp >> 3);
+  const int unit_pad = static_cast<int>(2 * l8.steps) - nu_int;
   uint32_t ubase[NU], ushift[NU];  // 16-byte-aligned offset into the staging area, byte shift; 0xFFFFFFFF: not plain
   uint32_t ucol[NU];
 #pragma unroll
@@ -1002,7 +1003,8 @@ __global__ __launch_bounds__(kRingThreads) void quantize_tile8_ring_kernel(
         c.y = __builtin_amdgcn_alignbyte(w[2], w[1], ushift[j]);
         c.z = __builtin_amdgcn_alignbyte(w[3], w[2], ushift[j]);
         c.w = __builtin_amdgcn_alignbyte(w[4], w[3], ushift[j]);
-        *unit_at(tid + j * T) = c;
+        const int u = tid + j * T;  // outlier units start behind the filled-up integer steps
+        *unit_at(u < nu_int ? u : u + unit_pad) = c;
       }
     }
     if (has_gather) {
@@ -1780,11 +1782,11 @@ extern "C" int quik_colmap_streaming(const void *colmap, int64_t cols, int64_t n
   return (flags & kColmapStreams) ? 1 : 0;
 }
 
-extern "C" int quik_asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
-                                      int64_t num_int, int64_t num_fp, void *out6, void *meta, void *stream) {
+int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
+                            int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (rows < 0 || cols <= 0 || num_int <= 0 || num_fp < 0 || num_int + num_fp != cols) return QUIK_ERR_SHAPE;
-  if (num_int % 128 != 0 || num_fp % 32 != 0 || cols > kStreamMaxCols) return QUIK_ERR_ALIGN;
+  if (num_int % k_multiple != 0 || num_fp % 32 != 0 || cols > kStreamMaxCols) return QUIK_ERR_ALIGN;
   if (rows == 0) return QUIK_OK;
   if (!x || !colmap || !out6 || !meta) return QUIK_ERR_NULL;
   if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(out6) % 256 != 0) return QUIK_ERR_ALIGN;
@@ -1796,11 +1798,16 @@ extern "C" int quik_asym_quantize_fp6(const void *x, int dtype, int64_t rows, in
                            : launch_fp6_wave<true, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st);
 }
 
-extern "C" int quik_asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
-                                        int64_t num_int, int64_t num_fp, void *out8, void *meta, void *stream) {
+extern "C" int quik_asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
+                                      int64_t num_int, int64_t num_fp, void *out6, void *meta, void *stream) {
+  return quik::asym_quantize_fp6(x, dtype, rows, cols, colmap, num_int, num_fp, out6, meta, stream, 128);
+}
+
+int quik::asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
+                              int64_t num_fp, void *out8, void *meta, void *stream, int64_t k_multiple) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (rows < 0 || cols <= 0 || num_int <= 0 || num_fp < 0 || num_int + num_fp != cols) return QUIK_ERR_SHAPE;
-  if (num_int % 64 != 0 || num_fp % 32 != 0 || cols > kStreamMaxCols) return QUIK_ERR_ALIGN;
+  if (num_int % k_multiple != 0 || num_fp % 32 != 0 || cols > kStreamMaxCols) return QUIK_ERR_ALIGN;
   if (rows == 0) return QUIK_OK;
   if (!x || !colmap || !out8 || !meta) return QUIK_ERR_NULL;
   if (reinterpret_cast<uintptr_t>(x) % 16 != 0 || reinterpret_cast<uintptr_t>(out8) % 256 != 0) return QUIK_ERR_ALIGN;
@@ -1816,13 +1823,18 @@ extern "C" int quik_asym_quantize_tile8(const void *x, int dtype, int64_t rows, 
                                                            st, true, words[1], words[3]);
 }
 
-extern "C" int quik_sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
-                                        int64_t num_fp, int bits, float divisor, int tiled, void *dst, void *scale,
-                                        void *fp_x, void *stream) {
+extern "C" int quik_asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
+                                        int64_t num_int, int64_t num_fp, void *out8, void *meta, void *stream) {
+  return quik::asym_quantize_tile8(x, dtype, rows, cols, colmap, num_int, num_fp, out8, meta, stream, 64);
+}
+
+int quik::sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp,
+                              int bits, float divisor, int tiled, void *dst, void *scale, void *fp_x, void *stream,
+                              int64_t k_multiple) {
   if (bits != 4 && bits != 8) return QUIK_ERR_BITS;
   if (rows < 0 || cols <= 0 || num_int <= 0 || num_fp < 0 || num_int + num_fp != cols) return QUIK_ERR_SHAPE;
   if (cols % 8 != 0 || cols > kStreamMaxCols || !(divisor > 0.0f)) return QUIK_ERR_SHAPE;
-  if (tiled && (num_int % (bits == 4 ? 128 : 64) != 0 || num_fp % 32 != 0)) return QUIK_ERR_ALIGN;
+  if (tiled && (num_int % k_multiple != 0 || num_fp % 32 != 0)) return QUIK_ERR_ALIGN;
   if (bits == 4 && num_int % 2 != 0) return QUIK_ERR_ALIGN;
   if (rows == 0) return QUIK_OK;
   if (!x || !colmap || !dst || !scale || (!tiled && num_fp > 0 && !fp_x)) return QUIK_ERR_NULL;
@@ -1837,6 +1849,13 @@ extern "C" int quik_sym_quantize_mapped(const void *x, int64_t rows, int64_t col
   if (bits == 4 && tiled) return launch_fp6_wave<false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
   return bits == 4 ? launch_sym_stream<4>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor)
                    : launch_sym_stream<8>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor);
+}
+
+extern "C" int quik_sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
+                                        int64_t num_fp, int bits, float divisor, int tiled, void *dst, void *scale,
+                                        void *fp_x, void *stream) {
+  return quik::sym_quantize_mapped(x, rows, cols, colmap, num_int, num_fp, bits, divisor, tiled, dst, scale, fp_x, stream,
+                                   bits == 4 ? 128 : 64);
 }
 
 extern "C" int quik_asym_find_meta(const void *x, int64_t rows, int64_t cols, int bits, void *meta, void *stream) {

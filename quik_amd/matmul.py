@@ -216,6 +216,27 @@ def pack_weight_tile8(int_weight: torch.Tensor, fp_weight: torch.Tensor) -> torc
     return out
 
 
+def pack_weight_layer(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor, bits: int) -> torch.Tensor:
+    """Tile-ordered weight copy for the one-call layer forward, any number of integer columns that fills whole
+    fragments (4 bits: a multiple of 32, 8 bits: of 16); the last k-steps are filled up with zeros."""
+    L.check_cuda_contiguous("pack_weight_layer", int_weight=int_weight, fp_weight=fp_weight, colmap=colmap)
+    N, K, F = int_weight.size(0), int_weight.size(1) * (2 if bits == 4 else 1), fp_weight.size(1)
+    if int_weight.dtype != (torch.uint8 if bits == 4 else torch.int8) or fp_weight.size(0) != N or \
+            fp_weight.dtype not in (torch.float16, torch.bfloat16):
+        raise RuntimeError("pack_weight_layer: int_weight and fp_weight do not match")
+    lib = L.load()
+    if colmap.dtype != torch.uint8 or colmap.numel() != lib.quik_colmap_bytes(K + F, K, F):
+        raise RuntimeError(f"pack_weight_layer: the column map was not built for {K} integer and {F} outlier columns")
+    nbytes = lib.quik_layer_weight_bytes(N, K, F, bits)
+    if nbytes == 0:
+        raise RuntimeError("pack_weight_layer: shape not supported by the tile-ordered operand format")
+    with L.device_guard(int_weight.device):
+        out = torch.empty((nbytes,), dtype=torch.uint8, device=int_weight.device)
+        L.check(lib.quik_layer_pack_weight(L.ptr(int_weight), L.ptr(fp_weight) if F else None, N, K, F, bits,
+                                           L.ptr(colmap), L.ptr(out), L.stream()), "pack_weight_layer")
+    return out
+
+
 def mixed_linear_tile8(x8, w8, meta, weights_scales, reduced_w, bias, M, N, K, F, out_dtype):
     """mixed_linear (asymmetric, 8 bits) on tile-ordered operand buffers (asymmetric.quantize_mapped_tile8,
     pack_weight_tile8): same result bit for bit, every operand cache line fetched once per tile."""

@@ -221,10 +221,11 @@ class MixedQLinear(torch.nn.Module):
     Asymmetric calls with at least `six_bit_min_rows` token rows (everything above decode size) read both
     operands in tile order (`tiled_path`; the quantize kernel writes the activation that way, the weights
     get a second, repacked copy on first use), so every operand cache line is fetched once per tile.
+    (Integer columns that do not fill whole k-steps, multiples of 32 / 16 instead of 128 / 64, take it through the one-call
+    forward, whose operand buffers are filled up with zeros.)
     W4A4: the int4 products run on the 6-bit (E2M3) matrix-core instructions, which have twice the int8 rate:
-    levels code + 8 are exact E2M3 numbers and the integer accumulator is recovered exactly (needs
-    int_features % 128 == 0; 0.75 bytes per weight).  W8A8: int8 MFMA as before (int_features % 64 == 0;
-    1 byte per weight).  Both need fp_features % 32 == 0 and ascending int_indices and give the output bits
+    levels code + 8 are exact E2M3 numbers and the integer accumulator is recovered exactly (0.75
+    bytes per weight).  W8A8: int8 MFMA as before (1 byte per weight).  Both need fp_features % 32 == 0 and ascending int_indices and give the output bits
     of the row-major kernels; `six_bit_path = False` turns them off."""
 
     # Profiling hook: a torch.cuda.Event (created, i.e. recorded once before) stored here is recorded between the
@@ -317,13 +318,25 @@ class MixedQLinear(torch.nn.Module):
             return False
         if self.symmetric and self.dtype != torch.float16:      # symmetric activations are fp16 (as in the reference)
             return False
-        k_multiple = 128 if self.bits == 4 else 64
         min_rows = self.six_bit_min_rows if self.bits == 4 else self.tile8_min_rows
-        if rows < min_rows or self.int_features_num % k_multiple != 0 or self.fp_features_num % 32 != 0:
+        if rows < min_rows or self.int_features_num % (32 if self.bits == 4 else 16) != 0 or \
+                self.fp_features_num % 32 != 0:
             return False
         if self.bits == 4 and self.int_features_num > 74496:   # the 6-bit path's fp32 sums are exact up to here
             return False
         return self._streams_flag()
+
+    def _whole_steps(self):
+        """True if the integer columns fill whole pairs of k-steps: then the stand-alone operations of the tile-ordered
+        path take the shape too; otherwise only the one-call forward does (its operand buffers are filled up)."""
+        return self.int_features_num % (128 if self.bits == 4 else 64) == 0
+
+    def _pack_tiled(self, fp_w):
+        if not self._whole_steps():
+            return matmul.pack_weight_layer(self.int_weight, fp_w, self._column_map(), self.bits)
+        if self.bits == 4:    # in the column map's in-place order, as the activation is quantized
+            return matmul.pack_weight_fp6(self.int_weight, fp_w, self._column_map())
+        return matmul.pack_weight_tile8(self.int_weight, fp_w)
 
     def _weight6(self):
         if self._row_major_released:
@@ -332,16 +345,11 @@ class MixedQLinear(torch.nn.Module):
             torch.empty((self.out_features, 0), dtype=self.dtype, device=self.int_weight.device)
         if self.transient_tiled_copy:    # a fresh buffer per call, never kept
             self._w6 = self._w6_key = None
-            if self.bits == 4:
-                return matmul.pack_weight_fp6(self.int_weight, fp_w, self._column_map())
-            return matmul.pack_weight_tile8(self.int_weight, fp_w)
+            return self._pack_tiled(fp_w)
         key = (self.int_weight.data_ptr(), self.int_weight._version, fp_w.data_ptr(), fp_w._version,
                self.int_weight.device, self._column_map().data_ptr())
         if self._w6 is None or self._w6_key != key:
-            if self.bits == 4:    # in the column map's in-place order, as the activation is quantized
-                self._w6 = matmul.pack_weight_fp6(self.int_weight, fp_w, self._column_map())
-            else:
-                self._w6 = matmul.pack_weight_tile8(self.int_weight, fp_w)
+            self._w6 = self._pack_tiled(fp_w)
             self._w6_key = key
         return self._w6
 
@@ -377,7 +385,7 @@ class MixedQLinear(torch.nn.Module):
         one row, takes the tile-ordered path (same output bits above 32 rows; up to 32 rows equal within rounding
         of the fp32 sums, and slower than the weight-streaming kernel, which reads the packed nibbles).  The
         module can no longer be saved in the reference's checkpoint format or moved to another device."""
-        if not self._six_bit_ok(max(self.six_bit_min_rows, self.tile8_min_rows)):
+        if not (self._six_bit_ok(max(self.six_bit_min_rows, self.tile8_min_rows)) and self._whole_steps()):
             raise RuntimeError("this layer does not take the tile-ordered path (shape, dtype or column map)")
         w6 = self._weight6()
         self._row_major_released = True
@@ -539,7 +547,7 @@ class MixedQLinear(torch.nn.Module):
         shared_input = self.shared_input if self.shared_input is not None else SharedQuantizedInput(1)
         with device_guard(x.device):
             if x2.data_ptr() % 16 == 0 and (not self.symmetric or x2.dtype == torch.float16) \
-                    and self._six_bit_ok(x2.shape[0]):
+                    and self._six_bit_ok(x2.shape[0]) and self._whole_steps():
                 quantize6 = asymmetric.quantize_mapped_fp6 if self.bits == 4 else asymmetric.quantize_mapped_tile8
                 linear6 = matmul.mixed_linear_fp6 if self.bits == 4 else matmul.mixed_linear_tile8
                 if shared_input.x6 is None:
