@@ -12,6 +12,7 @@
 
 #include <ATen/Tensor.h>
 #include <ATen/hip/EmptyTensor.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 #include <c10/hip/HIPCachingAllocator.h>
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
@@ -139,11 +140,17 @@ at::Tensor new_empty(at::IntArrayRef size, at::ScalarType type, c10::DeviceIndex
   return at::Tensor(at::detail::empty_cuda(size, type, at::Device(at::kCUDA, dev), std::nullopt));
 }
 
+// Dispatch modes (tracing, fake tensors, counters) see the operations of the Python functions, and tensors of vmap, grad
+// and functionalization levels have no memory of their own: both stay with those functions.
+constexpr c10::DispatchKeySet kInterposedKeys({c10::DispatchKey::FuncTorchBatched, c10::DispatchKey::FuncTorchGradWrapper,
+                                               c10::DispatchKey::Functionalize, c10::DispatchKey::Python,
+                                               c10::DispatchKey::BatchedNestedTensor});
+
 // A plain contiguous tensor on the current GPU, or null.
 const at::Tensor *plain(PyObject *o, c10::DeviceIndex dev) {
-  if (!THPVariable_CheckExact(o)) return nullptr;
+  if (!THPVariable_CheckExact(o) || c10::impl::TorchDispatchModeTLS::any_modes_set()) return nullptr;
   const at::Tensor &t = THPVariable_Unpack(o);
-  if (!t.defined() || !t.is_cuda() || t.get_device() != dev || t.layout() != at::kStrided || !t.is_contiguous() ||
+  if (!t.defined() || t.key_set().has_any(kInterposedKeys) || !t.has_storage() || !t.is_cuda() || t.get_device() != dev || t.layout() != at::kStrided || !t.is_contiguous() ||
       t.is_conj() || t.is_neg())
     return nullptr;
   return &t;
@@ -226,8 +233,21 @@ PyObject *none_or_error() {
   Py_RETURN_NONE;
 }
 
+// C++ exceptions end here: out of memory goes back to the Python path, which raises torch's own error
+template <typename F>
+PyObject *guarded(F &&f) {
+  try {
+    return f();
+  } catch (const c10::OutOfMemoryError &) {
+    Py_RETURN_NONE;
+  } catch (const std::exception &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
+}
+
 // forward(plan, module, x) -> Tensor [.., N] or None
-PyObject *py_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *forward(PyObject *const *args, Py_ssize_t n) {
   if (n != 3) return PyErr_Format(PyExc_TypeError, "forward takes 3 arguments");
   const Plan *p = static_cast<const Plan *>(PyCapsule_GetPointer(args[0], kPlanName));
   if (!p) return nullptr;
@@ -241,8 +261,12 @@ PyObject *py_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
   return THPVariable_Wrap(std::move(out));
 }
 
+PyObject *py_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  return guarded([&] { return forward(args, n); });
+}
+
 // group_forward(group, index, module, x) -> member `index`'s columns [.., N_index] or None
-PyObject *py_group_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
+PyObject *group_forward(PyObject *const *args, Py_ssize_t n) {
   if (n != 4) return PyErr_Format(PyExc_TypeError, "group_forward takes 4 arguments");
   const Group *g = static_cast<const Group *>(PyCapsule_GetPointer(args[0], kGroupName));
   if (!g) return nullptr;
@@ -298,6 +322,10 @@ PyObject *py_group_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
   r.p = PyObject_CallMethodNoArgs(shared, s_finish);
   if (!r.p) return nullptr;
   return THPVariable_Wrap(std::move(view));
+}
+
+PyObject *py_group_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
+  return guarded([&] { return group_forward(args, n); });
 }
 
 // plan(module, names, row_desc, tiled_desc, tiled_from, device_index, is_bf16, device, splitk_fn, keep)
@@ -356,18 +384,6 @@ PyObject *py_group(PyObject *, PyObject *args) {
 // ---------------------------------------------------------------------------------------------- stand-alone operations
 const void *ptr(const at::Tensor &t) { return t.numel() ? data_of(t) : nullptr; }
 void *out_ptr(const at::Tensor &t) { return const_cast<void *>(t.numel() ? data_of(t) : nullptr); }
-
-template <typename F>
-PyObject *guarded(F &&f) {
-  try {
-    return f();
-  } catch (const c10::OutOfMemoryError &) {
-    Py_RETURN_NONE;
-  } catch (const std::exception &e) {
-    PyErr_SetString(PyExc_RuntimeError, e.what());
-    return nullptr;
-  }
-}
 
 PyObject *triple(at::Tensor a, at::Tensor b, at::Tensor c) {
   PyObject *t = PyTuple_New(3);

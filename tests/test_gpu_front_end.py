@@ -102,3 +102,29 @@ def test_a_planned_group_sees_every_change(rows):
     outs += [mods[1](x), mods[2](x)]
     assert all(_same(o, a(x)) for o, a in zip(outs, alone))
     assert shared.cur_group_elem == 0
+
+
+def test_interposed_inputs_stay_with_the_python_functions():
+    from torch.utils._python_dispatch import TorchDispatchMode
+    import quik
+    mod = _module(0, 256, 1024, 0, 4)
+    x = torch.randn(4, 1024, generator=torch.Generator().manual_seed(0)).half().to(DEV)
+    first = mod(x)
+    assert _planned(mod)
+    ii, fi = mod.int_indices, mod.fp_indices
+    for call in (mod, lambda t: quik.asymmetric.quantize(t, ii, fi, 4)[0]):
+        # a level's tensor has no memory to hand to a kernel: the error of its data pointer, not an abort
+        with pytest.raises(RuntimeError):
+            torch.vmap(call)(x[None])
+        with pytest.raises(RuntimeError):
+            torch.func.jvp(call, (x,), (x,))
+
+    class Seen(TorchDispatchMode):
+        ops = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.ops.append(str(func))
+            return func(*args, **(kwargs or {}))
+    with Seen():
+        out = mod(x)
+    assert _same(out, first) and any("empty" in op for op in Seen.ops)
