@@ -11,6 +11,7 @@
 #define GEMV_MAX_ROWS 2
 #endif
 #include "gemm_direct.h"
+#include "gemm_rows.h"
 #include "gemm_tile8.h"
 #include "gemm_kernels.h"
 
@@ -24,6 +25,7 @@ using CfgH = Cfg<256, 128, 2, 2, 2>;   // half-width tile that evens out the las
 using CfgM = Cfg<128, 128, 2, 2, 2>;   // mid-size problems, two workgroups per CU
 using CfgN = Cfg<128, 64, 2, 2, 2>;    // few tiles: narrower ones put more CUs to work, three workgroups per CU
 using CfgN6 = Cfg<128, 64, 2, 2, 2>;   // 6-bit path, 86 .. ~150 tiles of 128x128 and no K split: twice as many workgroups
+using CfgN8 = Cfg<128, 64, 2, 2, 2, 8>; // the same, one workgroup per CU with eight stages of copies
 using CfgL8 = Cfg<256, 256, 2, 4, 2>;  // 6-bit path, launches of 256x256 tiles only: two waves per SIMD (1-5 % faster than CfgL)
 using CfgLp = Cfg<256, 256, 2, 2, 0>;  // plain fallbacks
 using CfgMp = Cfg<128, 128, 2, 2, 0>;
@@ -320,10 +322,58 @@ int check_gemm_args(const void *A, const void *B, const void *C, int64_t M, int6
   return QUIK_OK;
 }
 
+// Which row-streaming tile (gemm_rows.h) serves a product, as its number of 32-row blocks; 0: the ring kernels.
+//   one round of 64x64 tiles: always (256 x 4096 x 4096 13.7 -> 8.6 us int4, 18.2 -> 9.9 int8; 512 x 2048 x 11008
+//   30.1 -> 15.8 and 42.1 -> 22.9);
+//   two rounds, few rows and long K, where the weights come from memory and the ring kernels wait for them: 64x64 tiles
+//   (256 x 8192 x 7936 int4 24.4 -> 21.6, 64 x 28672 x 7936 int4 41.9 -> 31.4, int8 61.4 -> 51.5), or for int8 one round of
+//   128x64 tiles (128 x 13824 x 4864 30.7 -> 22.6, 256 x 8192 x 7936 46.6 -> 32.3; int4 is bound by its unpacking there:
+//   23.1).  Shorter K: 128 x 13824 x 4864 int4 (2432 bytes) 16.5 against 16.2 .. 17.2; more rows: 1024 x 4096 x 3840 int4
+//   21.5 against 26.7, 512 x 4096 x 3968 int8 16.2 against 17.4.
+int rows_blocks(int64_t M, int64_t N, int64_t kbytes, int mode) {
+  if (M <= 32 || kbytes % 64 != 0) return 0;
+  const int64_t tiles_n = (N + 63) / 64, tiles = (M + 63) / 64 * tiles_n;
+  if (tiles <= num_cus()) return 2;
+  if (M > 256 || kbytes < 3072) return 0;
+  if (mode == kInt8 && M > 64 && (M + 127) / 128 * tiles_n <= num_cus()) return 4;
+  return tiles <= 2 * num_cus() ? 2 : 0;
+}
+// 128x64 tiles on the ring kernels: int8 with one tile per CU takes the ring of eight stages, which covers the memory's
+// latency (512 x 4096 x 3968 19.4 -> 16.5 us, 2048 x 1024 x 7936 33.9 -> 28.6); int4 steps are bound by their unpacking
+// (14.6 against 14.2), and a second workgroup per CU is worth more than the depth (int8 1024 x 4096 x 3840 27.7 / 29.8).
+bool deep_ring(int64_t M, int64_t N, int mode) {
+  return mode == kInt8 && (M + 127) / 128 * ((N + 63) / 64) <= num_cus();
+}
+
+template <class R, int MODE>
+int launch_i32_rows(const I32Args &a, hipStream_t st) {
+  int tiles_m, tiles_n;
+  const int grid = grid_of<R>(a.M, a.N, tiles_m, tiles_n);
+  auto kern = gemm_i32_rows_kernel<R, MODE>;
+  if (int rc = prepare(kern, R::SMEM)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(R::kThreads), R::SMEM, st, a, tiles_m, tiles_n);
+  return check_launch();
+}
+template <class R, int MODE, bool ASYM>
+int launch_chain_rows(const I32Args &a, const ChainArgs &e, hipStream_t st) {
+  int tiles_m, tiles_n;
+  const int grid = grid_of<R>(a.M, a.N, tiles_m, tiles_n);
+  auto kern = gemm_chain_rows_kernel<R, MODE, ASYM>;
+  if (int rc = prepare(kern, R::SMEM)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(R::kThreads), R::SMEM, st, a, e, tiles_m, tiles_n);
+  return check_launch();
+}
+
 template <int MODE>
 int run_i32(const uint8_t *X, const uint8_t *W, int32_t *C, int64_t M, int64_t N, int64_t kbytes, hipStream_t st) {
   I32Args a{X, W, C, static_cast<int>(M), static_cast<int>(N), static_cast<int>(N), static_cast<int>(kbytes)};
   const Plan plan = make_plan(M, N, kbytes % 64 == 0);
+  switch (rows_blocks(M, N, kbytes, MODE)) {
+    case 2: return launch_i32_rows<RowsCfg<2>, MODE>(a, st);
+    case 4:
+      if constexpr (MODE == kInt8) return launch_i32_rows<RowsCfg<4>, MODE>(a, st);
+    default: break;
+  }
   switch (plan.kind) {
     case Plan::kSmall: {
       FusedArgs p{};
@@ -335,7 +385,11 @@ int run_i32(const uint8_t *X, const uint8_t *W, int32_t *C, int64_t M, int64_t N
       return launch_decode<MODE, false, false>(p, C, a.ldc, st);
     }
     case Plan::kMid: return launch_i32<CfgM, MODE>(a, st);
-    case Plan::kNarrow: return launch_i32<CfgN, MODE>(a, st);
+    case Plan::kNarrow:
+      if constexpr (MODE == kInt8) {
+        if (deep_ring(M, N, MODE)) return launch_i32<CfgN8, MODE>(a, st);
+      }
+      return launch_i32<CfgN, MODE>(a, st);
     case Plan::kMidPlain: return launch_i32<CfgMp, MODE>(a, st);
     case Plan::kLargePlain: return launch_i32<CfgLp, MODE>(a, st);
     default: break;
@@ -358,16 +412,54 @@ int launch_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
   return check_launch();
 }
 
+template <class CW, class CT, int MODE, bool ASYM>
+int launch_chain_split(const I32Args &a, const ChainArgs &e, int64_t n_wide, hipStream_t st) {
+  if (n_wide <= 0) return launch_chain<CT, MODE, ASYM>(a, e, st);
+  if (n_wide >= a.N) return launch_chain<CW, MODE, ASYM>(a, e, st);
+  I32Args wide = a, tail = a;
+  ChainArgs etail = e;
+  wide.N = static_cast<int>(n_wide);
+  tail.N = static_cast<int>(a.N - n_wide);
+  tail.W = a.W + n_wide * a.kbytes;
+  etail.s_col = e.s_col + n_wide;
+  etail.w_red = e.w_red ? e.w_red + n_wide : nullptr;
+  etail.y = e.y + n_wide;
+  etail.out = e.out + n_wide;
+  int tail_blocks;
+  const SplitGrid grid = split_grid<CW, CT>(a.M, wide.N, tail.N, tail_blocks);
+  auto kern = gemm_chain_split_kernel<CW, CT, MODE, ASYM>;
+  constexpr int smem = CW::SMEM > CT::SMEM ? CW::SMEM : CT::SMEM;
+  if (int rc = prepare(kern, smem)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid.wide_blocks + tail_blocks), dim3(CW::kThreads), smem, st, wide, tail, e, etail, grid);
+  return check_launch();
+}
+
 template <int MODE, bool ASYM>
 int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
-  switch (make_plan(a.M, a.N, a.kbytes % 64 == 0).kind) {
+  switch (rows_blocks(a.M, a.N, a.kbytes, MODE)) {
+    case 2: return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
+    case 4:
+      if constexpr (MODE == kInt8) return launch_chain_rows<RowsCfg<4>, MODE, ASYM>(a, e, st);
+    default: break;
+  }
+  const Plan plan = make_plan(a.M, a.N, a.kbytes % 64 == 0);
+  switch (plan.kind) {
     case Plan::kSmall: return kChainNotHandled;  // at most 32 rows: the weight-streaming kernel has no such epilogue
     case Plan::kMid: return launch_chain<CfgM, MODE, ASYM>(a, e, st);
-    case Plan::kNarrow: return launch_chain<CfgN, MODE, ASYM>(a, e, st);
+    case Plan::kNarrow:
+      if constexpr (MODE == kInt8) {
+        if (deep_ring(a.M, a.N, MODE)) return launch_chain<CfgN8, MODE, ASYM>(a, e, st);
+      }
+      return launch_chain<CfgN, MODE, ASYM>(a, e, st);
     case Plan::kMidPlain:
     case Plan::kLargePlain: return launch_chain<CfgMp, MODE, ASYM>(a, e, st);
-    default: return launch_chain<CfgL, MODE, ASYM>(a, e, st);
+    default: break;
   }
+  // The epilogue is exposed where one workgroup has the CU to itself: with few int4 k-steps two 128x128 tiles per CU hide
+  // more of it than the large tiles gain (777 x 5120 x 4864 33.5 against 36.6 us, 2048 x 11008 x 3840 92.7 / 97.1; at
+  // 2048 x 8192 x 7936 119 against 110).  (256x256 tiles alone: 65.5, 121 and 110 us.)
+  if (MODE == kInt4 && a.kbytes <= 2560) return launch_chain<CfgM, MODE, ASYM>(a, e, st);
+  return launch_chain_split<CfgL, CfgH, MODE, ASYM>(a, e, plan.n_wide, st);
 }
 
 // Tile plan of the 6-bit path (gemm_fp6.h).  Costs in percent of a 256x256 tile, measured at K = 7936, F = 256:

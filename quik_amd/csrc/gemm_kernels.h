@@ -38,7 +38,7 @@ typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
 
 enum Mode { kInt4 = 0, kInt8 = 1, kF16 = 2, kBF16 = 3 };
 
-template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int PIPE_ = 0>
+template <int BM_, int BN_, int WAVES_M_, int WAVES_N_, int PIPE_ = 0, int STAGES_ = 4>
 struct Cfg {
   static constexpr int BM = BM_, BN = BN_, WAVES_M = WAVES_M_, WAVES_N = WAVES_N_;
   static constexpr int BKB = 64;        // K bytes per row and stage
@@ -56,7 +56,7 @@ struct Cfg {
   static constexpr int B_LOADS = (BN * CHUNKS + kThreads - 1) / kThreads;
   // direct-to-LDS loop: unpadded, XOR-swizzled rows
   static constexpr int DMA_STAGE = (BM + BN) * BKB;
-  static constexpr int DMA_STAGES = 4;
+  static constexpr int DMA_STAGES = STAGES_;
   static constexpr int SMEM = PIPE == 2 ? DMA_STAGES * DMA_STAGE : 2 * STAGE;
   static_assert(WM % 32 == 0 && WN % 32 == 0, "tile shape");
 };
@@ -244,7 +244,7 @@ struct DmaPipe {
   __device__ __forceinline__ void init(uint8_t *smem_, const uint8_t *X0, int64_t ldx0, const uint8_t *W0,
                                        int64_t ldw0, int kbytes0, const uint8_t *X1, int64_t ldx1,
                                        const uint8_t *W1, int64_t ldw1, int kbytes1, int rows_x, int rows_w) {
-    static_assert(C::BM % (16 * C::WAVES) == 0 && C::BN % (16 * C::WAVES) == 0 && NS == 4, "DMA tile shape");
+    static_assert(C::BM % (16 * C::WAVES) == 0 && C::BN % (16 * C::WAVES) == 0 && NS >= 4 && (NS & (NS - 1)) == 0, "DMA tile shape");
     smem = smem_;
     lds0 = lds_address(smem_);
     const int lane = threadIdx.x & 63;
@@ -309,10 +309,8 @@ struct DmaPipe {
 
   // Fill the ring: afterwards stages 0 and 1 are visible and stage 2 is in flight.
   __device__ __forceinline__ void start() const {
-    issue(0);
-    issue(1);
-    issue(2);
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPerStage));
+    static_for<NS - 1>([&](auto s) { issue(s); });
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPerStage * (NS - 3)));
     __syncthreads();
   }
 
@@ -385,15 +383,15 @@ struct DmaPipe {
     using I1 = std::integral_constant<int, 1>;
     for (int kt = kt_begin; kt < kt_end; ++kt) {
       if constexpr (MODE == kInt4) {
-        substep(I0{}, I0{}, kt + 1, 0, kt + 3);
-        substep(I1{}, I1{}, kt + 1, 1, kt + 3);
+        substep(I0{}, I0{}, kt + 1, 0, kt + NS - 1);
+        substep(I1{}, I1{}, kt + 1, 1, kt + NS - 1);
       } else {
-        substep(I0{}, I0{}, kt, 1, kt + 3);
-        substep(I1{}, I1{}, kt + 1, 0, kt + 3);
+        substep(I0{}, I0{}, kt, 1, kt + NS - 1);
+        substep(I1{}, I1{}, kt + 1, 0, kt + NS - 1);
       }
       // Stage kt+2 has landed (stage kt+3 may stay in flight), then a bare barrier: the LDS reads
       // still outstanding target a slot nobody writes before the next barrier, so they need no wait.
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPerStage));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm(kPerStage * (NS - 3)));
       __builtin_amdgcn_s_barrier();
     }
   }
@@ -590,29 +588,16 @@ struct I32Args {
   int M, N, ldc, kbytes;
 };
 
+// Integer sums of a wave's blocks (tile at m0, n0) -> C, through the staging area `smem` of the workgroup.
 template <class C, int MODE>
-__device__ __forceinline__ void i32_tile(const I32Args &a, int tm, int tn, uint8_t *smem) {
-  const uint8_t *__restrict__ X = a.X;
-  const uint8_t *__restrict__ W = a.W;
-  int32_t *__restrict__ Cm = a.C;
-  const int M = a.M, N = a.N, ldc = a.ldc, kbytes = a.kbytes;
-  const int m0 = tm * C::BM, n0 = tn * C::BN;
-  v16i acc[C::MI][C::NI];
-#pragma unroll
-  for (int mi = 0; mi < C::MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
-  run_mainloop<C, MODE>(X + int64_t(m0) * kbytes, kbytes, M - m0, W + int64_t(n0) * kbytes, kbytes, N - n0, kbytes,
-                        smem, acc);
+__device__ __forceinline__ void i32_store(const I32Args &a, int m0, int n0, uint8_t *smem, const v16i (&acc)[C::MI][C::NI]) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   constexpr int kShift = MODE == kInt4 ? 8 : 0;
   using Store = BlockStore<C, int32_t>;
   static_assert(Store::kBytes * C::WAVES <= C::SMEM, "staging fits in the (now idle) operand buffers");
   uint8_t *stage = smem + wave * Store::kBytes;
-  const bool vec = (ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(Cm) & 15) == 0;
+  const bool vec = (a.ldc & 3) == 0 && (reinterpret_cast<uintptr_t>(a.C) & 15) == 0;
   const int nw = n0 + wn * C::WN;
 #pragma unroll
   for (int mi = 0; mi < C::MI; ++mi) {
@@ -625,9 +610,24 @@ __device__ __forceinline__ void i32_tile(const I32Args &a, int tm, int tn, uint8
                               acc[mi][ni][4 * g + 2] >> kShift, acc[mi][ni][4 * g + 3] >> kShift};
         Store::put(stage, lane, ni, g, v);
       }
-    if (mb < M && nw < N)
-      Store::flush(stage, lane, Cm + int64_t(mb) * ldc + nw, ldc, M - mb, N - nw, vec);
+    if (mb < a.M && nw < a.N)
+      Store::flush(stage, lane, a.C + int64_t(mb) * a.ldc + nw, a.ldc, a.M - mb, a.N - nw, vec);
   }
+}
+
+template <class C, int MODE>
+__device__ __forceinline__ void i32_tile(const I32Args &a, int tm, int tn, uint8_t *smem) {
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+  v16i acc[C::MI][C::NI];
+#pragma unroll
+  for (int mi = 0; mi < C::MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < C::NI; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
+  run_mainloop<C, MODE>(a.X + int64_t(m0) * a.kbytes, a.kbytes, a.M - m0, a.W + int64_t(n0) * a.kbytes, a.kbytes, a.N - n0,
+                        a.kbytes, smem, acc);
+  i32_store<C, MODE>(a, m0, n0, smem, acc);
 }
 
 template <class C, int MODE>
@@ -654,18 +654,9 @@ struct ChainArgs {
 };
 
 template <class C, int MODE, bool ASYM>
-__device__ __forceinline__ void chain_tile(const I32Args &a, const ChainArgs &e, int tm, int tn, uint8_t *smem) {
-  const int M = a.M, N = a.N, kbytes = a.kbytes;
-  const int m0 = tm * C::BM, n0 = tn * C::BN;
-  v16i acc[C::MI][C::NI];
-#pragma unroll
-  for (int mi = 0; mi < C::MI; ++mi)
-#pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
-  run_mainloop<C, MODE>(a.X + int64_t(m0) * kbytes, kbytes, M - m0, a.W + int64_t(n0) * kbytes, kbytes, N - n0, kbytes,
-                        smem, acc);
+__device__ __forceinline__ void chain_store(const I32Args &a, const ChainArgs &e, int m0, int n0, uint8_t *smem,
+                                            const v16i (&acc)[C::MI][C::NI]) {
+  const int M = a.M, N = a.N;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   constexpr int kShift = MODE == kInt4 ? 8 : 0;
@@ -716,6 +707,21 @@ __device__ __forceinline__ void chain_tile(const I32Args &a, const ChainArgs &e,
 }
 
 template <class C, int MODE, bool ASYM>
+__device__ __forceinline__ void chain_tile(const I32Args &a, const ChainArgs &e, int tm, int tn, uint8_t *smem) {
+  const int m0 = tm * C::BM, n0 = tn * C::BN;
+  v16i acc[C::MI][C::NI];
+#pragma unroll
+  for (int mi = 0; mi < C::MI; ++mi)
+#pragma unroll
+    for (int ni = 0; ni < C::NI; ++ni)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
+  run_mainloop<C, MODE>(a.X + int64_t(m0) * a.kbytes, a.kbytes, a.M - m0, a.W + int64_t(n0) * a.kbytes, a.kbytes, a.N - n0,
+                        a.kbytes, smem, acc);
+  chain_store<C, MODE, ASYM>(a, e, m0, n0, smem, acc);
+}
+
+template <class C, int MODE, bool ASYM>
 __global__ __launch_bounds__(C::kThreads) void gemm_chain_kernel(I32Args a, ChainArgs e, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
@@ -752,6 +758,19 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_i32_split_kernel(I32Args wi
   }
 }
 
+template <class CW, class CT, int MODE, bool ASYM>
+__global__ __launch_bounds__(CW::kThreads) void gemm_chain_split_kernel(I32Args wide, I32Args tail, ChainArgs e_wide,
+                                                                        ChainArgs e_tail, SplitGrid grid) {
+  static_assert(CW::kThreads == CT::kThreads && CW::BM == CT::BM, "one block size, one tile height");
+  extern __shared__ __align__(16) uint8_t smem[];
+  int tm, tn;
+  const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
+  if (kind == 1) {
+    chain_tile<CW, MODE, ASYM>(wide, e_wide, tm, tn, smem);
+  } else if (kind == 2) {
+    chain_tile<CT, MODE, ASYM>(tail, e_tail, tm, tn, smem);
+  }
+}
 
 struct FusedArgs {
   const uint8_t *qx, *qw;

@@ -1,0 +1,59 @@
+"""The row-streaming integer GEMMs (csrc/gemm_rows.h) and the other routes of the stand-alone products above decode size,
+at the edges of their tiles: half a stage, fewer stages than waves, unequal shares, one row or column more or less than a
+tile, odd widths (no 16-byte stores), two rounds of tiles, 128-row tiles, the deep ring, wide and half-wide tiles in one
+launch.  Integer sums equal a 64-bit product, the fused forms have the oracle's bits."""
+import numpy as np
+import pytest
+import torch
+
+from oracle import quik_oracle as qo
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+CASES = [  # M, N, bytes of K per row, bits (0: both)
+    (33, 1, 64, 0), (64, 8, 128, 0), (65, 63, 192, 0), (40, 65, 512, 0), (130, 136, 576, 0), (63, 4096, 640, 0),
+    (256, 4001, 1088, 0), (97, 200, 2496, 0),
+    (60, 64 * 260, 3072, 0), (255, 64 * 110 + 5, 3136, 4),     # 64x64 tiles, two rounds
+    (100, 64 * 200, 3136, 8), (255, 64 * 101 + 3, 3072, 8),    # 128x64 tiles
+    (300, 4500, 512, 0), (513, 2000, 832, 0),                  # ring kernels, 128x64 tiles
+    (777, 5128, 256, 0), (1000, 8203, 2624, 0),                # large tiles, both widths
+]
+
+
+def _operands(M, N, kbytes, bits, g):
+    if bits == 8:
+        a, b = (torch.randint(-128, 128, (n, kbytes), generator=g, device=DEV, dtype=torch.int16).to(torch.int8) for n in (M, N))
+        return a, b, a, b
+    a, b = (torch.randint(0, 256, (n, kbytes), generator=g, device=DEV, dtype=torch.int16).to(torch.uint8) for n in (M, N))
+
+    def codes(t):
+        t = t.to(torch.int16)
+        lo, hi = t & 15, t >> 4
+        both = torch.stack([lo, hi], -1).reshape(t.shape[0], -1)
+        return torch.where(both > 7, both - 16, both)
+    return a, b, codes(a), codes(b)
+
+
+@pytest.mark.parametrize("M,N,kbytes,bits", [(m, n, k, b) for m, n, k, w in CASES for b in ((4, 8) if w == 0 else (w,))])
+def test_products_and_fused_forms(M, N, kbytes, bits):
+    import quik
+    g = torch.Generator(device=DEV).manual_seed(M + N + kbytes)
+    a, b, ca, cb = _operands(M, N, kbytes, bits, g)
+    acc = (ca.double() @ cb.double().t().contiguous()).to(torch.int32)
+    mm = quik.matmul.int4Matmul if bits == 4 else quik.matmul.int8Matmul
+    assert torch.equal(mm(a, b), acc)
+
+    def half(*shape):
+        return (torch.rand(*shape, generator=g, device=DEV) * 0.1).half()
+    s_row, s_col, zero, w_red, y = half(M, 1), half(1, N), -half(M, 1), half(1, N), half(M, N)
+    host = [t.cpu().numpy() for t in (s_row, s_col, zero, w_red, y)]
+    with np.errstate(all="ignore"):
+        want = qo.asym_fused_dequantize(acc.cpu().numpy(), host[0], host[1], 8.0, host[2], host[3], host[4])
+        want_sym = qo.sym_dequantize(acc.cpu().numpy(), host[0], host[1], host[4], 32)
+    asym = quik.asymmetric.int4FusedDequantize if bits == 4 else quik.asymmetric.int8FusedDequantize
+    sym = quik.symmetric.int4FusedDequantize if bits == 4 else quik.symmetric.int8FusedDequantize
+    for got, w in ((asym(a, b, s_row, s_col, 8.0, zero, w_red, y), want), (sym(a, b, s_row, s_col, y), want_sym)):
+        got = got.cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(w))
+        assert np.array_equal(got[~np.isnan(w)].view(np.uint16), w[~np.isnan(w)].view(np.uint16))
