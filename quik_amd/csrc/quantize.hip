@@ -1343,6 +1343,111 @@ __global__ __launch_bounds__(64 * W) void quantize_fp6_wave_kernel(
   }
 }
 
+// ---------------------------------------------------------------------------------------
+// Stand-alone quantize straight from the index lists: no column map, one launch.
+//
+// What bounded the two launches it replaces at a few hundred rows was the map: one workgroup builds it, 6.3 us in front of
+// 6.2 us of quantizing 512 x 4096.  Here every workgroup loads the integer columns of its code groups itself, once
+// (clamped and packed to 16 bits in registers), together with its first row, marks the outlier columns in an LDS mask,
+// and then walks over rows blockIdx.x, blockIdx.x + gridDim.x, ..., the next row's loads in flight behind the gathers.
+// The results are those of a column map that does not stream (gather_rows), for any lists: minimum and maximum over the
+// columns that are not in the outlier list, codes in the order of the integer list, indices outside the row clamped.
+// A workgroup reads 8 bytes of list per integer column, which the L2 serves; two workgroups per CU bound that traffic.
+// Needs cols % 8 == 0, num_int % 8 == 0, 16-byte aligned rows and 8-byte aligned codes; NV: groups of 8 columns per lane.
+//
+// Measured (map + quantize -> this kernel, us in a graph, int4): 1 x 4096 9.1 -> 3.7, 512 x 4096 10.9 -> 5.2, 2048 x 8192
+// 21.6 -> 16.3, 512 x 13824 18.9 -> 12.8, 2048 x 16384 39.7 -> 29.8; int8 the same within 0.5.  At 2048 rows it is the
+// walk over four rows per workgroup that counts, 33 MB in 16 us.
+template <int BITS, bool BF16, int NV>
+__global__ __launch_bounds__(kThreads) void asym_quantize_list_kernel(
+    const uint16_t *__restrict__ x, int rows, int cols, const int64_t *__restrict__ int_idx, int num_int,
+    const int64_t *__restrict__ fp_idx, int num_fp, uint8_t *__restrict__ dst, uint16_t *__restrict__ meta,
+    uint16_t *__restrict__ fp_x) {
+  extern __shared__ __align__(16) uint16_t row_s[];  // the row, the outlier columns, the outlier mask
+  __shared__ float red[8];
+  const int tid = threadIdx.x, nvec = cols >> 3, groups = num_int >> 3, words = (cols + 31) / 32;
+  uint16_t *const fp_s = row_s + cols;
+  uint32_t *const mask_s = reinterpret_cast<uint32_t *>(fp_s + (num_fp + 7) / 8 * 8);
+  auto clamp = [&](int64_t c) { return static_cast<uint32_t>(c < 0 ? 0 : (c >= cols ? cols - 1 : c)); };
+  uint4 next[NV];
+  auto load = [&](int row) {
+    const uint4 *xv = reinterpret_cast<const uint4 *>(x + int64_t(row < rows ? row : rows - 1) * cols);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) next[i] = xv[tid + i * kThreads < nvec ? tid + i * kThreads : 0];
+  };
+  load(blockIdx.x);
+  uint32_t src[NV][4];  // this lane's code groups: eight byte offsets into the row
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int64_t *list = int_idx + (tid + i * kThreads < groups ? tid + i * kThreads : 0) * 8;
+    int64_t c[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) c[e] = list[e];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) src[i][e] = clamp(c[2 * e]) * 2u | clamp(c[2 * e + 1]) << 17;
+  }
+  for (int w = tid; w < words; w += kThreads) mask_s[w] = 0u;
+  __syncthreads();
+  for (int f = tid; f < num_fp; f += kThreads) {
+    const uint32_t c = clamp(fp_idx[f]);
+    fp_s[f] = static_cast<uint16_t>(c);
+    atomicOr(&mask_s[c >> 5], 1u << (c & 31u));
+  }
+  __syncthreads();
+  uint32_t skip[NV];  // this lane's row groups: their outlier columns
+#pragma unroll
+  for (int i = 0; i < NV; ++i) {
+    const int g = tid + i * kThreads;
+    skip[i] = g < nvec ? (mask_s[g >> 2] >> ((g & 3) * 8)) & 0xFFu : 0xFFu;
+  }
+  for (int row = blockIdx.x; row < rows; row += gridDim.x) {
+    float mn = __builtin_inff(), mx = -__builtin_inff();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      if (tid + i * kThreads < nvec) reinterpret_cast<uint4 *>(row_s)[tid + i * kThreads] = next[i];
+      const uint32_t w[4] = {next[i].x, next[i].y, next[i].z, next[i].w};
+#pragma unroll
+      for (int e = 0; e < 8; ++e) {
+        const float v = to_f32<BF16>(static_cast<uint16_t>(w[e >> 1] >> (16 * (e & 1))));
+        const bool out = (skip[i] >> e) & 1u;
+        mn = fminf(mn, out ? __builtin_inff() : v);
+        mx = fmaxf(mx, out ? -__builtin_inff() : v);
+      }
+    }
+    load(row + gridDim.x);
+    block_minmax<kThreads>(mn, mx, red);  // also orders the row's LDS writes before the gathers
+    RowQuant<BF16> rq;
+    rq.init(mn, mx, BITS);
+    if (tid == 0) {
+      meta[2 * row] = rq.scale_bits;
+      meta[2 * row + 1] = rq.zero_bits;
+    }
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+      const int g = tid + i * kThreads;
+      if (g >= groups) continue;
+      uint32_t w[4];
+#pragma unroll
+      for (int e = 0; e < 4; ++e) {
+        const uint8_t *base = reinterpret_cast<const uint8_t *>(row_s);
+        const uint32_t lo = *reinterpret_cast<const uint16_t *>(base + (src[i][e] & 0xFFFFu));
+        const uint32_t hi = *reinterpret_cast<const uint16_t *>(base + (src[i][e] >> 16));
+        w[e] = lo | hi << 16;
+      }
+      const uint4 v = make_uint4(w[0], w[1], w[2], w[3]);
+      const uint2 c = rq.slow ? group_codes<BITS, BF16, true>(v, rq) : group_codes<BITS, BF16, false>(v, rq);
+      if constexpr (BITS == 4) {
+        const uint32_t a = c.x | (c.x >> 4), b = c.y | (c.y >> 4);  // bytes 0 and 2: two codes each
+        reinterpret_cast<uint32_t *>(dst + int64_t(row) * (num_int >> 1))[g] = __builtin_amdgcn_perm(b, a, 0x06040200u);
+      } else {
+        reinterpret_cast<uint2 *>(dst + int64_t(row) * num_int)[g] = c;
+      }
+    }
+    for (int f = tid; f < num_fp; f += kThreads) fp_x[int64_t(row) * num_fp + f] = row_s[fp_s[f]];
+    __syncthreads();  // the next row overwrites row_s
+  }
+}
+
 // Rows too long for LDS: same arithmetic, gathers go to global memory (L2-resident row).
 template <typename IdxT, int BITS, bool BF16>
 __global__ __launch_bounds__(kThreads) void asym_quantize_longrow_kernel(
@@ -1694,6 +1799,50 @@ int launch_fp6_wave(const void *x, int64_t rows, int64_t cols, const uint8_t *cm
   if (per_cu >= 2) return go(quantize_fp6_wave_kernel<BF16, SYM, 0, 2>, 2);
   return go(quantize_fp6_wave_kernel<BF16, SYM, 0, 1>, 1);
 }
+// asym_quantize_list_kernel: calls that it takes (everything else, and every error, is left to the column map's path).
+// Up to 16384 columns it was the faster one at every row count from 1 to 2048 (2048 x 11008 27.1 -> 25.5, the least); with
+// 16 groups per lane only where a CU has one row (256 x 28672 26.0 -> 18.0 us, 512 rows 31.0 -> 33.8).
+bool list_quantize_ok(const void *x, int dtype, int64_t rows, int64_t cols, const int64_t *int_idx, int64_t num_int,
+                      const int64_t *fp_idx, int64_t num_fp, int bits, const void *colmap, const void *dst, const void *meta,
+                      const void *fp_x) {
+  if ((bits != 4 && bits != 8) || (dtype != QUIK_F16 && dtype != QUIK_BF16)) return false;
+  if (rows <= 0 || rows >= (1 << 30) || cols <= 0 || cols > kStreamMaxCols || num_int <= 0 || num_fp < 0 || num_int + num_fp != cols) return false;
+  if (cols > 16384 && rows > num_cus()) return false;
+  if (!x || !int_idx || !colmap || !dst || !meta || (num_fp > 0 && (!fp_idx || !fp_x))) return false;
+  return cols % 8 == 0 && num_int % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 8 == 0;
+}
+int launch_list(const void *x, int dtype, int64_t rows, int64_t cols, const int64_t *int_idx, int64_t num_int,
+                const int64_t *fp_idx, int64_t num_fp, int bits, void *dst, void *meta, void *fp_x, hipStream_t st) {
+  const int64_t lds = cols * 2 + (num_fp + 7) / 8 * 16 + (cols + 31) / 32 * 4;
+  const int64_t grid = rows < 2 * num_cus() ? rows : 2 * num_cus();
+  auto go = [&](auto kern) {
+    if (lds > 48 * 1024) {
+      if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                             static_cast<int>(kMaxLdsRowBytes));
+          e != hipSuccess) {
+        set_last_hip_error(e);
+        return static_cast<int>(QUIK_ERR_LAUNCH);
+      }
+    }
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kThreads), static_cast<size_t>(lds), st,
+                       static_cast<const uint16_t *>(x), static_cast<int>(rows), static_cast<int>(cols), int_idx,
+                       static_cast<int>(num_int), fp_idx, static_cast<int>(num_fp), static_cast<uint8_t *>(dst),
+                       static_cast<uint16_t *>(meta), static_cast<uint16_t *>(fp_x));
+    return static_cast<int>(check_launch());
+  };
+#define QUIK_LIST_NV(BITS, BF16)                                                   \
+  return cols <= 4096    ? go(asym_quantize_list_kernel<BITS, BF16, 2>)            \
+         : cols <= 8192  ? go(asym_quantize_list_kernel<BITS, BF16, 4>)            \
+         : cols <= 16384 ? go(asym_quantize_list_kernel<BITS, BF16, 8>)            \
+                         : go(asym_quantize_list_kernel<BITS, BF16, 16>)
+  if (bits == 4) {
+    if (dtype == QUIK_F16) QUIK_LIST_NV(4, false);
+    QUIK_LIST_NV(4, true);
+  }
+  if (dtype == QUIK_F16) QUIK_LIST_NV(8, false);
+  QUIK_LIST_NV(8, true);
+#undef QUIK_LIST_NV
+}
 }  // namespace
 }  // namespace quik
 
@@ -1740,6 +1889,8 @@ extern "C" int quik_asym_quantize_indexed(const void *x, int dtype, int64_t rows
                                           int64_t num_int, const int64_t *fp_indices, int64_t num_fp, int bits,
                                           void *colmap_workspace, void *dst, void *meta, void *fp_x, void *stream) {
   if (rows == 0) return QUIK_OK;
+  if (list_quantize_ok(x, dtype, rows, cols, int_indices, num_int, fp_indices, num_fp, bits, colmap_workspace, dst, meta, fp_x))
+    return launch_list(x, dtype, rows, cols, int_indices, num_int, fp_indices, num_fp, bits, dst, meta, fp_x, as_stream(stream));
   if (int rc = build_colmap(int_indices, num_int, fp_indices, num_fp, cols, colmap_workspace, stream, 1)) return rc;
   return quik_asym_quantize(x, dtype, rows, cols, colmap_workspace, num_int, num_fp, bits, dst, meta, fp_x, stream);
 }
