@@ -26,6 +26,7 @@ using CfgM = Cfg<128, 128, 2, 2, 2>;   // mid-size problems, two workgroups per 
 using CfgN = Cfg<128, 64, 2, 2, 2>;    // few tiles: narrower ones put more CUs to work, three workgroups per CU
 using CfgN6 = Cfg<128, 64, 2, 2, 2>;   // 6-bit path, 86 .. ~150 tiles of 128x128 and no K split: twice as many workgroups
 using CfgN8 = Cfg<128, 64, 2, 2, 2, 8>; // the same, one workgroup per CU with eight stages of copies
+using CfgD6 = Cfg<128, 64, 2, 2, 2, 8>; // the same with one workgroup per CU and twelve slots
 using CfgL8 = Cfg<256, 256, 2, 4, 2>;  // 6-bit path, launches of 256x256 tiles only: two waves per SIMD (1-5 % faster than CfgL)
 using CfgLp = Cfg<256, 256, 2, 2, 0>;  // plain fallbacks
 using CfgMp = Cfg<128, 128, 2, 2, 0>;
@@ -655,7 +656,14 @@ int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t wor
     const int64_t mid_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128);
     // (up to 0.62 tiles per CU: measured 6 - 12 % less time on 13B gate_proj at 128 tokens, 70B k_proj and the
     // 512 x 4096 x 4096 configuration; with 0.88 tiles per CU, 70B gate_proj at 64 tokens, 11 % more)
-    if (mid_tiles * 8 <= int64_t(num_cus()) * 5) return launch_fused6<CfgN6, BF16>(p, st);
+    if (mid_tiles * 8 <= int64_t(num_cus()) * 5) {
+      // One tile per CU: a ring of twelve slots (110 KB of LDS) instead of six, nine steps in flight instead of three.  Layer
+      // forward 300 x 4544 -> 4544 19.1 -> 18.6 us, 2048 x 8192 -> 1024 31.3 -> 30.7, 128 x 5120 -> 13824 20.3 -> 20.0, 256 x
+      // 8192 -> 8192 26.5 -> 25.9: a step still takes about 240 cycles for 64 of MFMA (two steps between barriers, or no
+      // second copy of the W block, changed nothing on top).  More tiles need two workgroups per CU, which six slots allow.
+      if ((p.M + 127) / 128 * ((p.N + 63) / 64) <= num_cus()) return launch_fused6<CfgD6, BF16>(p, st);
+      return launch_fused6<CfgN6, BF16>(p, st);
+    }
     return launch_fused6<CfgM, BF16>(p, st);
   }
   Fused6Args wide = p, tail = p;

@@ -45,7 +45,8 @@ __device__ __forceinline__ void dma_load16k(const uint8_t *sbase, uint32_t voff,
 
 template <class C>
 struct Fp6Pipe {
-  static constexpr int MI = C::MI, NI = C::NI, NS = 6, NF = MI + NI;
+  static constexpr int MI = C::MI, NI = C::NI, NF = MI + NI;
+  static constexpr int NS = C::DMA_STAGES > 4 ? 12 : 6;  // LDS slots; one step is multiplied, NS - 1 are landed or in flight
   // a wave's fragments start at a 64-row block of the operand, or the wave has a single 32-row fragment (then it may
   // be the second half of a block)
   static_assert(C::WM % 64 == 0 || C::MI == 1, "a wave's token rows");
@@ -66,7 +67,7 @@ struct Fp6Pipe {
   static_assert((XB == 4 && (WB == 4 || WB == 2)) || (XB == 2 && (WB == 2 || WB == 1)), "supported tile shapes");
   static_assert(C::WAVES == 4 || XB + WB == 8, "eight waves copy eight blocks");
   static constexpr int P = 3 + NB;  // copies per wave and step
-  static_assert(3 * P <= 63, "three steps in flight must fit the vmcnt counter");
+  static_assert((NS - 3) * P <= 63, "the steps in flight must fit the vmcnt counter");
 
   uint8_t *smem;
   uint32_t lds0;
@@ -78,7 +79,7 @@ struct Fp6Pipe {
   uint32_t rd;              // byte offset of the slot the next fragment read looks at
   int steps0, steps;        // integer steps, all steps
   uint32_t x_head, w_head;  // this lane's head offsets inside a slot (fragment j: + 1024 j)
-  uint32_t x_head3[3], w_head3[3], tail3[3][NF];  // the same offsets inside slots 0, 2 and 4 (for steps whose slot is
+  uint32_t x_head3[NS / 2], w_head3[NS / 2], tail3[NS / 2][NF];  // the same inside slots 0, 2, 4, .. (for steps whose slot is
                                                   // known at compile time: the odd slot is an immediate offset away)
   uint32_t tail[NF];        // this lane's tail offsets inside a slot, one register per fragment: reads that share
                             // a base register are paired into one 4-register read by the compiler, and the halves
@@ -138,7 +139,7 @@ struct Fp6Pipe {
       asm volatile("" : "+v"(tail[j]));  // unrelated values as far as the compiler can tell (empty statement: no hazard)
     }
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 0; q < NS / 2; ++q) {
       x_head3[q] = x_head + q * 2 * STAGE;
       w_head3[q] = w_head + q * 2 * STAGE;
 #pragma unroll
@@ -180,15 +181,11 @@ struct Fp6Pipe {
     }
   }
 
-  // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. 4 are in flight; the copies of step 5
-  // are made during the MFMAs of step 0.
+  // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. NS - 2 are in flight; the copies of step
+  // NS - 1 are made during the MFMAs of step 0.
   __device__ __forceinline__ void start() {
-    issue();
-    issue();
-    issue();
-    issue();
-    issue();
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * P));
+    static_for<NS - 1>([&](auto) { issue(); });
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
     __syncthreads();
   }
 
@@ -259,14 +256,14 @@ struct Fp6Pipe {
   }
 
   // One step, cut into P chunks: chunk G holds its share of the step's MFMAs (on the fragments in `cur`),
-  // of the next step's fragment reads (into `nxt`) and one of the P copies of the step five ahead of the
-  // one in the MFMAs.  A copy instruction occupies the wave until the memory pipeline has taken its 64
+  // of the next step's fragment reads (into `nxt`) and one of the P copies of the step NS - 1 ahead of
+  // the one in the MFMAs.  A copy instruction occupies the wave until the memory pipeline has taken its 64
   // addresses; six of them in a row at the start of a step stall the MFMA issue for as long as the copies
   // take, so they go one by one between groups of MFMAs.  Then: wait until the step after next has
-  // landed (the three newer ones stay in flight) and a barrier makes it visible; behind it every wave has
+  // landed (the NS - 3 newer ones stay in flight) and a barrier makes it visible; behind it every wave has
   // issued the MFMAs of this step, which waited for their fragments, so this step's slot may be overwritten
   // by the copies issued during the next step.
-  // RS / FS: the slots read and filled during this step when they are known at compile time (six steps in a
+  // RS / FS: the slots read and filled during this step when they are known at compile time (NS steps in a
   // row return to the same slots, so `rd` and `fill` stay valid without being touched), -1: `rd` / `fill`
   template <int RS = -1, int FS = -1, int G = 0>
   __device__ __forceinline__ void step6(const v4i (&ch)[NF], const v2i (&ct)[NF], v4i (&nh)[NF], v2i (&nt)[NF],
@@ -289,7 +286,7 @@ struct Fp6Pipe {
       step6<RS, FS, G + 1>(ch, ct, nh, nt, acc);
     } else {
       if constexpr (RS < 0) next_read_slot();
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * P));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
       __builtin_amdgcn_s_barrier();
     }
   }
@@ -327,7 +324,7 @@ struct Fp6Pipe {
       step16<BF16, G + 1>(cf, nf, acc);
     } else {
       next_read_slot();
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * P));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
       __builtin_amdgcn_s_barrier();
     }
   }
@@ -351,16 +348,15 @@ struct Fp6Pipe {
     v4i h0[NF], h1[NF];
     v2i t0[NF], t1[NF];
     read6(h0, t0);
-    // here: step 0 in h0 / t0, `rd` at slot 1, `fill` at slot 5.  Six steps at a time with the slots as
+    // here: step 0 in h0 / t0, `rd` at slot 1, `fill` at slot NS - 1.  NS steps at a time with the slots as
     // immediates (no address arithmetic in the loop), then the remaining pairs with `rd` / `fill`
     int j = 0;
-    for (; j + 6 <= steps0; j += 6) {
-      step6<1, 5>(h0, t0, h1, t1, acc);
-      step6<2, 0>(h1, t1, h0, t0, acc);
-      step6<3, 1>(h0, t0, h1, t1, acc);
-      step6<4, 2>(h1, t1, h0, t0, acc);
-      step6<5, 3>(h0, t0, h1, t1, acc);
-      step6<0, 4>(h1, t1, h0, t0, acc);
+    for (; j + NS <= steps0; j += NS) {
+      static_for<NS / 2>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = 2 * I;
+        step6<i + 1, (i + NS - 1) % NS>(h0, t0, h1, t1, acc);
+        step6<(i + 2) % NS, i>(h1, t1, h0, t0, acc);
+      });
     }
     for (; j < steps0; j += 2) {
       step6(h0, t0, h1, t1, acc);

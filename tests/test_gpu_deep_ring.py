@@ -1,0 +1,30 @@
+"""128x64 tiles of the 6-bit GEMM with one tile per CU (ring of twelve slots): fewer steps than slots, exactly as many, one
+pair more, whole turns with every remainder, none and more outlier steps than slots.  Same output bits as the row-major
+int8-MFMA kernels, which other tests hold against the oracle."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("M,N,K,F", [(128, 13824, 128, 0), (100, 13830, 640, 32), (128, 13824, 768, 288), (127, 13800, 896, 0),
+                                     (120, 13824, 1536, 64), (128, 13001, 1792, 256), (300, 5120, 2688, 96), (257, 4544, 4416, 128)])
+def test_same_bits_as_the_row_major_kernels(M, N, K, F, dtype):
+    from quik_amd.qlinear import MixedQLinear
+    g = torch.Generator().manual_seed(M + N + K + F)
+    fi = torch.randperm(K + F, generator=g)[:F]
+    s_w = (torch.rand(N, 1, generator=g) * 0.009 + 0.001).to(dtype)
+    W = (torch.randint(-8, 8, (N, K + F), generator=g).float() * s_w.float()).to(dtype)
+    lin = torch.nn.Linear(K + F, N, bias=True, dtype=dtype)
+    mod = MixedQLinear.from_float(lin, W, s_w, None, fi, bits=4).to(DEV)
+    x = torch.randn(M, K + F, generator=g)
+    x[:, fi] *= 50
+    x = x.to(dtype).to(DEV)
+    got = [mod(x) for _ in range(2)]
+    assert mod._w6 is not None
+    mod.six_bit_path = False
+    want = mod(x)
+    for o in got:
+        assert torch.equal(o.view(torch.int16), want.view(torch.int16))
