@@ -688,4 +688,22 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_split_kernel(Fused6A
   }
 }
 
+// One launch of whole rounds of 256x256 tiles and, for the columns that are left (from `first` on, in 128-column tiles), 128x128
+// tiles: at most one per CU.  Both regions start at multiples of 8 workgroups.
+struct RestGrid {
+  int tiles_m_wide, tiles_n_wide, wide_blocks, tiles_m, tiles_n, first;
+};
+template <class CW, class CT, bool BF16>
+__global__ __launch_bounds__(CW::kThreads) void gemm_fused6_rest_kernel(Fused6Args p, RestGrid g) {
+  static_assert(CW::kThreads == CT::kThreads, "one block size");
+  extern __shared__ __align__(16) uint8_t smem[];
+  int tm, tn;
+  const int bid = blockIdx.x;
+  if (bid < g.wide_blocks) {
+    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused6_tile<CW, BF16>(p, tm, tn, smem);
+  } else if (tile_of_block<CT::BM>(bid - g.wide_blocks, g.tiles_m, g.tiles_n, tm, tn)) {
+    fused6_tile<CT, BF16>(p, tm, g.first + tn, smem);
+  }
+}
+
 }  // namespace quik
