@@ -643,7 +643,8 @@ int run_direct(const Args &p, hipStream_t st, void *workspace, int64_t workspace
 // The 6-bit matrix-core path (gemm_fp6.h): 256x256 tiles alone (eight waves), 256x256 + 256x128 tiles in one
 // launch (four waves), or 128x128 tiles.
 // Whole rounds of 256x256 tiles with little left over: a last round of 256x128 tiles costs 59, on part of the CUs; the same
-// columns in 128x128 tiles are one per CU at 36 (percent of a wide tile).  2048 x 8192 -> 10240: 126.3 -> 115.8 us per forward.
+// columns in 128x128 tiles are one per CU at 36 (percent of a wide tile).  2048 x 8192 -> 10240: 126.3 -> 112.6 us per
+// forward, int8 188 -> 176.
 // Only behind whole rounds: narrow tiles that run beside wide ones are slower than the costs say (777 x 4096 -> 22016 by
 // the same costs 159 -> 136, measured 72.2 -> 73.8 us), and two of them per CU cost more than a 256x128 tile.
 // Returns the columns of the wide part, 0: the plan of make_plan6 stands.
@@ -655,14 +656,12 @@ int64_t plan_rest(int64_t M, int64_t N, const Plan &plan) {
   const int64_t now = makespan(tiles_m * ((nw + 255) / 256), tiles_m * ((N - nw + 127) / 128), 59);
   return rest > 0 && rest <= cus && rounds * kCostWide + 36 < now ? wide_n * 256 : 0;
 }
-template <class CW, class CT, bool BF16>
-int launch_fused6_rest(const Fused6Args &p, int64_t n_wide, hipStream_t st) {
+template <class CW, class CT, class Args, class Kernel>
+int launch_rest(Kernel kern, int smem, const Args &p, int64_t n_wide, hipStream_t st) {
   RestGrid g{};
   g.wide_blocks = grid_of<CW>(p.M, n_wide, g.tiles_m_wide, g.tiles_n_wide);
   const int rest_blocks = grid_of<CT>(p.M, p.N - n_wide, g.tiles_m, g.tiles_n);
   g.first = static_cast<int>(n_wide / CT::BN);
-  auto kern = gemm_fused6_rest_kernel<CW, CT, BF16>;
-  constexpr int smem = fused6_smem<CW>() > fused6_smem<CT>() ? fused6_smem<CW>() : fused6_smem<CT>();
   if (int rc = prepare(kern, smem)) return rc;
   hipLaunchKernelGGL(kern, dim3(g.wide_blocks + rest_blocks), dim3(CW::kThreads), smem, st, p, g);
   return check_launch();
@@ -674,7 +673,8 @@ int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t wor
   // callers that keep both weight copies route such calls there
   if (const int rc = run_direct<true, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
   const Plan plan = make_plan6(p.M, p.N, 1);
-  if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0) return launch_fused6_rest<CfgL, CfgM, BF16>(p, n_wide, st);
+  if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0)
+    return launch_rest<CfgL, CfgM>(gemm_fused6_rest_kernel<CfgL, CfgM, BF16>, fused6_smem<CfgL>(), p, n_wide, st);
   if (plan.kind == Plan::kSplit && plan.n_wide >= p.N) return launch_fused6<CfgL8, BF16>(p, st);
   if (plan.kind != Plan::kSplit) {
     const SplitPlan sp = plan_splitk(p.M, p.N, tile_steps(p.K, 4), kSplitMinSteps6, 1, 3);
@@ -741,6 +741,8 @@ int run_fused8t(const Fused8Args &p, hipStream_t st, void *workspace, int64_t wo
     if (sp.splits > 1 && workspace && workspace_bytes >= sp.bytes) return launch_fused8t_splitk<BF16>(p, sp, workspace, st);
     return launch_fused8t<CfgM, BF16>(p, st);
   }
+  if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0)
+    return launch_rest<CfgL, CfgM>(gemm_fused8t_rest_kernel<CfgL, CfgM, BF16>, fused8t_smem<CfgL>(), p, n_wide, st);
   if (plan.n_wide >= p.N) return launch_fused8t<CfgL8, BF16>(p, st);
   Fused8Args wide = p, tail = p;
   const int64_t nw = plan.n_wide;

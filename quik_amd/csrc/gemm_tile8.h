@@ -416,4 +416,18 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused8t_split_kernel(Fused8
   }
 }
 
+// whole rounds of wide tiles and a rest of 128x128 ones (see gemm_fused6_rest_kernel)
+template <class CW, class CT, bool BF16>
+__global__ __launch_bounds__(CW::kThreads) void gemm_fused8t_rest_kernel(Fused8Args p, RestGrid g) {
+  static_assert(CW::kThreads == CT::kThreads, "one block size");
+  extern __shared__ __align__(16) uint8_t smem[];
+  int tm, tn;
+  const int bid = blockIdx.x;
+  if (bid < g.wide_blocks) {
+    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused8t_tile<CW, BF16>(p, tm, tn, smem);
+  } else if (tile_of_block<CT::BM>(bid - g.wide_blocks, g.tiles_m, g.tiles_n, tm, tn)) {
+    fused8t_tile<CT, BF16>(p, tm, g.first + tn, smem);
+  }
+}
+
 }  // namespace quik
