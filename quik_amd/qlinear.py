@@ -411,15 +411,19 @@ class MixedQLinear(torch.nn.Module):
         return self._streams
 
     # -- one library call per forward (quik_layer_forward): the layer's buffers described once
-    def _descriptor(self, tiled):
-        """(ctypes quik_layer, workspace sizes by row count) for this module, with or without the tile-ordered weight
-        copy; cached, rebuilt when a buffer moves or is written in place."""
+    def _descriptor_source(self):
+        """(the buffers a descriptor is made from, the key of their state): a cached descriptor holds for an equal key."""
         bufs = (self.int_weight, self.weights_scales, self.int_indices, self.fp_indices,
                 self.reduced_w if not self.symmetric else None, self.fp_weight if self.fp_features_num > 0 else None,
                 self.bias)
         # (the scalar switches below are baked into the descriptor too: changing one after a forward rebuilds it)
-        key = tuple((b.data_ptr(), b._version) if b is not None else None for b in bufs) + \
+        return bufs, tuple((b.data_ptr(), b._version) if b is not None else None for b in bufs) + \
             (self.six_bit_min_rows, self.tile8_min_rows, float(self.sym_divisor), bool(self.six_bit_path))
+
+    def _descriptor(self, tiled):
+        """(ctypes quik_layer, workspace sizes by row count) for this module, with or without the tile-ordered weight
+        copy; cached, rebuilt when a buffer moves or is written in place."""
+        bufs, key = self._descriptor_source()
         transient = tiled and self.transient_tiled_copy and not self._row_major_released
         if transient:
             # the cached descriptor of the row-major form, copied, with this call's temporary operand buffer
@@ -483,6 +487,12 @@ class MixedQLinear(torch.nn.Module):
         unchanged module are one crossing into C++, which makes the same checks, allocations and library call."""
         if L.load() is not L._lib or type(self).mid_event is not None or self.mid_event is not None:
             return        # (a substituted binding, a class-wide profiling hook: the Python path serves those)
+        # A forward brings the descriptor of its own path up to date; the other path's may date from before the buffers
+        # changed.  The plan compares the buffers with what they are now, so nothing later would find that out.
+        key = self._descriptor_source()[1]
+        for t in (False, True):
+            if t in self._descs and self._descs[t][0] != key:
+                del self._descs[t]
         row, til = self._descs.get(False), self._descs.get(True)
         if (til if tiled else row) is None:
             return        # transient_tiled_copy: the operand is repacked by every call

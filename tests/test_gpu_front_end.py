@@ -12,10 +12,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def _module(seed, N, n_in, F, bits, shared=None, bias=False):
+def _module(seed, N, n_in, F, bits, shared=None, bias=False, outlier_seed=1):
     from quik_amd.qlinear import MixedQLinear
     rng = np.random.default_rng(seed)
-    fi = torch.from_numpy(np.sort(np.random.default_rng(1).permutation(n_in)[:F]))
+    fi = torch.from_numpy(np.sort(np.random.default_rng(outlier_seed).permutation(n_in)[:F]))
     s_w = torch.from_numpy(rng.uniform(0.001, 0.01, (N, 1)).astype(np.float16))
     lo, hi = (-8, 8) if bits == 4 else (-127, 128)
     W = torch.from_numpy((rng.integers(lo, hi, (N, n_in)) * s_w.float().numpy()).astype(np.float16))
@@ -74,6 +74,35 @@ def test_a_planned_forward_sees_every_change(rows, bits):
     finally:
         MixedQLinear._forward_one_call = real
     assert MixedQLinear.six_bit_min_rows == keep
+
+
+def _rewrite(mod, other):
+    mod.load_state_dict(other.state_dict())
+
+
+def _assign(mod, other):
+    mod.load_state_dict({k: v.clone() for k, v in other.state_dict().items()}, assign=True)
+
+
+def _move(mod, other):
+    mod.cpu()
+    mod.load_state_dict(other.state_dict())
+    mod.to(DEV)
+
+
+@pytest.mark.parametrize("change", [_rewrite, _assign, _move])
+@pytest.mark.parametrize("outliers", [1, 2])               # the same outlier columns as before, or others
+@pytest.mark.parametrize("before,after", [((64, 1), (1, 64)), ((1, 64), (64, 1)), ((64, 1), (64, 1)), ((64,), (1, 64))])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_both_paths_see_a_change_of_the_weights(bits, before, after, outliers, change):
+    N, n_in, F = 264, 1024 + 64, 64
+    mod, other = (_module(s, N, n_in, F, bits, bias=True, outlier_seed=o) for s, o in ((0, 1), (7, outliers)))
+    xs = {r: torch.randn(r, n_in, generator=torch.Generator().manual_seed(r)).half().to(DEV) for r in (1, 64)}
+    for rows in before + before:
+        mod(xs[rows])
+    change(mod, other)
+    for rows in after + after:
+        assert _same(mod(xs[rows]), other(xs[rows]))
 
 
 @pytest.mark.parametrize("rows", [1, 40])

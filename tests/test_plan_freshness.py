@@ -1,0 +1,131 @@
+"""Plans for the native front end hold only what the module's buffers are when the plan is made.
+
+A layer keeps one descriptor per path (row-major, tile-ordered), and a forward brings only its own up to date.  Here the
+library, the packing kernels and the front end are stand-ins on CPU tensors, so that the descriptors a plan receives can
+be compared with the module's buffers: addresses, and the contents that the tile-ordered operand was packed from.
+"""
+import ctypes
+import itertools
+
+import pytest
+import torch
+
+from quik_amd import _lib as L
+from quik_amd import asymmetric, matmul, qlinear
+from quik_amd.qlinear import MixedQLinear
+
+N, N_IN, F = 24, 160, 32
+DECODE, PREFILL = 1, 64     # row-major and tile-ordered path
+
+
+class Binding:
+    def __init__(self):
+        self.calls, self.packed, self.plans = [], {}, []
+
+    # the library
+    def quik_layer_workspace_bytes(self, desc, rows):
+        return 16
+
+    def quik_layer_forward(self, desc, x, rows, *rest):
+        self.calls.append((rows, L.QuikLayer.from_buffer_copy(desc._obj)))
+        return 0
+
+    # the packing kernels: an operand that is a copy of what it was made from
+    def pack(self, int_weight, fp_weight, colmap, *rest):
+        w6 = torch.cat([int_weight.reshape(-1), fp_weight.contiguous().view(torch.uint8).reshape(-1), colmap])
+        self.packed[w6.data_ptr()] = w6.clone()
+        return w6
+
+    # the front end
+    def plan(self, module, names, row, tiled, tiled_from, device, bf16, dev, splitk, keep):
+        self.plans.append([None if b is None else L.QuikLayer.from_buffer_copy(b) for b in (row, tiled)])
+        return object()
+
+
+def colmap_of(int_indices, fp_indices, cols):
+    return torch.cat([int_indices, fp_indices]).to(torch.uint8)
+
+
+@pytest.fixture
+def binding(monkeypatch):
+    b = Binding()
+    monkeypatch.setattr(L, "load", lambda: b)
+    monkeypatch.setattr(L, "_lib", b)
+    monkeypatch.setattr(L, "front", lambda: b)
+    monkeypatch.setattr(L, "stream", lambda: 0)
+    monkeypatch.setattr(qlinear, "_front", None)
+    monkeypatch.setattr(asymmetric, "build_colmap", colmap_of)
+    monkeypatch.setattr(asymmetric, "colmap_streams", lambda *a: True)
+    monkeypatch.setattr(matmul, "_splitk_workspace", lambda *a: (None, 0))
+    for name in ("pack_weight_layer", "pack_weight_fp6"):
+        monkeypatch.setattr(matmul, name, b.pack)
+    return b
+
+
+def layer(seed):
+    g = torch.Generator().manual_seed(seed)
+    m = MixedQLinear(N_IN, N, fp_features_num=F)
+    perm = torch.randperm(N_IN, generator=g)
+    m.int_indices.copy_(perm[F:].sort()[0])
+    m.fp_indices.copy_(perm[:F])
+    m.int_weight.random_(0, 256, generator=g)
+    for name in ("weights_scales", "fp_weight", "reduced_w", "bias"):
+        getattr(m, name).normal_(generator=g)
+    return m
+
+
+def call(m, rows):
+    assert m._forward_one_call(torch.zeros(rows, N_IN, dtype=torch.float16)) is not None
+
+
+def check(b, m, desc, tiled):
+    """`desc` describes the module as it is now."""
+    for field in ("int_weight", "weights_scales", "reduced_w", "fp_weight", "bias"):
+        t = getattr(m, field)
+        assert getattr(desc, field) == (None if t is None else t.data_ptr()), field
+    assert desc.colmap == m._column_map().data_ptr()
+    colmap = colmap_of(m.int_indices, m.fp_indices, N_IN)
+    held = (ctypes.c_uint8 * len(colmap)).from_address(desc.colmap)
+    assert bytes(held) == bytes(colmap.tolist())
+    if tiled:
+        assert torch.equal(b.packed[desc.tiled_weight], b.pack(m.int_weight, m.fp_weight, colmap))
+
+
+def in_place(m):
+    m.load_state_dict(layer(1).state_dict())
+
+
+def replaced(m):
+    m.load_state_dict(layer(1).state_dict(), assign=True)
+
+
+def one_replaced(m):
+    m.bias = layer(1).bias
+
+
+def no_bias(m):
+    m.bias = None
+
+
+def new_outliers(m):
+    other = layer(2)
+    m.int_indices.copy_(other.int_indices)
+    m.fp_indices.copy_(other.fp_indices)
+
+
+@pytest.mark.parametrize("change", [in_place, replaced, one_replaced, no_bias, new_outliers])
+@pytest.mark.parametrize("before", [(), (DECODE,), (PREFILL,), (DECODE, PREFILL), (PREFILL, DECODE)])
+def test_a_plan_holds_current_descriptors(binding, before, change):
+    for after in itertools.product((DECODE, PREFILL), repeat=3):
+        m = layer(0)
+        for rows in before:
+            call(m, rows)
+        change(m)
+        for rows in after:
+            call(m, rows)
+            check(binding, m, binding.calls[-1][1], rows >= 33)
+            row, tiled = binding.plans[-1]
+            assert (tiled if rows >= 33 else row) is not None
+            for desc, t in ((row, False), (tiled, True)):
+                if desc is not None:
+                    check(binding, m, desc, t)
