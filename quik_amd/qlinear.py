@@ -424,8 +424,11 @@ class MixedQLinear(torch.nn.Module):
         """(ctypes quik_layer, workspace sizes by row count) for this module, with or without the tile-ordered weight
         copy; cached, rebuilt when a buffer moves or is written in place."""
         bufs, key = self._descriptor_source()
-        transient = tiled and self.transient_tiled_copy and not self._row_major_released
-        if transient:
+        transient = self.transient_tiled_copy and not self._row_major_released
+        if transient:     # (set after a prefill: the copy that one kept goes)
+            self._descs.pop(True, None)
+            self._w6 = self._w6_key = None
+        if transient and tiled:
             # the cached descriptor of the row-major form, copied, with this call's temporary operand buffer
             base, sizes = self._descriptor(False)
             d = L.QuikLayer.from_buffer_copy(base)
@@ -485,6 +488,7 @@ class MixedQLinear(torch.nn.Module):
     def _make_fast(self, tiled, device):
         """A plan for the native front end (csrc/front.cpp) from the descriptors this forward used: later calls on the
         unchanged module are one crossing into C++, which makes the same checks, allocations and library call."""
+        self._descs.pop("fast", None)     # (a plan keeps the tensors it was made from)
         if L.load() is not L._lib or type(self).mid_event is not None or self.mid_event is not None:
             return        # (a substituted binding, a class-wide profiling hook: the Python path serves those)
         # A forward brings the descriptor of its own path up to date; the other path's may date from before the buffers

@@ -105,6 +105,22 @@ def test_both_paths_see_a_change_of_the_weights(bits, before, after, outliers, c
         assert _same(mod(xs[rows]), other(xs[rows]))
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+def test_transient_policy_set_after_a_prefill(bits):
+    N, n_in, F = 264, 1024 + 64, 64
+    mod, other = _module(0, N, n_in, F, bits), _module(7, N, n_in, F, bits)
+    xs = {r: torch.randn(r, n_in, generator=torch.Generator().manual_seed(r)).half().to(DEV) for r in (1, 64)}
+    for rows in (64, 1, 64):
+        mod(xs[rows])
+    mod.transient_tiled_copy = True
+    for rows in (64, 1, 64):
+        mod(xs[rows])
+        assert mod.weight_bytes()["tiled"] == 0
+    mod.load_state_dict(other.state_dict())
+    for rows in (64, 1, 64, 64):
+        assert _same(mod(xs[rows]), other(xs[rows]))
+
+
 @pytest.mark.parametrize("rows", [1, 40])
 def test_a_planned_group_sees_every_change(rows):
     from quik_amd.qlinear import SharedQuantizedInput

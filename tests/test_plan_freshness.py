@@ -129,3 +129,25 @@ def test_a_plan_holds_current_descriptors(binding, before, change):
             for desc, t in ((row, False), (tiled, True)):
                 if desc is not None:
                     check(binding, m, desc, t)
+
+
+@pytest.mark.parametrize("on_class", [False, True])
+@pytest.mark.parametrize("first", [DECODE, PREFILL])
+def test_no_tiled_copy_stays_with_the_transient_policy(binding, monkeypatch, first, on_class):
+    m = layer(0)
+    call(m, PREFILL)
+    call(m, DECODE)
+    assert m.weight_bytes()["tiled"] > 0
+    if on_class:
+        monkeypatch.setattr(MixedQLinear, "transient_tiled_copy", True)
+    else:
+        m.transient_tiled_copy = True
+    for rows in (first, DECODE, PREFILL, DECODE):
+        made = len(binding.plans)
+        call(m, rows)
+        check(binding, m, binding.calls[-1][1], rows >= 33)
+        assert m.weight_bytes()["tiled"] == 0 and True not in m._descs
+        if rows >= 33:                                    # each such call packs its own operand: no plan serves it
+            assert len(binding.plans) == made and "fast" not in m._descs
+        else:
+            assert binding.plans[-1][1] is None
