@@ -105,9 +105,10 @@ class SharedQuantizedInput:
             self.cur_group_elem = 0
 
     def _members_key(self, mods):
-        return tuple((id(m), m.int_weight.data_ptr(), m.int_weight._version, m.weights_scales.data_ptr(),
-                      m.int_indices._version, m.fp_indices._version, bool(m.six_bit_path), m.six_bit_min_rows,
-                      m.tile8_min_rows) for m in mods)
+        """Everything of the members that the concatenated layer is made from: their buffers and their switches."""
+        return tuple((id(m),) + tuple(getattr(m, name) for name in _SWITCH_NAMES) +
+                     tuple(None if t is None else (t.data_ptr(), t._version)
+                           for t in (m._buffers.get(name) for name in _BUFFER_NAMES)) for m in mods)
 
     def _fused_layer(self):
         """The members' weights as one MixedQLinear (None when the group is not complete or not compatible).  Built
@@ -132,6 +133,8 @@ class SharedQuantizedInput:
                         for m in mods[1:])
         if not ok:
             self._fused, self._fused_key = False, self._members_key(mods)
+            for m in mods:      # (plans of an earlier round keep that round's concatenated buffers)
+                m._descs.pop("fast", None)
             return None
         fused = _concatenate_layers(mods)
         fused.six_bit_path = first.six_bit_path
@@ -182,7 +185,7 @@ class SharedQuantizedInput:
         """Hand the round just served by Python to the native front end: later rounds on unchanged members go through
         `_front.group_forward`, which every member finds under its own "fast" entry."""
         inner = fused._descs.get("fast")
-        if inner is None or inner[1] is not None or not all(type(m).fuse_shared_groups for m in mods):
+        if inner is None or inner[1] is not None or not all(m.fuse_shared_groups and m.shared_input is self for m in mods):
             return
         names = _BUFFER_NAMES
         plan = _front.group(weakref.ref(self), fused, inner[0],
@@ -194,6 +197,8 @@ class SharedQuantizedInput:
 
 
 _BUFFER_NAMES = ("int_weight", "weights_scales", "int_indices", "fp_indices", "reduced_w", "fp_weight", "bias")
+_SWITCH_NAMES = ("fused", "six_bit_path", "six_bit_min_rows", "tile8_min_rows", "transient_tiled_copy", "sym_divisor", "dtype",
+                 "_row_major_released")
 
 
 def _concatenate_layers(layers):

@@ -149,6 +149,50 @@ def test_a_planned_group_sees_every_change(rows):
     assert shared.cur_group_elem == 0
 
 
+@pytest.mark.parametrize("name", ["int_weight", "weights_scales", "fp_weight", "reduced_w", "bias"])
+@pytest.mark.parametrize("change", [_rewrite, _assign])
+def test_both_paths_of_a_group_see_a_change_of_one_buffer(change, name):
+    from quik_amd.qlinear import SharedQuantizedInput
+    n_in, F, sizes = 1024 + 64, 64, (256, 64)
+    xs = {r: torch.randn(r, n_in, generator=torch.Generator().manual_seed(r)).half().to(DEV) for r in (1, 64)}
+    for before, after in (((64, 1), (1, 64)), ((1, 64), (64, 1)), ((64, 1), (64, 1))):
+        shared = SharedQuantizedInput(2)
+        mods = [_module(i, n, n_in, F, 4, shared, bias=True) for i, n in enumerate(sizes)]
+        alone = [_module(i, n, n_in, F, 4, bias=True) for i, n in enumerate(sizes)]
+        for rows in before + before:
+            for m in mods:
+                m(xs[rows])
+        assert shared._fast is not None
+        new = {name: getattr(_module(9, sizes[1], n_in, F, 4, bias=True), name)}
+        if change is _rewrite:
+            mods[1].load_state_dict(new, strict=False)
+        else:
+            mods[1].load_state_dict({name: new[name].clone()}, strict=False, assign=True)
+        alone[1].load_state_dict(new, strict=False)
+        for rows in after + after:
+            for m, a in zip(mods, alone):
+                assert _same(m(xs[rows]), a(xs[rows]))
+            assert shared._fast is not None
+
+
+def test_a_switch_of_one_member_is_seen():
+    from quik_amd.qlinear import SharedQuantizedInput
+    n_in, F, sizes = 1024 + 64, 64, (256, 64)
+    x = torch.randn(64, n_in, generator=torch.Generator().manual_seed(0)).half().to(DEV)
+    shared = SharedQuantizedInput(2)
+    mods = [_module(i, n, n_in, F, 4, shared) for i, n in enumerate(sizes)]
+    alone = [_module(i, n, n_in, F, 4) for i, n in enumerate(sizes)]
+    for switch in (None, "fused", "fuse_shared_groups"):
+        if switch is not None:
+            for m in (mods[1], alone[1]):
+                setattr(m, switch, False)
+        for _ in range(2):
+            assert all(_same(m(x), a(x)) for m, a in zip(mods, alone))
+        assert switch is None or "fast" not in mods[1]._descs
+        for m in (mods[1], alone[1]):
+            m.fused = m.fuse_shared_groups = True
+
+
 def test_interposed_inputs_stay_with_the_python_functions():
     from torch.utils._python_dispatch import TorchDispatchMode
     import quik

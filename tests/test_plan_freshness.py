@@ -12,7 +12,7 @@ import torch
 
 from quik_amd import _lib as L
 from quik_amd import asymmetric, matmul, qlinear
-from quik_amd.qlinear import MixedQLinear
+from quik_amd.qlinear import MixedQLinear, SharedQuantizedInput
 
 N, N_IN, F = 24, 160, 32
 DECODE, PREFILL = 1, 64     # row-major and tile-ordered path
@@ -20,7 +20,7 @@ DECODE, PREFILL = 1, 64     # row-major and tile-ordered path
 
 class Binding:
     def __init__(self):
-        self.calls, self.packed, self.plans = [], {}, []
+        self.calls, self.packed, self.plans, self.groups = [], {}, [], 0
 
     # the library
     def quik_layer_workspace_bytes(self, desc, rows):
@@ -37,6 +37,10 @@ class Binding:
         return w6
 
     # the front end
+    def group(self, shared, fused, plan, members):
+        self.groups += 1
+        return object()
+
     def plan(self, module, names, row, tiled, tiled_from, device, bf16, dev, splitk, keep):
         self.plans.append([None if b is None else L.QuikLayer.from_buffer_copy(b) for b in (row, tiled)])
         return object()
@@ -62,9 +66,9 @@ def binding(monkeypatch):
     return b
 
 
-def layer(seed):
+def layer(seed, shared=None):
     g = torch.Generator().manual_seed(seed)
-    m = MixedQLinear(N_IN, N, fp_features_num=F)
+    m = MixedQLinear(N_IN, N, shared, fp_features_num=F)
     perm = torch.randperm(N_IN, generator=g)
     m.int_indices.copy_(perm[F:].sort()[0])
     m.fp_indices.copy_(perm[:F])
@@ -151,3 +155,72 @@ def test_no_tiled_copy_stays_with_the_transient_policy(binding, monkeypatch, fir
             assert len(binding.plans) == made and "fast" not in m._descs
         else:
             assert binding.plans[-1][1] is None
+
+
+MEMBER_BUFFERS = ("int_weight", "weights_scales", "fp_weight", "reduced_w", "bias")
+
+
+def round_of(b, shared, mods, rows):
+    """One round of the group's members; the fused layer it ran through, or None."""
+    for m in mods:
+        out = shared.group_forward(m, torch.zeros(rows, N_IN, dtype=torch.float16))
+        if out is None:
+            return None
+        assert out.shape == (rows, m.out_features)
+    fused = shared._fused
+    for name in MEMBER_BUFFERS:
+        ts = [getattr(m, name) for m in mods]
+        if ts[0] is not None:
+            assert torch.equal(getattr(fused, name), torch.cat(ts, dim=1 if name == "reduced_w" else 0)), name
+    check(b, fused, b.calls[-1][1], rows >= 33)
+    for desc, t in zip(b.plans[-1], (False, True)):
+        if desc is not None:
+            check(b, fused, desc, t)
+    return fused
+
+
+@pytest.mark.parametrize("how", ["written", "assigned", "loaded"])
+@pytest.mark.parametrize("name", MEMBER_BUFFERS + ("fp_indices",))
+def test_a_group_sees_every_buffer_of_its_members(binding, monkeypatch, name, how):
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    for orders in itertools.product((DECODE, PREFILL), repeat=3):
+        shared = SharedQuantizedInput(2)
+        mods = [layer(0, shared), layer(0, shared)]
+        for rows in orders[:2]:
+            assert round_of(binding, shared, mods, rows) is not None
+        for m, seed in ((mods[1], 1), (mods[0], 2)):       # one member, then the other
+            new = getattr(layer(seed), name).clone()
+            if how == "written":
+                getattr(m, name).copy_(new)
+            elif how == "assigned":
+                setattr(m, name, new)
+            else:
+                m.load_state_dict({name: new}, assign=True, strict=False)
+            for rows in orders[1:]:
+                fused = round_of(binding, shared, mods, rows)
+                # (members with other outlier columns have no quantized input in common)
+                assert (fused is None) == (name == "fp_indices"), (name, how)
+
+
+@pytest.mark.parametrize("switch", [("fused", False), ("fuse_shared_groups", False), ("sym_divisor", 7.0), ("six_bit_path", False),
+                                    ("transient_tiled_copy", True)])
+def test_a_group_sees_the_switches_of_its_members(binding, monkeypatch, switch):
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    name, value = switch
+    shared = SharedQuantizedInput(2)
+    mods = [layer(0, shared), layer(0, shared)]
+    for rows in (DECODE, PREFILL):
+        round_of(binding, shared, mods, rows)
+    assert all("fast" in m._descs for m in mods)
+    for k, m in enumerate(mods):
+        setattr(m, name, value)
+        made = binding.groups
+        fused = round_of(binding, shared, mods, DECODE)
+        if name == "fuse_shared_groups":                  # the member's own forward asks for this one
+            assert binding.groups == made and "fast" not in m._descs and shared._fast is None
+        elif name == "fused" or (k == 0 and name in ("sym_divisor", "six_bit_path")):
+            assert fused is None                          # the members differ, or one replays the op sequence
+        elif name != "transient_tiled_copy" or k == 0:
+            assert getattr(fused, name) == value
+    if name == "transient_tiled_copy":
+        assert round_of(binding, shared, mods, PREFILL).weight_bytes()["tiled"] == 0
