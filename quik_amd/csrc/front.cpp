@@ -21,6 +21,8 @@
 #include <cstdint>
 #include <cstring>
 #include <memory>
+#include <optional>
+#include <utility>
 #include <vector>
 
 #include "../../include/quik_hip.h"
@@ -37,6 +39,10 @@ struct PyRef {  // owned reference
   PyRef(PyRef &&o) noexcept : p(o.p) { o.p = nullptr; }
   PyRef(const PyRef &) = delete;
   PyRef &operator=(const PyRef &) = delete;
+  PyRef &operator=(PyRef &&o) noexcept {
+    std::swap(p, o.p);
+    return *this;
+  }
   ~PyRef() { Py_XDECREF(p); }
 };
 
@@ -51,11 +57,13 @@ unsigned type_tag(PyTypeObject *t) {
   return t->tp_version_tag;
 }
 
+// What was found under `name` in the module's _buffers: no tensor, or one whose object and storage are known weakly (a plan
+// keeps no weights alive, and a tensor or block that got the address of a freed one is another), with address and version.
 struct Buffer {
-  PyRef name, tensor;  // tensor: the object (or None) found under `name` in the module's _buffers
+  PyRef name, weak;  // weak: the tensor's weak reference, or what stood in its place (None, or nothing)
+  std::optional<c10::weak_intrusive_ptr<c10::StorageImpl>> storage;  // of a tensor
   const void *data = nullptr;
   uint32_t version = 0;
-  bool present = false;
 };
 
 const void *data_of(const at::Tensor &t) { return t.unsafeGetTensorImpl()->data(); }
@@ -64,14 +72,17 @@ uint32_t version_of(const at::Tensor &t) { return t.unsafeGetTensorImpl()->versi
 bool snapshot(PyObject *buffers, PyObject *names, std::vector<Buffer> &out) {
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(names); ++i) {
     PyObject *name = PyTuple_GET_ITEM(names, i), *t = PyDict_GetItemWithError(buffers, name);
-    Buffer b{PyRef(name), PyRef(t)};
+    Buffer b{PyRef(name), PyRef()};
     if (t && t != Py_None) {
       if (!THPVariable_CheckExact(t)) return false;
       const at::Tensor &v = THPVariable_Unpack(t);
-      if (v.is_inference()) return false;
-      b.present = true;
+      if (v.is_inference() || !v.has_storage()) return false;
+      if (!(b.weak.p = PyWeakref_NewRef(t, nullptr))) return false;
+      b.storage.emplace(v.storage().getWeakStorageImpl());
       b.data = v.numel() ? data_of(v) : nullptr;
       b.version = version_of(v);
+    } else {
+      b.weak = PyRef(t);
     }
     out.push_back(std::move(b));
   }
@@ -83,14 +94,19 @@ PyObject *dict_of(PyObject *o) {
   return d ? *d : nullptr;
 }
 
-// the module's buffers are the tensors they were: same objects, same addresses, not written in place since
+// the module's buffers are the tensors they were: same objects, storages and addresses, not written in place since
 bool unchanged(PyObject *module_dict, const std::vector<Buffer> &bufs) {
   PyObject *buffers = PyDict_GetItemWithError(module_dict, s_buffers);
   if (!buffers || !PyDict_Check(buffers)) return false;
   for (const Buffer &b : bufs) {
-    if (PyDict_GetItemWithError(buffers, b.name.p) != b.tensor.p) return false;
-    if (!b.present) continue;
-    const at::Tensor &v = THPVariable_Unpack(b.tensor.p);
+    PyObject *t = PyDict_GetItemWithError(buffers, b.name.p);
+    if (!b.storage) {
+      if (t != b.weak.p) return false;
+      continue;
+    }
+    if (!t || t == Py_None || PyWeakref_GetObject(b.weak.p) != t) return false;
+    const at::Tensor &v = THPVariable_Unpack(t);
+    if (!v.has_storage() || v.storage().unsafeGetStorageImpl() != b.storage->_unsafe_get_target()) return false;
     if (version_of(v) != b.version || (v.numel() ? data_of(v) : nullptr) != b.data) return false;
   }
   return true;
@@ -329,7 +345,7 @@ PyObject *py_group_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // plan(module, names, row_desc, tiled_desc, tiled_from, device_index, is_bf16, device, splitk_fn, keep)
-PyObject *py_plan(PyObject *, PyObject *args) {
+PyObject *plan(PyObject *args) {
   PyObject *module, *names, *row, *tiled, *device, *fn, *keep;
   long long from;
   int dev, bf16;
@@ -355,8 +371,12 @@ PyObject *py_plan(PyObject *, PyObject *args) {
                        [](PyObject *c) { delete static_cast<Plan *>(PyCapsule_GetPointer(c, kPlanName)); });
 }
 
+PyObject *py_plan(PyObject *, PyObject *args) {
+  return guarded([&] { return plan(args); });
+}
+
 // group(shared_weakref, fused_module, fused_plan, ((weakref, key, out_features, names), ...))
-PyObject *py_group(PyObject *, PyObject *args) {
+PyObject *group(PyObject *args) {
   PyObject *shared, *fused, *inner, *members;
   if (!PyArg_ParseTuple(args, "OOOO!", &shared, &fused, &inner, &PyTuple_Type, &members)) return nullptr;
   if (!PyCapsule_IsValid(inner, kPlanName)) Py_RETURN_NONE;
@@ -379,6 +399,10 @@ PyObject *py_group(PyObject *, PyObject *args) {
   }
   return PyCapsule_New(g.release(), kGroupName,
                        [](PyObject *c) { delete static_cast<Group *>(PyCapsule_GetPointer(c, kGroupName)); });
+}
+
+PyObject *py_group(PyObject *, PyObject *args) {
+  return guarded([&] { return group(args); });
 }
 
 // ---------------------------------------------------------------------------------------------- stand-alone operations

@@ -22,6 +22,7 @@ import weakref
 
 import torch
 from torch import Tensor
+from torch.multiprocessing.reductions import StorageWeakRef
 
 from . import _lib as L
 from . import asymmetric, matmul, symmetric
@@ -54,6 +55,41 @@ class _PerObjectCache(dict):
 
     def __reduce__(self):
         return _PerObjectCache, ()
+
+
+class _Stamp:
+    """The state of the tensors (or None) that something cached was made from; `holds` asks if they are still in it.
+
+    Address and version alone are not enough: a freed block goes to the next tensor of its size, whose version may well
+    be the same.  So a stamp also knows the tensor and its storage, both weakly: it keeps no memory, and what took the
+    place of a freed one is another.  `values` are plain values that belong to the state (switches).  A copied stamp
+    holds for nothing, since the tensors beside it are copies too."""
+
+    __slots__ = ("items", "values")
+
+    def __init__(self, tensors=None, values=()):
+        self.items = None if tensors is None else tuple(
+            None if t is None else (weakref.ref(t), StorageWeakRef(t.untyped_storage()), t.data_ptr(), t._version)
+            for t in tensors)
+        self.values = values
+
+    def holds(self, tensors, values=()):
+        if self.items is None or self.values != values or len(self.items) != len(tensors):
+            return False
+        for item, t in zip(self.items, tensors):
+            if item is None or t is None:
+                if item is not t:
+                    return False
+            elif item[0]() is not t or t._version != item[3] or t.data_ptr() != item[2] or \
+                    t.untyped_storage()._cdata != item[1].cdata:
+                return False
+        return True
+
+    def __deepcopy__(self, memo):
+        return _Stamp()
+
+    def __reduce__(self):
+        return _Stamp, ()
 
 
 class SharedQuantizedInput:
@@ -104,11 +140,10 @@ class SharedQuantizedInput:
             self._outs = None
             self.cur_group_elem = 0
 
-    def _members_key(self, mods):
+    def _members_state(self, mods):
         """Everything of the members that the concatenated layer is made from: their buffers and their switches."""
-        return tuple((id(m),) + tuple(getattr(m, name) for name in _SWITCH_NAMES) +
-                     tuple(None if t is None else (t.data_ptr(), t._version)
-                           for t in (m._buffers.get(name) for name in _BUFFER_NAMES)) for m in mods)
+        return ([m._buffers.get(name) for m in mods for name in _BUFFER_NAMES],
+                tuple((id(m),) + tuple(getattr(m, name) for name in _SWITCH_NAMES) for m in mods))
 
     def _fused_layer(self):
         """The members' weights as one MixedQLinear (None when the group is not complete or not compatible).  Built
@@ -117,10 +152,8 @@ class SharedQuantizedInput:
         mods = [r() for r in self._members]
         if len(mods) != self.group_size or any(m is None for m in mods) or self.group_size < 2:
             return None
-        if self._fused is not None and self._fused is not False and self._fused_key == self._members_key(mods):
-            return self._fused
-        if self._fused is False and self._fused_key == self._members_key(mods):
-            return None
+        if self._fused is not None and self._fused_key.holds(*self._members_state(mods)):
+            return self._fused or None
         first = mods[0]
         ok = all(m.fused and not m._row_major_released and m.int_features_num > 0 and m.int_weight.is_cuda and
                  m.int_weight.device == first.int_weight.device and m.in_features == first.in_features and
@@ -132,7 +165,7 @@ class SharedQuantizedInput:
         ok = ok and all(torch.equal(m.fp_indices, first.fp_indices) and torch.equal(m.int_indices, first.int_indices)
                         for m in mods[1:])
         if not ok:
-            self._fused, self._fused_key = False, self._members_key(mods)
+            self._fused, self._fused_key = False, _Stamp(*self._members_state(mods))
             for m in mods:      # (plans of an earlier round keep that round's concatenated buffers)
                 m._descs.pop("fast", None)
             return None
@@ -156,7 +189,7 @@ class SharedQuantizedInput:
             m._w6 = m._w6_key = None      # a member's own tile-ordered copy is not read while the group serves it
             m._descs.clear()
             lo = hi
-        self._fused, self._fused_key = fused, self._members_key(mods)
+        self._fused, self._fused_key = fused, _Stamp(*self._members_state(mods))
         self._split = [m.out_features for m in mods]
         return fused
 
@@ -297,6 +330,12 @@ class MixedQLinear(torch.nn.Module):
                     shared._fast = None
         super().__setattr__(name, value)
 
+    def __setstate__(self, state):
+        super().__setstate__(state)
+        for name in ("_colmap_key", "_w6_key"):     # (older files hold addresses there)
+            if not isinstance(self.__dict__.get(name), _Stamp):
+                self.__dict__[name] = _Stamp()
+
     def _apply(self, fn, recurse=True):
         """`.to()` / `.half()` / `.bfloat16()` convert the floating-point buffers; `dtype` (a plain attribute in the
         reference, qlinear.py:52, fixed at construction) follows them, so that a converted module computes in the
@@ -306,13 +345,13 @@ class MixedQLinear(torch.nn.Module):
             self.dtype = self.weights_scales.dtype
         return out
 
-    # -- cached column map: rebuilt when the index buffers move or are written in place
+    # -- cached column map: rebuilt when the index buffers are replaced or written in place
     def _column_map(self):
-        key = (self.int_indices.data_ptr(), self.fp_indices.data_ptr(), self.int_indices._version,
-               self.fp_indices._version, self.int_indices.device)
-        if self._colmap is None or self._colmap_key != key:
+        state = (self.int_indices, self.fp_indices)
+        if self._colmap is None or not self._colmap_key.holds(state):
+            stamp = _Stamp(state)
             self._colmap = asymmetric.build_colmap(self.int_indices, self.fp_indices, self.in_features)
-            self._colmap_key = key
+            self._colmap_key = stamp
             self._streams = None
         return self._colmap
 
@@ -351,11 +390,11 @@ class MixedQLinear(torch.nn.Module):
         if self.transient_tiled_copy:    # a fresh buffer per call, never kept
             self._w6 = self._w6_key = None
             return self._pack_tiled(fp_w)
-        key = (self.int_weight.data_ptr(), self.int_weight._version, fp_w.data_ptr(), fp_w._version,
-               self.int_weight.device, self._column_map().data_ptr())
-        if self._w6 is None or self._w6_key != key:
+        state = (self.int_weight, fp_w if self.fp_features_num > 0 else None, self.int_indices, self.fp_indices)
+        if self._w6 is None or not self._w6_key.holds(state):
+            stamp = _Stamp(state)
             self._w6 = self._pack_tiled(fp_w)
-            self._w6_key = key
+            self._w6_key = stamp
         return self._w6
 
     # -- which copies of the weights stay resident
@@ -417,18 +456,17 @@ class MixedQLinear(torch.nn.Module):
 
     # -- one library call per forward (quik_layer_forward): the layer's buffers described once
     def _descriptor_source(self):
-        """(the buffers a descriptor is made from, the key of their state): a cached descriptor holds for an equal key."""
+        """The state that a descriptor is made from: buffers, switches."""
         bufs = (self.int_weight, self.weights_scales, self.int_indices, self.fp_indices,
                 self.reduced_w if not self.symmetric else None, self.fp_weight if self.fp_features_num > 0 else None,
                 self.bias)
         # (the scalar switches below are baked into the descriptor too: changing one after a forward rebuilds it)
-        return bufs, tuple((b.data_ptr(), b._version) if b is not None else None for b in bufs) + \
-            (self.six_bit_min_rows, self.tile8_min_rows, float(self.sym_divisor), bool(self.six_bit_path))
+        return bufs, (self.six_bit_min_rows, self.tile8_min_rows, float(self.sym_divisor), bool(self.six_bit_path), self.dtype)
 
     def _descriptor(self, tiled):
         """(ctypes quik_layer, workspace sizes by row count) for this module, with or without the tile-ordered weight
-        copy; cached, rebuilt when a buffer moves or is written in place."""
-        bufs, key = self._descriptor_source()
+        copy; cached, rebuilt when a buffer is replaced or written in place."""
+        bufs, switches = self._descriptor_source()
         transient = self.transient_tiled_copy and not self._row_major_released
         if transient:     # (set after a prefill: the copy that one kept goes)
             self._descs.pop(True, None)
@@ -442,7 +480,8 @@ class MixedQLinear(torch.nn.Module):
             d._keep = w6     # (alive until the caller drops the descriptor, i.e. behind the launch)
             return d, self._descs.setdefault("transient_sizes", {})
         entry = self._descs.get(tiled)
-        if entry is None or entry[0] != key:
+        if entry is None or not entry[0].holds(bufs, switches):
+            stamp = _Stamp(bufs, switches)
             w6 = self._weight6() if tiled else None
             colmap = self._column_map()
             d = L.QuikLayer()
@@ -460,7 +499,7 @@ class MixedQLinear(torch.nn.Module):
             d.fp_weight = bufs[5].data_ptr() if bufs[5] is not None and bufs[5].numel() > 0 else None
             d.bias = bufs[6].data_ptr() if bufs[6] is not None and bufs[6].numel() > 0 else None
             d.tiled_weight = w6.data_ptr() if w6 is not None else None
-            entry = self._descs[tiled] = (key, d, {}, (colmap, w6))   # the tensors the pointers refer to stay alive
+            entry = self._descs[tiled] = (stamp, d, {}, (colmap, w6))   # the tensors the pointers refer to stay alive
         return entry[1], entry[2]
 
     def _forward_one_call(self, x2):
@@ -498,9 +537,9 @@ class MixedQLinear(torch.nn.Module):
             return        # (a substituted binding, a class-wide profiling hook: the Python path serves those)
         # A forward brings the descriptor of its own path up to date; the other path's may date from before the buffers
         # changed.  The plan compares the buffers with what they are now, so nothing later would find that out.
-        key = self._descriptor_source()[1]
+        state = self._descriptor_source()
         for t in (False, True):
-            if t in self._descs and self._descs[t][0] != key:
+            if t in self._descs and not self._descs[t][0].holds(*state):
                 del self._descs[t]
         row, til = self._descs.get(False), self._descs.get(True)
         if (til if tiled else row) is None:

@@ -90,7 +90,15 @@ def _move(mod, other):
     mod.to(DEV)
 
 
-@pytest.mark.parametrize("change", [_rewrite, _assign, _move])
+def _offload(mod, other):                                  # (the blocks given back are handed out again)
+    for name, b in mod.named_buffers():
+        b.data = b.data.cpu()
+    for name, b in mod.named_buffers():
+        b.data.copy_(getattr(other, name))
+        b.data = b.data.to(DEV)
+
+
+@pytest.mark.parametrize("change", [_rewrite, _assign, _move, _offload])
 @pytest.mark.parametrize("outliers", [1, 2])               # the same outlier columns as before, or others
 @pytest.mark.parametrize("before,after", [((64, 1), (1, 64)), ((1, 64), (64, 1)), ((64, 1), (64, 1)), ((64,), (1, 64))])
 @pytest.mark.parametrize("bits", [4, 8])
@@ -103,6 +111,16 @@ def test_both_paths_see_a_change_of_the_weights(bits, before, after, outliers, c
     change(mod, other)
     for rows in after + after:
         assert _same(mod(xs[rows]), other(xs[rows]))
+
+
+def test_a_plan_keeps_no_weights_alive():
+    mod = _module(0, 4096, 4096 + 64, 64, 4)
+    x = torch.randn(1, 4096 + 64, generator=torch.Generator().manual_seed(0)).half().to(DEV)
+    mod(x)
+    assert _planned(mod)
+    before, held = torch.cuda.memory_allocated(), mod.weight_bytes()["row_major"]
+    mod.cpu()
+    assert before - torch.cuda.memory_allocated() >= held
 
 
 @pytest.mark.parametrize("bits", [4, 8])

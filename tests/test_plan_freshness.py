@@ -4,8 +4,10 @@ A layer keeps one descriptor per path (row-major, tile-ordered), and a forward b
 library, the packing kernels and the front end are stand-ins on CPU tensors, so that the descriptors a plan receives can
 be compared with the module's buffers: addresses, and the contents that the tile-ordered operand was packed from.
 """
+import copy
 import ctypes
 import itertools
+import pickle
 
 import pytest
 import torch
@@ -20,7 +22,7 @@ DECODE, PREFILL = 1, 64     # row-major and tile-ordered path
 
 class Binding:
     def __init__(self):
-        self.calls, self.packed, self.plans, self.groups = [], {}, [], 0
+        self.calls, self.packed, self.plans, self.groups, self.packs = [], {}, [], 0, 0
 
     # the library
     def quik_layer_workspace_bytes(self, desc, rows):
@@ -34,6 +36,7 @@ class Binding:
     def pack(self, int_weight, fp_weight, colmap, *rest):
         w6 = torch.cat([int_weight.reshape(-1), fp_weight.contiguous().view(torch.uint8).reshape(-1), colmap])
         self.packed[w6.data_ptr()] = w6.clone()
+        self.packs += 1
         return w6
 
     # the front end
@@ -224,3 +227,68 @@ def test_a_group_sees_the_switches_of_its_members(binding, monkeypatch, switch):
             assert getattr(fused, name) == value
     if name == "transient_tiled_copy":
         assert round_of(binding, shared, mods, PREFILL).weight_bytes()["tiled"] == 0
+
+
+class Memory:
+    """Tensors over one piece of memory, as an allocator hands a freed block out again: same address, same version."""
+
+    def __init__(self, like):
+        self.bytes, self.like = bytearray(like.numel() * like.element_size()), (like.dtype, like.shape)
+
+    def tensor(self, values):
+        self.bytes[:] = values.contiguous().view(torch.uint8).numpy().tobytes()
+        return torch.frombuffer(self.bytes, dtype=self.like[0]).view(self.like[1])
+
+
+def set_attribute(m, name, memory, values):
+    setattr(m, name, None)
+    setattr(m, name, memory.tensor(values))
+
+
+def set_buffer(m, name, memory, values):          # (as Module.to and load hooks do)
+    m._buffers[name] = None
+    m._buffers[name] = memory.tensor(values)
+
+
+def set_data(m, name, memory, values):
+    getattr(m, name).data = torch.empty(0, dtype=values.dtype)
+    getattr(m, name).data = memory.tensor(values)
+
+
+@pytest.mark.parametrize("setter", [set_attribute, set_buffer, set_data])
+@pytest.mark.parametrize("name", MEMBER_BUFFERS + ("int_indices",))
+def test_a_buffer_that_got_the_address_of_a_freed_one(binding, name, setter):
+    m = layer(0)
+    memory = Memory(getattr(m, name))
+    setter(m, name, memory, getattr(m, name).clone())
+    for rows in (PREFILL, DECODE, PREFILL):
+        call(m, rows)
+    where = getattr(m, name).data_ptr()
+    setter(m, name, memory, getattr(layer(2), name))
+    assert getattr(m, name).data_ptr() == where
+    for rows in (DECODE, PREFILL, PREFILL):
+        call(m, rows)
+        check(binding, m, binding.calls[-1][1], rows >= 33)
+        for desc, t in zip(binding.plans[-1], (False, True)):
+            assert desc is None or check(binding, m, desc, t) is None
+
+
+def test_stamps_do_not_travel(binding):
+    m = layer(0)
+    call(m, PREFILL)
+    for other in (copy.deepcopy(m), pickle.loads(pickle.dumps(m))):
+        packs = binding.packs
+        call(other, PREFILL)
+        assert binding.packs > packs
+        check(binding, other, binding.calls[-1][1], True)
+
+
+def test_forwards_under_inference_mode(binding):
+    m = layer(0)
+    with torch.inference_mode():       # (what a forward makes for itself has no version there)
+        for rows in (PREFILL, DECODE, PREFILL):
+            call(m, rows)
+    packs = binding.packs
+    call(m, PREFILL)
+    assert binding.packs == packs
+    check(binding, m, binding.calls[-1][1], True)
