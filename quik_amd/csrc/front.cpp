@@ -46,7 +46,7 @@ struct PyRef {  // owned reference
   ~PyRef() { Py_XDECREF(p); }
 };
 
-PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_finish, *s_workspaces, *s_split_k;
+PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_finish, *s_workspaces, *s_split_k, *s_group_size;
 
 // A class keeps its version tag until one of its attributes (or of its bases') is set: methods and class-wide
 // switches are as they were when the plan was made.
@@ -134,9 +134,11 @@ struct Group {
     std::vector<Buffer> bufs;
     Member(PyObject *w, PyObject *k) : weak(w), key(k) {}
   };
-  PyRef shared_weak, fused, inner;  // inner: the fused layer's plan capsule
+  PyRef shared_weak, fused, inner, methods;  // inner: the fused layer's plan capsule; methods: names that the front end goes past
+  PyTypeObject *type = nullptr;              // of the shared object
+  unsigned tag = 0;
   std::vector<Member> members;
-  Group(PyObject *s, PyObject *f, PyObject *i) : shared_weak(s), fused(f), inner(i) {}
+  Group(PyObject *s, PyObject *f, PyObject *i, PyObject *m) : shared_weak(s), fused(f), inner(i), methods(m) {}
 };
 
 PyObject *fail(const char *op, int rc) {
@@ -294,6 +296,12 @@ PyObject *group_forward(PyObject *const *args, Py_ssize_t n) {
   PyObject *sd = shared && shared != Py_None ? dict_of(shared) : nullptr;
   if (!sd || PyDict_GetItemWithError(sd, s_fast) != args[0] || PyDict_GetItemWithError(sd, s_fused) != g->fused.p)
     Py_RETURN_NONE;
+  // the shared object is of the class it was, has no methods of its own, and the group is as large as its members
+  if (Py_TYPE(shared) != g->type || g->tag == 0 || type_tag(g->type) != g->tag) Py_RETURN_NONE;
+  for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(g->methods.p); ++i)
+    if (PyDict_GetItemWithError(sd, PyTuple_GET_ITEM(g->methods.p, i))) Py_RETURN_NONE;
+  PyObject *size = PyDict_GetItemWithError(sd, s_group_size);
+  if (!size || !PyLong_Check(size) || PyLong_AsSize_t(size) != g->members.size()) return none_or_error();
   if (current_gpu() != p->device) Py_RETURN_NONE;
   const at::Tensor *x = plain(args[3], p->device);
   if (!x || (x->dim() != 2 && x->dim() != 3)) Py_RETURN_NONE;
@@ -375,12 +383,16 @@ PyObject *py_plan(PyObject *, PyObject *args) {
   return guarded([&] { return plan(args); });
 }
 
-// group(shared_weakref, fused_module, fused_plan, ((weakref, key, out_features, names), ...))
+// group(shared_weakref, fused_module, fused_plan, method_names, ((weakref, key, out_features, names), ...))
 PyObject *group(PyObject *args) {
-  PyObject *shared, *fused, *inner, *members;
-  if (!PyArg_ParseTuple(args, "OOOO!", &shared, &fused, &inner, &PyTuple_Type, &members)) return nullptr;
-  if (!PyCapsule_IsValid(inner, kPlanName)) Py_RETURN_NONE;
-  auto g = std::make_unique<Group>(shared, fused, inner);
+  PyObject *shared, *fused, *inner, *methods, *members;
+  if (!PyArg_ParseTuple(args, "OOOO!O!", &shared, &fused, &inner, &PyTuple_Type, &methods, &PyTuple_Type, &members)) return nullptr;
+  PyObject *obj = PyCapsule_IsValid(inner, kPlanName) ? PyWeakref_GetObject(shared) : Py_None;
+  if (!obj) return nullptr;
+  if (obj == Py_None) Py_RETURN_NONE;
+  auto g = std::make_unique<Group>(shared, fused, inner, methods);
+  g->type = Py_TYPE(obj);
+  g->tag = type_tag(g->type);
   g->members.reserve(static_cast<size_t>(PyTuple_GET_SIZE(members)));
   for (Py_ssize_t i = 0; i < PyTuple_GET_SIZE(members); ++i) {
     PyObject *weak, *key, *names;
@@ -563,6 +575,7 @@ PyMODINIT_FUNC PyInit__front() {
   s_fused = PyUnicode_InternFromString("_fused");
   s_finish = PyUnicode_InternFromString("finish");
   s_workspaces = PyUnicode_InternFromString("_splitk_workspaces");
+  s_group_size = PyUnicode_InternFromString("group_size");
   s_split_k = PyUnicode_InternFromString("split_k");
   return PyModule_Create(&kModule);
 }

@@ -217,16 +217,27 @@ class SharedQuantizedInput:
     def _make_fast(self, mods, fused):
         """Hand the round just served by Python to the native front end: later rounds on unchanged members go through
         `_front.group_forward`, which every member finds under its own "fast" entry."""
+        self._fast = plan = None
         inner = fused._descs.get("fast")
-        if inner is None or inner[1] is not None or not all(m.fuse_shared_groups and m.shared_input is self for m in mods):
-            return
-        names = _BUFFER_NAMES
-        plan = _front.group(weakref.ref(self), fused, inner[0],
-                               tuple((r, id(m), m.out_features, names) for r, m in zip(self._members, mods)))
+        if inner is not None and inner[1] is None and _own_methods(self, _GROUP_METHODS) and \
+                all(m.fuse_shared_groups and m.shared_input is self for m in mods):
+            plan = _front.group(weakref.ref(self), fused, inner[0], tuple(_GROUP_METHODS),
+                                tuple((r, id(m), m.out_features, _BUFFER_NAMES) for r, m in zip(self._members, mods)))
         self._fast = plan
-        if plan is not None:
-            for i, m in enumerate(mods):
+        for i, m in enumerate(mods):
+            if plan is not None:
                 m._descs["fast"] = (plan, i)
+            else:
+                m._descs.pop("fast", None)
+
+
+# What a round or a forward calls on the way that the native front end goes past: a plan is made only where all of them are
+# the classes' own, so that an override (of a subclass, on the class, on one object) is called by every forward.
+_GROUP_METHODS = {name: SharedQuantizedInput.__dict__[name] for name in ("group_forward", "_fused_layer", "_members_state")}
+
+
+def _own_methods(obj, methods):
+    return all(getattr(getattr(obj, name), "__func__", None) is f for name, f in methods.items())
 
 
 _BUFFER_NAMES = ("int_weight", "weights_scales", "int_indices", "fp_indices", "reduced_w", "fp_weight", "bias")
@@ -535,6 +546,8 @@ class MixedQLinear(torch.nn.Module):
         self._descs.pop("fast", None)     # (a plan keeps the tensors it was made from)
         if L.load() is not L._lib or type(self).mid_event is not None or self.mid_event is not None:
             return        # (a substituted binding, a class-wide profiling hook: the Python path serves those)
+        if not _own_methods(self, _LAYER_METHODS):
+            return
         # A forward brings the descriptor of its own path up to date; the other path's may date from before the buffers
         # changed.  The plan compares the buffers with what they are now, so nothing later would find that out.
         state = self._descriptor_source()
@@ -705,6 +718,11 @@ class MixedQLinear(torch.nn.Module):
         if mod.fp_features_num > 0:
             mod.fp_weight.copy_(weight_matrix[:, fp_indices.to(dev)].to(weight_matrix.dtype))
         return mod
+
+
+_LAYER_METHODS = {name: MixedQLinear.__dict__[name] for name in
+                  ("_forward_one_call", "_six_bit_ok", "_descriptor", "_descriptor_source", "_weight6", "_pack_tiled",
+                   "_whole_steps", "_column_map", "_streams_flag")}
 
 
 class FusedMixedQLinearGroup(torch.nn.Module):

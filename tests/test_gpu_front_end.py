@@ -20,6 +20,8 @@ def _module(seed, N, n_in, F, bits, shared=None, bias=False, outlier_seed=1):
     lo, hi = (-8, 8) if bits == 4 else (-127, 128)
     W = torch.from_numpy((rng.integers(lo, hi, (N, n_in)) * s_w.float().numpy()).astype(np.float16))
     lin = torch.nn.Linear(n_in, N, bias=bias, dtype=torch.float16)
+    if bias:
+        lin.bias.data = torch.from_numpy(rng.standard_normal(N).astype(np.float16))
     return MixedQLinear.from_float(lin, W, s_w, shared, fi, bits=bits).to(DEV)
 
 
@@ -69,8 +71,9 @@ def test_a_planned_forward_sees_every_change(rows, bits):
     real = MixedQLinear._forward_one_call
     try:
         MixedQLinear._forward_one_call = lambda self, x2: calls.append(1) or real(self, x2)
-        mod(x)
-        assert calls == [1]
+        for n in (1, 2, 3):
+            mod(x)
+            assert calls == [1] * n
     finally:
         MixedQLinear._forward_one_call = real
     assert MixedQLinear.six_bit_min_rows == keep
@@ -191,6 +194,32 @@ def test_both_paths_of_a_group_see_a_change_of_one_buffer(change, name):
             for m, a in zip(mods, alone):
                 assert _same(m(xs[rows]), a(xs[rows]))
             assert shared._fast is not None
+
+
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+def test_an_override_of_the_group_is_called_by_every_round(where, monkeypatch):
+    from quik_amd.qlinear import SharedQuantizedInput
+    n_in, F, sizes, calls = 1024 + 64, 64, (256, 64), []
+    real = SharedQuantizedInput.group_forward
+
+    def override(self, *args):
+        calls.append(1)
+        return real(self, *args)
+
+    x = torch.randn(1, n_in, generator=torch.Generator().manual_seed(0)).half().to(DEV)
+    shared = SharedQuantizedInput(2)
+    mods = [_module(i, n, n_in, F, 4, shared) for i, n in enumerate(sizes)]
+    first = [m(x) for m in mods]
+    assert shared._fast is not None and all(_same(m(x), f) for m, f in zip(mods, first))
+    if where == "subclass":
+        shared.__class__ = type("Sub", (SharedQuantizedInput,), {"group_forward": override})
+    elif where == "class":
+        monkeypatch.setattr(SharedQuantizedInput, "group_forward", override)
+    else:
+        shared.group_forward = override.__get__(shared)
+    for n in (1, 2, 3):
+        assert all(_same(m(x), f) for m, f in zip(mods, first))
+        assert len(calls) == 2 * n
 
 
 def test_a_switch_of_one_member_is_seen():

@@ -40,7 +40,7 @@ class Binding:
         return w6
 
     # the front end
-    def group(self, shared, fused, plan, members):
+    def group(self, shared, fused, plan, methods, members):
         self.groups += 1
         return object()
 
@@ -292,3 +292,51 @@ def test_forwards_under_inference_mode(binding):
     call(m, PREFILL)
     assert binding.packs == packs
     check(binding, m, binding.calls[-1][1], True)
+
+
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+@pytest.mark.parametrize("method", ["_forward_one_call", "_six_bit_ok", "_descriptor", "_weight6", "_column_map"])
+def test_an_override_is_called_by_every_forward(binding, monkeypatch, method, where):
+    real, seen = getattr(MixedQLinear, method), []
+
+    def override(self, *args):
+        seen.append(method)
+        return real(self, *args)
+
+    m = layer(0)
+    for rows in (PREFILL, DECODE):
+        call(m, rows)
+    if where == "subclass":
+        m.__class__ = type("Sub", (MixedQLinear,), {method: override})
+    elif where == "class":
+        monkeypatch.setattr(MixedQLinear, method, override)
+    else:
+        setattr(m, method, override.__get__(m))
+    for rows in (PREFILL, DECODE, PREFILL):
+        del seen[:]
+        call(m, rows)
+        assert "fast" not in m._descs
+        assert seen or method in ("_weight6", "_column_map")    # (what a descriptor is made from once)
+
+
+@pytest.mark.parametrize("where", ["subclass", "class", "instance"])
+@pytest.mark.parametrize("method", ["group_forward", "_fused_layer"])
+def test_an_override_of_the_group_is_called_by_every_round(binding, monkeypatch, method, where):
+    monkeypatch.setattr(torch.Tensor, "is_cuda", True, raising=False)
+    real = getattr(SharedQuantizedInput, method)
+
+    def override(self, *args):
+        return real(self, *args)
+
+    shared = SharedQuantizedInput(2)
+    mods = [layer(0, shared), layer(0, shared)]
+    round_of(binding, shared, mods, DECODE)
+    if where == "subclass":
+        shared.__class__ = type("Sub", (SharedQuantizedInput,), {method: override})
+    elif where == "class":
+        monkeypatch.setattr(SharedQuantizedInput, method, override)
+    else:
+        setattr(shared, method, override.__get__(shared))
+    made = binding.groups
+    round_of(binding, shared, mods, DECODE)
+    assert binding.groups == made and shared._fast is None
