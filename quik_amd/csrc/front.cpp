@@ -178,7 +178,7 @@ const at::Tensor *plain(PyObject *o, c10::DeviceIndex dev) {
 // (no error set) or failed (error set).
 bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &x, at::IntArrayRef shape, at::Tensor &out) {
   PyObject *dict = dict_of(module);
-  if (!dict || Py_TYPE(module) != p.type || p.tag == 0 || type_tag(p.type) != p.tag || !unchanged(dict, p.bufs)) return false;
+  if (!dict || Py_TYPE(module) != p.type || p.tag == 0 || type_tag(p.type) != p.tag) return false;
   const quik_layer &probe = p.has_row ? p.row : p.tiled;
   const int64_t n_in = probe.in_features;
   if (x.scalar_type() != p.dtype || x.size(-1) != n_in || x.numel() == 0 ||
@@ -188,14 +188,6 @@ bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &
   const bool tiled = rows >= p.tiled_from;
   if (tiled ? !p.has_tiled : !p.has_row) return false;
   const quik_layer &l = tiled ? p.tiled : p.row;
-  void *mid = nullptr;
-  if (PyObject *ev = PyDict_GetItemWithError(dict, s_mid_event); ev && ev != Py_None) {  // profiling hook of the module
-    PyObject *raw = PyObject_GetAttr(ev, s_cuda_event);
-    if (!raw) return false;
-    mid = PyLong_AsVoidPtr(raw);
-    Py_DECREF(raw);
-    if (PyErr_Occurred() || PyDict_SetItem(dict, s_mid_event, Py_None) < 0) return false;
-  }
   void *sk = nullptr;
   int64_t sk_bytes = 0;
   PyRef sk_tensor;
@@ -227,10 +219,20 @@ bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &
       }
     }
   }
+  // (no Python code runs from here to the launch: what the buffers are now is what the kernels read)
+  if (!unchanged(dict, p.bufs)) return false;
   try {
     const int64_t nbytes = quik_layer_workspace_bytes(&l, rows);
     const c10::DataPtr ws = c10::hip::HIPCachingAllocator::get()->allocate(static_cast<size_t>(nbytes));
     out = new_empty(shape, p.dtype, p.device);
+    void *mid = nullptr;  // profiling hook of the module, taken once nothing sends the call back to the Python function
+    const PyRef ev(PyDict_GetItemWithError(dict, s_mid_event));
+    if (ev.p && ev.p != Py_None) {
+      PyRef raw;
+      if (!(raw.p = PyObject_GetAttr(ev.p, s_cuda_event))) return false;
+      mid = PyLong_AsVoidPtr(raw.p);
+      if (PyErr_Occurred() || PyDict_SetItem(dict, s_mid_event, Py_None) < 0) return false;
+    }
     const int rc = quik_layer_forward(&l, data_of(x), rows, ws.get(), nbytes, sk, sk_bytes, const_cast<void *>(data_of(out)), mid,
                                       stream_of(p.device));
     if (rc != QUIK_OK) {

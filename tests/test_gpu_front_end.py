@@ -142,6 +142,31 @@ def test_transient_policy_set_after_a_prefill(bits):
         assert _same(mod(xs[rows]), other(xs[rows]))
 
 
+def test_a_call_that_goes_back_keeps_its_event():
+    N, n_in, rows = 16384, 1024, 8192
+    mod = _module(0, N, n_in, 0, 4)
+    x = torch.zeros(rows, n_in, dtype=torch.float16, device=DEV)
+    mod(x[:64])
+    assert _planned(mod)
+    event = torch.cuda.Event()
+    event.record()
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    total = torch.cuda.get_device_properties(0).total_memory
+    try:                                                   # no room for the 256 MB result
+        torch.cuda.set_per_process_memory_fraction((torch.cuda.memory_reserved() + (64 << 20)) / total)
+        mod.mid_event = event
+        with pytest.raises(torch.OutOfMemoryError):
+            mod(x)
+        assert mod.mid_event is event and _planned(mod)
+    finally:
+        torch.cuda.set_per_process_memory_fraction(1.0)
+    mod(x)
+    assert mod.mid_event is None
+    torch.cuda.synchronize()
+    assert event.query()
+
+
 @pytest.mark.parametrize("rows", [1, 40])
 def test_a_planned_group_sees_every_change(rows):
     from quik_amd.qlinear import SharedQuantizedInput
