@@ -3,6 +3,8 @@ from __future__ import annotations
 
 import ctypes
 import os
+import sys
+import warnings
 
 import torch
 
@@ -91,21 +93,36 @@ def load():
     return _lib
 
 
+class _NoFront:
+    """Stands where the front end cannot be used: every call is left to the Python functions, as the front end leaves those
+    that it does not serve."""
+    def __getattr__(self, name):
+        return lambda *args: None
+
+
 _front = None
 
 
 def front():
-    """The native host front end (csrc/front.cpp); like the library it loads, there is no fallback when it is missing."""
+    """The native host front end (csrc/front.cpp): the hot calls' host work in one crossing.  It is built for one Python and
+    one torch; without it, or with one built for others, every call runs through the Python functions on the same
+    library, with a warning (a small call then takes some 10 us longer)."""
     global _front
     if _front is None:
         load()
+        why, here = None, f"python {sys.version_info[0]}.{sys.version_info[1]} torch {torch.__version__}"
         try:
             from . import _front as module
+            if module.built_for != here:
+                why = f"it was built for {module.built_for}, this is {here}"
         except ImportError as e:
-            raise RuntimeError(
-                f"{_HERE}/_front.so cannot be loaded ({e}): build it with `make -C quik_amd/csrc` (or "
-                "__graft_entry__.build())") from e
-        _front = module
+            why = str(e)
+        if why is None:
+            _front = module
+        else:
+            _front = _NoFront()
+            warnings.warn(f"{_HERE}/_front.so cannot be used ({why}): quik_amd's calls take longer on the host; build it with "
+                          "`make -C quik_amd/csrc` (or __graft_entry__.build())", RuntimeWarning, stacklevel=2)
     return _front
 
 

@@ -579,5 +579,7 @@ PyMODINIT_FUNC PyInit__front() {
   s_workspaces = PyUnicode_InternFromString("_splitk_workspaces");
   s_group_size = PyUnicode_InternFromString("group_size");
   s_split_k = PyUnicode_InternFromString("split_k");
-  return PyModule_Create(&kModule);
+  PyObject *m = PyModule_Create(&kModule);
+  if (m && PyModule_AddStringConstant(m, "built_for", QUIK_BUILT_FOR) < 0) Py_CLEAR(m);
+  return m;
 }

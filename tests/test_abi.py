@@ -5,6 +5,7 @@ import ctypes
 import inspect
 import os
 import re
+import warnings
 
 import pytest
 
@@ -256,3 +257,37 @@ def test_layer_forward_validates_without_gpu():
     assert fwd(d, ws=odd) == -4
     assert fwd(d, nb=1024) == -6                             # workspace too small
     assert fwd(layer(symmetric=1, dtype=L.QUIK_BF16)) == -3  # symmetric activations are fp16
+
+
+def test_front_end_is_built_for_this_python_and_torch():
+    from quik_amd import _lib as L
+    assert L.front().__name__ == "quik_amd._front"
+
+
+@pytest.mark.parametrize("why", ["missing", "built for others"])
+def test_operations_run_without_the_front_end(monkeypatch, why):
+    """The Python functions answer then (here: with their own error for tensors that are not on a GPU)."""
+    import sys
+    import torch
+    import quik
+    import quik_amd
+    from quik_amd import _lib as L
+    monkeypatch.setattr(L, "_front", None)
+    if why == "missing":
+        monkeypatch.delattr(quik_amd, "_front", raising=False)
+        monkeypatch.setitem(sys.modules, "quik_amd._front", None)
+    else:
+        monkeypatch.setattr(L.front(), "built_for", "python 2.7 torch 0.1")
+        monkeypatch.setattr(L, "_front", None)
+    a = torch.zeros(4, 32, dtype=torch.uint8)
+    with pytest.warns(RuntimeWarning, match="_front.so cannot be used"):
+        with pytest.raises(RuntimeError, match="on a CUDA"):
+            quik.matmul.int4Matmul(a, a)
+    i = torch.arange(32)
+    with warnings.catch_warnings():
+        warnings.simplefilter("error")                    # said once
+        for call in (lambda: quik.asymmetric.quantize(a.half(), i, i[:0], 4),
+                     lambda: quik.asymmetric.dequantize(a.int(), a, a, a, a, 4),
+                     lambda: quik.asymmetric.int4FusedDequantize(a, a, a, a, 8.0, a, a, a)):
+            with pytest.raises(RuntimeError, match="on a CUDA"):
+                call()

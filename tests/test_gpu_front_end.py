@@ -265,6 +265,27 @@ def test_a_switch_of_one_member_is_seen():
             m.fused = m.fuse_shared_groups = True
 
 
+def test_same_bits_without_the_front_end(monkeypatch):
+    import quik
+    from quik_amd import _lib as L
+    mod = _module(0, 264, 1024 + 64, 64, 4)
+    xs = [torch.randn(r, 1024 + 64, generator=torch.Generator().manual_seed(r)).half().to(DEV) for r in (1, 64)]
+
+    def ops(x):
+        q, meta, fp_x = quik.asymmetric.quantize(x, mod.int_indices, mod.fp_indices, 4)
+        acc = quik.matmul.int4Matmul(q, mod.int_weight)
+        y = torch.nn.functional.linear(fp_x, mod.fp_weight)
+        return [q, meta, fp_x, acc, quik.asymmetric.dequantize(acc, meta, mod.weights_scales, mod.reduced_w, y, 4)]
+    want = [(mod(x), ops(x)) for x in xs]
+    assert _planned(mod)
+    monkeypatch.setattr(L, "_front", L._NoFront())
+    bare = _module(0, 264, 1024 + 64, 64, 4)
+    for x, (out, parts) in zip(xs, want):
+        for _ in range(2):
+            assert _same(bare(x), out) and not _planned(bare)
+        assert all(torch.equal(a, b) for a, b in zip(ops(x), parts))
+
+
 def test_interposed_inputs_stay_with_the_python_functions():
     from torch.utils._python_dispatch import TorchDispatchMode
     import quik
