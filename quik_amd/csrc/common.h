@@ -11,6 +11,14 @@ namespace quik {
 // Last HIP error text, for quik_last_hip_error().
 void set_last_hip_error(hipError_t e);
 int check_launch();  // QUIK_OK or QUIK_ERR_LAUNCH after a kernel launch
+constexpr int kLdsBytes = 160 * 1024;  // per CU, and the most one workgroup may ask for
+// Raises the kernel's dynamic LDS limit to `smem` bytes: once per kernel and device, with one size per kernel (the most that
+// any of its launches asks for).  Nothing to do up to 48 KB.
+int prepare_lds(const void *kern, int smem);
+template <typename K>
+int prepare(K kern, int smem) {
+  return smem > 48 * 1024 ? prepare_lds(reinterpret_cast<const void *>(kern), smem) : QUIK_OK;
+}
 int num_cus();       // compute units of the GPU (asked once per process; 256 when no device answers)
 
 inline hipStream_t as_stream(void *s) { return reinterpret_cast<hipStream_t>(s); }

@@ -39,49 +39,6 @@ constexpr int kMaxCUs = 256;  // MI355X; sizes the static K-split scratch array
 __global__ __launch_bounds__(256) void clear_words_kernel(uint32_t *p, int words) {
   for (int i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) p[i] = 0u;
 }
-constexpr int kLdsBytes = 160 * 1024;  // per CU, and the most one workgroup may ask for
-
-// Kernels that ask for more than 48 KB of dynamic LDS need the attribute raised once per device; the (kernel,
-// device) pairs already done are remembered, so a launch costs a table look-up, not a runtime call.
-struct PreparedKernels {
-  static constexpr int kSlots = 512;  // open addressing; far more than the instantiations in this file
-  std::atomic<uintptr_t> key[kSlots];
-  bool seen_or_insert(uintptr_t k, bool insert) {
-    for (int i = 0, h = static_cast<int>((k >> 4) % kSlots); i < kSlots; ++i, h = (h + 1) % kSlots) {
-      uintptr_t cur = key[h].load(std::memory_order_acquire);
-      if (cur == k) return true;
-      if (cur == 0) {
-        if (!insert) return false;
-        if (key[h].compare_exchange_strong(cur, k, std::memory_order_acq_rel) || cur == k) return true;
-      }
-    }
-    return false;
-  }
-};
-PreparedKernels g_prepared;
-
-template <typename K>
-int prepare(K kern, int smem) {
-  if (smem > 48 * 1024) {
-    int dev = 0;
-    hipError_t e = hipGetDevice(&dev);
-    if (e != hipSuccess) {
-      set_last_hip_error(e);
-      return QUIK_ERR_LAUNCH;
-    }
-    // kernel entry addresses are at least 16-byte aligned: the low bits carry the device, bit 0 marks a used slot
-    const uintptr_t k = (reinterpret_cast<uintptr_t>(kern) << 8) | (static_cast<uintptr_t>(dev & 0x7F) << 1) | 1u;
-    if (g_prepared.seen_or_insert(k, false)) return QUIK_OK;
-    e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, smem);
-    if (e != hipSuccess) {
-      set_last_hip_error(e);
-      return QUIK_ERR_LAUNCH;
-    }
-    g_prepared.seen_or_insert(k, true);
-  }
-  return QUIK_OK;
-}
-
 template <class C>
 int grid_of(int64_t M, int64_t N, int &tiles_m, int &tiles_n) {
   tiles_m = static_cast<int>((M + C::BM - 1) / C::BM);

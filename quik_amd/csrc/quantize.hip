@@ -1813,16 +1813,14 @@ bool list_quantize_ok(const void *x, int dtype, int64_t rows, int64_t cols, cons
 }
 int launch_list(const void *x, int dtype, int64_t rows, int64_t cols, const int64_t *int_idx, int64_t num_int,
                 const int64_t *fp_idx, int64_t num_fp, int bits, void *dst, void *meta, void *fp_x, hipStream_t st) {
+  // the row, the outlier columns and their mask: most with 32768 columns that are all outliers but eight
+  constexpr int64_t kMost = kStreamMaxCols * 2 + kStreamMaxCols * 2 + kStreamMaxCols / 8;
+  static_assert(kMost + 1024 <= kLdsBytes, "with the static LDS of the reductions");
   const int64_t lds = cols * 2 + (num_fp + 7) / 8 * 16 + (cols + 31) / 32 * 4;
   const int64_t grid = rows < 2 * num_cus() ? rows : 2 * num_cus();
   auto go = [&](auto kern) {
     if (lds > 48 * 1024) {
-      if (hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                             static_cast<int>(kMaxLdsRowBytes));
-          e != hipSuccess) {
-        set_last_hip_error(e);
-        return static_cast<int>(QUIK_ERR_LAUNCH);
-      }
+      if (int rc = prepare(kern, static_cast<int>(kMost))) return rc;
     }
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kThreads), static_cast<size_t>(lds), st,
                        static_cast<const uint16_t *>(x), static_cast<int>(rows), static_cast<int>(cols), int_idx,

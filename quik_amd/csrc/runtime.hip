@@ -32,6 +32,45 @@ int num_cus() {
   return n;
 }
 
+namespace {
+// The (kernel, device) pairs whose LDS limit is raised: a launch costs a table look-up, not a runtime call.
+struct PreparedKernels {
+  static constexpr int kSlots = 1024;  // open addressing; far more than the instantiations in this library
+  std::atomic<uintptr_t> key[kSlots];
+  bool seen_or_insert(uintptr_t k, bool insert) {
+    for (int i = 0, h = static_cast<int>((k >> 4) % kSlots); i < kSlots; ++i, h = (h + 1) % kSlots) {
+      uintptr_t cur = key[h].load(std::memory_order_acquire);
+      if (cur == k) return true;
+      if (cur == 0) {
+        if (!insert) return false;
+        if (key[h].compare_exchange_strong(cur, k, std::memory_order_acq_rel) || cur == k) return true;
+      }
+    }
+    return false;
+  }
+};
+PreparedKernels g_prepared;
+}  // namespace
+
+int prepare_lds(const void *kern, int smem) {
+  int dev = 0;
+  hipError_t e = hipGetDevice(&dev);
+  if (e != hipSuccess) {
+    set_last_hip_error(e);
+    return QUIK_ERR_LAUNCH;
+  }
+  // kernel entry addresses are at least 16-byte aligned: the low bits carry the device, bit 0 marks a used slot
+  const uintptr_t k = (reinterpret_cast<uintptr_t>(kern) << 8) | (static_cast<uintptr_t>(dev & 0x7F) << 1) | 1u;
+  if (g_prepared.seen_or_insert(k, false)) return QUIK_OK;
+  e = hipFuncSetAttribute(kern, hipFuncAttributeMaxDynamicSharedMemorySize, smem);
+  if (e != hipSuccess) {
+    set_last_hip_error(e);
+    return QUIK_ERR_LAUNCH;
+  }
+  g_prepared.seen_or_insert(k, true);
+  return QUIK_OK;
+}
+
 // ---- flags of the column maps this process has used -----------------------------------------------------------
 // The flags word of a column map (colmap.h) lives on the device.  Entry points that have no kernel path for a map
 // without the streaming flag (or without the in-place order) must refuse such a map instead of launching a kernel
