@@ -533,10 +533,12 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
 }
 
 // Register-streaming kernel (gemm_direct.h) or ring kernel, for problems below the 256-row tiles.  Both are priced in ns:
-// a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (45 .. 50 per cycle, whichever kernel asks),
-// never less than the weights at 5.5 TB/s, and for a K split the exchange (its partial sums cross memory: 16 KB per
-// workgroup here, 64 KB in the ring kernel).  Constants fitted to 21 shapes of 40 .. 2048 rows and 1024 .. 28672 columns,
-// both widths; the choice was right on all of them to within 0.5 us.
+// a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (alone, over K, 87 .. 94 here and 87 in the
+// ring kernel), never less than the weights at 5.5 TB/s, and for a K split the exchange (its partial sums cross memory:
+// 16 KB per workgroup here, 64 KB in the ring kernel).  Against every variant on 29 shapes of 40 .. 2048 rows, 1024 ..
+// 28672 columns, both widths, weights in the Infinity Cache: within 0.5 us of the fastest on 25; 1.5 us behind on 64 x 8192
+// -> 8192, 64 x 5120 -> 13824 and (8 bits) 64 x 11008 -> 4096, 7 us on (8 bits) 64 x 28672 -> 8192 (44.0 against 36.9 with
+// 64x32 tiles): all variants cost the stream's floor there, and from that cache the weights come faster.
 struct DirectPlan {
   int bn, splits;  // tile width (64 or 32; 0: ring kernel), workgroups per tile
   int64_t bytes;   // workspace of the split
@@ -600,8 +602,8 @@ int run_direct(const Args &p, hipStream_t st, void *workspace, int64_t workspace
 // The 6-bit matrix-core path (gemm_fp6.h): 256x256 tiles alone (eight waves), 256x256 + 256x128 tiles in one
 // launch (four waves), or 128x128 tiles.
 // Whole rounds of 256x256 tiles with little left over: a last round of 256x128 tiles costs 59, on part of the CUs; the same
-// columns in 128x128 tiles are one per CU at 36 (percent of a wide tile).  2048 x 8192 -> 10240: 126.3 -> 112.6 us per
-// forward, int8 188 -> 176.
+// columns in 128x128 tiles are one per CU at 36 (percent of a wide tile).  2048 x 8192 -> 10240: 111.5 -> 102.6 us per
+// forward (with the bands of tile_of_block), int8 179 -> 168.
 // Only behind whole rounds: narrow tiles that run beside wide ones are slower than the costs say (777 x 4096 -> 22016 by
 // the same costs 159 -> 136, measured 72.2 -> 73.8 us), and two of them per CU cost more than a 256x128 tile.
 // Returns the columns of the wide part, 0: the plan of make_plan6 stands.
@@ -643,8 +645,9 @@ int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t wor
     if (mid_tiles * 8 <= int64_t(num_cus()) * 5) {
       // One tile per CU: a ring of twelve slots (110 KB of LDS) instead of six, nine steps in flight instead of three.  Layer
       // forward 300 x 4544 -> 4544 19.1 -> 18.6 us, 2048 x 8192 -> 1024 31.3 -> 30.7, 128 x 5120 -> 13824 20.3 -> 20.0, 256 x
-      // 8192 -> 8192 26.5 -> 25.9: a step still takes about 240 cycles for 64 of MFMA (two steps between barriers, or no
-      // second copy of the W block, changed nothing on top).  More tiles need two workgroups per CU, which six slots allow.
+      // 8192 -> 8192 26.5 -> 25.9: a step takes 106 ns, some 210 cycles, for 64 of MFMA, against 111 ns with six slots (two
+      // steps between barriers, or no second copy of the W block, changed nothing on top).  More tiles need two
+      // workgroups per CU, which six slots allow.
       if ((p.M + 127) / 128 * ((p.N + 63) / 64) <= num_cus()) return launch_fused6<CfgD6, BF16>(p, st);
       return launch_fused6<CfgN6, BF16>(p, st);
     }

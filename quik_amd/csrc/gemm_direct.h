@@ -3,20 +3,20 @@
 //
 // What bounds the ring kernels (gemm_fp6.h, gemm_tile8.h) on few and narrow tiles is the step itself: a 128x64 tile has
 // two MFMAs per wave and k-step, 64 cycles of work between two barriers, an LDS round trip and a wait for copies
-// (measured 250 .. 300 cycles a step; 13824 columns at 128 rows: 16 us for 53 MB of weights).  The operand buffers hold
+// (measured over K: 106 .. 112 ns a step, some 210 cycles).  The operand buffers hold
 // each fragment as one contiguous kilobyte (fp6_format.h), so a wave can load fragments directly, and nothing has to be
 // shared inside the workgroup if the waves split K instead of the tile: each of the four waves computes the WHOLE tile
 // (64x64 or 64x32) over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of
-// loads in flight.  What bounds it is the rate at which a CU takes in operands, 45 .. 50 bytes per cycle (a ring kernel
-// with the same tile moves the same bytes).  Afterwards the waves add their
+// loads in flight.  What bounds it is the rate at which a CU takes in operands: over K, 70 ns per step of 6 KB (88 bytes
+// per ns) for 64x64 tiles at 6 bits, 33 ns per 3 KB (94) for 64x32 tiles at 8.  Afterwards the waves add their
 // integer sums through LDS (exact, so in any order), each ending up with the blocks it owns, convert them, run the
 // outlier steps on them in the same order as the ring kernels and store: the same output bits.
 //
 // Workgroups may share a tile's K further (SplitK, as in gemm_fp6.h): when the tiles are fewer than the CUs.
 //
-// Measured against the ring kernels (GEMM launch in a graph, us): W4A4 64 x 8192 x 7936 22.7 -> 12.6, 64 x 10240 x 7936
-// 23.0 -> 14.9, 128 x 8192 x 7936 23.4 -> 14.4, 40 x 4096 x 3840 11.9 -> 8.5, 256 x 4096 x 3840 12.1 -> 9.8,
-// 512 x 1024 x 3968 9.9 -> 7.7; W8A8 64 x 5120 x 13568 27.1 -> 18.0, 64 x 4096 x 10752 26.6 -> 13.9.
+// Measured against the ring kernels (GEMM launch in a graph, us): W4A4 64 x 8192 x 7936 22.3 -> 13.7, 64 x 10240 x 7936
+// 22.5 -> 14.3, 128 x 8192 x 7936 22.8 -> 13.8, 40 x 4096 x 3840 10.5 -> 7.1, 256 x 4096 x 3840 10.8 -> 8.6,
+// 512 x 1024 x 3840 10.5 -> 7.3; W8A8 64 x 5120 x 13568 26.7 -> 18.1, 64 x 4096 x 10752 26.2 -> 15.1.
 #pragma once
 #include <type_traits>
 

@@ -430,8 +430,8 @@ __device__ __forceinline__ void run_mainloop(const uint8_t *__restrict__ X, int6
 // kBandRows token rows, M fastest inside a band: the 32 (or 64) tiles an XCD has in flight then form a block of about as
 // many rows as columns, and what the XCD has to fetch past its 4 MB L2 per k-step, their rows plus their columns, is
 // smallest.  (With M fastest over ALL rows, 8192 rows are 32 tiles of one column each: 8448 operand rows per k-step
-// instead of 3072.  6-bit GEMM 8192 x 28672 x 8192: 1057 -> 919 us, int8 8192 x 8192 x 28672: 1494 -> 1417 us, 2048 rows
-// of 28672 x 8192: 256 -> 247 us; up to 1024 rows nothing changes.)
+// instead of 3072.  Layer forward: 6 bit 8192 x 8192 -> 8192 366 -> 316 us, 2048 x 8192 -> 28672 272.4 -> 269.9; int8 8192 x
+// 28672 -> 8192 1660 -> 1600; up to 1024 rows nothing changes.)
 // `bid` is the workgroup's index inside its launch region; regions start at multiples of 8.
 constexpr int kBandRows = 1024;
 template <int BM>

@@ -2,17 +2,18 @@
 // through a private LDS ring.
 //
 // What bounds the shared rings of gemm_kernels.h on few and narrow tiles is the step: 64 bytes of K per row between two
-// barriers, two to eight MFMAs per wave, a wait for copies issued two steps before (measured 450 .. 850 cycles a step where
-// the operands take 170 .. 260).  Here the four waves of a workgroup split K: each computes the WHOLE 64x64 (128x64) tile
+// barriers, two to eight MFMAs per wave, a wait for copies issued two steps before (256 rows, 4096 columns, over K: 312 ns a
+// step at 4 bits, 233 at 8).  Here the four waves of a workgroup split K: each computes the WHOLE 64x64 (128x64) tile
 // over every fourth 128-byte stage, copies only what it multiplies itself and never meets a barrier in the main loop.  A
 // copy instruction takes 8 rows of a whole cache line: with 64-byte pieces of 16 rows a CU took in 23 bytes per cycle
-// instead of 45 (int8 256 x 4096 x 4096: 13.8 .. 14.9 us against 9.9).  Two stages are in flight or in LDS and one in
+// instead of about 45 (int8 256 x 4096 x 4096: 13.8 .. 14.9 us against 9.9).  Two stages are in flight or in LDS and one in
 // registers; 128x64 tiles have room for one and one, enough for the longer multiplication of a stage.  Afterwards the
 // waves add their sums through LDS (integers: in any order), each ending up with the blocks it stores.
 //
 // Measured (launch in a graph, us): int4 256 x 4096 x 4096 13.7 -> 8.6 (fused dequantize 15.2 -> 9.2), 40 x 4096 x 3968
-// 12.6 -> 7.4; int8 256 x 4096 x 4096 18.2 -> 9.9, 128 x 13824 x 4864 30.7 -> 22.6.  What is left: about 6 us of launch,
-// first copies, exchange and stores, then 103 operand bytes per ns and CU.
+// 12.6 -> 7.4; int8 256 x 4096 x 4096 18.2 -> 9.9, 128 x 13824 x 4864 30.7 -> 22.6.  What is left (256 rows, 4096
+// columns, over K): 4 .. 5 us of launch, first copies, exchange and stores, then per stage of 16 KB 174 ns at 8 bits (94
+// bytes per ns and CU) and 220 .. 260 at 4 bits, where a stage is twice the products and has to be unpacked.
 #pragma once
 #include "gemm_kernels.h"
 

@@ -271,7 +271,8 @@ class MixedQLinear(torch.nn.Module):
     operands in tile order (`tiled_path`; the quantize kernel writes the activation that way, the weights
     get a second, repacked copy on first use), so every operand cache line is fetched once per tile.
     (Integer columns that do not fill whole k-steps, multiples of 32 / 16 instead of 128 / 64, take it through the one-call
-    forward, whose operand buffers are filled up with zeros.)
+    forward, whose operand buffers are filled up with zeros.)  That copy stays beside the reference's buffers, see
+    `weight_bytes` and `transient_tiled_copy`.
     W4A4: the int4 products run on the 6-bit (E2M3) matrix-core instructions, which have twice the int8 rate:
     levels code + 8 are exact E2M3 numbers and the integer accumulator is recovered exactly (0.75
     bytes per weight).  W8A8: int8 MFMA as before (1 byte per weight).  Both need fp_features % 32 == 0 and ascending int_indices and give the output bits
