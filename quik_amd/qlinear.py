@@ -552,10 +552,12 @@ class MixedQLinear(torch.nn.Module):
         # A forward brings the descriptor of its own path up to date; the other path's may date from before the buffers
         # changed.  The plan compares the buffers with what they are now, so nothing later would find that out.
         state = self._descriptor_source()
-        for t in (False, True):
-            if t in self._descs and not self._descs[t][0].holds(*state):
-                del self._descs[t]
-        row, til = self._descs.get(False), self._descs.get(True)
+        entries = [self._descs.get(t) for t in (False, True)]
+        for t, entry in enumerate(entries):
+            if entry is not None and not entry[0].holds(*state):
+                self._descs.pop(bool(t), None)
+                entries[t] = None
+        row, til = entries
         if (til if tiled else row) is None:
             return        # transient_tiled_copy: the operand is repacked by every call
         min_rows = self.six_bit_min_rows if self.bits == 4 else self.tile8_min_rows
