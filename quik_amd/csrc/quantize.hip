@@ -371,7 +371,7 @@ __device__ __forceinline__ void stream_rows(const uint16_t *__restrict__ x, int6
   // vec_out: 0 byte-wise output, 1 16-byte output,
   // 3 (8 bits only): dst is an int8 operand buffer in tile order for gemm_tile8.h, which also takes the outlier
   // values (fp_x is not written); needs num_int % 16 == 0 and num_fp % 32 == 0
-  // (the 6-bit operand buffers of gemm_fp6.h are written by quantize_fp6_wave_kernel below)
+  // (the 6-bit operand buffers of gemm_fp6.h are written by quantize_fp6_row_kernel below)
   const Tile8Layout l8 = tile8_layout(rows, num_int, num_fp);
   const bool to8 = BITS == 8 && vec_out == 3;
   const int tid = threadIdx.x;
@@ -1048,298 +1048,254 @@ __device__ __forceinline__ uint32_t level_pair_fast(uint32_t w, const RQ &rq) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, tb) + h2{magic, magic});
 }
 
+// ---- pieces of the kernel that writes 6-bit operand buffers (quantize_fp6_row_kernel)
+
+// Byte offset of source column c inside a row image in LDS.  A copy instruction moves one contiguous kilobyte (64 groups
+// of 8 columns = 16 fragments of 32 consecutive columns; whole cache lines) and deals it to the LDS slots transposed:
+// slot 16 i + m of the kilobyte holds group 4 m + i, i.e. the i-th group of the kilobyte's fragment m.  The i-th 16-byte
+// reads of 16 neighbouring fragments cover 256 consecutive bytes, so all reads are free of bank conflicts.
+__device__ __forceinline__ uint32_t img_of_col(uint32_t c) {
+  const uint32_t g = c >> 3, f = g >> 2, i = g & 3u;
+  return ((f >> 4) << 10) + ((16u * i + (f & 15u)) << 4) + ((c & 7u) << 1);
+}
+// the four groups of fragment f
+__device__ __forceinline__ void img_fragment(const uint8_t *img, int f, uint4 (&v)[4]) {
+#pragma unroll
+  for (int i = 0; i < 4; ++i) v[i] = *reinterpret_cast<const uint4 *>(img + ((f >> 4) << 10) + ((16 * i + (f & 15)) << 4));
+}
+// address of the row, in scalar registers
+// (the intrinsic returns int: each half goes through uint32_t, or the low half would be sign-extended)
+__device__ __forceinline__ const uint8_t *uniform_row(const uint16_t *x, int64_t row, int cols) {
+  const uint64_t a = reinterpret_cast<uint64_t>(x + row * cols);
+  const uint32_t a_hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32)));
+  const uint32_t a_lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a & 0xFFFFFFFFu)));
+  return reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(a_hi) << 32) | a_lo);
+}
+
+// Running min / max (symmetric: largest |x| pattern) over fragments.
+template <bool BF16, bool SYM>
+struct FragmentRange {
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+  uint32_t pmn = 0x7C007C00u, pmx = 0xFC00FC00u;  // fp16: +inf / -inf in both halves
+  u2 amax = u2{0, 0};
+  __device__ __forceinline__ void add(const uint4 (&v)[4]) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
+      if constexpr (SYM) {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) amax = __builtin_elementwise_max(amax, __builtin_bit_cast(u2, w[k] & 0x7FFF7FFFu));
+      } else if constexpr (!BF16) {
+        // packed fp16 min / max skip NaN operands, as the reference's __hmin / __hmax do
+        pmn = pk_min_f16(pmn, pk_min_f16(pk_min_f16(w[0], w[1]), pk_min_f16(w[2], w[3])));
+        pmx = pk_max_f16(pmx, pk_max_f16(pk_max_f16(w[0], w[1]), pk_max_f16(w[2], w[3])));
+      } else {
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          const float f0 = __uint_as_float(w[k] << 16), f1 = __uint_as_float(w[k] & 0xFFFF0000u);
+          mn = fminf(mn, fminf(f0, f1));
+          mx = fmaxf(mx, fmaxf(f0, f1));
+        }
+      }
+    }
+  }
+  // wave-wide (lo, hi); symmetric: hi is the largest pattern, a 15-bit integer (exact, ordered like the patterns)
+  __device__ __forceinline__ void reduce(float &lo, float &hi) const {
+    const h2 a = __builtin_bit_cast(h2, pmn), b = __builtin_bit_cast(h2, pmx);
+    lo = SYM ? 0.0f : BF16 ? mn : fminf(static_cast<float>(a.x), static_cast<float>(a.y));
+    hi = SYM ? static_cast<float>(amax.x > amax.y ? amax.x : amax.y)
+             : BF16 ? mx : fmaxf(static_cast<float>(b.x), static_cast<float>(b.y));
+    lo = wave_min(lo);
+    hi = wave_max(hi);
+  }
+};
+
+// Scale and zero of a row from its range, written to meta by the one thread that says so.
+template <bool BF16, bool SYM>
+__device__ __forceinline__ RowQuant<BF16> row_quant4(float lo, float hi, float sym_divisor, bool writes, uint16_t *meta,
+                                                     int64_t row) {
+  RowQuant<BF16> rq;
+  if constexpr (SYM) {
+    rq.init_sym(static_cast<uint32_t>(hi), sym_divisor);
+    if (writes) meta[row] = rq.scale_bits;
+  } else {
+    rq.init(lo, hi, 4);
+    if (writes) {
+      meta[2 * row] = rq.scale_bits;
+      meta[2 * row + 1] = rq.zero_bits;
+    }
+  }
+  return rq;
+}
+
+// Where the row's fragments go in the operand buffer: the row's part of the address is wave-uniform, the fragment's part is
+// the unit 3072 (f / 2) and its half.
+struct Fp6RowOut {
+  uint8_t *head, *tail;
+  uint32_t swap16;
+  __device__ __forceinline__ Fp6RowOut(uint8_t *dst, const Fp6Layout &l, int64_t row) {
+    uint8_t *rb = dst + (row >> 6) * l.block_bytes;
+    head = rb + ((row >> 5) & 1) * 1024 + (row & 31) * 32;
+    tail = rb + 2048 + (row & 63) * 8;
+    swap16 = static_cast<uint32_t>((row >> 3) & 1) << 4;
+  }
+};
+
+// One fragment: 32 values -> 32 levels -> 24 bytes, stored; returns the sum of its levels.
+template <bool BF16, bool SYM, bool SLOW>
+__device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQuant<BF16> &rq, int f, const Fp6RowOut &out) {
+  uint32_t b[8];  // 32 levels, one per byte
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    if constexpr (!SLOW && !BF16) {
+      const uint32_t p0 = level_pair_fast<SYM>(v[i].x, rq), p1 = level_pair_fast<SYM>(v[i].y, rq);
+      const uint32_t p2 = level_pair_fast<SYM>(v[i].z, rq), p3 = level_pair_fast<SYM>(v[i].w, rq);
+      b[2 * i] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);  // bytes 0, 2 of p0 then bytes 0, 2 of p1
+      b[2 * i + 1] = __builtin_amdgcn_perm(p3, p2, 0x06040200u);
+    } else {
+      const uint2 c = group_codes<4, BF16, SLOW, SYM>(v[i], rq);  // code nibbles (two's complement), one per byte
+      b[2 * i] = c.x ^ 0x08080808u;                               // level = code + 8
+      b[2 * i + 1] = c.y ^ 0x08080808u;
+    }
+  }
+  int sum = 0;
+#pragma unroll
+  for (int i = 0; i < 8; ++i) sum = __builtin_amdgcn_udot4(b[i], 0x01010101u, sum, false);
+  uint32_t o[6];
+  fp6_pack_fragment(b, o);
+  const uint32_t unit = static_cast<uint32_t>(f >> 1) * 3072u, h = static_cast<uint32_t>(f & 1);
+  // (default cache policy: a 128-byte line of the operand buffer takes pieces of 4 (heads) or 16 (tails) rows,
+  // which meet in the XCD's L2; as streaming stores every piece went to memory on its own and the launch
+  // took 29 us instead of 12)
+  *reinterpret_cast<uint4 *>(out.head + unit + ((h << 4) ^ out.swap16)) = make_uint4(o[0], o[1], o[2], o[3]);
+  *reinterpret_cast<uint2 *>(out.tail + unit + h * 512u) = make_uint2(o[4], o[5]);
+  return sum;
+}
+
 // ---------------------------------------------------------------------------------------
 // 6-bit operand buffers (consumer: gemm_fp6.h), written in the in-place order of the column map.
 //
-// One wave per row.  The wave copies the row global -> LDS with 16-byte-per-lane direct copies (no
-// registers are held while the row is in flight).  A copy instruction moves one contiguous kilobyte
-// (64 groups of 8 columns = 16 fragments of 32 consecutive source columns; whole cache lines) and deals
-// it to the LDS slots transposed: slot 16 i + m of the kilobyte holds group 4 m + i, i.e. the i-th group
-// of the kilobyte's fragment m.  Lane L owns the fragments L, L + 64, ...; its i-th 16-byte read of a
-// fragment and those of its 15 neighbours cover 256 consecutive bytes, so all reads are free of bank
-// conflicts.  In the image the holes (outlier columns among the first num_int columns) are
-// overwritten with their fillers (integer columns of the tail), two-byte LDS copies with row-invariant
-// addresses held in registers; after that the first num_int columns ARE the integer operand, in place:
-// one pass over the image for min / max, a second one that turns each fragment into 32 levels, packs
-// them to 24 bytes in registers and stores head and tail.  No barrier, no cross-wave reduction (a wave's
-// LDS operations execute in order), no data moved between lanes except the two reductions.
-// A workgroup (= wave) walks over rows w, w + grid, ...; up to eight of them share a CU (two per SIMD),
-// so one wave's arithmetic covers the other's transfer and LDS waits.  JT > 0: fragments per lane known at
-// compile time (rows up to 10240 columns); 0: a run-time loop over them.
-template <bool BF16, bool SYM, int JT, int W>
-__global__ __launch_bounds__(64 * W) void quantize_fp6_wave_kernel(
+// One workgroup per row; a lane owns JT fragments of 32 columns, one for rows of up to 16384 columns (a wave per 2048
+// columns).  The row is copied global -> LDS with direct copies (no registers are held while it is in flight).  In the image
+// the holes (outlier columns among the first num_int columns) are overwritten with their fillers (integer columns of the
+// tail); after that the first num_int columns ARE the integer operand, in place: a lane reads its fragment once, takes
+// part in the reduction of the range, turns the fragment into 32 levels in registers, packs them to 24 bytes and stores
+// head and tail.
+//
+// What bounds a launch is the chain of one row (launch, transfer, range, levels, stores) as long as the rows are few, the
+// memory system from about 2000 rows on.  A wave per row, two or eight of them in a workgroup and without any barrier, was
+// the form before: its two passes over up to five fragments per lane stood behind the transfer, and 64 rows occupied 64 of
+// 1024 SIMDs.  Here a pass takes as long as one fragment, for four barriers (image landed, outlier values read, holes
+// patched, range exchanged).  us per launch in a graph, wave per row -> this, 256 outlier columns, fp16: 16 x 4096 4.0 ->
+// 3.5, 64 x 8192 5.3 -> 3.7, 128 x 5120 4.7 -> 3.5, 777 x 4096 5.6 -> 4.8, 1024 x 8192 9.7 -> 8.1, 2048 x 8192 12.4 -> 12.5,
+// 8192 x 8192 49.0 -> 45.4, 64 x 28672 12.8 -> 5.8, 2048 x 28672 61.9 -> 40.7; slower only about 2000 rows of 4096 or 5120
+// columns, 7.9 -> 8.4 and 9.4 -> 10.1.  bf16: 64 x 8192 7.5 -> 4.2, 777 x 4096 7.6 -> 5.9, 2048 x 28672 94 -> 47.
+template <bool BF16, bool SYM, int JT>
+__global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     const uint16_t *__restrict__ x, int64_t rows, int cols, const uint32_t *__restrict__ patch,
-    const uint16_t *__restrict__ fp_col, int nholes, int num_int, int num_fp,
-    uint8_t *__restrict__ dst, uint16_t *__restrict__ meta, float sym_divisor) {
+    const uint16_t *__restrict__ fp_col, int nholes, int num_int, int num_fp, uint8_t *__restrict__ dst,
+    uint16_t *__restrict__ meta, float sym_divisor, int64_t first, int64_t count) {
   static_assert(!(BF16 && SYM), "symmetric activations are fp16");
-  constexpr int kTogether = 2;  // waves that issue their copies at the same time (measured: 1, 2, 4 and all 8)
-  extern __shared__ __align__(16) uint8_t images[];
-  __shared__ int turn_s;
-  if constexpr (!BF16 && !SYM) treat_all_nans_alike();  // pass 1 uses pk_min_f16 / pk_max_f16 on the raw row
+  extern __shared__ __align__(16) uint8_t img[];
+  __shared__ float red[16];
+  __shared__ uint32_t total_s;
+  if constexpr (!BF16 && !SYM) treat_all_nans_alike();  // the range uses pk_min_f16 / pk_max_f16 on the raw row
   // (nholes: the column map's count of holes, which the host knows: the entry points look the map's flag words up
   // before launching, and refuse a map without the in-place order; the kernel starts without a dependent load)
-  const int lane = threadIdx.x & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
-  const int frags_all = cols >> 5, frags = num_int >> 5, nchunk = num_fp >> 3;
-  const int J = JT > 0 ? JT : (frags_all + 63) >> 6;
-  uint8_t *row_img = images + wave * (J * 4096);
-  if (threadIdx.x == 0) turn_s = 0;
-  __syncthreads();
-  const Fp6Layout l6 = fp6_layout(rows, num_int, num_fp);
-  const uint32_t lds0 = lds_address(row_img);
-
-  constexpr int PREG = 4;
-  uint32_t p_hole[PREG], p_fill[PREG], o_addr[8];
-  // byte offset of source column c inside a row image
-  auto img_of_col = [](uint32_t c) -> uint32_t {
-    const uint32_t g = c >> 3, f = g >> 2, i = g & 3u;
-    return ((f >> 4) << 10) + ((16u * i + (f & 15u)) << 4) + ((c & 7u) << 1);
-  };
-  // body(j) for this lane's fragment slots j = 0 .. J-1, unrolled when their number is known at compile time
-  auto for_j = [&](auto body) {
-    if constexpr (JT > 0) {
-#pragma unroll
-      for (int j = 0; j < JT; ++j) body(j);
-    } else {
-      for (int j = 0; j < J; ++j) body(j);
-    }
-  };
-  auto issue = [&](int64_t row) {
-    const uint64_t a = reinterpret_cast<uint64_t>(x + row * cols);
-    // (the intrinsic returns int: each half goes through uint32_t, or the low half would be sign-extended)
-    const uint32_t a_hi = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a >> 32)));
-    const uint32_t a_lo = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(a & 0xFFFFFFFFu)));
-    const uint8_t *rp = reinterpret_cast<const uint8_t *>((static_cast<uint64_t>(a_hi) << 32) | a_lo);
-    // kilobyte q of the row: this lane copies group 64 q + 4 (lane % 16) + lane / 16 to slot 64 q + lane.
-    // The kilobytes are requested in an order that starts at a row-dependent one and wraps around: all waves of
-    // the launch issue their copies at about the same time, and with every row starting at its kilobyte 0 (rows
-    // are a multiple of 1 KB apart) the requests in flight at any moment would share their low address bits and
-    // crowd onto a few memory channels (measured with the input in HBM: 15.8 -> 14.0 us for 2048 x 8192).
+  const int tid = threadIdx.x, lane = tid & 63, T = blockDim.x, W = T >> 6;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int frags = num_int >> 5, nchunk = num_fp >> 3;
+  // Rows [first, first + count); workgroup g takes number (g % 8) * count / 8 + g / 8: a cache line of the operand buffer takes pieces of 4 (heads) or 16
+  // (tails) consecutive rows; workgroups are dealt round-robin to the 8 XCDs, so rows that share lines run on the same XCD
+  // at about the same time and meet in its L2.
+  const int64_t per_xcd = (count + 7) >> 3, at = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  if (at >= count) return;
+  const int64_t row = first + at;
+  {
+    const uint8_t *rp = uniform_row(x, row, cols);
+    const uint32_t lds0 = lds_address(img);
     const int g_in = 4 * (lane & 15) + (lane >> 4), g_last = (cols >> 3) - 1;
-    const int nkb = 4 * J;
-    const int rot = __builtin_amdgcn_readfirstlane(static_cast<int>((row * 5) % nkb));
-    for_j([&](int j) {
+#pragma unroll
+    for (int j = 0; j < JT; ++j)
 #pragma unroll
       for (int t = 0; t < 4; ++t) {
-        int q = 4 * j + t + rot;
-        q = q >= nkb ? q - nkb : q;
-        const int g = 64 * q + g_in;
-        const uint32_t voff = static_cast<uint32_t>(g < g_last ? g : g_last) * 16u;  // past the row: any valid group
-        dma_load16(rp, voff, lds0 + q * 1024);
+        const int q = 4 * (wave + j * W) + t, g = 64 * q + g_in;
+        dma_load16(rp, static_cast<uint32_t>(g < g_last ? g : g_last) * 16u, lds0 + q * 1024);  // past the row: any valid group
       }
-    });
-  };
-
-  auto process = [&](int64_t row, uint8_t *img) {
-    auto ld16 = [&](uint32_t off) { return *reinterpret_cast<const uint16_t *>(img + off); };
-    // ---- outlier values, 8 per lane, to the outlier units of the operand buffer (before the holes are patched:
-    // holes are outlier columns)
-    if (lane < nchunk) {
-      uint4 o;
-      o.x = ld16(o_addr[0]) | (static_cast<uint32_t>(ld16(o_addr[1])) << 16);
-      o.y = ld16(o_addr[2]) | (static_cast<uint32_t>(ld16(o_addr[3])) << 16);
-      o.z = ld16(o_addr[4]) | (static_cast<uint32_t>(ld16(o_addr[5])) << 16);
-      o.w = ld16(o_addr[6]) | (static_cast<uint32_t>(ld16(o_addr[7])) << 16);
-      *reinterpret_cast<uint4 *>(dst + fp6_outlier_offset(l6, row, lane >> 1, lane & 1)) = o;
-    }
-    for (int c = lane + 64; c < nchunk; c += 64) {
-      uint32_t w[4];
-#pragma unroll
-      for (int k = 0; k < 4; ++k)
-        w[k] = ld16(img_of_col(fp_col[c * 8 + 2 * k])) |
-               (static_cast<uint32_t>(ld16(img_of_col(fp_col[c * 8 + 2 * k + 1]))) << 16);
-      *reinterpret_cast<uint4 *>(dst + fp6_outlier_offset(l6, row, c >> 1, c & 1)) = make_uint4(w[0], w[1], w[2], w[3]);
-    }
-    // ---- holes <- fillers
-#pragma unroll
-    for (int k = 0; k < PREG; ++k)
-      if (lane + 64 * k < nholes) *reinterpret_cast<uint16_t *>(img + p_hole[k]) = ld16(p_fill[k]);
-    for (int e = lane + 64 * PREG; e < nholes; e += 64) {
-      const uint32_t pe = patch[e];
-      *reinterpret_cast<uint16_t *>(img + img_of_col(pe & 0xFFFFu)) = ld16(img_of_col(pe >> 16));
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");  // other lanes read the patched halves below
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-
-    auto load_fragment = [&](int j, uint4 (&v)[4]) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-        v[i] = *reinterpret_cast<const uint4 *>(img + ((4 * j + (lane >> 4)) << 10) + ((16 * i + (lane & 15)) << 4));
-    };
-    // ---- pass 1: min / max (symmetric: largest |x| pattern) over this lane's fragments
-    const float inf = __builtin_inff();
-    float mn = inf, mx = -inf;
-    uint32_t pmn_b = 0x7C007C00u, pmx_b = 0xFC00FC00u;  // +inf / -inf in both halves
-    u2 amax = u2{0, 0};
-    // up to four fragments per lane stay in registers from the first pass to the second (64 registers): the second
-    // pass then has no LDS round trip in front of its arithmetic
-    constexpr bool kKeep = JT > 0 && JT <= 4;
-    uint4 kept[kKeep ? JT : 1][4];
-    for_j([&](int j) {
-      if (lane + 64 * j < frags) {
-        uint4 v[4];
-        load_fragment(j, v);
-        if constexpr (kKeep) {
-#pragma unroll
-          for (int i = 0; i < 4; ++i) kept[j][i] = v[i];
-        }
-#pragma unroll
-        for (int i = 0; i < 4; ++i) {
-          const uint32_t w[4] = {v[i].x, v[i].y, v[i].z, v[i].w};
-          if constexpr (SYM) {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) amax = __builtin_elementwise_max(amax, __builtin_bit_cast(u2, w[k] & 0x7FFF7FFFu));
-          } else if constexpr (!BF16) {
-            // packed fp16 min / max skip NaN operands, as the reference's __hmin / __hmax do
-            const uint32_t lo = pk_min_f16(pk_min_f16(w[0], w[1]), pk_min_f16(w[2], w[3]));
-            const uint32_t hi = pk_max_f16(pk_max_f16(w[0], w[1]), pk_max_f16(w[2], w[3]));
-            pmn_b = pk_min_f16(pmn_b, lo);
-            pmx_b = pk_max_f16(pmx_b, hi);
-          } else {
-#pragma unroll
-            for (int k = 0; k < 4; ++k) {
-              const float f0 = __uint_as_float(w[k] << 16), f1 = __uint_as_float(w[k] & 0xFFFF0000u);
-              mn = fminf(mn, fminf(f0, f1));
-              mx = fmaxf(mx, fmaxf(f0, f1));
-            }
-          }
-        }
-      }
-    });
-    const h2 pmn = __builtin_bit_cast(h2, pmn_b), pmx = __builtin_bit_cast(h2, pmx_b);
-    if constexpr (SYM) {
-      mn = 0.0f;
-      mx = static_cast<float>(amax.x > amax.y ? amax.x : amax.y);  // a 15-bit integer: exact, ordered like the patterns
-    } else if constexpr (!BF16) {
-      mn = fminf(static_cast<float>(pmn.x), static_cast<float>(pmn.y));
-      mx = fmaxf(static_cast<float>(pmx.x), static_cast<float>(pmx.y));
-    }
-    mn = wave_min(mn);
-    mx = wave_max(mx);
-    RowQuant<BF16> rq;
-    if constexpr (SYM) {
-      rq.init_sym(static_cast<uint32_t>(mx), sym_divisor);
-      if (lane == 0) meta[row] = rq.scale_bits;
-    } else {
-      rq.init(mn, mx, 4);
-      if (lane == 0) {
-        meta[2 * row] = rq.scale_bits;
-        meta[2 * row + 1] = rq.zero_bits;
-      }
-    }
-    // ---- pass 2: fragment -> 32 levels -> 24 bytes
-    // (store addresses: the row's part is wave-uniform, the fragment's part is the unit 3072 (f / 2) and its half)
-    const int64_t rb = (row >> 6) * l6.block_bytes;
-    uint8_t *head_row = dst + rb + ((row >> 5) & 1) * 1024 + (row & 31) * 32;
-    uint8_t *tail_row = dst + rb + 2048 + (row & 63) * 8;
-    const uint32_t swap16 = static_cast<uint32_t>((row >> 3) & 1) << 4;
-    int sum = 0;
-    auto quantise = [&](auto slow_c) {
-      constexpr bool SLOW = decltype(slow_c)::value;
-      for_j([&](int j) {
-        const int f = lane + 64 * j;
-        if (f < frags) {
-          uint4 v[4];
-          if constexpr (kKeep) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i) v[i] = kept[j][i];
-          } else {
-            load_fragment(j, v);
-          }
-          uint32_t b[8];  // 32 levels, one per byte
-#pragma unroll
-          for (int i = 0; i < 4; ++i) {
-            if constexpr (!SLOW && !BF16) {
-              const uint32_t p0 = level_pair_fast<SYM>(v[i].x, rq), p1 = level_pair_fast<SYM>(v[i].y, rq);
-              const uint32_t p2 = level_pair_fast<SYM>(v[i].z, rq), p3 = level_pair_fast<SYM>(v[i].w, rq);
-              b[2 * i] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);  // bytes 0, 2 of p0 then bytes 0, 2 of p1
-              b[2 * i + 1] = __builtin_amdgcn_perm(p3, p2, 0x06040200u);
-            } else {
-              const uint2 c = group_codes<4, BF16, SLOW, SYM>(v[i], rq);  // code nibbles (two's complement), one per byte
-              b[2 * i] = c.x ^ 0x08080808u;                               // level = code + 8
-              b[2 * i + 1] = c.y ^ 0x08080808u;
-            }
-          }
-#pragma unroll
-          for (int i = 0; i < 8; ++i) sum = __builtin_amdgcn_udot4(b[i], 0x01010101u, sum, false);
-          uint32_t o[6];
-          fp6_pack_fragment(b, o);
-          const uint32_t unit = static_cast<uint32_t>(f >> 1) * 3072u, h = static_cast<uint32_t>(f & 1);
-          // (default cache policy: a 128-byte line of the operand buffer takes pieces of 4 (heads) or 16 (tails) rows,
-          // which meet in the XCD's L2; as streaming stores every piece went to memory on its own and the launch
-          // took 29 us instead of 12)
-          *reinterpret_cast<uint4 *>(head_row + unit + ((h << 4) ^ swap16)) = make_uint4(o[0], o[1], o[2], o[3]);
-          *reinterpret_cast<uint2 *>(tail_row + unit + h * 512u) = make_uint2(o[4], o[5]);
-        }
-      });
-    };
-    if (__builtin_amdgcn_readfirstlane(rq.slow ? 1 : 0)) {
-      quantise(std::true_type{});
-    } else {
-      quantise(std::false_type{});
-    }
-    sum = wave_sum(sum);
-    if (lane == 0) reinterpret_cast<int32_t *>(dst + l6.sums_off)[row] = sum;
-  };
-
-  // Workgroup g takes the rows (g % 8) * rows / 8 + (g / 8) * W + wave (a cache line of the operand buffer takes
-  // pieces of 4 (heads) or 16 (tails) consecutive rows; workgroups are dealt round-robin to the 8 XCDs, so rows that
-  // share lines run on the same XCD at about the same time and meet in its L2), then every gridDim.x-th further group.
-  //
-  // The waves of a workgroup issue their copies kTogether at a time, in the order of a counter in LDS: the memory
-  // system serves a CU's requests about in the order they arrive, so the rows land in that order and a wave does
-  // its arithmetic while the later rows are still in flight.  (With all waves issuing at once the requests
-  // interleave, all rows land together at the end of the transfer, and transfer and arithmetic add up instead of
-  // overlapping.)  Every wave takes every one of its turns, with or without a row, so the counter always advances.
-  const int64_t per_xcd = (rows + 7) >> 3, groups_per_xcd = (per_xcd + W - 1) / W, groups = groups_per_xcd * 8;
-  auto row_of = [&](int64_t g) -> int64_t {
-    const int64_t i = (g >> 3) * W + wave;
-    const int64_t r = (g & 7) * per_xcd + i;
-    return i < per_xcd && r < rows ? r : -1;
-  };
-  volatile int *turn_v = &turn_s;
-  auto take_turn = [&](int t, int64_t row) {
-    const int need = t / kTogether * kTogether;  // all waves of the earlier sets have issued
-    while (__builtin_amdgcn_readfirstlane(*turn_v) < need) __builtin_amdgcn_s_sleep(1);
-    if (row >= 0) issue(row);
-    if (lane == 0) __hip_atomic_fetch_add(&turn_s, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-  };
-  int64_t g = blockIdx.x;
-  if (g >= groups) return;
-  int t = wave;
-  take_turn(t, row_of(g));
-  // Row-invariant addresses in registers: this lane's first four patches and its first chunk of 8 outliers.  The
-  // loads are unconditional (clamped indices, one 16-byte load for the eight outlier columns) and come after the
-  // first row's copies, so they are all in flight together and behind the row, not in front of it.
-  {
-    const int last_hole = nholes > 0 ? nholes - 1 : 0;
-    uint32_t e[PREG];
-#pragma unroll
-    for (int k = 0; k < PREG; ++k) e[k] = patch[lane + 64 * k < nholes ? lane + 64 * k : last_hole];
-    const int chunk = lane < nchunk ? lane : 0;
-    const uint4 oc = nchunk > 0 ? *reinterpret_cast<const uint4 *>(fp_col + chunk * 8) : make_uint4(0, 0, 0, 0);
-#pragma unroll
-    for (int k = 0; k < PREG; ++k) {
-      p_hole[k] = img_of_col(e[k] & 0xFFFFu);
-      p_fill[k] = img_of_col(e[k] >> 16);
-    }
-    const uint32_t ow[4] = {oc.x, oc.y, oc.z, oc.w};
-#pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      o_addr[2 * k] = img_of_col(ow[k] & 0xFFFFu);
-      o_addr[2 * k + 1] = img_of_col(ow[k] >> 16);
-    }
   }
-  for (; g < groups; g += gridDim.x) {
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // this row's image has landed
-    const int64_t row = row_of(g);
-    if (row >= 0) process(row, row_img);
-    if (g + gridDim.x < groups) {
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");  // this row's LDS reads are done before the image is overwritten (a wait only: no hazard)
-      t += W;
-      take_turn(t, row_of(g + gridDim.x));
+  // (unconditional loads, in flight together with the row)
+  constexpr int PREG = 2;
+  uint32_t pe[PREG];
+#pragma unroll
+  for (int k = 0; k < PREG; ++k) pe[k] = patch[tid + k * T < nholes ? tid + k * T : 0];
+  const uint4 oc = *reinterpret_cast<const uint4 *>(fp_col + (tid < nchunk ? tid : 0) * 8);
+  if (tid == 0) total_s = 0;
+  const Fp6Layout l6 = fp6_layout(rows, num_int, num_fp);
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  __syncthreads();
+
+  auto ld16 = [&](uint32_t c) -> uint32_t { return *reinterpret_cast<const uint16_t *>(img + img_of_col(c)); };
+  // outlier values first: holes are outlier columns
+  auto outliers = [&](int c, const uint4 &cols8) {
+    const uint32_t ow[4] = {cols8.x, cols8.y, cols8.z, cols8.w};
+    uint32_t o[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) o[k] = ld16(ow[k] & 0xFFFFu) | (ld16(ow[k] >> 16) << 16);
+    *reinterpret_cast<uint4 *>(dst + fp6_outlier_offset(l6, row, c >> 1, c & 1)) = make_uint4(o[0], o[1], o[2], o[3]);
+  };
+  if (tid < nchunk) outliers(tid, oc);
+  for (int c = tid + T; c < nchunk; c += T) outliers(c, *reinterpret_cast<const uint4 *>(fp_col + c * 8));
+  __syncthreads();
+  // holes <- fillers (integer columns: none of them is a hole)
+  auto fill = [&](uint32_t e) {
+    *reinterpret_cast<uint16_t *>(img + img_of_col(e & 0xFFFFu)) = static_cast<uint16_t>(ld16(e >> 16));
+  };
+#pragma unroll
+  for (int k = 0; k < PREG; ++k)
+    if (tid + k * T < nholes) fill(pe[k]);
+  for (int e = tid + PREG * T; e < nholes; e += T) fill(patch[e]);
+  __syncthreads();
+
+  FragmentRange<BF16, SYM> range;
+  uint4 v[JT][4];
+#pragma unroll
+  for (int j = 0; j < JT; ++j)
+    if (tid + j * T < frags) {
+      img_fragment(img, tid + j * T, v[j]);
+      range.add(v[j]);
     }
+  float mn, mx;
+  range.reduce(mn, mx);
+  if (lane == 0) {
+    red[wave] = mn;
+    red[8 + wave] = mx;
+  }
+  __syncthreads();
+  for (int w = 0; w < W; ++w) {
+    mn = fminf(mn, red[w]);
+    mx = fmaxf(mx, red[8 + w]);
+  }
+  const RowQuant<BF16> rq = row_quant4<BF16, SYM>(mn, mx, sym_divisor, tid == 0, meta, row);
+  const Fp6RowOut out(dst, l6, row);
+  int sum = 0;
+  auto quantise = [&](auto slow_c) {
+#pragma unroll
+    for (int j = 0; j < JT; ++j)
+      if (tid + j * T < frags)
+        sum += quantise_fragment<BF16, SYM, decltype(slow_c)::value>(v[j], rq, tid + j * T, out);
+  };
+  if (__builtin_amdgcn_readfirstlane(rq.slow ? 1 : 0)) {
+    quantise(std::true_type{});
+  } else {
+    quantise(std::false_type{});
+  }
+  // the wave that adds its sum last writes the row's: count in the high byte, sums below 2^19 (32768 columns of level 15)
+  sum = wave_sum(sum);
+  if (lane == 0) {
+    const uint32_t mine = (1u << 24) | static_cast<uint32_t>(sum);
+    const uint32_t all = __hip_atomic_fetch_add(&total_s, mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP) + mine;
+    if ((all >> 24) == static_cast<uint32_t>(W))
+      reinterpret_cast<int32_t *>(dst + l6.sums_off)[row] = static_cast<int32_t>(all & 0xFFFFFFu);
   }
 }
 
@@ -1742,62 +1698,31 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
 }
 
 
-// 6-bit operand output through quantize_fp6_wave_kernel; meta: (scale, zero) pairs, or one scale per row (SYM)
+// 6-bit operand output through quantize_fp6_row_kernel; meta: (scale, zero) pairs, or one scale per row (SYM)
 template <bool BF16, bool SYM>
-int launch_fp6_wave(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, const ColmapLayout &l, int64_t num_int,
-                    int64_t num_fp, void *dst, void *meta, hipStream_t st, float sym_divisor = 1.0f) {
+int launch_fp6_row(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, const ColmapLayout &l, int64_t num_int,
+                   int64_t num_fp, void *dst, void *meta, hipStream_t st, float sym_divisor = 1.0f) {
   uint32_t words[4];
   if (int rc = colmap_words(cm, cols, num_int, num_fp, st, words)) return rc;
   if ((words[0] & (kColmapStreams | kColmapInPlace)) != (kColmapStreams | kColmapInPlace)) return QUIK_ERR_COLMAP;
-  const int nholes = static_cast<int>(words[2]);
-  const int J = static_cast<int>((cols / 32 + 63) / 64);
-  // one workgroup per CU: as many waves as their row images fit (160 KB of LDS), at most 8 (two per SIMD)
-  const int per_cu = 156 / (J * 4) < 8 ? 156 / (J * 4) : 8;
-  auto go = [&](auto kern, int W) {
-    const int lds = W * J * 4096;  // one row image per wave
-    if (lds > 48 * 1024) {
-      hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern), hipFuncAttributeMaxDynamicSharedMemorySize, lds);
-      if (e != hipSuccess) {
-        set_last_hip_error(e);
-        return static_cast<int>(QUIK_ERR_LAUNCH);
-      }
+  auto go = [&](auto kern, int jt) {
+    const int per_wave = 64 * 32 * jt, W = static_cast<int>((cols + per_wave - 1) / per_wave);
+    if (int rc = prepare(kern, 8 * jt * 4096)) return rc;
+    constexpr int64_t kMost = 1 << 20;  // rows per launch: a grid holds fewer than 2^32 threads
+    for (int64_t first = 0; first < rows; first += kMost) {
+      const int64_t count = rows - first < kMost ? rows - first : kMost;
+      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((count + 7) / 8 * 8)), dim3(64 * W),
+                         static_cast<size_t>(W * jt * 4096), st, static_cast<const uint16_t *>(x), rows,
+                         static_cast<int>(cols), reinterpret_cast<const uint32_t *>(cm + l.off_patch),
+                         reinterpret_cast<const uint16_t *>(cm + l.off_fp), static_cast<int>(words[2]),
+                         static_cast<int>(num_int), static_cast<int>(num_fp), static_cast<uint8_t *>(dst),
+                         static_cast<uint16_t *>(meta), sym_divisor, first, count);
+      if (int rc = check_launch()) return rc;
     }
-    const int64_t per_xcd = (rows + 7) / 8, groups = (per_xcd + W - 1) / W * 8;
-    const int64_t resident = int64_t(num_cus()) * (per_cu / W) / 8 * 8;
-    const int grid = static_cast<int>(groups < resident ? groups : resident);
-    hipLaunchKernelGGL(kern, dim3(grid), dim3(64 * W), static_cast<size_t>(lds), st, static_cast<const uint16_t *>(x), rows,
-                       static_cast<int>(cols), reinterpret_cast<const uint32_t *>(cm + l.off_patch),
-                       reinterpret_cast<const uint16_t *>(cm + l.off_fp), nholes,
-                       static_cast<int>(num_int), static_cast<int>(num_fp), static_cast<uint8_t *>(dst),
-                       static_cast<uint16_t *>(meta), sym_divisor);
-    return check_launch();
+    return static_cast<int>(QUIK_OK);
   };
-  // Few rows: workgroups of two waves, so that the launch still reaches every CU (512 rows in workgroups of eight
-  // are 64 workgroups, a quarter of the CUs, each taking eight rows in turn).  Measured at 8192 columns, period per
-  // launch with two / eight waves: 1280 rows 8.7 / 9.1 us, 1536 rows 9.4 / 9.7, 1792 rows 10.5 / 10.4, 2048 rows
-  // 11.7 / 11.5: the switch is at six rows per CU.
-  if (rows <= int64_t(6) * num_cus()) {
-    switch (J) {
-      case 1: return go(quantize_fp6_wave_kernel<BF16, SYM, 1, 2>, 2);
-      case 2: return go(quantize_fp6_wave_kernel<BF16, SYM, 2, 2>, 2);
-      case 3: return go(quantize_fp6_wave_kernel<BF16, SYM, 3, 2>, 2);
-      case 4: return go(quantize_fp6_wave_kernel<BF16, SYM, 4, 2>, 2);
-      case 5: return go(quantize_fp6_wave_kernel<BF16, SYM, 5, 2>, 2);
-      default: break;
-    }
-  }
-  switch (J) {  // fragments per lane known at compile time: the loops over them unroll
-    case 1: return go(quantize_fp6_wave_kernel<BF16, SYM, 1, 8>, 8);
-    case 2: return go(quantize_fp6_wave_kernel<BF16, SYM, 2, 8>, 8);
-    case 3: return go(quantize_fp6_wave_kernel<BF16, SYM, 3, 8>, 8);
-    case 4: return go(quantize_fp6_wave_kernel<BF16, SYM, 4, 8>, 8);
-    case 5: return go(quantize_fp6_wave_kernel<BF16, SYM, 5, 7>, 7);
-    default: break;
-  }
-  // longer rows: as many waves as fit one CU's LDS, at least one (rows up to 32768 columns: 64 KB per image)
-  if (per_cu >= 4) return go(quantize_fp6_wave_kernel<BF16, SYM, 0, 4>, 4);
-  if (per_cu >= 2) return go(quantize_fp6_wave_kernel<BF16, SYM, 0, 2>, 2);
-  return go(quantize_fp6_wave_kernel<BF16, SYM, 0, 1>, 1);
+  // at most eight waves per workgroup; kStreamMaxCols columns are two fragments per lane
+  return cols <= 8 * 64 * 32 ? go(quantize_fp6_row_kernel<BF16, SYM, 1>, 1) : go(quantize_fp6_row_kernel<BF16, SYM, 2>, 2);
 }
 // asym_quantize_list_kernel: calls that it takes (everything else, and every error, is left to the column map's path).
 // Up to 16384 columns it was the faster one at every row count from 1 to 2048 (2048 x 11008 27.1 -> 25.5, the least); with
@@ -1943,8 +1868,8 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   hipStream_t st = as_stream(stream);
-  return dtype == QUIK_F16 ? launch_fp6_wave<false, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st)
-                           : launch_fp6_wave<true, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st);
+  return dtype == QUIK_F16 ? launch_fp6_row<false, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st)
+                           : launch_fp6_row<true, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st);
 }
 
 extern "C" int quik_asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
@@ -1995,7 +1920,7 @@ int quik::sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const v
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   hipStream_t st = as_stream(stream);
-  if (bits == 4 && tiled) return launch_fp6_wave<false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
+  if (bits == 4 && tiled) return launch_fp6_row<false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
   return bits == 4 ? launch_sym_stream<4>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor)
                    : launch_sym_stream<8>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor);
 }
