@@ -247,8 +247,10 @@ Plan make_plan(int64_t M, int64_t N, bool dma_ok) {
   const int64_t tiles_m = (M + 255) / 256;
   auto rounds = [](int64_t tiles) { return (tiles + num_cus() - 1) / num_cus(); };
   if (!dma_ok) {
-    if (M <= 128 || tiles_m * ((N + 255) / 256) < num_cus() / 2) return {Plan::kMidPlain, 0};
-    return {Plan::kLargePlain, 0};
+    // a round of 128x128 tiles, two per CU, takes 0.64 of a round of 256x256 ones (int4 2048 x 4096 x 3904, one round each:
+    // 45 against 66 us; 4096 x 4096 x 10720, two against one: 190 / 168)
+    const int64_t large = rounds(tiles_m * ((N + 255) / 256)) * 100, pairs = (((M + 127) / 128) * ((N + 127) / 128) + 1) / 2;
+    return {M <= 128 || rounds(pairs) * 64 < large ? Plan::kMidPlain : Plan::kLargePlain, 0};
   }
   const int64_t mid = rounds(((M + 127) / 128) * ((N + 127) / 128)) * kCostMid;
   int64_t best = INT64_MAX, best_n = 0;
@@ -280,21 +282,24 @@ int check_gemm_args(const void *A, const void *B, const void *C, int64_t M, int6
   return QUIK_OK;
 }
 
-// Which row-streaming tile (gemm_rows.h) serves a product, as its number of 32-row blocks; 0: the ring kernels.
-//   one round of 64x64 tiles: always (256 x 4096 x 4096 13.7 -> 8.6 us int4, 18.2 -> 9.9 int8; 512 x 2048 x 11008
-//   30.1 -> 15.8 and 42.1 -> 22.9);
-//   two rounds, few rows and long K, where the weights come from memory and the ring kernels wait for them: 64x64 tiles
-//   (256 x 8192 x 7936 int4 24.4 -> 21.6, 64 x 28672 x 7936 int4 41.9 -> 31.4, int8 61.4 -> 51.5), or for int8 one round of
-//   128x64 tiles (128 x 13824 x 4864 30.7 -> 22.6, 256 x 8192 x 7936 46.6 -> 32.3; int4 is bound by its unpacking there:
-//   23.1).  Shorter K: 128 x 13824 x 4864 int4 (2432 bytes) 16.5 against 16.2 .. 17.2; more rows: 1024 x 4096 x 3840 int4
-//   21.5 against 26.7, 512 x 4096 x 3968 int8 16.2 against 17.4.
+// Which row-streaming tile (gemm_rows.h) serves a product, as its number of 32-row blocks; 0: the ring or plain kernels.
+//   one round of 64x64 tiles: always (256 x 4096 x 4096 13.7 -> 8.3 us int4, 18.2 -> 9.9 int8; 122 x 2312 x 1344 int4 11.6 -> 5.0);
+//   one round of 128x64 tiles, K long enough for their exchange, 2 us more than the ring kernels' epilogue (512 x 4096 x 3968
+//   int4 14.7 -> 13.5, int8 16.9 -> 14.9; 2048 x 1024 x 7936 24.8 -> 19.7 and 29.7 -> 24.7; 300 x 4544 x 4352 14.8 -> 12.9; 128 x
+//   13824 x 4864 16.4 -> 13.6; but 512 x 4096 x 1024 int4 6.9 -> 7.2, 512 x 4096 x 2048 int8 10.9 -> 11.6);
+//   two rounds of 64x64 tiles, few rows and long K, where the weights come from memory and the ring kernels wait for them
+//   (64 x 28672 x 7936 int4 41.1 -> 31.8, int8 61.4 -> 51.5; 64 x 28672 x 2048 int4 12.2 -> 11.5, int8 13.6 -> 16.0);
+//   rows that are no multiple of 64 bytes, which leave only the plain kernels otherwise: up to four rounds (155 x 5120 x 13792
+//   int4 75 -> 18, int8 178 -> 37; 680 x 4096 x 10944 int4 61.6 -> 43.7; 300 x 11008 x 3904 34 -> 27; 2048 x 4096 x 3904, eight
+//   rounds, 53.6 against 45 of the plain 128x128 tiles).
 int rows_blocks(int64_t M, int64_t N, int64_t kbytes, int mode) {
-  if (M <= 32 || kbytes % 64 != 0) return 0;
-  const int64_t tiles_n = (N + 63) / 64, tiles = (M + 63) / 64 * tiles_n;
-  if (tiles <= num_cus()) return 2;
-  if (M > 256 || kbytes < 3072) return 0;
-  if (mode == kInt8 && M > 64 && (M + 127) / 128 * tiles_n <= num_cus()) return 4;
-  return tiles <= 2 * num_cus() ? 2 : 0;
+  if (M <= 32 || kbytes > (1 << 24)) return 0;  // (32-bit offsets inside a tile)
+  const int64_t tiles_n = (N + 63) / 64, tiles2 = (M + 63) / 64 * tiles_n, tiles4 = (M + 127) / 128 * tiles_n, cus = num_cus();
+  const bool ragged = kbytes % 64 != 0, long_k = kbytes >= (mode == kInt4 ? 1024 : 3072);
+  if (tiles2 <= cus) return 2;
+  if (tiles4 <= cus && (long_k || ragged)) return 4;
+  if (ragged) return tiles2 <= 4 * cus ? 2 : 0;
+  return M <= 256 && long_k && tiles2 <= 2 * cus ? 2 : 0;
 }
 // 128x64 tiles on the ring kernels: int8 with one tile per CU takes the ring of eight stages, which covers the memory's
 // latency (512 x 4096 x 3968 19.4 -> 16.5 us, 2048 x 1024 x 7936 33.9 -> 28.6); int4 steps are bound by their unpacking
@@ -328,8 +333,7 @@ int run_i32(const uint8_t *X, const uint8_t *W, int32_t *C, int64_t M, int64_t N
   const Plan plan = make_plan(M, N, kbytes % 64 == 0);
   switch (rows_blocks(M, N, kbytes, MODE)) {
     case 2: return launch_i32_rows<RowsCfg<2>, MODE>(a, st);
-    case 4:
-      if constexpr (MODE == kInt8) return launch_i32_rows<RowsCfg<4>, MODE>(a, st);
+    case 4: return launch_i32_rows<RowsCfg<4>, MODE>(a, st);
     default: break;
   }
   switch (plan.kind) {
@@ -396,8 +400,7 @@ template <int MODE, bool ASYM>
 int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
   switch (rows_blocks(a.M, a.N, a.kbytes, MODE)) {
     case 2: return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
-    case 4:
-      if constexpr (MODE == kInt8) return launch_chain_rows<RowsCfg<4>, MODE, ASYM>(a, e, st);
+    case 4: return launch_chain_rows<RowsCfg<4>, MODE, ASYM>(a, e, st);
     default: break;
   }
   const Plan plan = make_plan(a.M, a.N, a.kbytes % 64 == 0);

@@ -85,6 +85,16 @@ struct FragOps {
       u[0] = raw;
     }
   }
+  template <int PART>
+  static __device__ __forceinline__ void unpack_part(const v4i raw, v4i &u) {
+    if constexpr (MODE == kInt4) {
+      v4i other;
+      if constexpr (PART == 0) unpack_i4(raw, u, other);
+      if constexpr (PART == 1) unpack_i4(raw, other, u);
+    } else {
+      u = raw;
+    }
+  }
   // acc += w_frag (rows: output columns n) x x_frag (columns: token rows m)
   template <typename AccT>
   static __device__ __forceinline__ void mma(const v4i x, const v4i w, AccT &acc) {

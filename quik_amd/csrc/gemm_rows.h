@@ -10,10 +10,13 @@
 // registers; 128x64 tiles have room for one and one, enough for the longer multiplication of a stage.  Afterwards the
 // waves add their sums through LDS (integers: in any order), each ending up with the blocks it stores.
 //
-// Measured (launch in a graph, us): int4 256 x 4096 x 4096 13.7 -> 8.6 (fused dequantize 15.2 -> 9.2), 40 x 4096 x 3968
-// 12.6 -> 7.4; int8 256 x 4096 x 4096 18.2 -> 9.9, 128 x 13824 x 4864 30.7 -> 22.6.  What is left (256 rows, 4096
-// columns, over K): 4 .. 5 us of launch, first copies, exchange and stores, then per stage of 16 KB 174 ns at 8 bits (94
-// bytes per ns and CU) and 220 .. 260 at 4 bits, where a stage is twice the products and has to be unpacked.
+// One wave per SIMD: whatever else it issues stands between its MFMAs.  A copy holds the wave until the memory pipeline has
+// taken its addresses, so the copies go one by one between MFMAs (128x64 tiles: of the first half, so that the next stage
+// has landed when it is read), the unpacking of int4 and the LDS reads of the next stage too.  Launch in a graph, us: int4 256 x
+// 4096 x 4096 13.7 (ring) -> 8.6 (copies in a burst) -> 8.3, 40 x 4096 x 3968 12.6 -> 7.6 -> 7.0, 128x64 tiles 256 x 8192 x 7936 24.1 (ring)
+// -> 24.8 -> 18.9.  What is left, 128x64 tiles at 4 bits over K: 28 ns per MFMA, the sum of its 32 cycles and of six vector
+// instructions and half a copy (at 8 bits 24 KB of operands in 290 ns, 83 bytes per ns and CU).  One ring shared by the four
+// waves, six stages deep, each wave taking 32 bytes of every stage behind a barrier, was slower (256 x 4096 x 4096 10.2 us).
 #pragma once
 #include "gemm_kernels.h"
 
@@ -61,30 +64,35 @@ __device__ __forceinline__ void rows_mainloop(const uint8_t *__restrict__ X, int
     const int row = (j < 4 * MI ? j : j - 4 * MI) * 8 + lrow, rows = j < 4 * MI ? rows_x : rows_w;
     voff[j] = static_cast<uint32_t>(row < rows ? row : rows - 1) * static_cast<uint32_t>(kbytes) + gchunk * 16;
   }
-  // stages wave, wave + WAVES, ...; the last one may be half a stage, whose second half is never multiplied: its
-  // copies take the first half twice, to stay inside the rows
-  const int stages = (kbytes + R::BKB - 1) / R::BKB;
+  // whole stages wave, wave + WAVES, ...; what is left behind the last whole stage goes straight into registers, 32 bytes
+  // per wave and zeros past the end, and is multiplied last
+  const int stages = kbytes / R::BKB, rest = kbytes - stages * R::BKB;
   const int mine = stages > wave ? (stages - wave + WAVES - 1) / WAVES : 0;
-  const uint32_t half_off = gchunk >= 4 ? 64u : 0u;
-  auto issue = [&](int i) QUIK_INLINE {
-    const int kb = (i * WAVES + wave) * R::BKB;
-    const uint32_t back = kb + R::BKB > kbytes ? half_off : 0u;
-    const uint32_t slot = lds0 + (i & (NS - 1)) * R::STAGE;
-    static_for<R::kLoads>([&](auto J) QUIK_INLINE {
-      constexpr int j = J;
-      dma_load16((j < 4 * MI ? X : W) + kb, voff[j] - back, slot + j * 1024);
-    });
+  const int h = lane >> 5;
+  v4i rest_f[NF];
+#pragma unroll
+  for (int j = 0; j < NF; ++j) rest_f[j] = v4i{0, 0, 0, 0};
+  if (rest > 32 * wave + 16 * h) {
+#pragma unroll
+    for (int j = 0; j < NF; ++j) {
+      const int row = (j < MI ? j : j - MI) * 32 + (lane & 31), rows = j < MI ? rows_x : rows_w;
+      rest_f[j] = *reinterpret_cast<const v4i *>((j < MI ? X : W) + static_cast<uint32_t>(row < rows ? row : rows - 1) * static_cast<uint32_t>(kbytes) +
+                                                 stages * R::BKB + 32 * wave + 16 * h);
+    }
+  }
+  auto issue_one = [&](int i, auto J) QUIK_INLINE {
+    constexpr int j = J;
+    dma_load16((j < 4 * MI ? X : W) + (i * WAVES + wave) * R::BKB, voff[j], lds0 + (i & (NS - 1)) * R::STAGE + j * 1024);
   };
+  auto issue = [&](int i) QUIK_INLINE { static_for<R::kLoads>([&](auto J) QUIK_INLINE { issue_one(i, J); }); };
   v4i raw[NS][KS][NF];  // [parity][sub-step][row blocks of X, of W]
-  const int r_off = (lane & 31) * R::BKB, swz = lane & 7, h = lane >> 5;
-  auto read = [&](auto P, int i) QUIK_INLINE {
+  const int r_off = (lane & 31) * R::BKB, swz = lane & 7;
+  auto read_one = [&](auto P, int i, auto S, auto J) QUIK_INLINE {
     const uint8_t *slot = ring + (i & (NS - 1)) * R::STAGE + r_off;
-    static_for<KS>([&](auto S) QUIK_INLINE {
-      const int place = ((2 * S + h) ^ swz) << 4;
-      static_for<NF>([&](auto J) QUIK_INLINE {
-        raw[P][S][J] = *reinterpret_cast<const v4i *>(slot + place + J * 32 * R::BKB);
-      });
-    });
+    raw[P][S][J] = *reinterpret_cast<const v4i *>(slot + (((2 * S + h) ^ swz) << 4) + J * 32 * R::BKB);
+  };
+  auto read = [&](auto P, int i) QUIK_INLINE {
+    static_for<KS>([&](auto S) QUIK_INLINE { static_for<NF>([&](auto J) QUIK_INLINE { read_one(P, i, S, J); }); });
   };
   v16i acc[MI][2];
 #pragma unroll
@@ -93,24 +101,55 @@ __device__ __forceinline__ void rows_mainloop(const uint8_t *__restrict__ X, int
     for (int ni = 0; ni < 2; ++ni)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
-  auto multiply = [&](auto P, int i) QUIK_INLINE {
-    const int live = kbytes - (i * WAVES + wave) * R::BKB;
+  // The products of stage i (in raw[P]), one MFMA at a time with what else the wave has to issue between them: a share of the
+  // next sub-step's unpacking, one copy of stage i + NS (COPY; its slot is free: the caller has waited for the reads of
+  // stage i) and, in the last sub-step, the reads of stage i + 1 (READ).  A copy holds the wave until the memory pipeline
+  // has taken its addresses: in one burst in front of the products they cost a stage as much as its products.
+  v4i u[2][NF][H];
+  auto unpack = [&](const v4i (&f)[NF], auto S, auto Q) QUIK_INLINE {  // piece Q of sub-step S
+    v4i &to = u[S & 1][Q / H][Q % H];
+    Ops::template unpack_part<Q % H>(f[Q / H], to);
+    if constexpr (H > 1) asm volatile("" : "+v"(to));  // (stays between its MFMAs; empty statement: no hazard)
+  };
+  constexpr int MM = H * 2 * MI, PIECES = NF * H;
+  auto mma = [&](auto S, auto T) QUIK_INLINE {
+    constexpr int s = S, t = T, hh = t / (2 * MI), ni = t / MI % 2, mi = t % MI;
+    Ops::mma(u[s & 1][mi][hh], u[s & 1][MI + ni][hh], acc[mi][ni]);
+  };
+  constexpr std::integral_constant<int, 0> kZero{};
+  auto multiply = [&](auto P, int i, auto COPY, auto READ) QUIK_INLINE {
+    // the copies share the MFMAs of the sub-steps in front of the reads; with one slot, where the next stage is awaited right
+    // behind the products, those of the first half
+    constexpr int SLOTS = (NS > 1 ? KS - 1 : KS / 2) * MM;
+    static_for<PIECES>([&](auto Q) QUIK_INLINE { unpack(raw[P][0], kZero, Q); });
+    __builtin_amdgcn_sched_barrier(0);
     static_for<KS>([&](auto S) QUIK_INLINE {
-      if (S >= KS / 2 && live < R::BKB) return;
-      v4i ux[MI][H], uw[2][H];
-#pragma unroll
-      for (int j = 0; j < MI; ++j) Ops::unpack(raw[P][S][j], ux[j]);
-#pragma unroll
-      for (int j = 0; j < 2; ++j) Ops::unpack(raw[P][S][MI + j], uw[j]);
-#pragma unroll
-      for (int hh = 0; hh < H; ++hh)
-#pragma unroll
-        for (int ni = 0; ni < 2; ++ni)
-#pragma unroll
-          for (int mi = 0; mi < MI; ++mi) Ops::mma(ux[mi][hh], uw[ni][hh], acc[mi][ni]);
+      if constexpr (READ && S == KS - 1) wait_copies<(COPY && NS > 1 ? R::kLoads : 0)>();
+      static_for<MM>([&](auto T) QUIK_INLINE {
+        constexpr int s = S, t = T, at = s * MM + t;
+        mma(S, T);
+        if constexpr (s + 1 < KS)
+          static_for<(t + 1) * PIECES / MM - t * PIECES / MM>([&](auto Q) QUIK_INLINE {
+            unpack(raw[P][s + 1], std::integral_constant<int, s + 1>{}, std::integral_constant<int, t * PIECES / MM + Q>{});
+          });
+        if constexpr (COPY && at < SLOTS)
+          static_for<(at + 1) * R::kLoads / SLOTS - at * R::kLoads / SLOTS>(
+              [&](auto J) QUIK_INLINE { issue_one(i + NS, std::integral_constant<int, at * R::kLoads / SLOTS + J>{}); });
+        if constexpr (READ && s == KS - 1)
+          static_for<(t + 1) * KS * NF / MM - t * KS * NF / MM>([&](auto J) QUIK_INLINE {
+            constexpr int k = t * KS * NF / MM + J;
+            read_one(std::integral_constant<int, (NS > 1 ? 1 - P : 0)>{}, i + 1, std::integral_constant<int, k / NF>{},
+                     std::integral_constant<int, k % NF>{});
+          });
+        __builtin_amdgcn_sched_barrier(0);
+      });
     });
   };
 
+  // (a wait only: no hazard)
+  auto in_registers = [&]() QUIK_INLINE { asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory"); };
+  constexpr std::true_type kYes{};
+  constexpr std::false_type kNo{};
   if (mine > 0) issue(0);
   if (NS > 1 && mine > 1) {
     issue(1);
@@ -118,33 +157,36 @@ __device__ __forceinline__ void rows_mainloop(const uint8_t *__restrict__ X, int
   } else {
     wait_copies<0>();
   }
-  if (mine > 0) read(std::integral_constant<int, 0>{}, 0);
-  auto step = [&](auto P, int i) QUIK_INLINE {
-    asm volatile("s_waitcnt lgkmcnt(0)" : : : "memory");  // stage i is in registers: its slot is free
-    if constexpr (NS == 1) {
-      if (i + 1 < mine) issue(i + 1);
-      multiply(P, i);
-      __builtin_amdgcn_sched_barrier(0);  // (the wait stays behind the products)
-      if (i + 1 < mine) {
-        wait_copies<0>();
-        read(P, i + 1);
-      }
-    } else {
-      if (i + 1 < mine) {
-        if (i + 2 < mine) {
-          issue(i + 2);
-          wait_copies<R::kLoads>();
-        } else {
-          wait_copies<0>();
-        }
-        read(std::integral_constant<int, 1 - P>{}, i + 1);
-      }
-      multiply(P, i);
-    }
+  if (mine > 0) read(kZero, 0);
+  int i = 0;
+  auto step = [&](auto P, auto COPY, auto READ) QUIK_INLINE {
+    in_registers();
+    multiply(P, i, COPY, READ);
+    ++i;
   };
-  for (int i = 0; i < mine; i += NS) {
-    step(std::integral_constant<int, 0>{}, i);
-    if (NS > 1 && i + 1 < mine) step(std::integral_constant<int, P1>{}, i + 1);
+  constexpr std::integral_constant<int, P1> kOne{};
+  if constexpr (NS == 1) {
+    while (i + 1 < mine) step(kZero, kYes, kYes);
+    if (i < mine) step(kZero, kNo, kNo);
+  } else {
+    while (i + 3 < mine) {
+      step(kZero, kYes, kYes);
+      step(kOne, kYes, kYes);
+    }
+    if (i + 2 < mine) {  // three left
+      step(kZero, kYes, kYes);
+      step(kOne, kNo, kYes);
+      step(kZero, kNo, kNo);
+    } else if (i + 1 < mine) {
+      step(kZero, kNo, kYes);
+      step(kOne, kNo, kNo);
+    } else if (i < mine) {
+      step(kZero, kNo, kNo);
+    }
+  }
+  if (rest > 0) {
+    static_for<PIECES>([&](auto Q) QUIK_INLINE { unpack(rest_f, kZero, Q); });
+    static_for<MM>([&](auto T) QUIK_INLINE { mma(kZero, T); });
   }
 
   // exchange: wave w leaves its sums of the blocks that wave o owns in slots (o, block, w), o adds the three it finds

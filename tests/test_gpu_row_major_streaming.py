@@ -18,6 +18,11 @@ CASES = [  # M, N, bytes of K per row, bits (0: both)
     (100, 64 * 200, 3136, 8), (255, 64 * 101 + 3, 3072, 8),    # 128x64 tiles
     (300, 4500, 512, 0), (513, 2000, 832, 0),                  # ring kernels, 128x64 tiles
     (777, 5128, 256, 0), (1000, 8203, 2624, 0),                # large tiles, both widths
+    # rows that end inside a stage, in every wave's share of it: nothing but the rest, one to five stages in front of it
+    (33, 7, 16, 0), (64, 65, 112, 0), (70, 130, 144, 0), (40, 64, 32 * 9, 0), (129, 100, 416, 0), (100, 72, 5 * 128 + 80, 0),
+    (130, 64 * 129, 1040, 0), (300, 64 * 61 + 3, 560, 0),      # the same on 128x64 tiles
+    (200, 64 * 230, 240, 0), (600, 6700, 688, 0), (1100, 9000, 208, 0),  # and on several rounds, and on the plain kernels
+    (130, 64 * 128, 1024, 4), (257, 64 * 85, 1088, 4), (130, 64 * 128, 3072, 8),  # 128x64 tiles, whole stages
 ]
 
 
