@@ -248,15 +248,15 @@ __device__ __forceinline__ void block_minmax(float &mn, float &mx, float *red) {
     const int wave = threadIdx.x >> 6;
     if ((threadIdx.x & 63) == 0) {
       red[wave] = mn;
-      red[4 + wave] = mx;
+      red[TPR / 64 + wave] = mx;
     }
     __syncthreads();
     mn = red[0];
-    mx = red[4];
+    mx = red[TPR / 64];
 #pragma unroll
     for (int w = 1; w < TPR / 64; ++w) {
       mn = fminf(mn, red[w]);
-      mx = fmaxf(mx, red[4 + w]);
+      mx = fmaxf(mx, red[TPR / 64 + w]);
     }
   }
 }
@@ -692,13 +692,16 @@ __global__ __launch_bounds__(TPR) void asym_quantize_stream_kernel(
     const IdxT *__restrict__ fp_col, const uint32_t *__restrict__ mask, const uint32_t *__restrict__ grp,
     const uint32_t *__restrict__ dirty, const uint16_t *__restrict__ dirty_grp, const uint32_t *__restrict__ flags,
     int64_t num_int, int64_t num_fp, uint8_t *__restrict__ dst, uint16_t *__restrict__ meta,
-    uint16_t *__restrict__ fp_x, int vec_out, float sym_divisor) {
+    uint16_t *__restrict__ fp_x, int vec_out, float sym_divisor, int known_ndirty) {
   static_assert(sizeof(IdxT) == 2, "streaming needs cols <= 32768");
   extern __shared__ __align__(16) uint16_t row_s[];
   __shared__ float red[64];
-  if (flags[0] & 1u) {
+  // known_ndirty: the map streams and has that many dirty groups, says the host (-1: it does not know).  Its flag words
+  // are a round trip to memory in front of everything else otherwise.
+  if (known_ndirty >= 0 || (flags[0] & 1u)) {
     uint8_t *codes_s = reinterpret_cast<uint8_t *>(row_s);
-    stream_rows<BITS, BF16, NV, TPR, SYM, PF>(x, rows, cols, grp, dirty, dirty_grp, static_cast<int>(flags[1]),
+    stream_rows<BITS, BF16, NV, TPR, SYM, PF>(x, rows, cols, grp, dirty, dirty_grp,
+                                          known_ndirty >= 0 ? known_ndirty : static_cast<int>(flags[1]),
                                           reinterpret_cast<const uint16_t *>(fp_col), num_int, num_fp, dst, meta, fp_x,
                                           codes_s, red, vec_out, sym_divisor);
   } else if constexpr (!SYM) {
@@ -1537,6 +1540,11 @@ int grid_for(int64_t work_items, int64_t per_block) {
 
 constexpr int64_t kMaxLdsRowBytes = 128 * 1024;  // of the 160 KB per CU
 
+// Few rows of more than 4096 columns: eight waves per row instead of four, while the rows leave half of the CUs without one
+// (us per launch: int8 16 x 13824 5.2 -> 4.8, 32 x 28672 7.6 -> 6.8, bf16 16 x 13824 5.7 -> 5.1, int4 32 x 8192 4.1 -> 3.8; 256 x 28672 bf16
+// 11.8 -> 10.7, 512 x 11008 9.3 -> 8.8 but fp16 256 x 8192 4.3 -> 4.4; sixteen waves were slower than eight everywhere).
+int64_t wide_rows() { return num_cus() / 2; }
+
 template <typename IdxT, int BITS, bool BF16, int NV, int TPR, bool SYM = false, bool PF = false>
 int launch_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, const ColmapLayout &l, int64_t num_int,
                   int64_t num_fp, void *dst, void *meta, void *fp_x, hipStream_t st, bool tiled,
@@ -1552,6 +1560,9 @@ int launch_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, 
       return QUIK_ERR_LAUNCH;
     }
   }
+  uint32_t words[4];
+  const bool known = colmap_words_known(cm, cols, num_int, num_fp, words) && (words[0] & kColmapStreams);
+  const int known_ndirty = known ? static_cast<int>(words[1]) : -1;
   const int64_t items = tiled ? (rows + 7) / 8 * 8 : rows;
   int grid = static_cast<int>(items < (int64_t(1) << 30) ? items : (int64_t(1) << 30));
   if (PF && grid > 2 * num_cus()) grid = 2 * num_cus();  // persistent: the workgroups that are resident at once
@@ -1565,7 +1576,7 @@ int launch_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, 
                      reinterpret_cast<const uint16_t *>(cm + l.off_slot),
                      reinterpret_cast<const uint32_t *>(cm + l.off_flags), num_int, num_fp,
                      static_cast<uint8_t *>(dst), static_cast<uint16_t *>(meta), static_cast<uint16_t *>(fp_x), vec_out,
-                     sym_divisor);
+                     sym_divisor, known_ndirty);
   return check_launch();
 }
 
@@ -1575,13 +1586,18 @@ int launch_sym_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *
                       int64_t num_int, int64_t num_fp, void *dst, void *scale, void *fp_x, hipStream_t st, bool tiled,
                       float divisor) {
   const int64_t groups = cols / 8;
-#define QUIK_SYM_STREAM(NV)                                                                                       \
-  return launch_stream<uint16_t, BITS, false, NV, kThreads, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, \
-                                                                  fp_x, st, tiled, divisor)
-  if (groups <= 512) QUIK_SYM_STREAM(2);
-  if (groups <= 1024) QUIK_SYM_STREAM(4);
-  if (groups <= 2048) QUIK_SYM_STREAM(8);
-  QUIK_SYM_STREAM(16);
+#define QUIK_SYM_STREAM(NV, TPR)                                                                             \
+  return launch_stream<uint16_t, BITS, false, NV, TPR, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, \
+                                                             fp_x, st, tiled, divisor)
+  if (groups <= 512) QUIK_SYM_STREAM(2, kThreads);
+  if (rows <= wide_rows()) {
+    if (groups <= 1024) QUIK_SYM_STREAM(2, 512);
+    if (groups <= 2048) QUIK_SYM_STREAM(4, 512);
+    QUIK_SYM_STREAM(8, 512);
+  }
+  if (groups <= 1024) QUIK_SYM_STREAM(4, kThreads);
+  if (groups <= 2048) QUIK_SYM_STREAM(8, kThreads);
+  QUIK_SYM_STREAM(16, kThreads);
 #undef QUIK_SYM_STREAM
 }
 
@@ -1648,13 +1664,18 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
     // Four waves per row, one row per workgroup: more, shorter waves hide the load and LDS latencies
     // better than fewer waves with less per-row fixed work (measured with 64, 128 and 256 threads).
     const int64_t groups = cols / 8;
-#define QUIK_STREAM(NV) \
-  return launch_stream<IdxT, BITS, BF16, NV, kThreads>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, tiled)
+#define QUIK_STREAM(NV, TPR) \
+  return launch_stream<IdxT, BITS, BF16, NV, TPR>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, tiled)
     // fp16 rows beyond 8192 columns with tile-ordered int8 output: the LDS ring kernel
     if constexpr (BITS == 8 && !BF16) {
       if (tiled && ring_fits(cols, num_int, num_fp, ndirty) && ngather <= kRingThreads)
         return launch_tile8_ring(x, rows, cols, cm, l, num_int, num_fp, static_cast<int>(ndirty),
                                  static_cast<int>(ngather), dst, meta, st);
+    }
+    if (groups > 512 && rows <= wide_rows()) {
+      if (groups <= 1024) QUIK_STREAM(2, 512);
+      if (groups <= 2048) QUIK_STREAM(4, 512);
+      QUIK_STREAM(8, 512);
     }
     // bf16 rows beyond 16384 columns (and fp16 ones the ring kernel does not take: more than 512 outlier columns):
     // 180 registers per lane leave room for two workgroups per CU, so the launch is persistent and prefetches the
@@ -1665,10 +1686,10 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
         return launch_stream<IdxT, BITS, BF16, 16, kThreads, false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, meta,
                                                                           fp_x, st, tiled);
     }
-    if (groups <= 512) QUIK_STREAM(2);
-    if (groups <= 1024) QUIK_STREAM(4);
-    if (groups <= 2048) QUIK_STREAM(8);
-    QUIK_STREAM(16);
+    if (groups <= 512) QUIK_STREAM(2, kThreads);
+    if (groups <= 1024) QUIK_STREAM(4, kThreads);
+    if (groups <= 2048) QUIK_STREAM(8, kThreads);
+    QUIK_STREAM(16, kThreads);
 #undef QUIK_STREAM
   }
   if (tiled) return QUIK_ERR_SHAPE;  // tile-ordered output exists on the streaming path only
