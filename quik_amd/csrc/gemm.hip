@@ -24,9 +24,11 @@ using CfgL = Cfg<256, 256, 2, 2, 2>;   // prefill: 128x128 per wave, 256 accumul
 using CfgH = Cfg<256, 128, 2, 2, 2>;   // half-width tile that evens out the last round
 using CfgM = Cfg<128, 128, 2, 2, 2>;   // mid-size problems, two workgroups per CU
 using CfgN = Cfg<128, 64, 2, 2, 2>;    // few tiles: narrower ones put more CUs to work, three workgroups per CU
-using CfgN6 = Cfg<128, 64, 2, 2, 2>;   // 6-bit path, 86 .. ~150 tiles of 128x128 and no K split: twice as many workgroups
-using CfgN8 = Cfg<128, 64, 2, 2, 2, 8>; // the same, one workgroup per CU with eight stages of copies
-using CfgD6 = Cfg<128, 64, 2, 2, 2, 8>; // the same with one workgroup per CU and twelve slots
+// with one workgroup per CU, the LDS of a CU full of copies in flight: eight stages here, up to twelve slots in the tile-ordered
+// rings (ring_slots)
+using CfgDN = Cfg<128, 64, 2, 2, 2, 8>;
+using CfgDM = Cfg<128, 128, 2, 2, 2, 8>;
+using CfgDH = Cfg<256, 128, 2, 2, 2, 8>;
 using CfgL8 = Cfg<256, 256, 2, 4, 2>;  // 6-bit path, launches of 256x256 tiles only: two waves per SIMD (1-5 % faster than CfgL)
 using CfgLp = Cfg<256, 256, 2, 2, 0>;  // plain fallbacks
 using CfgMp = Cfg<128, 128, 2, 2, 0>;
@@ -349,7 +351,7 @@ int run_i32(const uint8_t *X, const uint8_t *W, int32_t *C, int64_t M, int64_t N
     case Plan::kMid: return launch_i32<CfgM, MODE>(a, st);
     case Plan::kNarrow:
       if constexpr (MODE == kInt8) {
-        if (deep_ring(M, N, MODE)) return launch_i32<CfgN8, MODE>(a, st);
+        if (deep_ring(M, N, MODE)) return launch_i32<CfgDN, MODE>(a, st);
       }
       return launch_i32<CfgN, MODE>(a, st);
     case Plan::kMidPlain: return launch_i32<CfgMp, MODE>(a, st);
@@ -409,7 +411,7 @@ int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
     case Plan::kMid: return launch_chain<CfgM, MODE, ASYM>(a, e, st);
     case Plan::kNarrow:
       if constexpr (MODE == kInt8) {
-        if (deep_ring(a.M, a.N, MODE)) return launch_chain<CfgN8, MODE, ASYM>(a, e, st);
+        if (deep_ring(a.M, a.N, MODE)) return launch_chain<CfgDN, MODE, ASYM>(a, e, st);
       }
       return launch_chain<CfgN, MODE, ASYM>(a, e, st);
     case Plan::kMidPlain:
@@ -535,40 +537,47 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
   return check_launch();
 }
 
-// Register-streaming kernel (gemm_direct.h) or ring kernel, for problems below the 256-row tiles.  Both are priced in ns:
-// a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (alone, over K, 87 .. 94 here and 87 in the
-// ring kernel), never less than the weights at 5.5 TB/s, and for a K split the exchange (its partial sums cross memory:
-// 16 KB per workgroup here, 64 KB in the ring kernel).  Against every variant on 29 shapes of 40 .. 2048 rows, 1024 ..
-// 28672 columns, both widths, weights in the Infinity Cache: within 0.5 us of the fastest on 25; 1.5 us behind on 64 x 8192
-// -> 8192, 64 x 5120 -> 13824 and (8 bits) 64 x 11008 -> 4096, 7 us on (8 bits) 64 x 28672 -> 8192 (44.0 against 36.9 with
-// 64x32 tiles): all variants cost the stream's floor there, and from that cache the weights come faster.
+// Register-streaming kernel (gemm_direct.h), ring kernel or ring kernel with a K split, for problems below the 256-row
+// tiles.  All are priced in ns: a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (87 in the ring
+// of 128x64 tiles), never less than the weights take: up to 64 MB, which the Infinity Cache keeps beside other layers' of
+// that size, at 8 TB/s (64 x 8192 -> 8192, 52 MB: 64x32 tiles 15.9 us per forward, 64x64 17.6); more from memory, at what each
+// kernel reaches, and at most 24 bytes per ns for each CU that works (8 bits, 64 x 28672 -> 8192, 232 MB: 64x64 tiles 78 us on
+// 128 CUs, 56 on 256, 64x32 tiles 67; 64 x 8192 -> 28672, 176 MB: ring 34).  A K split adds the exchange: its partial sums
+// cross memory, 16 KB per workgroup in the register-streaming kernel, 64 KB in the ring kernel (measured 13 us with its start
+// for two workgroups per tile, 22 .. 24 for three to eight).
 struct DirectPlan {
-  int bn, splits;  // tile width (64 or 32; 0: ring kernel), workgroups per tile
-  int64_t bytes;   // workspace of the split
+  int bn, splits;   // tile width (64 or 32; 0: ring kernel), workgroups per tile
+  int64_t bytes;    // workspace of the split
+  bool ring_split;  // the ring kernel splits K (plan_splitk)
 };
 DirectPlan plan_direct(int64_t M, int64_t N, int64_t K, int bits, int64_t workspace_bytes) {
-  const DirectPlan ring{0, 1, 0};
-  if (make_plan6(M, N, 1).kind != Plan::kMid) return ring;
+  DirectPlan plan{0, 1, 0, false};
+  if (make_plan6(M, N, 1).kind != Plan::kMid) return plan;
   const int64_t steps = tile_steps(K, bits), unit = bits == 4 ? 3072 : 2048, cus = num_cus();
-  const int64_t stream = N * steps * unit / 64 * 10 / 55000;
+  const int64_t weights = N * steps * unit / 64;
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
-  auto busiest = [&](int64_t groups, int64_t per, int64_t step_bytes) {
-    const int64_t ns = up(groups, cus) * per * step_bytes / 103;
+  auto busiest = [&](int64_t groups, int64_t per, int64_t step_bytes, int64_t rate, int64_t memory) {
+    const int64_t ns = up(groups, cus) * per * step_bytes / rate, by_cus = 24 * (groups < cus ? groups : cus);
+    const int64_t stream = weights / (weights <= (64 << 20) ? 8000 : by_cus < memory ? by_cus : memory);
     return ns > stream ? ns : stream;
   };
-  const int64_t tiles128 = up(M, 128) * up(N, 128);
+  const int64_t tiles128 = up(M, 128) * up(N, 128), tiles64 = up(M, 128) * up(N, 64);
+  int64_t best = 5300 + (bits == 4 && tiles64 <= cus ? busiest(tiles64, steps, 3 * unit, 87, 5500)
+                                                     : busiest(tiles128, steps, 4 * unit, 103, 5500));
   const SplitPlan sp = plan_splitk(M, N, steps, bits == 4 ? kSplitMinSteps6 : kSplitMinSteps8, 1, bits == 4 ? 3 : 2);
-  int64_t best = sp.splits > 1 && workspace_bytes >= sp.bytes ? 10000 + 1500 * sp.splits + busiest(tiles128 * sp.splits, sp.per, 4 * unit)
-                 : bits == 4 && tiles128 * 8 <= cus * 5        ? 5800 + busiest(up(M, 128) * up(N, 64), steps, 3 * unit)
-                                                               : 5800 + busiest(tiles128, steps, 4 * unit);
-  DirectPlan plan = ring;
+  if (sp.splits > 1 && workspace_bytes >= sp.bytes) {
+    const int64_t ns = (sp.splits == 2 ? 13500 : 23500) + busiest(tiles128 * sp.splits, sp.per, 4 * unit, 103, 5500);
+    if (ns < best) best = ns, plan.ring_split = true;
+  }
   for (const int bn : {64, 32}) {
     const int64_t tiles = up(M, 64) * up(N, bn);
     for (const int splits : {1, 2, 4}) {
       const int64_t bytes = splits > 1 ? kSplitCounterBytes + tiles * splits * DirectCfg<true, 2, 2, 4>::PARTIAL_BYTES : 0;
-      if (splits > 1 && (tiles * 4 > kSplitCounterBytes || bytes > workspace_bytes || up(steps, splits) * (splits - 1) >= steps)) continue;
-      const int64_t ns = 6300 + (splits > 1 ? 1500 + 500 * splits : 0) + busiest(tiles * splits, up(steps, splits), unit + unit * bn / 64);
-      if (ns < best) best = ns, plan = {bn, splits, bytes};
+      if (splits > 1 && (tiles * 4 > kSplitCounterBytes || bytes > workspace_bytes || up(steps, splits) * (splits - 1) >= steps))
+        continue;
+      const int64_t ns = 6300 + (splits > 1 ? 1500 + 500 * splits : 0) +
+                         busiest(tiles * splits, up(steps, splits), unit + unit * bn / 64, 103, bn == 64 ? 4300 : 3400);
+      if (ns < best) best = ns, plan = {bn, splits, bytes, false};
     }
   }
   return plan;
@@ -592,14 +601,11 @@ int launch_direct(const Args &p, int splits, void *workspace, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(grid), dim3(D::kThreads), D::SMEM, st, p, tiles_m, tiles_n);
   return check_launch();
 }
-// kChainNotHandled: the ring kernels serve this call.  SETS: as many steps in flight as registers allow with two
-// workgroups per CU; more measured no better
+// SETS: as many steps in flight as registers allow with two workgroups per CU; more measured no better
 template <bool SIX, bool BF16, class Args>
-int run_direct(const Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
-  const DirectPlan d = plan_direct(p.M, p.N, p.K, SIX ? 4 : 8, workspace ? workspace_bytes : 0);
+int run_direct(const Args &p, const DirectPlan &d, void *workspace, hipStream_t st) {
   if (d.bn == 64) return launch_direct<DirectCfg<SIX, 2, 2, SIX ? 4 : 6>, BF16>(p, d.splits, workspace, st);
-  if (d.bn == 32) return launch_direct<DirectCfg<SIX, 2, 1, SIX ? 8 : 10>, BF16>(p, d.splits, workspace, st);
-  return kChainNotHandled;
+  return launch_direct<DirectCfg<SIX, 2, 1, SIX ? 8 : 10>, BF16>(p, d.splits, workspace, st);
 }
 
 // The 6-bit matrix-core path (gemm_fp6.h): 256x256 tiles alone (eight waves), 256x256 + 256x128 tiles in one
@@ -633,27 +639,23 @@ template <bool BF16>
 int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
   // any row count: up to 32 rows the weight-streaming kernel on the packed nibbles reads a third fewer bytes, and
   // callers that keep both weight copies route such calls there
-  if (const int rc = run_direct<true, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
+  const DirectPlan d = plan_direct(p.M, p.N, p.K, 4, workspace ? workspace_bytes : 0);
+  if (d.bn) return run_direct<true, BF16>(p, d, workspace, st);
+  if (d.ring_split)
+    return launch_fused6_splitk<BF16>(p, plan_splitk(p.M, p.N, tile_steps(p.K, 4), kSplitMinSteps6, 1, 3), workspace, st);
   const Plan plan = make_plan6(p.M, p.N, 1);
   if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0)
     return launch_rest<CfgL, CfgM>(gemm_fused6_rest_kernel<CfgL, CfgM, BF16>, fused6_smem<CfgL>(), p, n_wide, st);
   if (plan.kind == Plan::kSplit && plan.n_wide >= p.N) return launch_fused6<CfgL8, BF16>(p, st);
   if (plan.kind != Plan::kSplit) {
-    const SplitPlan sp = plan_splitk(p.M, p.N, tile_steps(p.K, 4), kSplitMinSteps6, 1, 3);
-    if (sp.splits > 1 && workspace && workspace_bytes >= sp.bytes) return launch_fused6_splitk<BF16>(p, sp, workspace, st);
-    // too few 128x128 tiles for the CUs and no K split (it takes three workgroups per tile to pay): 128x64 tiles
-    const int64_t mid_tiles = ((p.M + 127) / 128) * ((p.N + 127) / 128);
-    // (up to 0.62 tiles per CU: measured 6 - 12 % less time on 13B gate_proj at 128 tokens, 70B k_proj and the
-    // 512 x 4096 x 4096 configuration; with 0.88 tiles per CU, 70B gate_proj at 64 tokens, 11 % more)
-    if (mid_tiles * 8 <= int64_t(num_cus()) * 5) {
-      // One tile per CU: a ring of twelve slots (110 KB of LDS) instead of six, nine steps in flight instead of three.  Layer
-      // forward 300 x 4544 -> 4544 19.1 -> 18.6 us, 2048 x 8192 -> 1024 31.3 -> 30.7, 128 x 5120 -> 13824 20.3 -> 20.0, 256 x
-      // 8192 -> 8192 26.5 -> 25.9: a step takes 106 ns, some 210 cycles, for 64 of MFMA, against 111 ns with six slots (two
-      // steps between barriers, or no second copy of the W block, changed nothing on top).  More tiles need two
-      // workgroups per CU, which six slots allow.
-      if ((p.M + 127) / 128 * ((p.N + 63) / 64) <= num_cus()) return launch_fused6<CfgD6, BF16>(p, st);
-      return launch_fused6<CfgN6, BF16>(p, st);
-    }
+    // One 128x64 tile per CU: a ring of twelve slots (110 KB of LDS) instead of six, nine steps in flight instead of three.
+    // Layer forward 300 x 4544 -> 4544 19.1 -> 18.6 us, 2048 x 8192 -> 1024 31.3 -> 30.7, 128 x 5120 -> 13824 20.3 -> 20.0, 256 x
+    // 8192 -> 8192 26.5 -> 25.9: a step takes 106 ns, some 210 cycles, for 64 of MFMA, against 111 ns with six slots (two
+    // steps between barriers, or no second copy of the W block, changed nothing on top).
+    // More of them than CUs, two on some, take longer than the half as many 128x128 tiles, one per CU: 512 x 4096 -> 5120
+    // 25.6 -> 20.8, 236 x 13824 -> 10240 80 -> 59.5.
+    if ((p.M + 127) / 128 * ((p.N + 63) / 64) <= num_cus()) return launch_fused6<CfgDN, BF16>(p, st);
+    if ((p.M + 127) / 128 * ((p.N + 127) / 128) <= num_cus()) return launch_fused6<CfgDM, BF16>(p, st);
     return launch_fused6<CfgM, BF16>(p, st);
   }
   Fused6Args wide = p, tail = p;
@@ -665,7 +667,9 @@ int run_fused6(const Fused6Args &p, hipStream_t st, void *workspace, int64_t wor
   tail.w_red = p.w_red ? p.w_red + nw : nullptr;
   tail.bias = p.bias ? p.bias + nw : nullptr;
   tail.out = p.out + nw;
-  return launch_fused6_split<CfgL, CfgH, BF16>(wide, tail, st);
+  // (the 256x128 tiles have the LDS of a CU to themselves as well: eight slots, int8 twelve; 946 x 13824 -> 5120 74.5 -> 73.1 us,
+  // int8 2048 x 11008 -> 4096 102.3 -> 101.0)
+  return launch_fused6_split<CfgL, CfgDH, BF16>(wide, tail, st);
 }
 
 template <class C, bool BF16>
@@ -697,11 +701,15 @@ int launch_fused8t_split(const Fused8Args &wide, const Fused8Args &tail, hipStre
 // W8A8 on tile-ordered operands (gemm_tile8.h): same plan and tile shapes as the 6-bit path.
 template <bool BF16>
 int run_fused8t(const Fused8Args &p, hipStream_t st, void *workspace, int64_t workspace_bytes) {
-  if (const int rc = run_direct<false, BF16>(p, st, workspace, workspace_bytes); rc != kChainNotHandled) return rc;
+  const DirectPlan d = plan_direct(p.M, p.N, p.K, 8, workspace ? workspace_bytes : 0);
+  if (d.bn) return run_direct<false, BF16>(p, d, workspace, st);
+  if (d.ring_split)
+    return launch_fused8t_splitk<BF16>(p, plan_splitk(p.M, p.N, tile_steps(p.K, 8), kSplitMinSteps8, 1, 2), workspace, st);
   const Plan plan = make_plan6(p.M, p.N, 1);  // any row count: with few rows this path competes with the weight-streaming kernel
   if (plan.kind != Plan::kSplit) {
-    const SplitPlan sp = plan_splitk(p.M, p.N, tile_steps(p.K, 8), kSplitMinSteps8, 1, 2);
-    if (sp.splits > 1 && workspace && workspace_bytes >= sp.bytes) return launch_fused8t_splitk<BF16>(p, sp, workspace, st);
+    // one tile per CU: twelve slots, 72 KB in flight instead of 24 (365 x 28672 -> 8192 157 -> 144 us, 652 x 11008 -> 4096
+    // 48.6 -> 46.3)
+    if ((p.M + 127) / 128 * ((p.N + 127) / 128) <= num_cus()) return launch_fused8t<CfgDM, BF16>(p, st);
     return launch_fused8t<CfgM, BF16>(p, st);
   }
   if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0)
@@ -716,7 +724,7 @@ int run_fused8t(const Fused8Args &p, hipStream_t st, void *workspace, int64_t wo
   tail.w_red = p.w_red ? p.w_red + nw : nullptr;
   tail.bias = p.bias ? p.bias + nw : nullptr;
   tail.out = p.out + nw;
-  return launch_fused8t_split<CfgL, CfgH, BF16>(wide, tail, st);
+  return launch_fused8t_split<CfgL, CfgDH, BF16>(wide, tail, st);
 }
 
 template <int MODE, bool BF16>

@@ -18,9 +18,9 @@
 // loop was bound by the cache-to-CU path at a quarter of its rate).  One MFMA k-step (64 elements)
 // of a lane is a 16-byte head read plus an 8-byte tail read, both free of bank conflicts.
 //
-// Pipeline: a ring of 6 LDS slots, one per k-step, filled by global_load_lds_dwordx4.  While step j
-// feeds the MFMAs, the fragments of step j + 1 are read into registers and steps j + 2 .. j + 5 are
-// landing (the slot of step j was handed to step j + 6 when step j's reads were done); the outlier
+// Pipeline: a ring of NS LDS slots (six to twelve), one per k-step, filled by global_load_lds_dwordx4.  While step j
+// feeds the MFMAs, the fragments of step j + 1 are read into registers and steps j + 2 .. j + NS - 1 are
+// landing (the slot of step j was handed to step j + NS when step j's reads were done); the outlier
 // GEMM's fp16/bf16 steps (16 elements each, 32 bytes per row like a head) run through the same ring
 // after the integer steps.
 #pragma once
@@ -43,10 +43,18 @@ __device__ __forceinline__ void dma_load16k(const uint8_t *sbase, uint32_t voff,
                : : "s"(lds_addr), "v"(voff), "s"(sbase), "n"(OFFSET) : "memory", "m0");
 }
 
+// LDS slots of the tile-ordered rings, `stage` bytes each: six, or with one workgroup per CU (DMA_STAGES > 4) as many as
+// fit 144 KB, an even number, at most twelve.
+template <class C>
+constexpr int ring_slots(int stage) {
+  const int most = 144 * 1024 / stage / 2 * 2;
+  return C::DMA_STAGES <= 4 ? 6 : most < 12 ? most : 12;
+}
+
 template <class C>
 struct Fp6Pipe {
   static constexpr int MI = C::MI, NI = C::NI, NF = MI + NI;
-  static constexpr int NS = C::DMA_STAGES > 4 ? 12 : 6;  // LDS slots; one step is multiplied, NS - 1 are landed or in flight
+  static constexpr int NS = ring_slots<C>((C::BM + C::BN) * 48);  // LDS slots; one step is multiplied, NS - 1 are landed or in flight
   // a wave's fragments start at a 64-row block of the operand, or the wave has a single 32-row fragment (then it may
   // be the second half of a block)
   static_assert(C::WM % 64 == 0 || C::MI == 1, "a wave's token rows");

@@ -13,8 +13,8 @@
 // A block's units are contiguous: K / 32 integer steps, then F / 16 outlier steps (16 fp16 / bf16 values =
 // 32 bytes per row, same image).  Needs K % 64 == 0 and F % 32 == 0 (steps are consumed in pairs).
 //
-// Pipeline: ring of 6 LDS slots of one step each ((BM + BN) x 32 bytes), mirroring the units; while step j
-// feeds the MFMAs, the fragments of step j + 1 are read into the second register set and steps j + 2 .. j + 5
+// Pipeline: ring of NS LDS slots (six to twelve) of one step each ((BM + BN) x 32 bytes), mirroring the units; while step j
+// feeds the MFMAs, the fragments of step j + 1 are read into the second register set and steps j + 2 .. j + NS - 1
 // are landing; copies go one by one between groups of MFMAs (see gemm_fp6.h for the reasons).
 #pragma once
 #include "gemm_fp6.h"
@@ -23,7 +23,7 @@ namespace quik {
 
 template <class C>
 struct Tile8Pipe {
-  static constexpr int MI = C::MI, NI = C::NI, NS = 6, NF = MI + NI, MM = MI * NI;
+  static constexpr int MI = C::MI, NI = C::NI, NS = ring_slots<C>((C::BM + C::BN) * 32), NF = MI + NI, MM = MI * NI;
   static_assert(C::WM % 64 == 0 && C::WN % 64 == 0, "a wave's rows start at a 64-row block");
   static_assert(C::WAVES == 4 || C::WAVES == 8, "copy assignment below");
   static constexpr int W_OFF = C::BM * 32;
@@ -38,7 +38,7 @@ struct Tile8Pipe {
   static_assert((XB == 4 && (WB == 4 || WB == 2)) || (XB == 2 && WB == 2), "supported tile shapes");
   static_assert(C::WAVES == 4 || XB + WB == 8, "eight waves copy eight blocks");
   static constexpr int P = 2 + NB;  // copies per wave and step
-  static_assert(3 * P <= 63, "three steps in flight must fit the vmcnt counter");
+  static_assert((NS - 3) * P <= 63, "the steps in flight must fit the vmcnt counter");
 
   uint8_t *smem;
   uint32_t lds0;
@@ -50,7 +50,7 @@ struct Tile8Pipe {
   uint32_t rd;              // byte offset of the slot the next fragment read looks at
   int steps0, steps;        // integer steps, all steps
   uint32_t x_head, w_head;  // this lane's fragment offsets inside a slot (fragment j: + 2048 (j / 2) + 1024 (j % 2))
-  uint32_t x_head3[3], w_head3[3];  // the same inside slots 0, 2, 4
+  uint32_t x_head3[NS / 2], w_head3[NS / 2];  // the same inside slots 0, 2, 4, ..
 
   // unit0: first unit (step) of every block to copy; n_int / n_f: integer and outlier steps from there on
   // (-1: all of the block's, from its first unit)
@@ -94,7 +94,7 @@ struct Tile8Pipe {
     x_head = (wm * C::WM / 64) * 2048 + r * 32 + slot16;
     w_head = W_OFF + (wn * C::WN / 64) * 2048 + r * 32 + slot16;
 #pragma unroll
-    for (int q = 0; q < 3; ++q) {
+    for (int q = 0; q < NS / 2; ++q) {
       x_head3[q] = x_head + q * 2 * STAGE;
       w_head3[q] = w_head + q * 2 * STAGE;
     }
@@ -130,14 +130,10 @@ struct Tile8Pipe {
     }
   }
 
-  // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. 4 are in flight.
+  // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. NS - 2 are in flight.
   __device__ __forceinline__ void start() {
-    issue();
-    issue();
-    issue();
-    issue();
-    issue();
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * P));
+    static_for<NS - 1>([&](auto) { issue(); });
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
     __syncthreads();
   }
 
@@ -200,25 +196,24 @@ struct Tile8Pipe {
       step<MODE, RS, FS, G + 1>(cf, nf, acc);
     } else {
       if constexpr (RS < 0) next_read_slot();
-      __builtin_amdgcn_s_waitcnt(vmcnt_imm(3 * P));
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
       __builtin_amdgcn_s_barrier();
     }
   }
 
   // Steps [first, last) in MODE (an even number of them); the fragments of step `first` are in f0 on entry and
-  // those of step `last` on exit.  Six steps at a time with the ring slots as immediates when `rd` is at slot
-  // 1 and `fill` at slot 5 (true at the first step of a tile), the rest with `rd` / `fill`.
+  // those of step `last` on exit.  NS steps at a time with the ring slots as immediates when `rd` is at slot
+  // 1 and `fill` at slot NS - 1 (true at the first step of a tile), the rest with `rd` / `fill`.
   template <int MODE, bool ALIGNED>
   __device__ __forceinline__ void run(int first, int last, v4i (&f0)[NF], v4i (&f1)[NF], v16f (&acc)[MI][NI]) {
     int j = first;
     if constexpr (ALIGNED) {
-      for (; j + 6 <= last; j += 6) {
-        step<MODE, 1, 5>(f0, f1, acc);
-        step<MODE, 2, 0>(f1, f0, acc);
-        step<MODE, 3, 1>(f0, f1, acc);
-        step<MODE, 4, 2>(f1, f0, acc);
-        step<MODE, 5, 3>(f0, f1, acc);
-        step<MODE, 0, 4>(f1, f0, acc);
+      for (; j + NS <= last; j += NS) {
+        static_for<NS / 2>([&](auto I) __attribute__((always_inline)) {
+          constexpr int i = 2 * I;
+          step<MODE, i + 1, (i + NS - 1) % NS>(f0, f1, acc);
+          step<MODE, (i + 2) % NS, i>(f1, f0, acc);
+        });
       }
     }
     for (; j < last; j += 2) {

@@ -1,6 +1,6 @@
-"""128x64 tiles of the 6-bit GEMM with one tile per CU (ring of twelve slots): fewer steps than slots, exactly as many, one
-pair more, whole turns with every remainder, none and more outlier steps than slots.  Same output bits as the row-major
-int8-MFMA kernels, which other tests hold against the oracle."""
+"""Tile-ordered GEMMs with one tile per CU (rings of twelve or eight slots): 128x64 tiles at 6 bits, 128x128 and 256x128
+ones at both widths; fewer steps than slots, exactly as many, one pair more, whole turns with every remainder, none and more
+outlier steps than slots.  Same output bits as the row-major int8-MFMA kernels, which other tests hold against the oracle."""
 import pytest
 import torch
 
@@ -12,13 +12,24 @@ DEV = "cuda:0"
 @pytest.mark.parametrize("M,N,K,F", [(128, 13824, 128, 0), (100, 13830, 640, 32), (128, 13824, 768, 288), (127, 13800, 896, 0),
                                      (120, 13824, 1536, 64), (128, 13001, 1792, 256), (300, 5120, 2688, 96), (257, 4544, 4416, 128)])
 def test_same_bits_as_the_row_major_kernels(M, N, K, F, dtype):
+    _same_bits(M, N, K, F, dtype, 4)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K,F", [(200, 10240, 128, 0), (365, 8190, 640, 32), (250, 10201, 768, 288), (380, 8192, 896, 0),
+                                     (300, 8192, 4736, 64), (520, 9100, 384, 32), (600, 9001, 1664, 128)])
+def test_one_wide_tile_per_cu(M, N, K, F, bits):
+    _same_bits(M, N, K, F, torch.float16, bits)
+
+
+def _same_bits(M, N, K, F, dtype, bits):
     from quik_amd.qlinear import MixedQLinear
     g = torch.Generator().manual_seed(M + N + K + F)
     fi = torch.randperm(K + F, generator=g)[:F]
     s_w = (torch.rand(N, 1, generator=g) * 0.009 + 0.001).to(dtype)
-    W = (torch.randint(-8, 8, (N, K + F), generator=g).float() * s_w.float()).to(dtype)
+    W = (torch.randint(-8, 8, (N, K + F), generator=g).float() * (1 if bits == 4 else 15) * s_w.float()).to(dtype)
     lin = torch.nn.Linear(K + F, N, bias=True, dtype=dtype)
-    mod = MixedQLinear.from_float(lin, W, s_w, None, fi, bits=4).to(DEV)
+    mod = MixedQLinear.from_float(lin, W, s_w, None, fi, bits=bits).to(DEV)
     x = torch.randn(M, K + F, generator=g)
     x[:, fi] *= 50
     x = x.to(dtype).to(DEV)
