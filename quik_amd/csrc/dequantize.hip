@@ -214,7 +214,7 @@ extern "C" int quik_asym_fused_dequantize(const void *A, const void *B, const vo
   const int rc = int_gemm_chain(A, B, scale_row, scale_col, zero_row, w_reduced, __builtin_bit_cast(uint16_t, shift), y,
                                 M, N, K, bits, out, as_stream(stream));
   if (rc != kChainNotHandled) return rc;
-  // at most 32 rows: product by the weight-streaming kernel into the workspace, epilogue as a second launch
+  // (of the calls of at most 32 rows) product by the weight-streaming kernel into the workspace, epilogue as a second launch
   if (!acc_workspace) return QUIK_ERR_NULL;
   if (int rc2 = int_matmul(A, B, acc_workspace, M, N, K, bits, stream)) return rc2;
   hipLaunchKernelGGL(asym_fused_chain_kernel, dim3(grid_for(M * N)), dim3(kThreads), 0, as_stream(stream),
@@ -239,7 +239,7 @@ extern "C" int quik_sym_fused_dequantize(const void *A, const void *B, const voi
   return quik_sym_dequantize(acc_workspace, 32, scale_row, scale_col, y, M, N, out, stream);
 }
 
-/* bytes of the int32 workspace the fused dequantize entry points need for this shape (0: none, one launch) */
+/* bytes of the int32 workspace the fused dequantize entry points may need for this shape (0: none, one launch) */
 extern "C" int64_t quik_fused_dequantize_workspace_bytes(int64_t M, int64_t N) {
   return (M > 0 && M <= 32 && N > 0) ? M * N * 4 : 0;
 }

@@ -516,7 +516,7 @@ PyObject *py_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
 }
 
 // fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits) -> out or None; zero_row and
-// w_reduced None: the symmetric form.  Calls of at most 32 rows need a workspace and stay with the Python function.
+// w_reduced None: the symmetric form.  Calls that need a workspace (some of at most 32 rows) stay with the Python function.
 PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 9) Py_RETURN_NONE;
   const c10::DeviceIndex dev = current_gpu();
@@ -536,8 +536,7 @@ PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
     Py_RETURN_NONE;
   const int64_t M = A->size(0), N = B->size(0), K = A->size(1) * (bits == 4 ? 2 : 1);
   auto half = [](const at::Tensor *t, int64_t count) { return t->scalar_type() == at::kHalf && t->numel() == count; };
-  if (M * N == 0 || K == 0 || !half(sr, M) || !half(sc, N) || !half(y, M * N) || (!sym && (!half(zr, M) || !half(wr, N))) ||
-      quik_fused_dequantize_workspace_bytes(M, N) != 0)
+  if (M * N == 0 || K == 0 || !half(sr, M) || !half(sc, N) || !half(y, M * N) || (!sym && (!half(zr, M) || !half(wr, N))))
     Py_RETURN_NONE;
   return guarded([&]() -> PyObject * {
     at::Tensor out = new_empty({M, N}, at::kHalf, dev);
@@ -546,6 +545,7 @@ PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
                        : quik_asym_fused_dequantize(ptr(*A), ptr(*B), ptr(*sr), ptr(*sc), static_cast<float>(shift), ptr(*zr),
                                                     ptr(*wr), ptr(*y), M, N, K, static_cast<int>(bits), nullptr, out_ptr(out),
                                                     stream_of(dev));
+    if (rc == QUIK_ERR_NULL) Py_RETURN_NONE;  // (no workspace was passed)
     if (rc != QUIK_OK) return fail(bits == 4 ? "int4FusedDequantize" : "int8FusedDequantize", rc);
     return THPVariable_Wrap(std::move(out));
   });

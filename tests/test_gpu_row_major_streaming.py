@@ -22,6 +22,7 @@ CASES = [  # M, N, bytes of K per row, bits (0: both)
     (33, 7, 16, 0), (64, 65, 112, 0), (70, 130, 144, 0), (40, 64, 32 * 9, 0), (129, 100, 416, 0), (100, 72, 5 * 128 + 80, 0),
     (130, 64 * 129, 1040, 0), (300, 64 * 61 + 3, 560, 0),      # the same on 128x64 tiles
     (200, 64 * 230, 240, 0), (600, 6700, 688, 0), (1100, 9000, 208, 0),  # and on several rounds, and on the plain kernels
+    (1, 64, 64, 0), (1, 1001, 4096, 0), (32, 64 * 257, 176, 0), (17, 8, 1040, 0),  # decode sizes, the fused forms in one launch
     (130, 64 * 128, 1024, 4), (257, 64 * 85, 1088, 4), (130, 64 * 128, 3072, 8),  # 128x64 tiles, whole stages
 ]
 
