@@ -222,6 +222,15 @@ struct Tile8Pipe {
     }
   }
 
+  // All steps of a wave whose rows or columns lie past the matrix: its copies, waits and barriers, no products.
+  __device__ __forceinline__ void run_idle() {
+    for (int j = 0; j < steps; ++j) {
+      issue();
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+      __builtin_amdgcn_s_barrier();
+    }
+  }
+
   __device__ __forceinline__ void drain() const {
     __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
     __syncthreads();
@@ -285,6 +294,11 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
   if constexpr (!SPLITK) {
     pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64);
     pipe.start();
+    if (wave_is_idle<C>(p, m0, n0)) {  // (nothing behind the drain meets another wave)
+      pipe.run_idle();
+      pipe.drain();
+      return;
+    }
     pipe.read_all(f0);
     pipe.template run<kInt8, true>(0, pipe.steps0, f0, f1, acc);
   } else {

@@ -22,6 +22,14 @@ def test_one_wide_tile_per_cu(M, N, K, F, bits):
     _same_bits(M, N, K, F, torch.float16, bits)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K,F", [(1025, 8200, 256, 32), (1100, 8300, 640, 0), (1217, 8321, 768, 96), (1280, 8448, 128, 0),
+                                     (257, 4545, 384, 64), (2049, 4097, 256, 0)])
+def test_waves_past_the_last_row_and_column(M, N, K, F, bits):
+    """1, 76, 193 or all rows and 1, 8, 108, 129 or all columns in the last tiles: whole waves without a result."""
+    _same_bits(M, N, K, F, torch.bfloat16, bits)
+
+
 def _same_bits(M, N, K, F, dtype, bits):
     from quik_amd.qlinear import MixedQLinear
     g = torch.Generator().manual_seed(M + N + K + F)
