@@ -1190,9 +1190,11 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
 // the form before: its two passes over up to five fragments per lane stood behind the transfer, and 64 rows occupied 64 of
 // 1024 SIMDs.  Here a pass takes as long as one fragment, for four barriers (image landed, outlier values read, holes
 // patched, range exchanged).  us per launch in a graph, wave per row -> this, 256 outlier columns, fp16: 16 x 4096 4.0 ->
-// 3.5, 64 x 8192 5.3 -> 3.7, 128 x 5120 4.7 -> 3.5, 777 x 4096 5.6 -> 4.8, 1024 x 8192 9.7 -> 8.1, 2048 x 8192 12.4 -> 12.5,
-// 8192 x 8192 49.0 -> 45.4, 64 x 28672 12.8 -> 5.8, 2048 x 28672 61.9 -> 40.7; slower only about 2000 rows of 4096 or 5120
-// columns, 7.9 -> 8.4 and 9.4 -> 10.1.  bf16: 64 x 8192 7.5 -> 4.2, 777 x 4096 7.6 -> 5.9, 2048 x 28672 94 -> 47.
+// 3.4, 64 x 8192 5.3 -> 3.6, 128 x 5120 4.7 -> 3.5, 777 x 4096 5.6 -> 4.6, 1024 x 8192 9.7 -> 8.1, 2048 x 8192 12.4 -> 12.1,
+// 8192 x 8192 49.0 -> 44.4, 64 x 28672 12.8 -> 5.5, 2048 x 28672 61.9 -> 40.4; slower only about 2000 rows of 4096 or 5120
+// columns, 7.9 -> 8.4 and 9.4 -> 10.1.  bf16: 64 x 8192 7.5 -> 4.1, 777 x 4096 7.6 -> 5.7, 2048 x 28672 94 -> 46.
+// (Fillers read beside the outlier values and the ranges of all waves in one LDS round trip, not one after the other:
+// 64 x 8192 3.68 -> 3.57, 2048 x 8192 12.3 -> 12.1, 64 x 28672 5.71 -> 5.48.)
 template <bool BF16, bool SYM, int JT>
 __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     const uint16_t *__restrict__ x, int64_t rows, int cols, const uint32_t *__restrict__ patch,
@@ -1200,7 +1202,7 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     uint16_t *__restrict__ meta, float sym_divisor, int64_t first, int64_t count) {
   static_assert(!(BF16 && SYM), "symmetric activations are fp16");
   extern __shared__ __align__(16) uint8_t img[];
-  __shared__ float red[16];
+  __shared__ __align__(16) float red[16];  // minimum and maximum of up to eight waves
   __shared__ uint32_t total_s;
   if constexpr (!BF16 && !SYM) treat_all_nans_alike();  // the range uses pk_min_f16 / pk_max_f16 on the raw row
   // (nholes: the column map's count of holes, which the host knows: the entry points look the map's flag words up
@@ -1233,6 +1235,7 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
   for (int k = 0; k < PREG; ++k) pe[k] = patch[tid + k * T < nholes ? tid + k * T : 0];
   const uint4 oc = *reinterpret_cast<const uint4 *>(fp_col + (tid < nchunk ? tid : 0) * 8);
   if (tid == 0) total_s = 0;
+  if (tid < 8 && tid >= W) red[tid] = __builtin_inff(), red[8 + tid] = -__builtin_inff();
   const Fp6Layout l6 = fp6_layout(rows, num_int, num_fp);
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   __syncthreads();
@@ -1246,17 +1249,20 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     for (int k = 0; k < 4; ++k) o[k] = ld16(ow[k] & 0xFFFFu) | (ld16(ow[k] >> 16) << 16);
     *reinterpret_cast<uint4 *>(dst + fp6_outlier_offset(l6, row, c >> 1, c & 1)) = make_uint4(o[0], o[1], o[2], o[3]);
   };
+  uint32_t filler[PREG];  // read together with the outlier values: integer columns, none of them is a hole
+#pragma unroll
+  for (int k = 0; k < PREG; ++k) filler[k] = ld16(tid + k * T < nholes ? pe[k] >> 16 : 0);
   if (tid < nchunk) outliers(tid, oc);
   for (int c = tid + T; c < nchunk; c += T) outliers(c, *reinterpret_cast<const uint4 *>(fp_col + c * 8));
   __syncthreads();
-  // holes <- fillers (integer columns: none of them is a hole)
-  auto fill = [&](uint32_t e) {
-    *reinterpret_cast<uint16_t *>(img + img_of_col(e & 0xFFFFu)) = static_cast<uint16_t>(ld16(e >> 16));
+  // holes <- fillers
+  auto fill = [&](uint32_t e, uint32_t value) {
+    *reinterpret_cast<uint16_t *>(img + img_of_col(e & 0xFFFFu)) = static_cast<uint16_t>(value);
   };
 #pragma unroll
   for (int k = 0; k < PREG; ++k)
-    if (tid + k * T < nholes) fill(pe[k]);
-  for (int e = tid + PREG * T; e < nholes; e += T) fill(patch[e]);
+    if (tid + k * T < nholes) fill(pe[k], filler[k]);
+  for (int e = tid + PREG * T; e < nholes; e += T) fill(patch[e], ld16(patch[e] >> 16));
   __syncthreads();
 
   FragmentRange<BF16, SYM> range;
@@ -1274,9 +1280,17 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     red[8 + wave] = mx;
   }
   __syncthreads();
-  for (int w = 0; w < W; ++w) {
-    mn = fminf(mn, red[w]);
-    mx = fmaxf(mx, red[8 + w]);
+  // all eight slots in one round trip to the LDS (those of waves that are not there are neutral)
+  float part[16];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    const float4 r = *reinterpret_cast<const float4 *>(red + 4 * k);
+    part[4 * k] = r.x, part[4 * k + 1] = r.y, part[4 * k + 2] = r.z, part[4 * k + 3] = r.w;
+  }
+#pragma unroll
+  for (int w = 0; w < 8; ++w) {
+    mn = fminf(mn, part[w]);
+    mx = fmaxf(mx, part[8 + w]);
   }
   const RowQuant<BF16> rq = row_quant4<BF16, SYM>(mn, mx, sym_divisor, tid == 0, meta, row);
   const Fp6RowOut out(dst, l6, row);
