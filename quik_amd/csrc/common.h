@@ -194,6 +194,15 @@ __device__ __forceinline__ void dma_load16(const uint8_t *sbase, uint32_t voff, 
   asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2" : : "s"(lds_addr), "v"(voff), "s"(sbase) : "memory", "m0");
 }
 
+// The same with 2 and 4 bytes per lane, any 2- and 4-byte aligned addresses: lane i's value lands in the four bytes at LDS
+// address m0 + 4 i (2 bytes: in the low half; the high half is not to be read).
+__device__ __forceinline__ void dma_load_u16(const void *sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_ushort %1, %2" : : "s"(lds_addr), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+__device__ __forceinline__ void dma_load_u32(const void *sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_nop 0\n\tglobal_load_lds_dword %1, %2" : : "s"(lds_addr), "v"(voff), "s"(sbase) : "memory", "m0");
+}
+
 __device__ __forceinline__ uint32_t lds_address(const void *p) {
   return static_cast<uint32_t>(reinterpret_cast<uintptr_t>((const __attribute__((address_space(3))) void *)p));
 }

@@ -191,11 +191,16 @@ struct Fp6Pipe {
 
   // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. NS - 2 are in flight; the copies of step
   // NS - 1 are made during the MFMAs of step 0.
-  __device__ __forceinline__ void start() {
+  // landed(): what this wave does in front of the barrier, behind the arrival of what it requested before the ring.
+  template <class Landed>
+  __device__ __forceinline__ void start(Landed landed) {
     static_for<NS - 1>([&](auto) { issue(); });
     __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+    asm volatile("" ::: "memory");  // (empty: LDS reads of what has landed stay behind the wait)
+    landed();
     __syncthreads();
   }
+  __device__ __forceinline__ void start() { start([] {}); }
 
   __device__ __forceinline__ void next_read_slot() {
     rd += STAGE;
@@ -425,6 +430,43 @@ struct TileVectors6 {
   }
 };
 
+// The scales, zero points, reduced weights and bias of a tile, requested in front of the ring's copies (a thread per row and
+// column, 16 bits each into the low half of its slot) and widened in place, by the same thread, when they have landed.  Read
+// into registers and written to the LDS they cost two trips to memory, one for the columns and one for the rows, before
+// the first copy left: 128 x 5120 -> 13824 19.1 -> 18.3 us per forward, 300 x 4544 -> 4544 18.1 -> 17.4, 512 x 4096 -> 4096
+// 18.2 -> 17.7, bf16 777 x 4096 -> 22016 70.1 -> 68.8, 2048 x 8192 -> 28672 269.4 -> 265.4; 2048 x 8192 -> 1024 30.35 ->
+// 30.12, int8 365 x 28672 -> 8192 144.9 -> 144.6.
+template <class C, class Vectors, class Args>
+__device__ __forceinline__ void tile_vector_request(const Vectors &tv, const Args &p, int m0, int n0, int wave) {
+  const int i = threadIdx.x;
+  if (wave * 64 < C::BN) {
+    const uint32_t off = static_cast<uint32_t>(n0 + i < p.N ? n0 + i : p.N - 1) * 2, at = wave * 256;
+    dma_load_u16(p.s_col, off, lds_address(tv.scol) + at);
+    if (p.w_red) dma_load_u16(p.w_red, off, lds_address(tv.wred) + at);
+    if (p.bias) dma_load_u16(p.bias, off, lds_address(tv.bias) + at);
+  }
+  if (wave * 64 < C::BM) {
+    const uint32_t m = static_cast<uint32_t>(m0 + i < p.M ? m0 + i : p.M - 1), at = wave * 256;
+    dma_load_u16(p.meta, p.w_red ? 4 * m : 2 * m, lds_address(tv.srow) + at);
+    if (p.w_red) dma_load_u16(p.meta, 4 * m + 2, lds_address(tv.zs) + at);
+  }
+}
+template <class C, bool BF16, class Vectors>
+__device__ __forceinline__ void tile_vector_widen(const Vectors &tv, bool bias, bool asym, float shift) {
+  const int i = threadIdx.x;
+  auto wide = [&](const float *v) { return to_f32<BF16>(static_cast<uint16_t>(__float_as_uint(v[i]))); };
+  if (i < C::BN) {
+    tv.scol[i] = wide(tv.scol);
+    tv.wred[i] = asym ? wide(tv.wred) : 0.0f;
+    tv.bias[i] = bias ? wide(tv.bias) : 0.0f;
+  }
+  if (i < C::BM) {
+    const float s = wide(tv.srow);
+    tv.srow[i] = s;
+    tv.zs[i] = asym ? wide(tv.zs) + shift * s : 0.0f;
+  }
+}
+
 template <class C>
 constexpr int fused6_smem() {
   return Fp6Pipe<C>::SMEM + TileVectors6<C>::kBytes;
@@ -553,25 +595,25 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   const Fp6Layout lx = fp6_layout(p.M, p.K, p.F), lw = fp6_layout(p.N_total, p.K, p.F);
   const TileVectors6<C> tv(smem + Pipe::SMEM);
-  {
-    const int32_t *xs = reinterpret_cast<const int32_t *>(p.xbuf + lx.sums_off);
-    const int32_t *ws = reinterpret_cast<const int32_t *>(p.wbuf + lw.sums_off);
-    for (int i = threadIdx.x; i < C::BN; i += C::kThreads) {
-      const int n = n0 + i < p.N ? n0 + i : p.N - 1;
-      tv.scol[i] = to_f32<BF16>(p.s_col[n]);
-      tv.wred[i] = p.w_red ? to_f32<BF16>(p.w_red[n]) : 0.0f;
-      tv.bias[i] = p.bias ? to_f32<BF16>(p.bias[n]) : 0.0f;
-      tv.colc[i] = static_cast<float>(ws[p.n_first + n]) * -0.125f;
-    }
-    for (int i = threadIdx.x; i < C::BM; i += C::kThreads) {
-      const int64_t m = m0 + i < p.M ? m0 + i : p.M - 1;
-      // asymmetric: meta holds (scale, zero) pairs; symmetric (no w_red): one scale per row and no zero term
-      const float s = to_f32<BF16>(p.meta[p.w_red ? 2 * m : m]);
-      tv.srow[i] = s;
-      tv.zs[i] = p.w_red ? to_f32<BF16>(p.meta[2 * m + 1]) + 8.0f * s : 0.0f;
-      tv.rowc[i] = static_cast<float>(8 * xs[m] - 64 * p.K);
-    }
-  }  // made visible by the first barrier of the pipeline
+  // thread i requests column i and row i of the vectors, raw, and widens them in place when they have landed
+  static_assert(C::BM <= C::kThreads && C::BN <= C::kThreads && C::BM % 64 == 0 && C::BN % 64 == 0, "a thread per row and column");
+  const int swave = __builtin_amdgcn_readfirstlane(wave);
+  const bool asym = p.w_red != nullptr;  // asymmetric: meta holds (scale, zero) pairs; symmetric: one scale per row, no zero term
+  tile_vector_request<C>(tv, p, m0, n0, swave);
+  if (swave * 64 < C::BN) {
+    const int i = threadIdx.x, n = n0 + i < p.N ? n0 + i : p.N - 1;
+    dma_load_u32(p.wbuf + lw.sums_off + static_cast<int64_t>(p.n_first) * 4, static_cast<uint32_t>(n) * 4, lds_address(tv.colc) + swave * 256);
+  }
+  if (swave * 64 < C::BM) {
+    const int i = threadIdx.x, m = m0 + i < p.M ? m0 + i : p.M - 1;
+    dma_load_u32(p.xbuf + lx.sums_off, static_cast<uint32_t>(m) * 4, lds_address(tv.rowc) + swave * 256);
+  }
+  auto widen = [&] {
+    const int i = threadIdx.x;
+    tile_vector_widen<C, BF16>(tv, p.bias != nullptr, asym, 8.0f);
+    if (i < C::BN) tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
+    if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * __float_as_int(tv.rowc[i]) - 64 * p.K);
+  };
 
   Pipe pipe;
   const int total = static_cast<int>(lx.steps);
@@ -583,7 +625,7 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
   } else {
     pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64);
   }
-  pipe.start();  // its barrier also makes the vectors visible
+  pipe.start(widen);  // its barrier also makes the vectors visible
   if constexpr (!SPLITK) {
     // (nothing behind the drain meets another wave)
     if (wave_is_idle<C>(p, m0, n0)) {

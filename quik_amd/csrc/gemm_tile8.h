@@ -131,11 +131,16 @@ struct Tile8Pipe {
   }
 
   // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. NS - 2 are in flight.
-  __device__ __forceinline__ void start() {
+  // landed(): what this wave does in front of the barrier, behind the arrival of everything it requested before the ring.
+  template <class Landed>
+  __device__ __forceinline__ void start(Landed landed) {
     static_for<NS - 1>([&](auto) { issue(); });
     __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+    asm volatile("" ::: "memory");  // (empty: LDS reads of what has landed stay behind the wait)
+    landed();
     __syncthreads();
   }
+  __device__ __forceinline__ void start() { start([] {}); }
 
   __device__ __forceinline__ void next_read_slot() {
     rd += STAGE;
@@ -267,19 +272,10 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
   const Tile8Layout lx = tile8_layout(p.M, p.K, p.F), lw = tile8_layout(p.N_total, p.K, p.F);
   const TileVectors<C> tv(smem + tile8_vectors_offset<C>());
-  for (int i = threadIdx.x; i < C::BN; i += C::kThreads) {
-    const int n = n0 + i < p.N ? n0 + i : p.N - 1;
-    tv.scol[i] = to_f32<BF16>(p.s_col[n]);
-    tv.wred[i] = p.w_red ? to_f32<BF16>(p.w_red[n]) : 0.0f;
-    tv.bias[i] = p.bias ? to_f32<BF16>(p.bias[n]) : 0.0f;
-  }
-  for (int i = threadIdx.x; i < C::BM; i += C::kThreads) {
-    const int64_t m = m0 + i < p.M ? m0 + i : p.M - 1;
-    // asymmetric: meta holds (scale, zero) pairs; symmetric (no w_red): one scale per row and no zero term
-    const float s = to_f32<BF16>(p.meta[p.w_red ? 2 * m : m]);
-    tv.srow[i] = s;
-    tv.zs[i] = p.w_red ? to_f32<BF16>(p.meta[2 * m + 1]) + 128.0f * s : 0.0f;
-  }  // made visible by the first barrier of the pipeline
+  static_assert(C::BM <= C::kThreads && C::BN <= C::kThreads && C::BM % 64 == 0 && C::BN % 64 == 0, "a thread per row and column");
+  tile_vector_request<C>(tv, p, m0, n0, __builtin_amdgcn_readfirstlane(wave));
+  // (asymmetric: meta holds (scale, zero) pairs; symmetric, no w_red: one scale per row and no zero term)
+  auto widen = [&] { tile_vector_widen<C, BF16>(tv, p.bias != nullptr, p.w_red != nullptr, 128.0f); };
 
   v16f acc[C::MI][C::NI];  // integer bit patterns during the first phase, floats afterwards
 #pragma unroll
@@ -293,7 +289,7 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
   v4i f0[Pipe::NF], f1[Pipe::NF];
   if constexpr (!SPLITK) {
     pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64);
-    pipe.start();
+    pipe.start(widen);  // its barrier also makes the vectors visible
     if (wave_is_idle<C>(p, m0, n0)) {  // (nothing behind the drain meets another wave)
       pipe.run_idle();
       pipe.drain();
@@ -305,7 +301,7 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
     const int total = static_cast<int>(lx.steps), k0 = split * sk->per;
     const int k1 = k0 + sk->per < total ? k0 + sk->per : total;
     pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64, k0, k1 - k0, 0);
-    pipe.start();
+    pipe.start(widen);
     pipe.read_all(f0);
     pipe.template run<kInt8, true>(0, pipe.steps0, f0, f1, acc);
     pipe.drain();  // the copies past the last step have landed too: the ring is free
