@@ -324,8 +324,8 @@ int launch_chain_rows(const I32Args &a, const ChainArgs &e, hipStream_t st) {
   int tiles_m, tiles_n;
   const int grid = grid_of<R>(a.M, a.N, tiles_m, tiles_n);
   auto kern = gemm_chain_rows_kernel<R, MODE, ASYM>;
-  if (int rc = prepare(kern, R::SMEM)) return rc;
-  hipLaunchKernelGGL(kern, dim3(grid), dim3(R::kThreads), R::SMEM, st, a, e, tiles_m, tiles_n);
+  if (int rc = prepare(kern, chain_rows_smem<R>())) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid), dim3(R::kThreads), chain_rows_smem<R>(), st, a, e, tiles_m, tiles_n);
   return check_launch();
 }
 
@@ -403,7 +403,7 @@ int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
   // Up to 32 rows: one launch on one round of row-streaming tiles, where the product by itself would go to the
   // weight-streaming kernel and the epilogue to a second launch: the intermediate and that launch cost a caller more than the
   // tiles lose on few columns.  us per call: 5 x 8192 -> 1024 15.6 -> 9.8, 21 x 1280 -> 544 15.6 -> 5.6, 32 x 4096 -> 11008 15.7
-  // -> 8.4, 24 x 8192 -> 8192 15.5 -> 10.8, int8 32 x 8192 -> 16000 46.9 -> 30.3 (kernels alone, int4: 9.0 / 9.5, 6.4 / 5.3, 13.1 / 8.5,
+  // -> 7.8, 24 x 8192 -> 8192 15.5 -> 10.8, int8 32 x 8192 -> 16000 46.9 -> 30.3 (kernels alone, int4: 9.0 / 9.5, 6.4 / 5.3, 13.1 / 8.5,
   // 13.5 / 11.0).  Rows of more than 11 KB leave a tile's waves too long a chain (int8 16 x 13824 -> 5120 24.8 / 27.1, 16 x
   // 28672 -> 8192 55 / 62).  Up to four tiles are too few for long rows (16 x 8192 -> 256 8.8 / 9.3, 1 x 8192 -> 256 7.8 / 9.3)
   // and keep the two launches.

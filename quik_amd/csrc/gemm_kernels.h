@@ -663,9 +663,20 @@ struct ChainArgs {
   uint16_t shift;   // fp16 bit pattern of the shift value (asymmetric)
 };
 
-template <class C, int MODE, bool ASYM>
+// Where chain_store finds its inputs: in global memory.  (row, col: of the matrix, inside it)
+struct ChainGlobal {
+  const ChainArgs &e;
+  __device__ __forceinline__ uint16_t s_row(int row) const { return e.s_row[row]; }
+  __device__ __forceinline__ uint16_t zero_row(int row) const { return e.zero_row[row]; }
+  __device__ __forceinline__ uint16_t s_col(int col) const { return e.s_col[col]; }
+  __device__ __forceinline__ uint16_t w_red(int col) const { return e.w_red[col]; }
+  __device__ __forceinline__ bool has_y() const { return false; }  // y goes through the staging area
+  __device__ __forceinline__ void y(int, int, uint16_t (&)[4]) const {}
+};
+
+template <class C, int MODE, bool ASYM, class In = ChainGlobal>
 __device__ __forceinline__ void chain_store(const I32Args &a, const ChainArgs &e, int m0, int n0, uint8_t *smem,
-                                            const v16i (&acc)[C::MI][C::NI]) {
+                                            const v16i (&acc)[C::MI][C::NI], const In &in) {
   const int M = a.M, N = a.N;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
@@ -683,29 +694,32 @@ __device__ __forceinline__ void chain_store(const I32Args &a, const ChainArgs &e
     const int mb = m0 + wm * C::WM + mi * 32;
     if (!(mb < M && nw < N)) continue;  // wave-uniform
     // y of this 32-row block through the staging area: global -> LDS as row segments, LDS -> this lane's places
-    Store::load(stage, lane, e.y + int64_t(mb) * e.ldy + nw, e.ldy, M - mb, N - nw, vec);
+    const bool has_y = in.has_y();
+    if (!has_y) Store::load(stage, lane, e.y + int64_t(mb) * e.ldy + nw, e.ldy, M - mb, N - nw, vec);
+    __builtin_amdgcn_wave_barrier();
     const int r = mb + (lane & 31) < M ? mb + (lane & 31) : M - 1;
-    const _Float16 sr = h(e.s_row[r]);
+    const _Float16 sr = h(in.s_row(r));
     _Float16 u0 = static_cast<_Float16>(0);
-    if constexpr (ASYM) u0 = h(e.zero_row[r]) + shift * sr;  // (zero_row + h(shift) * s_row), two roundings
+    if constexpr (ASYM) u0 = h(in.zero_row(r)) + shift * sr;  // (zero_row + h(shift) * s_row), two roundings
 #pragma unroll
     for (int ni = 0; ni < C::NI; ++ni)
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
         const int c0 = nw + ni * 32 + acc_col(g, lane);
         uint16_t yv[4], o[4];
-        Store::get(stage, lane, ni, g, yv);
+        if (has_y) in.y(r, c0, yv);
+        else Store::get(stage, lane, ni, g, yv);
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
           const int c = c0 + k < N ? c0 + k : N - 1;
           _Float16 t = static_cast<_Float16>(static_cast<float>(acc[mi][ni][4 * g + k] >> kShift));
           if constexpr (ASYM) {
-            t = t * h(e.s_col[c]);
+            t = t * h(in.s_col(c));
             t = t * sr;
-            t = t + u0 * h(e.w_red[c]);
+            t = t + u0 * h(in.w_red(c));
           } else {
             t = t * sr;
-            t = t * h(e.s_col[c]);
+            t = t * h(in.s_col(c));
           }
           t = t + h(yv[k]);
           o[k] = __builtin_bit_cast(uint16_t, t);
@@ -728,7 +742,7 @@ __device__ __forceinline__ void chain_tile(const I32Args &a, const ChainArgs &e,
       for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0;
   run_mainloop<C, MODE>(a.X + int64_t(m0) * a.kbytes, a.kbytes, a.M - m0, a.W + int64_t(n0) * a.kbytes, a.kbytes, a.N - n0,
                         a.kbytes, smem, acc);
-  chain_store<C, MODE, ASYM>(a, e, m0, n0, smem, acc);
+  chain_store<C, MODE, ASYM>(a, e, m0, n0, smem, acc, ChainGlobal{e});
 }
 
 template <class C, int MODE, bool ASYM>

@@ -231,15 +231,76 @@ __global__ __launch_bounds__(R::kThreads) void gemm_i32_rows_kernel(I32Args a, i
   i32_store<typename R::Tile, MODE>(a, m0, n0, smem + R::RED_BYTES, own);
 }
 
+// The inputs of chain_store for a tile, copied to the LDS behind the rings in front of the main loop: scales, zero points and
+// reduced weights as 16 bits in slots of four bytes, y as rows of 128 bytes whose 16-byte pieces are swapped as in the rings.
+// (y only where its pieces are aligned and whole: has.)  Read at the end instead, they were a chain of trips to memory
+// behind the products: us per call 256 x 4096 x 4096 int4 8.86 -> 8.24, 512 x 4096 x 4096 15.3 -> 13.7, 32 x 4096 x 11008 8.43 ->
+// 7.75, int8 64 x 8192 x 1024 14.15 -> 13.53; with y unaligned (130 x 4096 x 4100) 10.78 -> 10.76.
+template <class R>
+struct ChainStaged {
+  static constexpr int kBytes = (2 * R::BN + 2 * R::BM) * 4 + R::BM * R::BN * 2;
+  uint8_t *base;
+  int m0, n0;
+  bool has;
+  __device__ __forceinline__ uint16_t u16(int slot) const {
+    return static_cast<uint16_t>(*reinterpret_cast<const uint32_t *>(base + slot * 4));
+  }
+  __device__ __forceinline__ uint16_t s_col(int col) const { return u16(col - n0); }
+  __device__ __forceinline__ uint16_t w_red(int col) const { return u16(R::BN + col - n0); }
+  __device__ __forceinline__ uint16_t s_row(int row) const { return u16(2 * R::BN + row - m0); }
+  __device__ __forceinline__ uint16_t zero_row(int row) const { return u16(2 * R::BN + R::BM + row - m0); }
+  __device__ __forceinline__ bool has_y() const { return has; }
+  __device__ __forceinline__ uint8_t *y_rows() const { return base + (2 * R::BN + 2 * R::BM) * 4; }
+  __device__ __forceinline__ void y(int row, int col, uint16_t (&v)[4]) const {
+    const int r = row - m0, c = col - n0;
+    const uint2 w = *reinterpret_cast<const uint2 *>(y_rows() + r * 128 + (((c >> 3) ^ (r & 7)) << 4) + (c & 4) * 2);
+    v[0] = static_cast<uint16_t>(w.x), v[1] = static_cast<uint16_t>(w.x >> 16);
+    v[2] = static_cast<uint16_t>(w.y), v[3] = static_cast<uint16_t>(w.y >> 16);
+  }
+  // (visible to the other waves behind the barriers of the main loop's exchange; every wave waits for its own copies there)
+  template <bool ASYM>
+  __device__ __forceinline__ void request(const ChainArgs &e, int M, int N) const {
+    static_assert(R::BN == 64 && R::BM <= 64 * R::WAVES, "a wave per vector piece");
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t lds = __builtin_amdgcn_readfirstlane(lds_address(base));
+    if (wave == R::WAVES - 1) {
+      const uint32_t n = n0 + lane < N ? n0 + lane : N - 1;
+      dma_load_u16(e.s_col, 2 * n, lds);
+      if constexpr (ASYM) dma_load_u16(e.w_red, 2 * n, lds + R::BN * 4);
+    }
+    if (wave * 64 < R::BM) {
+      const uint32_t i = wave * 64 + lane, m = m0 + static_cast<int>(i) < M ? m0 + i : M - 1;
+      dma_load_u16(e.s_row, 2 * m, lds + (2 * R::BN + wave * 64) * 4);
+      if constexpr (ASYM) dma_load_u16(e.zero_row, 2 * m, lds + (2 * R::BN + R::BM + wave * 64) * 4);
+    }
+    if (has) {
+      const uint8_t *y0 = reinterpret_cast<const uint8_t *>(e.y + int64_t(m0) * e.ldy + n0);
+#pragma unroll
+      for (int j = 0; j < R::BM / 8 / R::WAVES; ++j) {
+        const int at = (j * R::WAVES + wave) * 8, row = at + (lane >> 3);
+        dma_load16(y0, static_cast<uint32_t>(m0 + row < M ? row : M - 1 - m0) * static_cast<uint32_t>(e.ldy) * 2u + (((lane & 7) ^ (lane >> 3)) << 4),
+                   lds + (2 * R::BN + 2 * R::BM) * 4 + at * 128);
+      }
+    }
+  }
+};
+template <class R>
+constexpr int chain_rows_smem() {
+  return R::SMEM + ChainStaged<R>::kBytes;
+}
+
 template <class R, int MODE, bool ASYM>
 __global__ __launch_bounds__(R::kThreads) void gemm_chain_rows_kernel(I32Args a, ChainArgs e, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_of_block<R::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   const int m0 = tm * R::BM, n0 = tn * R::BN;
+  const ChainStaged<R> in{smem + R::SMEM, m0, n0,
+                          n0 + R::BN <= a.N && (e.ldy & 7) == 0 && e.ldy < (1 << 23) && (reinterpret_cast<uintptr_t>(e.y) & 15) == 0};
+  in.template request<ASYM>(e, a.M, a.N);
   v16i own[R::OWN][1];
   rows_mainloop<R, MODE>(a.X + int64_t(m0) * a.kbytes, a.M - m0, a.W + int64_t(n0) * a.kbytes, a.N - n0, a.kbytes, smem, own);
-  chain_store<typename R::Tile, MODE, ASYM>(a, e, m0, n0, smem + R::RED_BYTES, own);
+  chain_store<typename R::Tile, MODE, ASYM>(a, e, m0, n0, smem + R::RED_BYTES, own, in);
 }
 
 }  // namespace quik

@@ -63,3 +63,18 @@ def test_products_and_fused_forms(M, N, kbytes, bits):
         got = got.cpu().numpy()
         assert np.array_equal(np.isnan(got), np.isnan(w))
         assert np.array_equal(got[~np.isnan(w)].view(np.uint16), w[~np.isnan(w)].view(np.uint16))
+
+
+@pytest.mark.parametrize("M,N,kbytes", [(64, 128, 256), (63, 136, 144), (1, 512, 64), (257, 64 * 85, 1088), (130, 64 * 128, 1024)])
+@pytest.mark.parametrize("off", [0, 1])
+def test_fused_form_with_y_in_the_lds_or_not(M, N, kbytes, off):
+    """Whole and partial column tiles of one call, y on a 16-byte boundary and two bytes behind one: the same bits as the
+    product and the stand-alone dequantize."""
+    import quik
+    g = torch.Generator(device=DEV).manual_seed(M + N + off)
+    a, b, _, _ = _operands(M, N, kbytes, 4, g)
+    s_row, s_col = ((torch.rand(*s, generator=g, device=DEV) * 0.1).half() for s in ((M, 1), (1, N)))
+    y = torch.randn(M * N + off, generator=g, device=DEV).half()[off:].view(M, N)
+    got = quik.symmetric.int4FusedDequantize(a, b, s_row, s_col, y)
+    want = quik.symmetric.dequantize(quik.matmul.int4Matmul(a, b), s_row, s_col, y.clone(), 32)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
