@@ -30,8 +30,6 @@ constexpr uint32_t kColmapStreams = 1u, kColmapInPlace = 2u;
 int colmap_flags(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, hipStream_t st, uint32_t *flags);
 // all four flag words of the map (flags, number of dirty groups, number of holes, reserved), same look-up
 int colmap_words(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, hipStream_t st, uint32_t (&out)[4]);
-// the same without a look at the device: false when the map is not known yet
-bool colmap_words_known(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, uint32_t (&out)[4]);
 void colmap_forget(const void *colmap);
 // QUIK_OK when the column map has all bits of `need` set, QUIK_ERR_COLMAP when not (or an error of colmap_flags)
 inline int colmap_require(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, hipStream_t st,

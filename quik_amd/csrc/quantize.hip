@@ -357,12 +357,56 @@ __device__ __forceinline__ void gather_rows(
 // lanes load their group (and every lane its outlier value) straight from the row, right after
 // the row's own loads, so the data arrives with them (same cache lines).  A last pass reads 16
 // code bytes per lane, packs them to nibbles (int4) and writes 8 or 16 contiguous bytes per lane.
-// One row is handled by the TPR threads of one workgroup (a multiple of 64, at most 256; the
-// launches use 256), which walks over rows blockIdx.x, blockIdx.x + gridDim.x, ...
+// One row is handled by the TPR threads of one workgroup (a multiple of 64; the launches use 256 and 512),
+// which walks over rows blockIdx.x, blockIdx.x + gridDim.x, ...
 // SYM: symmetric activations (scale = fp16(max |x| / sym_divisor), one scale per row in meta[row]); fp16 only.
+
+// A lane's row-invariant tables: its NV groups, its first ND dirty groups and outlier columns (so that the per-row loops
+// wait on no global load).  Every load is unconditional, from an address that always exists (lanes without an entry read
+// the first words of grp): behind a condition each load sits in a branch of its own with its own wait, and the kernel
+// starts with one round trip to the L2 after the other.  For the same reason `load` does not wait for the map's flag words:
+// it takes as many dirty entries as the map has room for, and `settle` drops those behind the map's own count.
+template <int NV, int TPR>
+struct StreamTables {
+  static constexpr int ND = TPR >= 256 ? 1 : 256 / TPR;
+  uint32_t g[NV], dirty[ND], dgrp[ND], fpcol[ND];
+  __device__ __forceinline__ void load(const uint32_t *grp, const uint32_t *dirty_map, const uint16_t *dirty_grp,
+                                       const uint16_t *fp_col, int64_t cols, int64_t num_fp) {
+    const int tid = threadIdx.x, nvec = static_cast<int>(cols >> 3), room = static_cast<int>(max_dirty_groups(cols, num_fp));
+    const uint16_t *spare16 = reinterpret_cast<const uint16_t *>(grp);
+#pragma unroll
+    for (int i = 0; i < NV; ++i) g[i] = grp[tid + i * TPR < nvec ? tid + i * TPR : 0];
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      const int j = tid + k * TPR;
+      dirty[k] = *(j < room ? dirty_map + j : grp);
+      dgrp[k] = *(j < room ? dirty_grp + j : spare16);
+      fpcol[k] = *(j < num_fp ? fp_col + j : spare16);
+    }
+  }
+  // the loads stay in front of whatever follows (the compiler would move them behind a branch that not all paths need
+  // them in, and the wait for the branch's condition in front of them)
+  __device__ __forceinline__ void pin() {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) asm volatile("" : "+v"(g[i]));
+#pragma unroll
+    for (int k = 0; k < ND; ++k) asm volatile("" : "+v"(dirty[k]), "+v"(dgrp[k]), "+v"(fpcol[k]));
+  }
+  __device__ __forceinline__ void settle(int nvec, int ndirty, int64_t num_fp) {
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) g[i] = tid + i * TPR < nvec ? g[i] : 0xFFFFFFFFu;
+#pragma unroll
+    for (int k = 0; k < ND; ++k) {
+      if (!(tid + k * TPR < ndirty)) dirty[k] = dgrp[k] = 0u;
+      if (!(tid + k * TPR < num_fp)) fpcol[k] = 0u;
+    }
+  }
+};
+
 template <int BITS, bool BF16, int NV, int TPR, bool SYM = false, bool PF = false>
 __device__ __forceinline__ void stream_rows(const uint16_t *__restrict__ x, int64_t rows, int64_t cols,
-                                            const uint32_t *__restrict__ grp, const uint32_t *__restrict__ dirty,
+                                            StreamTables<NV, TPR> &tables, const uint32_t *__restrict__ dirty,
                                             const uint16_t *__restrict__ dirty_grp, int ndirty,
                                             const uint16_t *__restrict__ fp_col, int64_t num_int, int64_t num_fp,
                                             uint8_t *__restrict__ dst, uint16_t *__restrict__ meta,
@@ -377,30 +421,10 @@ __device__ __forceinline__ void stream_rows(const uint16_t *__restrict__ x, int6
   const int tid = threadIdx.x;
   const int nvec = static_cast<int>(cols >> 3);
   const float inf = __builtin_inff();
-  // Row-invariant tables in registers.  Every load is unconditional, from an address that always exists (lanes
-  // without an entry read the first words of grp): behind a condition each load sits in a branch of its own with
-  // its own wait, and the kernel starts with one round trip to the L2 after the other.
-  uint32_t g[NV];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) g[i] = grp[tid + i * TPR < nvec ? tid + i * TPR : 0];
-#pragma unroll
-  for (int i = 0; i < NV; ++i) g[i] = tid + i * TPR < nvec ? g[i] : 0xFFFFFFFFu;
-  // this lane's first ND dirty groups and outliers, so that the per-row loops below wait on no global load
-  constexpr int ND = TPR >= 256 ? 1 : 256 / TPR;
-  uint32_t my_dirty[ND], my_dgrp[ND], my_fpcol[ND];
-  const uint16_t *spare16 = reinterpret_cast<const uint16_t *>(grp);
-#pragma unroll
-  for (int k = 0; k < ND; ++k) {
-    const bool has_d = tid + k * TPR < ndirty, has_f = tid + k * TPR < num_fp;
-    my_dirty[k] = *(has_d ? dirty + tid + k * TPR : grp);
-    my_dgrp[k] = *(has_d ? dirty_grp + tid + k * TPR : spare16);
-    my_fpcol[k] = *(has_f ? fp_col + tid + k * TPR : spare16);
-  }
-#pragma unroll
-  for (int k = 0; k < ND; ++k) {
-    if (!(tid + k * TPR < ndirty)) my_dirty[k] = my_dgrp[k] = 0u;
-    if (!(tid + k * TPR < num_fp)) my_fpcol[k] = 0u;
-  }
+  tables.settle(nvec, ndirty, num_fp);
+  constexpr int ND = StreamTables<NV, TPR>::ND;
+  const uint32_t(&g)[NV] = tables.g;
+  const uint32_t(&my_dirty)[ND] = tables.dirty, (&my_dgrp)[ND] = tables.dgrp, (&my_fpcol)[ND] = tables.fpcol;
 
   auto load_row = [&](int64_t row, uint4 (&v)[NV]) {
     const uint4 *xv = reinterpret_cast<const uint4 *>(x + row * cols);
@@ -692,18 +716,21 @@ __global__ __launch_bounds__(TPR) void asym_quantize_stream_kernel(
     const IdxT *__restrict__ fp_col, const uint32_t *__restrict__ mask, const uint32_t *__restrict__ grp,
     const uint32_t *__restrict__ dirty, const uint16_t *__restrict__ dirty_grp, const uint32_t *__restrict__ flags,
     int64_t num_int, int64_t num_fp, uint8_t *__restrict__ dst, uint16_t *__restrict__ meta,
-    uint16_t *__restrict__ fp_x, int vec_out, float sym_divisor, int known_ndirty) {
+    uint16_t *__restrict__ fp_x, int vec_out, float sym_divisor) {
   static_assert(sizeof(IdxT) == 2, "streaming needs cols <= 32768");
   extern __shared__ __align__(16) uint16_t row_s[];
   __shared__ float red[64];
-  // known_ndirty: the map streams and has that many dirty groups, says the host (-1: it does not know).  Its flag words
-  // are a round trip to memory in front of everything else otherwise.
-  if (known_ndirty >= 0 || (flags[0] & 1u)) {
+  // The flag words and the lane's tables in one round trip to memory: the map at this address may be another one at
+  // every launch (rebuilt, copied over, replayed in a graph), so the words are the device's, never the host's.
+  const uint32_t map_flags = flags[0], ndirty = flags[1];
+  StreamTables<NV, TPR> tables;
+  tables.load(grp, dirty, dirty_grp, reinterpret_cast<const uint16_t *>(fp_col), cols, num_fp);
+  tables.pin();
+  if (map_flags & kColmapStreams) {
     uint8_t *codes_s = reinterpret_cast<uint8_t *>(row_s);
-    stream_rows<BITS, BF16, NV, TPR, SYM, PF>(x, rows, cols, grp, dirty, dirty_grp,
-                                          known_ndirty >= 0 ? known_ndirty : static_cast<int>(flags[1]),
-                                          reinterpret_cast<const uint16_t *>(fp_col), num_int, num_fp, dst, meta, fp_x,
-                                          codes_s, red, vec_out, sym_divisor);
+    stream_rows<BITS, BF16, NV, TPR, SYM, PF>(x, rows, cols, tables, dirty, dirty_grp, static_cast<int>(ndirty),
+                                              reinterpret_cast<const uint16_t *>(fp_col), num_int, num_fp, dst, meta,
+                                              fp_x, codes_s, red, vec_out, sym_divisor);
   } else if constexpr (!SYM) {
     // Tile-ordered output exists on the streaming path only: a column map that does not stream (any other index
     // order) must not reach the row-major gather code with an operand buffer as `dst` and no `fp_x`.  Nothing is
@@ -1555,7 +1582,7 @@ int grid_for(int64_t work_items, int64_t per_block) {
 constexpr int64_t kMaxLdsRowBytes = 128 * 1024;  // of the 160 KB per CU
 
 // Few rows of more than 4096 columns: eight waves per row instead of four, while the rows leave half of the CUs without one
-// (us per launch: int8 16 x 13824 5.2 -> 4.8, 32 x 28672 7.6 -> 6.8, bf16 16 x 13824 5.7 -> 5.1, int4 32 x 8192 4.1 -> 3.8; 256 x 28672 bf16
+// (us per launch: int8 16 x 13824 5.2 -> 4.9, 32 x 28672 7.5 -> 6.9, bf16 16 x 13824 5.7 -> 5.2, int4 32 x 8192 4.1 -> 3.9; 256 x 28672 bf16
 // 11.8 -> 10.7, 512 x 11008 9.3 -> 8.8 but fp16 256 x 8192 4.3 -> 4.4; sixteen waves were slower than eight everywhere).
 int64_t wide_rows() { return num_cus() / 2; }
 
@@ -1574,9 +1601,6 @@ int launch_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, 
       return QUIK_ERR_LAUNCH;
     }
   }
-  uint32_t words[4];
-  const bool known = colmap_words_known(cm, cols, num_int, num_fp, words) && (words[0] & kColmapStreams);
-  const int known_ndirty = known ? static_cast<int>(words[1]) : -1;
   const int64_t items = tiled ? (rows + 7) / 8 * 8 : rows;
   int grid = static_cast<int>(items < (int64_t(1) << 30) ? items : (int64_t(1) << 30));
   if (PF && grid > 2 * num_cus()) grid = 2 * num_cus();  // persistent: the workgroups that are resident at once
@@ -1590,7 +1614,7 @@ int launch_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, 
                      reinterpret_cast<const uint16_t *>(cm + l.off_slot),
                      reinterpret_cast<const uint32_t *>(cm + l.off_flags), num_int, num_fp,
                      static_cast<uint8_t *>(dst), static_cast<uint16_t *>(meta), static_cast<uint16_t *>(fp_x), vec_out,
-                     sym_divisor, known_ndirty);
+                     sym_divisor);
   return check_launch();
 }
 

@@ -102,17 +102,16 @@ int colmap_flags(const void *colmap, int64_t cols, int64_t num_int, int64_t num_
   return QUIK_OK;
 }
 
-bool colmap_words_known(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, uint32_t (&out)[4]) {
-  std::lock_guard<std::mutex> lock(g_colmap_mutex);
-  auto it = g_colmap_flags.find(colmap);
-  if (it == g_colmap_flags.end() || it->second.cols != cols || it->second.num_int != num_int || it->second.num_fp != num_fp)
-    return false;
-  for (int i = 0; i < 4; ++i) out[i] = it->second.words[i];
-  return true;
-}
-
 int colmap_words(const void *colmap, int64_t cols, int64_t num_int, int64_t num_fp, hipStream_t st, uint32_t (&out)[4]) {
-  if (colmap_words_known(colmap, cols, num_int, num_fp, out)) return QUIK_OK;
+  {
+    std::lock_guard<std::mutex> lock(g_colmap_mutex);
+    auto it = g_colmap_flags.find(colmap);
+    if (it != g_colmap_flags.end() && it->second.cols == cols && it->second.num_int == num_int &&
+        it->second.num_fp == num_fp) {
+      for (int i = 0; i < 4; ++i) out[i] = it->second.words[i];
+      return QUIK_OK;
+    }
+  }
   hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
   if (hipStreamIsCapturing(st, &capture) != hipSuccess) {
     set_last_hip_error(hipGetLastError());
