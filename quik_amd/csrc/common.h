@@ -87,8 +87,8 @@ __device__ __forceinline__ float to_f32(uint16_t v) {
   }
 }
 
-// Two fp32 values -> bf16, round to nearest even, first value in the low half: one v_cvt_pk_bf16_f32 (checked against the
-// bit arithmetic for all 2^32 inputs: equal, subnormals included; a NaN stays some NaN).
+// Two fp32 values -> bf16, round to nearest even (subnormals included), first value in the low half: one v_cvt_pk_bf16_f32.
+// A NaN keeps its sign and the upper bits of its payload: what is stored goes through canonical_nans first.
 __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
   typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
   typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -118,6 +118,22 @@ __device__ __forceinline__ uint32_t pack2_from_f32(float a, float b) {
     typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
     typedef float float2_t __attribute__((ext_vector_type(2)));
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(float2_t{a, b}, half2_t));
+  }
+}
+
+// In front of pack2_from_f32 where the values are stored: every NaN becomes the one that from_f32 makes of it for bf16
+// (0x7FC0), so that a result's bits do not depend on the kernel that a call takes.  A compare for two values and a branch for
+// sixteen, not taken where there is no NaN.
+template <bool BF16, class V16>
+__device__ __forceinline__ void canonical_nans(V16 &v) {
+  if constexpr (BF16) {
+    bool any = false;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) any |= __builtin_isunordered(v[2 * k], v[2 * k + 1]);
+    if (__builtin_amdgcn_ballot_w64(any)) {
+#pragma unroll
+      for (int k = 0; k < 16; ++k) v[k] = v[k] != v[k] ? __uint_as_float(0x7FC00000u) : v[k];
+    }
   }
 }
 

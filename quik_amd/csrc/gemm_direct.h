@@ -292,6 +292,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   }
   __syncthreads();  // every wave has read its slots: the area becomes the output tile
   if (D::owns(wave)) {
+    canonical_nans<BF16>(own);
 #pragma unroll
     for (int g = 0; g < 4; ++g)
       *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (oni * 32 + acc_col(g, lane)) * 2) =

@@ -946,11 +946,13 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &p, int tm, int tn, u
   for (int mi = 0; mi < C::MI; ++mi) {
     const int mb = m0 + wm * C::WM + mi * 32;
 #pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni)
+    for (int ni = 0; ni < C::NI; ++ni) {
+      canonical_nans<BF16>(accf[mi][ni]);
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         Store::put_pairs(stage, lane, ni, g, pack2_from_f32<BF16>(accf[mi][ni][4 * g], accf[mi][ni][4 * g + 1]),
                          pack2_from_f32<BF16>(accf[mi][ni][4 * g + 2], accf[mi][ni][4 * g + 3]));
+    }
     if (mb < p.M && nw < p.N) Store::flush(stage, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec);
     __builtin_amdgcn_sched_barrier(0);
   }

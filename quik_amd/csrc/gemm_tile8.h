@@ -361,12 +361,14 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
 #pragma unroll
   for (int mi = 0; mi < C::MI; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni)
+    for (int ni = 0; ni < C::NI; ++ni) {
+      canonical_nans<BF16>(acc[mi][ni]);
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         Store::put_pairs(stage + mi * Store::kBytes, lane, ni, g,
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g], acc[mi][ni][4 * g + 1]),
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g + 2], acc[mi][ni][4 * g + 3]));
+    }
   if (vec && p.M - mw >= C::WM && p.N - nw >= C::WN) {  // interior (wave-uniform): straight-line code
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
