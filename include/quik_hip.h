@@ -118,8 +118,10 @@ int quik_sym_dequantize(const void *x, int x_bits, const void *scale_row,
  * memory.  Of the calls with at most 32 rows (quik_fused_dequantize_workspace_bytes(M, N) > 0) some run
  * on the weight-streaming kernel, which has no such epilogue: for those the exact int32 product goes to
  * acc_workspace ([M, N] int32, caller-provided) and a second launch applies the epilogue (QUIK_ERR_NULL
- * without a workspace); otherwise acc_workspace may be NULL. */
+ * without a workspace); otherwise acc_workspace may be NULL.  quik_fused_dequantize_acc_bytes: what a call
+ * of these sizes makes use of (0: one launch), at most the bytes of the former. */
 int64_t quik_fused_dequantize_workspace_bytes(int64_t M, int64_t N);
+int64_t quik_fused_dequantize_acc_bytes(int64_t M, int64_t N, int64_t K, int bits);
 int quik_asym_fused_dequantize(const void *A, const void *B, const void *scale_row,
                                const void *scale_col, float shift_value, const void *zero_row,
                                const void *w_reduced, const void *y, int64_t M, int64_t N,

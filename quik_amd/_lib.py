@@ -33,6 +33,7 @@ SIGNATURES = {
                                           _vp, _vp, _vp]),
     "quik_sym_fused_dequantize": (_int, [_vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _int, _vp, _vp, _vp]),
     "quik_fused_dequantize_workspace_bytes": (_i64, [_i64, _i64]),
+    "quik_fused_dequantize_acc_bytes": (_i64, [_i64, _i64, _i64, _int]),
     "quik_fp6_operand_bytes": (_i64, [_i64, _i64, _i64]),
     "quik_fp6_pack_weight": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp]),
     "quik_colmap_streaming": (_int, [_vp, _i64, _i64, _i64, _vp]),
@@ -98,6 +99,17 @@ class _NoFront:
     that it does not serve."""
     def __getattr__(self, name):
         return lambda *args: None
+
+
+def front_fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits):
+    """The fused dequantize through the front end, or None for a call that it does not serve.  Of the calls of at most 32
+    rows some are two launches with the int32 product between them, whose memory is made here once the call is known to fit."""
+    call = front().fused_dequantize
+    out = call(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, None)
+    if out is True:
+        acc = torch.empty((A.size(0), B.size(0)), dtype=torch.int32, device=A.device)
+        out = call(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, acc)
+    return out
 
 
 _front = None

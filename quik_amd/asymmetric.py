@@ -237,7 +237,7 @@ def _fused_operands(op, A, B, bits):
 
 def _fused_dequantize(op, bits, A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y):
     if zero_row is not None:
-        out = L.front().fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits)
+        out = L.front_fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits)
         if out is not None:
             return out
     L.check_cuda_contiguous(op, A=A, B=B, scale_row=scale_row, scale_col=scale_col, zero_row=zero_row,

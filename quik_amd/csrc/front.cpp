@@ -515,10 +515,11 @@ PyObject *py_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   });
 }
 
-// fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits) -> out or None; zero_row and
-// w_reduced None: the symmetric form.  Calls that need a workspace (some of at most 32 rows) stay with the Python function.
+// fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, acc) -> out, None or True; zero_row
+// and w_reduced None: the symmetric form.  acc: the int32 workspace of a call in two launches (some of at most 32 rows), or None;
+// True: the call fits but for that workspace, and nothing has been allocated or launched.
 PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
-  if (n != 9) Py_RETURN_NONE;
+  if (n != 10) Py_RETURN_NONE;
   const c10::DeviceIndex dev = current_gpu();
   const bool sym = args[5] == Py_None;
   const at::Tensor *A = plain(args[0], dev), *B = plain(args[1], dev), *sr = plain(args[2], dev), *sc = plain(args[3], dev),
@@ -538,14 +539,20 @@ PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   auto half = [](const at::Tensor *t, int64_t count) { return t->scalar_type() == at::kHalf && t->numel() == count; };
   if (M * N == 0 || K == 0 || !half(sr, M) || !half(sc, N) || !half(y, M * N) || (!sym && (!half(zr, M) || !half(wr, N))))
     Py_RETURN_NONE;
+  int32_t *acc = nullptr;
+  if (quik_fused_dequantize_acc_bytes(M, N, K, static_cast<int>(bits)) > 0) {
+    if (args[9] == Py_None) Py_RETURN_TRUE;
+    const at::Tensor *t = plain(args[9], dev);
+    if (!t || t->scalar_type() != at::kInt || t->numel() != M * N) Py_RETURN_NONE;
+    acc = static_cast<int32_t *>(out_ptr(*t));
+  }
   return guarded([&]() -> PyObject * {
     at::Tensor out = new_empty({M, N}, at::kHalf, dev);
     const int rc = sym ? quik_sym_fused_dequantize(ptr(*A), ptr(*B), ptr(*sr), ptr(*sc), ptr(*y), M, N, K, static_cast<int>(bits),
-                                                   nullptr, out_ptr(out), stream_of(dev))
+                                                   acc, out_ptr(out), stream_of(dev))
                        : quik_asym_fused_dequantize(ptr(*A), ptr(*B), ptr(*sr), ptr(*sc), static_cast<float>(shift), ptr(*zr),
-                                                    ptr(*wr), ptr(*y), M, N, K, static_cast<int>(bits), nullptr, out_ptr(out),
+                                                    ptr(*wr), ptr(*y), M, N, K, static_cast<int>(bits), acc, out_ptr(out),
                                                     stream_of(dev));
-    if (rc == QUIK_ERR_NULL) Py_RETURN_NONE;  // (no workspace was passed)
     if (rc != QUIK_OK) return fail(bits == 4 ? "int4FusedDequantize" : "int8FusedDequantize", rc);
     return THPVariable_Wrap(std::move(out));
   });

@@ -398,16 +398,19 @@ int launch_chain_split(const I32Args &a, const ChainArgs &e, int64_t n_wide, hip
   return check_launch();
 }
 
+// Fused dequantize of at most 32 rows: one round of row-streaming tiles can take the call.  Rows of more than 11 KB leave a
+// tile's waves too long a chain (int8 16 x 13824 -> 5120 24.8 us in two launches, 27.1 on the tiles, 16 x 28672 -> 8192 55 / 62), up to
+// four tiles are too few for long rows (16 x 8192 -> 256 8.8 / 9.3, 1 x 8192 -> 256 7.8 / 9.3).
+bool few_rows_on_tiles(int64_t M, int64_t N, int64_t kbytes) {
+  return M <= 32 && N > 256 && (N + 63) / 64 <= num_cus() && kbytes <= 11 * 1024;
+}
 template <int MODE, bool ASYM>
 int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
-  // Up to 32 rows: one launch on one round of row-streaming tiles, where the product by itself would go to the
-  // weight-streaming kernel and the epilogue to a second launch: the intermediate and that launch cost a caller more than the
-  // tiles lose on few columns.  us per call: 5 x 8192 -> 1024 15.6 -> 9.8, 21 x 1280 -> 544 15.6 -> 5.6, 32 x 4096 -> 11008 15.7
-  // -> 7.8, 24 x 8192 -> 8192 15.5 -> 10.8, int8 32 x 8192 -> 16000 46.9 -> 30.3 (kernels alone, int4: 9.0 / 9.5, 6.4 / 5.3, 13.1 / 8.5,
-  // 13.5 / 11.0).  Rows of more than 11 KB leave a tile's waves too long a chain (int8 16 x 13824 -> 5120 24.8 / 27.1, 16 x
-  // 28672 -> 8192 55 / 62).  Up to four tiles are too few for long rows (16 x 8192 -> 256 8.8 / 9.3, 1 x 8192 -> 256 7.8 / 9.3)
-  // and keep the two launches.
-  if (a.M <= 32 && a.N > 256 && (a.N + 63) / 64 <= num_cus() && a.kbytes <= 11 * 1024)
+  // Up to 32 rows: one launch, where the product by itself would go to the weight-streaming kernel and the epilogue to a second
+  // launch: the intermediate and that launch cost a caller more than the tiles lose on few columns.  us per call: 5 x 8192 ->
+  // 1024 15.6 -> 9.8, 21 x 1280 -> 544 15.6 -> 5.6, 32 x 4096 -> 11008 15.7 -> 7.8, 24 x 8192 -> 8192 15.5 -> 10.8, int8 32 x 8192 ->
+  // 16000 46.9 -> 30.3 (kernels alone, int4: 9.0 / 9.5, 6.4 / 5.3, 13.1 / 8.5, 13.5 / 11.0).
+  if (few_rows_on_tiles(a.M, a.N, a.kbytes))
     return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
   switch (rows_blocks(a.M, a.N, a.kbytes, MODE)) {
     case 2: return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
@@ -781,6 +784,11 @@ int int_gemm_chain(const void *A, const void *B, const void *s_row, const void *
 }  // namespace quik
 
 using namespace quik;
+
+extern "C" int64_t quik_fused_dequantize_acc_bytes(int64_t M, int64_t N, int64_t K, int bits) {
+  if (M <= 0 || M > 32 || N <= 0 || K <= 0 || (bits != 4 && bits != 8)) return 0;
+  return few_rows_on_tiles(M, N, bits == 4 ? K / 2 : K) ? 0 : M * N * 4;
+}
 
 extern "C" int quik_int4_matmul(const uint8_t *A, const uint8_t *B, int32_t *C, int64_t M, int64_t N, int64_t K,
                                 void *stream) {

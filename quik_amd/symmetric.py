@@ -66,7 +66,7 @@ def dequantize(x: torch.Tensor, scale_row: torch.Tensor, scale_col: torch.Tensor
 
 
 def _fused_dequantize(op, bits, A, B, scale_row, scale_col, y):
-    out = L.front().fused_dequantize(A, B, scale_row, scale_col, 0.0, None, None, y, bits)
+    out = L.front_fused_dequantize(A, B, scale_row, scale_col, 0.0, None, None, y, bits)
     if out is not None:
         return out
     L.check_cuda_contiguous(op, A=A, B=B, scale_row=scale_row, scale_col=scale_col, y=y)

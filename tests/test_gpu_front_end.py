@@ -310,3 +310,32 @@ def test_interposed_inputs_stay_with_the_python_functions():
     with Seen():
         out = mod(x)
     assert _same(out, first) and any("empty" in op for op in Seen.ops)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 200, 256), (1, 64, 4096), (8, 64 * 260, 256), (16, 512, 256), (40, 512, 256)])
+@pytest.mark.parametrize("bits", [4, 8])
+def test_fused_dequantize_allocates_what_it_uses(M, N, K, bits):
+    """The result, and for a call in two launches the int32 product: no result that is thrown away because the call turns
+    out to need the product's memory."""
+    import quik
+    from quik_amd import _lib as L
+    if isinstance(L.front(), L._NoFront):
+        pytest.skip("no native front end")
+    g = torch.Generator(device=DEV).manual_seed(M + N + K)
+    kbytes = K // 2 if bits == 4 else K
+    a, b = (torch.randint(-8, 8, (n, kbytes), generator=g, device=DEV, dtype=torch.int8) for n in (M, N))
+    if bits == 4:
+        a, b = a.view(torch.uint8), b.view(torch.uint8)
+    s_row, s_col = ((torch.rand(*s, generator=g, device=DEV) * 0.1).half() for s in ((M, 1), (1, N)))
+    y = torch.randn(M, N, generator=g, device=DEV).half()
+    op = quik.symmetric.int4FusedDequantize if bits == 4 else quik.symmetric.int8FusedDequantize
+    op(a, b, s_row, s_col, y)
+    made = torch.cuda.memory_stats()["allocation.all.allocated"]
+    got = op(a, b, s_row, s_col, y)
+    made = torch.cuda.memory_stats()["allocation.all.allocated"] - made
+    need = L.load().quik_fused_dequantize_acc_bytes(M, N, K, bits)
+    assert need in (0, M * N * 4) and (need == 0 or M <= 32)
+    assert made == (2 if need else 1)
+    mm = quik.matmul.int4Matmul if bits == 4 else quik.matmul.int8Matmul
+    want = quik.symmetric.dequantize(mm(a, b), s_row, s_col, y, 32)
+    assert torch.equal(got.view(torch.int16), want.view(torch.int16))
