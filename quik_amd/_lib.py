@@ -101,15 +101,9 @@ class _NoFront:
         return lambda *args: None
 
 
-def front_fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits):
-    """The fused dequantize through the front end, or None for a call that it does not serve.  Of the calls of at most 32
-    rows some are two launches with the int32 product between them, whose memory is made here once the call is known to fit."""
-    call = front().fused_dequantize
-    out = call(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, None)
-    if out is True:
-        acc = torch.empty((A.size(0), B.size(0)), dtype=torch.int32, device=A.device)
-        out = call(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, acc)
-    return out
+def product_memory(A, B):
+    """The int32 matrix between the two launches of a fused dequantize of few rows."""
+    return torch.empty((A.shape[0], B.shape[0]), dtype=torch.int32, device=A.device)
 
 
 _front = None

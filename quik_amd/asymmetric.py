@@ -237,7 +237,8 @@ def _fused_operands(op, A, B, bits):
 
 def _fused_dequantize(op, bits, A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y):
     if zero_row is not None:
-        out = L.front_fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits)
+        out = L.front().fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits,
+                                         L.product_memory)
         if out is not None:
             return out
     L.check_cuda_contiguous(op, A=A, B=B, scale_row=scale_row, scale_col=scale_col, zero_row=zero_row,
@@ -251,8 +252,7 @@ def _fused_dequantize(op, bits, A, B, scale_row, scale_col, shift_value, zero_ro
     lib = L.load()
     with L.device_guard(A.device):
         # one launch, no int32 matrix; only calls of at most 32 rows (weight-streaming kernel) need the workspace
-        acc = torch.empty((M, N), dtype=torch.int32, device=A.device) \
-            if lib.quik_fused_dequantize_workspace_bytes(M, N) else None
+        acc = L.product_memory(A, B) if lib.quik_fused_dequantize_workspace_bytes(M, N) else None
         out = torch.empty((M, N), dtype=torch.float16, device=A.device)
         L.check(lib.quik_asym_fused_dequantize(L.ptr(A), L.ptr(B), L.ptr(scale_row), L.ptr(scale_col),
                                                float(shift_value), L.ptr(zero_row), L.ptr(w_reduced), L.ptr(y), M, N,

@@ -68,11 +68,12 @@ int mixed_linear_tile8(const void *x8, const void *w8, const void *meta, const v
                        void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);
 
 // gemm.hip: integer GEMM + the fp16-arithmetic epilogue of the reference's fused ops in one launch (zero_row ==
-// NULL: symmetric form).  Returns kChainNotHandled for shapes it leaves to the two-launch path.
+// NULL: symmetric form).  Returns kChainNotHandled for calls it leaves to the two-launch path; two_launches: the caller has
+// the workspace for that one (without it the tiles take what they can).
 constexpr int kChainNotHandled = 1;
 int int_gemm_chain(const void *A, const void *B, const void *s_row, const void *s_col, const void *zero_row,
                    const void *w_red, uint16_t shift_bits, const void *y, int64_t M, int64_t N, int64_t K, int bits,
-                   void *out, hipStream_t st);
+                   void *out, bool two_launches, hipStream_t st);
 
 // ---- storage types as 16-bit patterns --------------------------------------------------
 // Half values are handled with the native _Float16 type; bfloat16 with explicit bit math

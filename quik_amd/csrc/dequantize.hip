@@ -212,7 +212,7 @@ extern "C" int quik_asym_fused_dequantize(const void *A, const void *B, const vo
   if (!scale_row || !scale_col || !zero_row || !w_reduced || !y || !out) return QUIK_ERR_NULL;
   const _Float16 shift = static_cast<_Float16>(shift_value);
   const int rc = int_gemm_chain(A, B, scale_row, scale_col, zero_row, w_reduced, __builtin_bit_cast(uint16_t, shift), y,
-                                M, N, K, bits, out, as_stream(stream));
+                                M, N, K, bits, out, acc_workspace != nullptr, as_stream(stream));
   if (rc != kChainNotHandled) return rc;
   // (of the calls of at most 32 rows) product by the weight-streaming kernel into the workspace, epilogue as a second launch
   if (!acc_workspace) return QUIK_ERR_NULL;
@@ -232,7 +232,7 @@ extern "C" int quik_sym_fused_dequantize(const void *A, const void *B, const voi
   if (M == 0 || N == 0) return QUIK_OK;
   if (!scale_row || !scale_col || !y || !out) return QUIK_ERR_NULL;
   const int rc = int_gemm_chain(A, B, scale_row, scale_col, nullptr, nullptr, 0, y, M, N, K, bits, out,
-                                as_stream(stream));
+                                acc_workspace != nullptr, as_stream(stream));
   if (rc != kChainNotHandled) return rc;
   if (!acc_workspace) return QUIK_ERR_NULL;
   if (int rc2 = int_matmul(A, B, acc_workspace, M, N, K, bits, stream)) return rc2;

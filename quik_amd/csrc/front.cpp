@@ -515,9 +515,9 @@ PyObject *py_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   });
 }
 
-// fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, acc) -> out, None or True; zero_row
-// and w_reduced None: the symmetric form.  acc: the int32 workspace of a call in two launches (some of at most 32 rows), or None;
-// True: the call fits but for that workspace, and nothing has been allocated or launched.
+// fused_dequantize(A, B, scale_row, scale_col, shift_value, zero_row, w_reduced, y, bits, product) -> out or None; zero_row and
+// w_reduced None: the symmetric form.  product(A, B): makes the int32 matrix of a call in two launches (some of at most 32
+// rows); called once the call is known to fit.
 PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   if (n != 10) Py_RETURN_NONE;
   const c10::DeviceIndex dev = current_gpu();
@@ -539,10 +539,12 @@ PyObject *py_fused_dequantize(PyObject *, PyObject *const *args, Py_ssize_t n) {
   auto half = [](const at::Tensor *t, int64_t count) { return t->scalar_type() == at::kHalf && t->numel() == count; };
   if (M * N == 0 || K == 0 || !half(sr, M) || !half(sc, N) || !half(y, M * N) || (!sym && (!half(zr, M) || !half(wr, N))))
     Py_RETURN_NONE;
+  PyRef product;
   int32_t *acc = nullptr;
   if (quik_fused_dequantize_acc_bytes(M, N, K, static_cast<int>(bits)) > 0) {
-    if (args[9] == Py_None) Py_RETURN_TRUE;
-    const at::Tensor *t = plain(args[9], dev);
+    product.p = PyObject_CallFunctionObjArgs(args[9], args[0], args[1], nullptr);
+    if (!product.p) return nullptr;
+    const at::Tensor *t = plain(product.p, dev);
     if (!t || t->scalar_type() != at::kInt || t->numel() != M * N) Py_RETURN_NONE;
     acc = static_cast<int32_t *>(out_ptr(*t));
   }

@@ -404,13 +404,25 @@ int launch_chain_split(const I32Args &a, const ChainArgs &e, int64_t n_wide, hip
 bool few_rows_on_tiles(int64_t M, int64_t N, int64_t kbytes) {
   return M <= 32 && N > 256 && (N + 63) / 64 <= num_cus() && kbytes <= 11 * 1024;
 }
+// .. but product (weight-streaming kernel) and epilogue in two launches are faster.  The tiles multiply 64 rows whatever M is and
+// keep N / 64 CUs busy, so their time grows with K alone; the product's grows with M and, where each CU has at most one slab of 32
+// columns, little with K.  us per call in a graph, two launches / tiles, 1024 columns unless said:
+//   int4, K = 8192   1 row 8.2 / 9.4, 16 rows 9.1 / 9.5, 24 rows 9.8 / 9.5; 8192 columns, 8 rows 9.5 / 10.4; 11008, 8 rows 13.5 / 11.1
+//   int4, K = 11264  16 rows 10.3 / 11.6, 24 rows 11.3 / 11.6, 32 rows 12.6 / 11.6; 8192 columns, 16 rows 13.1 / 12.6
+//   int4, K = 22016  24 rows 17.3 / 18.6, 32 rows 18.7 / 18.6; 4096 columns, 24 rows 19.4 / 19.1
+//   int8, K = 5632   8 rows 8.3 / 9.0, 16 rows 9.4 / 9.0; K = 8192 8 rows 10.1 / 11.0, 16 rows 11.7 / 11.0; 8192 columns, 1 row
+//                    17.7 / 13.5; K = 11008 8 rows 11.9 / 13.5
+// Not replayed, the second launch starts 1.5 us later (int4, K = 8192, 1 row 10.0 / 9.6; int8, K = 8192 10.1 / 11.0): calls with
+// shorter rows, which the two serve little faster (1 row: int4, K = 4096 6.6 / 6.8, int8, K = 4096 7.1 / 7.5), stay on the tiles.
+bool few_rows_two_launches(int64_t M, int64_t N, int64_t kbytes, int mode) {
+  if (kbytes >= 5120) return N <= 16 * num_cus() && M <= (mode == kInt4 ? 24 : 8);
+  return mode == kInt4 && kbytes >= 4096 && N <= 32 * num_cus() && M <= 16;
+}
+
+// two_launches: the caller has a workspace for the product
 template <int MODE, bool ASYM>
-int run_chain(const I32Args &a, const ChainArgs &e, hipStream_t st) {
-  // Up to 32 rows: one launch, where the product by itself would go to the weight-streaming kernel and the epilogue to a second
-  // launch: the intermediate and that launch cost a caller more than the tiles lose on few columns.  us per call: 5 x 8192 ->
-  // 1024 15.6 -> 9.8, 21 x 1280 -> 544 15.6 -> 5.6, 32 x 4096 -> 11008 15.7 -> 7.8, 24 x 8192 -> 8192 15.5 -> 10.8, int8 32 x 8192 ->
-  // 16000 46.9 -> 30.3 (kernels alone, int4: 9.0 / 9.5, 6.4 / 5.3, 13.1 / 8.5, 13.5 / 11.0).
-  if (few_rows_on_tiles(a.M, a.N, a.kbytes))
+int run_chain(const I32Args &a, const ChainArgs &e, bool two_launches, hipStream_t st) {
+  if (few_rows_on_tiles(a.M, a.N, a.kbytes) && !(two_launches && few_rows_two_launches(a.M, a.N, a.kbytes, MODE)))
     return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
   switch (rows_blocks(a.M, a.N, a.kbytes, MODE)) {
     case 2: return launch_chain_rows<RowsCfg<2>, MODE, ASYM>(a, e, st);
@@ -766,11 +778,11 @@ int run_fused(const FusedArgs &p, hipStream_t st) {
 }  // namespace
 
 // Integer GEMM with the fp16-arithmetic epilogue of the reference's fused ops in one launch (see ChainArgs in
-// gemm_kernels.h); kChainNotHandled when the shape belongs to the weight-streaming kernel (at most 32 rows), which
+// gemm_kernels.h); kChainNotHandled when the call belongs to the weight-streaming kernel (at most 32 rows), which
 // has no such epilogue: the caller then runs the product and the epilogue as two launches.
 int int_gemm_chain(const void *A, const void *B, const void *s_row, const void *s_col, const void *zero_row,
                    const void *w_red, uint16_t shift_bits, const void *y, int64_t M, int64_t N, int64_t K, int bits,
-                   void *out, hipStream_t st) {
+                   void *out, bool two_launches, hipStream_t st) {
   if (int rc = check_gemm_args(A, B, out, M, N, K, bits)) return rc;
   I32Args a{static_cast<const uint8_t *>(A), static_cast<const uint8_t *>(B), nullptr, static_cast<int>(M),
             static_cast<int>(N), static_cast<int>(N), static_cast<int>(bits == 4 ? K / 2 : K)};
@@ -778,8 +790,8 @@ int int_gemm_chain(const void *A, const void *B, const void *s_row, const void *
               static_cast<const uint16_t *>(zero_row), static_cast<const uint16_t *>(w_red),
               static_cast<const uint16_t *>(y), static_cast<uint16_t *>(out), static_cast<int>(N), shift_bits};
   const bool asym = zero_row != nullptr;
-  if (bits == 4) return asym ? run_chain<kInt4, true>(a, e, st) : run_chain<kInt4, false>(a, e, st);
-  return asym ? run_chain<kInt8, true>(a, e, st) : run_chain<kInt8, false>(a, e, st);
+  if (bits == 4) return asym ? run_chain<kInt4, true>(a, e, two_launches, st) : run_chain<kInt4, false>(a, e, two_launches, st);
+  return asym ? run_chain<kInt8, true>(a, e, two_launches, st) : run_chain<kInt8, false>(a, e, two_launches, st);
 }
 }  // namespace quik
 
@@ -787,7 +799,8 @@ using namespace quik;
 
 extern "C" int64_t quik_fused_dequantize_acc_bytes(int64_t M, int64_t N, int64_t K, int bits) {
   if (M <= 0 || M > 32 || N <= 0 || K <= 0 || (bits != 4 && bits != 8)) return 0;
-  return few_rows_on_tiles(M, N, bits == 4 ? K / 2 : K) ? 0 : M * N * 4;
+  const int64_t kbytes = bits == 4 ? K / 2 : K;
+  return few_rows_on_tiles(M, N, kbytes) && !few_rows_two_launches(M, N, kbytes, bits == 4 ? kInt4 : kInt8) ? 0 : M * N * 4;
 }
 
 extern "C" int quik_int4_matmul(const uint8_t *A, const uint8_t *B, int32_t *C, int64_t M, int64_t N, int64_t K,

@@ -66,7 +66,7 @@ def dequantize(x: torch.Tensor, scale_row: torch.Tensor, scale_col: torch.Tensor
 
 
 def _fused_dequantize(op, bits, A, B, scale_row, scale_col, y):
-    out = L.front_fused_dequantize(A, B, scale_row, scale_col, 0.0, None, None, y, bits)
+    out = L.front().fused_dequantize(A, B, scale_row, scale_col, 0.0, None, None, y, bits, L.product_memory)
     if out is not None:
         return out
     L.check_cuda_contiguous(op, A=A, B=B, scale_row=scale_row, scale_col=scale_col, y=y)
@@ -83,8 +83,7 @@ def _fused_dequantize(op, bits, A, B, scale_row, scale_col, y):
     lib = L.load()
     with L.device_guard(A.device):
         # one launch, no int32 matrix; only calls of at most 32 rows (weight-streaming kernel) need the workspace
-        acc = torch.empty((M, N), dtype=torch.int32, device=A.device) \
-            if lib.quik_fused_dequantize_workspace_bytes(M, N) else None
+        acc = L.product_memory(A, B) if lib.quik_fused_dequantize_workspace_bytes(M, N) else None
         out = torch.empty((M, N), dtype=torch.float16, device=A.device)
         L.check(lib.quik_sym_fused_dequantize(L.ptr(A), L.ptr(B), L.ptr(scale_row), L.ptr(scale_col), L.ptr(y), M, N, K,
                                               bits, L.ptr(acc), L.ptr(out), L.stream()), op)

@@ -78,3 +78,48 @@ def test_fused_form_with_y_in_the_lds_or_not(M, N, kbytes, off):
     got = quik.symmetric.int4FusedDequantize(a, b, s_row, s_col, y)
     want = quik.symmetric.dequantize(quik.matmul.int4Matmul(a, b), s_row, s_col, y.clone(), 32)
     assert torch.equal(got.view(torch.int16), want.view(torch.int16))
+
+
+@pytest.mark.parametrize("bits,M,N,kbytes", [(4, 1, 512, 4080), (4, 16, 8192, 4096), (4, 17, 512, 4096), (4, 1, 8256, 4096),
+                                             (4, 24, 4096, 5120), (4, 25, 4096, 5632), (4, 1, 4160, 5632), (8, 1, 320, 5104),
+                                             (8, 8, 4096, 5120), (8, 9, 321, 8192), (8, 1, 4160, 8192), (8, 3, 1001, 11264)])
+def test_few_rows_in_one_launch_or_two(bits, M, N, kbytes):
+    """Both sides of the rule between the row-streaming tiles and product + epilogue: the same bits, with a workspace and
+    without one (then the tiles take either), eager and replayed from a graph."""
+    import quik
+    from quik_amd import _lib as L
+    g = torch.Generator(device=DEV).manual_seed(M + N + kbytes)
+    a, b, ca, cb = _operands(M, N, kbytes, bits, g)
+    K = kbytes * (2 if bits == 4 else 1)
+    lib = L.load()
+    rows, most = (24 if bits == 4 else 8, 4096) if kbytes >= 5120 else (16, 8192) if bits == 4 and kbytes >= 4096 else (0, 0)
+    two = M <= rows and N <= most
+    assert lib.quik_fused_dequantize_acc_bytes(M, N, K, bits) == (M * N * 4 if two else 0)
+    s_row, s_col, zero, w_red, y = ((torch.rand(*s, generator=g, device=DEV) * 0.1).half()
+                                    for s in ((M, 1), (1, N), (M, 1), (1, N), (M, N)))
+    acc = (ca.double() @ cb.double().t().contiguous()).to(torch.int32)
+    host = [t.cpu().numpy() for t in (acc, s_row, s_col, zero, w_red, y)]
+    with np.errstate(all="ignore"):
+        want = qo.asym_fused_dequantize(host[0], host[1], host[2], 8.0, *host[3:])
+
+    def check(out):
+        got = out.cpu().numpy()
+        assert np.array_equal(np.isnan(got), np.isnan(want))
+        assert np.array_equal(got[~np.isnan(want)].view(np.uint16), want[~np.isnan(want)].view(np.uint16))
+    op = quik.asymmetric.int4FusedDequantize if bits == 4 else quik.asymmetric.int8FusedDequantize
+
+    def call():
+        return op(a, b, s_row, s_col, 8.0, zero, w_red, y)
+    check(call())
+    out = torch.empty(M, N, dtype=torch.float16, device=DEV)
+    L.check(lib.quik_asym_fused_dequantize(L.ptr(a), L.ptr(b), L.ptr(s_row), L.ptr(s_col), 8.0, L.ptr(zero), L.ptr(w_red), L.ptr(y),
+                                           M, N, K, bits, None, L.ptr(out), L.stream()), "without a workspace")
+    check(out)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        held = call()
+    for _ in range(3):
+        held.zero_()
+        call()
+        graph.replay()
+        check(held)
