@@ -563,12 +563,16 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
 
 // Register-streaming kernel (gemm_direct.h), ring kernel or ring kernel with a K split, for problems below the 256-row
 // tiles.  All are priced in ns: a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (87 in the ring
-// of 128x64 tiles), never less than the weights take: up to 64 MB, which the Infinity Cache keeps beside other layers' of
-// that size, at 8 TB/s (64 x 8192 -> 8192, 52 MB: 64x32 tiles 15.9 us per forward, 64x64 17.6); more from memory, at what each
-// kernel reaches, and at most 24 bytes per ns for each CU that works (8 bits, 64 x 28672 -> 8192, 232 MB: 64x64 tiles 78 us on
-// 128 CUs, 56 on 256, 64x32 tiles 67; 64 x 8192 -> 28672, 176 MB: ring 34).  A K split adds the exchange: its partial sums
-// cross memory, 16 KB per workgroup in the register-streaming kernel, 64 KB in the ring kernel (measured 13 us with its start
-// for two workgroups per tile, 22 .. 24 for three to eight).
+// of 128x64 tiles), never less than the weights take: up to 128 MB at 8 TB/s, more at what each kernel reaches from memory,
+// and at most 24 bytes per ns for each CU that works.  The 8 TB/s is not where such weights come from, a model's are cold; it is
+// what ranks the kernels as they were measured, warm and cold alike (layers over 700 MB in turn): over 24 layer shapes of 6 ..
+// 222 MB at 40 .. 192 rows, both widths, the pick is 0.6 % behind the fastest kernel warm and 1.7 % cold.  us per forward, warm /
+// cold, as picked and as the memory's rates would pick: 64 x 4096 -> 11008 13.6 / 18.2 (64x64 tiles) and 15.3 / 19.9 (ring),
+// 64 x 8192 -> 10240 18.4 / 27.2 and 20.8 / 29.9, 128 x 8192 -> 20480 28.8 / 46.5 (ring) and 36.5 / 54.2; int8 64 x 13824 -> 5120 23.4 /
+// 34.7 (64x64, two splits) and 27.9 / 35.8, but 64 x 14336 -> 8192 26.4 / 40.5 (64x32) and 29.0 / 36.4.  Beyond, the memory's rates
+// are the better ones cold: 64 x 28672 -> 8192 37.0 / 46.6 and 35.6 / 54.5 at 8 TB/s, int8 46.7 / 65.9 and 44.0 / 77.5.  A K split
+// adds the exchange: its partial sums cross memory, 16 KB per workgroup in the register-streaming kernel, 64 KB in the ring
+// kernel (measured 13 us with its start for two workgroups per tile, 22 .. 24 for three to eight).
 struct DirectPlan {
   int bn, splits;   // tile width (64 or 32; 0: ring kernel), workgroups per tile
   int64_t bytes;    // workspace of the split
@@ -582,7 +586,7 @@ DirectPlan plan_direct(int64_t M, int64_t N, int64_t K, int bits, int64_t worksp
   auto up = [](int64_t a, int64_t b) { return (a + b - 1) / b; };
   auto busiest = [&](int64_t groups, int64_t per, int64_t step_bytes, int64_t rate, int64_t memory) {
     const int64_t ns = up(groups, cus) * per * step_bytes / rate, by_cus = 24 * (groups < cus ? groups : cus);
-    const int64_t stream = weights / (weights <= (64 << 20) ? 8000 : by_cus < memory ? by_cus : memory);
+    const int64_t stream = weights / (weights <= (128 << 20) ? 8000 : by_cus < memory ? by_cus : memory);
     return ns > stream ? ns : stream;
   };
   const int64_t tiles128 = up(M, 128) * up(N, 128), tiles64 = up(M, 128) * up(N, 64);

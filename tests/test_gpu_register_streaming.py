@@ -22,10 +22,19 @@ CASES = [
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
 @pytest.mark.parametrize("case", CASES)
 def test_same_bits_as_the_row_major_kernels(case, dtype):
+    _same_bits(*case, dtype)
+
+
+@pytest.mark.parametrize("case", [(64, 5120, 13568, 256, 8), (96, 20480, 7936, 256, 4), (40, 8192, 10752, 256, 8)])
+def test_plans_of_large_weights(case):
+    """66, 116 and 84 MB of weights: 64x64 tiles with two splits, the ring of 128x128 tiles, 64x32 tiles."""
+    _same_bits(*case, torch.float16)
+
+
+def _same_bits(M, N, K, F, bits, dtype):
     from quik_amd import matmul
     from quik_amd.qlinear import MixedQLinear
-    M, N, K, F, bits = case
-    g = torch.Generator().manual_seed(sum(case))
+    g = torch.Generator().manual_seed(M + N + K + F + bits)
     fi = torch.randperm(K + F, generator=g)[:F]
     s_w = (torch.rand(N, 1, generator=g) * 0.009 + 0.001).to(dtype)
     lo, hi = (-8, 8) if bits == 4 else (-127, 128)
