@@ -30,6 +30,14 @@ def test_waves_past_the_last_row_and_column(M, N, K, F, bits):
     _same_bits(M, N, K, F, torch.bfloat16, bits)
 
 
+@pytest.mark.parametrize("bits", [4, 8])
+@pytest.mark.parametrize("M,N,K,F", [(2000, 11003, 256, 32), (1500, 11002, 1792, 64), (777, 21012, 640, 0)])
+def test_both_tile_widths_in_one_launch(M, N, K, F, bits):
+    """256x256 tiles with six slots beside 256x128 ones with eight or twelve, which start behind the first columns of every
+    vector; 208, 220 or 9 rows and 123, 122 or 20 columns in the last tiles."""
+    _same_bits(M, N, K, F, torch.bfloat16 if M == 777 else torch.float16, bits)
+
+
 def _same_bits(M, N, K, F, dtype, bits):
     from quik_amd.qlinear import MixedQLinear
     g = torch.Generator().manual_seed(M + N + K + F)
