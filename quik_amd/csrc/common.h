@@ -89,7 +89,7 @@ __device__ __forceinline__ float to_f32(uint16_t v) {
 }
 
 // Two fp32 values -> bf16, round to nearest even (subnormals included), first value in the low half: one v_cvt_pk_bf16_f32.
-// A NaN keeps its sign and the upper bits of its payload: what is stored goes through canonical_nans first.
+// A NaN keeps its sign and the upper bits of its payload: what is stored goes through canonical_nans.
 __device__ __forceinline__ uint32_t pack2_bf16(float a, float b) {
   typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
   typedef float float2_t __attribute__((ext_vector_type(2)));
@@ -122,20 +122,44 @@ __device__ __forceinline__ uint32_t pack2_from_f32(float a, float b) {
   }
 }
 
-// In front of pack2_from_f32 where the values are stored: every NaN becomes the one that from_f32 makes of it for bf16
-// (0x7FC0), so that a result's bits do not depend on the kernel that a call takes.  A compare for two values and a branch for
-// sixteen, not taken where there is no NaN.
-template <bool BF16, class V16>
-__device__ __forceinline__ void canonical_nans(V16 &v) {
-  if constexpr (BF16) {
-    bool any = false;
+// Where pairs of pack2_from_f32 are stored, every NaN becomes the one that from_f32 makes of it for bf16 (0x7FC0), so that a
+// result's bits do not depend on the kernel that a call takes.  A wave looks for NaNs in the packed words while it stores them,
+// one product with zero per word, and where it found one (or an infinity) it replaces the NaNs in what it has staged and stores
+// that again.  us per forward, without the watch and with it: 777 x 4096 -> 22016 65.4 / 65.4, 2048 x 4096 -> 4096 36.7 / 36.6, 777 x
+// 4096 -> 4096 23.0 / 23.5, int8 2048 x 28672 -> 8192 423 / 429.  (Looking at the accumulators instead costs registers that the
+// large tiles do not have: replacing NaNs there spilled up to 322 of them and took 777 x 4096 -> 22016 from 69 to 81 us, comparing
+// them alone spilled 34, 61.9 -> 66.5.)
+template <bool BF16>
+struct NanWatch {
+  float seen = 0.0f;  // NaN once one was seen
+  template <class V4>
+  __device__ __forceinline__ void add(const V4 &words) {
+    if constexpr (BF16) {
+      typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+      const bf2_t zero = {static_cast<__bf16>(0.0f), static_cast<__bf16>(0.0f)};
 #pragma unroll
-    for (int k = 0; k < 8; ++k) any |= __builtin_isunordered(v[2 * k], v[2 * k + 1]);
-    if (__builtin_amdgcn_ballot_w64(any)) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) v[k] = v[k] != v[k] ? __uint_as_float(0x7FC00000u) : v[k];
+      for (int k = 0; k < 4; ++k) seen = __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf2_t, static_cast<uint32_t>(words[k])), zero, seen, false);
     }
   }
+  // (wave-uniform)
+  __device__ __forceinline__ bool any() const {
+    if constexpr (BF16) return __builtin_amdgcn_ballot_w64(seen != seen) != 0;
+    return false;
+  }
+};
+__device__ __forceinline__ uint32_t canonical_bf16_pair(uint32_t w) {
+  const uint32_t lo = (w & 0x7FFFu) > 0x7F80u ? 0x7FC0u : w & 0xFFFFu, hi = (w & 0x7FFF0000u) > 0x7F800000u ? 0x7FC00000u : w & 0xFFFF0000u;
+  return lo | hi;
+}
+// stage: `bytes` (a multiple of 16) of LDS that this wave has staged and stored; afterwards it can be stored again
+__device__ __forceinline__ void canonical_nans(uint8_t *stage, int bytes) {
+#pragma unroll 1
+  for (int i = (threadIdx.x & 63) * 16; i < bytes; i += 1024) {
+    uint4 *at = reinterpret_cast<uint4 *>(stage + i);
+    const uint4 w = *at;
+    *at = make_uint4(canonical_bf16_pair(w.x), canonical_bf16_pair(w.y), canonical_bf16_pair(w.z), canonical_bf16_pair(w.w));
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (a wait only: no hazard; the first stores are done)
 }
 
 // Round an fp32 value to the storage type and return it as fp32 again.

@@ -292,7 +292,6 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   }
   __syncthreads();  // every wave has read its slots: the area becomes the output tile
   if (D::owns(wave)) {
-    canonical_nans<BF16>(own);
 #pragma unroll
     for (int g = 0; g < 4; ++g)
       *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (oni * 32 + acc_col(g, lane)) * 2) =
@@ -301,21 +300,34 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   __syncthreads();
   const bool vec = (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
   constexpr int kPieces = D::BN / 8;  // 16-byte pieces of a row
+  NanWatch<BF16> nans;
+  auto store = [&](auto again) QUIK_INLINE {
 #pragma unroll
-  for (int i = threadIdx.x; i < D::BM * kPieces; i += D::kThreads) {
-    const int row = i / kPieces, col = (i % kPieces) * 8;
-    if (m0 + row >= p.M || n0 + col >= p.N) continue;
-    const v4i piece = *reinterpret_cast<const v4i *>(smem + row * D::OUT_STRIDE + col * 2);
-    uint16_t *dst = p.out + int64_t(m0 + row) * p.ldo + n0 + col;
-    if (vec && n0 + col + 8 <= p.N) {
-      __builtin_nontemporal_store(piece, reinterpret_cast<v4i *>(dst));
-    } else {
-      uint16_t tmp[8];
-      __builtin_memcpy(tmp, &piece, 16);
+    for (int i = threadIdx.x; i < D::BM * kPieces; i += D::kThreads) {
+      const int row = i / kPieces, col = (i % kPieces) * 8;
+      if (m0 + row >= p.M || n0 + col >= p.N) continue;
+      v4i piece = *reinterpret_cast<const v4i *>(smem + row * D::OUT_STRIDE + col * 2);
+      if constexpr (again) {
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        if (n0 + col + e < p.N) dst[e] = tmp[e];
+        for (int k = 0; k < 4; ++k) piece[k] = static_cast<int>(canonical_bf16_pair(static_cast<uint32_t>(piece[k])));
+      }
+      uint16_t *dst = p.out + int64_t(m0 + row) * p.ldo + n0 + col;
+      if (vec && n0 + col + 8 <= p.N) {
+        __builtin_nontemporal_store(piece, reinterpret_cast<v4i *>(dst));
+      } else {
+        uint16_t tmp[8];
+        __builtin_memcpy(tmp, &piece, 16);
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (n0 + col + e < p.N) dst[e] = tmp[e];
+      }
+      if constexpr (!again) nans.add(piece);
     }
+  };
+  store(std::false_type{});
+  if (nans.any()) {
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // (a wait only: no hazard; the first stores are done)
+    store(std::true_type{});
   }
 }
 

@@ -434,8 +434,8 @@ struct TileVectors6 {
 // column, 16 bits each into the low half of its slot) and widened in place, by the same thread, when they have landed.  Read
 // into registers and written to the LDS they cost two trips to memory, one for the columns and one for the rows, before
 // the first copy left: 128 x 5120 -> 13824 19.1 -> 18.3 us per forward, 300 x 4544 -> 4544 18.1 -> 17.4, 512 x 4096 -> 4096
-// 18.2 -> 17.7, bf16 777 x 4096 -> 22016 70.1 -> 68.8, 2048 x 8192 -> 28672 269.4 -> 265.4; 2048 x 8192 -> 1024 30.35 ->
-// 30.12, int8 365 x 28672 -> 8192 144.9 -> 144.6.
+// 18.2 -> 17.7, bf16 777 x 4096 -> 22016 70.1 -> 68.8; where a tile takes long, no difference beyond the noise (2048 x 8192 -> 28672,
+// 2048 x 8192 -> 1024, int8 365 x 28672 -> 8192).
 template <class C, class Vectors, class Args>
 __device__ __forceinline__ void tile_vector_request(const Vectors &tv, const Args &p, int m0, int n0, int wave) {
   const int i = threadIdx.x;
@@ -706,14 +706,13 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
 #pragma unroll
   for (int mi = 0; mi < C::MI; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni) {
-      canonical_nans<BF16>(acc[mi][ni]);
+    for (int ni = 0; ni < C::NI; ++ni)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         Store::put_pairs(stage + mi * Store::kBytes, lane, ni, g,
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g], acc[mi][ni][4 * g + 1]),
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g + 2], acc[mi][ni][4 * g + 3]));
-    }
+  NanWatch<BF16> nans;
   if (vec && p.M - mw >= C::WM && p.N - nw >= C::WN) {  // interior (wave-uniform): straight-line code
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -722,13 +721,22 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
     for (int mi = 0; mi < C::MI; ++mi) Store::read_block(stage + mi * Store::kBytes, lane, piece[mi]);
 #pragma unroll
     for (int mi = 0; mi < C::MI; ++mi)
-      Store::write_block(piece[mi], lane, p.out + int64_t(mw + mi * 32) * p.ldo + nw, p.ldo);
+      Store::write_block(piece[mi], lane, p.out + int64_t(mw + mi * 32) * p.ldo + nw, p.ldo, nans);
   } else {
 #pragma unroll
     for (int mi = 0; mi < C::MI; ++mi) {
       const int mb = mw + mi * 32;
       if (mb < p.M && nw < p.N)
-        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec);
+        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec, nans);
+    }
+  }
+  if (nans.any()) {
+    canonical_nans(stage, C::MI * Store::kBytes);
+#pragma unroll 1
+    for (int mi = 0; mi < C::MI; ++mi) {
+      const int mb = mw + mi * 32;
+      if (mb < p.M && nw < p.N)
+        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec, nans);
     }
   }
 }

@@ -535,10 +535,13 @@ struct BlockStore {
       piece[it] = *reinterpret_cast<const v4i *>(stage + (it * kRowsPerInstr + lane / kLanesPerRow) * kRowBytes +
                                                  (lane % kLanesPerRow) * 16);
   }
-  static __device__ __forceinline__ void write_block(const v4i (&piece)[kIters], int lane, T *g, int64_t ld) {
+  template <class Watch>
+  static __device__ __forceinline__ void write_block(const v4i (&piece)[kIters], int lane, T *g, int64_t ld, Watch &watch) {
 #pragma unroll
-    for (int it = 0; it < kIters; ++it)
+    for (int it = 0; it < kIters; ++it) {
       store_piece(piece[it], g + int64_t(it * kRowsPerInstr + lane / kLanesPerRow) * ld + (lane % kLanesPerRow) * kElems);
+      watch.add(piece[it]);
+    }
   }
   // One 16-byte piece of an output row.  The fp16 / bf16 layer output is written once and not read again by this
   // launch: a streaming (non-temporal) store keeps its 100+ MB from displacing the operand lines that the tiles of
@@ -552,9 +555,10 @@ struct BlockStore {
     }
   }
 
-  // staged block -> g[row * ld + col], rows < rows_valid, cols < cols_valid
+  // staged block -> g[row * ld + col], rows < rows_valid, cols < cols_valid; watch: sees what is stored
+  template <class Watch = NanWatch<false>>
   static __device__ __forceinline__ void flush(const uint8_t *stage, int lane, T *g, int64_t ld, int rows_valid,
-                                               int cols_valid, bool vec) {
+                                               int cols_valid, bool vec, Watch &&watch = Watch{}) {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     if (vec && rows_valid >= 32 && cols_valid >= C::WN) {  // interior block (wave-uniform): straight-line code
@@ -565,8 +569,10 @@ struct BlockStore {
         piece[it] = *reinterpret_cast<const v4i *>(stage + (it * kRowsPerInstr + lane / kLanesPerRow) * kRowBytes +
                                                    (lane % kLanesPerRow) * 16);
 #pragma unroll
-      for (int it = 0; it < kIters; ++it)
+      for (int it = 0; it < kIters; ++it) {
         store_piece(piece[it], g + int64_t(it * kRowsPerInstr + lane / kLanesPerRow) * ld + (lane % kLanesPerRow) * kElems);
+        watch.add(piece[it]);
+      }
       __builtin_amdgcn_wave_barrier();
       return;
     }
@@ -575,6 +581,7 @@ struct BlockStore {
       const int r = it * kRowsPerInstr + lane / kLanesPerRow;
       const int c = (lane % kLanesPerRow) * kElems;
       const v4i piece = *reinterpret_cast<const v4i *>(stage + r * kRowBytes + (lane % kLanesPerRow) * 16);
+      watch.add(piece);
       if (r >= rows_valid) continue;
       T *dst = g + int64_t(r) * ld + c;
       if (vec && c + kElems <= cols_valid) {
@@ -946,14 +953,20 @@ __device__ __forceinline__ void fused_tile(const FusedArgs &p, int tm, int tn, u
   for (int mi = 0; mi < C::MI; ++mi) {
     const int mb = m0 + wm * C::WM + mi * 32;
 #pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni) {
-      canonical_nans<BF16>(accf[mi][ni]);
+    for (int ni = 0; ni < C::NI; ++ni)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         Store::put_pairs(stage, lane, ni, g, pack2_from_f32<BF16>(accf[mi][ni][4 * g], accf[mi][ni][4 * g + 1]),
                          pack2_from_f32<BF16>(accf[mi][ni][4 * g + 2], accf[mi][ni][4 * g + 3]));
+    if (mb < p.M && nw < p.N) {
+      NanWatch<BF16> nans;
+      uint16_t *out = p.out + int64_t(mb) * p.ldo + nw;
+      Store::flush(stage, lane, out, p.ldo, p.M - mb, p.N - nw, vec, nans);
+      if (nans.any()) {
+        canonical_nans(stage, Store::kBytes);
+        Store::flush(stage, lane, out, p.ldo, p.M - mb, p.N - nw, vec, nans);
+      }
     }
-    if (mb < p.M && nw < p.N) Store::flush(stage, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec);
     __builtin_amdgcn_sched_barrier(0);
   }
 }

@@ -361,14 +361,13 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
 #pragma unroll
   for (int mi = 0; mi < C::MI; ++mi)
 #pragma unroll
-    for (int ni = 0; ni < C::NI; ++ni) {
-      canonical_nans<BF16>(acc[mi][ni]);
+    for (int ni = 0; ni < C::NI; ++ni)
 #pragma unroll
       for (int g = 0; g < 4; ++g)
         Store::put_pairs(stage + mi * Store::kBytes, lane, ni, g,
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g], acc[mi][ni][4 * g + 1]),
                          pack2_from_f32<BF16>(acc[mi][ni][4 * g + 2], acc[mi][ni][4 * g + 3]));
-    }
+  NanWatch<BF16> nans;
   if (vec && p.M - mw >= C::WM && p.N - nw >= C::WN) {  // interior (wave-uniform): straight-line code
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
@@ -377,13 +376,22 @@ __device__ __forceinline__ void fused8t_tile(const Fused8Args &p, int tm, int tn
     for (int mi = 0; mi < C::MI; ++mi) Store::read_block(stage + mi * Store::kBytes, lane, piece[mi]);
 #pragma unroll
     for (int mi = 0; mi < C::MI; ++mi)
-      Store::write_block(piece[mi], lane, p.out + int64_t(mw + mi * 32) * p.ldo + nw, p.ldo);
+      Store::write_block(piece[mi], lane, p.out + int64_t(mw + mi * 32) * p.ldo + nw, p.ldo, nans);
   } else {
 #pragma unroll
     for (int mi = 0; mi < C::MI; ++mi) {
       const int mb = mw + mi * 32;
       if (mb < p.M && nw < p.N)
-        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec);
+        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec, nans);
+    }
+  }
+  if (nans.any()) {
+    canonical_nans(stage, C::MI * Store::kBytes);
+#pragma unroll 1
+    for (int mi = 0; mi < C::MI; ++mi) {
+      const int mb = mw + mi * 32;
+      if (mb < p.M && nw < p.N)
+        Store::flush(stage + mi * Store::kBytes, lane, p.out + int64_t(mb) * p.ldo + nw, p.ldo, p.M - mb, p.N - nw, vec, nans);
     }
   }
 }
