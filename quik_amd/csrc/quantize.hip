@@ -725,7 +725,9 @@ __global__ __launch_bounds__(TPR) void asym_quantize_stream_kernel(
   const uint32_t map_flags = flags[0], ndirty = flags[1];
   StreamTables<NV, TPR> tables;
   tables.load(grp, dirty, dirty_grp, reinterpret_cast<const uint16_t *>(fp_col), cols, num_fp);
-  tables.pin();
+  // (with sixteen groups per lane registers count for more: pinned / not, int8 1024 x 28672 27.5 / 26.1 us, bf16 in tile order
+  // 2048 x 28672 66.7 / 62.5)
+  if constexpr (NV < 16) tables.pin();
   if (map_flags & kColmapStreams) {
     uint8_t *codes_s = reinterpret_cast<uint8_t *>(row_s);
     stream_rows<BITS, BF16, NV, TPR, SYM, PF>(x, rows, cols, tables, dirty, dirty_grp, static_cast<int>(ndirty),
@@ -1699,8 +1701,8 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
   const IdxT *fp_col = reinterpret_cast<const IdxT *>(cm + l.off_fp);
   const uint32_t *mask = reinterpret_cast<const uint32_t *>(cm + l.off_mask);
   if constexpr (sizeof(IdxT) == 2) if (cols <= kStreamMaxCols && cols % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0) {
-    // Four waves per row, one row per workgroup: more, shorter waves hide the load and LDS latencies
-    // better than fewer waves with less per-row fixed work (measured with 64, 128 and 256 threads).
+    // Four waves per row, or eight (wide_rows), one row per workgroup: more, shorter waves hide the load and LDS latencies
+    // better than fewer waves with less per-row fixed work (64 and 128 threads were slower).
     const int64_t groups = cols / 8;
 #define QUIK_STREAM(NV, TPR) \
   return launch_stream<IdxT, BITS, BF16, NV, TPR>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, tiled)
