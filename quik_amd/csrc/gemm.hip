@@ -565,7 +565,7 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
 // tiles.  All are priced in ns: a fixed part, the operand bytes the busiest CU takes in at 103 bytes per ns (87 in the ring
 // of 128x64 tiles), never less than the weights take: up to 128 MB at 8 TB/s, more at what each kernel reaches from memory,
 // and at most 24 bytes per ns for each CU that works.  The 8 TB/s is not where such weights come from, a model's are cold; it is
-// what ranks the kernels as they were measured, warm and cold alike (layers over 700 MB in turn): over 24 layer shapes of 6 ..
+// what ranks the kernels as they were measured, warm and cold alike (layers over 700 MB in turn): over 23 layer shapes of 6 ..
 // 222 MB at 40 .. 192 rows, both widths, the pick is 0.6 % behind the fastest kernel warm and 1.7 % cold.  us per forward, warm /
 // cold, as picked and as the memory's rates would pick: 64 x 4096 -> 11008 13.6 / 18.2 (64x64 tiles) and 15.3 / 19.9 (ring),
 // 64 x 8192 -> 10240 18.4 / 27.2 and 20.8 / 29.9, 128 x 8192 -> 20480 28.8 / 46.5 (ring) and 36.5 / 54.2; int8 64 x 13824 -> 5120 23.4 /

@@ -9,10 +9,10 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 CASES = [
-    # M, N, K, F, bits, symmetric: every remainder, every quantize kernel (wave, streaming, LDS ring), GEMM tile and split
+    # M, N, K, F, bits, symmetric: every remainder, every quantize kernel (a workgroup per row, streaming, LDS ring), GEMM tile and split
     (33, 40, 32, 0, 4, False), (64, 96, 160, 32, 4, False), (65, 1000, 4288, 256, 4, False), (300, 4544, 4416, 128, 4, False),
     (257, 520, 1248, 64, 4, True), (2048, 4096, 1056, 96, 4, False), (1500, 8200, 672, 32, 4, False),
-    (64, 512, 8096, 96, 4, False), (1200, 300, 10848, 160, 4, False),
+    (64, 512, 8096, 96, 4, False), (1200, 300, 10848, 160, 4, False), (40, 96, 16480, 96, 4, False), (41, 64, 16416, 64, 4, True),
     (33, 40, 16, 0, 8, False), (64, 96, 80, 32, 8, False), (65, 1000, 4304, 256, 8, False), (300, 640, 11344, 256, 8, False),
     (2048, 4096, 1072, 96, 8, False), (100, 512, 20528, 480, 8, False),
 ]
