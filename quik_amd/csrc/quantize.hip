@@ -1218,13 +1218,15 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
 // memory system from about 2000 rows on.  A wave per row, two or eight of them in a workgroup and without any barrier, was
 // the form before: its two passes over up to five fragments per lane stood behind the transfer, and 64 rows occupied 64 of
 // 1024 SIMDs.  Here a pass takes as long as one fragment, for four barriers (image landed, outlier values read, holes
-// patched, range exchanged).  us per launch in a graph, wave per row -> this, 256 outlier columns, fp16: 16 x 4096 4.0 ->
-// 3.4, 64 x 8192 5.3 -> 3.6, 128 x 5120 4.7 -> 3.5, 777 x 4096 5.6 -> 4.6, 1024 x 8192 9.7 -> 8.1, 2048 x 8192 12.4 -> 12.1,
-// 8192 x 8192 49.0 -> 44.4, 64 x 28672 12.8 -> 5.5, 2048 x 28672 61.9 -> 40.4.  Slower where the wave form's rows were all
-// resident and each CU had seven or eight of them, if the input does not come from the cache's last launch: one input / four in
-// turn / 600 MB in turn, 2048 x 4096 6.8 / 7.8 / 8.3 -> 6.8 / 8.3 / 9.0, 2048 x 5120 8.7 / 9.2 / 9.9 -> 8.4 / 9.7 / 10.3, 1537 x 4096
-// 6.5 / 7.1 / 7.4 -> 6.2 / 7.4 / 7.9; from nine rows per CU on a quarter faster (2304 x 4096 9.9 / 11.3 / 12.5 -> 7.5 / 8.9 / 9.4).
-// Kept for these counts beside this one, on the same pieces, the wave form took 7.3 / 7.8 / 8.5 at 2048 x 4096.  bf16: 64 x 8192 7.5 -> 4.1, 777 x 4096 7.6 -> 5.7, 2048 x 28672 94 -> 46.
+// patched, range exchanged).  us per launch in a graph of twenty on one input, wave per row -> this, 256 outlier columns, fp16:
+// 16 x 4096 4.1 -> 3.5, 64 x 8192 5.3 -> 3.7, 128 x 5120 4.7 -> 3.6, 777 x 4096 5.4 -> 4.6, 1024 x 8192 7.9 -> 6.7, 8192 x 8192
+// 36.2 -> 31.0, 64 x 28672 12.5 -> 5.6, 2048 x 28672 56.8 -> 32.5; bf16 64 x 8192 9.6 -> 4.2, 777 x 4096 8.7 -> 5.5, 2048 x 28672
+// 115 -> 42 (with the rounding of quotient_pair_bf16).
+// Slower where the wave form's rows were all resident and each CU had seven or eight of them: 2048 x 8192 10.9 -> 11.3, and fewer
+// columns if the input does not come from the cache's last launch (one input / four in turn / 600 MB in turn: 2048 x 4096 6.8 /
+// 7.8 / 8.3 -> 6.8 / 8.3 / 9.0, 2048 x 5120 8.7 / 9.2 / 9.9 -> 8.4 / 9.7 / 10.3, 1537 x 4096 6.5 / 7.1 / 7.4 -> 6.2 / 7.4 / 7.9); from nine
+// rows per CU on a quarter faster (2304 x 4096 9.9 / 11.3 / 12.5 -> 7.5 / 8.9 / 9.4).  Kept for these counts beside this one, on the
+// same pieces, the wave form took 7.3 / 7.8 / 8.5 at 2048 x 4096.
 // (Fillers read beside the outlier values and the ranges of all waves in one LDS round trip, not one after the other:
 // 64 x 8192 3.68 -> 3.57, 2048 x 8192 12.3 -> 12.1, 64 x 28672 5.71 -> 5.48.)
 template <bool BF16, bool SYM, int JT>
