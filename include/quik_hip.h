@@ -117,9 +117,10 @@ int quik_sym_dequantize(const void *x, int x_bits, const void *scale_row,
  * One launch: the epilogue runs on the accumulators of the GEMM tiles; no int32 matrix goes through
  * memory.  Of the calls with at most 32 rows (quik_fused_dequantize_workspace_bytes(M, N) > 0) some run
  * on the weight-streaming kernel, which has no such epilogue: for those the exact int32 product goes to
- * acc_workspace ([M, N] int32, caller-provided) and a second launch applies the epilogue (QUIK_ERR_NULL
- * without a workspace); otherwise acc_workspace may be NULL.  quik_fused_dequantize_acc_bytes: what a call
- * of these sizes makes use of (0: one launch), at most the bytes of the former. */
+ * acc_workspace ([M, N] int32, caller-provided) and a second launch applies the epilogue; otherwise
+ * acc_workspace may be NULL.  quik_fused_dequantize_acc_bytes: what a call of these sizes makes use of (0: one
+ * launch), at most the bytes of the former.  A call that could use it and has none runs as one launch where the
+ * tiles take it (more slowly, with the same bits), and returns QUIK_ERR_NULL elsewhere. */
 int64_t quik_fused_dequantize_workspace_bytes(int64_t M, int64_t N);
 int64_t quik_fused_dequantize_acc_bytes(int64_t M, int64_t N, int64_t K, int bits);
 int quik_asym_fused_dequantize(const void *A, const void *B, const void *scale_row,
