@@ -181,6 +181,25 @@ int quik_mixed_linear_fwd_fp6(const void *x6, const void *w6, const void *meta, 
                               const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
                               int64_t K, int64_t F, void *out, void *stream);
 
+/* ---- the same path on 4-bit weights --------------------------------------------------------------------
+ * The 6-bit fields above hold levels of 4 bits; here a weight takes 4 bits in memory and is widened in registers, in
+ * front of its products: two thirds of the bytes, the same integers and the same output bits.  K % 32 == 0 suffices (the
+ * last k-steps are filled up).  The activation comes in one of two formats, in the order of the same column map:
+ *   x_bits 4   quik_asym_quantize_tile4 / quik_sym_quantize_mapped(tiled = QUIK_TILED_4), quik_tile4_operand_bytes(rows, ..)
+ *   x_bits 6   quik_asym_quantize_fp6 / quik_sym_quantize_mapped(tiled = 1), quik_fp6_operand_bytes(rows, ..) (K % 128 == 0)
+ * quik_tile4_activation_bits: the format whose kernels are the faster ones for a shape; either gives the same bits. */
+int64_t quik_tile4_operand_bytes(int64_t rows, int64_t K, int64_t F);
+int quik_tile4_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F,
+                           const void *colmap, void *out, void *stream);
+int quik_asym_quantize_tile4(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
+                             int64_t num_int, int64_t num_fp, void *out4, void *meta, void *stream);
+int quik_tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F);
+int quik_mixed_linear_fwd_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
+                                const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
+                                int64_t K, int64_t F, void *out, void *stream);
+/* `tiled` of quik_sym_quantize_mapped (bits = 4): the 4-bit operand buffer; `tiled_format` of quik_layer: 4-bit weights */
+#define QUIK_TILED_4 0x344C5451
+
 /* ---- symmetric activations in one kernel --------------------------------------------------------
  * MixedQLinear's symmetric branch (experiments/qlinear.py:97-103) computes, with torch ops and
  * symmetric.quantize: int_x = x[:, int_indices]; fp_x = x[:, fp_indices];
@@ -261,6 +280,8 @@ int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *m
  *   int_weight [out, num_int/2] u8 or [out, num_int] i8; weights_scales [out]; reduced_w [out] (NULL when
  *   symmetric); fp_weight [out, num_fp] (NULL when num_fp == 0); bias [out] or NULL
  *   tiled_weight    quik_layer_pack_weight (or quik_fp6_pack_weight / quik_tile8_pack_weight) buffer, or NULL
+ *   tiled_format    QUIK_TILED_4: tiled_weight is a quik_tile4_pack_weight buffer (bits = 4; two thirds of the bytes); any
+ *                   other value: one of the buffers above
  *   tiled_min_rows  33 is what MixedQLinear uses.  With 1 every call takes the tile-ordered path and reads
  *                   only tiled_weight: int_weight and fp_weight may then be NULL, i.e. the layer can live
  *                   with ONE copy of its weights (0.75 byte per int4 weight, 1 per int8 weight) at the price
@@ -274,7 +295,7 @@ typedef struct quik_layer {
   int32_t struct_bytes, bits, dtype, symmetric;
   int64_t in_features, num_int, num_fp, out_features;
   float sym_divisor;
-  int32_t colmap_streams, tiled_min_rows, reserved;
+  int32_t colmap_streams, tiled_min_rows, tiled_format;
   const void *colmap, *int_weight, *weights_scales, *reduced_w, *fp_weight, *bias, *tiled_weight;
 } quik_layer;
 /* tiled_weight for a layer whose integer columns are no multiple of 128 (4 bits; then of 32) or 64 (8 bits; of 16):

@@ -39,6 +39,11 @@ SIGNATURES = {
     "quik_colmap_streaming": (_int, [_vp, _i64, _i64, _i64, _vp]),
     "quik_asym_quantize_fp6": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp]),
     "quik_mixed_linear_fwd_fp6": (_int, [_vp, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp]),
+    "quik_tile4_operand_bytes": (_i64, [_i64, _i64, _i64]),
+    "quik_tile4_pack_weight": (_int, [_vp, _vp, _i64, _i64, _i64, _vp, _vp, _vp]),
+    "quik_asym_quantize_tile4": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp]),
+    "quik_tile4_activation_bits": (_int, [_i64, _i64, _i64, _i64]),
+    "quik_mixed_linear_fwd_tile4": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp]),
     "quik_sym_quantize_mapped": (_int, [_vp, _i64, _i64, _vp, _i64, _i64, _int, ctypes.c_float, _int, _vp, _vp, _vp,
                                         _vp]),
     "quik_tile8_operand_bytes": (_i64, [_i64, _i64, _i64]),
@@ -63,6 +68,7 @@ SIGNATURES = {
                                      _vp, _vp]),
 }
 
+TILED_4 = 0x344C5451    # QUIK_TILED_4: operand buffers, tiled weights of 4 bits
 
 
 class QuikLayer(ctypes.Structure):
@@ -70,7 +76,7 @@ class QuikLayer(ctypes.Structure):
     _fields_ = [("struct_bytes", ctypes.c_int32), ("bits", ctypes.c_int32), ("dtype", ctypes.c_int32),
                 ("symmetric", ctypes.c_int32), ("in_features", _i64), ("num_int", _i64), ("num_fp", _i64),
                 ("out_features", _i64), ("sym_divisor", ctypes.c_float), ("colmap_streams", ctypes.c_int32),
-                ("tiled_min_rows", ctypes.c_int32), ("reserved", ctypes.c_int32), ("colmap", _vp), ("int_weight", _vp),
+                ("tiled_min_rows", ctypes.c_int32), ("tiled_format", ctypes.c_int32), ("colmap", _vp), ("int_weight", _vp),
                 ("weights_scales", _vp), ("reduced_w", _vp), ("fp_weight", _vp), ("bias", _vp), ("tiled_weight", _vp)]
 
 

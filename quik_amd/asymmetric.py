@@ -103,21 +103,22 @@ def colmap_streams(colmap: torch.Tensor, num_int: int, num_fp: int) -> bool:
     return rc == 1
 
 
-def quantize_mapped_fp6(src: torch.Tensor, colmap: torch.Tensor, num_int: int, num_fp: int):
+def quantize_mapped_fp6(src: torch.Tensor, colmap: torch.Tensor, num_int: int, num_fp: int, four_bit: bool = False):
     """quantize_mapped with bits = 4 whose codes and outlier values go to an operand buffer for
-    matmul.mixed_linear_fp6 (internal format, see include/quik_hip.h).  Returns (x6 uint8 buffer, meta)."""
+    matmul.mixed_linear_fp6 (internal format, see include/quik_hip.h), or with four_bit to one of the 4-bit format for
+    matmul.mixed_linear_tile4.  Returns (x6 uint8 buffer, meta)."""
     rows, cols = check_mapped_args("quantize", src, colmap, num_int, num_fp, need_streaming=True)
     dt = L.dtype_id(src, "quantize", allow_bf16=True)
     lib = L.load()
-    nbytes = lib.quik_fp6_operand_bytes(max(rows, 1), num_int, num_fp)
+    nbytes = (lib.quik_tile4_operand_bytes if four_bit else lib.quik_fp6_operand_bytes)(max(rows, 1), num_int, num_fp)
     if nbytes == 0:
         raise RuntimeError("quantize: the 6-bit operand format needs a multiple of 128 integer columns and a "
                            "multiple of 32 outlier columns")
     with L.device_guard(src.device):
         x6 = torch.empty((nbytes,), dtype=torch.uint8, device=src.device)
         meta = torch.empty((2 * rows,), dtype=src.dtype, device=src.device)
-        L.check(lib.quik_asym_quantize_fp6(L.ptr(src), dt, rows, cols, L.ptr(colmap), num_int, num_fp, L.ptr(x6),
-                                           L.ptr(meta), L.stream()), "quantize")
+        quantize = lib.quik_asym_quantize_tile4 if four_bit else lib.quik_asym_quantize_fp6
+        L.check(quantize(L.ptr(src), dt, rows, cols, L.ptr(colmap), num_int, num_fp, L.ptr(x6), L.ptr(meta), L.stream()), "quantize")
     return x6, meta
 
 

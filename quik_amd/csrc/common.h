@@ -53,8 +53,9 @@ int gemv_forward_one_launch(const void *x, int dtype, int64_t rows, int64_t cols
 constexpr int64_t kLayerK4 = 32, kLayerK8 = 16;
 int64_t fp6_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple);
 int64_t tile8_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple);
+int64_t tile4_operand_bytes(int64_t rows, int64_t K, int64_t F);
 int asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
-                      int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple);
+                      int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple, bool four = false);
 int asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
                         int64_t num_fp, void *out8, void *meta, void *stream, int64_t k_multiple);
 int sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp,
@@ -63,6 +64,10 @@ int sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *c
 int mixed_linear_fp6(const void *x6, const void *w6, const void *meta, const void *s_col, const void *w_reduced,
                      const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
                      void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);
+// 4-bit weights: the format (4 or 6 bits) in which the GEMM of this shape takes its activation, and the GEMM (either format)
+int tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F);
+int mixed_linear_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col, const void *w_reduced,
+                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out, void *stream);
 int mixed_linear_tile8(const void *x8, const void *w8, const void *meta, const void *s_col, const void *w_reduced,
                        const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
                        void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);

@@ -12,6 +12,8 @@ constexpr int kThreads = 256;
 // patterns) -> operand buffer; one workgroup per row, one lane per fragment / 16-byte outlier chunk.
 // Position k of the operand takes weight column kperm[k] (the in-place order of the column map, which the
 // quantize kernel writes the activation in); the row is staged in LDS and gathered nibble by nibble.
+// FOUR: the 4-bit format, else the 6-bit one.
+template <bool FOUR>
 __global__ __launch_bounds__(kThreads) void pack_weight_kernel(const uint8_t *__restrict__ qw,
                                                                const uint16_t *__restrict__ fp_w,
                                                                const uint16_t *__restrict__ kperm,
@@ -19,12 +21,32 @@ __global__ __launch_bounds__(kThreads) void pack_weight_kernel(const uint8_t *__
                                                                int64_t K, int64_t F, uint8_t *__restrict__ out) {
   extern __shared__ __align__(16) uint8_t row_s[];  // K / 2 bytes
   if (!(flags[0] & 2u)) return;  // the column map has no in-place order (the host refuses such a map first)
-  const Fp6Layout l = fp6_layout(rows, K, F);
+  const auto layout = [&] {
+    if constexpr (FOUR) {
+      return tile4_layout(rows, K, F);
+    } else {
+      return fp6_layout(rows, K, F);
+    }
+  };
+  const auto l = layout();
   const int64_t frags_per_row = l.steps * 2;
   const int64_t row = blockIdx.x;
+  auto store_fragment = [&](int64_t f, const uint32_t (&o)[6]) {
+    if constexpr (FOUR) {
+      *reinterpret_cast<uint4 *>(out + tile4_offset(l, row, f >> 1, static_cast<int>(f & 1))) = nib_squeeze(o);
+    } else {
+      fp6_store_fragment(out, l, row, f, o);
+    }
+  };
+  auto outlier_offset = [&](int64_t c) {
+    if constexpr (FOUR) {
+      return tile4_offset(l, row, l.steps + (c >> 1), static_cast<int>(c & 1));
+    } else {
+      return fp6_outlier_offset(l, row, c >> 1, static_cast<int>(c & 1));
+    }
+  };
   for (int64_t c = threadIdx.x; c < F / 8; c += kThreads)
-    *reinterpret_cast<uint4 *>(out + fp6_outlier_offset(l, row, c >> 1, static_cast<int>(c & 1))) =
-        *reinterpret_cast<const uint4 *>(fp_w + row * F + c * 8);
+    *reinterpret_cast<uint4 *>(out + outlier_offset(c)) = *reinterpret_cast<const uint4 *>(fp_w + row * F + c * 8);
   for (int64_t c = threadIdx.x; c < K / 32; c += kThreads)
     reinterpret_cast<uint4 *>(row_s)[c] = *reinterpret_cast<const uint4 *>(qw + row * (K / 2) + c * 16);
   __shared__ int total;
@@ -34,7 +56,7 @@ __global__ __launch_bounds__(kThreads) void pack_weight_kernel(const uint8_t *__
   for (int64_t f = threadIdx.x; f < frags_per_row; f += kThreads) {
     if (f >= K / 32) {  // positions past the integer columns: levels of 0
       const uint32_t zero[6] = {};
-      fp6_store_fragment(out, l, row, f, zero);
+      store_fragment(f, zero);
       continue;
     }
     uint32_t b[8];
@@ -53,7 +75,7 @@ __global__ __launch_bounds__(kThreads) void pack_weight_kernel(const uint8_t *__
     }
     uint32_t o[6];
     fp6_pack_fragment(b, o);
-    fp6_store_fragment(out, l, row, f, o);
+    store_fragment(f, o);
   }
   atomicAdd(&total, sum);
   __syncthreads();
@@ -90,7 +112,7 @@ int tile8_pack_weight(const int8_t *qw, const void *fp_w, int64_t N, int64_t K, 
 }
 
 int fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F, const void *colmap, void *out,
-                    void *stream, int64_t k_multiple) {
+                    void *stream, int64_t k_multiple, bool four = false) {
   if (N <= 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
   if (K % k_multiple != 0 || F % 32 != 0) return QUIK_ERR_ALIGN;
   if (!qw || !out || !colmap || (F > 0 && !fp_w)) return QUIK_ERR_NULL;
@@ -101,7 +123,7 @@ int fp6_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, i
   if (int rc = colmap_require(colmap, K + F, K, F, as_stream(stream), kColmapStreams | kColmapInPlace)) return rc;
   const ColmapLayout cl = colmap_layout(K + F, K, F);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
-  hipLaunchKernelGGL(pack_weight_kernel, dim3(static_cast<unsigned>(N)), dim3(kThreads), static_cast<size_t>(K / 2),
+  hipLaunchKernelGGL(four ? pack_weight_kernel<true> : pack_weight_kernel<false>, dim3(static_cast<unsigned>(N)), dim3(kThreads), static_cast<size_t>(K / 2),
                      as_stream(stream), qw, static_cast<const uint16_t *>(fp_w),
                      reinterpret_cast<const uint16_t *>(cm + cl.off_kperm),
                      reinterpret_cast<const uint32_t *>(cm + cl.off_flags), N, K, F, static_cast<uint8_t *>(out));
@@ -119,9 +141,20 @@ int64_t fp6_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multiple
   if (rows <= 0 || K <= 0 || K % k_multiple != 0 || K > 74496 || F < 0 || F % 32 != 0) return 0;
   return fp6_layout(rows, K, F).bytes;
 }
+int64_t tile4_operand_bytes(int64_t rows, int64_t K, int64_t F) {
+  if (rows <= 0 || K <= 0 || K % kLayerK4 != 0 || K > 74496 || F < 0 || F % 32 != 0) return 0;
+  return tile4_layout(rows, K, F).bytes;
+}
 }  // namespace quik
 
 using namespace quik;
+
+extern "C" int64_t quik_tile4_operand_bytes(int64_t rows, int64_t K, int64_t F) { return tile4_operand_bytes(rows, K, F); }
+
+extern "C" int quik_tile4_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64_t K, int64_t F,
+                                      const void *colmap, void *out, void *stream) {
+  return fp6_pack_weight(qw, fp_w, N, K, F, colmap, out, stream, kLayerK4, true);
+}
 
 extern "C" int64_t quik_tile8_operand_bytes(int64_t rows, int64_t K, int64_t F) { return tile8_operand_bytes(rows, K, F, 64); }
 

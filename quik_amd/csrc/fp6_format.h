@@ -79,6 +79,39 @@ __host__ __device__ inline int64_t tile8_offset(const Tile8Layout &l, int64_t ro
          ((h ^ ((row >> 3) & 1)) << 4);
 }
 
+// ---- 4-bit operands of the same order (consumers: gemm_tile8.h, gemm_direct.h with kNib), the layer's own int4 format.
+//
+// A 6-bit field of the MFMA operand holds a level 0 .. 15, so two of its six bits are zero and the 6-bit buffers above
+// carry a third of zeros.  Here 16 levels are two dwords instead of three: P0 is the first dword of the 6-bit fragment,
+// whose ten zero bits take the upper two bits of every field of the third; P1 is the second dword, whose ten zero bits
+// take the lower two.  The fields of the third dword end up in the very bit positions they come from, so the three
+// dwords are four VALU instructions away (nib_expand).  Unit (block B, step s) is 2 KB as in Tile8Layout: 64 elements,
+// 32 bytes per row, 16-byte chunk h holds fragment h (32 elements: P0, P1 of elements 0 .. 15, then of 16 .. 31).
+// Outlier units and the level sums behind the blocks as in the 6-bit format.
+struct Tile4Layout {
+  int64_t blocks, steps, fsteps, block_bytes, sums_off, bytes;
+};
+__host__ __device__ inline Tile4Layout tile4_layout(int64_t rows, int64_t K, int64_t F) {
+  Tile4Layout l;
+  l.blocks = (rows + 63) / 64;
+  l.steps = (K + 127) / 128 * 2;
+  l.fsteps = F / 16;
+  l.block_bytes = (l.steps + l.fsteps) * 2048;
+  l.sums_off = l.blocks * l.block_bytes;
+  l.bytes = l.sums_off + rows * 4;
+  return l;
+}
+// 16-byte chunk h of step `step` (integer steps first, then outlier steps) of row `row`
+__host__ __device__ inline int64_t tile4_offset(const Tile4Layout &l, int64_t row, int64_t step, int h) {
+  return (row >> 6) * l.block_bytes + step * 2048 + ((row >> 5) & 1) * 1024 + (row & 31) * 32 +
+         ((h ^ ((row >> 3) & 1)) << 4);
+}
+constexpr uint32_t kNibUpper = 0x30C30C30u, kNibLower = 0x0C30C30Cu;  // zero bits of a fragment's first and second dword
+// a fragment's 6 dwords (every field at most 15) -> its 4 dwords in the 4-bit format
+__device__ __forceinline__ uint4 nib_squeeze(const uint32_t (&o)[6]) {
+  return make_uint4(o[0] | (o[2] & kNibUpper), o[1] | (o[2] & kNibLower), o[3] | (o[5] & kNibUpper), o[4] | (o[5] & kNibLower));
+}
+
 // 4 levels (at most 63 each) in the bytes of w -> 24 bits, 6 per level: two byte dot products with the
 // weights (1, 64) give b0 + 64 b1 and b2 + 64 b3, one shift-or joins them
 __device__ __forceinline__ uint32_t fp6_squeeze4(uint32_t w) {

@@ -26,34 +26,41 @@
 
 namespace quik {
 
-// SIX: 6-bit operands (Fused6Args), else int8 (Fused8Args: the same fields)
-template <bool SIX_, int MI_, int NI_, int SETS_>
+// 6-bit operands (Fused6Args), int8 or 4-bit ones (Fused8Args: the same fields)
+enum DirectKind { kDirect6, kDirect8, kDirect4 };
+template <int KIND_, int MI_, int NI_, int SETS_>
 struct DirectCfg {
-  static constexpr bool SIX = SIX_;
+  static constexpr int KIND = KIND_;
+  static constexpr bool SIX = KIND != kDirect8;  // multiplied on the 6-bit instructions: fp32 sums and their corrections
   static constexpr int MI = MI_, NI = NI_, SETS = SETS_, NF = MI + NI;
   static constexpr int WAVES = 4, kThreads = 64 * WAVES;
   static constexpr int BM = 32 * MI, BN = 32 * NI;
-  static constexpr int UNIT = SIX ? 3072 : 2048;
-  // (larger tiles, 128x64 and 64x128, were slower at every shape tried: their exchange and outlier steps take 2 us more)
-  static_assert(MI == 2 && (NI == 2 || NI == 1), "supported tiles");
-  static constexpr int kOutlierSets = 16;  // outlier steps in flight: all of them for 256 columns
-  static constexpr int RED_BYTES = WAVES * (WAVES - 1) * 4096;
-  static constexpr int PARTIAL_BYTES = WAVES * 4096;  // a workgroup's partial sums (SplitK)
+  static constexpr int UNIT = KIND == kDirect6 ? 3072 : 2048;
+  static_assert((MI == 2 || MI == 4) && (NI == 1 || NI == 2 || NI == 4), "supported tiles");
+  // 32x32 blocks that a wave owns after the exchange: OM x ON, at (OM * (w & 1), ON * (w >> 1)); tiles of 32 columns: waves 2
+  // and 3 own none
+  static constexpr int OM = MI / 2, ON = NI == 1 ? 1 : NI / 2, OWN = OM * ON;
+  static constexpr int kOutlierSets = OWN <= 2 ? 16 : 8;  // outlier steps in flight (16: all of them for 256 columns)
+  static constexpr int kEarlySets = KIND != kDirect4 ? 0 : OWN <= 2 ? 8 : 0;  // .. requested in front of the last integer steps
+  // exchange: one owned block per round, in two areas by turns
+  static constexpr int ROUND_BYTES = WAVES * (WAVES - 1) * 4096;
+  static constexpr int RED_BYTES = (OWN > 1 ? 2 : 1) * ROUND_BYTES;
+  static constexpr int PARTIAL_BYTES = WAVES * OWN * 4096;  // a workgroup's partial sums (SplitK)
   static constexpr int OUT_STRIDE = BN * 2 + 16;
   static constexpr int VEC_OFF = RED_BYTES > BM * OUT_STRIDE ? RED_BYTES : BM * OUT_STRIDE;
   static constexpr int SMEM = VEC_OFF + (4 * BN + 3 * BM) * 4;
-  // the 32x32 block (mi, ni) that wave w owns after the exchange; 64x32 tiles have two blocks, waves 2 and 3 none
-  static constexpr int own_mi(int w) { return w & 1; }
-  static constexpr int own_ni(int w) { return w >> 1; }
+  static constexpr int own_mi(int w) { return OM * (w & 1); }
+  static constexpr int own_ni(int w) { return ON * (w >> 1); }
   static constexpr bool owns(int w) { return own_ni(w) < NI; }
 };
 
-// One step's fragments of a wave.  6-bit: head in dwords 0 .. 3, tail in 4 and 5, as the MFMA takes it.  (Kept as whole
+// One step's fragments of a wave.  6-bit: head in dwords 0 .. 3, tail in 4 and 5, as the MFMA takes it; 4-bit: as in memory,
+// expanded in front of its products.  (Kept as whole
 // operand vectors: with heads and tails in arrays of their own the compiler merges neighbouring elements into one
 // wider access, cannot split the arrays into registers any more and puts them into scratch memory.)
 template <class D>
 struct DirectFrag {
-  std::conditional_t<D::SIX, v8i, v4i> f[D::NF];
+  std::conditional_t<D::KIND == kDirect6, v8i, v4i> f[D::NF];
 };
 
 template <class D, bool BF16, bool SPLITK, class Args>
@@ -64,7 +71,12 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   const int m0 = tm * D::BM, n0 = tn * D::BN;
   int64_t x_blocks, w_blocks, block_bytes, x_sums = 0, w_sums = 0;
   int steps, fsteps;
-  if constexpr (D::SIX) {
+  if constexpr (D::KIND == kDirect4) {
+    const Tile4Layout lx = tile4_layout(p.M, p.K, p.F), lw = tile4_layout(p.N_total, p.K, p.F);
+    x_blocks = lx.blocks, w_blocks = lw.blocks, block_bytes = lx.block_bytes;
+    x_sums = lx.sums_off, w_sums = lw.sums_off;
+    steps = static_cast<int>(lx.steps), fsteps = static_cast<int>(lx.fsteps);
+  } else if constexpr (D::KIND == kDirect6) {
     const Fp6Layout lx = fp6_layout(p.M, p.K, p.F), lw = fp6_layout(p.N_total, p.K, p.F);
     x_blocks = lx.blocks, w_blocks = lw.blocks, block_bytes = lx.block_bytes;
     x_sums = lx.sums_off, w_sums = lw.sums_off;
@@ -95,7 +107,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
       constexpr int j = J, jj = j < MI ? j : j - MI, b = j < MI ? j / 2 : MI / 2 + jj / 2;
       const int half = j < MI || NI > 1 ? jj & 1 : whalf;
       const v4i head = *reinterpret_cast<const v4i *>(base[b] + step * UNIT + half * 1024 + ho);
-      if constexpr (D::SIX) {
+      if constexpr (D::KIND == kDirect6) {
         const v2i tail = *reinterpret_cast<const v2i *>(base[b] + step * UNIT + half * 256 + to);
         f.f[j] = v8i{head.x, head.y, head.z, head.w, tail.x, tail.y, 0, 0};
       } else {
@@ -125,6 +137,18 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     v_rs = reinterpret_cast<const int32_t *>(p.xbuf + x_sums)[vm];
   }
 
+  // 4 bits: the wave's next step to load, as the lane's offset to the (scalar) addresses of the blocks: one addition per
+  // step.  The instructions of a step are what bounds it, not the bytes.
+  uint32_t pos = head_off + static_cast<uint32_t>(k0 + wave + SETS * WAVES) * UNIT;
+  const uint8_t *const wbase = base[MI / 2] + (NI == 1 ? whalf * 1024 : 0);
+  auto load_next = [&](auto &f) QUIK_INLINE {
+    static_for<NF>([&](auto J) QUIK_INLINE {
+      constexpr int j = J, jj = j < MI ? j : j - MI, b = j < MI ? j / 2 : MI / 2 + jj / 2;
+      f.f[j] = *reinterpret_cast<const v4i *>((j < MI || NI > 1 ? base[b] : wbase) + pos + (jj & 1) * 1024);
+    });
+    pos += WAVES * UNIT;
+  };
+
   DirectFrag<D> set[SETS];
   const int last_step = k1 > 0 ? k1 - 1 : 0;
   static_for<SETS>([&](auto S) QUIK_INLINE { load_step(set[S], at(S) < last_step ? at(S) : last_step); });
@@ -136,17 +160,90 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     for (int ni = 0; ni < NI; ++ni)
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[mi][ni][v] = 0.0f;
-  auto multiply = [&](const DirectFrag<D> &f) QUIK_INLINE {
-    static_for<MI * NI>([&](auto I) QUIK_INLINE {
-      constexpr int mi = I % MI, ni = I / MI;
-      if constexpr (D::SIX) {
-        acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.f[MI + ni], f.f[mi], acc[mi][ni], 2, 2, 0, 0, 0, 0);
-      } else {
-        FragOps<kInt8>::mma(f.f[mi], f.f[MI + ni], acc[mi][ni]);
-      }
+  // outlier steps of the blocks that this wave will own; the first ones are requested in front of the exchange, some of them in
+  // front of the last integer steps
+  constexpr int OS = D::kOutlierSets, OM = D::OM, ON = D::ON, OWN = D::OWN;
+  v4i ox[OS][OM], ow[OS][ON];
+  const int omi = D::own_mi(wave), oni = D::owns(wave) ? D::own_ni(wave) : 0;
+  const uint8_t *ox_base[OM], *ow_base[ON];
+#pragma unroll
+  for (int i = 0; i < OM; ++i) ox_base[i] = p.xbuf + block((m0 + 32 * (omi + i)) / 64, x_blocks) + ((omi + i) & 1) * 1024;
+#pragma unroll
+  for (int j = 0; j < ON; ++j) {
+    const int row = wrow + 32 * (oni + j);
+    ow_base[j] = p.wbuf + block(row / 64, w_blocks) + ((row >> 5) & 1) * 1024;
+  }
+  auto load_outlier = [&](auto S, int t) QUIK_INLINE {
+    const int64_t step = steps + t;
+    static_for<OM>([&](auto I) QUIK_INLINE { ox[S][I] = *reinterpret_cast<const v4i *>(ox_base[I] + step * UNIT + head_off); });
+    static_for<ON>([&](auto J) QUIK_INLINE { ow[S][J] = *reinterpret_cast<const v4i *>(ow_base[J] + step * UNIT + head_off); });
+  };
+  // sets [LO, HI) of a round; without outlier columns: the last integer step, not used
+  auto load_outliers = [&](auto LO, auto HI, int t0) QUIK_INLINE {
+    static_for<HI - LO>([&](auto I) QUIK_INLINE {
+      constexpr int S = LO + I;
+      load_outlier(std::integral_constant<int, S>{}, t0 + S < fsteps ? t0 + S : fsteps - 1);
     });
   };
-  {
+  using std::integral_constant;
+  constexpr integral_constant<int, 0> kNone{};
+  constexpr integral_constant<int, D::kEarlySets> kEarly{};
+  constexpr integral_constant<int, OS> kAll{};
+  if constexpr (D::KIND == kDirect4) {
+    // A step's fragments are expanded (eight VALU instructions each) while the step before is multiplied: a wave has its SIMD
+    // to itself, nothing else would run under its products.
+    v6i u[2][NF];
+    auto expand = [&](v6i (&to)[NF], const DirectFrag<D> &f) QUIK_INLINE {
+      static_for<NF>([&](auto J) QUIK_INLINE { to[J] = nib_expand(f.f[J]); });
+    };
+    auto multiply = [&](const v6i (&v)[NF]) QUIK_INLINE {
+      static_for<MI * NI>([&](auto I) QUIK_INLINE {
+        constexpr int mi = I % MI, ni = I / MI;
+        nib_mma(v[mi], v[MI + ni], acc[mi][ni]);
+      });
+    };
+    static_assert(SETS % 2 == 0, "operand sets alternate");
+    expand(u[0], set[0]);
+    // (unconditional, as every load in front of the loop: the compiler's waits in it count on them)
+    load_step(set[0], at(SETS) < last_step ? at(SETS) : last_step);
+    pos += WAVES * UNIT;
+    int it = 0;  // step `it` is in u[it & 1], steps it + 1 .. it + SETS are in the sets (it + k in set (it + k) % SETS)
+    for (; it + 2 * SETS < mine; it += SETS) {
+      static_for<SETS>([&](auto S) QUIK_INLINE {
+        constexpr int next = (S + 1) % SETS;
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1) * NF));  // (one wait for the set, not one per fragment)
+        __builtin_amdgcn_sched_barrier(0);
+        expand(u[(S + 1) & 1], set[next]);
+        multiply(u[S & 1]);
+        load_next(set[next]);
+        static_for<MI * NI>([&](auto) QUIK_INLINE {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, (8 * NF + MI * NI - 1) / (MI * NI), 0);
+        });
+        static_for<NF>([&](auto J) QUIK_INLINE { pin(u[(S + 1) & 1][J]); });
+        __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
+      });
+    }
+    if constexpr (!SPLITK) load_outliers(kNone, kEarly, 0);
+    static_for<2 * SETS>([&](auto S) QUIK_INLINE {
+      constexpr int next = (S + 1) % SETS;
+      if (it + S < mine) {
+        multiply(u[S & 1]);
+        if (it + S + 1 < mine) expand(u[(S + 1) & 1], set[next]);
+        if (it + S + 1 + SETS < mine) load_next(set[next]);
+      }
+    });
+  } else {
+    auto multiply = [&](const DirectFrag<D> &f) QUIK_INLINE {
+      static_for<MI * NI>([&](auto I) QUIK_INLINE {
+        constexpr int mi = I % MI, ni = I / MI;
+        if constexpr (D::KIND == kDirect6) {
+          acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.f[MI + ni], f.f[mi], acc[mi][ni], 2, 2, 0, 0, 0, 0);
+        } else {
+          FragOps<kInt8>::mma(f.f[mi], f.f[MI + ni], acc[mi][ni]);
+        }
+      });
+    };
     int it = 0;
     for (; it + 2 * SETS <= mine; it += SETS) {
       static_for<SETS>([&](auto S) QUIK_INLINE {
@@ -155,6 +252,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
       });
     }
+    if constexpr (!SPLITK) load_outliers(kNone, kEarly, 0);
     static_for<SETS>([&](auto S) QUIK_INLINE {
       if (it + S < mine) multiply(set[S]);
       if (it + SETS + S < mine) load_step(set[S], at(it + SETS + S));
@@ -179,66 +277,60 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     rowc[vi] = D::SIX ? static_cast<float>(8 * v_rs - 64 * p.K) : 0.0f;
   }  // (visible behind the exchange's barrier)
 
-  // the first outlier steps of the block this wave will own are requested in front of the exchange
-  constexpr int OS = D::kOutlierSets;
-  v4i ox[OS], ow[OS];
-  const int omi = D::own_mi(wave), oni = D::owns(wave) ? D::own_ni(wave) : 0;
-  const uint8_t *const ox_base = p.xbuf + block(m0 / 64, x_blocks) + omi * 1024;
-  const uint8_t *const ow_base = p.wbuf + block((wrow + 32 * oni) / 64, w_blocks) + (((wrow + 32 * oni) >> 5) & 1) * 1024;
-  auto load_outlier = [&](auto S, int t) QUIK_INLINE {
-    const int64_t step = steps + t;
-    ox[S] = *reinterpret_cast<const v4i *>(ox_base + step * UNIT + head_off);
-    ow[S] = *reinterpret_cast<const v4i *>(ow_base + step * UNIT + head_off);
-  };
-  auto load_outliers = [&](int t0) QUIK_INLINE {
-    static_for<OS>([&](auto S) QUIK_INLINE { load_outlier(S, t0 + S < fsteps ? t0 + S : fsteps - 1); });
-  };
-  if (!SPLITK && fsteps > 0) load_outliers(0);
+  if constexpr (!SPLITK) load_outliers(kEarly, kAll, 0);
 
-  // exchange: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the three it finds
-  v16f own = {};
+  // exchange, owned block by owned block: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the
+  // three it finds
+  v16f own[OWN];
   auto add = [](float a, int b) QUIK_INLINE {
     return D::SIX ? a + __int_as_float(b) : __int_as_float(__float_as_int(a) + b);
   };
-  static_for<WAVES>([&](auto O) QUIK_INLINE {
-    constexpr int o = O;
-    if constexpr (D::owns(o)) {
-      const v16f &b = acc[D::own_mi(o)][D::own_ni(o)];
-      if (o == wave) {
-        own = b;
-      } else {
-        uint8_t *slot = smem + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
+  static_for<OWN>([&](auto B) QUIK_INLINE {
+    constexpr int bm = B % OM, bn = B / OM;
+    uint8_t *const area = smem + (B & 1) * D::ROUND_BYTES;
+    own[B] = v16f{};
+    static_for<WAVES>([&](auto O) QUIK_INLINE {
+      constexpr int o = O;
+      if constexpr (D::owns(o)) {
+        const v16f &b = acc[D::own_mi(o) + bm][D::own_ni(o) + bn];
+        if (o == wave) {
+          own[B] = b;
+        } else {
+          uint8_t *slot = area + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
-          *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
+          for (int g = 0; g < 4; ++g)
+            *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
+        }
+      }
+    });
+    __syncthreads();  // (an area is written again two rounds later: behind a barrier that its readers have passed)
+    if (D::owns(wave)) {
+#pragma unroll
+      for (int s = 0; s < WAVES - 1; ++s) {
+        const uint8_t *slot = area + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
+#pragma unroll
+        for (int g = 0; g < 4; ++g) {
+          const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
+#pragma unroll
+          for (int e = 0; e < 4; ++e) own[B][4 * g + e] = add(own[B][4 * g + e], t[e]);
+        }
       }
     }
   });
-  __syncthreads();
-  if (D::owns(wave)) {
-#pragma unroll
-    for (int s = 0; s < WAVES - 1; ++s) {
-      const uint8_t *slot = smem + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
-#pragma unroll
-      for (int g = 0; g < 4; ++g) {
-        const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) own[4 * g + e] = add(own[4 * g + e], t[e]);
-      }
-    }
-  }
 
   if constexpr (SPLITK) {
     // the same between the workgroups of a tile, through memory (see splitk_combine in gemm_fp6.h): partial sums
-    // [tile][split][wave][group of 4][lane][4]
+    // [tile][split][owned block][wave][group of 4][lane][4]
     constexpr int kPer = D::PARTIAL_BYTES / 4;
     int32_t *part = sk->partials + int64_t(tile_id) * sk->splits * kPer + wave * 1024 + lane * 4;
     if (D::owns(wave)) {
+      static_for<OWN>([&](auto B) QUIK_INLINE {
 #pragma unroll
-      for (int g = 0; g < 4; ++g)
-        splitk_store4(part + int64_t(split) * kPer + g * 256,
-                      v4i{__float_as_int(own[4 * g]), __float_as_int(own[4 * g + 1]), __float_as_int(own[4 * g + 2]),
-                          __float_as_int(own[4 * g + 3])});
+        for (int g = 0; g < 4; ++g)
+          splitk_store4(part + int64_t(split) * kPer + B * (WAVES * 1024) + g * 256,
+                        v4i{__float_as_int(own[B][4 * g]), __float_as_int(own[B][4 * g + 1]), __float_as_int(own[B][4 * g + 2]),
+                            __float_as_int(own[B][4 * g + 3])});
+      });
     }
     splitk_stores_done();
     __syncthreads();
@@ -249,53 +341,62 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     }
     __syncthreads();
     if (*last_s == 0) return;
-    if (fsteps > 0) load_outliers(0);
+    load_outliers(kNone, kAll, 0);
     if (D::owns(wave)) {
       for (int o = 0; o < sk->splits; ++o) {
         if (o == split) continue;
-        v4i t[4];
-        splitk_load4<256>(part + int64_t(o) * kPer, t);
+        static_for<OWN>([&](auto B) QUIK_INLINE {
+          v4i t[4];
+          splitk_load4<256>(part + int64_t(o) * kPer + B * (WAVES * 1024), t);
 #pragma unroll
-        for (int g = 0; g < 4; ++g)
+          for (int g = 0; g < 4; ++g)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) own[4 * g + e] = add(own[4 * g + e], t[g][e]);
+            for (int e = 0; e < 4; ++e) own[B][4 * g + e] = add(own[B][4 * g + e], t[g][e]);
+        });
       }
     }
     if (threadIdx.x == 0) __hip_atomic_store(sk->counters + tile_id, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 
-  // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned block
+  // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned blocks
   if (D::owns(wave)) {
-    const float rs = srow[32 * omi + r], rz = zs[32 * omi + r], rc = rowc[32 * omi + r];
+    static_for<OWN>([&](auto B) QUIK_INLINE {
+      constexpr int bm = B % OM, bn = B / OM;
+      const float rs = srow[32 * (omi + bm) + r], rz = zs[32 * (omi + bm) + r], rc = rowc[32 * (omi + bm) + r];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int c = oni * 32 + acc_col(g, lane);
-      const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
-                   bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
-      const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
-                  ccv[4] = {cc.x, cc.y, cc.z, cc.w};
+      for (int g = 0; g < 4; ++g) {
+        const int c = (oni + bn) * 32 + acc_col(g, lane);
+        const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
+                     bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
+        const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
+                    ccv[4] = {cc.x, cc.y, cc.z, cc.w};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const float raw = own[4 * g + e];
-        const float iacc = D::SIX ? __builtin_fmaf(raw + ccv[e], 64.0f, -rc)  // exact: integers below 2^24
-                                  : static_cast<float>(__float_as_int(raw));
-        own[4 * g + e] = __builtin_fmaf(iacc, rs * scv[e], __builtin_fmaf(rz, wrv[e], bsv[e]));
+        for (int e = 0; e < 4; ++e) {
+          const float raw = own[B][4 * g + e];
+          const float iacc = D::SIX ? __builtin_fmaf(raw + ccv[e], 64.0f, -rc)  // exact: integers below 2^24
+                                    : static_cast<float>(__float_as_int(raw));
+          own[B][4 * g + e] = __builtin_fmaf(iacc, rs * scv[e], __builtin_fmaf(rz, wrv[e], bsv[e]));
+        }
       }
-    }
+    });
     for (int t0 = 0; t0 < fsteps; t0 += OS) {
       const bool more = t0 + OS < fsteps;
       static_for<OS>([&](auto S) QUIK_INLINE {
-        if (t0 + S < fsteps) FragOps<BF16 ? kBF16 : kF16>::mma(ox[S], ow[S], own);
+        if (t0 + S < fsteps)
+          static_for<OWN>([&](auto B) QUIK_INLINE { FragOps<BF16 ? kBF16 : kF16>::mma(ox[S][B % OM], ow[S][B / OM], own[B]); });
         if (more) load_outlier(S, t0 + OS + S < fsteps ? t0 + OS + S : fsteps - 1);
       });
     }
   }
   __syncthreads();  // every wave has read its slots: the area becomes the output tile
   if (D::owns(wave)) {
+    static_for<OWN>([&](auto B) QUIK_INLINE {
+      constexpr int bm = B % OM, bn = B / OM;
 #pragma unroll
-    for (int g = 0; g < 4; ++g)
-      *reinterpret_cast<uint2 *>(smem + (32 * omi + r) * D::OUT_STRIDE + (oni * 32 + acc_col(g, lane)) * 2) =
-          make_uint2(pack2_from_f32<BF16>(own[4 * g], own[4 * g + 1]), pack2_from_f32<BF16>(own[4 * g + 2], own[4 * g + 3]));
+      for (int g = 0; g < 4; ++g)
+        *reinterpret_cast<uint2 *>(smem + (32 * (omi + bm) + r) * D::OUT_STRIDE + ((oni + bn) * 32 + acc_col(g, lane)) * 2) =
+            make_uint2(pack2_from_f32<BF16>(own[B][4 * g], own[B][4 * g + 1]), pack2_from_f32<BF16>(own[B][4 * g + 2], own[B][4 * g + 3]));
+    });
   }
   __syncthreads();
   const bool vec = (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
@@ -332,14 +433,14 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
 }
 
 template <class D, bool BF16, class Args>
-__global__ __launch_bounds__(D::kThreads, 2) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__(D::kThreads, D::OWN == 1 ? 2 : 1) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_of_block<D::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   direct_tile<D, BF16, false>(p, tm, tn, smem, 0, 0, nullptr);
 }
 template <class D, bool BF16, class Args>
-__global__ __launch_bounds__(D::kThreads, 2) void gemm_direct_splitk_kernel(Args p, int tiles_m, int tiles_n, SplitK sk) {
+__global__ __launch_bounds__(D::kThreads, D::OWN == 1 ? 2 : 1) void gemm_direct_splitk_kernel(Args p, int tiles_m, int tiles_n, SplitK sk) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int split = blockIdx.x / sk.grid_tiles;

@@ -43,6 +43,14 @@ __device__ __forceinline__ void dma_load16k(const uint8_t *sbase, uint32_t voff,
                : : "s"(lds_addr), "v"(voff), "s"(sbase), "n"(OFFSET) : "memory", "m0");
 }
 
+// The same for all lanes or none (`lanes`: all bits set or none): a copy that only some waves make, in a stream whose outstanding copies all
+// waves count alike (with no lane active the copy moves nothing and is counted as any other).  exec holds all lanes outside.
+template <int OFFSET>
+__device__ __forceinline__ void dma_load16k_if(uint32_t lanes, const uint8_t *sbase, uint32_t voff, uint32_t lds_addr) {
+  asm volatile("s_mov_b32 m0, %0\n\ts_mov_b32 exec_lo, %4\n\ts_mov_b32 exec_hi, %4\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %1, %2 offset:%3\n\ts_mov_b64 exec, -1"
+               : : "s"(lds_addr), "v"(voff), "s"(sbase), "n"(OFFSET), "s"(lanes) : "memory", "m0", "exec");
+}
+
 // LDS slots of the tile-ordered rings, `stage` bytes each: six, or with one workgroup per CU (DMA_STAGES > 4) as many as
 // fit 144 KB, an even number, at most twelve.
 template <class C>
@@ -51,10 +59,28 @@ constexpr int ring_slots(int stage) {
   return C::DMA_STAGES <= 4 ? 6 : most < 12 ? most : 12;
 }
 
-template <class C>
+// a fragment of the 4-bit format -> its 6 operand dwords (fp6_format.h)
+typedef int v6i __attribute__((ext_vector_type(6)));
+__device__ __forceinline__ v6i nib_expand(const v4i q) {
+  constexpr int kU = static_cast<int>(kNibUpper), kL = static_cast<int>(kNibLower);
+  return v6i{q.x & ~kU, q.y & ~kL, (q.x & kU) | (q.y & kL), q.z & ~kU, q.w & ~kL, (q.z & kU) | (q.w & kL)};
+}
+// acc += w_frag x x_frag, 64 levels (block scales 0, 0: the unscaled instruction, see gemm_fp6.h)
+__device__ __forceinline__ void nib_mma(const v6i &x, const v6i &w, v16f &acc) {
+  const v8i w8 = {w[0], w[1], w[2], w[3], w[4], w[5], 0, 0}, x8 = {x[0], x[1], x[2], x[3], x[4], x[5], 0, 0};
+  acc = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(w8, x8, acc, 2, 2, 0, 0, 0, 0);
+}
+// the value is there at this point (empty statement: no hazard): a fragment is expanded where the source says, not later, in
+// front of the products that read it, where nothing covers it
+__device__ __forceinline__ void pin(v6i &x) { asm volatile("" : "+v"(x)); }
+
+// W4: the weights are in the 4-bit format
+template <class C, bool W4 = false>
 struct Fp6Pipe {
   static constexpr int MI = C::MI, NI = C::NI, NF = MI + NI;
-  static constexpr int NS = ring_slots<C>((C::BM + C::BN) * 48);  // LDS slots; one step is multiplied, NS - 1 are landed or in flight
+  static constexpr int NT = W4 ? MI : NF;  // fragments that have a tail
+  static constexpr int WU = W4 ? 2048 : 3072;  // bytes of a weight unit
+  static constexpr int NS = ring_slots<C>(C::BM * 48 + C::BN * (WU / 64));  // LDS slots; one step is multiplied, NS - 1 are landed or in flight
   // a wave's fragments start at a 64-row block of the operand, or the wave has a single 32-row fragment (then it may
   // be the second half of a block)
   static_assert(C::WM % 64 == 0 || C::MI == 1, "a wave's token rows");
@@ -62,16 +88,17 @@ struct Fp6Pipe {
   static_assert(C::WAVES == 4 || C::WAVES == 8, "copy assignment below");
   // LDS slot of one step: the 3 KB units of the tile's X blocks, then of its W blocks, as they are in memory
   static constexpr int W_OFF = C::BM * 48;
-  static constexpr int STAGE = (C::BM + C::BN) * 48;
+  static constexpr int STAGE = C::BM * 48 + C::BN * (WU / 64);
   static constexpr int SMEM = NS * STAGE;
-  // Copies per step: 3 per 64-row block (head image of rows 0..31, of rows 32..63, tail image), XB + WB blocks.
+  // Copies per step: 3 per 64-row block, 2 per weight block in the 4-bit format (head image of rows 0..31, of rows 32..63, tail image), XB + WB blocks.
   // Every wave copies one whole block from its source A (X block w, or W block w - XB when the tile has
   // fewer than 4 X blocks), and NB further kilobytes from its source B:
   //   256x256: W block w (3);  256x128: W block w % 2, pieces w / 2 and w / 2 + 1 (piece 1 is copied twice);
   //   128x128: none;  128x64: none (two waves copy the one W block: the same bytes to the same place).
+  // (W4: a wave whose source A is a W block makes its third copy with no lane; 256x128: one further kilobyte, none twice)
   static constexpr int XB = C::BM / 64, WB = C::BN / 64;
   // (eight waves, 256x256: one block per wave, no source B)
-  static constexpr int NB = C::WAVES == 8 ? 0 : XB + WB == 8 ? 3 : XB + WB == 6 ? 2 : 0;
+  static constexpr int NB = C::WAVES == 8 ? 0 : XB + WB == 8 ? WU / 1024 : XB + WB == 6 ? (W4 ? 1 : 2) : 0;
   static_assert((XB == 4 && (WB == 4 || WB == 2)) || (XB == 2 && (WB == 2 || WB == 1)), "supported tile shapes");
   static_assert(C::WAVES == 4 || XB + WB == 8, "eight waves copy eight blocks");
   static constexpr int P = 3 + NB;  // copies per wave and step
@@ -81,23 +108,26 @@ struct Fp6Pipe {
   uint32_t lds0;
   const uint8_t *pa, *pb;   // wave-uniform: sources of the next step to be copied
   uint32_t da, db;          // wave-uniform: destinations inside a slot
+  int adv_a;                // W4: bytes of source A's units
+  uint32_t third;           // W4: lanes of source A's third copy: none where it is a W block
   uint32_t fill;            // wave-uniform: LDS address of the slot the next copy fills
   int left;                 // steps whose copy has not been issued yet
   uint32_t lane16;
   uint32_t rd;              // byte offset of the slot the next fragment read looks at
   int steps0, steps;        // integer steps, all steps
   uint32_t x_head, w_head;  // this lane's head offsets inside a slot (fragment j: + 1024 j)
-  uint32_t x_head3[NS / 2], w_head3[NS / 2], tail3[NS / 2][NF];  // the same inside slots 0, 2, 4, .. (for steps whose slot is
+  uint32_t x_head3[NS / 2], w_head3[NS / 2], tail3[NS / 2][NT];  // the same inside slots 0, 2, 4, .. (for steps whose slot is
                                                   // known at compile time: the odd slot is an immediate offset away)
-  uint32_t tail[NF];        // this lane's tail offsets inside a slot, one register per fragment: reads that share
+  uint32_t tail[NT];        // this lane's tail offsets inside a slot, one register per fragment: reads that share
                             // a base register are paired into one 4-register read by the compiler, and the halves
                             // then have to be copied into the operand tuples behind an exposed LDS round trip
 
   // xb0 / wb0: first 64-row block of the tile in each operand buffer
   // unit0: first unit (step) of every block to copy; n_int / n_f: integer and outlier steps from there on
   // (-1: all of the block's, from its first unit)
+  template <class LayoutW>
   __device__ __forceinline__ void init(uint8_t *smem_, const uint8_t *xbuf, const Fp6Layout &lx, int64_t xb0,
-                                       const uint8_t *wbuf, const Fp6Layout &lw, int64_t wb0, int unit0 = 0,
+                                       const uint8_t *wbuf, const LayoutW &lw, int64_t wb0, int unit0 = 0,
                                        int n_int = -1, int n_f = -1) {
     smem = smem_;
     lds0 = lds_address(smem_);
@@ -105,22 +135,27 @@ struct Fp6Pipe {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
     auto block_ptr = [&](bool is_x, int blk) {
-      const Fp6Layout &l = is_x ? lx : lw;
+      const int64_t blocks = is_x ? lx.blocks : lw.blocks, bytes = is_x ? lx.block_bytes : lw.block_bytes;
       int64_t B = (is_x ? xb0 : wb0) + blk;
-      B = B < l.blocks ? B : l.blocks - 1;  // blocks past the matrix: any valid block, results never stored
-      return (is_x ? xbuf : wbuf) + B * l.block_bytes + int64_t(unit0) * 3072;
+      B = B < blocks ? B : blocks - 1;  // blocks past the matrix: any valid block, results never stored
+      return (is_x ? xbuf : wbuf) + B * bytes + int64_t(unit0) * (is_x ? 3072 : WU);
     };
     {
       const bool is_x = wave < XB;
       const int blk = is_x ? wave : (wave - XB) % WB;
       pa = block_ptr(is_x, blk);
-      da = (is_x ? 0 : W_OFF) + blk * 3072;
+      da = is_x ? blk * 3072 : W_OFF + blk * WU;
+      adv_a = is_x ? 3072 : WU;
+      third = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(is_x ? -1 : 0));
     }
     pb = pa;
     db = da;
-    if constexpr (NB == 3) {
+    if constexpr (XB + WB == 8 && C::WAVES == 4) {
       pb = block_ptr(false, wave);
-      db = W_OFF + wave * 3072;
+      db = W_OFF + wave * WU;
+    } else if constexpr (W4 && NB == 1) {
+      pb = block_ptr(false, wave & 1) + (wave >> 1) * 1024;
+      db = W_OFF + (wave & 1) * WU + (wave >> 1) * 1024;
     } else if constexpr (NB == 2) {
       pb = block_ptr(false, wave & 1) + (wave >> 1) * 1024;
       db = W_OFF + (wave & 1) * 3072 + (wave >> 1) * 1024;
@@ -137,9 +172,9 @@ struct Fp6Pipe {
     // a single fragment)
     const int fx0 = wm * C::WM / 32, fw0 = wn * C::WN / 32;
     x_head = (fx0 >> 1) * 3072 + (fx0 & 1) * 1024 + r * 32 + slot16;
-    w_head = W_OFF + (fw0 >> 1) * 3072 + (fw0 & 1) * 1024 + r * 32 + slot16;
+    w_head = W_OFF + (fw0 >> 1) * WU + (fw0 & 1) * 1024 + r * 32 + slot16;
 #pragma unroll
-    for (int j = 0; j < NF; ++j) {
+    for (int j = 0; j < NT; ++j) {
       const int jj = j < MI ? j : j - MI;
       const int f0 = j < MI ? fx0 : fw0;
       tail[j] = (j < MI ? 0 : W_OFF) + (f0 >> 1) * 3072 + (jj >> 1) * 3072 + 2048 + h * 512 +
@@ -151,7 +186,7 @@ struct Fp6Pipe {
       x_head3[q] = x_head + q * 2 * STAGE;
       w_head3[q] = w_head + q * 2 * STAGE;
 #pragma unroll
-      for (int j = 0; j < NF; ++j) {
+      for (int j = 0; j < NT; ++j) {
         tail3[q][j] = tail[j] + q * 2 * STAGE;
         asm volatile("" : "+v"(tail3[q][j]));
       }
@@ -166,15 +201,19 @@ struct Fp6Pipe {
   __device__ __forceinline__ void issue_one() {
     const uint32_t slot = FS < 0 ? fill : lds0 + (FS < 0 ? 0 : FS) * STAGE;
     if constexpr (G < 3) {
-      dma_load16k<G * 1024>(pa, lane16, slot + da);
+      if constexpr (W4 && G == 2 && !(XB == 4 && C::WAVES == 4)) {  // (some waves' source A is a W block)
+        dma_load16k_if<2048>(third, pa, lane16, slot + da);
+      } else {
+        dma_load16k<G * 1024>(pa, lane16, slot + da);
+      }
     } else {
       dma_load16k<(G - 3) * 1024>(pb, lane16, slot + db);
     }
     if constexpr (G == P - 1) {
-      const int adv = left > 1 ? 3072 : 0;
+      const bool more = left > 1;
       left -= 1;
-      pa += adv;
-      pb += adv;
+      pa += more ? (W4 ? adv_a : 3072) : 0;
+      pb += more ? WU : 0;
       if constexpr (FS < 0) {
         fill += STAGE;
         fill = fill == lds0 + NS * STAGE ? lds0 : fill;
@@ -213,7 +252,14 @@ struct Fp6Pipe {
   template <int J, int RS = -1>
   __device__ __forceinline__ void read6_one(v4i (&fh)[NF], v2i (&ft)[NF]) const {
     constexpr int jj = J < MI ? J : J - MI;
-    if constexpr (RS < 0) {
+    if constexpr (J >= NT) {  // 4-bit format: no tail
+      if constexpr (RS < 0) {
+        fh[J] = *reinterpret_cast<const v4i *>(smem + rd + w_head + (jj >> 1) * WU + (jj & 1) * 1024);
+      } else {
+        constexpr int q = (RS < 0 ? 0 : RS) / 2, odd = ((RS < 0 ? 0 : RS) % 2) * STAGE;
+        fh[J] = *reinterpret_cast<const v4i *>(smem + w_head3[q] + odd + (jj >> 1) * WU + (jj & 1) * 1024);
+      }
+    } else if constexpr (RS < 0) {
       const uint8_t *s = smem + rd;
       fh[J] = *reinterpret_cast<const v4i *>(s + (J < MI ? x_head : w_head) + (jj >> 1) * 3072 + (jj & 1) * 1024);
       ft[J] = *reinterpret_cast<const v2i *>(s + tail[J]);
@@ -227,7 +273,7 @@ struct Fp6Pipe {
   template <int J>
   __device__ __forceinline__ void read16_one(v4i (&f)[NF]) const {
     constexpr int jj = J < MI ? J : J - MI;
-    f[J] = *reinterpret_cast<const v4i *>(smem + rd + (J < MI ? x_head : w_head) + (jj >> 1) * 3072 + (jj & 1) * 1024);
+    f[J] = *reinterpret_cast<const v4i *>(smem + rd + (J < MI ? x_head : w_head) + (jj >> 1) * (J < MI ? 3072 : WU) + (jj & 1) * 1024);
   }
   template <int J = 0>
   __device__ __forceinline__ void read6(v4i (&fh)[NF], v2i (&ft)[NF]) {
@@ -303,6 +349,80 @@ struct Fp6Pipe {
       __builtin_amdgcn_s_barrier();
     }
   }
+  // W4: the same step.  The weight fragments are read first, as they are in memory, and expanded behind the reads of the
+  // activation's, in the last chunks of the step, in front of the one that multiplies them.
+  template <int LO, int HI>
+  static __device__ __forceinline__ void chunk_expand(const v4i (&h)[NF], v6i (&w)[NI]) {
+    if constexpr (LO < HI) {
+      w[LO] = nib_expand(h[MI + LO]);
+      chunk_expand<LO + 1, HI>(h, w);
+    }
+  }
+  template <int LO, int HI>
+  static __device__ __forceinline__ void chunk_mfmas64(const v4i (&ch)[NF], const v2i (&ct)[NF], const v6i (&cw)[NI], v16f (&acc)[MI][NI]) {
+    if constexpr (LO < HI) {
+      constexpr int mi = LO % MI, ni = LO / MI;
+      nib_mma(v6i{ch[mi].x, ch[mi].y, ch[mi].z, ch[mi].w, ct[mi].x, ct[mi].y}, cw[ni], acc[mi][ni]);
+      chunk_mfmas64<LO + 1, HI>(ch, ct, cw, acc);
+    }
+  }
+  template <int RS, int LO, int HI>  // in the order W, X
+  __device__ __forceinline__ void chunk_reads64(v4i (&nh)[NF], v2i (&nt)[NF]) const {
+    if constexpr (LO < HI) {
+      read6_one<(LO < NI ? MI + LO : LO - NI), RS>(nh, nt);
+      chunk_reads64<RS, LO + 1, HI>(nh, nt);
+    }
+  }
+  template <int RS = -1, int FS = -1, int G = 0>
+  __device__ __forceinline__ void step64(const v4i (&ch)[NF], const v2i (&ct)[NF], const v6i (&cw)[NI], v4i (&nh)[NF], v2i (&nt)[NF],
+                                         v6i (&nw)[NI], v16f (&acc)[MI][NI]) {
+    constexpr int MM = MI * NI, E0 = (P - 1) / 2 + 1;  // reads in chunks 0 .. E0 - 1, expansion in E0 .. P - 1
+    if constexpr (G < P) {
+      constexpr int m_lo = G * MM / P, m_hi = (G + 1) * MM / P;
+      constexpr int r_lo = G < E0 ? G * NF / E0 : NF, r_hi = G < E0 ? (G + 1) * NF / E0 : NF;
+      constexpr int e_lo = G < E0 ? 0 : (G - E0) * NI / (P - E0), e_hi = G < E0 ? 0 : (G - E0 + 1) * NI / (P - E0);
+      chunk_reads64<RS, r_lo, r_hi>(nh, nt);
+      chunk_expand<e_lo, e_hi>(nh, nw);
+      chunk_mfmas64<m_lo, m_hi>(ch, ct, cw, acc);
+      if constexpr (m_hi > m_lo) {
+#pragma unroll
+        for (int i = m_lo; i < m_hi; ++i) {
+          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x100, (2 * (r_hi - r_lo) + (m_hi - m_lo) - 1) / (m_hi - m_lo), 0);
+          __builtin_amdgcn_sched_group_barrier(0x002, (8 * (e_hi - e_lo) + (m_hi - m_lo) - 1) / (m_hi - m_lo), 0);
+        }
+      }
+      static_for<e_hi - e_lo>([&](auto J) __attribute__((always_inline)) { pin(nw[e_lo + J]); });
+      __builtin_amdgcn_sched_barrier(0);
+      issue_one<G, FS>();
+      __builtin_amdgcn_sched_barrier(0);
+      step64<RS, FS, G + 1>(ch, ct, cw, nh, nt, nw, acc);
+    } else {
+      if constexpr (RS < 0) next_read_slot();
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+      __builtin_amdgcn_s_barrier();
+    }
+  }
+  __device__ __forceinline__ void run_fp64(v16f (&acc)[MI][NI]) {
+    v4i h0[NF], h1[NF];
+    v2i t0[NF], t1[NF];
+    v6i w0[NI], w1[NI];
+    read6(h0, t0);
+    chunk_expand<0, NI>(h0, w0);
+    int j = 0;
+    for (; j + NS <= steps0; j += NS) {
+      static_for<NS / 2>([&](auto I) __attribute__((always_inline)) {
+        constexpr int i = 2 * I;
+        step64<i + 1, (i + NS - 1) % NS>(h0, t0, w0, h1, t1, w1, acc);
+        step64<(i + 2) % NS, i>(h1, t1, w1, h0, t0, w0, acc);
+      });
+    }
+    for (; j < steps0; j += 2) {
+      step64(h0, t0, w0, h1, t1, w1, acc);
+      step64(h1, t1, w1, h0, t0, w0, acc);
+    }
+    previous_read_slot();
+  }
   template <int RS, int LO, int HI>
   __device__ __forceinline__ void chunk_reads6(v4i (&nh)[NF], v2i (&nt)[NF]) const {
     if constexpr (LO < HI) {
@@ -358,6 +478,7 @@ struct Fp6Pipe {
 
   // Integer steps [0, steps0): acc += (Lw / 8)(Lx / 8) summed over 64 elements per MFMA.
   __device__ __forceinline__ void run_fp6(v16f (&acc)[MI][NI]) {
+    if constexpr (W4) return run_fp64(acc);
     v4i h0[NF], h1[NF];
     v2i t0[NF], t1[NF];
     read6(h0, t0);
@@ -467,9 +588,35 @@ __device__ __forceinline__ void tile_vector_widen(const Vectors &tv, bool bias, 
   }
 }
 
-template <class C>
+// The level sums behind the operand blocks of a 4- or 6-bit buffer, in the same way.
+template <class C, class Vectors, class Args>
+__device__ __forceinline__ void tile_sums_request(const Vectors &tv, const Args &p, int64_t x_sums, int64_t w_sums, int m0, int n0,
+                                                  int wave) {
+  const int i = threadIdx.x;
+  if (wave * 64 < C::BN) {
+    const int n = n0 + i < p.N ? n0 + i : p.N - 1;
+    dma_load_u32(p.wbuf + w_sums + static_cast<int64_t>(p.n_first) * 4, static_cast<uint32_t>(n) * 4, lds_address(tv.colc) + wave * 256);
+  }
+  if (wave * 64 < C::BM) {
+    const int m = m0 + i < p.M ? m0 + i : p.M - 1;
+    dma_load_u32(p.xbuf + x_sums, static_cast<uint32_t>(m) * 4, lds_address(tv.rowc) + wave * 256);
+  }
+}
+template <class C, class Vectors>
+__device__ __forceinline__ void tile_sums_widen(const Vectors &tv, int K) {
+  const int i = threadIdx.x;
+  if (i < C::BN) tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
+  if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * __float_as_int(tv.rowc[i]) - 64 * K);
+}
+
+template <class C, bool W4 = false>
+constexpr int fused6_vectors_offset() {
+  constexpr int staging = BlockStore<C, uint16_t>::kBytes * C::MI * C::WAVES;
+  return staging > Fp6Pipe<C, W4>::SMEM ? staging : Fp6Pipe<C, W4>::SMEM;
+}
+template <class C, bool W4 = false>
 constexpr int fused6_smem() {
-  return Fp6Pipe<C>::SMEM + TileVectors6<C>::kBytes;
+  return fused6_vectors_offset<C, W4>() + TileVectors6<C>::kBytes;
 }
 
 // Split over K (few tiles, long K): `splits` workgroups per tile take `per` integer steps each and add their raw
@@ -586,33 +733,32 @@ __device__ __forceinline__ bool wave_is_idle(const Args &p, int m0, int n0) {
   return m0 + wave / C::WAVES_N * C::WM >= p.M || n0 + wave % C::WAVES_N * C::WN >= p.N;
 }
 
-template <class C, bool BF16, bool SPLITK = false>
+template <class C, bool BF16, bool SPLITK = false, bool W4 = false>
 __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn, uint8_t *smem, int split = 0,
                                             int tile_id = 0, const SplitK *sk = nullptr) {
-  using Pipe = Fp6Pipe<C>;
+  using Pipe = Fp6Pipe<C, W4>;
   const int m0 = tm * C::BM, n0 = tn * C::BN;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int wm = wave / C::WAVES_N, wn = wave % C::WAVES_N;
-  const Fp6Layout lx = fp6_layout(p.M, p.K, p.F), lw = fp6_layout(p.N_total, p.K, p.F);
-  const TileVectors6<C> tv(smem + Pipe::SMEM);
+  const Fp6Layout lx = fp6_layout(p.M, p.K, p.F);
+  const auto layout_w = [&] {
+    if constexpr (W4) {
+      return tile4_layout(p.N_total, p.K, p.F);
+    } else {
+      return fp6_layout(p.N_total, p.K, p.F);
+    }
+  };
+  const auto lw = layout_w();
+  const TileVectors6<C> tv(smem + fused6_vectors_offset<C, W4>());
   // thread i requests column i and row i of the vectors, raw, and widens them in place when they have landed
   static_assert(C::BM <= C::kThreads && C::BN <= C::kThreads && C::BM % 64 == 0 && C::BN % 64 == 0, "a thread per row and column");
   const int swave = __builtin_amdgcn_readfirstlane(wave);
   const bool asym = p.w_red != nullptr;  // asymmetric: meta holds (scale, zero) pairs; symmetric: one scale per row, no zero term
   tile_vector_request<C>(tv, p, m0, n0, swave);
-  if (swave * 64 < C::BN) {
-    const int i = threadIdx.x, n = n0 + i < p.N ? n0 + i : p.N - 1;
-    dma_load_u32(p.wbuf + lw.sums_off + static_cast<int64_t>(p.n_first) * 4, static_cast<uint32_t>(n) * 4, lds_address(tv.colc) + swave * 256);
-  }
-  if (swave * 64 < C::BM) {
-    const int i = threadIdx.x, m = m0 + i < p.M ? m0 + i : p.M - 1;
-    dma_load_u32(p.xbuf + lx.sums_off, static_cast<uint32_t>(m) * 4, lds_address(tv.rowc) + swave * 256);
-  }
+  tile_sums_request<C>(tv, p, lx.sums_off, lw.sums_off, m0, n0, swave);
   auto widen = [&] {
-    const int i = threadIdx.x;
     tile_vector_widen<C, BF16>(tv, p.bias != nullptr, asym, 8.0f);
-    if (i < C::BN) tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
-    if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * __float_as_int(tv.rowc[i]) - 64 * p.K);
+    tile_sums_widen<C>(tv, p.K);
   };
 
   Pipe pipe;
@@ -699,7 +845,7 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
   // the store issue are paid once per tile and not once per row block.  The per-column vectors are read once;
   // the fragment registers are free by now.
   using Store = BlockStore<C, uint16_t>;
-  static_assert(Store::kBytes * C::MI * C::WAVES <= Pipe::SMEM, "staging fits in the ring");
+  static_assert(Store::kBytes * C::MI * C::WAVES <= fused6_vectors_offset<C, W4>(), "staging ends before the vectors");
   uint8_t *stage = smem + wave * (Store::kBytes * C::MI);
   const bool vec = (p.ldo & 7) == 0 && (reinterpret_cast<uintptr_t>(p.out) & 15) == 0;
   const int nw = n0 + wn * C::WN, mw = m0 + wm * C::WM;
@@ -741,27 +887,27 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
   }
 }
 
-template <class C, bool BF16>
+template <class C, bool BF16, bool W4 = false>
 __global__ __launch_bounds__(C::kThreads) void gemm_fused6_kernel(Fused6Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
-  fused6_tile<C, BF16>(p, tm, tn, smem);
+  fused6_tile<C, BF16, false, W4>(p, tm, tn, smem);
 }
 
 // K split over sk.splits workgroups per tile: block b works on tile b % grid_tiles, split b / grid_tiles.
-template <class C, bool BF16>
+template <class C, bool BF16, bool W4 = false>
 __global__ __launch_bounds__(C::kThreads) void gemm_fused6_splitk_kernel(Fused6Args p, int tiles_m, int tiles_n,
                                                                           SplitK sk) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int split = blockIdx.x / sk.grid_tiles;
   if (!tile_of_block<C::BM>(blockIdx.x - split * sk.grid_tiles, tiles_m, tiles_n, tm, tn)) return;
-  fused6_tile<C, BF16, true>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
+  fused6_tile<C, BF16, true, W4>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
 }
 
 // One launch, two tile shapes (see gemm_i32_split_kernel).
-template <class CW, class CT, bool BF16>
+template <class CW, class CT, bool BF16, bool W4 = false>
 __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_split_kernel(Fused6Args wide, Fused6Args tail,
                                                                          SplitGrid grid) {
   static_assert(CW::kThreads == CT::kThreads && CW::BM == CT::BM, "one block size, one tile height");
@@ -769,9 +915,9 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_split_kernel(Fused6A
   int tm, tn;
   const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
   if (kind == 1) {
-    fused6_tile<CW, BF16>(wide, tm, tn, smem);
+    fused6_tile<CW, BF16, false, W4>(wide, tm, tn, smem);
   } else if (kind == 2) {
-    fused6_tile<CT, BF16>(tail, tm, tn, smem);
+    fused6_tile<CT, BF16, false, W4>(tail, tm, tn, smem);
   }
 }
 
@@ -780,16 +926,16 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_split_kernel(Fused6A
 struct RestGrid {
   int tiles_m_wide, tiles_n_wide, wide_blocks, tiles_m, tiles_n, first;
 };
-template <class CW, class CT, bool BF16>
+template <class CW, class CT, bool BF16, bool W4 = false>
 __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_rest_kernel(Fused6Args p, RestGrid g) {
   static_assert(CW::kThreads == CT::kThreads, "one block size");
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int bid = blockIdx.x;
   if (bid < g.wide_blocks) {
-    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused6_tile<CW, BF16>(p, tm, tn, smem);
+    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused6_tile<CW, BF16, false, W4>(p, tm, tn, smem);
   } else if (tile_of_block<CT::BM>(bid - g.wide_blocks, g.tiles_m, g.tiles_n, tm, tn)) {
-    fused6_tile<CT, BF16>(p, tm, g.first + tn, smem);
+    fused6_tile<CT, BF16, false, W4>(p, tm, g.first + tn, smem);
   }
 }
 

@@ -16,7 +16,7 @@ inline int64_t align256(int64_t v) { return (v + 255) & ~int64_t(255); }
 std::atomic<bool> layer_one_launch{true};  // (read by every forward, possibly from several host threads)
 
 struct LayerPlan {
-  bool tiled;
+  bool tiled, four_x;  // four_x: the activation in the 4-bit format
   int64_t off_q, off_meta, off_fp, bytes;
 };
 
@@ -26,13 +26,23 @@ bool layer_valid(const quik_layer *l) {
          l->num_int + l->num_fp == l->in_features && l->out_features > 0;
 }
 
+bool four_bit(const quik_layer *l) { return l->bits == 4 && l->tiled_format == QUIK_TILED_4; }
+// the activation comes in the 4-bit format (4-bit weights, tiles whose kernels take it so)
+bool four_bit_x(const quik_layer *l, int64_t rows) {
+  return four_bit(l) && tile4_activation_bits(rows, l->out_features, l->num_int, l->num_fp) == 4;
+}
+int64_t operand_bytes(const quik_layer *l, int64_t rows, bool four_x) {
+  return four_x         ? tile4_operand_bytes(rows, l->num_int, l->num_fp)
+         : l->bits == 4 ? fp6_operand_bytes(rows, l->num_int, l->num_fp, kLayerK4)
+                        : tile8_operand_bytes(rows, l->num_int, l->num_fp, kLayerK8);
+}
+
 // tile-ordered path: the layer has a tile-ordered weight copy, enough rows, a column map that streams, a shape the
 // operand formats take; symmetric activations are fp16 only
 bool use_tiled(const quik_layer *l, int64_t rows) {
   if (!l->tiled_weight || rows < l->tiled_min_rows || !l->colmap_streams) return false;
   if (l->symmetric && l->dtype != QUIK_F16) return false;
-  return (l->bits == 4 ? fp6_operand_bytes(rows, l->num_int, l->num_fp, kLayerK4)
-                       : tile8_operand_bytes(rows, l->num_int, l->num_fp, kLayerK8)) > 0;
+  return operand_bytes(l, rows, false) > 0;
 }
 
 LayerPlan plan_layer(const quik_layer *l, int64_t rows) {
@@ -40,10 +50,9 @@ LayerPlan plan_layer(const quik_layer *l, int64_t rows) {
   p.tiled = use_tiled(l, rows);
   const int64_t meta_bytes = align256((l->symmetric ? 1 : 2) * rows * 2);
   if (p.tiled) {
-    const int64_t qb = l->bits == 4 ? fp6_operand_bytes(rows, l->num_int, l->num_fp, kLayerK4)
-                                    : tile8_operand_bytes(rows, l->num_int, l->num_fp, kLayerK8);
+    p.four_x = four_bit_x(l, rows);
     p.off_q = 0;
-    p.off_meta = align256(qb);
+    p.off_meta = align256(operand_bytes(l, rows, p.four_x));
     p.off_fp = p.off_meta + meta_bytes;
     p.bytes = p.off_fp;
   } else {
@@ -103,11 +112,11 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
   if (l.symmetric) {
     if (l.dtype != QUIK_F16 || !l.colmap_streams) return QUIK_ERR_DTYPE;  // the caller's op sequence serves these
     if (int rc = sym_quantize_mapped(x, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, l.sym_divisor,
-                                     p.tiled ? 1 : 0, q, meta, fp_x, stream, l.bits == 4 ? kLayerK4 : kLayerK8))
+                                     !p.tiled ? 0 : p.four_x ? QUIK_TILED_4 : 1, q, meta, fp_x, stream, l.bits == 4 ? kLayerK4 : kLayerK8))
       return rc;
   } else if (p.tiled) {
     if (int rc = l.bits == 4 ? asym_quantize_fp6(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, q,
-                                                      meta, stream, kLayerK4)
+                                                      meta, stream, kLayerK4, p.four_x)
                              : asym_quantize_tile8(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp,
                                                         q, meta, stream, kLayerK8))
       return rc;
@@ -124,6 +133,9 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
     }
   }
   if (p.tiled) {
+    if (four_bit(layer))
+      return mixed_linear_tile4(q, p.four_x ? 4 : 6, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype, rows,
+                                l.out_features, l.num_int, l.num_fp, out, stream);
     return l.bits == 4 ? mixed_linear_fp6(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
                                                       rows, l.out_features, l.num_int, l.num_fp, out, splitk_workspace,
                                                       splitk_bytes, stream, kLayerK4)

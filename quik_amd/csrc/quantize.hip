@@ -1161,11 +1161,15 @@ __device__ __forceinline__ RowQuant<BF16> row_quant4(float lo, float hi, float s
 }
 
 // Where the row's fragments go in the operand buffer: the row's part of the address is wave-uniform, the fragment's part is
-// the unit 3072 (f / 2) and its half.
+// the unit f / 2 and its half.
+// (4-bit format: the unit is 2048 bytes and has no tails)
+template <bool FOUR>
 struct Fp6RowOut {
+  static constexpr uint32_t kUnit = FOUR ? 2048u : 3072u;
   uint8_t *head, *tail;
   uint32_t swap16;
-  __device__ __forceinline__ Fp6RowOut(uint8_t *dst, const Fp6Layout &l, int64_t row) {
+  template <class Layout>
+  __device__ __forceinline__ Fp6RowOut(uint8_t *dst, const Layout &l, int64_t row) {
     uint8_t *rb = dst + (row >> 6) * l.block_bytes;
     head = rb + ((row >> 5) & 1) * 1024 + (row & 31) * 32;
     tail = rb + 2048 + (row & 63) * 8;
@@ -1173,9 +1177,9 @@ struct Fp6RowOut {
   }
 };
 
-// One fragment: 32 values -> 32 levels -> 24 bytes, stored; returns the sum of its levels.
-template <bool BF16, bool SYM, bool SLOW>
-__device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQuant<BF16> &rq, int f, const Fp6RowOut &out) {
+// One fragment: 32 values -> 32 levels -> 24 bytes (16 in the 4-bit format), stored; returns the sum of its levels.
+template <bool BF16, bool SYM, bool SLOW, bool FOUR>
+__device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQuant<BF16> &rq, int f, const Fp6RowOut<FOUR> &out) {
   uint32_t b[8];  // 32 levels, one per byte
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -1195,12 +1199,16 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
   for (int i = 0; i < 8; ++i) sum = __builtin_amdgcn_udot4(b[i], 0x01010101u, sum, false);
   uint32_t o[6];
   fp6_pack_fragment(b, o);
-  const uint32_t unit = static_cast<uint32_t>(f >> 1) * 3072u, h = static_cast<uint32_t>(f & 1);
+  const uint32_t unit = static_cast<uint32_t>(f >> 1) * out.kUnit, h = static_cast<uint32_t>(f & 1);
   // (default cache policy: a 128-byte line of the operand buffer takes pieces of 4 (heads) or 16 (tails) rows,
   // which meet in the XCD's L2; as streaming stores every piece went to memory on its own and the launch
   // took 29 us instead of 12)
-  *reinterpret_cast<uint4 *>(out.head + unit + ((h << 4) ^ out.swap16)) = make_uint4(o[0], o[1], o[2], o[3]);
-  *reinterpret_cast<uint2 *>(out.tail + unit + h * 512u) = make_uint2(o[4], o[5]);
+  if constexpr (FOUR) {
+    *reinterpret_cast<uint4 *>(out.head + unit + ((h << 4) ^ out.swap16)) = nib_squeeze(o);
+  } else {
+    *reinterpret_cast<uint4 *>(out.head + unit + ((h << 4) ^ out.swap16)) = make_uint4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<uint2 *>(out.tail + unit + h * 512u) = make_uint2(o[4], o[5]);
+  }
   return sum;
 }
 
@@ -1229,7 +1237,7 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
 // same pieces, the wave form took 7.3 / 7.8 / 8.5 at 2048 x 4096.
 // (Fillers read beside the outlier values and the ranges of all waves in one LDS round trip, not one after the other:
 // 64 x 8192 3.68 -> 3.57, 2048 x 8192 12.3 -> 12.1, 64 x 28672 5.71 -> 5.48.)
-template <bool BF16, bool SYM, int JT>
+template <bool BF16, bool SYM, int JT, bool FOUR>
 __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     const uint16_t *__restrict__ x, int64_t rows, int cols, const uint32_t *__restrict__ patch,
     const uint16_t *__restrict__ fp_col, int nholes, int num_int, int num_fp, uint8_t *__restrict__ dst,
@@ -1270,7 +1278,21 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
   const uint4 oc = *reinterpret_cast<const uint4 *>(fp_col + (tid < nchunk ? tid : 0) * 8);
   if (tid == 0) total_s = 0;
   if (tid < 8 && tid >= W) red[tid] = __builtin_inff(), red[8 + tid] = -__builtin_inff();
-  const Fp6Layout l6 = fp6_layout(rows, num_int, num_fp);
+  const auto layout = [&] {
+    if constexpr (FOUR) {
+      return tile4_layout(rows, num_int, num_fp);
+    } else {
+      return fp6_layout(rows, num_int, num_fp);
+    }
+  };
+  const auto l6 = layout();
+  auto outlier_offset = [&](int c) {
+    if constexpr (FOUR) {
+      return tile4_offset(l6, row, l6.steps + (c >> 1), c & 1);
+    } else {
+      return fp6_outlier_offset(l6, row, c >> 1, c & 1);
+    }
+  };
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   __syncthreads();
 
@@ -1281,7 +1303,7 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     uint32_t o[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) o[k] = ld16(ow[k] & 0xFFFFu) | (ld16(ow[k] >> 16) << 16);
-    *reinterpret_cast<uint4 *>(dst + fp6_outlier_offset(l6, row, c >> 1, c & 1)) = make_uint4(o[0], o[1], o[2], o[3]);
+    *reinterpret_cast<uint4 *>(dst + outlier_offset(c)) = make_uint4(o[0], o[1], o[2], o[3]);
   };
   uint32_t filler[PREG];  // read together with the outlier values: integer columns, none of them is a hole
 #pragma unroll
@@ -1327,13 +1349,13 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
     mx = fmaxf(mx, part[8 + w]);
   }
   const RowQuant<BF16> rq = row_quant4<BF16, SYM>(mn, mx, sym_divisor, tid == 0, meta, row);
-  const Fp6RowOut out(dst, l6, row);
+  const Fp6RowOut<FOUR> out(dst, l6, row);
   int sum = 0;
   auto quantise = [&](auto slow_c) {
 #pragma unroll
     for (int j = 0; j < JT; ++j)
       if (tid + j * T < frags)
-        sum += quantise_fragment<BF16, SYM, decltype(slow_c)::value>(v[j], rq, tid + j * T, out);
+        sum += quantise_fragment<BF16, SYM, decltype(slow_c)::value, FOUR>(v[j], rq, tid + j * T, out);
   };
   if (__builtin_amdgcn_readfirstlane(rq.slow ? 1 : 0)) {
     quantise(std::true_type{});
@@ -1764,10 +1786,10 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
 }
 
 
-// 6-bit operand output through quantize_fp6_row_kernel; meta: (scale, zero) pairs, or one scale per row (SYM)
-template <bool BF16, bool SYM>
+// 6-bit (FOUR: 4-bit) operand output through quantize_fp6_row_kernel; meta: (scale, zero) pairs, or one scale per row (SYM)
+template <bool BF16, bool SYM, bool FOUR>
 int launch_fp6_row(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, const ColmapLayout &l, int64_t num_int,
-                   int64_t num_fp, void *dst, void *meta, hipStream_t st, float sym_divisor = 1.0f) {
+                   int64_t num_fp, void *dst, void *meta, hipStream_t st, float sym_divisor) {
   uint32_t words[4];
   if (int rc = colmap_words(cm, cols, num_int, num_fp, st, words)) return rc;
   if ((words[0] & (kColmapStreams | kColmapInPlace)) != (kColmapStreams | kColmapInPlace)) return QUIK_ERR_COLMAP;
@@ -1788,7 +1810,8 @@ int launch_fp6_row(const void *x, int64_t rows, int64_t cols, const uint8_t *cm,
     return static_cast<int>(QUIK_OK);
   };
   // at most eight waves per workgroup; kStreamMaxCols columns are two fragments per lane
-  return cols <= 8 * 64 * 32 ? go(quantize_fp6_row_kernel<BF16, SYM, 1>, 1) : go(quantize_fp6_row_kernel<BF16, SYM, 2>, 2);
+  return cols <= 8 * 64 * 32 ? go(quantize_fp6_row_kernel<BF16, SYM, 1, FOUR>, 1)
+                             : go(quantize_fp6_row_kernel<BF16, SYM, 2, FOUR>, 2);
 }
 // asym_quantize_list_kernel: calls that it takes (everything else, and every error, is left to the column map's path).
 // Up to 16384 columns it was the faster one at every row count from 1 to 2048 (2048 x 11008 27.1 -> 25.5, the least); with
@@ -1923,7 +1946,7 @@ extern "C" int quik_colmap_streaming(const void *colmap, int64_t cols, int64_t n
 }
 
 int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
-                            int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple) {
+                            int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple, bool four) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (rows < 0 || cols <= 0 || num_int <= 0 || num_fp < 0 || num_int + num_fp != cols) return QUIK_ERR_SHAPE;
   if (num_int % k_multiple != 0 || num_fp % 32 != 0 || cols > kStreamMaxCols) return QUIK_ERR_ALIGN;
@@ -1934,8 +1957,14 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   hipStream_t st = as_stream(stream);
-  return dtype == QUIK_F16 ? launch_fp6_row<false, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st)
-                           : launch_fp6_row<true, false>(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st);
+  auto go = [&](auto launch) { return launch(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st, 1.0f); };
+  if (four) return dtype == QUIK_F16 ? go(launch_fp6_row<false, false, true>) : go(launch_fp6_row<true, false, true>);
+  return dtype == QUIK_F16 ? go(launch_fp6_row<false, false, false>) : go(launch_fp6_row<true, false, false>);
+}
+
+extern "C" int quik_asym_quantize_tile4(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
+                                        int64_t num_int, int64_t num_fp, void *out4, void *meta, void *stream) {
+  return quik::asym_quantize_fp6(x, dtype, rows, cols, colmap, num_int, num_fp, out4, meta, stream, kLayerK4, true);
 }
 
 extern "C" int quik_asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
@@ -1986,7 +2015,9 @@ int quik::sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const v
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   hipStream_t st = as_stream(stream);
-  if (bits == 4 && tiled) return launch_fp6_row<false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
+  if (bits == 4 && tiled == QUIK_TILED_4)
+    return launch_fp6_row<false, true, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
+  if (bits == 4 && tiled) return launch_fp6_row<false, true, false>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
   return bits == 4 ? launch_sym_stream<4>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor)
                    : launch_sym_stream<8>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor);
 }
@@ -1995,7 +2026,7 @@ extern "C" int quik_sym_quantize_mapped(const void *x, int64_t rows, int64_t col
                                         int64_t num_fp, int bits, float divisor, int tiled, void *dst, void *scale,
                                         void *fp_x, void *stream) {
   return quik::sym_quantize_mapped(x, rows, cols, colmap, num_int, num_fp, bits, divisor, tiled, dst, scale, fp_x, stream,
-                                   bits == 4 ? 128 : 64);
+                                   bits == 8 ? 64 : tiled == QUIK_TILED_4 ? kLayerK4 : 128);
 }
 
 extern "C" int quik_asym_find_meta(const void *x, int64_t rows, int64_t cols, int bits, void *meta, void *stream) {

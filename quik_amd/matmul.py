@@ -14,7 +14,8 @@ import torch
 
 from . import _lib as L
 
-__all__ = ["int4Matmul", "int8Matmul", "mixed_linear", "pack_weight_fp6", "mixed_linear_fp6", "pack_weight_tile8",
+__all__ = ["int4Matmul", "int8Matmul", "mixed_linear", "pack_weight_fp6", "mixed_linear_fp6", "mixed_linear_tile4",
+           "pack_weight_tile8",
            "mixed_linear_tile8"]
 
 
@@ -133,9 +134,11 @@ def _splitk_workspace(device, M, N, K, bits):
     return ws, ws.numel()
 
 
-def pack_weight_fp6(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor) -> torch.Tensor:
-    """Nibble-packed int4 weights [N, K/2] and outlier weights [N, F] -> operand buffer for mixed_linear_fp6
-    (once per layer).  `colmap` is the layer's column map (asymmetric.build_colmap): the operand buffers of this
+def pack_weight_fp6(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor,
+                    four_bit: bool = False) -> torch.Tensor:
+    """Nibble-packed int4 weights [N, K/2] and outlier weights [N, F] -> operand buffer for mixed_linear_fp6, or with
+    four_bit for mixed_linear_tile4 (once per layer; the 4-bit buffer stands at the front of the bytes that the 6-bit one
+    takes, so that what a program has set aside for a layer fits either).  `colmap` is the layer's column map (asymmetric.build_colmap): the operand buffers of this
     path keep the integer columns in the map's in-place order, weights and activations alike."""
     L.check_cuda_contiguous("pack_weight_fp6", int_weight=int_weight, fp_weight=fp_weight, colmap=colmap)
     if int_weight.dtype != torch.uint8 or int_weight.dim() != 2:
@@ -159,8 +162,9 @@ def pack_weight_fp6(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: t
                            "int_indices that partition the columns with fp_indices)")
     with L.device_guard(int_weight.device):
         out = torch.empty((nbytes,), dtype=torch.uint8, device=int_weight.device)
-        L.check(lib.quik_fp6_pack_weight(L.ptr(int_weight), L.ptr(fp_weight) if F else None, N, K, F, L.ptr(colmap),
-                                         L.ptr(out), L.stream()), "pack_weight_fp6")
+        pack = lib.quik_tile4_pack_weight if four_bit else lib.quik_fp6_pack_weight
+        L.check(pack(L.ptr(int_weight), L.ptr(fp_weight) if F else None, N, K, F, L.ptr(colmap), L.ptr(out), L.stream()),
+                "pack_weight_fp6")
     return out
 
 
@@ -195,6 +199,38 @@ def mixed_linear_fp6(x6, w6, meta, weights_scales, reduced_w, bias, M, N, K, F, 
     return out
 
 
+def mixed_linear_tile4(x, w4, meta, weights_scales, reduced_w, bias, M, N, K, F, out_dtype):
+    """mixed_linear_fp6 on weights of the 4-bit format (pack_weight_fp6 with four_bit); x: an operand buffer of either format
+    (asymmetric.quantize_mapped_fp6 with or without four_bit).  Same result bit for bit."""
+    tensors = dict(x=x, w4=w4, meta=meta, weights_scales=weights_scales)
+    symmetric = reduced_w is None
+    if not symmetric:
+        tensors["reduced_w"] = reduced_w
+    if bias is not None and bias.numel() > 0:
+        tensors["bias"] = bias
+    L.check_cuda_contiguous("mixed_linear_tile4", **tensors)
+    dt = L.QUIK_F16 if out_dtype == torch.float16 else L.QUIK_BF16 if out_dtype == torch.bfloat16 else None
+    if dt is None:
+        raise RuntimeError(f"mixed_linear_tile4: unsupported dtype {out_dtype}")
+    for name, t in tensors.items():
+        if name not in ("x", "w4") and t.dtype != out_dtype:
+            raise RuntimeError(f"mixed_linear_tile4: expected {name} of dtype {out_dtype} but got {t.dtype}")
+    lib = L.load()
+    x_bits = {lib.quik_tile4_operand_bytes(M, K, F): 4, lib.quik_fp6_operand_bytes(M, K, F): 6}.get(x.numel())
+    need = lib.quik_tile4_operand_bytes(N, K, F)
+    if x_bits is None or need == 0 or w4.numel() < need:
+        raise RuntimeError("mixed_linear_tile4: operand buffers do not match M, N, K, F")
+    if meta.numel() != (M if symmetric else 2 * M) or weights_scales.numel() != N or \
+            (not symmetric and reduced_w.numel() != N):
+        raise RuntimeError("mixed_linear_tile4: meta / weights_scales / reduced_w sizes are inconsistent with M, N")
+    with L.device_guard(x.device):
+        out = torch.empty((M, N), dtype=out_dtype, device=x.device)
+        L.check(lib.quik_mixed_linear_fwd_tile4(L.ptr(x), x_bits, L.ptr(w4), L.ptr(meta), L.ptr(weights_scales),
+                                                L.ptr(tensors.get("reduced_w")), L.ptr(tensors.get("bias")), dt, M, N, K, F,
+                                                L.ptr(out), L.stream()), "mixed_linear_tile4")
+    return out
+
+
 def pack_weight_tile8(int_weight: torch.Tensor, fp_weight: torch.Tensor) -> torch.Tensor:
     """int8 weights [N, K] and outlier weights [N, F] -> tile-ordered operand buffer for mixed_linear_tile8
     (once per layer)."""
@@ -216,9 +252,11 @@ def pack_weight_tile8(int_weight: torch.Tensor, fp_weight: torch.Tensor) -> torc
     return out
 
 
-def pack_weight_layer(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor, bits: int) -> torch.Tensor:
+def pack_weight_layer(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor, bits: int,
+                      four_bit: bool = False) -> torch.Tensor:
     """Tile-ordered weight copy for the one-call layer forward, any number of integer columns that fills whole
-    fragments (4 bits: a multiple of 32, 8 bits: of 16); the last k-steps are filled up with zeros."""
+    fragments (4 bits: a multiple of 32, 8 bits: of 16); the last k-steps are filled up with zeros.  four_bit (bits=4): in the
+    4-bit format, as pack_weight_fp6."""
     L.check_cuda_contiguous("pack_weight_layer", int_weight=int_weight, fp_weight=fp_weight, colmap=colmap)
     N, K, F = int_weight.size(0), int_weight.size(1) * (2 if bits == 4 else 1), fp_weight.size(1)
     if int_weight.dtype != (torch.uint8 if bits == 4 else torch.int8) or fp_weight.size(0) != N or \
@@ -232,8 +270,10 @@ def pack_weight_layer(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap:
         raise RuntimeError("pack_weight_layer: shape not supported by the tile-ordered operand format")
     with L.device_guard(int_weight.device):
         out = torch.empty((nbytes,), dtype=torch.uint8, device=int_weight.device)
-        L.check(lib.quik_layer_pack_weight(L.ptr(int_weight), L.ptr(fp_weight) if F else None, N, K, F, bits,
-                                           L.ptr(colmap), L.ptr(out), L.stream()), "pack_weight_layer")
+        fp = L.ptr(fp_weight) if F else None
+        L.check(lib.quik_tile4_pack_weight(L.ptr(int_weight), fp, N, K, F, L.ptr(colmap), L.ptr(out), L.stream()) if four_bit else
+                lib.quik_layer_pack_weight(L.ptr(int_weight), fp, N, K, F, bits, L.ptr(colmap), L.ptr(out), L.stream()),
+                "pack_weight_layer")
     return out
 
 

@@ -292,6 +292,8 @@ class MixedQLinear(torch.nn.Module):
     # (see weight_bytes(); set on the class for every layer or on single modules).
     transient_tiled_copy = False
 
+    _w6_four = False    # the tile-ordered copy is in the 4-bit format (csrc/fp6_format.h)
+
     def __init__(self, in_features, out_features, shared_input=None,
                  fp_features_num=0, symm=False, bits=4, dtype=torch.float16, fused=True, allocate=True):
         """allocate=False: the buffers are registered empty (the caller assigns them); otherwise as in the reference."""
@@ -388,10 +390,11 @@ class MixedQLinear(torch.nn.Module):
         return self.int_features_num % (128 if self.bits == 4 else 64) == 0
 
     def _pack_tiled(self, fp_w):
+        self._w6_four = self.bits == 4     # (written with the copy: one read from an older file may be in the 6-bit format)
         if not self._whole_steps():
-            return matmul.pack_weight_layer(self.int_weight, fp_w, self._column_map(), self.bits)
+            return matmul.pack_weight_layer(self.int_weight, fp_w, self._column_map(), self.bits, self._w6_four)
         if self.bits == 4:    # in the column map's in-place order, as the activation is quantized
-            return matmul.pack_weight_fp6(self.int_weight, fp_w, self._column_map())
+            return matmul.pack_weight_fp6(self.int_weight, fp_w, self._column_map(), True)
         return matmul.pack_weight_tile8(self.int_weight, fp_w)
 
     def _weight6(self):
@@ -489,6 +492,7 @@ class MixedQLinear(torch.nn.Module):
             d = L.QuikLayer.from_buffer_copy(base)
             w6 = self._weight6()
             d.tiled_weight = w6.data_ptr()
+            d.tiled_format = L.TILED_4 if self._w6_four else 0
             d._keep = w6     # (alive until the caller drops the descriptor, i.e. behind the launch)
             return d, self._descs.setdefault("transient_sizes", {})
         entry = self._descs.get(tiled)
@@ -511,6 +515,7 @@ class MixedQLinear(torch.nn.Module):
             d.fp_weight = bufs[5].data_ptr() if bufs[5] is not None and bufs[5].numel() > 0 else None
             d.bias = bufs[6].data_ptr() if bufs[6] is not None and bufs[6].numel() > 0 else None
             d.tiled_weight = w6.data_ptr() if w6 is not None else None
+            d.tiled_format = L.TILED_4 if w6 is not None and self._w6_four else 0
             entry = self._descs[tiled] = (stamp, d, {}, (colmap, w6))   # the tensors the pointers refer to stay alive
         return entry[1], entry[2]
 
@@ -622,17 +627,23 @@ class MixedQLinear(torch.nn.Module):
         with device_guard(x.device):
             if x2.data_ptr() % 16 == 0 and (not self.symmetric or x2.dtype == torch.float16) \
                     and self._six_bit_ok(x2.shape[0]) and self._whole_steps():
-                quantize6 = asymmetric.quantize_mapped_fp6 if self.bits == 4 else asymmetric.quantize_mapped_tile8
-                linear6 = matmul.mixed_linear_fp6 if self.bits == 4 else matmul.mixed_linear_tile8
-                if shared_input.x6 is None:
+                w6 = self._weight6()
+                linear6 = matmul.mixed_linear_tile8 if self.bits == 8 else \
+                    matmul.mixed_linear_tile4 if self._w6_four else matmul.mixed_linear_fp6
+                if shared_input.x6 is None or linear6 is matmul.mixed_linear_fp6 and shared_input.x6.numel() != \
+                        L.load().quik_fp6_operand_bytes(x2.shape[0], self.int_features_num, self.fp_features_num):
+                    # (the members of a group share the first one's: the kernels of 4-bit weights take either format)
+                    four = self._w6_four and L.load().quik_tile4_activation_bits(
+                        x2.shape[0], self.out_features, self.int_features_num, self.fp_features_num) == 4
+                    shape = (x2, self._column_map(), self.int_features_num, self.fp_features_num)
                     if self.symmetric:
                         shared_input.x6, shared_input.qscale_x, _ = symmetric.quantize_mapped(
-                            x2, self._column_map(), self.int_features_num, self.fp_features_num, self.bits,
-                            self.sym_divisor, True)
+                            *shape, self.bits, self.sym_divisor, True, four)
+                    elif self.bits == 4:
+                        shared_input.x6, shared_input.meta = asymmetric.quantize_mapped_fp6(*shape, four)
                     else:
-                        shared_input.x6, shared_input.meta = quantize6(
-                            x2, self._column_map(), self.int_features_num, self.fp_features_num)
-                output = linear6(shared_input.x6, self._weight6(),
+                        shared_input.x6, shared_input.meta = asymmetric.quantize_mapped_tile8(*shape)
+                output = linear6(shared_input.x6, w6,
                                  shared_input.qscale_x if self.symmetric else shared_input.meta,
                                  self.weights_scales, None if self.symmetric else self.reduced_w, self.bias,
                                  x2.shape[0], self.out_features, self.int_features_num, self.fp_features_num,

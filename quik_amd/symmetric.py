@@ -102,12 +102,13 @@ def int8FusedDequantize(A, B, scale_row, scale_col, y):
 
 
 def quantize_mapped(src: torch.Tensor, colmap: torch.Tensor, num_int: int, num_fp: int, bits: int, divisor: float,
-                    tiled: bool):
+                    tiled: bool, four_bit: bool = False):
     """MixedQLinear's symmetric activation branch (experiments/qlinear.py:97-103) in one kernel: outlier gather,
     scale = fp16(max|x[:, int]| / divisor) and rne(fp16(x / scale)) codes.  fp16 only; the column map must select
     the streaming kernel (asymmetric.colmap_streams).  Returns (q, scale [rows, 1], fp_x) with q / fp_x as
     symmetric.quantize would give them, or, with tiled=True, (operand buffer, scale, None) for
-    matmul.mixed_linear_fp6 (bits=4) / matmul.mixed_linear_tile8 (bits=8)."""
+    matmul.mixed_linear_fp6 (bits=4) / matmul.mixed_linear_tile8 (bits=8); four_bit (bits=4, tiled): one of the 4-bit format
+    for matmul.mixed_linear_tile4."""
     from .asymmetric import check_mapped_args
     if bits not in (4, 8):
         raise RuntimeError("Unsupported data type")
@@ -116,8 +117,9 @@ def quantize_mapped(src: torch.Tensor, colmap: torch.Tensor, num_int: int, num_f
     lib = L.load()
     with L.device_guard(src.device):
         if tiled:
-            nbytes = (lib.quik_fp6_operand_bytes if bits == 4 else lib.quik_tile8_operand_bytes)(max(rows, 1), num_int,
-                                                                                                  num_fp)
+            operand_bytes = lib.quik_tile8_operand_bytes if bits == 8 else \
+                lib.quik_tile4_operand_bytes if four_bit else lib.quik_fp6_operand_bytes
+            nbytes = operand_bytes(max(rows, 1), num_int, num_fp)
             if nbytes == 0:
                 raise RuntimeError("quantize: shape not supported by the tile-ordered operand format")
             dst = torch.empty((nbytes,), dtype=torch.uint8, device=src.device)
@@ -128,7 +130,7 @@ def quantize_mapped(src: torch.Tensor, colmap: torch.Tensor, num_int: int, num_f
             fp_x = torch.empty((rows, num_fp), dtype=src.dtype, device=src.device)
         scale = torch.empty((rows, 1), dtype=torch.float16, device=src.device)
         L.check(lib.quik_sym_quantize_mapped(L.ptr(src), rows, cols, L.ptr(colmap), num_int, num_fp, bits,
-                                             float(divisor), 1 if tiled else 0, L.ptr(dst), L.ptr(scale),
+                                             float(divisor), 0 if not tiled else L.TILED_4 if four_bit else 1, L.ptr(dst), L.ptr(scale),
                                              L.ptr(fp_x) if fp_x is not None and num_fp else None, L.stream()),
                 "quantize")
     return dst, scale, fp_x
