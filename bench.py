@@ -51,7 +51,7 @@ WORKLOADS = {
     "llama2-70b.down_proj.int8.t1": (1, 28672, 8192, 256, 8),
     "llama2-13b.down_proj.int8.t16": (16, 13824, 5120, 256, 8),
     "llama2-70b.gate_proj.t64": (64, 8192, 28672, 256, 4),
-    "llama2-70b.gate_proj.t32": (32, 8192, 28672, 256, 4),          # weight-streaming kernel, token rows in LDS
+    "llama2-70b.gate_proj.t32": (32, 8192, 28672, 256, 4),          # weight-streaming kernel
     "llama2-70b.down_proj.int8.t64": (64, 28672, 8192, 256, 8),     # 64 tiles, K = 28416: split over K
 }
 
@@ -668,7 +668,7 @@ def main():
     elif mod.fused:
         gemm_kernel = "gemv_decode_kernel (one or two token rows: quantize and weight-streaming matrix-vector product " \
             "in ONE launch)" \
-            if M <= 2 else "gemm_decode_kernel (weight streaming, one launch per step)" if M <= 32 else \
+            if M <= 2 else "gemm_skinny_kernel (weight streaming, one launch per step)" if M <= 32 else \
             "gemm_fused_split_kernel / gemm_fused_kernel (one launch per step)"
         dtype = "int8" if bits == 8 else "int4 (dot-product instructions)" if M <= 2 else "int4 (on int8 MFMA)"
     else:

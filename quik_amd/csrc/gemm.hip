@@ -3,13 +3,13 @@
 #include <cstdint>
 
 #include "colmap.h"
-#include "gemm_decode.h"
 #include "gemm_gemv.h"
 #ifndef GEMV_MAX_ROWS
 #define GEMV_MAX_ROWS 2
 #endif
 #include "gemm_rows.h"
 #include "gemm_kernels.h"
+#include "gemm_skinny.h"
 #include "gemm_plan.h"
 
 namespace quik {
@@ -64,37 +64,57 @@ int launch_fused_split(const FusedArgs &wide, const FusedArgs &tail, hipStream_t
   return check_launch();
 }
 
-// M <= 32: the weight-streaming kernel of gemm_decode.h.  8 waves per 32-column slab when there are few
-// slabs (so that enough loads are in flight chip-wide) and K gives every wave at least two 128-byte
-// chunks per row; otherwise 4 waves, which lets two workgroups share a CU.
-int decode_waves(int64_t N, int64_t kbytes) {
-  const int64_t slabs = (N + 31) / 32, chunks = (kbytes + kDecodeChunk - 1) / kDecodeChunk;
-  return (chunks >= 16 && slabs <= num_cus()) ? 8 : 4;
-}
-
-template <int MODE, bool BF16, bool FUSED, int WAVES, bool XLDS>
-int launch_decode_w(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) {
-  auto kern = gemm_decode_kernel<MODE, BF16, FUSED, WAVES, XLDS>;
-  const int smem = decode_smem<WAVES, FUSED, XLDS>() + (XLDS ? static_cast<int>(decode_x_lds_bytes(p.M, p.kbytes)) : 0);
-  // XLDS: the LDS size varies from call to call with the row count, and prepare() sets the attribute once per
-  // kernel and device: set it to the most any call may ask for
-  if (int rc = prepare(kern, XLDS ? kLdsBytes : smem)) return rc;
-  // persistent workgroups: as many as are resident at once (8 waves per CU at this register count; the LDS copy
-  // of the token rows leaves room for one workgroup)
-  // Every workgroup walks the same number of slabs (one more or less): with 896 slabs, 224 workgroups of 4 slabs
-  // finish when 256 workgroups of 3 or 4 do, and share the memory system among fewer.
-  const int64_t slabs = (p.N + 31) / 32, resident = int64_t(num_cus()) * (XLDS ? 1 : 8 / WAVES);
-  const int64_t per = (slabs + resident - 1) / resident, grid = (slabs + per - 1) / per;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(WAVES * 64), smem, st, p, C, ldc);
+// M <= 32: the weight-streaming kernel of gemm_skinny.h.  The columns go to the CUs in equal shares, in as few rounds as the
+// registers allow: seven blocks of 16 columns with one block of token rows, four with two.  (28672 columns in rounds of 56
+// instead of one of 112: int4 8192 -> 28672, 4 rows, 22.7 against 22.0 us; 20480 in two of 40, 7168 deep, 17.5 against 15.7.)
+template <class C, int MODE, bool BF16, bool FUSED>
+int launch_skinny_cfg(const FusedArgs &p, int bn, int32_t *C_, int ldc, hipStream_t st) {
+  auto kern = gemm_skinny_kernel<C, MODE, BF16, FUSED>;
+  if (int rc = prepare(kern, C::smem(16 * C::MT, FUSED))) return rc;
+  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((p.N + bn - 1) / bn)), dim3(C::kThreads), C::smem(p.M, FUSED), st, p, bn, C_, ldc);
   return check_launch();
 }
-
-// The token rows stay in LDS when they fit beside the reduction area and there is more than one slab per
-// workgroup to reuse them for (with fewer than 4 rows the L2 reads they replace cost less than the copy).
-template <int WAVES, bool FUSED>
-bool decode_x_fits(const FusedArgs &p) {
-  return p.M >= 4 && decode_smem<WAVES, FUSED, true>() + decode_x_lds_bytes(p.M, p.kbytes) <= kLdsBytes &&
-         (p.N + 31) / 32 > num_cus();
+// Register turns in flight: three of one block are as fast as two or faster (int4 11008 -> 4096, 4 rows, 5.5 against 5.8 us),
+// three of two blocks slower (int8 13824 -> 5120, 16 rows, 14.2 against 13.8), two of four blocks slower than one (int4 8192 ->
+// 28672, 32 rows, 29.2 against 26.4).
+template <int MT, int MODE, bool BF16, bool FUSED>
+int launch_skinny_rows(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) {
+  constexpr int64_t kMost = MT == 1 ? 112 : 64;
+  const int64_t cus = num_cus(), longest = p.kbytes > int64_t(p.F) * 2 ? p.kbytes : int64_t(p.F) * 2;
+  int64_t most = (int64_t(1) << 32) / longest / 4 * 4 - 4;  // (32-bit offsets inside a workgroup)
+  most = most < 4 ? 4 : most > kMost ? kMost : most;
+  const int64_t rounds = (p.N + most * cus - 1) / (most * cus), share = (p.N + rounds * cus - 1) / (rounds * cus);
+  const int bn = static_cast<int>((share + 3) / 4 * 4);  // (whole 8-byte pieces of the output rows)
+  if (bn <= 16) return launch_skinny_cfg<SkinnyCfg<1, MT, 3>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  if (bn <= 32) return launch_skinny_cfg<SkinnyCfg<2, MT, 2>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  if (bn <= 48) return launch_skinny_cfg<SkinnyCfg<3, MT, 2>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  if (bn <= 64) return launch_skinny_cfg<SkinnyCfg<4, MT, 1>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  if constexpr (MT == 1) {
+    if (bn <= 96) return launch_skinny_cfg<SkinnyCfg<6, MT, 1>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+    return launch_skinny_cfg<SkinnyCfg<7, MT, 1>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  }
+  return QUIK_ERR_SHAPE;  // (not reached: bn is at most kMost)
+}
+template <int MODE, bool BF16, bool FUSED>
+int launch_skinny(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) {
+  const int64_t longest = p.kbytes > int64_t(p.F) * 2 ? p.kbytes : int64_t(p.F) * 2;
+  if (p.M * longest > 0xffffffffll) {  // (32-bit offsets of the token rows: as many of them per launch as these reach)
+    const int some = static_cast<int>(0xffffffffll / longest);
+    for (int m = 0; m < p.M; m += some) {
+      FusedArgs q = p;
+      q.M = p.M - m < some ? p.M - m : some;
+      q.qx += int64_t(m) * p.kbytes;
+      if constexpr (FUSED) {
+        q.meta += int64_t(m) * p.meta_stride;
+        q.fp_x = p.F > 0 ? q.fp_x + int64_t(m) * p.F : nullptr;
+        q.out += int64_t(m) * p.ldo;
+      }
+      const int rc = launch_skinny<MODE, BF16, FUSED>(q, FUSED ? nullptr : C + int64_t(m) * ldc, ldc, st);
+      if (rc != QUIK_OK) return rc;
+    }
+    return QUIK_OK;
+  }
+  return p.M <= 16 ? launch_skinny_rows<1, MODE, BF16, FUSED>(p, C, ldc, st) : launch_skinny_rows<2, MODE, BF16, FUSED>(p, C, ldc, st);
 }
 
 // At most kGemvMaxRows token rows (fused form): one wave per output column, gemm_gemv.h.  Needs 16-byte aligned rows
@@ -139,9 +159,7 @@ int launch_decode(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) {
       if (rc != kChainNotHandled) return rc;
     }
   }
-  if (decode_x_fits<8, FUSED>(p)) return launch_decode_w<MODE, BF16, FUSED, 8, true>(p, C, ldc, st);
-  if (decode_waves(p.N, p.kbytes) == 8) return launch_decode_w<MODE, BF16, FUSED, 8, false>(p, C, ldc, st);
-  return launch_decode_w<MODE, BF16, FUSED, 4, false>(p, C, ldc, st);
+  return launch_skinny<MODE, BF16, FUSED>(p, C, ldc, st);
 }
 
 Plan make_plan(int64_t M, int64_t N, bool dma_ok) {

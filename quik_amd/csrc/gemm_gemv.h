@@ -1,9 +1,9 @@
 // MixedQLinear forward for very few token rows (single-stream decode; the host uses it for one and two): a
 // matrix-vector product per token row, bound by one pass over the weights.
 //
-// With so few token rows a 32-row MFMA block is mostly padding, and what the weight-streaming MFMA kernel
-// (gemm_decode.h) does around the MFMAs (LDS transpose of every weight chunk, partial sums of eight waves meeting
-// in LDS at every slab end, four barriers per slab) costs more than the products.  Here a WAVE owns whole output
+// With so few token rows a 16-row MFMA block is mostly padding, and what the weight-streaming MFMA kernel
+// (gemm_skinny.h) does around the MFMAs (LDS transpose of every weight chunk, partial sums of eight waves meeting
+// in LDS at the end) costs more than the products.  Here a WAVE owns whole output
 // columns: it streams a column's weight row with 16-byte loads (1 KB per instruction, whole lines), multiplies with
 // the packed dot-product instructions (v_dot8_i32_i4 / v_dot4_i32_i8: the codes of both operands are two's
 // complement nibbles / bytes in the same element order) against the token rows' codes, which every workgroup
