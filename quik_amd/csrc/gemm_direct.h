@@ -12,6 +12,14 @@
 // integer sums through LDS (exact, so in any order), each ending up with the blocks it owns, convert them, run the
 // outlier steps on them in the same order as the ring kernels and store: the same output bits.
 //
+// Beside the stream (what a CU takes in, 80 to 85 bytes per ns with 128x64 tiles at 4 bits, or 34 MB of weights in 5 us), a
+// launch of 128x64 tiles spends 12 us like this (128 x 5120 -> 13824; clock of the chip, per workgroup, before / now): arguments and
+// first addresses 1.2 / 1.0, stream and last steps 6.6 / 6.7, exchange 1.8 / 1.4, conversion and outlier steps 1.6 / 1.4, output 1.0.
+// The exchange reads a block's twelve pieces in one burst, not pair by pair; the outlier steps are requested in front of the last
+// integer steps and in place of what those and the exchange leave; a usual count of them has no loads between its products.
+// us per forward: 128 x 5120 -> 13824 17.6 -> 16.8, 300 x 4544 -> 4544 16.2 -> 15.3, 64 x 8192 -> 10240 15.4 -> 14.9, 40 x 4096 -> 4096
+// 10.2 -> 9.6, 523 x 7616 -> 1808 23.7 -> 22.6, int8 136 x 13824 -> 5120 31.4 -> 30.5, 64 x 28672 -> 8192 46.8 -> 46.9.
+//
 // Workgroups may share a tile's K further (SplitK, as in gemm_fp6.h): when the tiles are fewer than the CUs.
 //
 // Measured against the ring kernels (GEMM launch in a graph, us): W4A4 64 x 8192 x 7936 22.3 -> 13.7, 64 x 10240 x 7936
@@ -42,6 +50,7 @@ struct DirectCfg {
   static constexpr int OM = MI / 2, ON = NI == 1 ? 1 : NI / 2, OWN = OM * ON;
   static constexpr int kOutlierSets = OWN <= 2 ? 16 : 8;  // outlier steps in flight (16: all of them for 256 columns)
   static constexpr int kEarlySets = KIND != kDirect4 ? 0 : OWN <= 2 ? 8 : 0;  // .. requested in front of the last integer steps
+  static constexpr int kSetsInExchange = OWN <= 2 ? 12 : kOutlierSets;        // .. in front of the exchange (its reads take the registers of the others)
   // exchange: one owned block per round, in two areas by turns
   static constexpr int ROUND_BYTES = WAVES * (WAVES - 1) * 4096;
   static constexpr int RED_BYTES = (OWN > 1 ? 2 : 1) * ROUND_BYTES;
@@ -98,17 +107,19 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   for (int b = 0; b < MI / 2; ++b) base[b] = p.xbuf + block(m0 / 64 + b, x_blocks);
 #pragma unroll
   for (int b = 0; b < (NI + 1) / 2; ++b) base[MI / 2 + b] = p.wbuf + block(wrow / 64 + b, w_blocks);
-  auto load_step = [&](DirectFrag<D> &f, int64_t step) QUIK_INLINE {
+  // nothing: the registers only have to be written (the compiler's waits count loads), all lanes read the block's first bytes
+  auto load_step = [&](DirectFrag<D> &f, int64_t step, bool nothing) QUIK_INLINE {
     // (opaque per step: the lane offsets stay 32-bit offsets to a scalar base, instead of being folded into a 64-bit
     // vector address per fragment that every step then has to advance)
-    uint32_t ho = head_off, to = tail_off;
+    uint32_t ho = nothing ? 0 : head_off, to = nothing ? 0 : tail_off;
     asm volatile("" : "+v"(ho), "+v"(to));
+    const int64_t at = nothing ? 0 : step * UNIT;
     static_for<NF>([&](auto J) QUIK_INLINE {
       constexpr int j = J, jj = j < MI ? j : j - MI, b = j < MI ? j / 2 : MI / 2 + jj / 2;
       const int half = j < MI || NI > 1 ? jj & 1 : whalf;
-      const v4i head = *reinterpret_cast<const v4i *>(base[b] + step * UNIT + half * 1024 + ho);
+      const v4i head = *reinterpret_cast<const v4i *>(base[b] + at + half * 1024 + ho);
       if constexpr (D::KIND == kDirect6) {
-        const v2i tail = *reinterpret_cast<const v2i *>(base[b] + step * UNIT + half * 256 + to);
+        const v2i tail = *reinterpret_cast<const v2i *>(base[b] + at + half * 256 + to);
         f.f[j] = v8i{head.x, head.y, head.z, head.w, tail.x, tail.y, 0, 0};
       } else {
         f.f[j] = head;
@@ -121,9 +132,16 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     k0 = split * sk->per;
     k1 = k0 + sk->per < steps ? k0 + sk->per : steps;
   }
-  // this wave's steps: k0 + wave, k0 + wave + WAVES, ...
+  // This wave's steps: k0 + wave, k0 + wave + WAVES, ...  4 bits: in front of them stand as many empty ones (loaded from the
+  // block's first bytes, not multiplied) as make the loop's rounds whole, so that what is left behind the loop is always the same code, with loads and
+  // waits that do not depend on the remainder.  (With the remainder behind the loop, each of its up to 2 SETS steps with its
+  // loads under a condition, the compiler's waits there were waits for every load.)
   const int mine = k1 - k0 > wave ? (k1 - k0 - wave + WAVES - 1) / WAVES : 0;
-  auto at = [&](int i) { return static_cast<int64_t>(k0 + wave + i * WAVES); };
+  auto at = [&](int i) { return k0 + wave + i * WAVES; };
+  constexpr int kAhead = SETS + 1;                                         // steps in registers: one expanded, the others loaded
+  const int more = mine > kAhead ? (mine - kAhead + SETS - 1) / SETS : 0;  // rounds of the loop
+  const int empty = D::KIND == kDirect4 ? kAhead + more * SETS - mine : 0;
+  const int last_step = k1 > 0 ? k1 - 1 : 0;
   // per-row and per-column scalars of this thread: requested first, unconditionally (a load under a branch would make
   // the waits of everything around it waits for all loads), used after the main loop
   const int vi = threadIdx.x;
@@ -139,7 +157,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
 
   // 4 bits: the wave's next step to load, as the lane's offset to the (scalar) addresses of the blocks: one addition per
   // step.  The instructions of a step are what bounds it, not the bytes.
-  uint32_t pos = head_off + static_cast<uint32_t>(k0 + wave + SETS * WAVES) * UNIT;
+  uint32_t pos = head_off + static_cast<uint32_t>(at(kAhead - empty)) * UNIT;
   const uint8_t *const wbase = base[MI / 2] + (NI == 1 ? whalf * 1024 : 0);
   auto load_next = [&](auto &f) QUIK_INLINE {
     static_for<NF>([&](auto J) QUIK_INLINE {
@@ -150,8 +168,13 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   };
 
   DirectFrag<D> set[SETS];
-  const int last_step = k1 > 0 ? k1 - 1 : 0;
-  static_for<SETS>([&](auto S) QUIK_INLINE { load_step(set[S], at(S) < last_step ? at(S) : last_step); });
+  // step i of this wave, empty ones included (unconditional, as every load in front of the loop: the compiler's waits in it
+  // count on them)
+  auto load_one = [&](DirectFrag<D> &f, int i) QUIK_INLINE {
+    const int step = at(i - empty);
+    load_step(f, step < last_step ? step : last_step, i < empty);
+  };
+  static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
 
   v16f acc[MI][NI];  // fp32 sums (SIX) or int32 bit patterns
 #pragma unroll
@@ -173,16 +196,20 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     const int row = wrow + 32 * (oni + j);
     ow_base[j] = p.wbuf + block(row / 64, w_blocks) + ((row >> 5) & 1) * 1024;
   }
+  // (a step behind the last one: not used, the block's first bytes to all lanes)
   auto load_outlier = [&](auto S, int t) QUIK_INLINE {
-    const int64_t step = steps + t;
-    static_for<OM>([&](auto I) QUIK_INLINE { ox[S][I] = *reinterpret_cast<const v4i *>(ox_base[I] + step * UNIT + head_off); });
-    static_for<ON>([&](auto J) QUIK_INLINE { ow[S][J] = *reinterpret_cast<const v4i *>(ow_base[J] + step * UNIT + head_off); });
+    const bool real = t < fsteps;
+    const int64_t at_step = real ? int64_t(steps + t) * UNIT : 0;
+    const uint32_t off = real ? head_off : 0;
+    auto from = [&](const uint8_t *b) QUIK_INLINE { return *reinterpret_cast<const v4i *>(b + at_step + off); };
+    static_for<OM>([&](auto I) QUIK_INLINE { ox[S][I] = from(ox_base[I]); });
+    static_for<ON>([&](auto J) QUIK_INLINE { ow[S][J] = from(ow_base[J]); });
   };
-  // sets [LO, HI) of a round; without outlier columns: the last integer step, not used
+  // sets [LO, HI) of a round
   auto load_outliers = [&](auto LO, auto HI, int t0) QUIK_INLINE {
     static_for<HI - LO>([&](auto I) QUIK_INLINE {
       constexpr int S = LO + I;
-      load_outlier(std::integral_constant<int, S>{}, t0 + S < fsteps ? t0 + S : fsteps - 1);
+      load_outlier(std::integral_constant<int, S>{}, t0 + S);
     });
   };
   using std::integral_constant;
@@ -204,35 +231,52 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     };
     static_assert(SETS % 2 == 0, "operand sets alternate");
     expand(u[0], set[0]);
-    // (unconditional, as every load in front of the loop: the compiler's waits in it count on them)
-    load_step(set[0], at(SETS) < last_step ? at(SETS) : last_step);
-    pos += WAVES * UNIT;
-    int it = 0;  // step `it` is in u[it & 1], steps it + 1 .. it + SETS are in the sets (it + k in set (it + k) % SETS)
-    for (; it + 2 * SETS < mine; it += SETS) {
-      static_for<SETS>([&](auto S) QUIK_INLINE {
-        constexpr int next = (S + 1) % SETS;
-        __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1) * NF));  // (one wait for the set, not one per fragment)
-        __builtin_amdgcn_sched_barrier(0);
+    load_one(set[0], SETS);
+    // step i: expanded in u[i & 1]; steps i + 1 .. i + SETS are in the sets (i + k in set (i + k) % SETS)
+    auto interleave = [&]() QUIK_INLINE {
+      static_for<MI * NI>([&](auto) QUIK_INLINE {
+        __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x002, (8 * NF + MI * NI - 1) / (MI * NI), 0);
+      });
+    };
+    // steps of a round in front of the first real one are skipped; skip: how many
+    auto step = [&](auto S, int skip) QUIK_INLINE {
+      constexpr int next = (S + 1) % SETS;
+      if (S >= skip) {
         expand(u[(S + 1) & 1], set[next]);
         multiply(u[S & 1]);
-        load_next(set[next]);
-        static_for<MI * NI>([&](auto) QUIK_INLINE {
-          __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
-          __builtin_amdgcn_sched_group_barrier(0x002, (8 * NF + MI * NI - 1) / (MI * NI), 0);
-        });
+        interleave();
         static_for<NF>([&](auto J) QUIK_INLINE { pin(u[(S + 1) & 1][J]); });
+      } else if (S + 1 == skip) {
+        expand(u[(S + 1) & 1], set[next]);
+      }
+    };
+    auto round = [&](int skip) QUIK_INLINE {
+      static_for<SETS>([&](auto S) QUIK_INLINE {
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1) * NF));  // (one wait for the set, not one per fragment)
+        __builtin_amdgcn_sched_barrier(0);
+        step(S, skip);
+        load_next(set[(S + 1) % SETS]);
         __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
       });
-    }
+    };
+    if (more > 0) round(empty);
+    for (int i = 1; i < more; ++i) round(0);
+    // the last steps: outlier steps are requested in front of them and in place of the sets they leave
     if constexpr (!SPLITK) load_outliers(kNone, kEarly, 0);
-    static_for<2 * SETS>([&](auto S) QUIK_INLINE {
-      constexpr int next = (S + 1) % SETS;
-      if (it + S < mine) {
-        multiply(u[S & 1]);
-        if (it + S + 1 < mine) expand(u[(S + 1) & 1], set[next]);
-        if (it + S + 1 + SETS < mine) load_next(set[next]);
-      }
+    const int skip = more > 0 ? 0 : empty;
+    static_for<SETS>([&](auto S) QUIK_INLINE {
+      constexpr int late = D::kSetsInExchange - D::kEarlySets;
+      constexpr int sets = D::kEarlySets + late * S / SETS, sets_then = D::kEarlySets + late * (S + 1) / SETS;
+      constexpr int behind = SPLITK ? 0 : sets * (OM + ON);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1 - S) * NF + behind));
+      __builtin_amdgcn_sched_barrier(0);
+      step(S, skip);
+      if constexpr (!SPLITK)
+        load_outliers(integral_constant<int, sets>{}, integral_constant<int, sets_then>{}, 0);
+      __builtin_amdgcn_sched_barrier(0);
     });
+    if (mine > 0) multiply(u[SETS & 1]);
   } else {
     auto multiply = [&](const DirectFrag<D> &f) QUIK_INLINE {
       static_for<MI * NI>([&](auto I) QUIK_INLINE {
@@ -248,14 +292,13 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     for (; it + 2 * SETS <= mine; it += SETS) {
       static_for<SETS>([&](auto S) QUIK_INLINE {
         multiply(set[S]);
-        load_step(set[S], at(it + SETS + S));
+        load_step(set[S], at(it + SETS + S), false);
         __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
       });
     }
-    if constexpr (!SPLITK) load_outliers(kNone, kEarly, 0);
     static_for<SETS>([&](auto S) QUIK_INLINE {
       if (it + S < mine) multiply(set[S]);
-      if (it + SETS + S < mine) load_step(set[S], at(it + SETS + S));
+      if (it + SETS + S < mine) load_step(set[S], at(it + SETS + S), false);
     });
     static_for<SETS>([&](auto S) QUIK_INLINE {
       if (it + SETS + S < mine) multiply(set[S]);
@@ -277,7 +320,8 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     rowc[vi] = D::SIX ? static_cast<float>(8 * v_rs - 64 * p.K) : 0.0f;
   }  // (visible behind the exchange's barrier)
 
-  if constexpr (!SPLITK) load_outliers(kEarly, kAll, 0);
+  constexpr integral_constant<int, D::kSetsInExchange> kExchanged{};
+  if constexpr (!SPLITK && D::KIND != kDirect4) load_outliers(kNone, kExchanged, 0);
 
   // exchange, owned block by owned block: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the
   // three it finds
@@ -285,36 +329,47 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   auto add = [](float a, int b) QUIK_INLINE {
     return D::SIX ? a + __int_as_float(b) : __int_as_float(__float_as_int(a) + b);
   };
-  static_for<OWN>([&](auto B) QUIK_INLINE {
-    constexpr int bm = B % OM, bn = B / OM;
-    uint8_t *const area = smem + (B & 1) * D::ROUND_BYTES;
-    own[B] = v16f{};
-    static_for<WAVES>([&](auto O) QUIK_INLINE {
-      constexpr int o = O;
-      if constexpr (D::owns(o)) {
-        const v16f &b = acc[D::own_mi(o) + bm][D::own_ni(o) + bn];
-        if (o == wave) {
-          own[B] = b;
-        } else {
-          uint8_t *slot = area + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
+  constexpr int AREAS = OWN > 1 ? 2 : 1;
+  static_for<OWN / AREAS>([&](auto G) QUIK_INLINE {
+    if constexpr (G > 0) __syncthreads();  // every wave has read the areas
+    static_for<AREAS>([&](auto Q) QUIK_INLINE {
+      constexpr int B = G * AREAS + Q, bm = B % OM, bn = B / OM;
+      own[B] = v16f{};
+      static_for<WAVES>([&](auto O) QUIK_INLINE {
+        constexpr int o = O;
+        if constexpr (D::owns(o)) {
+          const v16f &b = acc[D::own_mi(o) + bm][D::own_ni(o) + bn];
+          if (o == wave) {
+            own[B] = b;
+          } else {
+            uint8_t *slot = smem + Q * D::ROUND_BYTES + (o * (WAVES - 1) + (wave < o ? wave : wave - 1)) * 4096 + lane * 16;
+#pragma unroll
+            for (int g = 0; g < 4; ++g)
+              *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
+          }
+        }
+      });
+    });
+    if constexpr (!SPLITK && G == OWN / AREAS - 1) load_outliers(kExchanged, kAll, 0);  // (in place of the sums just written)
+    __syncthreads();
+    if (D::owns(wave)) {
+      // (a block's reads in one burst: left alone the compiler waits for every pair)
+      static_for<AREAS>([&](auto Q) QUIK_INLINE {
+        v4i t[WAVES - 1][4];
+#pragma unroll
+        for (int s = 0; s < WAVES - 1; ++s)
 #pragma unroll
           for (int g = 0; g < 4; ++g)
-            *reinterpret_cast<float4 *>(slot + g * 1024) = make_float4(b[4 * g], b[4 * g + 1], b[4 * g + 2], b[4 * g + 3]);
-        }
-      }
-    });
-    __syncthreads();  // (an area is written again two rounds later: behind a barrier that its readers have passed)
-    if (D::owns(wave)) {
+            t[s][g] = *reinterpret_cast<const v4i *>(smem + Q * D::ROUND_BYTES + (wave * (WAVES - 1) + s) * 4096 + lane * 16 + g * 1024);
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-      for (int s = 0; s < WAVES - 1; ++s) {
-        const uint8_t *slot = area + (wave * (WAVES - 1) + s) * 4096 + lane * 16;
+        for (int s = 0; s < WAVES - 1; ++s)
 #pragma unroll
-        for (int g = 0; g < 4; ++g) {
-          const v4i t = *reinterpret_cast<const v4i *>(slot + g * 1024);
+          for (int g = 0; g < 4; ++g)
 #pragma unroll
-          for (int e = 0; e < 4; ++e) own[B][4 * g + e] = add(own[B][4 * g + e], t[e]);
-        }
-      }
+            for (int e = 0; e < 4; ++e) own[G * AREAS + Q][4 * g + e] = add(own[G * AREAS + Q][4 * g + e], t[s][g][e]);
+        __builtin_amdgcn_sched_barrier(0);
+      });
     }
   });
 
@@ -360,14 +415,24 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
 
   // conversion, outlier steps, storage type: the arithmetic of fused6_tile / fused8t_tile on the owned blocks
   if (D::owns(wave)) {
+    struct Columns {
+      float4 sc, wr, bs, cc;
+    };
+    Columns columns[ON][4];
+#pragma unroll
+    for (int j = 0; j < ON; ++j)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        const int c = (oni + j) * 32 + acc_col(g, lane);
+        columns[j][g] = {*reinterpret_cast<const float4 *>(scol + c), *reinterpret_cast<const float4 *>(wred + c),
+                         *reinterpret_cast<const float4 *>(bias + c), *reinterpret_cast<const float4 *>(colc + c)};
+      }
     static_for<OWN>([&](auto B) QUIK_INLINE {
       constexpr int bm = B % OM, bn = B / OM;
       const float rs = srow[32 * (omi + bm) + r], rz = zs[32 * (omi + bm) + r], rc = rowc[32 * (omi + bm) + r];
 #pragma unroll
       for (int g = 0; g < 4; ++g) {
-        const int c = (oni + bn) * 32 + acc_col(g, lane);
-        const float4 sc = *reinterpret_cast<const float4 *>(scol + c), wr = *reinterpret_cast<const float4 *>(wred + c),
-                     bs = *reinterpret_cast<const float4 *>(bias + c), cc = *reinterpret_cast<const float4 *>(colc + c);
+        const float4 sc = columns[bn][g].sc, wr = columns[bn][g].wr, bs = columns[bn][g].bs, cc = columns[bn][g].cc;
         const float scv[4] = {sc.x, sc.y, sc.z, sc.w}, wrv[4] = {wr.x, wr.y, wr.z, wr.w}, bsv[4] = {bs.x, bs.y, bs.z, bs.w},
                     ccv[4] = {cc.x, cc.y, cc.z, cc.w};
 #pragma unroll
@@ -379,14 +444,24 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         }
       }
     });
-    for (int t0 = 0; t0 < fsteps; t0 += OS) {
-      const bool more = t0 + OS < fsteps;
-      static_for<OS>([&](auto S) QUIK_INLINE {
-        if (t0 + S < fsteps)
-          static_for<OWN>([&](auto B) QUIK_INLINE { FragOps<BF16 ? kBF16 : kF16>::mma(ox[S][B % OM], ow[S][B / OM], own[B]); });
-        if (more) load_outlier(S, t0 + OS + S < fsteps ? t0 + OS + S : fsteps - 1);
+    auto outlier_step = [&](auto S) QUIK_INLINE {
+      static_for<OWN>([&](auto B) QUIK_INLINE { FragOps<BF16 ? kBF16 : kF16>::mma(ox[S][B % OM], ow[S][B / OM], own[B]); });
+    };
+    auto outlier_round = [&](int t0) QUIK_INLINE {
+      const bool again = t0 + OS < fsteps;
+      static_for<OS / 4>([&](auto G) QUIK_INLINE {
+        constexpr int S = 4 * G;
+        if (t0 + S < fsteps) {  // (an even number of steps: outlier columns are a multiple of 32)
+          outlier_step(integral_constant<int, S>{}), outlier_step(integral_constant<int, S + 1>{});
+          if (t0 + S + 2 < fsteps) outlier_step(integral_constant<int, S + 2>{}), outlier_step(integral_constant<int, S + 3>{});
+          int next = t0 + OS;
+          asm volatile("" : "+s"(next));  // (opaque: else the addresses of all steps advance together, in registers)
+          if (again) load_outliers(integral_constant<int, S>{}, integral_constant<int, S + 4>{}, next);
+        }
       });
-    }
+    };
+    if (fsteps > 0) outlier_round(0);  // (usually the only one, with waits of its own)
+    for (int t0 = OS; t0 < fsteps; t0 += OS) outlier_round(t0);
   }
   __syncthreads();  // every wave has read its slots: the area becomes the output tile
   if (D::owns(wave)) {
@@ -436,6 +511,8 @@ template <class D, bool BF16, class Args>
 __global__ __launch_bounds__(D::kThreads, D::OWN == 1 ? 2 : 1) void gemm_direct_kernel(Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
+  asm volatile("" : : "s"(p.xbuf), "s"(p.wbuf), "s"(p.M), "s"(p.N), "s"(p.K), "s"(p.F), "s"(p.n_first), "s"(p.N_total), "s"(p.meta), "s"(p.s_col),
+               "s"(p.w_red), "s"(p.bias));  // (all arguments in one trip, not those behind the branch in a second one; no instruction)
   if (!tile_of_block<D::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
   direct_tile<D, BF16, false>(p, tm, tn, smem, 0, 0, nullptr);
 }
