@@ -46,7 +46,8 @@ struct PyRef {  // owned reference
   ~PyRef() { Py_XDECREF(p); }
 };
 
-PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_finish, *s_workspaces, *s_split_k, *s_group_size;
+PyObject *s_buffers, *s_mid_event, *s_cuda_event, *s_cur, *s_outs, *s_fast, *s_fused, *s_workspaces, *s_split_k, *s_group_size;
+PyObject *s_shared[6];  // what SharedQuantizedInput.finish drops at the end of a round
 
 // A class keeps its version tag until one of its attributes (or of its bases') is set: methods and class-wide
 // switches are as they were when the plan was made.
@@ -285,6 +286,12 @@ PyObject *py_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
   return guarded([&] { return forward(args, n); });
 }
 
+// columns [at, at + n) of rows that are `stride` elements apart, as [lead0, lead1, n]; `at`: in elements from the storage's start
+at::Tensor columns(const at::Tensor &t, int64_t lead0, int64_t lead1, int64_t stride, int64_t at, int64_t n) {
+  const int64_t shape[3] = {lead0, lead1, n}, strides[3] = {lead1 * stride, stride, 1};
+  return t.as_strided(at::IntArrayRef(shape, 3), at::IntArrayRef(strides, 3), at);
+}
+
 // group_forward(group, index, module, x) -> member `index`'s columns [.., N_index] or None
 PyObject *group_forward(PyObject *const *args, Py_ssize_t n) {
   if (n != 4) return PyErr_Format(PyExc_TypeError, "group_forward takes 4 arguments");
@@ -318,16 +325,16 @@ PyObject *group_forward(PyObject *const *args, Py_ssize_t n) {
       PyObject *d = dict_of(mod);
       if (!d || !unchanged(d, m.bufs)) Py_RETURN_NONE;
     }
-    const int64_t shape[2] = {lead0 * lead1, (p->has_row ? p->row : p->tiled).out_features};
+    const int64_t total = (p->has_row ? p->row : p->tiled).out_features, shape[3] = {lead0, lead1, total};
     at::Tensor whole;
-    if (!layer_run(*p, g->fused.p, args[3], *x, at::IntArrayRef(shape, 2), whole)) return none_or_error();
+    if (!layer_run(*p, g->fused.p, args[3], *x, at::IntArrayRef(shape, 3), whole)) return none_or_error();
     PyRef outs;
     outs.p = PyDict_New();
     if (!outs.p) return nullptr;
     int64_t lo = 0;
-    for (const Group::Member &m : g->members) {
+    for (const Group::Member &m : g->members) {  // (in the shape the members are called for: nothing is left to do then)
       PyRef v;
-      v.p = THPVariable_Wrap(whole.narrow(1, lo, m.out));
+      v.p = THPVariable_Wrap(columns(whole, lead0, lead1, total, lo, m.out));
       if (!v.p || PyDict_SetItem(outs.p, m.key.p, v.p) < 0) return nullptr;
       lo += m.out;
     }
@@ -337,17 +344,28 @@ PyObject *group_forward(PyObject *const *args, Py_ssize_t n) {
   if (!outs || !PyDict_Check(outs)) return none_or_error();
   PyObject *mine = PyDict_GetItemWithError(outs, g->members[index].key.p);
   if (!mine || !THPVariable_CheckExact(mine)) return none_or_error();
-  at::Tensor view;
+  PyRef r;
   {
     const at::Tensor &t = THPVariable_Unpack(mine);
-    if (t.size(0) != lead0 * lead1) Py_RETURN_NONE;
-    const int64_t shape[3] = {lead0, lead1, t.size(1)}, strides[3] = {lead1 * t.stride(0), t.stride(0), 1};
-    view = t.as_strided(at::IntArrayRef(shape, 3), at::IntArrayRef(strides, 3));
+    const int64_t dim = t.dim();
+    if (dim == 3 && t.size(0) == lead0 && t.size(1) == lead1) {
+      r = PyRef(mine);
+    } else {  // (of a round begun by the Python function, or with other leading sizes)
+      if ((dim == 3 ? t.size(0) * t.size(1) : t.size(0)) != lead0 * lead1) Py_RETURN_NONE;
+      r.p = THPVariable_Wrap(columns(t, lead0, lead1, t.stride(dim - 2), t.storage_offset(), t.size(dim - 1)));
+      if (!r.p) return nullptr;
+    }
   }
-  PyRef r;
-  r.p = PyObject_CallMethodNoArgs(shared, s_finish);
-  if (!r.p) return nullptr;
-  return THPVariable_Wrap(std::move(view));
+  // SharedQuantizedInput.finish (the class's own: see the plan's methods)
+  PyRef next;
+  const bool last = at_elem + 1 == static_cast<long>(g->members.size());
+  next.p = PyLong_FromLong(last ? 0 : at_elem + 1);
+  if (!next.p) return nullptr;
+  if (last)
+    for (PyObject *name : s_shared)
+      if (PyDict_SetItem(sd, name, Py_None) < 0) return nullptr;
+  if (PyDict_SetItem(sd, s_cur, next.p) < 0) return nullptr;
+  return std::exchange(r.p, nullptr);
 }
 
 PyObject *py_group_forward(PyObject *, PyObject *const *args, Py_ssize_t n) {
@@ -584,7 +602,8 @@ PyMODINIT_FUNC PyInit__front() {
   s_outs = PyUnicode_InternFromString("_outs");
   s_fast = PyUnicode_InternFromString("_fast");
   s_fused = PyUnicode_InternFromString("_fused");
-  s_finish = PyUnicode_InternFromString("finish");
+  const char *shared[6] = {"qint_x", "qscale_x", "meta", "fp_x", "x6", "_outs"};
+  for (int i = 0; i < 6; ++i) s_shared[i] = PyUnicode_InternFromString(shared[i]);
   s_workspaces = PyUnicode_InternFromString("_splitk_workspaces");
   s_group_size = PyUnicode_InternFromString("group_size");
   s_split_k = PyUnicode_InternFromString("split_k");

@@ -233,7 +233,7 @@ class SharedQuantizedInput:
 
 # What a round or a forward calls on the way that the native front end goes past: a plan is made only where all of them are
 # the classes' own, so that an override (of a subclass, on the class, on one object) is called by every forward.
-_GROUP_METHODS = {name: SharedQuantizedInput.__dict__[name] for name in ("group_forward", "_fused_layer", "_members_state")}
+_GROUP_METHODS = {name: SharedQuantizedInput.__dict__[name] for name in ("group_forward", "_fused_layer", "_members_state", "finish")}
 
 
 def _own_methods(obj, methods):
