@@ -310,12 +310,13 @@ int64_t quik_layer_workspace_bytes(const quik_layer *layer, int64_t rows);
 int quik_layer_forward(const quik_layer *layer, const void *x, int64_t rows, void *workspace,
                        int64_t workspace_bytes, void *splitk_workspace, int64_t splitk_bytes, void *out,
                        void *mid_event, void *stream);
-/* Calls of one or two token rows (a column map that streams; symmetric activations: fp16) take ONE launch: the
- * weight-streaming kernel quantises the rows itself, with the arithmetic of quik_asym_quantize /
- * quik_sym_quantize_mapped, and the workspace
- * stays untouched; mid_event is then recorded behind that launch.  quik_layer_set_one_launch(0) switches this off
- * for the process (the two-launch form; same output bits), 1 switches it on again (the default).  No counterpart in
- * the reference. */
+/* Calls of one token row, and of two where it is the faster form (few or very many columns), take ONE launch (a column map
+ * that streams; symmetric activations: fp16): the matrix-vector kernel quantises the rows itself, with the arithmetic of
+ * quik_asym_quantize / quik_sym_quantize_mapped, and the workspace stays untouched; mid_event is then recorded behind that
+ * launch.  For the process, quik_layer_set_one_launch(0) switches this off (two launches, the second on the same
+ * matrix-vector kernel; same output bits), 1 takes it for every call of one or two rows, -1 is the default again.  (Two rows
+ * in two launches by default: mostly the weight-streaming kernel, whose fp32 outlier sums are added in another order.)  No
+ * counterpart in the reference. */
 void quik_layer_set_one_launch(int on);
 
 /* ---- the reference's simulated (fake-quant) activation path ---------------------------------------

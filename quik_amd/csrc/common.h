@@ -42,10 +42,16 @@ inline int colmap_require(const void *colmap, int64_t cols, int64_t num_int, int
 // gemm.hip: MixedQLinear forward for one or two token rows in ONE launch, the quantize inside the kernel
 // (w_red == NULL: symmetric activations with scale = max |x| / sym_divisor, fp16 only).  Returns kChainNotHandled
 // (below) for shapes it leaves to the two-launch path.
+bool gemv_one_launch_pays(int64_t rows, int64_t cols, int64_t N);
 int gemv_forward_one_launch(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
                             int64_t num_fp, int bits, const void *qw, const void *s_col, const void *w_red,
                             const void *fp_w, const void *bias, int64_t N, void *out, float sym_divisor,
                             hipStream_t st);
+
+// quik_mixed_linear_fwd; columns_per_wave: two rows on the matrix-vector kernel too
+int mixed_linear_rows(const void *qx, const void *qw, const void *meta, const void *s_col, const void *w_reduced, const void *fp_x,
+                      const void *fp_w, const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, int bits, void *out,
+                      bool columns_per_wave, void *stream);
 
 // The tile-ordered steps of a layer forward, for any number of integer columns that fills whole fragments (4 bits: a
 // multiple of kLayerK4, 8 bits: of kLayerK8).  The exported functions of the same steps (quik_asym_quantize_fp6, ...) ask

@@ -1,4 +1,4 @@
-// MixedQLinear forward for very few token rows (single-stream decode; the host uses it for one and two): a
+// MixedQLinear forward for very few token rows (single-stream decode; the host uses it for one, and for two where that pays): a
 // matrix-vector product per token row, bound by one pass over the weights.
 //
 // With so few token rows a 16-row MFMA block is mostly padding, and what the weight-streaming MFMA kernel
@@ -24,6 +24,7 @@
 // in place of min / max, scale = fp16(max |x| / divisor), codes rne(fp16(x / scale)), no zero-point term
 // (reference: experiments/qlinear.py:97-103, src/symmetric/symmetric.cu:6-61).
 #pragma once
+#include "colmap.h"
 #include "gemm_kernels.h"
 #include "quantize_math.h"
 
@@ -274,8 +275,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     const GemvQuantLds ql = gemv_quant_lds(quant.cols, quant.num_int);
     const uint32_t area_lds = lds_address(area);
     gemv_copy_in(quant.x, quant.cols * 2, area_lds + ql.raw, wave, lane);
-    gemv_copy_in(quant.grp, (quant.cols >> 3) * 4, area_lds + ql.grp, wave, lane);
-    gemv_copy_in(quant.unit, (quant.num_int >> 4) * 2, area_lds + ql.unit, wave, lane);
+    // (the tables in whole 16-byte pieces: the map's sections are padded to them, colmap.h)
+    gemv_copy_in(quant.grp, static_cast<int>(align16((quant.cols >> 3) * 4)), area_lds + ql.grp, wave, lane);
+    gemv_copy_in(quant.unit, static_cast<int>(align16((quant.num_int >> 4) * 2)), area_lds + ql.unit, wave, lane);
     const uint16_t *spare = reinterpret_cast<const uint16_t *>(quant.grp);  // (always there; the other tables may be empty)
     const bool has_g = tid < quant.ngather, has_f = tid < quant.num_fp;
     const int gunit = *(has_g ? quant.gather_unit + tid : spare);
