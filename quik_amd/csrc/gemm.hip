@@ -442,12 +442,16 @@ extern "C" int quik_int8_matmul(const int8_t *A, const int8_t *B, int32_t *C, in
 // One launch or two.  One row: one.  Two rows: every workgroup quantises both, one after the other in front of its products, and
 // multiplies them without matrix instructions; the other kernels' second launch is cheaper (us per forward, one after the other on a
 // stream, two launches / one: int4 4096 -> 4096 8.5 / 9.5, 4096 -> 11008 9.7 / 12.0, 11008 -> 4096 9.7 / 14.4, int8 13824 -> 5120
-// 18.0 / 20.6, 1024 -> 16384 8.4 / 10.5), but for few columns, at most one per wave of a workgroup on each CU, where the second
-// launch is all there is (2048 -> 2048 7.6 / 6.7, 1280 -> 1664 7.8 / 6.5, 4096 -> 1024 8.2 / 7.4, int8 2048 -> 2048 8.4 / 6.8; 2048 ->
-// 4096 7.7 / 8.4; rows too long: 8192 -> 512 8.6 / 8.8, 14272 -> 1024 9.7 / 11.0), and very many, whose stream hides the rest (8192 -> 22016 21.6 / 21.1, 8192 -> 28672 25.5 /
-// 24.9, int8 42.8 / 40.6; 14272 -> 9816 19.6 / 19.5).
+// 18.0 / 20.6, 1024 -> 16384 8.4 / 10.5), but for
+//   few columns, at most one per wave of a workgroup on each CU, or twice as many of short rows, where the second launch is all
+//   there is (2048 -> 2048 7.6 / 6.7, 1280 -> 1664 7.8 / 6.5, 4096 -> 1024 8.2 / 7.4, int8 2048 -> 2048 8.4 / 6.8; 1024 -> 4096
+//   8.1 / 8.2, 1472 -> 3200 with 448 outlier columns 9.4 / 7.8; rows too long: 2048 -> 4096 7.7 / 8.4, 8192 -> 512 8.6 / 8.8, 14272 ->
+//   1024 9.7 / 11.0);
+//   very many columns, whose stream hides the rest (8192 -> 22016 21.6 / 21.1, 8192 -> 28672 25.5 / 24.9, int8 42.8 / 40.6; but
+//   14272 -> 9816 19.6 / 19.5).
 bool quik::gemv_one_launch_pays(int64_t rows, int64_t cols, int64_t N) {
-  return rows <= 1 || (N <= kGemvWaves * num_cus() && cols <= 6144) || N > 80 * num_cus();
+  const int64_t each = kGemvWaves * num_cus();
+  return rows <= 1 || (N <= each && cols <= 6144) || (N <= 2 * each && cols <= 1536) || N > 10 * each;
 }
 
 // MixedQLinear forward for at most kGemvMaxRows token rows in ONE launch: the kernel of gemm_gemv.h quantises the

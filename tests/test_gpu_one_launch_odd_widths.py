@@ -39,8 +39,8 @@ def test_same_bits_as_two_launches(rows, N, n_in, F, bits, dtype, runs):
 
 
 # (the last: long int4 rows, two launches on the matrix-vector kernel)
-@pytest.mark.parametrize("N,K,one", [(2048, 512, True), (2056, 512, False), (20480, 512, False), (20488, 512, True), (2048, 6112, True),
-                                     (2048, 6144, False), (100, 13120, False)])
+@pytest.mark.parametrize("N,K,one", [(4096, 512, True), (4104, 512, False), (20480, 512, False), (20488, 512, True), (4096, 1504, True),
+                                     (2056, 1536, False), (2048, 1536, True), (2048, 6112, True), (2048, 6144, False), (100, 13120, False)])
 def test_two_rows_take_one_launch_with_few_or_very_many_columns(N, K, one):
     from quik_amd import _lib as L
     from oracle import quik_oracle as qo
