@@ -313,10 +313,8 @@ int quik_layer_forward(const quik_layer *layer, const void *x, int64_t rows, voi
 /* Calls of one token row, and of two where it is the faster form (few or very many columns), take ONE launch (a column map
  * that streams; symmetric activations: fp16): the matrix-vector kernel quantises the rows itself, with the arithmetic of
  * quik_asym_quantize / quik_sym_quantize_mapped, and the workspace stays untouched; mid_event is then recorded behind that
- * launch.  For the process, quik_layer_set_one_launch(0) switches this off (two launches, the second on the same
- * matrix-vector kernel; same output bits), 1 takes it for every call of one or two rows, -1 is the default again.  (Two rows
- * in two launches by default: mostly the weight-streaming kernel, whose fp32 outlier sums are added in another order.)  No
- * counterpart in the reference. */
+ * launch.  For the process, quik_layer_set_one_launch(0) switches this off (two launches), 1 takes it for every call of one or
+ * two rows, -1 is the default again; same output bits.  No counterpart in the reference. */
 void quik_layer_set_one_launch(int on);
 
 /* ---- the reference's simulated (fake-quant) activation path ---------------------------------------

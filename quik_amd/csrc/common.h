@@ -48,11 +48,6 @@ int gemv_forward_one_launch(const void *x, int dtype, int64_t rows, int64_t cols
                             const void *fp_w, const void *bias, int64_t N, void *out, float sym_divisor,
                             hipStream_t st);
 
-// quik_mixed_linear_fwd; columns_per_wave: two rows on the matrix-vector kernel too
-int mixed_linear_rows(const void *qx, const void *qw, const void *meta, const void *s_col, const void *w_reduced, const void *fp_x,
-                      const void *fp_w, const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, int bits, void *out,
-                      bool columns_per_wave, void *stream);
-
 // The tile-ordered steps of a layer forward, for any number of integer columns that fills whole fragments (4 bits: a
 // multiple of kLayerK4, 8 bits: of kLayerK8).  The exported functions of the same steps (quik_asym_quantize_fp6, ...) ask
 // for whole pairs of k-steps, 128 / 64 columns, and pass that as `k_multiple`.

@@ -152,13 +152,12 @@ int launch_gemv(const FusedArgs &p, const GemvQuant &q, hipStream_t st) {
 }
 
 template <int MODE, bool BF16, bool FUSED>
-int launch_decode(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st, bool columns_per_wave = false) {
+int launch_decode(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) {
   if constexpr (FUSED) {
     // One row.  Two are faster on the kernel below, 4096 -> 11008 int4 11.4 -> 9.7 us per forward, 2176 -> 15032 int8 13.2 -> 10.9,
     // 13824 -> 5120 int8 19.4 -> 18.0, unless the rows are long int4 ones: 11008 -> 4096 10.6 -> 9.7, 13824 -> 5120 13.2 -> 13.4,
-    // 14272 -> 9816 18.6 -> 19.6.  columns_per_wave: a caller that compares with the one-launch form, whose outlier sums are
-    // taken in this kernel's order.
-    const bool two_here = columns_per_wave || (MODE == kInt4 && p.kbytes > 6400);
+    // 14272 -> 9816 18.6 -> 19.6.  (The same bits on either.)
+    const bool two_here = MODE == kInt4 && p.kbytes > 6400;
     if ((p.M <= 1 || two_here) && gemv_ok(p)) {
       const int rc = launch_gemv<MODE, BF16>(p, GemvQuant{}, st);
       if (rc != kChainNotHandled) return rc;
@@ -373,10 +372,10 @@ int run_chain(const I32Args &a, const ChainArgs &e, bool two_launches, hipStream
 }
 
 template <int MODE, bool BF16>
-int run_fused(const FusedArgs &p, bool columns_per_wave, hipStream_t st) {
+int run_fused(const FusedArgs &p, hipStream_t st) {
   const Plan plan = make_plan(p.M, p.N, p.kbytes % 64 == 0 && (p.F * 2) % 64 == 0);
   switch (plan.kind) {
-    case Plan::kSmall: return launch_decode<MODE, BF16, true>(p, nullptr, 0, st, columns_per_wave);
+    case Plan::kSmall: return launch_decode<MODE, BF16, true>(p, nullptr, 0, st);
     case Plan::kMid: return launch_fused<CfgM, MODE, BF16>(p, st);
     case Plan::kNarrow: return launch_fused<CfgN, MODE, BF16>(p, st);
     case Plan::kMidPlain: return launch_fused<CfgMp, MODE, BF16>(p, st);
@@ -444,8 +443,8 @@ extern "C" int quik_int8_matmul(const int8_t *A, const int8_t *B, int32_t *C, in
 // stream, two launches / one: int4 4096 -> 4096 8.5 / 9.5, 4096 -> 11008 9.7 / 12.0, 11008 -> 4096 9.7 / 14.4, int8 13824 -> 5120
 // 18.0 / 20.6, 1024 -> 16384 8.4 / 10.5), but for
 //   few columns, at most one per wave of a workgroup on each CU, or twice as many of short rows, where the second launch is all
-//   there is (2048 -> 2048 7.6 / 6.7, 1280 -> 1664 7.8 / 6.5, 4096 -> 1024 8.2 / 7.4, int8 2048 -> 2048 8.4 / 6.8; 1024 -> 4096
-//   8.1 / 8.2, 1472 -> 3200 with 448 outlier columns 9.4 / 7.8; rows too long: 2048 -> 4096 7.7 / 8.4, 8192 -> 512 8.6 / 8.8, 14272 ->
+//   there is (2048 -> 2048 7.6 / 6.9, 1280 -> 1664 7.8 / 6.6, 4096 -> 1024 8.2 / 7.5, int8 2048 -> 2048 8.4 / 6.8; 1024 -> 4096
+//   8.1 / 8.2, 1472 -> 3200 with 448 outlier columns 9.4 / 8.2; rows too long: 2048 -> 4096 7.7 / 8.4, 8192 -> 512 8.6 / 8.8, 14272 ->
 //   1024 9.7 / 11.0);
 //   very many columns, whose stream hides the rest (8192 -> 22016 21.6 / 21.1, 8192 -> 28672 25.5 / 24.9, int8 42.8 / 40.6; but
 //   14272 -> 9816 19.6 / 19.5).
@@ -505,9 +504,10 @@ int quik::gemv_forward_one_launch(const void *x, int dtype, int64_t rows, int64_
   return dtype == QUIK_F16 ? launch_gemv<kInt8, false, kGemvAsym>(p, q, st) : launch_gemv<kInt8, true, kGemvAsym>(p, q, st);
 }
 
-int quik::mixed_linear_rows(const void *qx, const void *qw, const void *meta, const void *s_col, const void *w_reduced,
-                            const void *fp_x, const void *fp_w, const void *bias, int dtype, int64_t M, int64_t N, int64_t K,
-                            int64_t F, int bits, void *out, bool columns_per_wave, void *stream) {
+extern "C" int quik_mixed_linear_fwd(const void *qx, const void *qw, const void *meta, const void *s_col,
+                                     const void *w_reduced, const void *fp_x, const void *fp_w, const void *bias,
+                                     int dtype, int64_t M, int64_t N, int64_t K, int64_t F, int bits, void *out,
+                                     void *stream) {
   if (bits != 4 && bits != 8) return QUIK_ERR_BITS;
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (F < 0) return QUIK_ERR_SHAPE;
@@ -537,14 +537,6 @@ int quik::mixed_linear_rows(const void *qx, const void *qw, const void *meta, co
   p.shift = bits == 4 ? 8.0f : 128.0f;
   hipStream_t st = as_stream(stream);
   if (bits == 4)
-    return dtype == QUIK_F16 ? run_fused<kInt4, false>(p, columns_per_wave, st) : run_fused<kInt4, true>(p, columns_per_wave, st);
-  return dtype == QUIK_F16 ? run_fused<kInt8, false>(p, columns_per_wave, st) : run_fused<kInt8, true>(p, columns_per_wave, st);
+    return dtype == QUIK_F16 ? run_fused<kInt4, false>(p, st) : run_fused<kInt4, true>(p, st);
+  return dtype == QUIK_F16 ? run_fused<kInt8, false>(p, st) : run_fused<kInt8, true>(p, st);
 }
-
-extern "C" int quik_mixed_linear_fwd(const void *qx, const void *qw, const void *meta, const void *s_col,
-                                     const void *w_reduced, const void *fp_x, const void *fp_w, const void *bias,
-                                     int dtype, int64_t M, int64_t N, int64_t K, int64_t F, int bits, void *out,
-                                     void *stream) {
-  return mixed_linear_rows(qx, qw, meta, s_col, w_reduced, fp_x, fp_w, bias, dtype, M, N, K, F, bits, out, false, stream);
-}
-

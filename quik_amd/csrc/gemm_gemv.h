@@ -11,8 +11,15 @@
 // copy of the token rows, no cross-wave sums.  The outlier columns (fp16 / bf16 weights and values) travel through
 // the same stream of loads as further 16-byte pieces of the column, kGemvPieces pieces ahead, across column
 // boundaries; a column's three epilogue scalars wait in a small LDS table that the workgroup fills at the start.
-// Integer sums are exact; the fp32 outlier sum is taken in lane order, then over the wave.  Epilogue as in the other
-// fused kernels: (f32(acc) (s_row s_col) + outliers) + (zs w_red + bias).
+// Integer sums are exact; the fp32 outlier sum of one row is taken in lane order, then over the wave.  Epilogue as in the
+// other fused kernels: (f32(acc) (s_row s_col) + outliers) + (zs w_red + bias).
+//
+// Two rows also go to gemm_skinny.h, by the number of columns, and a column has to come out the same on either way (a group
+// of layers is one call of their columns together, and each of them promises the bits of the layer alone).  So the outlier
+// sums of two rows are taken on the same instruction in the same order: 32 columns per step, step t added to partial sum
+// t % 8, the eight partial sums added in order.  One 16x16x32 product has them all: its rows are the steps of the column's
+// weights, its columns (token row, step), and partial sum i of row m is element [i][8 m + i].  us per forward, the sums in lane
+// order as for one row / now: 2 x 2048 -> 2048 6.7 / 6.8, 2 x 1472 -> 3200 with 448 outlier columns 7.9 / 8.2, 2 x 8192 -> 28672 25.0 / 25.1.
 //
 // QUANT: the kernel also quantises the token rows itself (one launch per forward).  Every workgroup does it for all
 // of the (at most kGemvMaxRows) rows, redundantly: a row is a few KB out of L2, against a launch and a trip through
@@ -211,6 +218,9 @@ __device__ __forceinline__ float wave_total(float v) {
   return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 63));
 }
 
+// lanes 8 .. 15 of every 16 in place of lanes 0 .. 7 and the other way round
+__device__ __forceinline__ int swap_eights(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x128 /* row_ror:8 */, 0xF, 0xF, false); }
+
 // QUANT: kGemvNoQuant (the token rows' codes come from a quantize launch), kGemvAsym / kGemvSym (quantised here)
 constexpr int kGemvNoQuant = 0, kGemvAsym = 1, kGemvSym = 2;
 template <int MODE, bool BF16, int MT, int QUANT = kGemvNoQuant>
@@ -243,6 +253,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
   const uint8_t *fw = fbytes > 0 ? reinterpret_cast<const uint8_t *>(p.fp_w) : p.qw;
   const int frow = fbytes > 0 ? fbytes : kbytes;
   int ld_n = n_first, ld_p = 0;  // next item to load
+  constexpr bool kByMatrix = MT == 2;  // outlier sums on the matrix instruction: lane l has the 16 bytes l / 16 of step l % 16
+  const int outlier_lane = (lane & 15) * 64 + (lane >> 4) * 16;
   // Every item is ONE unconditional 16-byte load from a wave-uniform base plus a lane offset (with loads under a
   // branch the number in flight is unknown at compile time and every wait becomes a wait for all of them).
   auto issue = [&](v4i &b) __attribute__((always_inline)) {
@@ -251,6 +263,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     const uint8_t *base = is_int ? p.qw + int64_t(n) * kbytes : fw + int64_t(n) * frow;      // wave-uniform
     const int q = is_int ? ld_p : ld_p - ipieces, row_bytes = is_int ? kbytes : frow;
     int off = (q << 10) + lane * 16;
+    if constexpr (kByMatrix) off = (q << 10) + (is_int ? lane * 16 : outlier_lane);
     off = off < row_bytes ? off : row_bytes - 16;  // past the row's end: a repeated piece, masked where it is used
     b = *reinterpret_cast<const v4i *>(base + off);
     if (++ld_p == pieces) {
@@ -350,6 +363,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
   int n = n_first, piece = 0;  // the item being consumed
   int32_t acc[MT];
   float accf[MT];
+  v4f accd = {};  // kByMatrix
 #pragma unroll
   for (int m = 0; m < MT; ++m) acc[m] = 0, accf[m] = 0.0f;
   int it = 0;  // how many columns this wave has finished
@@ -373,6 +387,20 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
           acc[m] = __builtin_amdgcn_sdot4(x.w, b.w, acc[m], false);
         }
       }
+    } else if constexpr (kByMatrix) {
+      // (both operands are masked behind the last outlier column: an infinity may stand against a repeated piece)
+      const int first = (piece - ipieces) << 10;
+      const int keep = first + outlier_lane < fbytes ? -1 : 0;
+      v4i w = v4i{b_.x & keep, b_.y & keep, b_.z & keep, b_.w & keep};
+      static_for<2>([&](auto H) __attribute__((always_inline)) {  // steps 0 .. 7 of the piece, 8 .. 15
+        if (H == 0 || first + 512 < fbytes) {
+          const int off = first + H * 512 + (lane & 7) * 64 + (lane >> 4) * 16, there = off < fbytes ? -1 : 0;
+          const v4i r = *reinterpret_cast<const v4i *>(fs + ((lane >> 3) & 1) * fstride + (there ? off : 0));
+          const v4i x = v4i{r.x & there, r.y & there, r.z & there, r.w & there};
+          if constexpr (H == 1) w = v4i{swap_eights(w.x), swap_eights(w.y), swap_eights(w.z), swap_eights(w.w)};
+          mma16_outlier<BF16>(x, w, accd);
+        }
+      });
     } else {
       const int off = ((piece - ipieces) << 10) + lane * 16;
       const bool live = off < fbytes;  // (lanes past the outlier columns hold a repeated piece)
@@ -400,15 +428,24 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
       const float wr = to_f32<BF16>(static_cast<uint16_t>(e.x >> 16)), bs = to_f32<BF16>(static_cast<uint16_t>(e.y));
       int32_t ti = 0;
       float tf = 0.0f;
+      // kByMatrix: partial sum i of token row m is element i % 4 of lane 16 (i / 4) + 8 m + i
+      const int mine = __builtin_bit_cast(int, lane & 2 ? (lane & 1 ? accd[3] : accd[2]) : (lane & 1 ? accd[1] : accd[0]));
 #pragma unroll
       for (int m = 0; m < MT; ++m) {
         const int32_t si = wave_total(acc[m]);
-        const float sf = wave_total(accf[m]);
+        float sf = 0.0f;
+        if constexpr (kByMatrix) {
+#pragma unroll
+          for (int i = 0; i < 8; ++i) sf += __builtin_bit_cast(float, __builtin_amdgcn_readlane(mine, 16 * (i / 4) + 8 * m + i));
+        } else {
+          sf = wave_total(accf[m]);
+        }
         ti = lane == m ? si : ti;
         tf = lane == m ? sf : tf;
         acc[m] = 0;
         accf[m] = 0.0f;
       }
+      accd = v4f{};
       if (lane < p.M) {
         const float val = (static_cast<float>(ti) * (srow * sc) + tf) + (zs * wr + bs);
         p.out[int64_t(lane) * p.ldo + n] = from_f32<BF16>(val);

@@ -32,9 +32,20 @@ namespace quik {
 
 typedef int v4i __attribute__((ext_vector_type(4)));
 typedef int v16i __attribute__((ext_vector_type(16)));
+typedef float v4f __attribute__((ext_vector_type(4)));
 typedef float v16f __attribute__((ext_vector_type(16)));
 typedef _Float16 v8h __attribute__((ext_vector_type(8)));
 typedef __bf16 v8bf __attribute__((ext_vector_type(8)));
+
+// acc += w x of 32 outlier columns: 16 columns of the output by 16 token rows (decode kernels)
+template <bool BF16>
+__device__ __forceinline__ void mma16_outlier(const v4i &x, const v4i &w, v4f &acc) {
+  if constexpr (BF16) {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w), __builtin_bit_cast(v8bf, x), acc, 0, 0, 0);
+  } else {
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), acc, 0, 0, 0);
+  }
+}
 
 enum Mode { kInt4 = 0, kInt8 = 1, kF16 = 2, kBF16 = 3 };
 

@@ -23,8 +23,6 @@
 
 namespace quik {
 
-typedef float v4f __attribute__((ext_vector_type(4)));
-
 constexpr int kSkinnyWaves = 8;
 template <int NT_, int MT_, int SETS_>
 struct SkinnyCfg {
@@ -38,15 +36,6 @@ struct SkinnyCfg {
     return stream > sums ? stream : sums;
   }
 };
-
-template <bool BF16>
-__device__ __forceinline__ void mma16_outlier(const v4i &x, const v4i &w, v4f &acc) {
-  if constexpr (BF16) {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(v8bf, w), __builtin_bit_cast(v8bf, x), acc, 0, 0, 0);
-  } else {
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(v8h, w), __builtin_bit_cast(v8h, x), acc, 0, 0, 0);
-  }
-}
 
 // FUSED: p.out receives the MixedQLinear output.  !FUSED: Cm receives the int32 product.
 // bn * K bytes, bn * outlier bytes and the same of the token rows fit 32 bits.

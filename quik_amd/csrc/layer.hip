@@ -146,6 +146,6 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
                                                         rows, l.out_features, l.num_int, l.num_fp, out,
                                                         splitk_workspace, splitk_bytes, stream, kLayerK8);
   }
-  return mixed_linear_rows(q, l.int_weight, meta, l.weights_scales, w_red, fp_x, l.fp_weight, l.bias, l.dtype, rows,
-                           l.out_features, l.num_int, l.num_fp, l.bits, out, one_launch == 0, stream);
+  return quik_mixed_linear_fwd(q, l.int_weight, meta, l.weights_scales, w_red, fp_x, l.fp_weight, l.bias, l.dtype, rows,
+                               l.out_features, l.num_int, l.num_fp, l.bits, out, stream);
 }
