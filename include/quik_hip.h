@@ -197,6 +197,12 @@ int quik_tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F);
 int quik_mixed_linear_fwd_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
                                 const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
                                 int64_t K, int64_t F, void *out, void *stream);
+/* the same with a K split where it pays (few columns, long rows; x_bits 4): quik_tile4_splitk_bytes(..) bytes of a workspace as
+ * the _ws entry points below take it; 0: the shape is not split, no workspace is read */
+int64_t quik_tile4_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t F);
+int quik_mixed_linear_fwd_tile4_ws(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
+                                   const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
+                                   int64_t K, int64_t F, void *out, void *workspace, int64_t workspace_bytes, void *stream);
 /* `tiled` of quik_sym_quantize_mapped (bits = 4): the 4-bit operand buffer; `tiled_format` of quik_layer: 4-bit weights */
 #define QUIK_TILED_4 0x344C5451
 
@@ -287,7 +293,8 @@ int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *m
  *                   with ONE copy of its weights (0.75 byte per int4 weight, 1 per int8 weight) at the price
  *                   of slower calls of at most 32 rows (the weight-streaming kernel reads the packed nibbles)
  * workspace: quik_layer_workspace_bytes(layer, rows) bytes, 256-byte aligned, holds the quantized activation
- * between the two launches; splitk_workspace as for the _ws entry points (may be NULL).
+ * between the two launches; splitk_workspace as for the _ws entry points (may be NULL; tiled_format QUIK_TILED_4:
+ * quik_tile4_splitk_bytes(rows, out_features, num_int, num_fp) bytes).
  * mid_event: NULL, or a hipEvent_t that is recorded on the stream between the quantize launch and the
  * GEMM launch (profiling hook: lets a caller time the two kernels of a one-call forward).
  * x [rows, in_features] dtype, out [rows, out_features] dtype. */

@@ -68,7 +68,8 @@ int mixed_linear_fp6(const void *x6, const void *w6, const void *meta, const voi
 // 4-bit weights: the format (4 or 6 bits) in which the GEMM of this shape takes its activation, and the GEMM (either format)
 int tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F);
 int mixed_linear_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col, const void *w_reduced,
-                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out, void *stream);
+                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out, void *workspace,
+                       int64_t workspace_bytes, void *stream);
 int mixed_linear_tile8(const void *x8, const void *w8, const void *meta, const void *s_col, const void *w_reduced,
                        const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out,
                        void *workspace, int64_t workspace_bytes, void *stream, int64_t k_multiple);

@@ -192,7 +192,9 @@ bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &
   void *sk = nullptr;
   int64_t sk_bytes = 0;
   PyRef sk_tensor;
-  if (tiled && quik_splitk_workspace_bytes(rows, l.out_features, l.num_int, l.bits) > 0) {
+  const bool four_bit = l.tiled_format == QUIK_TILED_4;  // (whose GEMMs split K by a plan of their own)
+  if (tiled && (four_bit ? quik_tile4_splitk_bytes(rows, l.out_features, l.num_int, l.num_fp)
+                         : quik_splitk_workspace_bytes(rows, l.out_features, l.num_int, l.bits)) > 0) {
     // the stream's workspace as matmul._splitk_workspace keeps it, or that function where there is none yet
     PyObject *globals = PyFunction_GetGlobals(p.splitk_fn.p), *known = PyDict_GetItemWithError(globals, s_workspaces);
     hipStreamCaptureStatus capture = hipStreamCaptureStatusNone;
@@ -208,9 +210,9 @@ bool layer_run(const Plan &p, PyObject *module, PyObject *xo, const at::Tensor &
       }
     }
     if (!sk) {
-      PyObject *r = PyObject_CallFunction(p.splitk_fn.p, "OLLLi", p.device_obj.p, static_cast<long long>(rows),
+      PyObject *r = PyObject_CallFunction(p.splitk_fn.p, "OLLLiL", p.device_obj.p, static_cast<long long>(rows),
                                           static_cast<long long>(l.out_features), static_cast<long long>(l.num_int),
-                                          static_cast<int>(l.bits));
+                                          static_cast<int>(l.bits), static_cast<long long>(four_bit ? l.num_fp : -1));
       if (!r) return false;
       sk_tensor.p = r;
       PyObject *t = PyTuple_GET_ITEM(r, 0);

@@ -146,5 +146,25 @@ int launch_rest(Kernel kern, int smem, const Args &p, int64_t n_wide, hipStream_
   return check_launch();
 }
 
+// Zero-fill of a few words by a kernel: the arrival counters of the K split are cleared with it, not with
+// hipMemsetAsync, because the caller's stream may be under capture and a memset node in a captured graph is not
+// reliable on replays.
+__global__ __launch_bounds__(256) void clear_words_kernel(uint32_t *p, int words) {
+  for (int i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) p[i] = 0u;
+}
+constexpr int64_t kSplitCounterBytes = 4096;  // arrival counters of a K split, one per tile, in front of the partial sums
+// The arrival counters are zero between launches because every launch that completes returns them there.  After a
+// launch that was refused nothing ran, but the caller may not know how far an earlier one got: clear the counters
+// behind a failed launch so that the next one on this workspace starts clean.
+int splitk_launch_status(void *workspace, hipStream_t st) {
+  const int rc = check_launch();
+  if (rc != QUIK_OK) {
+    hipLaunchKernelGGL(clear_words_kernel, dim3(static_cast<unsigned>(kSplitCounterBytes / 4 / 256)), dim3(256), 0, st,
+                       static_cast<uint32_t *>(workspace), static_cast<int>(kSplitCounterBytes / 4));
+    (void)hipGetLastError();  // the status reported is that of the launch that failed
+  }
+  return rc;
+}
+
 }  // namespace
 }  // namespace quik

@@ -58,6 +58,43 @@ Tiles4 plan_tile4(int64_t M, int64_t N, int64_t K, int64_t F) {
   return best;
 }
 
+// K split over `splits` workgroups per 64x32 tile (SplitK): few tiles of a long K leave most CUs idle, and with them what the
+// chip can have open towards memory.  The exchange through memory costs 1.5 us and 0.3 per workgroup, against 24.6 ns for each step
+// that a workgroup has less (same fit), so it is taken from some 150 k-steps on.  us per forward, warm / cold weights, without and
+// with the split: 64 x 14336 -> 512 15.0 / 17.8, 13.4 / 14.8 (4); 128 x 14336 -> 1024 15.5 / 20.2, 15.0 / 16.7 (4); 64 x 12288 -> 1024
+// 14.0 / 18.4, 13.4 / 15.1 (3); 40 x 14336 -> 4096 15.3 / 20.9, 15.0 / 19.1 (2).  At 8192 columns it costs warm what it gives cold (64 ->
+// 1024 12.0 / 14.3, 12.3 / 13.6); eight workgroups per tile, or 64x64 tiles, were nowhere the faster form.
+constexpr int kMostSplits4 = 4;
+int plan_splits4(int64_t M, int64_t N, int64_t K, int64_t F) {
+  const int64_t steps = tile4_layout(N, K, F).steps, tiles = (M + 63) / 64 * ((N + 31) / 32);
+  if (2 * tiles > num_cus() || tiles * 4 > kSplitCounterBytes || plan_tile4(M, N, K, F) != Tiles4::k64x32) return 1;
+  int best = 1;
+  int64_t least = steps * 24600;
+  for (int splits = 2; splits <= kMostSplits4 && splits * tiles <= num_cus(); ++splits) {
+    const int64_t per = (steps + splits - 1) / splits, c = 1500000 + 300000 * splits + per * 24600;
+    if ((splits - 1) * per < steps && c < least) least = c, best = splits;
+  }
+  return best;
+}
+int64_t split_bytes4(int64_t M, int64_t N, int64_t K, int64_t F) {
+  const int splits = plan_splits4(M, N, K, F);
+  return splits == 1 ? 0 : kSplitCounterBytes + (M + 63) / 64 * ((N + 31) / 32) * splits * Direct64x32::PARTIAL_BYTES;
+}
+
+template <bool BF16>
+int launch_split4(const Fused8Args &p, int splits, void *workspace, hipStream_t st) {
+  using D = Direct64x32;
+  int tiles_m, tiles_n;
+  const int grid = grid_of<D>(p.M, p.N, tiles_m, tiles_n);
+  const int steps = static_cast<int>(tile4_layout(p.M, p.K, p.F).steps);
+  SplitK sk{splits, (steps + splits - 1) / splits, grid, static_cast<uint32_t *>(workspace),
+            reinterpret_cast<int32_t *>(static_cast<uint8_t *>(workspace) + kSplitCounterBytes)};
+  auto kern = gemm_direct_splitk_kernel<D, BF16, Fused8Args>;
+  if (int rc = prepare(kern, D::SMEM)) return rc;
+  hipLaunchKernelGGL(kern, dim3(grid * splits), dim3(D::kThreads), D::SMEM, st, p, tiles_m, tiles_n, sk);
+  return splitk_launch_status(workspace, st);
+}
+
 template <class D, bool BF16>
 int launch_direct4(const Fused8Args &p, hipStream_t st) {
   int tiles_m, tiles_n;
@@ -70,7 +107,11 @@ int launch_direct4(const Fused8Args &p, hipStream_t st) {
 
 // the activation in 4 bits; any size (where the plan is the ring, the widest tiles: a caller that did not ask)
 template <bool BF16>
-int run_direct4(const Fused8Args &p, hipStream_t st) {
+int run_direct4(const Fused8Args &p, void *workspace, int64_t workspace_bytes, hipStream_t st) {
+  if (workspace) {
+    const int splits = plan_splits4(p.M, p.N, p.K, p.F);
+    if (splits > 1 && workspace_bytes >= split_bytes4(p.M, p.N, p.K, p.F)) return launch_split4<BF16>(p, splits, workspace, st);
+  }
   switch (plan_tile4(p.M, p.N, p.K, p.F)) {
     case Tiles4::k64x32: return launch_direct4<Direct64x32, BF16>(p, st);
     case Tiles4::k64x64: return launch_direct4<Direct64x64, BF16>(p, st);
@@ -149,9 +190,10 @@ int tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F) {
   return plan_tile4(M, N, K, F) == Tiles4::kRing ? 6 : 4;
 }
 
-// checks as mixed_linear_fp6
+// checks as mixed_linear_fp6; without a workspace (16-byte aligned) no K split
 int mixed_linear_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col, const void *w_reduced,
-                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out, void *stream) {
+                       const void *bias, int dtype, int64_t M, int64_t N, int64_t K, int64_t F, void *out, void *workspace,
+                       int64_t workspace_bytes, void *stream) {
   if (dtype != QUIK_F16 && dtype != QUIK_BF16) return QUIK_ERR_DTYPE;
   if (x_bits != 4 && x_bits != 6) return QUIK_ERR_BITS;
   if (M < 0 || N < 0 || K <= 0 || F < 0) return QUIK_ERR_SHAPE;
@@ -161,10 +203,12 @@ int mixed_linear_tile4(const void *x, int x_bits, const void *w4, const void *me
   auto misaligned = [](const void *p) { return reinterpret_cast<uintptr_t>(p) % 256 != 0; };
   if (misaligned(x) || misaligned(w4)) return QUIK_ERR_ALIGN;
   if (M > (1 << 30) || N > (1 << 30) || K > 74496) return QUIK_ERR_RANGE;  // 225 K < 2^24: the fp32 sums stay exact
+  if (reinterpret_cast<uintptr_t>(workspace) % 16 != 0) workspace = nullptr;
   hipStream_t st = as_stream(stream);
   if (x_bits == 4) {
     const Fused8Args p = args_of<Fused8Args>(x, w4, meta, s_col, w_reduced, bias, M, N, K, F, out);
-    return dtype == QUIK_F16 ? run_direct4<false>(p, st) : run_direct4<true>(p, st);
+    return dtype == QUIK_F16 ? run_direct4<false>(p, workspace, workspace_bytes, st)
+                             : run_direct4<true>(p, workspace, workspace_bytes, st);
   }
   const Fused6Args p = args_of<Fused6Args>(x, w4, meta, s_col, w_reduced, bias, M, N, K, F, out);
   return dtype == QUIK_F16 ? run_ring4<false>(p, st) : run_ring4<true>(p, st);
@@ -178,8 +222,20 @@ extern "C" int quik_tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64
   return tile4_activation_bits(M, N, K, F);
 }
 
+extern "C" int64_t quik_tile4_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t F) {
+  if (M <= 0 || N <= 0 || K <= 0 || F < 0) return 0;
+  return split_bytes4(M, N, K, F);
+}
+
 extern "C" int quik_mixed_linear_fwd_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
                                            const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
                                            int64_t K, int64_t F, void *out, void *stream) {
-  return mixed_linear_tile4(x, x_bits, w4, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, stream);
+  return mixed_linear_tile4(x, x_bits, w4, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, nullptr, 0, stream);
+}
+
+extern "C" int quik_mixed_linear_fwd_tile4_ws(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
+                                           const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
+                                           int64_t K, int64_t F, void *out, void *workspace, int64_t workspace_bytes,
+                                           void *stream) {
+  return mixed_linear_tile4(x, x_bits, w4, meta, s_col, w_reduced, bias, dtype, M, N, K, F, out, workspace, workspace_bytes, stream);
 }

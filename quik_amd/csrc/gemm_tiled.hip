@@ -10,16 +10,9 @@
 namespace quik {
 namespace {
 
-// Zero-fill of a few words by a kernel: the arrival counters of the K split are cleared with it, not with
-// hipMemsetAsync, because the caller's stream may be under capture and a memset node in a captured graph is not
-// reliable on replays.
-__global__ __launch_bounds__(256) void clear_words_kernel(uint32_t *p, int words) {
-  for (int i = blockIdx.x * 256 + threadIdx.x; i < words; i += gridDim.x * 256) p[i] = 0u;
-}
 // Split over K for the tile-ordered kernels: few 128x128 tiles (at most half the CUs) and a long K.  Each of
 // `splits` workgroups per tile takes `per` steps (even); workspace = counters (one per tile, zero between launches)
 // followed by the partial accumulators.
-constexpr int64_t kSplitCounterBytes = 4096;
 constexpr int64_t kSplitMinSteps = 32;  // at least 1024 (int8) / 2048 (6-bit) elements of K per workgroup
 enum Operands { kOperands6, kOperands8 };
 // integer k-steps of an operand buffer and bytes of a 64-row unit (fp6_layout, tile8_layout)
@@ -43,19 +36,6 @@ SplitPlan plan_splitk(int64_t M, int64_t N, int64_t K, Operands ops) {
       return {static_cast<int>(splits), static_cast<int>(per), kSplitCounterBytes + tiles * splits * 128 * 128 * 4};
   }
   return none;
-}
-
-// The arrival counters are zero between launches because every launch that completes returns them there.  After a
-// launch that was refused nothing ran, but the caller may not know how far an earlier one got: clear the counters
-// behind a failed launch so that the next one on this workspace starts clean.
-int splitk_launch_status(void *workspace, hipStream_t st) {
-  const int rc = check_launch();
-  if (rc != QUIK_OK) {
-    hipLaunchKernelGGL(clear_words_kernel, dim3(static_cast<unsigned>(kSplitCounterBytes / 4 / 256)), dim3(256), 0, st,
-                       static_cast<uint32_t *>(workspace), static_cast<int>(kSplitCounterBytes / 4));
-    (void)hipGetLastError();  // the status reported is that of the launch that failed
-  }
-  return rc;
 }
 
 template <bool BF16>

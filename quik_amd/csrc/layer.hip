@@ -138,7 +138,7 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
   if (p.tiled) {
     if (four_bit(layer))
       return mixed_linear_tile4(q, p.four_x ? 4 : 6, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype, rows,
-                                l.out_features, l.num_int, l.num_fp, out, stream);
+                                l.out_features, l.num_int, l.num_fp, out, splitk_workspace, splitk_bytes, stream);
     return l.bits == 4 ? mixed_linear_fp6(q, l.tiled_weight, meta, l.weights_scales, w_red, l.bias, l.dtype,
                                                       rows, l.out_features, l.num_int, l.num_fp, out, splitk_workspace,
                                                       splitk_bytes, stream, kLayerK4)

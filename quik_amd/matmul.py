@@ -107,13 +107,17 @@ _splitk_needed = {}
 _splitk_lock = threading.Lock()
 
 
-def _splitk_workspace(device, M, N, K, bits):
+def _splitk_workspace(device, M, N, K, bits, four_bit_outliers=-1):
+    """four_bit_outliers: the number of outlier columns where the weights are of the 4-bit format, whose GEMMs split by a plan of
+    their own."""
     if not split_k:
         return None, 0
-    key = (M, N, K, bits)
+    key = (M, N, K, bits, four_bit_outliers)
     need = _splitk_needed.get(key)
     if need is None:
-        need = _splitk_needed[key] = L.load().quik_splitk_workspace_bytes(M, N, K, bits)
+        lib = L.load()
+        need = _splitk_needed[key] = lib.quik_tile4_splitk_bytes(M, N, K, four_bit_outliers) if four_bit_outliers >= 0 else \
+            lib.quik_splitk_workspace_bytes(M, N, K, bits)
     if need == 0:
         return None, 0
     capturing = torch.cuda.is_current_stream_capturing()
@@ -225,9 +229,10 @@ def mixed_linear_tile4(x, w4, meta, weights_scales, reduced_w, bias, M, N, K, F,
         raise RuntimeError("mixed_linear_tile4: meta / weights_scales / reduced_w sizes are inconsistent with M, N")
     with L.device_guard(x.device):
         out = torch.empty((M, N), dtype=out_dtype, device=x.device)
-        L.check(lib.quik_mixed_linear_fwd_tile4(L.ptr(x), x_bits, L.ptr(w4), L.ptr(meta), L.ptr(weights_scales),
-                                                L.ptr(tensors.get("reduced_w")), L.ptr(tensors.get("bias")), dt, M, N, K, F,
-                                                L.ptr(out), L.stream()), "mixed_linear_tile4")
+        ws, ws_bytes = _splitk_workspace(x.device, M, N, K, 4, F) if x_bits == 4 else (None, 0)
+        L.check(lib.quik_mixed_linear_fwd_tile4_ws(L.ptr(x), x_bits, L.ptr(w4), L.ptr(meta), L.ptr(weights_scales),
+                                                   L.ptr(tensors.get("reduced_w")), L.ptr(tensors.get("bias")), dt, M, N, K, F,
+                                                   L.ptr(out), L.ptr(ws), ws_bytes, L.stream()), "mixed_linear_tile4")
     return out
 
 

@@ -536,7 +536,8 @@ class MixedQLinear(torch.nn.Module):
             nbytes = ws_bytes[rows] = lib.quik_layer_workspace_bytes(ctypes.byref(desc), rows)
         ws = torch.empty((nbytes,), dtype=torch.uint8, device=x2.device)
         out = torch.empty((rows, self.out_features), dtype=self.dtype, device=x2.device)
-        sk, sk_bytes = matmul._splitk_workspace(x2.device, rows, self.out_features, self.int_features_num, self.bits) \
+        sk, sk_bytes = matmul._splitk_workspace(x2.device, rows, self.out_features, self.int_features_num, self.bits,
+                                                self.fp_features_num if desc.tiled_format == L.TILED_4 else -1) \
             if tiled else (None, 0)
         mid = None
         if self.mid_event is not None:   # profiling hook, see the class comment

@@ -1224,13 +1224,13 @@ def test_symmetric_module_on_tile_ordered_operands(case):
 
 
 SPLIT_K_CASES = [
-    # M, N, in, F, bits, symm, bf16: few 128x128 tiles and a long K
-    (64, 512, 8192 + 64, 64, 4, False, False),
-    (64, 1024, 8192, 256, 4, False, True),
+    # M, N, in, F, bits, symm, bf16: few tiles and a long K
+    (64, 512, 14336 + 64, 64, 4, False, False),
+    (64, 1024, 14336, 256, 4, False, True),
     (100, 640, 4096 + 32, 32, 8, False, False),
     (256, 520, 2048 + 64, 64, 8, False, True),      # ragged N
-    (64, 384, 8192, 0, 4, False, False),            # no outlier columns
-    (33, 130, 8192 + 64, 64, 4, True, False),       # symmetric activations, ragged M and N
+    (64, 384, 12288, 0, 4, False, False),           # no outlier columns
+    (33, 130, 12288 + 64, 64, 4, True, False),      # symmetric activations, ragged M and N
     (200, 8192, 28672, 256, 8, False, False),       # Llama-2-70B down_proj at 200 tokens
 ]
 
@@ -1243,7 +1243,8 @@ def test_split_k_gives_the_same_bits(case):
     from quik_amd import _lib, matmul
     M, N, n_in, F, bits, symm, bf16 = case
     K = n_in - F
-    assert _lib.load().quik_splitk_workspace_bytes(M, N, K, bits) > 0       # the shape does split
+    lib = _lib.load()                                                       # the shape does split
+    assert (lib.quik_tile4_splitk_bytes(M, N, K, F) if bits == 4 else lib.quik_splitk_workspace_bytes(M, N, K, bits)) > 0
     rng = np.random.default_rng(sum(case[:5]))
     W, s_w, ii, fi = _layer(rng, N, n_in, F, bits)
     bias = rng.standard_normal(N).astype(np.float16)
