@@ -30,8 +30,10 @@ enum class Tiles4 { k64x32, k64x64, k128x64, kRing };
 // The register-streaming kernels against the ring of 128x128 tiles, below the 256-row tiles.  Picoseconds; r: tiles of the
 // busiest CU, s: k-steps, outlier steps included, w: kilobytes of weights,
 //   t = a + r (b s + c) + d w
-// fitted to 16 row counts of 40 .. 3072 on each of 12 layer shapes (2048 -> 2048 to 13824 -> 5120), warm weights: the pick is 0.3 %
-// behind the fastest of the four (0.6 % with cold weights).  Two 128x128 tiles share a CU: 1.9 of a single one's time.
+// fitted to 16 row counts of 40 .. 3072 on each of 12 layer shapes (2048 -> 2048 to 13824 -> 5120), warm weights; the ring of one
+// tile per CU to 130 calls, warm and cold alike.  The pick is 0.02 % behind the fastest of the four over the 150 calls of 100 .. 1024
+// rows and the few columns of plan_splits4, 0.2 % with cold weights (at most 9 %: 300 x 4096 -> 4096 18.7 / 17.2 us on 128x64
+// tiles).  Two 128x128 tiles share a CU: 1.9 of a single one's time.
 int64_t direct_cost(Tiles4 t, int64_t M, int64_t N, int64_t s, int64_t w) {
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); };
@@ -41,8 +43,9 @@ int64_t direct_cost(Tiles4 t, int64_t M, int64_t N, int64_t s, int64_t w) {
     case Tiles4::k64x64: return 3420000 + rounds(tiles(64, 64), cus) * (33700 * s + 880000) + 52 * w;
     case Tiles4::k128x64: return 700000 + rounds(tiles(128, 64), cus) * (53600 * s + 5800000) + 25 * w;
     default: {
-      const int64_t n = tiles(128, 128), tenths = n <= cus ? 10 : 19 * rounds(n, 2 * cus);
-      return 4070000 + tenths * (116200 * s + 670000) / 10 + 34 * w;
+      const int64_t n = tiles(128, 128);
+      if (n <= cus) return 3750000 + 106000 * s + 670000 + 20 * w;  // (the deep ring)
+      return 4070000 + 19 * rounds(n, 2 * cus) * (116200 * s + 670000) / 10 + 34 * w;
     }
   }
 }
@@ -158,7 +161,13 @@ int run_ring4(const Fused6Args &p, hipStream_t st) {
   const Plan plan = make_plan6(p.M, p.N, 1);
   if (const int64_t n_wide = plan_rest(p.M, p.N, plan); n_wide > 0)
     return launch_rest<CfgL, CfgM>(gemm_fused6_rest_kernel<CfgL, CfgM, BF16, true>, fused6_smem<CfgL, true>(), p, n_wide, st);
-  if (plan.kind != Plan::kSplit) return launch_ring4<CfgM, BF16>(p, st);
+  if (plan.kind != Plan::kSplit) {
+    // One tile per CU: twelve slots, 90 KB in flight instead of 30.  us per forward, warm / cold weights: 300 x 8192 -> 8192 26.8 /
+    // 33.6 -> 26.7 / 30.8, 777 x 11008 -> 4096 38.9 / 44.0 -> 38.2 / 40.5, 400 x 5120 -> 5120 21.6 / 25.9 -> 21.7 / 24.2.  (128x64 tiles in
+    // that ring are behind it and the register-streaming tiles everywhere: 300 x 4096 -> 4096 17.6 against 14.5.)
+    if ((p.M + 127) / 128 * ((p.N + 127) / 128) <= num_cus()) return launch_ring4<CfgDM, BF16>(p, st);
+    return launch_ring4<CfgM, BF16>(p, st);
+  }
   if (plan.n_wide >= p.N) return launch_ring4<CfgL8, BF16>(p, st);
   return launch_ring4_split<CfgL, CfgDH, BF16>(p, plan.n_wide, st);
 }
