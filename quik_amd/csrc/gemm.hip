@@ -321,24 +321,25 @@ int launch_chain_split(const I32Args &a, const ChainArgs &e, int64_t n_wide, hip
 }
 
 // Fused dequantize of at most 32 rows: one round of row-streaming tiles can take the call.  Rows of more than 11 KB leave a
-// tile's waves too long a chain (int8 16 x 13824 -> 5120 24.8 us in two launches, 27.1 on the tiles, 16 x 28672 -> 8192 55 / 62), up to
-// four tiles are too few for long rows (16 x 8192 -> 256 8.8 / 9.3, 1 x 8192 -> 256 7.8 / 9.3).
+// tile's waves too long a chain (two launches / tiles, us in a graph: int8 16 x 13824 -> 5120 14.8 / 18.1, 16 x 28672 -> 8192 35.9 / 36.5),
+// up to four tiles are too few for long rows (int4 16 x 8192 -> 256 6.0 / 9.4).
 bool few_rows_on_tiles(int64_t M, int64_t N, int64_t kbytes) {
   return M <= 32 && N > 256 && (N + 63) / 64 <= num_cus() && kbytes <= 11 * 1024;
 }
-// .. but product (weight-streaming kernel) and epilogue in two launches are faster.  The tiles multiply 64 rows whatever M is and
-// keep N / 64 CUs busy, so their time grows with K alone; the product's grows with M and, where each CU has at most one slab of 32
-// columns, little with K.  us per call in a graph, two launches / tiles, 1024 columns unless said:
-//   int4, K = 8192   1 row 8.2 / 9.4, 16 rows 9.1 / 9.5, 24 rows 9.8 / 9.5; 8192 columns, 8 rows 9.5 / 10.4; 11008, 8 rows 13.5 / 11.1
-//   int4, K = 11264  16 rows 10.3 / 11.6, 24 rows 11.3 / 11.6, 32 rows 12.6 / 11.6; 8192 columns, 16 rows 13.1 / 12.6
-//   int4, K = 22016  24 rows 17.3 / 18.6, 32 rows 18.7 / 18.6; 4096 columns, 24 rows 19.4 / 19.1
-//   int8, K = 5632   8 rows 8.3 / 9.0, 16 rows 9.4 / 9.0; K = 8192 8 rows 10.1 / 11.0, 16 rows 11.7 / 11.0; 8192 columns, 1 row
-//                    17.7 / 13.5; K = 11008 8 rows 11.9 / 13.5
-// Not replayed, the second launch starts 1.5 us later (int4, K = 8192, 1 row 10.0 / 9.6; int8, K = 8192 10.1 / 11.0): calls with
-// shorter rows, which the two serve little faster (1 row: int4, K = 4096 6.6 / 6.8, int8, K = 4096 7.1 / 7.5), stay on the tiles.
+// .. but product (gemm_skinny.h) and epilogue in two launches are faster.  The tiles multiply 64 rows whatever M is and keep N / 64
+// CUs busy, so their time grows with K alone; the product has every CU stream its share of the columns.  us per call in a graph /
+// launched one by one (the second launch starts later then: no call of two takes less than 8.3 us), two launches, tiles:
+//   int4, K = 8192   1024 columns, 16 rows 6.4 / 8.7, 9.4 / 9.7; 32 rows 7.7 / 8.6, 9.4 / 9.7; 8192 columns, 16 rows 8.3 / 8.6, 10.0 / 9.8,
+//                    32 rows 10.2 / 10.3, 10.1 / 9.8; 11008 columns, 8 rows 11.6 / 11.7, 10.9 / 10.7
+//   int4, K = 22016  1024 columns, 32 rows 11.8 / 12.1, 18.2 / 18.7; 4096 columns, 32 rows 14.3 / 14.2, 18.8 / 18.7
+//   int4, K = 16384  4096 columns, 16 rows 8.6 / 8.7, 15.1 / 14.9; 8192 columns, 16 rows 17.9 / 17.6, 15.6 / 15.2
+//   int8, K = 8192   1024 columns, 16 rows 6.8 / 9.1, 11.0 / 11.1; 4096 columns, 32 rows 9.8 / 10.0, 12.3 / 11.6
+//   int8, K = 5632   4096 columns, 8 rows 5.9 / 8.9, 9.1 / 9.2; 2048 columns, 16 rows 6.1 / 9.5, 9.0 / 9.2
+// Shorter rows are faster in two launches only where they are replayed (int4, K = 4096, 16 rows, 1024 columns 5.2 / 8.7, 6.9 / 7.0): they
+// stay on the tiles, as do calls of more than 4096 columns, whose shares outgrow one turn of registers, but for int4 rows of 4 to 5 KB.
 bool few_rows_two_launches(int64_t M, int64_t N, int64_t kbytes, int mode) {
-  if (kbytes >= 5120) return N <= 16 * num_cus() && M <= (mode == kInt4 ? 24 : 8);
-  return mode == kInt4 && kbytes >= 4096 && N <= 32 * num_cus() && M <= 16;
+  if (N <= 16 * num_cus()) return kbytes >= (mode == kInt4 ? 4096 : M <= 8 ? 5120 : 7168);
+  return mode == kInt4 && kbytes >= 4096 && kbytes < 5120 && N <= 32 * num_cus() && M <= 16;
 }
 
 // two_launches: the caller has a workspace for the product

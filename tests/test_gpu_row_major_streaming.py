@@ -82,7 +82,9 @@ def test_fused_form_with_y_in_the_lds_or_not(M, N, kbytes, off):
 
 @pytest.mark.parametrize("bits,M,N,kbytes", [(4, 1, 512, 4080), (4, 16, 8192, 4096), (4, 17, 512, 4096), (4, 1, 8256, 4096),
                                              (4, 24, 4096, 5120), (4, 25, 4096, 5632), (4, 1, 4160, 5632), (8, 1, 320, 5104),
-                                             (8, 8, 4096, 5120), (8, 9, 321, 8192), (8, 1, 4160, 8192), (8, 3, 1001, 11264)])
+                                             (8, 8, 4096, 5120), (8, 9, 321, 8192), (8, 1, 4160, 8192), (8, 3, 1001, 11264),
+                                             (4, 32, 4096, 11008), (4, 17, 8192, 4096), (4, 8, 4104, 5120), (8, 9, 4096, 7152),
+                                             (8, 32, 600, 7168), (8, 9, 333, 5120)])
 def test_few_rows_in_one_launch_or_two(bits, M, N, kbytes):
     """Both sides of the rule between the row-streaming tiles and product + epilogue: the same bits, with a workspace and
     without one (then the tiles take either), eager and replayed from a graph."""
@@ -92,8 +94,8 @@ def test_few_rows_in_one_launch_or_two(bits, M, N, kbytes):
     a, b, ca, cb = _operands(M, N, kbytes, bits, g)
     K = kbytes * (2 if bits == 4 else 1)
     lib = L.load()
-    rows, most = (24 if bits == 4 else 8, 4096) if kbytes >= 5120 else (16, 8192) if bits == 4 and kbytes >= 4096 else (0, 0)
-    two = M <= rows and N <= most
+    two = kbytes >= (4096 if bits == 4 else 5120 if M <= 8 else 7168) if N <= 4096 else \
+        bits == 4 and 4096 <= kbytes < 5120 and N <= 8192 and M <= 16
     assert lib.quik_fused_dequantize_acc_bytes(M, N, K, bits) == (M * N * 4 if two else 0)
     s_row, s_col, zero, w_red, y = ((torch.rand(*s, generator=g, device=DEV) * 0.1).half()
                                     for s in ((M, 1), (1, N), (M, 1), (1, N), (M, N)))
