@@ -141,9 +141,9 @@ def _splitk_workspace(device, M, N, K, bits, four_bit_outliers=-1):
 def pack_weight_fp6(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: torch.Tensor,
                     four_bit: bool = False) -> torch.Tensor:
     """Nibble-packed int4 weights [N, K/2] and outlier weights [N, F] -> operand buffer for mixed_linear_fp6, or with
-    four_bit for mixed_linear_tile4 (once per layer; the 4-bit buffer stands at the front of the bytes that the 6-bit one
-    takes, so that what a program has set aside for a layer fits either).  `colmap` is the layer's column map (asymmetric.build_colmap): the operand buffers of this
-    path keep the integer columns in the map's in-place order, weights and activations alike."""
+    four_bit for mixed_linear_tile4 (once per layer; two thirds of the bytes).  `colmap` is the layer's column map
+    (asymmetric.build_colmap): the operand buffers of this path keep the integer columns in the map's in-place order, weights and
+    activations alike."""
     L.check_cuda_contiguous("pack_weight_fp6", int_weight=int_weight, fp_weight=fp_weight, colmap=colmap)
     if int_weight.dtype != torch.uint8 or int_weight.dim() != 2:
         raise RuntimeError("pack_weight_fp6: expected a uint8 [N, K/2] int_weight")
@@ -155,6 +155,8 @@ def pack_weight_fp6(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap: t
     nbytes = lib.quik_fp6_operand_bytes(N, K, F)
     if nbytes == 0:
         raise RuntimeError("pack_weight_fp6: K must be a multiple of 128 and F a multiple of 32")
+    if four_bit:
+        nbytes = lib.quik_tile4_operand_bytes(N, K, F)
     if colmap.dtype != torch.uint8 or colmap.numel() != lib.quik_colmap_bytes(K + F, K, F):
         raise RuntimeError(f"pack_weight_fp6: the column map was not built for {K} integer and {F} outlier columns")
     from .asymmetric import colmap_streams
@@ -273,6 +275,8 @@ def pack_weight_layer(int_weight: torch.Tensor, fp_weight: torch.Tensor, colmap:
     nbytes = lib.quik_layer_weight_bytes(N, K, F, bits)
     if nbytes == 0:
         raise RuntimeError("pack_weight_layer: shape not supported by the tile-ordered operand format")
+    if four_bit:
+        nbytes = lib.quik_tile4_operand_bytes(N, K, F)
     with L.device_guard(int_weight.device):
         out = torch.empty((nbytes,), dtype=torch.uint8, device=int_weight.device)
         fp = L.ptr(fp_weight) if F else None

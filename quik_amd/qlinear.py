@@ -274,8 +274,8 @@ class MixedQLinear(torch.nn.Module):
     forward, whose operand buffers are filled up with zeros.)  That copy stays beside the reference's buffers, see
     `weight_bytes` and `transient_tiled_copy`.
     W4A4: the int4 products run on the 6-bit (E2M3) matrix-core instructions, which have twice the int8 rate:
-    levels code + 8 are exact E2M3 numbers and the integer accumulator is recovered exactly (0.75
-    bytes per weight).  W8A8: int8 MFMA as before (1 byte per weight).  Both need fp_features % 32 == 0 and ascending int_indices and give the output bits
+    levels code + 8 are exact E2M3 numbers and the integer accumulator is recovered exactly; a weight takes 4 bits in that copy
+    and is widened in registers.  W8A8: int8 MFMA as before (1 byte per weight).  Both need fp_features % 32 == 0 and ascending int_indices and give the output bits
     of the row-major kernels; `six_bit_path = False` turns them off."""
 
     # Profiling hook: a torch.cuda.Event (created, i.e. recorded once before) stored here is recorded between the
@@ -416,7 +416,8 @@ class MixedQLinear(torch.nn.Module):
     def weight_bytes(self):
         """Bytes of weight storage this module holds on its device: the reference's buffers (int_weight + fp_weight,
         qlinear.py:53-78 of the reference) and the tile-ordered copy the prefill GEMMs read (made by the first call
-        that takes that path; 0.75 byte per int4 weight, 1 per int8 weight, outlier columns included)."""
+        that takes that path: 0.5 byte per int4 weight, 1 per int8 weight, 2 per outlier weight, in whole blocks of 64
+        output by 128 / 64 input columns)."""
         fp = self.fp_weight if self.fp_features_num > 0 else None
         row_major = self.int_weight.numel() * self.int_weight.element_size() + \
             (fp.numel() * fp.element_size() if fp is not None else 0)

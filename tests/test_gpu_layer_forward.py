@@ -206,7 +206,9 @@ def test_one_resident_copy_of_the_weights(bits, symm, n_in, F):
     ref = {M: both(torch.from_numpy(x).to(DEV)) for M, x in xs.items()}
     wb = both.weight_bytes()
     assert wb["row_major"] == wb["reference_layout"] == N * ((n_in - F) * bits // 8 + F * 2)
-    assert wb["tiled"] >= N * ((n_in - F) * (6 if bits == 4 else 8) // 8 + F * 2)
+    from quik_amd import _lib as L      # (what the kernels read and no more)
+    assert wb["tiled"] == (L.load().quik_tile4_operand_bytes if bits == 4 else L.load().quik_tile8_operand_bytes)(N, n_in - F, F)
+    assert wb["tiled"] < 1.04 * wb["reference_layout"]
     tiled_only.release_row_major_weights()
     wt = tiled_only.weight_bytes()
     assert wt["row_major"] == 0 and wt["tiled"] == wb["tiled"]
