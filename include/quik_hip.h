@@ -194,6 +194,8 @@ int quik_tile4_pack_weight(const uint8_t *qw, const void *fp_w, int64_t N, int64
 int quik_asym_quantize_tile4(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
                              int64_t num_int, int64_t num_fp, void *out4, void *meta, void *stream);
 int quik_tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64_t F);
+/* the register-streaming tile that a shape takes, rows << 16 | columns; 0: the ring kernels (activation in 6 bits) */
+int quik_tile4_tile(int64_t M, int64_t N, int64_t K, int64_t F);
 int quik_mixed_linear_fwd_tile4(const void *x, int x_bits, const void *w4, const void *meta, const void *s_col,
                                 const void *w_reduced, const void *bias, int dtype, int64_t M, int64_t N,
                                 int64_t K, int64_t F, void *out, void *stream);
@@ -290,7 +292,7 @@ int quik_mixed_linear_fwd_tile8_ws(const void *x8, const void *w8, const void *m
  *                   other value: one of the buffers above
  *   tiled_min_rows  33 is what MixedQLinear uses.  With 1 every call takes the tile-ordered path and reads
  *                   only tiled_weight: int_weight and fp_weight may then be NULL, i.e. the layer can live
- *                   with ONE copy of its weights (0.75 byte per int4 weight, 1 per int8 weight) at the price
+ *                   with ONE copy of its weights (0.5 byte per int4 weight with QUIK_TILED_4, else 0.75; 1 per int8 weight) at the price
  *                   of slower calls of at most 32 rows (the weight-streaming kernel reads the packed nibbles)
  * workspace: quik_layer_workspace_bytes(layer, rows) bytes, 256-byte aligned, holds the quantized activation
  * between the two launches; splitk_workspace as for the _ws entry points (may be NULL; tiled_format QUIK_TILED_4:

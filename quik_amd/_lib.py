@@ -44,6 +44,7 @@ SIGNATURES = {
     "quik_asym_quantize_tile4": (_int, [_vp, _int, _i64, _i64, _vp, _i64, _i64, _vp, _vp, _vp]),
     "quik_tile4_activation_bits": (_int, [_i64, _i64, _i64, _i64]),
     "quik_mixed_linear_fwd_tile4": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp]),
+    "quik_tile4_tile": (_int, [_i64, _i64, _i64, _i64]),
     "quik_tile4_splitk_bytes": (_i64, [_i64, _i64, _i64, _i64]),
     "quik_mixed_linear_fwd_tile4_ws": (_int, [_vp, _int, _vp, _vp, _vp, _vp, _vp, _int, _i64, _i64, _i64, _i64, _vp, _vp, _i64, _vp]),
     "quik_sym_quantize_mapped": (_int, [_vp, _i64, _i64, _vp, _i64, _i64, _int, ctypes.c_float, _int, _vp, _vp, _vp,

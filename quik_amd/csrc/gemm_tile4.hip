@@ -231,6 +231,16 @@ extern "C" int quik_tile4_activation_bits(int64_t M, int64_t N, int64_t K, int64
   return tile4_activation_bits(M, N, K, F);
 }
 
+extern "C" int quik_tile4_tile(int64_t M, int64_t N, int64_t K, int64_t F) {
+  if (M <= 0 || N <= 0 || K <= 0 || F < 0) return 0;
+  switch (plan_tile4(M, N, K, F)) {
+    case Tiles4::k64x32: return Direct64x32::BM << 16 | Direct64x32::BN;
+    case Tiles4::k64x64: return Direct64x64::BM << 16 | Direct64x64::BN;
+    case Tiles4::k128x64: return Direct128x64::BM << 16 | Direct128x64::BN;
+    default: return 0;
+  }
+}
+
 extern "C" int64_t quik_tile4_splitk_bytes(int64_t M, int64_t N, int64_t K, int64_t F) {
   if (M <= 0 || N <= 0 || K <= 0 || F < 0) return 0;
   return split_bytes4(M, N, K, F);

@@ -1,8 +1,10 @@
-"""Tile-ordered GEMMs with one tile per CU (rings of twelve or eight slots): 128x64 tiles at 6 bits, 128x128 and 256x128
-ones at both widths; fewer steps than slots, exactly as many, one pair more, whole turns with every remainder, none and more
+"""Tile-ordered GEMMs with one tile per CU (rings of twelve or eight slots): 128x64 tiles on 6-bit weights, 128x128 and 256x128
+ones on 4-bit (the layer), 6-bit (the stand-alone operations) and int8 weights; fewer steps than slots, exactly as many, one pair more, whole turns with every remainder, none and more
 outlier steps than slots.  Same output bits as the row-major int8-MFMA kernels, which other tests hold against the oracle."""
 import pytest
 import torch
+
+from test_gpu_register_streaming import six_bit_operands
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -49,7 +51,7 @@ def _same_bits(M, N, K, F, dtype, bits):
     x = torch.randn(M, K + F, generator=g)
     x[:, fi] *= 50
     x = x.to(dtype).to(DEV)
-    got = [mod(x) for _ in range(2)]
+    got = [mod(x) for _ in range(2)] + six_bit_operands(mod, x)
     assert mod._w6 is not None
     mod.six_bit_path = False
     want = mod(x)

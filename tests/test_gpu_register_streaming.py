@@ -1,7 +1,7 @@
 """The register-streaming layer GEMM (csrc/gemm_direct.h) at the edges of its tiles: fewer k-steps than waves, step counts
 that leave the waves unequal shares, one row more or less than a 64-row block, ragged and odd column counts, tiles that
 start in the second half of a weight block, none, few and more outlier steps than it keeps in flight, K split over
-workgroups.  Same output bits as the row-major int8-MFMA kernels, which other tests hold against the oracle."""
+workgroups.  Int4 cases run on 4-bit weights (the layer) and on the 6-bit operands (their stand-alone operations).  Same output bits as the row-major int8-MFMA kernels, which other tests hold against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -31,6 +31,19 @@ def test_plans_of_large_weights(case):
     _same_bits(*case, torch.float16)
 
 
+def six_bit_operands(mod, x):
+    """The forward of an int4 layer on 6-bit weights and activations, where its shape has such buffers."""
+    from quik_amd import asymmetric, matmul
+    if mod.bits != 4 or mod.int_features_num % 128 != 0:
+        return []
+    K, F, cm = mod.int_features_num, mod.fp_features_num, mod._column_map()
+    fp_w = mod.fp_weight if F else torch.empty(mod.out_features, 0, dtype=mod.dtype, device=DEV)
+    x6, meta = asymmetric.quantize_mapped_fp6(x, cm, K, F)
+    out = matmul.mixed_linear_fp6(x6, matmul.pack_weight_fp6(mod.int_weight, fp_w, cm), meta, mod.weights_scales, mod.reduced_w, mod.bias,
+                                  x.shape[0], mod.out_features, K, F, mod.dtype)
+    return [out[None]]
+
+
 def _same_bits(M, N, K, F, bits, dtype):
     from quik_amd import matmul
     from quik_amd.qlinear import MixedQLinear
@@ -46,9 +59,11 @@ def _same_bits(M, N, K, F, bits, dtype):
     x = x.to(dtype).to(DEV)
     got = [mod(x) for _ in range(2)]
     assert mod._w6 is not None
+    got += six_bit_operands(mod, x)
     matmul.split_k = False
     try:
         got.append(mod(x))
+        got += six_bit_operands(mod, x)
     finally:
         matmul.split_k = True
     mod.six_bit_path = False
