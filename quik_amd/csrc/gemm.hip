@@ -132,9 +132,12 @@ template <int MODE, bool BF16, int MT, int QUANT>
 int launch_gemv_mt(const FusedArgs &p, const GemvQuant &q, hipStream_t st) {
   auto kern = gemv_decode_kernel<MODE, BF16, MT, QUANT>;
   if (int rc = prepare(kern, kLdsBytes)) return rc;  // (the size varies with the layer: set once to the most)
-  // persistent waves, one column at a time each: two workgroups per CU when their LDS fits twice
+  // persistent waves, one column at a time each: two workgroups per CU when their LDS fits twice.  But one where each wave then has
+  // at most two columns of two rows that are quantised here: two workgroups quantise both rows twice on their CU (us per forward,
+  // two / one: 1472 -> 3200 8.6 / 7.2, 1024 -> 4096 8.4 / 7.2, int8 1536 -> 4096 8.7 / 7.8).
   const int64_t fixed = gemv_smem(MT, p.kbytes, p.F) + (QUANT != kGemvNoQuant ? gemv_quant_lds(q.cols, q.num_int).bytes : 0);
-  const int64_t per_cu = 2 * (fixed + 4096) <= kLdsBytes ? 2 : 1;
+  const bool quantise_bound = QUANT != kGemvNoQuant && MT == 2 && p.N <= 2 * kGemvWaves * num_cus();
+  const int64_t per_cu = 2 * (fixed + 4096) <= kLdsBytes && !quantise_bound ? 2 : 1;
   int64_t grid = (p.N + kGemvWaves - 1) / kGemvWaves;
   if (grid > per_cu * num_cus()) grid = per_cu * num_cus();
   const int64_t smem = fixed + gemv_table_bytes((p.N + kGemvWaves * grid - 1) / (kGemvWaves * grid));
@@ -444,9 +447,9 @@ extern "C" int quik_int8_matmul(const int8_t *A, const int8_t *B, int32_t *C, in
 // stream, two launches / one: int4 4096 -> 4096 8.5 / 9.5, 4096 -> 11008 9.7 / 12.0, 11008 -> 4096 9.7 / 14.4, int8 13824 -> 5120
 // 18.0 / 20.6, 1024 -> 16384 8.4 / 10.5), but for
 //   few columns, at most one per wave of a workgroup on each CU, or twice as many of short rows, where the second launch is all
-//   there is (2048 -> 2048 7.6 / 6.9, 1280 -> 1664 7.8 / 6.6, 4096 -> 1024 8.2 / 7.5, int8 2048 -> 2048 8.4 / 6.8; 1024 -> 4096
-//   8.1 / 8.2, 1472 -> 3200 with 448 outlier columns 9.4 / 8.2; rows too long: 2048 -> 4096 7.7 / 8.4, 8192 -> 512 8.6 / 8.8, 14272 ->
-//   1024 9.7 / 11.0);
+//   there is (2048 -> 2048 7.6 / 6.8, 1280 -> 1664 7.8 / 6.6, 4096 -> 1024 8.2 / 7.5, int8 2048 -> 2048 8.4 / 6.9; 1024 -> 4096
+//   7.6 / 7.1, 1472 -> 3200 with 448 outlier columns 7.6 / 7.0; replayed from a graph two are as fast, 1472 -> 3200 with none 6.0 / 6.5;
+//   rows too long: 2048 -> 4096 7.7 / 8.4, 8192 -> 512 8.6 / 8.8, 14272 -> 1024 9.7 / 11.0);
 //   very many columns, whose stream hides the rest (8192 -> 22016 21.6 / 21.1, 8192 -> 28672 25.5 / 24.9, int8 42.8 / 40.6; but
 //   14272 -> 9816 19.6 / 19.5).
 bool quik::gemv_one_launch_pays(int64_t rows, int64_t cols, int64_t N) {
