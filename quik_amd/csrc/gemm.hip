@@ -85,6 +85,16 @@ int launch_skinny_rows(const FusedArgs &p, int32_t *C, int ldc, hipStream_t st) 
   most = most < 4 ? 4 : most > kMost ? kMost : most;
   const int64_t rounds = (p.N + most * cus - 1) / (most * cus), share = (p.N + rounds * cus - 1) / (rounds * cus);
   const int bn = static_cast<int>((share + 3) / 4 * 4);  // (whole 8-byte pieces of the output rows)
+  if constexpr (MT == 1 && !FUSED) {
+    // Integer products, whose waves request nothing else: many columns of few rows in two rounds of at most 64 instead of one, and
+    // longer rows with three turns of two blocks in flight.  us, weights from memory / in the Infinity Cache, otherwise and so:
+    // int4 2 x 8192 -> 28672 27.0 / 19.2, 24.9 / 18.7; 8 x 8192 -> 20480 20.8 / 15.0, 19.1 / 15.2; int8 8 x 8192 -> 28672 46.3 / 37.6, 44.6 /
+    // 36.5 (16 rows: int4 8192 -> 28672 27.7 / 19.4, 28.0 / 20.7); int8 2 x 28672 -> 8192 47.7 / 34.1, 43.1 / 34.1, 16 x 20480 -> 6144 27.8 /
+    // 20.4, 26.3 / 20.3, 8 x 16384 -> 8192 32.3 / 27.1, 31.2 / 25.5 (but 8 x 14336 -> 8192 21.6 / 18.1, 22.0 / 18.3).
+    if (rounds == 1 && bn > 64 && p.M <= 8)
+      return launch_skinny_cfg<SkinnyCfg<4, MT, 1>, MODE, BF16, FUSED>(p, (bn / 2 + 3) / 4 * 4, C, ldc, st);
+    if (bn > 16 && bn <= 32 && p.kbytes >= 16384) return launch_skinny_cfg<SkinnyCfg<2, MT, 3>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
+  }
   if (bn <= 16) return launch_skinny_cfg<SkinnyCfg<1, MT, 3>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
   if (bn <= 32) return launch_skinny_cfg<SkinnyCfg<2, MT, 2>, MODE, BF16, FUSED>(p, bn, C, ldc, st);
   if (bn <= 48) return launch_skinny_cfg<SkinnyCfg<3, MT, 2>, MODE, BF16, FUSED>(p, bn, C, ldc, st);

@@ -38,6 +38,15 @@ def test_int32_product_is_exact(M, N, K, bits):
     assert torch.equal(mm(_packed(a, bits), _packed(b, bits)), want)
 
 
+# products of their own plan: more than 64 columns per CU and at most 8 rows in two rounds, whole and ragged; rows of 16 KB and more
+# with three turns in flight (a wave's turns a multiple of three and one and two more, a tail)
+@pytest.mark.parametrize("bits,M,N,kbytes", [(4, 8, 65 * FULL + 3, 1040), (8, 1, 80 * FULL - 9, 2048), (4, 9, 72 * FULL, 384), (8, 7, 112 * FULL, 128),
+                                             (4, 3, 17 * FULL + 1, 16384), (8, 16, 4500, 16384 + 128 * 9), (4, 16, 5000, 18432 + 112),
+                                             (8, 1, 32 * FULL - 2, 16384 + 16), (8, 17, 4500, 16384), (8, 4, 4400, 16384 - 16)])
+def test_products_of_many_columns_and_of_long_rows(bits, M, N, kbytes):
+    test_int32_product_is_exact(M, N, kbytes * 8 // bits, bits)
+
+
 @pytest.mark.parametrize("bits", [4, 8])
 @pytest.mark.parametrize("i", range(len(SHAPES)))
 def test_fused_form(i, bits):
