@@ -65,7 +65,7 @@ PEAK_HBM_GBPS = 8000.0    # MI355X HBM3E, published
 # (`traffic_source`).  (gemm6 / quantize6: the kernels of the 6-bit matrix-core path, the default; gemm / quantize:
 # --int8-mfma)
 MEASURED_TRAFFIC_BYTES = {
-    "llama2-70b.gate_proj": {"gemm": 809.4e6, "quantize": 43.0e6, "gemm6": 754.7e6, "quantize6": 46.9e6},
+    "llama2-70b.gate_proj": {"gemm": 809.4e6, "quantize": 43.0e6, "gemm6": 596.1e6, "quantize6": 46.9e6},
 }
 TRAFFIC_SOURCE = {
     "gemm6": "offline: profiles/gemm_fused6_split_kernel__llama2-70b.gate_proj.md (rocprofv3 --pmc FETCH_SIZE / "
@@ -650,15 +650,22 @@ def main():
     int_ops = 2.0 * M * N * K
     tops = int_ops / (ms_step * 1e-3) / 1e12
     gemm_tops = int_ops / (g_avg * 1e-3) / 1e12
-    # read the row once; write the codes (6 bits each in the operand format of the 6-bit path, plus a 4-byte
-    # level sum per row), the outlier values and the (scale, zero) pair
-    quant_bytes = M * n_in * 2 + (M * K * 6 // 8 + M * 4 if six and bits == 4 else M * K * bits // 8) + M * F * 2 + M * 4
+    # read the row once; write the codes (in the operand buffers of int4 layers 4 or 6 bits each, by the GEMM that reads them, plus
+    # a 4-byte level sum per row), the outlier values and the (scale, zero) pair
+    lib = _lib.load()
+    x_bits = lib.quik_tile4_activation_bits(M, N, K, F) if six and bits == 4 else bits
+    quant_bytes = M * n_in * 2 + M * K * x_bits // 8 + (M * 4 if six and bits == 4 else 0) + M * F * 2 + M * 4
     quant_gbps = quant_bytes / (q_avg * 1e-3) / 1e9
     peak = PEAK_FP6_TOPS if six and bits == 4 else PEAK_INT8_TOPS
-    split_k = six and matmul.split_k and _lib.load().quik_splitk_workspace_bytes(M, N, K, bits) > 0
+    split_k = six and matmul.split_k and (lib.quik_tile4_splitk_bytes(M, N, K, F) if bits == 4 else
+                                          lib.quik_splitk_workspace_bytes(M, N, K, bits)) > 0
+    # (one launch: the event that the library records between the two launches then stands behind the only one)
+    one_launch = mod.fused and not six and M <= 2 and g_ms[len(g_ms) // 2] < 0.5 * q_ms[len(q_ms) // 2]
     if six and bits == 4:
-        gemm_kernel = "gemm_fused6_splitk_kernel (K split over several workgroups per tile)" if split_k else \
-            "gemm_fused6_split_kernel / gemm_fused6_kernel (one launch per step)"
+        tile = lib.quik_tile4_tile(M, N, K, F)
+        gemm_kernel = "gemm_direct_splitk_kernel (4-bit weights, K split over several workgroups per tile)" if split_k else \
+            f"gemm_direct_kernel (4-bit weights, {tile >> 16}x{tile & 65535} tiles)" if tile else \
+            "gemm_fused6_split_kernel / gemm_fused6_kernel (4-bit weights, one launch per step)"
         dtype = "int4 (exact, as E2M3 on the 6-bit MFMA path)"
     elif six:
         gemm_kernel = "gemm_fused8t_splitk_kernel (tile-ordered int8 operands, K split over several workgroups per " \
@@ -668,9 +675,9 @@ def main():
     elif mod.fused:
         gemm_kernel = "gemv_decode_kernel (one or two token rows: quantize and weight-streaming matrix-vector product " \
             "in ONE launch)" \
-            if M <= 2 else "gemm_skinny_kernel (weight streaming, one launch per step)" if M <= 32 else \
+            if one_launch else "gemm_skinny_kernel (weight streaming, one launch per step)" if M <= 32 else \
             "gemm_fused_split_kernel / gemm_fused_kernel (one launch per step)"
-        dtype = "int8" if bits == 8 else "int4 (dot-product instructions)" if M <= 2 else "int4 (on int8 MFMA)"
+        dtype = "int8" if bits == 8 else "int4 (dot-product instructions)" if one_launch else "int4 (on int8 MFMA)"
     else:
         gemm_kernel = "gemm_i32_split_kernel + dequantize + F.linear"
         dtype = "int8" if bits == 8 else "int4 (on int8 MFMA)"
@@ -684,7 +691,6 @@ def main():
                 if mod.fused and traffic.get("gemm6" if six else "gemm") else None,
                 "avg_ms": round(g_avg, 4), "median_ms": round(g_ms[len(g_ms) // 2], 4),
                 "timed_launches": len(g_ms), "algorithmic_ops": int_ops}
-    one_launch = mod.fused and not six and M <= 2
     if mod.fused and not six and M <= 32:
         # the weight-streaming kernels are bound by HBM: every weight byte once, plus the small operands
         stream_bytes = N * K * bits // 8 + N * F * 2 + 3 * N * 2 + M * n_in * 2 + M * N * 2
@@ -719,7 +725,7 @@ def main():
         "verified_vs_oracle": None if spot is None else {"tiles": 3, "max_abs_err_over_rms": round(spot, 6),
                                                          "tolerance": 1e-2},
         "roofline": roofline,
-        "roofline_quantize": None if one_launch else {"kernel": ("quantize_fp6_row_kernel (one workgroup per token row, 6-bit operand output)" if six and bits == 4
+        "roofline_quantize": None if one_launch else {"kernel": (f"quantize_fp6_row_kernel (one workgroup per token row, {x_bits}-bit operand output)" if six and bits == 4
                                          else "quantize_tile8_ring_kernel (row copied into an LDS ring, int8 operand output in tile order)"
                                          if six and bits == 8 and n_in > 8192 and str(x.dtype) == "torch.float16"
                                          else "asym_quantize_stream_kernel" + (" (tile-ordered operand output)" if six else "")),

@@ -79,7 +79,7 @@ __host__ __device__ inline int64_t tile8_offset(const Tile8Layout &l, int64_t ro
          ((h ^ ((row >> 3) & 1)) << 4);
 }
 
-// ---- 4-bit operands of the same order (consumers: gemm_tile8.h, gemm_direct.h with kNib), the layer's own int4 format.
+// ---- 4-bit operands of the same order (consumers: gemm_fp6.h with W4, gemm_direct.h with kDirect4), the layer's own int4 format.
 //
 // A 6-bit field of the MFMA operand holds a level 0 .. 15, so two of its six bits are zero and the 6-bit buffers above
 // carry a third of zeros.  Here 16 levels are two dwords instead of three: P0 is the first dword of the 6-bit fragment,

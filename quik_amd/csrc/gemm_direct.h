@@ -6,7 +6,7 @@
 // (measured over K: 106 .. 112 ns a step, some 210 cycles).  The operand buffers hold
 // each fragment as one contiguous kilobyte (fp6_format.h), so a wave can load fragments directly, and nothing has to be
 // shared inside the workgroup if the waves split K instead of the tile: each of the four waves computes the WHOLE tile
-// (64x64 or 64x32) over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of
+// (64x64 or 64x32, at 4 bits also 128x64) over every fourth k-step, without a barrier or an LDS access in the main loop, with SETS steps of
 // loads in flight.  What bounds it is the rate at which a CU takes in operands: over K, 70 ns per step of 6 KB (88 bytes
 // per ns) for 64x64 tiles at 6 bits, 33 ns per 3 KB (94) for 64x32 tiles at 8.  Afterwards the waves add their
 // integer sums through LDS (exact, so in any order), each ending up with the blocks it owns, convert them, run the

@@ -896,14 +896,14 @@ __global__ __launch_bounds__(C::kThreads) void gemm_fused6_kernel(Fused6Args p, 
 }
 
 // K split over sk.splits workgroups per tile: block b works on tile b % grid_tiles, split b / grid_tiles.
-template <class C, bool BF16, bool W4 = false>
+template <class C, bool BF16>
 __global__ __launch_bounds__(C::kThreads) void gemm_fused6_splitk_kernel(Fused6Args p, int tiles_m, int tiles_n,
                                                                           SplitK sk) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   const int split = blockIdx.x / sk.grid_tiles;
   if (!tile_of_block<C::BM>(blockIdx.x - split * sk.grid_tiles, tiles_m, tiles_n, tm, tn)) return;
-  fused6_tile<C, BF16, true, W4>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
+  fused6_tile<C, BF16, true>(p, tm, tn, smem, split, tm * tiles_n + tn, &sk);
 }
 
 // One launch, two tile shapes (see gemm_i32_split_kernel).

@@ -257,10 +257,10 @@ MM_CASES = [
     (128, 512, 4864),
     (300, 260, 7936),
     (512, 1024, 3968),
-    # at most 32 token rows: the weight-streaming kernel (slabs of 32 columns, 128-byte K chunks per wave)
-    (5, 40, 32),         # one chunk, fewer chunks than waves, ragged last slab
-    (32, 8200, 4864),    # more slabs than resident workgroups: several slabs per workgroup
-    (17, 96, 4096 + 32), # 8 waves per slab (long K, few slabs), K tail of half a 32-byte step for int4
+    # at most 32 token rows: the weight-streaming kernel (even shares of the columns, 128-byte K chunks per wave)
+    (5, 40, 32),         # one chunk, fewer chunks than waves, ragged last share
+    (32, 8200, 4864),    # shares of 36 columns, a ragged last block of 16
+    (17, 96, 4096 + 32), # few workgroups, long K, K tail of half a 32-byte step for int4
 ]
 
 
@@ -433,10 +433,10 @@ FWD_CASES = [
     (260, 300, 1280, 256, 8, True, "x50"),
     (64, 128, 512, 0, 4, True, "x50"),
     (1, 384, 1024, 64, 4, False, "x50"),
-    (5, 40, 72, 8, 4, True, "x50"),          # decode kernel: one K chunk, half an outlier piece, ragged slab
+    (5, 40, 72, 8, 4, True, "x50"),          # decode kernel: one K chunk, half an outlier piece, ragged share
     (7, 100, 200, 8, 8, True, "student"),
-    (32, 8200, 1056, 32, 4, False, "x50"),   # decode kernel: several slabs per workgroup
-    (20, 64, 8192 + 520, 520, 8, True, "x50"),  # decode kernel: 8 waves per slab, more outlier pieces than prefetched
+    (32, 8200, 1056, 32, 4, False, "x50"),   # decode kernel: shares of 36 columns
+    (20, 64, 8192 + 520, 520, 8, True, "x50"),  # decode kernel: long K, more outlier steps than waves
     (9, 8300, 1000, 40, 4, True, "x50"),     # decode kernel, token rows in LDS: last K chunk and last outlier piece cut short
     (12, 70, 456, 24, 8, False, "student"),  # decode kernel, token rows streamed: the same for int8
 ]
@@ -777,7 +777,7 @@ def test_full_size_properties(case):
 
 
 DECODE_RESIDENT = [
-    # M, N, in, F, bits: N > 8192, so a workgroup of the weight-streaming kernel walks over several slabs
+    # M, N, in, F, bits: N > 8192, shares of more than 32 columns in the weight-streaming kernel
     (16, 8192 + 4128, 1024 + 64, 64, 4),
     (32, 8192 + 167, 2048 + 32, 32, 8),
     (7, 9000, 512, 0, 4),
@@ -788,9 +788,9 @@ DECODE_RESIDENT = [
 
 @pytest.mark.parametrize("case", DECODE_RESIDENT)
 def test_decode_kernel_with_token_rows_resident_in_lds(case):
-    """At most 32 token rows and more than 8192 output columns: the weight-streaming kernel keeps the token rows in
-    LDS.  Its output must have the bits of the same layer cut into column halves of at most 8192 columns (which
-    stream the token rows from L2), and agree with the oracle."""
+    """At most 32 token rows and more than 8192 output columns: large shares per workgroup in the weight-streaming kernel.
+    The output must have the bits of the same layer cut into column halves (smaller shares, fewer blocks of 16 columns),
+    and agree with the oracle."""
     M, N, n_in, F, bits = case
     rng = np.random.default_rng(sum(case))
     W, s_w, ii, fi = _layer(rng, N, n_in, F, bits)
