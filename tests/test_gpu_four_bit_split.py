@@ -54,3 +54,27 @@ def test_no_workspace_where_nothing_is_split():
             mod(x)
     side.synchronize()
     assert (torch.cuda.current_device(), side.cuda_stream) not in matmul._splitk_workspaces
+
+
+@pytest.mark.gpu
+def test_a_split_call_in_a_graph():
+    """Replayed several times with eager split calls of another input between the replays, on the capture's stream and another."""
+    mod = _module(3, 512, 14336, 256, 4)
+    g = torch.Generator().manual_seed(0)
+    xs = [torch.randn(64, 14336, generator=g).half().to(DEV) for _ in range(4)]
+    want = [mod(x).clone() for x in xs]
+    held = xs[0].clone()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        out = mod(held)
+    side = torch.cuda.Stream()
+    for i in (1, 2, 3, 0, 2):
+        held.copy_(xs[i])
+        graph.replay()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            other = mod(xs[3 - i])
+        mine = mod(xs[(i + 1) % 4])
+        torch.cuda.synchronize()
+        for got, k in ((out, i), (other, 3 - i), (mine, (i + 1) % 4)):
+            assert torch.equal(got.view(torch.int16), want[k].view(torch.int16))
