@@ -7,9 +7,10 @@
 // 2^24), so the fp32 accumulation is exact in any order, and
 //     sum_k a_k w_k = 64 S - 8 sum_k La_k - 8 sum_k Lw_k + 64 K,      S = sum_k (La_k / 8)(Lw_k / 8)
 // recovers the integer accumulator exactly (every term is an integer below 2^24).  The accumulators
-// start at -(8 sum_k Lw_k) / 64 (a multiple of 1/8, so still exact), and one fused multiply-add per value,
-// 64 acc - (8 sum_k La_k - 64 K), finishes the job.  From there the epilogue is the one of
-// gemm_kernels.h, so the output is bit-identical to the int8-MFMA path.
+// start at K - sum_k La_k / 8 - sum_k Lw_k / 8 (between -176 K and 64 K 64ths, from where they only rise, to the result:
+// still exact) and end at a 64th of the integer; the 64 is in the column's scale.  From there the epilogue is the one of
+// gemm_kernels.h, so the output is bit-identical to the int8-MFMA path (as long as 64 times a column's scale is finite: in
+// bf16 it is up to 5e36).
 //
 // Operand format: fp6_format.h.  Both operand buffers are stored as the sequence of LDS images the
 // tiles need, so a copy instruction moves one contiguous kilobyte and every cache line is requested
@@ -230,22 +231,31 @@ struct Fp6Pipe {
 
   // Fill the ring: afterwards steps 0 and 1 are visible and steps 2 .. NS - 2 are in flight; the copies of step
   // NS - 1 are made during the MFMAs of step 0.
-  // landed(): what this wave does in front of the barrier, behind the arrival of what it requested before the ring.
+  // In two parts: landed() is what this wave does with what it requested before the ring, behind the first part the others have
+  // done so too, and what needs that goes in front of the second, under the first steps' way here.
   template <class Landed>
-  __device__ __forceinline__ void start(Landed landed) {
+  __device__ __forceinline__ void start_vectors(Landed landed) {
     static_for<NS - 1>([&](auto) { issue(); });
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+    static_assert((NS - 1) * P <= 63, "the vmcnt counter");
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 1) * P));
     asm volatile("" ::: "memory");  // (empty: LDS reads of what has landed stay behind the wait)
     landed();
     __syncthreads();
   }
-  __device__ __forceinline__ void start() { start([] {}); }
+  __device__ __forceinline__ void start_steps() {
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm((NS - 3) * P));
+    asm volatile("" ::: "memory");  // (empty, as above)
+    __syncthreads();
+  }
+  __device__ __forceinline__ void start() {
+    static_for<NS - 1>([&](auto) { issue(); });
+    start_steps();
+  }
 
   __device__ __forceinline__ void next_read_slot() {
     rd += STAGE;
     rd = rd == NS * STAGE ? 0 : rd;
   }
-  __device__ __forceinline__ void previous_read_slot() { rd = rd == 0 ? (NS - 1) * STAGE : rd - STAGE; }
 
   // fragment j (32 rows) of this wave: head image j, tail image j / 2 at row offset 32 (j % 2)
   // RS: slot being read when known at compile time, -1: `rd`
@@ -403,8 +413,8 @@ struct Fp6Pipe {
       __builtin_amdgcn_s_barrier();
     }
   }
-  __device__ __forceinline__ void run_fp64(v16f (&acc)[MI][NI]) {
-    v4i h0[NF], h1[NF];
+  __device__ __forceinline__ void run_fp64(v16f (&acc)[MI][NI], v4i (&h0)[NF]) {
+    v4i h1[NF];
     v2i t0[NF], t1[NF];
     v6i w0[NI], w1[NI];
     read6(h0, t0);
@@ -421,7 +431,6 @@ struct Fp6Pipe {
       step64(h0, t0, w0, h1, t1, w1, acc);
       step64(h1, t1, w1, h0, t0, w0, acc);
     }
-    previous_read_slot();
   }
   template <int RS, int LO, int HI>
   __device__ __forceinline__ void chunk_reads6(v4i (&nh)[NF], v2i (&nt)[NF]) const {
@@ -437,11 +446,13 @@ struct Fp6Pipe {
       chunk_mfmas6<LO + 1, HI>(ch, ct, acc);
     }
   }
+  // The next step's fragments are read in the first chunks, the weights' first, as the MFMAs take them: read over the whole
+  // step, the last one was on its way when the next step began with it.
   template <bool BF16, int G = 0>
   __device__ __forceinline__ void step16(const v4i (&cf)[NF], v4i (&nf)[NF], v16f (&acc)[MI][NI]) {
-    constexpr int MM = MI * NI;
+    constexpr int MM = MI * NI, E0 = (P - 1) / 2 + 1;
     if constexpr (G < P) {
-      constexpr int r_lo = G * NF / P, r_hi = (G + 1) * NF / P, m_lo = G * MM / P, m_hi = (G + 1) * MM / P;
+      constexpr int r_lo = G < E0 ? G * NF / E0 : NF, r_hi = G < E0 ? (G + 1) * NF / E0 : NF, m_lo = G * MM / P, m_hi = (G + 1) * MM / P;
       chunk_reads16<r_lo, r_hi>(nf);
       chunk_mfmas16<BF16, m_lo, m_hi>(cf, acc);
       if constexpr (m_hi > m_lo) {
@@ -463,8 +474,8 @@ struct Fp6Pipe {
   }
   template <int LO, int HI>
   __device__ __forceinline__ void chunk_reads16(v4i (&nf)[NF]) const {
-    if constexpr (LO < HI) {
-      read16_one<LO>(nf);
+    if constexpr (LO < HI) {  // in the order W, X
+      read16_one<(LO < NI ? MI + LO : LO - NI)>(nf);
       chunk_reads16<LO + 1, HI>(nf);
     }
   }
@@ -476,10 +487,11 @@ struct Fp6Pipe {
     }
   }
 
-  // Integer steps [0, steps0): acc += (Lw / 8)(Lx / 8) summed over 64 elements per MFMA.
-  __device__ __forceinline__ void run_fp6(v16f (&acc)[MI][NI]) {
-    if constexpr (W4) return run_fp64(acc);
-    v4i h0[NF], h1[NF];
+  // Integer steps [0, steps0): acc += (Lw / 8)(Lx / 8) summed over 64 elements per MFMA.  h0: afterwards the heads of the
+  // step behind them, the fragments of the first outlier step.
+  __device__ __forceinline__ void run_fp6(v16f (&acc)[MI][NI], v4i (&h0)[NF]) {
+    if constexpr (W4) return run_fp64(acc, h0);
+    v4i h1[NF];
     v2i t0[NF], t1[NF];
     read6(h0, t0);
     // here: step 0 in h0 / t0, `rd` at slot 1, `fill` at slot NS - 1.  NS steps at a time with the slots as
@@ -496,14 +508,12 @@ struct Fp6Pipe {
       step6(h0, t0, h1, t1, acc);
       step6(h1, t1, h0, t0, acc);
     }
-    previous_read_slot();  // the last read looked at the first outlier step (or a dead slot) as 6-bit data
   }
 
-  // Outlier steps [steps0, steps): acc += fp_w fp_x^T, 16 elements per MFMA.
+  // Outlier steps [steps0, steps): acc += fp_w fp_x^T, 16 elements per MFMA.  f0: the first one's fragments
   template <bool BF16>
-  __device__ __forceinline__ void run_f16(v16f (&acc)[MI][NI]) {
-    v4i f0[NF], f1[NF];
-    read16(f0);
+  __device__ __forceinline__ void run_f16(v16f (&acc)[MI][NI], v4i (&f0)[NF]) {
+    v4i f1[NF];
     for (int j = steps0; j < steps; j += 2) {
       step16<BF16>(f0, f1, acc);
       step16<BF16>(f1, f0, acc);
@@ -535,7 +545,7 @@ struct Fused6Args {
 };
 
 // Per-tile vectors in LDS behind the ring: the five of TileVectors plus the two integer corrections
-//   rowc[m] = 8 sum_k Lx - 64 K,  colc[n] = -(8 sum_k Lw) / 64 (the accumulators' start value)   (exact in fp32).
+//   rowc[m] = K - sum_k Lx / 8,  colc[n] = -sum_k Lw / 8: the accumulators start at their sum (exact in fp32).
 template <class C>
 struct TileVectors6 {
   static constexpr int kBytes = (4 * C::BN + 3 * C::BM) * 4;
@@ -605,8 +615,11 @@ __device__ __forceinline__ void tile_sums_request(const Vectors &tv, const Args 
 template <class C, class Vectors>
 __device__ __forceinline__ void tile_sums_widen(const Vectors &tv, int K) {
   const int i = threadIdx.x;
-  if (i < C::BN) tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
-  if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * __float_as_int(tv.rowc[i]) - 64 * K);
+  if (i < C::BN) {
+    tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
+    tv.scol[i] *= 64.0f;  // (behind tile_vector_widen, by the same thread)
+  }
+  if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * K - __float_as_int(tv.rowc[i])) * 0.125f;
 }
 
 template <class C, bool W4 = false>
@@ -733,7 +746,54 @@ __device__ __forceinline__ bool wave_is_idle(const Args &p, int m0, int n0) {
   return m0 + wave / C::WAVES_N * C::WM >= p.M || n0 + wave % C::WAVES_N * C::WN >= p.N;
 }
 
-template <class C, bool BF16, bool SPLITK = false, bool W4 = false>
+// The accumulators of a tile between its two MFMA phases: finish(acc, s_row * s_col, zs * w_red + bias), 32x32 block by block.
+// What bounds it is the issue of its instructions: a wave issues one in four cycles, one that needs the result of the one
+// before in eight.  So four values go side by side.  AGPR: the accumulators are in accumulation registers, which the VALU cannot
+// address; where a wave holds at most 128 of them they are ordinary registers (two instructions less per value).
+template <class C, bool BF16, bool AGPR, class Vectors, class Finish>
+__device__ __forceinline__ void convert_tile(v16f (&acc)[C::MI][C::NI], const Vectors &tv, int wm, int wn, int lane, Finish finish) {
+  float srow[C::MI], zsr[C::MI];
+#pragma unroll
+  for (int mi = 0; mi < C::MI; ++mi) {
+    srow[mi] = tv.srow[wm * C::WM + mi * 32 + (lane & 31)];
+    zsr[mi] = tv.zs[wm * C::WM + mi * 32 + (lane & 31)];
+  }
+  if constexpr (AGPR) asm volatile("s_nop 15\n\ts_nop 15");  // the last MFMA results are architecturally visible to the reads below
+#pragma unroll
+  for (int ni = 0; ni < C::NI; ++ni) {
+    float scv[16], wrv[16], bsv[16];
+#pragma unroll
+    for (int g = 0; g < 4; ++g) {
+      const int c = wn * C::WN + ni * 32 + acc_col(g, lane);
+      const float4 sc = *reinterpret_cast<const float4 *>(tv.scol + c);
+      const float4 wr = *reinterpret_cast<const float4 *>(tv.wred + c);
+      const float4 bs = *reinterpret_cast<const float4 *>(tv.bias + c);
+      scv[4 * g] = sc.x, scv[4 * g + 1] = sc.y, scv[4 * g + 2] = sc.z, scv[4 * g + 3] = sc.w;
+      wrv[4 * g] = wr.x, wrv[4 * g + 1] = wr.y, wrv[4 * g + 2] = wr.z, wrv[4 * g + 3] = wr.w;
+      bsv[4 * g] = bs.x, bsv[4 * g + 1] = bs.y, bsv[4 * g + 2] = bs.z, bsv[4 * g + 3] = bs.w;
+    }
+#pragma unroll
+    for (int mi = 0; mi < C::MI; ++mi)
+#pragma unroll
+      for (int g = 0; g < 4; ++g) {
+        float a[4], t[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = AGPR ? agpr_read(acc[mi][ni][4 * g + e]) : acc[mi][ni][4 * g + e];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(zsr[mi], wrv[4 * g + e], bsv[4 * g + e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) a[e] = finish(a[e], srow[mi] * scv[4 * g + e], t[e]);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) acc[mi][ni][4 * g + e] = AGPR ? agpr_write(a[e]) : a[e];
+      }
+  }
+}
+
+// AGPR: see convert_tile
+template <class C>
+constexpr bool acc_in_agpr() { return C::MI * C::NI > 8; }
+
+template <class C, bool BF16, bool SPLITK = false, bool W4 = false, bool AGPR = acc_in_agpr<C>()>
 __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn, uint8_t *smem, int split = 0,
                                             int tile_id = 0, const SplitK *sk = nullptr) {
   using Pipe = Fp6Pipe<C, W4>;
@@ -771,73 +831,50 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
   } else {
     pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64);
   }
-  pipe.start(widen);  // its barrier also makes the vectors visible
+  pipe.start_vectors(widen);
   if constexpr (!SPLITK) {
     // (nothing behind the drain meets another wave)
     if (wave_is_idle<C>(p, m0, n0)) {
+      pipe.start_steps();
       pipe.run_idle();
       pipe.drain();
       return;
     }
   }
-
   v16f acc[C::MI][C::NI];
+  // The start values are an outer sum, K = 2 of the fp32 MFMA: column term times 1 plus 1 times row term, both exact.
+  {
+    const bool upper = lane >= 32;
+    const float once = !SPLITK || split == 0 ? 1.0f : 0.0f;  // (both terms enter once)
+    float rc[C::MI], cc[C::NI];
 #pragma unroll
-  for (int ni = 0; ni < C::NI; ++ni)
+    for (int mi = 0; mi < C::MI; ++mi) rc[mi] = upper ? tv.rowc[wm * C::WM + mi * 32 + (lane & 31)] : once;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      float4 cc = *reinterpret_cast<const float4 *>(tv.colc + wn * C::WN + ni * 32 + acc_col(g, lane));
-      if (SPLITK && split != 0) cc = make_float4(0.0f, 0.0f, 0.0f, 0.0f);  // the column term enters once
+    for (int ni = 0; ni < C::NI; ++ni) cc[ni] = upper ? once : tv.colc[wn * C::WN + ni * 32 + (lane & 31)];
 #pragma unroll
-      for (int mi = 0; mi < C::MI; ++mi)
-        acc[mi][ni][4 * g] = cc.x, acc[mi][ni][4 * g + 1] = cc.y, acc[mi][ni][4 * g + 2] = cc.z, acc[mi][ni][4 * g + 3] = cc.w;
-    }
-  pipe.run_fp6(acc);
+    for (int ni = 0; ni < C::NI; ++ni)
+#pragma unroll
+      for (int mi = 0; mi < C::MI; ++mi) acc[mi][ni] = __builtin_amdgcn_mfma_f32_32x32x2f32(cc[ni], rc[mi], v16f{}, 0, 0, 0);
+  }
+  pipe.start_steps();
+
+  v4i frag[Pipe::NF];
+  pipe.run_fp6(acc, frag);
   if constexpr (SPLITK) {
     pipe.drain();  // the copies past the last step have landed too: the ring is free
     if (!splitk_combine<C, false>(acc, *sk, tile_id, split, smem)) return;
     if (lx.fsteps > 0) {
       pipe.init(smem, p.xbuf, lx, m0 / 64, p.wbuf, lw, (p.n_first + n0) / 64, total, 0, static_cast<int>(lx.fsteps));
       pipe.start();
+      pipe.read16(frag);
     } else {
       pipe.steps0 = pipe.steps = 0;
     }
   }
 
-  // acc = S - colc / 64  ->  f32(integer accumulator) * (s_row * s_col) + (zs * w_red + bias), in place, one 32x32
-  // block at a time.  The zero-point and bias term goes in here, as the addend of the multiply that is needed anyway:
-  // the epilogue then only converts and stores (one instruction per value less than adding it there).
-  float srow[C::MI], rowc[C::MI], zsr[C::MI];
-#pragma unroll
-  for (int mi = 0; mi < C::MI; ++mi) {
-    srow[mi] = tv.srow[wm * C::WM + mi * 32 + (lane & 31)];
-    rowc[mi] = tv.rowc[wm * C::WM + mi * 32 + (lane & 31)];
-    zsr[mi] = tv.zs[wm * C::WM + mi * 32 + (lane & 31)];
-  }
-  asm volatile("s_nop 15\n\ts_nop 15");  // the last MFMA results are architecturally visible to the reads below
-#pragma unroll
-  for (int ni = 0; ni < C::NI; ++ni) {
-    float scv[16], wrv[16], bsv[16];
-#pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int c = wn * C::WN + ni * 32 + acc_col(g, lane);
-      const float4 sc = *reinterpret_cast<const float4 *>(tv.scol + c);
-      const float4 wr = *reinterpret_cast<const float4 *>(tv.wred + c);
-      const float4 bs = *reinterpret_cast<const float4 *>(tv.bias + c);
-      scv[4 * g] = sc.x, scv[4 * g + 1] = sc.y, scv[4 * g + 2] = sc.z, scv[4 * g + 3] = sc.w;
-      wrv[4 * g] = wr.x, wrv[4 * g + 1] = wr.y, wrv[4 * g + 2] = wr.z, wrv[4 * g + 3] = wr.w;
-      bsv[4 * g] = bs.x, bsv[4 * g + 1] = bs.y, bsv[4 * g + 2] = bs.z, bsv[4 * g + 3] = bs.w;
-    }
-#pragma unroll
-    for (int mi = 0; mi < C::MI; ++mi) {
-#pragma unroll
-      for (int v = 0; v < 16; ++v) {
-        const float iacc = __builtin_fmaf(agpr_read(acc[mi][ni][v]), 64.0f, -rowc[mi]);  // exact: integers below 2^24
-        acc[mi][ni][v] = agpr_write(__builtin_fmaf(iacc, srow[mi] * scv[v], __builtin_fmaf(zsr[mi], wrv[v], bsv[v])));
-      }
-    }
-  }
-  pipe.template run_f16<BF16>(acc);
+  // acc, a 64th of the integer accumulator -> f32(integer) * (s_row * s_col) + (zs * w_red + bias), in place
+  convert_tile<C, BF16, AGPR>(acc, tv, wm, wn, lane, [](float a, float s, float t) { return __builtin_fmaf(a, s, t); });
+  pipe.template run_f16<BF16>(acc, frag);
   pipe.drain();
 
   // out = storage(acc), written through a staging area in the (now idle) ring: all MI row
@@ -888,7 +925,7 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
 }
 
 template <class C, bool BF16, bool W4 = false>
-__global__ __launch_bounds__(C::kThreads) void gemm_fused6_kernel(Fused6Args p, int tiles_m, int tiles_n) {
+__global__ __launch_bounds__(C::kThreads, acc_in_agpr<C>() ? 1 : 2) void gemm_fused6_kernel(Fused6Args p, int tiles_m, int tiles_n) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
   if (!tile_of_block<C::BM>(blockIdx.x, tiles_m, tiles_n, tm, tn)) return;
@@ -897,7 +934,7 @@ __global__ __launch_bounds__(C::kThreads) void gemm_fused6_kernel(Fused6Args p, 
 
 // K split over sk.splits workgroups per tile: block b works on tile b % grid_tiles, split b / grid_tiles.
 template <class C, bool BF16>
-__global__ __launch_bounds__(C::kThreads) void gemm_fused6_splitk_kernel(Fused6Args p, int tiles_m, int tiles_n,
+__global__ __launch_bounds__(C::kThreads, 2) void gemm_fused6_splitk_kernel(Fused6Args p, int tiles_m, int tiles_n,
                                                                           SplitK sk) {
   extern __shared__ __align__(16) uint8_t smem[];
   int tm, tn;
@@ -915,9 +952,9 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_split_kernel(Fused6A
   int tm, tn;
   const int kind = grid.template locate<CW::BM>(blockIdx.x, tm, tn);
   if (kind == 1) {
-    fused6_tile<CW, BF16, false, W4>(wide, tm, tn, smem);
+    fused6_tile<CW, BF16, false, W4, true>(wide, tm, tn, smem);
   } else if (kind == 2) {
-    fused6_tile<CT, BF16, false, W4>(tail, tm, tn, smem);
+    fused6_tile<CT, BF16, false, W4, true>(tail, tm, tn, smem);
   }
 }
 
@@ -933,9 +970,9 @@ __global__ __launch_bounds__(CW::kThreads) void gemm_fused6_rest_kernel(Fused6Ar
   int tm, tn;
   const int bid = blockIdx.x;
   if (bid < g.wide_blocks) {
-    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused6_tile<CW, BF16, false, W4>(p, tm, tn, smem);
+    if (tile_of_block<CW::BM>(bid, g.tiles_m_wide, g.tiles_n_wide, tm, tn)) fused6_tile<CW, BF16, false, W4, true>(p, tm, tn, smem);
   } else if (tile_of_block<CT::BM>(bid - g.wide_blocks, g.tiles_m, g.tiles_n, tm, tn)) {
-    fused6_tile<CT, BF16, false, W4>(p, tm, g.first + tn, smem);
+    fused6_tile<CT, BF16, false, W4, true>(p, tm, g.first + tn, smem);
   }
 }
 
