@@ -140,20 +140,29 @@ bool gemv_ok(const FusedArgs &p, bool quant = false) {
 }
 template <int MODE, bool BF16, int MT, int QUANT>
 int launch_gemv_mt(const FusedArgs &p, const GemvQuant &q, hipStream_t st) {
-  auto kern = gemv_decode_kernel<MODE, BF16, MT, QUANT>;
-  if (int rc = prepare(kern, kLdsBytes)) return rc;  // (the size varies with the layer: set once to the most)
   // persistent waves, one column at a time each: two workgroups per CU when their LDS fits twice.  But one where each wave then has
-  // at most two columns of two rows that are quantised here: two workgroups quantise both rows twice on their CU (us per forward,
-  // two / one: 1472 -> 3200 8.6 / 7.2, 1024 -> 4096 8.4 / 7.2, int8 1536 -> 4096 8.7 / 7.8).
+  // at most two columns of rows that are quantised here: two workgroups quantise them twice on their CU.  us per forward, two / one:
+  // one row, int4 2048 -> 4096 6.8 / 5.8, 4096 -> 4096 7.4 / 6.6, 11008 -> 4096 10.2 / 9.3, 16384 -> 4096 12.3 / 11.3, int8 4096 -> 4096 8.2 /
+  // 7.5, 6144 -> 4096 8.9 / 8.5, but with longer int8 rows the stream counts for more, from memory 8192 -> 4096 11.3 / 11.3, 11008 -> 4096
+  // 13.5 / 14.2, 13824 -> 4096 13.8 / 14.7; two rows 1472 -> 3200 8.6 / 7.2, 1024 -> 4096 8.4 / 7.2, int8 1536 -> 4096 8.7 / 7.8.  (One
+  // workgroup for up to four columns of a wave: 8192 -> 8192 10.5 / 10.4, but 13824 -> 5120 11.2 / 11.8.)
   const int64_t fixed = gemv_smem(MT, p.kbytes, p.F) + (QUANT != kGemvNoQuant ? gemv_quant_lds(q.cols, q.num_int).bytes : 0);
-  const bool quantise_bound = QUANT != kGemvNoQuant && MT == 2 && p.N <= 2 * kGemvWaves * num_cus();
+  const bool short_rows = MODE == kInt4 || p.kbytes <= 6400;
+  const bool quantise_bound = QUANT != kGemvNoQuant && (MT == 2 || short_rows) && p.N <= 2 * kGemvWaves * num_cus();
   const int64_t per_cu = 2 * (fixed + 4096) <= kLdsBytes && !quantise_bound ? 2 : 1;
   int64_t grid = (p.N + kGemvWaves - 1) / kGemvWaves;
   if (grid > per_cu * num_cus()) grid = per_cu * num_cus();
   const int64_t smem = fixed + gemv_table_bytes((p.N + kGemvWaves * grid - 1) / (kGemvWaves * grid));
   if (smem > kLdsBytes) return kChainNotHandled;
-  hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kGemvWaves * 64), static_cast<size_t>(smem), st, p, q);
-  return check_launch();
+  auto launch = [&](auto kern) {
+    if (int rc = prepare(kern, kLdsBytes)) return rc;  // (the size varies with the layer: set once to the most)
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kGemvWaves * 64), static_cast<size_t>(smem), st, p, q);
+    return check_launch();
+  };
+  if constexpr (QUANT != kGemvNoQuant) {
+    if (quantise_bound) return launch(gemv_decode_kernel<MODE, BF16, MT, QUANT, true>);
+  }
+  return launch(gemv_decode_kernel<MODE, BF16, MT, QUANT>);
 }
 template <int MODE, bool BF16, int QUANT = kGemvNoQuant>
 int launch_gemv(const FusedArgs &p, const GemvQuant &q, hipStream_t st) {

@@ -222,11 +222,13 @@ __device__ __forceinline__ float wave_total(float v) {
 __device__ __forceinline__ int swap_eights(int v) { return __builtin_amdgcn_update_dpp(0, v, 0x128 /* row_ror:8 */, 0xF, 0xF, false); }
 
 // QUANT: kGemvNoQuant (the token rows' codes come from a quantize launch), kGemvAsym / kGemvSym (quantised here)
+// FEW: at most two columns per wave, in one workgroup per CU
 constexpr int kGemvNoQuant = 0, kGemvAsym = 1, kGemvSym = 2;
-template <int MODE, bool BF16, int MT, int QUANT = kGemvNoQuant>
+template <int MODE, bool BF16, int MT, int QUANT = kGemvNoQuant, bool FEW = false>
 __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs args, GemvQuant quant) {
   static_assert(MODE == kInt4 || MODE == kInt8, "integer codes");
   static_assert(QUANT != kGemvSym || !BF16, "symmetric activations are fp16");
+  static_assert(!FEW || QUANT != kGemvNoQuant, "few columns: the rows are quantised here");
   struct {
     const uint8_t *qx, *qw;
     const uint16_t *meta, *s_col, *w_red, *fp_x, *fp_w, *bias;
@@ -276,6 +278,15 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     static_for<kGemvPieces - 1>([&](auto I) __attribute__((always_inline)) { issue(buf[I.value]); });
   };
 
+  // The epilogue scalars of the workgroup's columns, in the LDS: read back at each column's end, so that no global load whose result
+  // is needed at once sits between the pieces in flight.
+  uint16_t *table = reinterpret_cast<uint16_t *>(smem + MT * (xstride + fstride));
+  // FEW: waves 0 .. 2 request the scales, reduced weights and biases of all of them (16 at most) in front of the quantize: behind it their
+  // trip to memory stands in front of the stream (us per forward, one row: 4096 -> 4096 6.6 -> 6.4, 4096 -> 2560 6.5 -> 6.35).  Of a
+  // long stream it is no part: requested so, 8192 -> 28672 from memory takes 24.9 instead of 24.6.
+  const uint16_t *const given = wave == 1 ? p.w_red : wave == 2 ? p.bias : p.s_col;
+  uint16_t few = 0;
+
   float srow = 0.0f, zs = 0.0f;  // lane m keeps token row m's scale and zero-point term
   if constexpr (QUANT != kGemvNoQuant) {
     // ---- token rows -> codes and outlier values in LDS, quantised here.  The first row and the column map's
@@ -301,12 +312,17 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     __builtin_amdgcn_sched_barrier(0);
     first_pieces();
     __builtin_amdgcn_sched_barrier(0);
+    if constexpr (FEW) {
+      const int n = n_first - wave + (lane & (kGemvWaves - 1)) + ((lane / kGemvWaves) & 1) * step;
+      few = (given ? given : p.s_col)[n < p.N ? n : p.N - 1];  // (by all waves and lanes: under a condition every wait would be for all loads)
+      __builtin_amdgcn_sched_barrier(0);
+    }
     for (int m = 0; m < p.M; ++m) {
       // A second row takes the first one's place (both requested at once at the start were no faster, measured, and
       // cost a second row of LDS); it sits behind the weight pieces, which have long landed by then.
       if (m > 0) gemv_copy_in(quant.x + int64_t(m) * quant.cols, quant.cols * 2, area_lds + ql.raw, wave, lane);
-      // the first row: everything but the weight pieces, which were issued last
-      if (m == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(kGemvPieces - 1));
+      // the first row: everything but the weight pieces and the scalar, which were issued last
+      if (m == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(kGemvPieces - 1 + FEW));
       else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
       __syncthreads();
       float sc, zr;
@@ -343,10 +359,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     zs = p.w_red ? to_f32<BF16>(p.meta[2 * int64_t(m) + 1]) + p.shift * srow : 0.0f;
   }
 
-  // ---- the epilogue scalars of the workgroup's columns -> LDS (a few hundred bytes; read back at each column's end,
-  // so that no global load whose result is needed at once sits between the pieces in flight)
-  uint16_t *table = reinterpret_cast<uint16_t *>(smem + MT * (xstride + fstride));
-  {
+  if constexpr (FEW) {
+    if (wave < 3 && lane < (p.N + step - 1) / step * kGemvWaves) table[lane * 4 + wave] = given ? few : uint16_t(0);  // (16 or 8 columns)
+  } else {
     const int step_ = step;
     const int iters = (p.N - blockIdx.x * kGemvWaves + step_ - 1) / step_;
     for (int j = tid; j < iters * kGemvWaves * 3; j += kGemvWaves * 64) {
@@ -456,7 +471,7 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     }
   };
 
-  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the token rows (and the first pieces) have landed
+  if constexpr (!FEW) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the token rows (and the first pieces) have landed
   __syncthreads();
   while (n < p.N) {  // (a wave's own column sequence; nothing is shared between the waves any more)
     static_for<kGemvPieces>([&](auto I) __attribute__((always_inline)) {
