@@ -132,10 +132,12 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     k0 = split * sk->per;
     k1 = k0 + sk->per < steps ? k0 + sk->per : steps;
   }
-  // This wave's steps: k0 + wave, k0 + wave + WAVES, ...  4 bits: in front of them stand as many empty ones (loaded from the
-  // block's first bytes, not multiplied) as make the loop's rounds whole, so that what is left behind the loop is always the same code, with loads and
-  // waits that do not depend on the remainder.  (With the remainder behind the loop, each of its up to 2 SETS steps with its
-  // loads under a condition, the compiler's waits there were waits for every load.)
+  // This wave's steps: k0 + wave, k0 + wave + WAVES, ...  4 bits: the loop's rounds are whole and what is left behind the loop is
+  // always the same code, with loads and waits that do not depend on the remainder; the first round begins in its middle, `empty`
+  // steps late, with code of its own for each number of them.  (With the remainder behind the loop, each of its up to 2 SETS steps
+  // with its loads under a condition, the compiler's waits there were waits for every load.  With empty steps loaded like the others, from
+  // the block's first bytes, each took its share of what a CU takes in: us per forward 64 x 4096 -> 8192 9.8 -> 9.6, 90 x 5120 -> 5120 11.5 ->
+  // 11.3, 300 x 4544 -> 4544 15.6 -> 15.4.)  Where a wave has no whole round, empty steps are loaded so.
   const int mine = k1 - k0 > wave ? (k1 - k0 - wave + WAVES - 1) / WAVES : 0;
   auto at = [&](int i) { return k0 + wave + i * WAVES; };
   constexpr int kAhead = SETS + 1;                                         // steps in registers: one expanded, the others loaded
@@ -174,7 +176,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     const int step = at(i - empty);
     load_step(f, step < last_step ? step : last_step, i < empty);
   };
-  static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
+  if constexpr (D::KIND != kDirect4) static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
 
   v16f acc[MI][NI];  // fp32 sums (SIX) or int32 bit patterns
 #pragma unroll
@@ -230,8 +232,6 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
       });
     };
     static_assert(SETS % 2 == 0, "operand sets alternate");
-    expand(u[0], set[0]);
-    load_one(set[0], SETS);
     // step i: expanded in u[i & 1]; steps i + 1 .. i + SETS are in the sets (i + k in set (i + k) % SETS)
     auto interleave = [&]() QUIK_INLINE {
       static_for<MI * NI>([&](auto) QUIK_INLINE {
@@ -239,8 +239,8 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         __builtin_amdgcn_sched_group_barrier(0x002, (8 * NF + MI * NI - 1) / (MI * NI), 0);
       });
     };
-    // steps of a round in front of the first real one are skipped; skip: how many
-    auto step = [&](auto S, int skip) QUIK_INLINE {
+    // steps in front of the first real one are skipped; skip: how many
+    auto step = [&](auto S, auto skip) QUIK_INLINE {
       constexpr int next = (S + 1) % SETS;
       if (S >= skip) {
         expand(u[(S + 1) & 1], set[next]);
@@ -251,7 +251,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         expand(u[(S + 1) & 1], set[next]);
       }
     };
-    auto round = [&](int skip) QUIK_INLINE {
+    auto round = [&](auto skip) QUIK_INLINE {
       static_for<SETS>([&](auto S) QUIK_INLINE {
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1) * NF));  // (one wait for the set, not one per fragment)
         __builtin_amdgcn_sched_barrier(0);
@@ -260,8 +260,22 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
       });
     };
-    if (more > 0) round(empty);
-    for (int i = 1; i < more; ++i) round(0);
+    // The first steps and the first round, a copy for every number of empty steps in front of them.
+    if (more > 0) {
+      static_for<SETS>([&](auto E) QUIK_INLINE {
+        if (empty == E) {
+          static_for<SETS - E>([&](auto S) QUIK_INLINE { load_one(set[E + S], E + S); });
+          if constexpr (E == 0) expand(u[0], set[0]);
+          load_one(set[0], SETS);
+          round(E);
+        }
+      });
+    } else {
+      static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
+      expand(u[0], set[0]);
+      load_one(set[0], SETS);
+    }
+    for (int i = 1; i < more; ++i) round(integral_constant<int, 0>{});
     // the last steps: outlier steps are requested in front of them and in place of the sets they leave
     if constexpr (!SPLITK) load_outliers(kNone, kEarly, 0);
     const int skip = more > 0 ? 0 : empty;

@@ -21,9 +21,17 @@
 namespace quik {
 namespace {
 
-using Direct64x32 = DirectCfg<kDirect4, 2, 1, 8>;
+// Steps in flight: what bounds the stream is what a CU takes in, not its latency, so no more than cover it.  us per forward with more
+// and with these: 64x32 tiles, eight and four, 64 x 5120 -> 5120 10.65 / 9.95, 40 x 4096 -> 4096 9.7 / 9.35, 64 x 14336 -> 4096 15.55 / 15.1;
+// 64x64 tiles, four and two, where two of them share a CU, 300 x 4096 -> 4096 14.55 / 14.15, 64 x 5120 -> 20480 19.2 / 18.35, 777 x 4096 ->
+// 1280 16.2 / 15.5, and where one has it alone 64 x 8192 -> 10240 15.3 / 16.1; 128x64 tiles, four and two, of at most two rows of tiles,
+// whose weights each come from beyond the L2, 128 x 5120 -> 13824 17.05 / 16.75 (22.5 / 22.1 from memory), 200 x 5120 -> 5120 15.35 / 15.3
+// (19.3 / 19.15), and of more 500 x 4096 -> 2048 12.65 / 12.95, 300 x 4544 -> 4544 15.4 / 15.35 (17.7 / 18.05).
+using Direct64x32 = DirectCfg<kDirect4, 2, 1, 4>;
 using Direct64x64 = DirectCfg<kDirect4, 2, 2, 4>;
+using Direct64x64Pairs = DirectCfg<kDirect4, 2, 2, 2>;
 using Direct128x64 = DirectCfg<kDirect4, 4, 2, 4>;
+using Direct128x64Few = DirectCfg<kDirect4, 4, 2, 2>;
 
 enum class Tiles4 { k64x32, k64x64, k128x64, kRing };
 
@@ -117,8 +125,12 @@ int run_direct4(const Fused8Args &p, void *workspace, int64_t workspace_bytes, h
   }
   switch (plan_tile4(p.M, p.N, p.K, p.F)) {
     case Tiles4::k64x32: return launch_direct4<Direct64x32, BF16>(p, st);
-    case Tiles4::k64x64: return launch_direct4<Direct64x64, BF16>(p, st);
-    default: return launch_direct4<Direct128x64, BF16>(p, st);
+    case Tiles4::k64x64:
+      if ((p.M + 63) / 64 * ((p.N + 63) / 64) > num_cus()) return launch_direct4<Direct64x64Pairs, BF16>(p, st);
+      return launch_direct4<Direct64x64, BF16>(p, st);
+    default:
+      if (p.M <= 256) return launch_direct4<Direct128x64Few, BF16>(p, st);
+      return launch_direct4<Direct128x64, BF16>(p, st);
   }
 }
 

@@ -10,7 +10,7 @@ from test_gpu_register_streaming import _same_bits
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 OUTLIERS = (0, 32, 64, 96, 192, 224, 256, 288, 544)
-# 128-column groups: two steps each, dealt to four waves.  Rounds of 8 steps (64x32 tiles; 9 in registers), of 4 (64x64 and 128x64; 5)
+# 128-column groups: two steps each, dealt to four waves.  Rounds of 4 steps, 5 in registers
 LONG, SHORT = (13, 15, 17, 18, 19, 20, 33, 34, 35, 36, 37), (1, 2, 3, 9, 10, 11, 12, 13, 17, 18, 19, 26)
 
 
