@@ -49,7 +49,7 @@ struct DirectCfg {
   // and 3 own none
   static constexpr int OM = MI / 2, ON = NI == 1 ? 1 : NI / 2, OWN = OM * ON;
   static constexpr int kOutlierSets = OWN <= 2 ? 16 : 8;  // outlier steps in flight (16: all of them for 256 columns)
-  static constexpr int kEarlySets = KIND != kDirect4 ? 0 : OWN <= 2 ? 8 : 0;  // .. requested in front of the last integer steps
+  static constexpr int kEarlySets = KIND == kDirect6 ? 0 : OWN <= 2 ? 8 : 0;  // .. requested in front of the last integer steps
   static constexpr int kSetsInExchange = OWN <= 2 ? 12 : kOutlierSets;        // .. in front of the exchange (its reads take the registers of the others)
   // exchange: one owned block per round, in two areas by turns
   static constexpr int ROUND_BYTES = WAVES * (WAVES - 1) * 4096;
@@ -132,7 +132,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     k0 = split * sk->per;
     k1 = k0 + sk->per < steps ? k0 + sk->per : steps;
   }
-  // This wave's steps: k0 + wave, k0 + wave + WAVES, ...  4 bits: the loop's rounds are whole and what is left behind the loop is
+  // This wave's steps: k0 + wave, k0 + wave + WAVES, ...  4 and 8 bits: the loop's rounds are whole and what is left behind the loop is
   // always the same code, with loads and waits that do not depend on the remainder; the first round begins in its middle, `empty`
   // steps late, with code of its own for each number of them.  (With the remainder behind the loop, each of its up to 2 SETS steps
   // with its loads under a condition, the compiler's waits there were waits for every load.  With empty steps loaded like the others, from
@@ -140,9 +140,10 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   // 11.3, 300 x 4544 -> 4544 15.6 -> 15.4.)  Where a wave has no whole round, empty steps are loaded so.
   const int mine = k1 - k0 > wave ? (k1 - k0 - wave + WAVES - 1) / WAVES : 0;
   auto at = [&](int i) { return k0 + wave + i * WAVES; };
-  constexpr int kAhead = SETS + 1;                                         // steps in registers: one expanded, the others loaded
+  constexpr bool kWhole = D::KIND != kDirect6;                             // the rounds are whole
+  constexpr int kAhead = SETS + (D::KIND == kDirect4 ? 1 : 0);             // steps in registers: loaded, at 4 bits one more expanded
   const int more = mine > kAhead ? (mine - kAhead + SETS - 1) / SETS : 0;  // rounds of the loop
-  const int empty = D::KIND == kDirect4 ? kAhead + more * SETS - mine : 0;
+  const int empty = kWhole ? kAhead + more * SETS - mine : 0;
   const int last_step = k1 > 0 ? k1 - 1 : 0;
   // per-row and per-column scalars of this thread: requested first, unconditionally (a load under a branch would make
   // the waits of everything around it waits for all loads), used after the main loop
@@ -157,7 +158,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     v_rs = reinterpret_cast<const int32_t *>(p.xbuf + x_sums)[vm];
   }
 
-  // 4 bits: the wave's next step to load, as the lane's offset to the (scalar) addresses of the blocks: one addition per
+  // 4 and 8 bits: the wave's next step to load, as the lane's offset to the (scalar) addresses of the blocks: one addition per
   // step.  The instructions of a step are what bounds it, not the bytes.
   uint32_t pos = head_off + static_cast<uint32_t>(at(kAhead - empty)) * UNIT;
   const uint8_t *const wbase = base[MI / 2] + (NI == 1 ? whalf * 1024 : 0);
@@ -176,7 +177,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     const int step = at(i - empty);
     load_step(f, step < last_step ? step : last_step, i < empty);
   };
-  if constexpr (D::KIND != kDirect4) static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
+  if constexpr (!kWhole) static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
 
   v16f acc[MI][NI];  // fp32 sums (SIX) or int32 bit patterns
 #pragma unroll
@@ -218,21 +219,26 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   constexpr integral_constant<int, 0> kNone{};
   constexpr integral_constant<int, D::kEarlySets> kEarly{};
   constexpr integral_constant<int, OS> kAll{};
-  if constexpr (D::KIND == kDirect4) {
-    // A step's fragments are expanded (eight VALU instructions each) while the step before is multiplied: a wave has its SIMD
-    // to itself, nothing else would run under its products.
+  if constexpr (kWhole) {
+    constexpr bool FOUR = D::KIND == kDirect4;
+    // 4 bits: a step's fragments are expanded (eight VALU instructions each) while the step before is multiplied: a wave has its SIMD
+    // to itself, nothing else would run under its products.  Step i is expanded in u[i & 1], steps i + 1 .. i + SETS are in the sets
+    // (i + k in set (i + k) % SETS); 8 bits: steps i .. i + SETS - 1 are.
     v6i u[2][NF];
     auto expand = [&](v6i (&to)[NF], const DirectFrag<D> &f) QUIK_INLINE {
       static_for<NF>([&](auto J) QUIK_INLINE { to[J] = nib_expand(f.f[J]); });
     };
-    auto multiply = [&](const v6i (&v)[NF]) QUIK_INLINE {
+    auto multiply = [&](const auto &v) QUIK_INLINE {
       static_for<MI * NI>([&](auto I) QUIK_INLINE {
         constexpr int mi = I % MI, ni = I / MI;
-        nib_mma(v[mi], v[MI + ni], acc[mi][ni]);
+        if constexpr (FOUR) {
+          nib_mma(v[mi], v[MI + ni], acc[mi][ni]);
+        } else {
+          FragOps<kInt8>::mma(v[mi], v[MI + ni], acc[mi][ni]);
+        }
       });
     };
     static_assert(SETS % 2 == 0, "operand sets alternate");
-    // step i: expanded in u[i & 1]; steps i + 1 .. i + SETS are in the sets (i + k in set (i + k) % SETS)
     auto interleave = [&]() QUIK_INLINE {
       static_for<MI * NI>([&](auto) QUIK_INLINE {
         __builtin_amdgcn_sched_group_barrier(0x008, 1, 0);
@@ -241,14 +247,18 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
     };
     // steps in front of the first real one are skipped; skip: how many
     auto step = [&](auto S, auto skip) QUIK_INLINE {
-      constexpr int next = (S + 1) % SETS;
-      if (S >= skip) {
-        expand(u[(S + 1) & 1], set[next]);
-        multiply(u[S & 1]);
-        interleave();
-        static_for<NF>([&](auto J) QUIK_INLINE { pin(u[(S + 1) & 1][J]); });
-      } else if (S + 1 == skip) {
-        expand(u[(S + 1) & 1], set[next]);
+      if constexpr (FOUR) {
+        constexpr int next = (S + 1) % SETS;
+        if (S >= skip) {
+          expand(u[(S + 1) & 1], set[next]);
+          multiply(u[S & 1]);
+          interleave();
+          static_for<NF>([&](auto J) QUIK_INLINE { pin(u[(S + 1) & 1][J]); });
+        } else if (S + 1 == skip) {
+          expand(u[(S + 1) & 1], set[next]);
+        }
+      } else {
+        if (S >= skip) multiply(set[S].f);
       }
     };
     auto round = [&](auto skip) QUIK_INLINE {
@@ -256,7 +266,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         __builtin_amdgcn_s_waitcnt(vmcnt_imm((SETS - 1) * NF));  // (one wait for the set, not one per fragment)
         __builtin_amdgcn_sched_barrier(0);
         step(S, skip);
-        load_next(set[(S + 1) % SETS]);
+        load_next(set[FOUR ? (S + 1) % SETS : S]);
         __builtin_amdgcn_sched_barrier(0);  // (left alone the scheduler delays the loads behind later steps' MFMAs)
       });
     };
@@ -265,15 +275,19 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
       static_for<SETS>([&](auto E) QUIK_INLINE {
         if (empty == E) {
           static_for<SETS - E>([&](auto S) QUIK_INLINE { load_one(set[E + S], E + S); });
-          if constexpr (E == 0) expand(u[0], set[0]);
-          load_one(set[0], SETS);
+          if constexpr (FOUR) {
+            if constexpr (E == 0) expand(u[0], set[0]);
+            load_one(set[0], SETS);
+          }
           round(E);
         }
       });
     } else {
       static_for<SETS>([&](auto S) QUIK_INLINE { load_one(set[S], S); });
-      expand(u[0], set[0]);
-      load_one(set[0], SETS);
+      if constexpr (FOUR) {
+        expand(u[0], set[0]);
+        load_one(set[0], SETS);
+      }
     }
     for (int i = 1; i < more; ++i) round(integral_constant<int, 0>{});
     // the last steps: outlier steps are requested in front of them and in place of the sets they leave
@@ -290,16 +304,14 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
         load_outliers(integral_constant<int, sets>{}, integral_constant<int, sets_then>{}, 0);
       __builtin_amdgcn_sched_barrier(0);
     });
-    if (mine > 0) multiply(u[SETS & 1]);
+    if constexpr (FOUR) {
+      if (mine > 0) multiply(u[SETS & 1]);
+    }
   } else {
     auto multiply = [&](const DirectFrag<D> &f) QUIK_INLINE {
       static_for<MI * NI>([&](auto I) QUIK_INLINE {
         constexpr int mi = I % MI, ni = I / MI;
-        if constexpr (D::KIND == kDirect6) {
-          acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.f[MI + ni], f.f[mi], acc[mi][ni], 2, 2, 0, 0, 0, 0);
-        } else {
-          FragOps<kInt8>::mma(f.f[mi], f.f[MI + ni], acc[mi][ni]);
-        }
+        acc[mi][ni] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(f.f[MI + ni], f.f[mi], acc[mi][ni], 2, 2, 0, 0, 0, 0);
       });
     };
     int it = 0;
@@ -335,7 +347,7 @@ __device__ __forceinline__ void direct_tile(const Args &p, int tm, int tn, uint8
   }  // (visible behind the exchange's barrier)
 
   constexpr integral_constant<int, D::kSetsInExchange> kExchanged{};
-  if constexpr (!SPLITK && D::KIND != kDirect4) load_outliers(kNone, kExchanged, 0);
+  if constexpr (!SPLITK && !kWhole) load_outliers(kNone, kExchanged, 0);
 
   // exchange, owned block by owned block: wave w leaves its sums of the block that wave o owns in slot (o, w), o adds the
   // three it finds

@@ -158,11 +158,14 @@ int launch_direct(const Args &p, int splits, void *workspace, hipStream_t st) {
   hipLaunchKernelGGL(kern, dim3(grid), dim3(D::kThreads), D::SMEM, st, p, tiles_m, tiles_n);
   return check_launch();
 }
-// SETS: as many steps in flight as registers allow with two workgroups per CU; more measured no better
+// Steps in flight: what bounds the stream is what a CU takes in, not its latency.  int8, six of 64x64 and ten of 64x32 tiles with the
+// remainder behind the loop / six and ten / four and six / two and four, us per forward: 96 x 8192 -> 8192 21.9 / 21.7 / 21.05 / 22.5, 256 x
+// 4096 -> 4096 14.2 / 14.0 / 13.75 / 14.4, 136 x 13824 -> 5120 29.5 / 29.15 / 28.85 / 31.5, 64 x 1024 -> 4096 8.75 / 8.55 / 8.3 / 8.2, 64 x
+// 4096 -> 4096 from memory 15.55 / 15.1 / 15.1 / 15.15, but 128 x 11008 -> 4096 20.75 / 20.6 / 20.85 / 21.6.
 template <int KIND, bool BF16, class Args>
 int run_direct(const Args &p, const DirectPlan &d, void *workspace, hipStream_t st) {
-  if (d.bn == 64) return launch_direct<DirectCfg<KIND, 2, 2, KIND == kDirect6 ? 4 : 6>, BF16>(p, d.splits, workspace, st);
-  return launch_direct<DirectCfg<KIND, 2, 1, KIND == kDirect6 ? 8 : 10>, BF16>(p, d.splits, workspace, st);
+  if (d.bn == 64) return launch_direct<DirectCfg<KIND, 2, 2, 4>, BF16>(p, d.splits, workspace, st);
+  return launch_direct<DirectCfg<KIND, 2, 1, KIND == kDirect6 ? 8 : 6>, BF16>(p, d.splits, workspace, st);
 }
 
 template <bool BF16>

@@ -41,3 +41,12 @@ def test_step_counts_128x64_of_few_rows(groups):
     F = (0, 32, 256, 288)[groups % 4]
     assert L.load().quik_tile4_tile(M, N, 128 * groups, F) == 0
     _same_bits_as_six(M, N, 128 * groups, F, torch.bfloat16 if groups % 4 == 3 else torch.float16)
+
+
+# int8: steps of 32 columns, two per 64, dealt to four waves; rounds of six steps on 64x32 tiles, of four on 64x64 ones
+@pytest.mark.parametrize("blocks", [1, 2, 3, 5, 8, 11, 12, 13, 14, 15, 17, 19, 21, 22, 24, 25, 26, 37])
+def test_step_counts_int8(blocks):
+    from test_gpu_register_streaming import _same_bits
+    F, dtype = (0, 32, 256, 288)[blocks % 4], torch.bfloat16 if blocks % 3 == 2 else torch.float16
+    _same_bits(50, 300, 64 * blocks, F, 8, dtype)
+    _same_bits(60, 8200, 64 * blocks, F, 8, dtype)
