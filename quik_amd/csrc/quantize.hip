@@ -1237,11 +1237,13 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
 // same pieces, the wave form took 7.3 / 7.8 / 8.5 at 2048 x 4096.
 // (Fillers read beside the outlier values and the ranges of all waves in one LDS round trip, not one after the other:
 // 64 x 8192 3.68 -> 3.57, 2048 x 8192 12.3 -> 12.1, 64 x 28672 5.71 -> 5.48.)
+// (arguments in the order in which they are needed: the first sixteen words are there when a wave starts, the Makefile's
+// kernarg-preload-count)
 template <bool BF16, bool SYM, int JT, bool FOUR>
 __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
-    const uint16_t *__restrict__ x, int64_t rows, int cols, const uint32_t *__restrict__ patch,
-    const uint16_t *__restrict__ fp_col, int nholes, int num_int, int num_fp, uint8_t *__restrict__ dst,
-    uint16_t *__restrict__ meta, float sym_divisor, int64_t first, int64_t count) {
+    const uint16_t *__restrict__ x, int64_t first, int count, int cols, const uint32_t *__restrict__ patch,
+    const uint16_t *__restrict__ fp_col, int nholes, int num_fp, int num_int, float sym_divisor, uint8_t *__restrict__ dst,
+    int64_t rows, uint16_t *__restrict__ meta) {
   static_assert(!(BF16 && SYM), "symmetric activations are fp16");
   extern __shared__ __align__(16) uint8_t img[];
   __shared__ __align__(16) float red[16];  // minimum and maximum of up to eight waves
@@ -1255,7 +1257,7 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
   // Rows [first, first + count); workgroup g takes number (g % 8) * count / 8 + g / 8: a cache line of the operand buffer takes pieces of 4 (heads) or 16
   // (tails) consecutive rows; workgroups are dealt round-robin to the 8 XCDs, so rows that share lines run on the same XCD
   // at about the same time and meet in its L2.
-  const int64_t per_xcd = (count + 7) >> 3, at = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
+  const int per_xcd = (count + 7) >> 3, at = (blockIdx.x & 7) * per_xcd + (blockIdx.x >> 3);
   if (at >= count) return;
   const int64_t row = first + at;
   {
@@ -1800,11 +1802,10 @@ int launch_fp6_row(const void *x, int64_t rows, int64_t cols, const uint8_t *cm,
     for (int64_t first = 0; first < rows; first += kMost) {
       const int64_t count = rows - first < kMost ? rows - first : kMost;
       hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>((count + 7) / 8 * 8)), dim3(64 * W),
-                         static_cast<size_t>(W * jt * 4096), st, static_cast<const uint16_t *>(x), rows,
-                         static_cast<int>(cols), reinterpret_cast<const uint32_t *>(cm + l.off_patch),
-                         reinterpret_cast<const uint16_t *>(cm + l.off_fp), static_cast<int>(words[2]),
-                         static_cast<int>(num_int), static_cast<int>(num_fp), static_cast<uint8_t *>(dst),
-                         static_cast<uint16_t *>(meta), sym_divisor, first, count);
+                         static_cast<size_t>(W * jt * 4096), st, static_cast<const uint16_t *>(x), first,
+                         static_cast<int>(count), static_cast<int>(cols), reinterpret_cast<const uint32_t *>(cm + l.off_patch),
+                         reinterpret_cast<const uint16_t *>(cm + l.off_fp), static_cast<int>(words[2]), static_cast<int>(num_fp),
+                         static_cast<int>(num_int), sym_divisor, static_cast<uint8_t *>(dst), rows, static_cast<uint16_t *>(meta));
       if (int rc = check_launch()) return rc;
     }
     return static_cast<int>(QUIK_OK);
