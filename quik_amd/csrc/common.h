@@ -57,6 +57,8 @@ int64_t tile8_operand_bytes(int64_t rows, int64_t K, int64_t F, int64_t k_multip
 int64_t tile4_operand_bytes(int64_t rows, int64_t K, int64_t F);
 int asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
                       int64_t num_fp, void *out6, void *meta, void *stream, int64_t k_multiple, bool four = false);
+int asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int bits,
+                      void *dst, void *meta, void *fp_x, void *stream);
 int asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int,
                         int64_t num_fp, void *out8, void *meta, void *stream, int64_t k_multiple);
 int sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp,

@@ -124,8 +124,7 @@ extern "C" int quik_layer_forward(const quik_layer *layer, const void *x, int64_
                                                         q, meta, stream, kLayerK8))
       return rc;
   } else {
-    if (int rc = quik_asym_quantize(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, q, meta, fp_x,
-                                    stream))
+    if (int rc = asym_quantize_few(x, l.dtype, rows, l.in_features, l.colmap, l.num_int, l.num_fp, l.bits, q, meta, fp_x, stream))
       return rc;
   }
   if (mid_event) {  // profiling hook: the boundary between the two launches, on the launch stream

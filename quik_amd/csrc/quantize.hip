@@ -1375,6 +1375,148 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
+// A few rows -> row-major codes (calls of the weight-streaming GEMM, gemm_skinny.h), a workgroup of eight waves per row.
+//
+// What bounds such a launch is the chain of one row.  asym_quantize_stream_kernel makes two trips to memory, one for the lane's tables and
+// one for the groups and values that they name, and writes the codes at odd places of the LDS.  Here the row goes to the LDS beside the
+// one trip for all tables, a lane has its groups of 8 columns whole, outliers masked, and what is squeezed is read on the way out: the codes
+// lie in source order, 16 integer columns that follow each other are two aligned reads and a shift (the column map's units), the others
+// are gathered by the byte.  The same arithmetic.
+// us per forward, asym_quantize_stream_kernel / this: int4 4 x 2048 -> 4096 7.0 / 6.6, 8 x 4096 -> 4096 7.55 / 7.25, 16 x 8192 -> 8192 12.5 / 11.85,
+// 3 x 13824 -> 5120 13.9 / 13.1, 16 x 8192 -> 28672 27.5 / 26.9, bf16 8 x 4096 -> 4096 7.95 / 7.5, int8 16 x 13824 -> 5120 19.4 / 18.15, 24 x
+// 28672 -> 8192 43.7 / 42.05.
+constexpr int kFewThreads = 512, kFewRows = 32;
+__host__ __device__ inline int64_t few_raw_bytes(int64_t cols) { return (cols * 2 + 1023) / 1024 * 1024; }
+__host__ __device__ inline int64_t few_lds_bytes(int64_t cols) { return few_raw_bytes(cols) + (cols + 47) / 16 * 16; }
+
+template <int BITS, bool BF16, int NV>
+__global__ __launch_bounds__(kFewThreads) void quantize_few_rows_kernel(
+    const uint16_t *__restrict__ x, const uint32_t *__restrict__ grp, const uint16_t *__restrict__ unit, int cols, int num_int, int num_fp,
+    int ngather, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
+    uint8_t *__restrict__ dst, uint16_t *__restrict__ fp_x, uint16_t *__restrict__ meta) {
+  extern __shared__ __align__(16) uint8_t lds[];
+  __shared__ __align__(16) float red[16];
+  constexpr int T = kFewThreads, W = T / 64, NU = (NV + 1) / 2;
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x;
+  const int nvec = cols >> 3, nu = num_int >> 4;
+  uint8_t *const raw = lds, *const stage = lds + few_raw_bytes(cols);
+  {
+    const uint8_t *rp = uniform_row(x, row, cols);
+    const uint32_t lds0 = lds_address(raw);
+#pragma unroll
+    for (int k = 0; k < NV; ++k) {  // (a kilobyte per wave and turn, past the row: its last group)
+      const int q = wave + k * W, g = q * 64 + lane;
+      if (q * 64 < nvec) dma_load16(rp, static_cast<uint32_t>(g < nvec ? g : nvec - 1) * 16u, lds0 + q * 1024);
+    }
+  }
+  // (unconditional loads from valid addresses, in flight together)
+  uint32_t info[NV], first[NU];
+#pragma unroll
+  for (int k = 0; k < NV; ++k) info[k] = grp[tid + k * T < nvec ? tid + k * T : 0];
+#pragma unroll
+  for (int k = 0; k < NU; ++k) first[k] = unit[tid + k * T < nu ? tid + k * T : 0];
+  const uint16_t *const spare = reinterpret_cast<const uint16_t *>(grp);  // (always there; the other tables may be empty)
+  const bool has_g = tid < ngather, has_f = tid < num_fp;
+  const uint32_t gunit = *(has_g ? gather_unit + tid : spare), fcol = *(has_f ? fp_col + tid : spare);
+  const uint4 *const gc = reinterpret_cast<const uint4 *>(has_g ? gather_cols + 16 * tid : spare);
+  const uint4 ga = gc[0], gb = gc[1];
+  if constexpr (!BF16) treat_all_nans_alike();  // pk_min_f16 / pk_max_f16 on the raw row
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+  __syncthreads();
+
+  auto value = [&](uint32_t c) { return reinterpret_cast<const uint16_t *>(raw)[c]; };
+  if (has_f) fp_x[static_cast<int64_t>(row) * num_fp + tid] = value(fcol);
+  for (int f = tid + T; f < num_fp; f += T) fp_x[static_cast<int64_t>(row) * num_fp + f] = value(fp_col[f]);
+  uint4 v[NV];
+  uint32_t pmn = 0x7C007C00u, pmx = 0xFC00FC00u;
+  float mn = __builtin_inff(), mx = -__builtin_inff();
+#pragma unroll
+  for (int k = 0; k < NV; ++k) {
+    const int g = tid + k * T;
+    v[k] = *reinterpret_cast<const uint4 *>(raw + (g < nvec ? g : 0) * 16);
+    const uint32_t w[4] = {v[k].x, v[k].y, v[k].z, v[k].w}, skip = g < nvec ? info[k] : 0xFFu;  // (bit e: column e is an outlier)
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(skip), 2 * t, 1));
+      const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(skip), 2 * t + 1, 1));
+      if constexpr (!BF16) {
+        const uint32_t m = w[t] | __builtin_amdgcn_perm(hi, lo, 0x07060100u);  // outliers: a NaN, which is skipped
+        pmn = pk_min_f16(pmn, m), pmx = pk_max_f16(pmx, m);
+      } else {
+        const float f0 = __uint_as_float((w[t] << 16) | lo), f1 = __uint_as_float((w[t] & 0xFFFF0000u) | hi);
+        mn = fminf(mn, fminf(f0, f1)), mx = fmaxf(mx, fmaxf(f0, f1));
+      }
+    }
+  }
+  if constexpr (!BF16) {
+    const h2 a = __builtin_bit_cast(h2, pmn), b = __builtin_bit_cast(h2, pmx);
+    mn = fminf(static_cast<float>(a.x), static_cast<float>(a.y)), mx = fmaxf(static_cast<float>(b.x), static_cast<float>(b.y));
+  }
+  mn = wave_min(mn), mx = wave_max(mx);
+  if (lane == 0) red[wave] = mn, red[W + wave] = mx;
+  __syncthreads();
+  float part[2 * W];
+#pragma unroll
+  for (int k = 0; k < 2 * W / 4; ++k) {
+    const float4 r = *reinterpret_cast<const float4 *>(red + 4 * k);
+    part[4 * k] = r.x, part[4 * k + 1] = r.y, part[4 * k + 2] = r.z, part[4 * k + 3] = r.w;
+  }
+#pragma unroll
+  for (int w = 0; w < W; ++w) mn = fminf(mn, part[w]), mx = fmaxf(mx, part[W + w]);
+  RowQuant<BF16> rq;
+  rq.init(mn, mx, BITS);
+  if (tid == 0) meta[2 * row] = rq.scale_bits, meta[2 * row + 1] = rq.zero_bits;
+  auto codes = [&](auto slow_c) {
+#pragma unroll
+    for (int k = 0; k < NV; ++k)
+      if (tid + k * T < nvec) *reinterpret_cast<uint2 *>(stage + (tid + k * T) * 8) = group_codes<BITS, BF16, decltype(slow_c)::value>(v[k], rq);
+  };
+  if (__builtin_amdgcn_readfirstlane(rq.slow ? 1 : 0)) {
+    codes(std::true_type{});
+  } else {
+    codes(std::false_type{});
+  }
+  __syncthreads();
+
+  uint8_t *const drow = dst + static_cast<int64_t>(row) * (BITS == 4 ? num_int >> 1 : num_int);
+  auto put = [&](int u, const uint4 &c) {
+    if constexpr (BITS == 8) {
+      *reinterpret_cast<uint4 *>(drow + u * 16) = c;
+    } else {
+      // byte pairs (c0, c1) -> c0 | c1 << 4: t = w | w >> 4 leaves them in bytes 0 and 2
+      const uint32_t t0 = c.x | (c.x >> 4), t1 = c.y | (c.y >> 4), t2 = c.z | (c.z >> 4), t3 = c.w | (c.w >> 4);
+      *reinterpret_cast<uint2 *>(drow + u * 8) = make_uint2(__builtin_amdgcn_perm(t1, t0, 0x06040200u), __builtin_amdgcn_perm(t3, t2, 0x06040200u));
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < NU; ++k) {
+    const uint32_t c0 = first[k];
+    if (tid + k * T < nu && c0 != 0xFFFFu) {
+      // two aligned reads, a shift by whole words (bit-mask selects) and by bytes
+      const uint4 a = *reinterpret_cast<const uint4 *>(stage + (c0 & ~15u)), b = *reinterpret_cast<const uint4 *>(stage + (c0 & ~15u) + 16);
+      uint32_t w[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
+      const uint32_t by2 = 0u - ((c0 >> 3) & 1u), by1 = 0u - ((c0 >> 2) & 1u);
+#pragma unroll
+      for (int t = 0; t < 6; ++t) w[t] = (w[t + 2] & by2) | (w[t] & ~by2);
+#pragma unroll
+      for (int t = 0; t < 5; ++t) w[t] = (w[t + 1] & by1) | (w[t] & ~by1);
+      put(tid + k * T, make_uint4(__builtin_amdgcn_alignbyte(w[1], w[0], c0), __builtin_amdgcn_alignbyte(w[2], w[1], c0),
+                                  __builtin_amdgcn_alignbyte(w[3], w[2], c0), __builtin_amdgcn_alignbyte(w[4], w[3], c0)));
+    }
+  }
+  if (has_g) {
+    const uint32_t at[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+    uint32_t c[4];
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+      const uint32_t b0 = stage[at[2 * t] & 0xFFFFu], b1 = stage[at[2 * t] >> 16], b2 = stage[at[2 * t + 1] & 0xFFFFu], b3 = stage[at[2 * t + 1] >> 16];
+      c[t] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
+    }
+    put(static_cast<int>(gunit), make_uint4(c[0], c[1], c[2], c[3]));
+  }
+}
+
+// ---------------------------------------------------------------------------------------
 // Stand-alone quantize straight from the index lists: no column map, one launch.
 //
 // What bounded the two launches it replaces at a few hundred rows was the map: one workgroup builds it, 6.3 us in front of
@@ -1961,6 +2103,44 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
   auto go = [&](auto launch) { return launch(x, rows, cols, cm, l, num_int, num_fp, out6, meta, st, 1.0f); };
   if (four) return dtype == QUIK_F16 ? go(launch_fp6_row<false, false, true>) : go(launch_fp6_row<true, false, true>);
   return dtype == QUIK_F16 ? go(launch_fp6_row<false, false, false>) : go(launch_fp6_row<true, false, false>);
+}
+
+// A layer's few rows: quantize_few_rows_kernel where it takes the shape, else as quik_asym_quantize.
+int quik::asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int bits,
+                            void *dst, void *meta, void *fp_x, void *stream) {
+  uint32_t words[4];
+  hipStream_t st = as_stream(stream);
+  if (rows > 0 && rows <= kFewRows && cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && num_fp >= 0 && num_int + num_fp == cols && x &&
+      colmap && dst && meta && (num_fp == 0 || fp_x) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
+      colmap_words(colmap, cols, num_int, num_fp, st, words) == QUIK_OK && (words[0] & kColmapStreams) && words[3] <= kFewThreads) {
+    const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
+    const uint8_t *cm = static_cast<const uint8_t *>(colmap);
+    auto go = [&](auto kern) {
+      if (int rc = prepare(kern, static_cast<int>(few_lds_bytes(kStreamMaxCols)))) return rc;
+      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(rows)), dim3(kFewThreads), static_cast<size_t>(few_lds_bytes(cols)), st,
+                         static_cast<const uint16_t *>(x), reinterpret_cast<const uint32_t *>(cm + l.off_grp),
+                         reinterpret_cast<const uint16_t *>(cm + l.off_unit), static_cast<int>(cols), static_cast<int>(num_int),
+                         static_cast<int>(num_fp), static_cast<int>(words[3]), reinterpret_cast<const uint16_t *>(cm + l.off_fp),
+                         reinterpret_cast<const uint16_t *>(cm + l.off_gunit), reinterpret_cast<const uint16_t *>(cm + l.off_gcols),
+                         static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x), static_cast<uint16_t *>(meta));
+      return check_launch();
+    };
+    auto wide = [&](auto bits_c, auto bf16_c) {
+      constexpr int B = bits_c;
+      constexpr bool BF = bf16_c;
+      const int64_t groups = cols / 8;
+      if (groups <= 512) return go(quantize_few_rows_kernel<B, BF, 1>);
+      if (groups <= 1024) return go(quantize_few_rows_kernel<B, BF, 2>);
+      if (groups <= 2048) return go(quantize_few_rows_kernel<B, BF, 4>);
+      return go(quantize_few_rows_kernel<B, BF, 8>);
+    };
+    using std::integral_constant;
+    if (bits == 4 && dtype == QUIK_F16) return wide(integral_constant<int, 4>{}, std::false_type{});
+    if (bits == 4 && dtype == QUIK_BF16) return wide(integral_constant<int, 4>{}, std::true_type{});
+    if (bits == 8 && dtype == QUIK_F16) return wide(integral_constant<int, 8>{}, std::false_type{});
+    if (bits == 8 && dtype == QUIK_BF16) return wide(integral_constant<int, 8>{}, std::true_type{});
+  }
+  return quik_asym_quantize(x, dtype, rows, cols, colmap, num_int, num_fp, bits, dst, meta, fp_x, stream);
 }
 
 extern "C" int quik_asym_quantize_tile4(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
