@@ -1375,7 +1375,8 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// A few rows -> row-major codes (calls of the weight-streaming GEMM, gemm_skinny.h), a workgroup of eight waves per row.
+// Rows -> row-major codes of a layer's few rows (calls of the weight-streaming GEMM, gemm_skinny.h), or int8 operand buffers in tile order, a
+// workgroup of eight waves per row.
 //
 // What bounds such a launch is the chain of one row.  asym_quantize_stream_kernel makes two trips to memory, one for the lane's tables and
 // one for the groups and values that they name, and writes the codes at odd places of the LDS.  Here the row goes to the LDS beside the
@@ -1384,22 +1385,29 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
 // are gathered by the byte.  The same arithmetic.
 // us per forward, asym_quantize_stream_kernel / this: int4 4 x 2048 -> 4096 7.0 / 6.6, 8 x 4096 -> 4096 7.55 / 7.25, 16 x 8192 -> 8192 12.5 / 11.85,
 // 3 x 13824 -> 5120 13.9 / 13.1, 16 x 8192 -> 28672 27.5 / 26.9, bf16 8 x 4096 -> 4096 7.95 / 7.5, int8 16 x 13824 -> 5120 19.4 / 18.15, 24 x
-// 28672 -> 8192 43.7 / 42.05.
-constexpr int kFewThreads = 512, kFewRows = 32;
-__host__ __device__ inline int64_t few_raw_bytes(int64_t cols) { return (cols * 2 + 1023) / 1024 * 1024; }
-__host__ __device__ inline int64_t few_lds_bytes(int64_t cols) { return few_raw_bytes(cols) + (cols + 47) / 16 * 16; }
+// 28672 -> 8192 43.7 / 42.05.  Tile order: 64 x 4096 -> 4096 11.1 / 10.6, 64 x 8192 -> 8192 18.25 / 17.3, 256 x 4096 -> 4096 14.95 / 14.35, 1024 x 13824 ->
+// 512 36.5 / 35.4, 2048 x 8192 -> 512 32.4 / 30.9, 8192 x 4096 -> 512 56.0 / 54.9, bf16 64 x 11008 -> 4096 18.6 / 18.0, 2048 x 13824 -> 512 51.85 / 48.0,
+// 1536 x 28672 -> 512 97.25 / 95.3; against quantize_tile8_ring_kernel: see asym_quantize_tile8.
+constexpr int kUnitThreads = 512, kFewRows = 32;
+__host__ __device__ inline int64_t unit_raw_bytes(int64_t cols) { return (cols * 2 + 1023) / 1024 * 1024; }
+__host__ __device__ inline int64_t unit_lds_bytes(int64_t cols) { return unit_raw_bytes(cols) + (cols + 47) / 16 * 16; }
 
-template <int BITS, bool BF16, int NV>
-__global__ __launch_bounds__(kFewThreads) void quantize_few_rows_kernel(
+// TILED (int8): into an operand buffer in tile order (gemm_tile8.h), outlier values included.
+template <int BITS, bool BF16, int NV, bool TILED>
+__global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
     const uint16_t *__restrict__ x, const uint32_t *__restrict__ grp, const uint16_t *__restrict__ unit, int cols, int num_int, int num_fp,
-    int ngather, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
+    int ngather, int rows, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
     uint8_t *__restrict__ dst, uint16_t *__restrict__ fp_x, uint16_t *__restrict__ meta) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ __align__(16) float red[16];
-  constexpr int T = kFewThreads, W = T / 64, NU = (NV + 1) / 2;
-  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x;
+  constexpr int T = kUnitThreads, W = T / 64, NU = (NV + 1) / 2;
+  static_assert(!TILED || BITS == 8, "tile order: int8");
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  // (tile order: rows that share cache lines of the operand buffer on one XCD)
+  const int row = TILED ? (blockIdx.x & 7) * ((rows + 7) >> 3) + (blockIdx.x >> 3) : blockIdx.x;
+  if (row >= rows) return;
   const int nvec = cols >> 3, nu = num_int >> 4;
-  uint8_t *const raw = lds, *const stage = lds + few_raw_bytes(cols);
+  uint8_t *const raw = lds, *const stage = lds + unit_raw_bytes(cols);
   {
     const uint8_t *rp = uniform_row(x, row, cols);
     const uint32_t lds0 = lds_address(raw);
@@ -1425,8 +1433,14 @@ __global__ __launch_bounds__(kFewThreads) void quantize_few_rows_kernel(
   __syncthreads();
 
   auto value = [&](uint32_t c) { return reinterpret_cast<const uint16_t *>(raw)[c]; };
-  if (has_f) fp_x[static_cast<int64_t>(row) * num_fp + tid] = value(fcol);
-  for (int f = tid + T; f < num_fp; f += T) fp_x[static_cast<int64_t>(row) * num_fp + f] = value(fp_col[f]);
+  const Tile8Layout l8 = tile8_layout(rows, num_int, num_fp);
+  auto outlier = [&](int f) -> uint16_t * {
+    if constexpr (TILED)
+      return reinterpret_cast<uint16_t *>(dst + tile8_offset(l8, row, l8.steps + (f >> 4), (f >> 3) & 1)) + (f & 7);
+    return fp_x + static_cast<int64_t>(row) * num_fp + f;
+  };
+  if (has_f) *outlier(tid) = value(fcol);
+  for (int f = tid + T; f < num_fp; f += T) *outlier(f) = value(fp_col[f]);
   uint4 v[NV];
   uint32_t pmn = 0x7C007C00u, pmx = 0xFC00FC00u;
   float mn = __builtin_inff(), mx = -__builtin_inff();
@@ -1480,7 +1494,9 @@ __global__ __launch_bounds__(kFewThreads) void quantize_few_rows_kernel(
 
   uint8_t *const drow = dst + static_cast<int64_t>(row) * (BITS == 4 ? num_int >> 1 : num_int);
   auto put = [&](int u, const uint4 &c) {
-    if constexpr (BITS == 8) {
+    if constexpr (TILED) {
+      *reinterpret_cast<uint4 *>(dst + tile8_offset(l8, row, u >> 1, u & 1)) = c;
+    } else if constexpr (BITS == 8) {
       *reinterpret_cast<uint4 *>(drow + u * 16) = c;
     } else {
       // byte pairs (c0, c1) -> c0 | c1 << 4: t = w | w >> 4 leaves them in bytes 0 and 2
@@ -2105,40 +2121,47 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
   return dtype == QUIK_F16 ? go(launch_fp6_row<false, false, false>) : go(launch_fp6_row<true, false, false>);
 }
 
-// A layer's few rows: quantize_few_rows_kernel where it takes the shape, else as quik_asym_quantize.
+namespace {
+// words: the column map's, which streams
+bool units_ok(const void *x, int64_t cols, int64_t num_int, const void *dst, const uint32_t (&words)[4]) {
+  return cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(dst) % 16 == 0 && (words[0] & kColmapStreams) && words[3] <= kUnitThreads;
+}
+template <int BITS, bool BF16, bool TILED>
+int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int ngather, void *dst,
+                    void *meta, void *fp_x, hipStream_t st) {
+  const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
+  const uint8_t *cm = static_cast<const uint8_t *>(colmap);
+  auto go = [&](auto kern) {
+    if (int rc = prepare(kern, static_cast<int>(unit_lds_bytes(kStreamMaxCols)))) return rc;
+    hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(TILED ? (rows + 7) / 8 * 8 : rows)), dim3(kUnitThreads),
+                       static_cast<size_t>(unit_lds_bytes(cols)), st, static_cast<const uint16_t *>(x),
+                       reinterpret_cast<const uint32_t *>(cm + l.off_grp), reinterpret_cast<const uint16_t *>(cm + l.off_unit),
+                       static_cast<int>(cols), static_cast<int>(num_int), static_cast<int>(num_fp), ngather, static_cast<int>(rows),
+                       reinterpret_cast<const uint16_t *>(cm + l.off_fp), reinterpret_cast<const uint16_t *>(cm + l.off_gunit),
+                       reinterpret_cast<const uint16_t *>(cm + l.off_gcols), static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x),
+                       static_cast<uint16_t *>(meta));
+    return check_launch();
+  };
+  const int64_t groups = cols / 8;
+  if (groups <= 512) return go(quantize_units_kernel<BITS, BF16, 1, TILED>);
+  if (groups <= 1024) return go(quantize_units_kernel<BITS, BF16, 2, TILED>);
+  if (groups <= 2048) return go(quantize_units_kernel<BITS, BF16, 4, TILED>);
+  return go(quantize_units_kernel<BITS, BF16, 8, TILED>);
+}
+}  // namespace
+
+// A layer's few rows: quantize_units_kernel where it takes the shape, else as quik_asym_quantize.
 int quik::asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int bits,
                             void *dst, void *meta, void *fp_x, void *stream) {
   uint32_t words[4];
   hipStream_t st = as_stream(stream);
-  if (rows > 0 && rows <= kFewRows && cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && num_fp >= 0 && num_int + num_fp == cols && x &&
-      colmap && dst && meta && (num_fp == 0 || fp_x) && reinterpret_cast<uintptr_t>(x) % 16 == 0 && reinterpret_cast<uintptr_t>(dst) % 16 == 0 &&
-      colmap_words(colmap, cols, num_int, num_fp, st, words) == QUIK_OK && (words[0] & kColmapStreams) && words[3] <= kFewThreads) {
-    const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
-    const uint8_t *cm = static_cast<const uint8_t *>(colmap);
-    auto go = [&](auto kern) {
-      if (int rc = prepare(kern, static_cast<int>(few_lds_bytes(kStreamMaxCols)))) return rc;
-      hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(rows)), dim3(kFewThreads), static_cast<size_t>(few_lds_bytes(cols)), st,
-                         static_cast<const uint16_t *>(x), reinterpret_cast<const uint32_t *>(cm + l.off_grp),
-                         reinterpret_cast<const uint16_t *>(cm + l.off_unit), static_cast<int>(cols), static_cast<int>(num_int),
-                         static_cast<int>(num_fp), static_cast<int>(words[3]), reinterpret_cast<const uint16_t *>(cm + l.off_fp),
-                         reinterpret_cast<const uint16_t *>(cm + l.off_gunit), reinterpret_cast<const uint16_t *>(cm + l.off_gcols),
-                         static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x), static_cast<uint16_t *>(meta));
-      return check_launch();
-    };
-    auto wide = [&](auto bits_c, auto bf16_c) {
-      constexpr int B = bits_c;
-      constexpr bool BF = bf16_c;
-      const int64_t groups = cols / 8;
-      if (groups <= 512) return go(quantize_few_rows_kernel<B, BF, 1>);
-      if (groups <= 1024) return go(quantize_few_rows_kernel<B, BF, 2>);
-      if (groups <= 2048) return go(quantize_few_rows_kernel<B, BF, 4>);
-      return go(quantize_few_rows_kernel<B, BF, 8>);
-    };
-    using std::integral_constant;
-    if (bits == 4 && dtype == QUIK_F16) return wide(integral_constant<int, 4>{}, std::false_type{});
-    if (bits == 4 && dtype == QUIK_BF16) return wide(integral_constant<int, 4>{}, std::true_type{});
-    if (bits == 8 && dtype == QUIK_F16) return wide(integral_constant<int, 8>{}, std::false_type{});
-    if (bits == 8 && dtype == QUIK_BF16) return wide(integral_constant<int, 8>{}, std::true_type{});
+  if (rows > 0 && rows <= kFewRows && num_int > 0 && num_fp >= 0 && num_int + num_fp == cols && (bits == 4 || bits == 8) &&
+      (dtype == QUIK_F16 || dtype == QUIK_BF16) && x && colmap && dst && meta && (num_fp == 0 || fp_x) &&
+      colmap_words(colmap, cols, num_int, num_fp, st, words) == QUIK_OK && units_ok(x, cols, num_int, dst, words)) {
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, static_cast<int>(words[3]), dst, meta, fp_x, st); };
+    if (bits == 4) return dtype == QUIK_F16 ? go(launch_units<4, false, false>) : go(launch_units<4, true, false>);
+    return dtype == QUIK_F16 ? go(launch_units<8, false, false>) : go(launch_units<8, true, false>);
   }
   return quik_asym_quantize(x, dtype, rows, cols, colmap, num_int, num_fp, bits, dst, meta, fp_x, stream);
 }
@@ -2164,9 +2187,17 @@ int quik::asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t co
   uint32_t words[4];
   if (int rc = colmap_words(colmap, cols, num_int, num_fp, as_stream(stream), words)) return rc;
   if (!(words[0] & kColmapStreams)) return QUIK_ERR_COLMAP;
+  hipStream_t st = as_stream(stream);
+  // fp16 rows of more than 16384 columns, eight groups per lane, where a CU has more than one: quantize_tile8_ring_kernel, whose next row is
+  // on its way while one is worked on (us per forward, units / ring: 256 x 28672 -> 1024 29.2 / 29.7, 512 x 28672 -> 512 40.65 / 39.45, 2048 x
+  // 28672 -> 512 100 / 85; 768 x 16384 -> 512 32.55 / 34.05, 2048 x 13824 -> 512 46.05 / 47.15)
+  // (a grid holds fewer than 2^32 threads)
+  if (rows <= (1 << 20) && (dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) && units_ok(x, cols, num_int, out8, words)) {
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, static_cast<int>(words[3]), out8, meta, nullptr, st); };
+    return dtype == QUIK_F16 ? go(launch_units<8, false, true>) : go(launch_units<8, true, true>);
+  }
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
-  hipStream_t st = as_stream(stream);
   return dtype == QUIK_F16 ? launch_asym<uint16_t, 8, false>(x, rows, cols, cm, l, num_int, num_fp, out8, meta, nullptr,
                                                             st, true, words[1], words[3])
                            : launch_asym<uint16_t, 8, true>(x, rows, cols, cm, l, num_int, num_fp, out8, meta, nullptr,

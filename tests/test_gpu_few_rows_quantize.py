@@ -1,4 +1,4 @@
-"""Quantize of a layer's few rows (quantize_few_rows_kernel in csrc/quantize.hip): codes, scales, zero points and outlier values of a
+"""Quantize of a layer's few rows (quantize_units_kernel in csrc/quantize.hip): codes, scales, zero points and outlier values of a
 forward's workspace, bit for bit those of the stand-alone operation, which other tests hold against the oracle."""
 import numpy as np
 import pytest
@@ -44,3 +44,45 @@ def test_workspace_is_what_the_operation_gives(rows, K, F, bits, runs, dtype):
         want = want.contiguous().view(torch.uint8).reshape(-1)
         assert torch.equal(ws[at:at + want.numel()], want)
         at += up(want.numel())
+
+
+# (rows: up to and beyond those of fp16 rows of more than 16384 columns)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,K,F,runs", [(1, 64, 32, False), (33, 480, 32, True), (65, 4096, 32, False), (130, 4064, 0, False), (40, 8192, 32, True),
+                                           (257, 7952, 256, False), (70, 16128, 256, True), (300, 16384, 32, False), (256, 16512, 128, False),
+                                           (257, 16512, 128, False), (35, 32512, 256, False), (9, 31744, 1024, False)])
+def test_tile_order_holds_what_the_operation_gives(rows, K, F, runs, dtype):
+    """The buffer's chunks (layout restated from quik_amd/csrc/fp6_format.h) against the codes and values in row order."""
+    from quik_amd import asymmetric
+    rng = np.random.default_rng(K + F + rows)
+    mod, _, _, fi, ii, _ = _layer(rng, 16, K + F, F, 8, dtype, runs)
+    x = rng.standard_normal((rows, K + F)).astype(np.float32)
+    x[:, fi] *= 50
+    x[0, ii[3]], x[rows // 2, ii[0]], x[rows // 2, ii[-1]] = np.nan, 6e4, -6e4
+    x[rows - 1, ii[K // 2]] = np.inf
+    xt = torch.from_numpy(x).to(DEV, dtype)
+    q, meta, fp_x = asymmetric.quantize_mapped(xt, mod._column_map(), K, F, 8)
+    buf, meta8 = asymmetric.quantize_mapped_tile8(xt, mod._column_map(), K, F) if K % 64 == 0 else _through_the_layer(mod, xt)
+    assert torch.equal(meta8.view(torch.int16)[:2 * rows], meta.view(torch.int16))
+    steps, r = (K + 63) // 64 * 2, torch.arange(rows, device=DEV)
+    units = buf[:(rows + 63) // 64 * (steps + F // 16) * 2048].view(-1, steps + F // 16, 2, 32, 2, 16)   # block, step, half, row, slot
+    swap = (r >> 3) & 1
+    for want, first in ((q.view(torch.uint8), 0), (fp_x.contiguous().view(torch.uint8).reshape(rows, -1), steps)):
+        chunks = want.shape[1] // 16
+        c = torch.arange(chunks, device=DEV)
+        got = units[(r >> 6)[:, None], first + (c >> 1)[None], ((r >> 5) & 1)[:, None], (r & 31)[:, None], (c & 1)[None] ^ swap[:, None]]
+        assert torch.equal(got.reshape(rows, -1), want)
+
+
+def _through_the_layer(mod, xt):
+    """Operand buffer and scales in the workspace of a forward on the tile-ordered path."""
+    import ctypes
+    from quik_amd import _lib as L
+    lib, rows = L.load(), xt.shape[0]
+    desc, _ = mod._descriptor(True)
+    n = lib.quik_layer_workspace_bytes(ctypes.byref(desc), rows)
+    ws, out = torch.zeros(n, dtype=torch.uint8, device=DEV), torch.empty(rows, mod.out_features, dtype=xt.dtype, device=DEV)
+    L.check(lib.quik_layer_forward(ctypes.byref(desc), xt.data_ptr(), rows, ws.data_ptr(), n, None, 0, out.data_ptr(), None, L.stream()), "forward")
+    K, F = mod.int_features_num, mod.fp_features_num
+    at = ((rows + 63) // 64 * ((K + 63) // 64 * 2 + F // 16) * 2048 + 255) // 256 * 256
+    return ws, ws[at:at + 4 * rows].view(xt.dtype)
