@@ -14,8 +14,8 @@
 // column), then each lane gathers two consecutive destination codes per step from LDS through a
 // compact source-column table and stores one packed byte (int4) or two bytes (int8).
 //
-// The quotient.  r = 1/scale is one IEEE division per row.  The gather kernel and the bf16
-// streaming path use q = d*r; e = fma(-q, s, d); q' = fma(e, r, q): q' is within
+// The quotient.  r = 1/scale is one IEEE division per row.  Pairs of bf16 values take d*r, two roundings
+// away (quotient_pair_bf16).  The gather kernel uses q = d*r; e = fma(-q, s, d); q' = fma(e, r, q): q' is within
 // 2^-24(1+eps) of d/s relative, while d/s with 11-bit (8-bit for bf16) significands stays more
 // than 2^-23 relative away from every rounding boundary of the storage type, so storage(q')
 // equals the correctly rounded storage(d/s).  The fp16 streaming path uses fp16(d*r) without
@@ -1080,6 +1080,24 @@ __device__ __forceinline__ uint32_t level_pair_fast(uint32_t w, const RQ &rq) {
   return __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2, tb) + h2{magic, magic});
 }
 
+// The levels of four bf16 values in the bytes of the result, rows on the fast path.  As above: t = max(t, 0), no upper clamp (x - zero <= max -
+// min, rounded up by at most 2^-9, and the scale is at least (max - min) / 15 less 2^-9: t is at most 15.125), and t + 1.5 2^23 holds rne(t) in its low byte.
+// (v_max_f32 by hand: the compiler's fmaxf first quiets an operand that may be a signalling NaN; a converted value is none.  Plain VALU
+// instruction, no hazard.)
+__device__ __forceinline__ uint32_t level_quad_bf16(uint32_t w0, uint32_t w1, const RowQuant<true> &rq) {
+  float t[4];
+  rq.quotient_pair_bf16<false>(w0, t[0], t[1]);
+  rq.quotient_pair_bf16<false>(w1, t[2], t[3]);
+  uint32_t m[4];
+#pragma unroll
+  for (int k = 0; k < 4; ++k) {
+    float c;
+    asm("v_max_f32 %0, 0, %1" : "=v"(c) : "v"(t[k]));
+    m[k] = __float_as_uint(c + 12582912.0f);
+  }
+  return __builtin_amdgcn_perm(m[1], m[0], 0x0C0C0400u) | (__builtin_amdgcn_perm(m[3], m[2], 0x0C0C0400u) << 16);
+}
+
 // ---- pieces of the kernel that writes 6-bit operand buffers (quantize_fp6_row_kernel)
 
 // Byte offset of source column c inside a row image in LDS.  A copy instruction moves one contiguous kilobyte (64 groups
@@ -1188,6 +1206,9 @@ __device__ __forceinline__ int quantise_fragment(const uint4 (&v)[4], const RowQ
       const uint32_t p2 = level_pair_fast<SYM>(v[i].z, rq), p3 = level_pair_fast<SYM>(v[i].w, rq);
       b[2 * i] = __builtin_amdgcn_perm(p1, p0, 0x06040200u);  // bytes 0, 2 of p0 then bytes 0, 2 of p1
       b[2 * i + 1] = __builtin_amdgcn_perm(p3, p2, 0x06040200u);
+    } else if constexpr (!SLOW) {
+      b[2 * i] = level_quad_bf16(v[i].x, v[i].y, rq);
+      b[2 * i + 1] = level_quad_bf16(v[i].z, v[i].w, rq);
     } else {
       const uint2 c = group_codes<4, BF16, SLOW, SYM>(v[i], rq);  // code nibbles (two's complement), one per byte
       b[2 * i] = c.x ^ 0x08080808u;                               // level = code + 8

@@ -42,7 +42,9 @@ struct RowQuant {
   // Both quotients of a pair (x0, x1 as fp32) with the path chosen at compile time (callers branch once per row on
   // `slow`), bf16: the pair is rounded by one conversion instruction.  Measured against rounding each value by itself with
   // integer arithmetic (30 against 11 instructions per element): 6-bit quantize of 777 x 4096 9.0 -> 7.6 us, 2048 x 8192
-  // 18.9 -> 15.7, int8 2048 x 28672 84 -> 67.
+  // 18.9 -> 15.7, int8 2048 x 28672 84 -> 67.  One product instead of three per quotient, and levels of four
+  // values together (level_quad_bf16), us per forward: 777 x 4096 -> 22016 64.1 -> 63.3, 2048 x 8192 -> 1024 30.8 -> 29.5, int8 2048 x 28672 ->
+  // 512 110.9 -> 107.3.
   template <bool SLOW>
   __device__ __forceinline__ void quotient_pair_bf16(uint32_t w, float &t0, float &t1) const {
     static_assert(BF16, "bf16 pairs");
@@ -52,9 +54,9 @@ struct RowQuant {
     if constexpr (SLOW) {
       q0 = d0 / scale, q1 = d1 / scale;
     } else {
+      // (two roundings, below 2^-23 relative: the quotient of two 8-bit significands stays more than 2^-18 away from every rounding boundary
+      // of bf16, tests/test_quotient_levels_bf16.py)
       q0 = d0 * rcp, q1 = d1 * rcp;
-      q0 = __builtin_fmaf(__builtin_fmaf(-q0, scale, d0), rcp, q0);
-      q1 = __builtin_fmaf(__builtin_fmaf(-q1, scale, d1), rcp, q1);
     }
     const uint32_t q = pack2_bf16(q0, q1);
     t0 = __uint_as_float(q << 16), t1 = __uint_as_float(q & 0xFFFF0000u);
