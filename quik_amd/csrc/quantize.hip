@@ -1404,9 +1404,9 @@ __global__ __launch_bounds__(512) void quantize_fp6_row_kernel(
 // one trip for all tables, a lane has its groups of 8 columns whole, outliers masked, and what is squeezed is read on the way out: the codes
 // lie in source order, 16 integer columns that follow each other are two aligned reads and a shift (the column map's units), the others
 // are gathered by the byte.  The same arithmetic.
-// us per forward, asym_quantize_stream_kernel / this: int4 4 x 2048 -> 4096 7.0 / 6.6, 8 x 4096 -> 4096 7.55 / 7.25, 16 x 8192 -> 8192 12.5 / 11.85,
-// 3 x 13824 -> 5120 13.9 / 13.1, 16 x 8192 -> 28672 27.5 / 26.9, bf16 8 x 4096 -> 4096 7.95 / 7.5, int8 16 x 13824 -> 5120 19.4 / 18.15, 24 x
-// 28672 -> 8192 43.7 / 42.05.  Tile order: 64 x 4096 -> 4096 11.1 / 10.6, 64 x 8192 -> 8192 18.25 / 17.3, 256 x 4096 -> 4096 14.95 / 14.35, 1024 x 13824 ->
+// us per forward, asym_quantize_stream_kernel / this: int4 4 x 2048 -> 4096 7.0 / 6.6, 8 x 4096 -> 4096 7.55 / 7.35, 16 x 8192 -> 8192 12.5 / 11.9,
+// 3 x 13824 -> 5120 13.9 / 13.1, 16 x 8192 -> 28672 27.5 / 26.9, bf16 8 x 4096 -> 4096 7.95 / 7.5, int8 16 x 13824 -> 5120 19.4 / 18.5, 24 x
+// 28672 -> 8192 43.7 / 42.05.  Tile order: 64 x 4096 -> 4096 11.1 / 10.6, 64 x 8192 -> 8192 18.25 / 17.55, 256 x 4096 -> 4096 14.95 / 14.3, 1024 x 13824 ->
 // 512 36.5 / 35.4, 2048 x 8192 -> 512 32.4 / 30.9, 8192 x 4096 -> 512 56.0 / 54.9, bf16 64 x 11008 -> 4096 18.6 / 18.0, 2048 x 13824 -> 512 51.85 / 48.0,
 // 1536 x 28672 -> 512 97.25 / 95.3; against quantize_tile8_ring_kernel: see asym_quantize_tile8.
 constexpr int kUnitThreads = 512, kFewRows = 32;
@@ -1417,10 +1417,11 @@ __host__ __device__ inline int64_t unit_lds_bytes(int64_t cols) { return unit_ra
 template <int BITS, bool BF16, int NV, bool TILED>
 __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
     const uint16_t *__restrict__ x, const uint32_t *__restrict__ grp, const uint16_t *__restrict__ unit, int cols, int num_int, int num_fp,
-    int ngather, int rows, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
-    uint8_t *__restrict__ dst, uint16_t *__restrict__ fp_x, uint16_t *__restrict__ meta) {
+    int rows, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
+    const uint32_t *__restrict__ flags, uint8_t *__restrict__ dst, uint16_t *__restrict__ fp_x, uint16_t *__restrict__ meta,
+    const uint16_t *__restrict__ src_col, const uint32_t *__restrict__ mask) {
   extern __shared__ __align__(16) uint8_t lds[];
-  __shared__ __align__(16) float red[16];
+  __shared__ __align__(16) float red[64];
   constexpr int T = kUnitThreads, W = T / 64, NU = (NV + 1) / 2;
   static_assert(!TILED || BITS == 8, "tile order: int8");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1445,13 +1446,25 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
 #pragma unroll
   for (int k = 0; k < NU; ++k) first[k] = unit[tid + k * T < nu ? tid + k * T : 0];
   const uint16_t *const spare = reinterpret_cast<const uint16_t *>(grp);  // (always there; the other tables may be empty)
-  const bool has_g = tid < ngather, has_f = tid < num_fp;
-  const uint32_t gunit = *(has_g ? gather_unit + tid : spare), fcol = *(has_f ? fp_col + tid : spare);
-  const uint4 *const gc = reinterpret_cast<const uint4 *>(has_g ? gather_cols + 16 * tid : spare);
+  const bool has_f = tid < num_fp;  // (at most num_fp gathered units)
+  const uint32_t gunit = *(has_f ? gather_unit + tid : spare), fcol = *(has_f ? fp_col + tid : spare);
+  const uint4 *const gc = reinterpret_cast<const uint4 *>(has_f ? gather_cols + 16 * tid : spare);
   const uint4 ga = gc[0], gb = gc[1];
-  if constexpr (!BF16) treat_all_nans_alike();  // pk_min_f16 / pk_max_f16 on the raw row
+  // The device's words: the map at this address may be another one at every launch.  (A vector load, beside the others: as a scalar one
+  // it is waited for with the arguments, 16 x 8192 -> 8192 12.0 instead of 11.85 us per forward.)
+  uint32_t none = 0;
+  asm volatile("" : "+v"(none));
+  const uint4 words = reinterpret_cast<const uint4 *>(flags)[none];
   __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
   __syncthreads();
+  const uint32_t map_flags = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(words.x)));
+  const uint32_t ngather = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(words.w)));
+  if (!(map_flags & kColmapStreams)) {  // any other order of the columns (tile order: refused before the launch, nothing is written)
+    if constexpr (!TILED)
+      gather_rows<uint16_t, BITS, BF16, T>(x, rows, cols, src_col, fp_col, mask, num_int, num_fp, dst, meta, fp_x, 1, reinterpret_cast<uint16_t *>(lds), red);
+    return;
+  }
+  if constexpr (!BF16) treat_all_nans_alike();  // pk_min_f16 / pk_max_f16 on the raw row
 
   auto value = [&](uint32_t c) { return reinterpret_cast<const uint16_t *>(raw)[c]; };
   const Tile8Layout l8 = tile8_layout(rows, num_int, num_fp);
@@ -1541,15 +1554,20 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
                                   __builtin_amdgcn_alignbyte(w[3], w[2], c0), __builtin_amdgcn_alignbyte(w[4], w[3], c0)));
     }
   }
-  if (has_g) {
-    const uint32_t at[8] = {ga.x, ga.y, ga.z, ga.w, gb.x, gb.y, gb.z, gb.w};
+  auto gather = [&](uint32_t u, const uint4 &a, const uint4 &b) {
+    const uint32_t at[8] = {a.x, a.y, a.z, a.w, b.x, b.y, b.z, b.w};
     uint32_t c[4];
 #pragma unroll
     for (int t = 0; t < 4; ++t) {
       const uint32_t b0 = stage[at[2 * t] & 0xFFFFu], b1 = stage[at[2 * t] >> 16], b2 = stage[at[2 * t + 1] & 0xFFFFu], b3 = stage[at[2 * t + 1] >> 16];
       c[t] = b0 | (b1 << 8) | (b2 << 16) | (b3 << 24);
     }
-    put(static_cast<int>(gunit), make_uint4(c[0], c[1], c[2], c[3]));
+    put(static_cast<int>(u), make_uint4(c[0], c[1], c[2], c[3]));
+  };
+  if (static_cast<uint32_t>(tid) < ngather) gather(gunit, ga, gb);
+  for (uint32_t i = tid + T; i < ngather; i += T) {
+    const uint4 *const more = reinterpret_cast<const uint4 *>(gather_cols + 16 * i);
+    gather(gather_unit[i], more[0], more[1]);
   }
 }
 
@@ -2143,14 +2161,13 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
 }
 
 namespace {
-// words: the column map's, which streams
-bool units_ok(const void *x, int64_t cols, int64_t num_int, const void *dst, const uint32_t (&words)[4]) {
-  return cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(dst) % 16 == 0 && (words[0] & kColmapStreams) && words[3] <= kUnitThreads;
+bool units_ok(const void *x, int64_t rows, int64_t cols, int64_t num_int, const void *dst) {
+  return rows <= (1 << 20) && cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(dst) % 16 == 0;  // (rows: a grid holds fewer than 2^32 threads)
 }
 template <int BITS, bool BF16, bool TILED>
-int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int ngather, void *dst,
-                    void *meta, void *fp_x, hipStream_t st) {
+int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, void *dst, void *meta,
+                 void *fp_x, hipStream_t st) {
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   auto go = [&](auto kern) {
@@ -2158,10 +2175,11 @@ int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, 
     hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(TILED ? (rows + 7) / 8 * 8 : rows)), dim3(kUnitThreads),
                        static_cast<size_t>(unit_lds_bytes(cols)), st, static_cast<const uint16_t *>(x),
                        reinterpret_cast<const uint32_t *>(cm + l.off_grp), reinterpret_cast<const uint16_t *>(cm + l.off_unit),
-                       static_cast<int>(cols), static_cast<int>(num_int), static_cast<int>(num_fp), ngather, static_cast<int>(rows),
+                       static_cast<int>(cols), static_cast<int>(num_int), static_cast<int>(num_fp), static_cast<int>(rows),
                        reinterpret_cast<const uint16_t *>(cm + l.off_fp), reinterpret_cast<const uint16_t *>(cm + l.off_gunit),
-                       reinterpret_cast<const uint16_t *>(cm + l.off_gcols), static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x),
-                       static_cast<uint16_t *>(meta));
+                       reinterpret_cast<const uint16_t *>(cm + l.off_gcols), reinterpret_cast<const uint32_t *>(cm + l.off_flags),
+                       static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x), static_cast<uint16_t *>(meta),
+                       reinterpret_cast<const uint16_t *>(cm), reinterpret_cast<const uint32_t *>(cm + l.off_mask));
     return check_launch();
   };
   const int64_t groups = cols / 8;
@@ -2175,12 +2193,11 @@ int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, 
 // A layer's few rows: quantize_units_kernel where it takes the shape, else as quik_asym_quantize.
 int quik::asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, int bits,
                             void *dst, void *meta, void *fp_x, void *stream) {
-  uint32_t words[4];
   hipStream_t st = as_stream(stream);
   if (rows > 0 && rows <= kFewRows && num_int > 0 && num_fp >= 0 && num_int + num_fp == cols && (bits == 4 || bits == 8) &&
       (dtype == QUIK_F16 || dtype == QUIK_BF16) && x && colmap && dst && meta && (num_fp == 0 || fp_x) &&
-      colmap_words(colmap, cols, num_int, num_fp, st, words) == QUIK_OK && units_ok(x, cols, num_int, dst, words)) {
-    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, static_cast<int>(words[3]), dst, meta, fp_x, st); };
+      units_ok(x, rows, cols, num_int, dst)) {
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, dst, meta, fp_x, st); };
     if (bits == 4) return dtype == QUIK_F16 ? go(launch_units<4, false, false>) : go(launch_units<4, true, false>);
     return dtype == QUIK_F16 ? go(launch_units<8, false, false>) : go(launch_units<8, true, false>);
   }
@@ -2212,9 +2229,8 @@ int quik::asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t co
   // fp16 rows of more than 16384 columns, eight groups per lane, where a CU has more than one: quantize_tile8_ring_kernel, whose next row is
   // on its way while one is worked on (us per forward, units / ring: 256 x 28672 -> 1024 29.2 / 29.7, 512 x 28672 -> 512 40.65 / 39.45, 2048 x
   // 28672 -> 512 100 / 85; 768 x 16384 -> 512 32.55 / 34.05, 2048 x 13824 -> 512 46.05 / 47.15)
-  // (a grid holds fewer than 2^32 threads)
-  if (rows <= (1 << 20) && (dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) && units_ok(x, cols, num_int, out8, words)) {
-    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, static_cast<int>(words[3]), out8, meta, nullptr, st); };
+  if ((dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) && units_ok(x, rows, cols, num_int, out8)) {
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, out8, meta, nullptr, st); };
     return dtype == QUIK_F16 ? go(launch_units<8, false, true>) : go(launch_units<8, true, true>);
   }
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);

@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 # rows, K, F, bits, outlier columns in runs: one, two, four and eight groups of eight columns per lane and their ends, more outlier columns than
-# lanes, none, rows of less than a kilobyte; the last two are left to the other kernels (more gathered units than lanes, more rows)
+# lanes, none, rows of less than a kilobyte; more gathered units than lanes; the last is left to the other kernel (more rows)
 CASES = [(2, 64, 32, 4, False), (3, 480, 32, 8, True), (16, 3840, 256, 4, False), (7, 4096, 8, 8, False), (32, 4064, 32, 4, True),
          (5, 8192, 8, 8, True), (4, 7936, 256, 4, False), (16, 13568, 256, 8, False), (3, 16128, 256, 4, False), (2, 16384, 8, 8, False),
          (3, 32512, 256, 8, False), (2, 32000, 768, 4, True), (9, 2048, 0, 8, False), (6, 4096, 1024, 4, False), (2, 31232, 1024, 4, False),
@@ -86,3 +86,35 @@ def _through_the_layer(mod, xt):
     K, F = mod.int_features_num, mod.fp_features_num
     at = ((rows + 63) // 64 * ((K + 63) // 64 * 2 + F // 16) * 2048 + 255) // 256 * 256
     return ws, ws[at:at + 4 * rows].view(xt.dtype)
+
+
+@pytest.mark.parametrize("bits", [4, 8])
+def test_a_few_rows_take_the_map_that_is_there(bits):
+    """A captured forward whose layer's map is another one at its replays: one with more gathered units, one that does not stream."""
+    from quik_amd import asymmetric
+    rows, K, F = 5, 1024, 64
+    rng = np.random.default_rng(0)
+    mod, _, _, fi, _, _ = _layer(rng, 16, K + F, F, bits, torch.float16, False)
+    x = torch.randn(rows, K + F, device=DEV).half()
+    orders = [(np.arange(K), np.arange(K, K + F))]                                     # no gathered unit
+    out = rng.permutation(K + F)[:F]
+    orders.append((np.setdiff1d(np.arange(K + F), out), out))                          # many
+    orders.append((orders[1][0][::-1].copy(), out))                                    # no ascending order
+    maps = [asymmetric.build_colmap(torch.from_numpy(i).to(DEV), torch.from_numpy(f).to(DEV), K + F) for i, f in orders]
+    cm = mod._column_map()
+    cm.copy_(maps[0])
+    mod(x)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        y = mod(x)
+    for k in (1, 2, 0, 1):
+        cm.copy_(maps[k])
+        graph.replay()
+        q, meta, fp_x = asymmetric.quantize_mapped(x, maps[k], K, F, bits)
+        from quik_amd import matmul
+        acc = (matmul.int4Matmul if bits == 4 else matmul.int8Matmul)(q, mod.int_weight)
+        z = torch.nn.functional.linear(fp_x, mod.fp_weight)
+        want = asymmetric.dequantize(acc, meta, mod.weights_scales, mod.reduced_w, z, bits).float() + mod.bias.float()
+        rms = want.pow(2).mean().sqrt()
+        assert (y.float() - want).abs().max() <= 1e-2 * rms, k   # (16-bit outlier products and results, as the fused forward's tests)
