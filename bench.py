@@ -727,8 +727,10 @@ def main():
         "roofline": roofline,
         "roofline_quantize": None if one_launch else {"kernel": (f"quantize_fp6_row_kernel (one workgroup per token row, {x_bits}-bit operand output)" if six and bits == 4
                                          else "quantize_tile8_ring_kernel (row copied into an LDS ring, int8 operand output in tile order)"
-                                         if six and bits == 8 and n_in > 8192 and str(x.dtype) == "torch.float16"
-                                         else "asym_quantize_stream_kernel" + (" (tile-ordered operand output)" if six else "")),
+                                         if six and bits == 8 and n_in > 16384 and str(x.dtype) == "torch.float16"
+                                         and M > torch.cuda.get_device_properties(0).multi_processor_count
+                                         else "quantize_units_kernel" + (" (tile-ordered operand output)" if six else "") if six or M <= 32
+                                         else "asym_quantize_stream_kernel"),
                               "bound": "hbm",
                               "achieved": round(quant_gbps, 1),
                               "peak": PEAK_HBM_GBPS, "unit": "GB/s", "frac": round(quant_gbps / PEAK_HBM_GBPS, 4),

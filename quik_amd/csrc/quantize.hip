@@ -744,10 +744,10 @@ __global__ __launch_bounds__(TPR) void asym_quantize_stream_kernel(
 }
 
 // ---------------------------------------------------------------------------------------
-// Rows of more than 8192 columns (the down_proj inputs) -> int8 operand buffer in tile order, fp16 input.
+// Rows of more than 16384 columns (the largest down_proj inputs) -> int8 operand buffer in tile order, fp16 input, more rows than CUs.
 //
-// One workgroup of eight waves per CU (two where two rings fit the LDS) walks over its rows; a row is copied global -> LDS with direct copies (no
-// registers, so two rows are in flight while a third is worked on) into a ring of two slots.  Per row:
+// One workgroup of eight waves per CU walks over its rows; a row is copied global -> LDS with direct copies (no registers, so two rows are in
+// flight while a third is worked on) into a ring of two slots.  Per row:
 //   wait for this wave's copies of the row, barrier (the row is in LDS)
 //   every lane reads its NV groups of 8 columns (and, lanes 0 .. ndirty-1, one group that holds outlier columns;
 //   lanes 0 .. num_fp-1 one outlier value, which goes straight to the staging area); barrier (the slot is free)
@@ -1870,9 +1870,9 @@ int launch_sym_stream(const void *x, int64_t rows, int64_t cols, const uint8_t *
 // Long fp16 rows -> int8 operand buffer through the LDS ring (quantize_tile8_ring_kernel).  `ndirty`: groups of 8
 // columns that hold outlier columns, from the host's copy of the column map's flag words.
 constexpr int64_t kLdsPerCu = 160 * 1024;
-// rows of more than 8192 columns: measured against the streaming kernel at 2048 rows, kernel time from a cold
-// cache: 8192 columns 17.4 against 16.8 us, 11008 19.9 against 20.9, 13824 23.7 against 26.3, 28672 41.6 against 51.0
-constexpr int64_t kRingMinGroups = 2 * kRingThreads + 1;
+// rows of more than 16384 columns (against quantize_units_kernel: asym_quantize_tile8); against the streaming kernel at 2048 rows, kernel
+// time from a cold cache: 28672 columns 41.6 against 51.0 us
+constexpr int64_t kRingMinGroups = 4 * kRingThreads + 1;
 bool ring_fits(int64_t cols, int64_t num_int, int64_t num_fp, int64_t ndirty) {
   const int64_t groups = cols / 8;
   return groups >= kRingMinGroups && groups <= 8 * kRingThreads && ndirty >= 0 && ndirty <= kRingThreads &&
@@ -1891,8 +1891,8 @@ int launch_tile8_ring_nv(const void *x, int64_t rows, int64_t cols, const uint8_
     return QUIK_ERR_LAUNCH;
   }
   const int64_t per_xcd = (rows + 7) / 8;
-  // one workgroup per CU when the ring takes most of its LDS, two when two fit; a multiple of the XCDs
-  int64_t grid = num_cus() / 8 * 8 * (2 * lds + 1024 <= kLdsPerCu ? 2 : 1);
+  // the ring takes most of a CU's LDS: one workgroup each; a multiple of the XCDs
+  int64_t grid = num_cus() / 8 * 8;
   if (grid < 8) grid = 8;
   if (grid > per_xcd * 8) grid = per_xcd * 8;
   hipLaunchKernelGGL(kern, dim3(static_cast<unsigned>(grid)), dim3(kRingThreads), static_cast<size_t>(lds), st,
@@ -1910,8 +1910,6 @@ int launch_tile8_ring(const void *x, int64_t rows, int64_t cols, const uint8_t *
                       int64_t num_int, int64_t num_fp, int ndirty, int ngather, void *dst, void *meta,
                       hipStream_t st) {
   switch ((cols / 8 + kRingThreads - 1) / kRingThreads) {
-    case 3: return launch_tile8_ring_nv<3>(x, rows, cols, cm, l, num_int, num_fp, ndirty, ngather, dst, meta, st);
-    case 4: return launch_tile8_ring_nv<4>(x, rows, cols, cm, l, num_int, num_fp, ndirty, ngather, dst, meta, st);
     case 5: return launch_tile8_ring_nv<5>(x, rows, cols, cm, l, num_int, num_fp, ndirty, ngather, dst, meta, st);
     case 6: return launch_tile8_ring_nv<6>(x, rows, cols, cm, l, num_int, num_fp, ndirty, ngather, dst, meta, st);
     case 7: return launch_tile8_ring_nv<7>(x, rows, cols, cm, l, num_int, num_fp, ndirty, ngather, dst, meta, st);
@@ -1932,7 +1930,7 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
     const int64_t groups = cols / 8;
 #define QUIK_STREAM(NV, TPR) \
   return launch_stream<IdxT, BITS, BF16, NV, TPR>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, tiled)
-    // fp16 rows beyond 8192 columns with tile-ordered int8 output: the LDS ring kernel
+    // fp16 rows beyond 16384 columns with tile-ordered int8 output: the LDS ring kernel
     if constexpr (BITS == 8 && !BF16) {
       if (tiled && ring_fits(cols, num_int, num_fp, ndirty) && ngather <= kRingThreads)
         return launch_tile8_ring(x, rows, cols, cm, l, num_int, num_fp, static_cast<int>(ndirty),
