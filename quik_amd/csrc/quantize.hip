@@ -1414,14 +1414,16 @@ __host__ __device__ inline int64_t unit_raw_bytes(int64_t cols) { return (cols *
 __host__ __device__ inline int64_t unit_lds_bytes(int64_t cols) { return unit_raw_bytes(cols) + (cols + 47) / 16 * 16; }
 
 // TILED (int8): into an operand buffer in tile order (gemm_tile8.h), outlier values included.
-template <int BITS, bool BF16, int NV, bool TILED>
+// SYM: symmetric activations, one scale per row, fp16; row-major only.
+template <int BITS, bool BF16, int NV, bool TILED, bool SYM = false>
 __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
     const uint16_t *__restrict__ x, const uint32_t *__restrict__ grp, const uint16_t *__restrict__ unit, int cols, int num_int, int num_fp,
     int rows, const uint16_t *__restrict__ fp_col, const uint16_t *__restrict__ gather_unit, const uint16_t *__restrict__ gather_cols,
     const uint32_t *__restrict__ flags, uint8_t *__restrict__ dst, uint16_t *__restrict__ fp_x, uint16_t *__restrict__ meta,
-    const uint16_t *__restrict__ src_col, const uint32_t *__restrict__ mask) {
+    const uint16_t *__restrict__ src_col, const uint32_t *__restrict__ mask, float sym_divisor) {
   extern __shared__ __align__(16) uint8_t lds[];
   __shared__ __align__(16) float red[64];
+  static_assert(!SYM || (!BF16 && !TILED), "symmetric activations: fp16, row-major");
   constexpr int T = kUnitThreads, W = T / 64, NU = (NV + 1) / 2;
   static_assert(!TILED || BITS == 8, "tile order: int8");
   const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1459,12 +1461,12 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
   __syncthreads();
   const uint32_t map_flags = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(words.x)));
   const uint32_t ngather = static_cast<uint32_t>(__builtin_amdgcn_readfirstlane(static_cast<int>(words.w)));
-  if (!(map_flags & kColmapStreams)) {  // any other order of the columns (tile order: refused before the launch, nothing is written)
-    if constexpr (!TILED)
+  if (!(map_flags & kColmapStreams)) {  // any other order of the columns (tile order, SYM: refused before the launch, nothing is written)
+    if constexpr (!TILED && !SYM)
       gather_rows<uint16_t, BITS, BF16, T>(x, rows, cols, src_col, fp_col, mask, num_int, num_fp, dst, meta, fp_x, 1, reinterpret_cast<uint16_t *>(lds), red);
     return;
   }
-  if constexpr (!BF16) treat_all_nans_alike();  // pk_min_f16 / pk_max_f16 on the raw row
+  if constexpr (!BF16 && !SYM) treat_all_nans_alike();  // pk_min_f16 / pk_max_f16 on the raw row
 
   auto value = [&](uint32_t c) { return reinterpret_cast<const uint16_t *>(raw)[c]; };
   const Tile8Layout l8 = tile8_layout(rows, num_int, num_fp);
@@ -1477,6 +1479,7 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
   for (int f = tid + T; f < num_fp; f += T) *outlier(f) = value(fp_col[f]);
   uint4 v[NV];
   uint32_t pmn = 0x7C007C00u, pmx = 0xFC00FC00u;
+  u2 amax = u2{0, 0};  // SYM: largest |x| pattern (a NaN's is larger than any number's)
   float mn = __builtin_inff(), mx = -__builtin_inff();
 #pragma unroll
   for (int k = 0; k < NV; ++k) {
@@ -1487,7 +1490,9 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
     for (int t = 0; t < 4; ++t) {
       const uint32_t lo = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(skip), 2 * t, 1));
       const uint32_t hi = static_cast<uint32_t>(__builtin_amdgcn_sbfe(static_cast<int>(skip), 2 * t + 1, 1));
-      if constexpr (!BF16) {
+      if constexpr (SYM) {
+        amax = __builtin_elementwise_max(amax, __builtin_bit_cast(u2, w[t] & 0x7FFF7FFFu & ~__builtin_amdgcn_perm(hi, lo, 0x07060100u)));
+      } else if constexpr (!BF16) {
         const uint32_t m = w[t] | __builtin_amdgcn_perm(hi, lo, 0x07060100u);  // outliers: a NaN, which is skipped
         pmn = pk_min_f16(pmn, m), pmx = pk_max_f16(pmx, m);
       } else {
@@ -1496,7 +1501,9 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
       }
     }
   }
-  if constexpr (!BF16) {
+  if constexpr (SYM) {
+    mn = 0.0f, mx = static_cast<float>(amax.x > amax.y ? amax.x : amax.y);  // a 15-bit integer: exact
+  } else if constexpr (!BF16) {
     const h2 a = __builtin_bit_cast(h2, pmn), b = __builtin_bit_cast(h2, pmx);
     mn = fminf(static_cast<float>(a.x), static_cast<float>(a.y)), mx = fmaxf(static_cast<float>(b.x), static_cast<float>(b.y));
   }
@@ -1512,12 +1519,17 @@ __global__ __launch_bounds__(kUnitThreads) void quantize_units_kernel(
 #pragma unroll
   for (int w = 0; w < W; ++w) mn = fminf(mn, part[w]), mx = fmaxf(mx, part[W + w]);
   RowQuant<BF16> rq;
-  rq.init(mn, mx, BITS);
-  if (tid == 0) meta[2 * row] = rq.scale_bits, meta[2 * row + 1] = rq.zero_bits;
+  if constexpr (SYM) {
+    rq.init_sym(static_cast<uint32_t>(mx), sym_divisor);
+    if (tid == 0) meta[row] = rq.scale_bits;
+  } else {
+    rq.init(mn, mx, BITS);
+    if (tid == 0) meta[2 * row] = rq.scale_bits, meta[2 * row + 1] = rq.zero_bits;
+  }
   auto codes = [&](auto slow_c) {
 #pragma unroll
     for (int k = 0; k < NV; ++k)
-      if (tid + k * T < nvec) *reinterpret_cast<uint2 *>(stage + (tid + k * T) * 8) = group_codes<BITS, BF16, decltype(slow_c)::value>(v[k], rq);
+      if (tid + k * T < nvec) *reinterpret_cast<uint2 *>(stage + (tid + k * T) * 8) = group_codes<BITS, BF16, decltype(slow_c)::value, SYM>(v[k], rq);
   };
   if (__builtin_amdgcn_readfirstlane(rq.slow ? 1 : 0)) {
     codes(std::true_type{});
@@ -2163,9 +2175,9 @@ bool units_ok(const void *x, int64_t rows, int64_t cols, int64_t num_int, const 
   return rows <= (1 << 20) && cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
          reinterpret_cast<uintptr_t>(dst) % 16 == 0;  // (rows: a grid holds fewer than 2^32 threads)
 }
-template <int BITS, bool BF16, bool TILED>
+template <int BITS, bool BF16, bool TILED, bool SYM = false>
 int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, void *dst, void *meta,
-                 void *fp_x, hipStream_t st) {
+                 void *fp_x, hipStream_t st, float sym_divisor = 1.0f) {
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
   auto go = [&](auto kern) {
@@ -2177,14 +2189,14 @@ int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, 
                        reinterpret_cast<const uint16_t *>(cm + l.off_fp), reinterpret_cast<const uint16_t *>(cm + l.off_gunit),
                        reinterpret_cast<const uint16_t *>(cm + l.off_gcols), reinterpret_cast<const uint32_t *>(cm + l.off_flags),
                        static_cast<uint8_t *>(dst), static_cast<uint16_t *>(fp_x), static_cast<uint16_t *>(meta),
-                       reinterpret_cast<const uint16_t *>(cm), reinterpret_cast<const uint32_t *>(cm + l.off_mask));
+                       reinterpret_cast<const uint16_t *>(cm), reinterpret_cast<const uint32_t *>(cm + l.off_mask), sym_divisor);
     return check_launch();
   };
   const int64_t groups = cols / 8;
-  if (groups <= 512) return go(quantize_units_kernel<BITS, BF16, 1, TILED>);
-  if (groups <= 1024) return go(quantize_units_kernel<BITS, BF16, 2, TILED>);
-  if (groups <= 2048) return go(quantize_units_kernel<BITS, BF16, 4, TILED>);
-  return go(quantize_units_kernel<BITS, BF16, 8, TILED>);
+  if (groups <= 512) return go(quantize_units_kernel<BITS, BF16, 1, TILED, SYM>);
+  if (groups <= 1024) return go(quantize_units_kernel<BITS, BF16, 2, TILED, SYM>);
+  if (groups <= 2048) return go(quantize_units_kernel<BITS, BF16, 4, TILED, SYM>);
+  return go(quantize_units_kernel<BITS, BF16, 8, TILED, SYM>);
 }
 }  // namespace
 
@@ -2195,7 +2207,7 @@ int quik::asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols
   if (rows > 0 && rows <= kFewRows && num_int > 0 && num_fp >= 0 && num_int + num_fp == cols && (bits == 4 || bits == 8) &&
       (dtype == QUIK_F16 || dtype == QUIK_BF16) && x && colmap && dst && meta && (num_fp == 0 || fp_x) &&
       units_ok(x, rows, cols, num_int, dst)) {
-    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, dst, meta, fp_x, st); };
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, dst, meta, fp_x, st, 1.0f); };
     if (bits == 4) return dtype == QUIK_F16 ? go(launch_units<4, false, false>) : go(launch_units<4, true, false>);
     return dtype == QUIK_F16 ? go(launch_units<8, false, false>) : go(launch_units<8, true, false>);
   }
@@ -2228,7 +2240,7 @@ int quik::asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t co
   // on its way while one is worked on (us per forward, units / ring: 256 x 28672 -> 1024 29.2 / 29.7, 512 x 28672 -> 512 40.65 / 39.45, 2048 x
   // 28672 -> 512 100 / 85; 768 x 16384 -> 512 32.55 / 34.05, 2048 x 13824 -> 512 46.05 / 47.15)
   if ((dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) && units_ok(x, rows, cols, num_int, out8)) {
-    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, out8, meta, nullptr, st); };
+    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, out8, meta, nullptr, st, 1.0f); };
     return dtype == QUIK_F16 ? go(launch_units<8, false, true>) : go(launch_units<8, true, true>);
   }
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
@@ -2265,6 +2277,11 @@ int quik::sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const v
   if (bits == 4 && tiled == QUIK_TILED_4)
     return launch_fp6_row<false, true, true>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
   if (bits == 4 && tiled) return launch_fp6_row<false, true, false>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
+  // few rows: as asym_quantize_few (us per forward, streaming kernel / units: 16 x 8192 -> 8192 12.4 / 12.0, 3 x 13824 -> 5120 13.75 / 13.3,
+  // 16 x 28672 -> 8192 28.05 / 26.95, 24 x 2048 -> 2048 7.35 / 7.15, 32 x 4096 -> 4096 8.85 / 8.7; 5120 columns the same)
+  if (!tiled && rows <= kFewRows && units_ok(x, rows, cols, num_int, dst))
+    return bits == 4 ? launch_units<4, false, false, true>(x, rows, cols, colmap, num_int, num_fp, dst, scale, fp_x, st, divisor)
+                     : launch_units<8, false, false, true>(x, rows, cols, colmap, num_int, num_fp, dst, scale, fp_x, st, divisor);
   return bits == 4 ? launch_sym_stream<4>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor)
                    : launch_sym_stream<8>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor);
 }

@@ -118,3 +118,24 @@ def test_a_few_rows_take_the_map_that_is_there(bits):
         want = asymmetric.dequantize(acc, meta, mod.weights_scales, mod.reduced_w, z, bits).float() + mod.bias.float()
         rms = want.pow(2).mean().sqrt()
         assert (y.float() - want).abs().max() <= 1e-2 * rms, k   # (16-bit outlier products and results, as the fused forward's tests)
+
+
+@pytest.mark.parametrize("K,F,bits,runs", [c[1:] for c in CASES])
+def test_symmetric_few_rows(K, F, bits, runs):
+    """Few rows of symmetric activations against the same rows in a call of more, which the streaming kernel takes: bit for bit."""
+    from quik_amd import symmetric
+    rng = np.random.default_rng(K + F)
+    mod, _, _, fi, ii, _ = _layer(rng, 16, K + F, F, bits, torch.float16, runs)
+    x = rng.standard_normal((40, K + F)).astype(np.float32)
+    x[:, fi] *= 50
+    x[0, ii[3]], x[1, ii[K // 2]], x[2], x[3, ii[-1]], x[4] = np.nan, -np.inf, 0, -6e4, 1e-7
+    xt = torch.from_numpy(x).to(DEV, torch.float16)
+    if F:
+        xt[5, fi] = float("nan")
+    cm, divisor = mod._column_map(), 7.0 if bits == 4 else 127.0
+    want = symmetric.quantize_mapped(xt, cm, K, F, bits, divisor, False)
+    for rows in (1, 7, 32):
+        got = symmetric.quantize_mapped(xt[:rows], cm, K, F, bits, divisor, False)
+        for g, w in zip(got, want):
+            if g is not None:
+                assert torch.equal(g.contiguous().view(torch.uint8), w[:rows].contiguous().view(torch.uint8))
