@@ -8,9 +8,8 @@
 //     sum_k a_k w_k = 64 S - 8 sum_k La_k - 8 sum_k Lw_k + 64 K,      S = sum_k (La_k / 8)(Lw_k / 8)
 // recovers the integer accumulator exactly (every term is an integer below 2^24).  The accumulators
 // start at K - sum_k La_k / 8 - sum_k Lw_k / 8 (between -176 K and 64 K 64ths, from where they only rise, to the result:
-// still exact) and end at a 64th of the integer; the 64 is in the column's scale.  From there the epilogue is the one of
-// gemm_kernels.h, so the output is bit-identical to the int8-MFMA path (as long as 64 times a column's scale is finite: in
-// bf16 it is up to 5e36).
+// still exact) and end at a 64th of the integer; the 64 goes into the row's scale where that is exact (scales_take_64), else onto
+// the sum.  From there the epilogue is the one of gemm_kernels.h, so the output is bit-identical to the int8-MFMA path.
 //
 // Operand format: fp6_format.h.  Both operand buffers are stored as the sequence of LDS images the
 // tiles need, so a copy instruction moves one contiguous kilobyte and every cache line is requested
@@ -615,10 +614,7 @@ __device__ __forceinline__ void tile_sums_request(const Vectors &tv, const Args 
 template <class C, class Vectors>
 __device__ __forceinline__ void tile_sums_widen(const Vectors &tv, int K) {
   const int i = threadIdx.x;
-  if (i < C::BN) {
-    tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
-    tv.scol[i] *= 64.0f;  // (behind tile_vector_widen, by the same thread)
-  }
+  if (i < C::BN) tv.colc[i] = static_cast<float>(__float_as_int(tv.colc[i])) * -0.125f;
   if (i < C::BM) tv.rowc[i] = static_cast<float>(8 * K - __float_as_int(tv.rowc[i])) * 0.125f;
 }
 
@@ -746,19 +742,47 @@ __device__ __forceinline__ bool wave_is_idle(const Args &p, int m0, int n0) {
   return m0 + wave / C::WAVES_N * C::WM >= p.M || n0 + wave % C::WAVES_N * C::WN >= p.N;
 }
 
-// The accumulators of a tile between its two MFMA phases: finish(acc, s_row * s_col, zs * w_red + bias), 32x32 block by block.
-// What bounds it is the issue of its instructions: a wave issues one in four cycles, one that needs the result of the one
-// before in eight.  So four values go side by side.  AGPR: the accumulators are in accumulation registers, which the VALU cannot
-// address; where a wave holds at most 128 of them they are ordinary registers (two instructions less per value).
-template <class C, bool BF16, bool AGPR, class Vectors, class Finish>
-__device__ __forceinline__ void convert_tile(v16f (&acc)[C::MI][C::NI], const Vectors &tv, int wm, int wn, int lane, Finish finish) {
+// Whether the factor 64 may go into this wave's row scales: neither does 64 s_row s_col overflow nor is s_row s_col subnormal.
+template <class C, class Vectors>
+__device__ __forceinline__ bool scales_take_64(const Vectors &tv, int wm, int wn, int lane) {
+  bool all = true;
+  auto look = [&](float s) {
+    const float a = __builtin_fabsf(s);
+    all &= (a >= 0x1p-60f && a <= 0x1p60f) || a == 0.0f;
+  };
+#pragma unroll
+  for (int mi = 0; mi < C::MI; ++mi) look(tv.srow[wm * C::WM + mi * 32 + (lane & 31)]);
+#pragma unroll
+  for (int ni = 0; ni < C::NI; ++ni) look(tv.scol[wn * C::WN + ni * 32 + (lane & 31)]);
+  return __all(all);
+}
+
+// The accumulators of a tile between its two MFMA phases, 64ths of the integers -> f32(integer) * (s_row * s_col) + (zs * w_red + bias),
+// 32x32 block by block.  What bounds it is the issue of its instructions: a wave issues one in four cycles, one that needs the result of
+// the one before in eight.  So four values go side by side, and the 64 goes into the row's scale wherever the wave's scales allow it (any
+// trained layer's do; the same bits), onto each value only elsewhere.  us per forward against a 64 in the scale whatever the scales are:
+// always onto each value bf16 777 x 4096 -> 22016 60.9 -> 61.7, 2048 x 8192 -> 28672 245.3 -> 247.4, by this rule 62.05 -> 62.3, 250.4 -> 251.8
+// (another card).  AGPR: the accumulators are in accumulation registers, which the VALU cannot address; where a wave holds at most 128 of
+// them they are ordinary registers (two instructions less per value).
+template <class C, bool AGPR, class Vectors>
+__device__ __forceinline__ void convert_tile(v16f (&acc)[C::MI][C::NI], const Vectors &tv, int wm, int wn, int lane, bool scaled) {
   float srow[C::MI], zsr[C::MI];
+  const float factor = scaled ? 64.0f : 1.0f;
 #pragma unroll
   for (int mi = 0; mi < C::MI; ++mi) {
-    srow[mi] = tv.srow[wm * C::WM + mi * 32 + (lane & 31)];
+    srow[mi] = tv.srow[wm * C::WM + mi * 32 + (lane & 31)] * factor;
     zsr[mi] = tv.zs[wm * C::WM + mi * 32 + (lane & 31)];
   }
   if constexpr (AGPR) asm volatile("s_nop 15\n\ts_nop 15");  // the last MFMA results are architecturally visible to the reads below
+  if (!scaled) {
+#pragma unroll
+    for (int ni = 0; ni < C::NI; ++ni)
+#pragma unroll
+      for (int mi = 0; mi < C::MI; ++mi)
+#pragma unroll
+        for (int v = 0; v < 16; ++v)
+          acc[mi][ni][v] = AGPR ? agpr_write(agpr_read(acc[mi][ni][v]) * 64.0f) : acc[mi][ni][v] * 64.0f;
+  }
 #pragma unroll
   for (int ni = 0; ni < C::NI; ++ni) {
     float scv[16], wrv[16], bsv[16];
@@ -782,7 +806,7 @@ __device__ __forceinline__ void convert_tile(v16f (&acc)[C::MI][C::NI], const Ve
 #pragma unroll
         for (int e = 0; e < 4; ++e) t[e] = __builtin_fmaf(zsr[mi], wrv[4 * g + e], bsv[4 * g + e]);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) a[e] = finish(a[e], srow[mi] * scv[4 * g + e], t[e]);
+        for (int e = 0; e < 4; ++e) a[e] = __builtin_fmaf(a[e], srow[mi] * scv[4 * g + e], t[e]);
 #pragma unroll
         for (int e = 0; e < 4; ++e) acc[mi][ni][4 * g + e] = AGPR ? agpr_write(a[e]) : a[e];
       }
@@ -841,6 +865,7 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
       return;
     }
   }
+  const bool scaled = scales_take_64<C>(tv, wm, wn, lane);  // (here, while the first steps are on their way)
   v16f acc[C::MI][C::NI];
   // The start values are an outer sum, K = 2 of the fp32 MFMA: column term times 1 plus 1 times row term, both exact.
   {
@@ -872,8 +897,7 @@ __device__ __forceinline__ void fused6_tile(const Fused6Args &p, int tm, int tn,
     }
   }
 
-  // acc, a 64th of the integer accumulator -> f32(integer) * (s_row * s_col) + (zs * w_red + bias), in place
-  convert_tile<C, BF16, AGPR>(acc, tv, wm, wn, lane, [](float a, float s, float t) { return __builtin_fmaf(a, s, t); });
+  convert_tile<C, AGPR>(acc, tv, wm, wn, lane, scaled);
   pipe.template run_f16<BF16>(acc, frag);
   pipe.drain();
 
