@@ -283,7 +283,8 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
   uint16_t *table = reinterpret_cast<uint16_t *>(smem + MT * (xstride + fstride));
   // FEW: waves 0 .. 2 request the scales, reduced weights and biases of all of them (16 at most) in front of the quantize: behind it their
   // trip to memory stands in front of the stream (us per forward, one row: 4096 -> 4096 6.6 -> 6.4, 4096 -> 2560 6.5 -> 6.35).  Of a
-  // long stream it is no part: requested so, 8192 -> 28672 from memory takes 24.9 instead of 24.6.
+  // long stream it is no part: requested so, 8192 -> 28672 from memory takes 24.9 instead of 24.6.  (Behind the wait for the row, whose
+  // count then does not hang on how these loads are compiled; in front of it the row would wait for them, 4096 -> 4096 6.02 -> 6.09.)
   const uint16_t *const given = wave == 1 ? p.w_red : wave == 2 ? p.bias : p.s_col;
   uint16_t few = 0;
 
@@ -312,6 +313,9 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     __builtin_amdgcn_sched_barrier(0);
     first_pieces();
     __builtin_amdgcn_sched_barrier(0);
+    // the first row: everything but the weight pieces, which were issued last
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(kGemvPieces - 1));
+    __syncthreads();
     if constexpr (FEW) {
       const int n = n_first - wave + (lane & (kGemvWaves - 1)) + ((lane / kGemvWaves) & 1) * step;
       few = (given ? given : p.s_col)[n < p.N ? n : p.N - 1];  // (by all waves and lanes: under a condition every wait would be for all loads)
@@ -320,11 +324,11 @@ __global__ __launch_bounds__(kGemvWaves * 64) void gemv_decode_kernel(FusedArgs 
     for (int m = 0; m < p.M; ++m) {
       // A second row takes the first one's place (both requested at once at the start were no faster, measured, and
       // cost a second row of LDS); it sits behind the weight pieces, which have long landed by then.
-      if (m > 0) gemv_copy_in(quant.x + int64_t(m) * quant.cols, quant.cols * 2, area_lds + ql.raw, wave, lane);
-      // the first row: everything but the weight pieces and the scalar, which were issued last
-      if (m == 0) __builtin_amdgcn_s_waitcnt(vmcnt_imm(kGemvPieces - 1 + FEW));
-      else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
-      __syncthreads();
+      if (m > 0) {
+        gemv_copy_in(quant.x + int64_t(m) * quant.cols, quant.cols * 2, area_lds + ql.raw, wave, lane);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
+        __syncthreads();
+      }
       float sc, zr;
       gemv_quantize_row<MODE == kInt4 ? 4 : 8, BF16, QUANT == kGemvSym>(area + ql.raw, reinterpret_cast<const uint32_t *>(area + ql.grp),
                                                      reinterpret_cast<const uint16_t *>(area + ql.unit), quant, goff,
