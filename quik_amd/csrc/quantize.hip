@@ -725,8 +725,7 @@ __global__ __launch_bounds__(TPR) void asym_quantize_stream_kernel(
   const uint32_t map_flags = flags[0], ndirty = flags[1];
   StreamTables<NV, TPR> tables;
   tables.load(grp, dirty, dirty_grp, reinterpret_cast<const uint16_t *>(fp_col), cols, num_fp);
-  // (with sixteen groups per lane registers count for more: pinned / not, int8 1024 x 28672 27.5 / 26.1 us, bf16 in tile order
-  // 2048 x 28672 66.7 / 62.5)
+  // (with sixteen groups per lane registers count for more: pinned / not, int8 1024 x 28672 27.5 / 26.1 us)
   if constexpr (NV < 16) tables.pin();
   if (map_flags & kColmapStreams) {
     uint8_t *codes_s = reinterpret_cast<uint8_t *>(row_s);
@@ -1931,8 +1930,7 @@ int launch_tile8_ring(const void *x, int64_t rows, int64_t cols, const uint8_t *
 
 template <typename IdxT, int BITS, bool BF16>
 int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, const ColmapLayout &l, int64_t num_int,
-                int64_t num_fp, void *dst, void *meta, void *fp_x, hipStream_t st, bool tiled = false,
-                int64_t ndirty = -1, int64_t ngather = 0) {
+                int64_t num_fp, void *dst, void *meta, void *fp_x, hipStream_t st) {
   const IdxT *src_col = reinterpret_cast<const IdxT *>(cm);
   const IdxT *fp_col = reinterpret_cast<const IdxT *>(cm + l.off_fp);
   const uint32_t *mask = reinterpret_cast<const uint32_t *>(cm + l.off_mask);
@@ -1941,26 +1939,11 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
     // better than fewer waves with less per-row fixed work (64 and 128 threads were slower).
     const int64_t groups = cols / 8;
 #define QUIK_STREAM(NV, TPR) \
-  return launch_stream<IdxT, BITS, BF16, NV, TPR>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, tiled)
-    // fp16 rows beyond 16384 columns with tile-ordered int8 output: the LDS ring kernel
-    if constexpr (BITS == 8 && !BF16) {
-      if (tiled && ring_fits(cols, num_int, num_fp, ndirty) && ngather <= kRingThreads)
-        return launch_tile8_ring(x, rows, cols, cm, l, num_int, num_fp, static_cast<int>(ndirty),
-                                 static_cast<int>(ngather), dst, meta, st);
-    }
+  return launch_stream<IdxT, BITS, BF16, NV, TPR>(x, rows, cols, cm, l, num_int, num_fp, dst, meta, fp_x, st, false)
     if (groups > 512 && rows <= wide_rows()) {
       if (groups <= 1024) QUIK_STREAM(2, 512);
       if (groups <= 2048) QUIK_STREAM(4, 512);
       QUIK_STREAM(8, 512);
-    }
-    // bf16 rows beyond 16384 columns (and fp16 ones the ring kernel does not take: more than 512 outlier columns):
-    // 180 registers per lane leave room for two workgroups per CU, so the launch is persistent and prefetches the
-    // next row (measured at 2048 x 28672: 67 -> 61 us inside the forward; at 2048 x 11008, where three workgroups
-    // fit, it is slower)
-    if constexpr (BITS == 8) {
-      if (tiled && groups > 2048)
-        return launch_stream<IdxT, BITS, BF16, 16, kThreads, false, true>(x, rows, cols, cm, l, num_int, num_fp, dst, meta,
-                                                                          fp_x, st, tiled);
     }
     if (groups <= 512) QUIK_STREAM(2, kThreads);
     if (groups <= 1024) QUIK_STREAM(4, kThreads);
@@ -1968,7 +1951,6 @@ int launch_asym(const void *x, int64_t rows, int64_t cols, const uint8_t *cm, co
     QUIK_STREAM(16, kThreads);
 #undef QUIK_STREAM
   }
-  if (tiled) return QUIK_ERR_SHAPE;  // tile-ordered output exists on the streaming path only
   const int grid = static_cast<int>(rows < 65535 * 8 ? rows : 65535 * 8);
   const int64_t lds = align16(cols * 2);
   if (lds <= kMaxLdsRowBytes) {
@@ -2171,9 +2153,10 @@ int quik::asym_quantize_fp6(const void *x, int dtype, int64_t rows, int64_t cols
 }
 
 namespace {
-bool units_ok(const void *x, int64_t rows, int64_t cols, int64_t num_int, const void *dst) {
-  return rows <= (1 << 20) && cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
-         reinterpret_cast<uintptr_t>(dst) % 16 == 0;  // (rows: a grid holds fewer than 2^32 threads)
+constexpr int64_t kUnitRows = 1 << 20;  // rows per launch: a grid holds fewer than 2^32 threads
+bool units_ok(const void *x, int64_t cols, int64_t num_int, const void *dst) {
+  return cols % 8 == 0 && cols <= kStreamMaxCols && num_int % 16 == 0 && reinterpret_cast<uintptr_t>(x) % 16 == 0 &&
+         reinterpret_cast<uintptr_t>(dst) % 16 == 0;
 }
 template <int BITS, bool BF16, bool TILED, bool SYM = false>
 int launch_units(const void *x, int64_t rows, int64_t cols, const void *colmap, int64_t num_int, int64_t num_fp, void *dst, void *meta,
@@ -2206,7 +2189,7 @@ int quik::asym_quantize_few(const void *x, int dtype, int64_t rows, int64_t cols
   hipStream_t st = as_stream(stream);
   if (rows > 0 && rows <= kFewRows && num_int > 0 && num_fp >= 0 && num_int + num_fp == cols && (bits == 4 || bits == 8) &&
       (dtype == QUIK_F16 || dtype == QUIK_BF16) && x && colmap && dst && meta && (num_fp == 0 || fp_x) &&
-      units_ok(x, rows, cols, num_int, dst)) {
+      units_ok(x, cols, num_int, dst)) {
     auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, dst, meta, fp_x, st, 1.0f); };
     if (bits == 4) return dtype == QUIK_F16 ? go(launch_units<4, false, false>) : go(launch_units<4, true, false>);
     return dtype == QUIK_F16 ? go(launch_units<8, false, false>) : go(launch_units<8, true, false>);
@@ -2239,16 +2222,28 @@ int quik::asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t co
   // fp16 rows of more than 16384 columns, eight groups per lane, where a CU has more than one: quantize_tile8_ring_kernel, whose next row is
   // on its way while one is worked on (us per forward, units / ring: 256 x 28672 -> 1024 29.2 / 29.7, 512 x 28672 -> 512 40.65 / 39.45, 2048 x
   // 28672 -> 512 100 / 85; 768 x 16384 -> 512 32.55 / 34.05, 2048 x 13824 -> 512 46.05 / 47.15)
-  if ((dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) && units_ok(x, rows, cols, num_int, out8)) {
-    auto go = [&](auto launch) { return launch(x, rows, cols, colmap, num_int, num_fp, out8, meta, nullptr, st, 1.0f); };
+  if (dtype == QUIK_BF16 || cols <= 16384 || rows <= num_cus()) {
+    auto go = [&](auto launch) {
+      static_assert(kUnitRows % 64 == 0, "whole blocks of the operand buffer");
+      const int64_t block = tile8_layout(rows, num_int, num_fp).block_bytes;
+      for (int64_t first = 0; first < rows; first += kUnitRows) {
+        const int64_t count = rows - first < kUnitRows ? rows - first : kUnitRows;
+        if (int rc = launch(static_cast<const uint16_t *>(x) + first * cols, count, cols, colmap, num_int, num_fp,
+                            static_cast<uint8_t *>(out8) + first / 64 * block, static_cast<uint16_t *>(meta) + 2 * first, nullptr, st, 1.0f))
+          return rc;
+      }
+      return static_cast<int>(QUIK_OK);
+    };
     return dtype == QUIK_F16 ? go(launch_units<8, false, true>) : go(launch_units<8, true, true>);
   }
   const ColmapLayout l = colmap_layout(cols, num_int, num_fp);
   const uint8_t *cm = static_cast<const uint8_t *>(colmap);
-  return dtype == QUIK_F16 ? launch_asym<uint16_t, 8, false>(x, rows, cols, cm, l, num_int, num_fp, out8, meta, nullptr,
-                                                            st, true, words[1], words[3])
-                           : launch_asym<uint16_t, 8, true>(x, rows, cols, cm, l, num_int, num_fp, out8, meta, nullptr,
-                                                           st, true, words[1], words[3]);
+  if (ring_fits(cols, num_int, num_fp, words[1]) && words[3] <= kRingThreads)
+    return launch_tile8_ring(x, rows, cols, cm, l, num_int, num_fp, static_cast<int>(words[1]), static_cast<int>(words[3]), out8, meta, st);
+  // What the ring does not take (more outlier columns or groups that hold some than lanes, rows whose ring exceeds the LDS): 180
+  // registers per lane leave room for two workgroups per CU, so the launch is persistent and requests the next row beside this one
+  // (2048 x 28672 inside the forward, 67 -> 61 us)
+  return launch_stream<uint16_t, 8, false, 16, kThreads, false, true>(x, rows, cols, cm, l, num_int, num_fp, out8, meta, nullptr, st, true);
 }
 
 extern "C" int quik_asym_quantize_tile8(const void *x, int dtype, int64_t rows, int64_t cols, const void *colmap,
@@ -2279,7 +2274,7 @@ int quik::sym_quantize_mapped(const void *x, int64_t rows, int64_t cols, const v
   if (bits == 4 && tiled) return launch_fp6_row<false, true, false>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, st, divisor);
   // few rows: as asym_quantize_few (us per forward, streaming kernel / units: 16 x 8192 -> 8192 12.4 / 12.0, 3 x 13824 -> 5120 13.75 / 13.3,
   // 16 x 28672 -> 8192 28.05 / 26.95, 24 x 2048 -> 2048 7.35 / 7.15, 32 x 4096 -> 4096 8.85 / 8.7; 5120 columns the same)
-  if (!tiled && rows <= kFewRows && units_ok(x, rows, cols, num_int, dst))
+  if (!tiled && rows <= kFewRows && units_ok(x, cols, num_int, dst))
     return bits == 4 ? launch_units<4, false, false, true>(x, rows, cols, colmap, num_int, num_fp, dst, scale, fp_x, st, divisor)
                      : launch_units<8, false, false, true>(x, rows, cols, colmap, num_int, num_fp, dst, scale, fp_x, st, divisor);
   return bits == 4 ? launch_sym_stream<4>(x, rows, cols, cm, l, num_int, num_fp, dst, scale, fp_x, st, tiled != 0, divisor)

@@ -1,7 +1,7 @@
-"""The row-major and int8 tile-ordered streaming quantize (asym_quantize_stream_kernel) on both sides of the row count up to
+"""The row-major streaming quantize (asym_quantize_stream_kernel) on both sides of the row count up to
 which a row of more than 4096 columns gets eight waves (half the CUs), and its persistent form, which prefetches the next row
-(int8 operand buffers, rows beyond 16384 columns, more rows than that), with workgroups that take more than one row.
-Against the oracle."""
+(int8 operand buffers of more fp16 rows than CUs, beyond 16384 columns, that the ring kernel does not take), with workgroups that take
+more than one row.  bf16 rows of that length take quantize_units_kernel.  Against the oracle."""
 import numpy as np
 import pytest
 import torch
@@ -93,8 +93,8 @@ def test_eight_waves_per_row_or_four_symmetric(beyond, n_in, F, bits):
 @pytest.mark.parametrize("rows,n_in,F,bf16", [(300, 28672, 256, True), (700, 16512, 128, True), (1100, 16416, 32, True),
                                               (600, 20480, 1024, False), (530, 32768, 256, False)])
 def test_persistent_workgroups(rows, n_in, F, bf16):
-    """bf16 rows, fp16 rows with an outlier column in each of more groups than the ring kernel takes, fp16 rows beyond what
-    its ring holds; two workgroups per CU, so more than 512 rows are more than one row for some of them."""
+    """bf16 rows (a workgroup each), fp16 rows with an outlier column in each of more groups than the ring kernel takes, fp16 rows
+    beyond what its ring holds; two workgroups per CU, so more than 512 rows are more than one row for some of them."""
     from quik_amd import asymmetric
     rng = np.random.default_rng(rows)
     fi = (np.arange(F) * 8 + rng.integers(0, 8, F) if F == 1024 else rng.permutation(n_in)[:F]).astype(np.int64)
