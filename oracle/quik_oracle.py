@@ -125,6 +125,9 @@ def find_meta_rows(xi, bits, dtype=F16):
     max / min with __hmax / __hmin (NaN operands are skipped), then
     scale = float2type(fmaxf((max_f - min_f) / divisor, 1e-6)), zero = min."""
     x32 = _as_f32(xi, dtype)
+    # (signalling NaNs made quiet: by the row's place in the array numpy's fmin / fmax answer one with a NaN, which the
+    # next step then drops together with what was accumulated)
+    x32 = np.where(np.isnan(x32), np.float32(np.nan), x32)
     with np.errstate(invalid="ignore", over="ignore"):
         mx = np.fmax.reduce(x32, axis=1)
         mn = np.fmin.reduce(x32, axis=1)
