@@ -1,14 +1,14 @@
 """Rows of more than 8192 columns -> int8 operand buffer in tile order (quik_asym_quantize_tile8).
 
-fp16 rows of that length go through a kernel of their own (the row is copied global -> LDS into a ring of two
-slots, one or two workgroups of eight waves per CU); every other case keeps the streaming kernel.  The buffer is decoded
+They go through the kernel of one workgroup per row (quantize_units_kernel), but for more fp16 rows than CUs of more than 16384
+columns, which are copied into an LDS ring (here 2100 x 28672; the others in test_gpu_ring_quantize.py).  The buffer is decoded
 here from the documented layout (quik_amd/csrc/gemm_tile8.h, restated) and compared, code for code and bit for bit,
 with the oracle's per-token quantize (src/asymmetric/asymmetric.cu:15-108 with the reference's index gather,
-quik/asymmetric.py), at every group count per lane the kernel is built for, with ragged row counts, edge rows
+quik/asymmetric.py), at every number of groups per lane, with ragged row counts, edge rows
 (constant, subnormal, overflowing range, infinity, NaN, all-NaN), outlier columns next to each other and at both
-ends of the row, no outlier columns at all, and more rows than one pass of the persistent grid takes.
+ends of the row, no outlier columns at all, and more rows than one pass of the ring's persistent grid takes.
 Signalling-NaN bit patterns, which no arithmetic produces but a caller may hand over, are skipped by min / max like
-every other NaN (the reference's __hmin / __hmax): checked for this kernel and for the 6-bit one.
+every other NaN (the reference's __hmin / __hmax): checked for quantize_units_kernel and for the 6-bit one.
 """
 import numpy as np
 import pytest
@@ -92,17 +92,17 @@ def _check(x, ii, fi, n_in):
     assert np.array_equal(outl, want_fp.view(np.uint16).reshape(rows, F))
 
 
-# rows, in_features, outlier columns: in / 8 / 512 rounded up = groups per lane (3 .. 8)
+# rows, in_features, outlier columns: a lane has in / 8 / 512 rounded up groups, in 2, 4 or 8 registers' room
 @pytest.mark.parametrize("rows,n_in,F", [
-    (300, 11008, 256),         # Llama-2-7B down_proj: 3 groups per lane, two workgroups per CU
-    (2048 + 7, 13824, 256),    # Llama-2-13B down_proj: 4; every workgroup takes several rows
-    (40, 8192 + 64, 64),       # the shortest row of the kernel
-    (37, 8192, 256),           # one column group fewer: the streaming kernel
+    (300, 11008, 256),         # Llama-2-7B down_proj: 3 groups per lane
+    (2048 + 7, 13824, 256),    # Llama-2-13B down_proj: 4
+    (40, 8192 + 64, 64),       # one column group more than 2 groups per lane hold
+    (37, 8192, 256),           # 2, exactly
     (70, 28672, 256),          # Llama-2-70B down_proj: 7 groups per lane, exactly
-    (2100, 28672, 256),        # more rows than the grid's first pass, ragged last block
+    (2100, 28672, 256),        # through the ring: more rows than the grid's first pass, ragged last block
     (41, 16384 + 64, 64),      # 5 groups per lane, most of the fifth past the row's end
     (64, 24576, 128),          # 6
-    (33, 31744, 256),          # 8: the longest row whose ring fits LDS
+    (33, 31744, 256),          # 8: the longest row whose ring would fit LDS
     (40, 20480 - 64, 0),       # no outlier columns; row length not a multiple of the 1 KB copies
     (36, 28672, 512),          # as many outlier columns as lanes
 ])
@@ -121,7 +121,7 @@ def test_long_rows_against_the_oracle(rows, n_in, F):
 
 @pytest.mark.parametrize("seed", range(12))
 def test_long_rows_random_shapes(seed):
-    """Seeded random shapes over the kernel's whole range: 8224 .. 31744 columns in steps of 32, 0 .. 512 outlier
+    """Seeded random shapes: 8224 .. 31744 columns in steps of 32, 0 .. 512 outlier
     columns (in runs, clustered at one end, or spread), 1 .. 300 rows."""
     rng = np.random.default_rng(1000 + seed)
     F = 32 * int(rng.integers(0, 17))
@@ -142,8 +142,7 @@ def test_long_rows_random_shapes(seed):
 
 
 def test_every_group_holds_an_outlier_column_falls_back():
-    """More groups with outlier columns than the ring kernel keeps per lane (512): the streaming kernel serves the
-    shape, same results."""
+    """More groups with outlier columns (1024) than the ring kernel takes (512), in fewer rows than it is used for."""
     rng = np.random.default_rng(5)
     n_in, F = 28672, 1024
     fi = np.arange(F) * 8 + rng.integers(0, 8, F)       # one outlier column in each of the first 1024 groups
