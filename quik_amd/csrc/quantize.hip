@@ -1080,7 +1080,8 @@ __device__ __forceinline__ uint32_t level_pair_fast(uint32_t w, const RQ &rq) {
 }
 
 // The levels of four bf16 values in the bytes of the result, rows on the fast path.  As above: t = max(t, 0), no upper clamp (x - zero <= max -
-// min, rounded up by at most 2^-9, and the scale is at least (max - min) / 15 less 2^-9: t is at most 15.125), and t + 1.5 2^23 holds rne(t) in its low byte.
+// min, rounded up by at most 2^-8, and the scale is at least (max - min) / 15 less 2^-8: the quotient is at most 15.118, t 15.125, which is
+// reached: tests/test_quotient_levels_bf16.py), and t + 1.5 2^23 holds rne(t) in its low byte.
 // (v_max_f32 by hand: the compiler's fmaxf first quiets an operand that may be a signalling NaN; a converted value is none.  Plain VALU
 // instruction, no hazard.)
 __device__ __forceinline__ uint32_t level_quad_bf16(uint32_t w0, uint32_t w1, const RowQuant<true> &rq) {
