@@ -39,9 +39,11 @@ enum class Tiles4 { k64x32, k64x64, k128x64, kRing };
 // busiest CU, s: k-steps, outlier steps included, w: kilobytes of weights,
 //   t = a + r (b s + c) + d w
 // fitted to 16 row counts of 40 .. 3072 on each of 12 layer shapes (2048 -> 2048 to 13824 -> 5120), warm weights; the ring of one
-// tile per CU to 130 calls, warm and cold alike.  The pick is 0.02 % behind the fastest of the four over the 150 calls of 100 .. 1024
-// rows and the few columns of plan_splits4, 0.2 % with cold weights (at most 9 %: 300 x 4096 -> 4096 18.7 / 17.2 us on 128x64
-// tiles).  Two 128x128 tiles share a CU: 1.9 of a single one's time.
+// tile per CU to 130 calls, warm and cold alike; all with eight (64x32) and four steps in flight and loaded empty steps, 0.02 % behind
+// the fastest of the four over 150 calls of 100 .. 1024 rows.  With the tiles above, which are up to 7 % faster, 64x32 and 64x64 ones most, the pick
+// is 0.6 % behind over 145 calls (40 .. 1024 rows, 13 layer shapes, warm), more than 1 % in 14 of them, eight of those on 128x64
+// tiles where 64x64 are faster: 300 x 5120 -> 5120 16.55 / 15.6 us, 200 x 4544 -> 4544 14.7 / 13.95, 300 x 4544 -> 4544 15.4 / 14.7.  Two 128x128 tiles
+// share a CU: 1.9 of a single one's time.
 int64_t direct_cost(Tiles4 t, int64_t M, int64_t N, int64_t s, int64_t w) {
   const int64_t cus = num_cus();
   auto tiles = [&](int64_t bm, int64_t bn) { return (M + bm - 1) / bm * ((N + bn - 1) / bn); };
@@ -71,7 +73,7 @@ Tiles4 plan_tile4(int64_t M, int64_t N, int64_t K, int64_t F) {
 
 // K split over `splits` workgroups per 64x32 tile (SplitK): few tiles of a long K leave most CUs idle, and with them what the
 // chip can have open towards memory.  The exchange through memory costs 1.5 us and 0.3 per workgroup, against 24.6 ns for each step
-// that a workgroup has less (same fit), so it is taken from some 150 k-steps on.  us per forward, warm / cold weights, without and
+// that a workgroup has less (same fit, of the tiles before), so it is taken from some 150 k-steps on.  us per forward, warm / cold weights, without and
 // with the split: 64 x 14336 -> 512 15.0 / 17.8, 13.4 / 14.8 (4); 128 x 14336 -> 1024 15.5 / 20.2, 15.0 / 16.7 (4); 64 x 12288 -> 1024
 // 14.0 / 18.4, 13.4 / 15.1 (3); 40 x 14336 -> 4096 15.3 / 20.9, 15.0 / 19.1 (2).  At 8192 columns it costs warm what it gives cold (64 ->
 // 1024 12.0 / 14.3, 12.3 / 13.6); eight workgroups per tile, or 64x64 tiles, were nowhere the faster form.

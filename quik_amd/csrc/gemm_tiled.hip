@@ -95,7 +95,9 @@ int launch_fused6_split(const Fused6Args &wide, const Fused6Args &tail, hipStrea
 // of 128x64 tiles), never less than the weights take: up to 128 MB at 8 TB/s, more at what each kernel reaches from memory,
 // and at most 24 bytes per ns for each CU that works.  The 8 TB/s is not where such weights come from, a model's are cold; it is
 // what ranks the kernels as they were measured, warm and cold alike (layers over 700 MB in turn): over 23 layer shapes of 6 ..
-// 222 MB at 40 .. 192 rows, both widths, the pick is 0.6 % behind the fastest kernel warm and 1.7 % cold.  us per forward, warm /
+// 222 MB at 40 .. 192 rows, both widths, the pick is 0.6 % behind the fastest kernel warm and 1.7 % cold.  (Fitted with ten and six int8 steps
+// in flight; with six and four, over 35 int8 calls of 40 .. 200 rows, it is 1.5 % behind warm, most where the ring is the faster one: 200 x 13824
+// -> 5120 42.2 / 37.2 us with its K split, 200 x 8192 -> 8192 34.3 / 31.1 without.)  us per forward, warm /
 // cold, as picked and as the memory's rates would pick: 64 x 4096 -> 11008 13.6 / 18.2 (64x64 tiles) and 15.3 / 19.9 (ring),
 // 64 x 8192 -> 10240 18.4 / 27.2 and 20.8 / 29.9, 128 x 8192 -> 20480 28.8 / 46.5 (ring) and 36.5 / 54.2; int8 64 x 13824 -> 5120 23.4 /
 // 34.7 (64x64, two splits) and 27.9 / 35.8, but 64 x 14336 -> 8192 26.4 / 40.5 (64x32) and 29.0 / 36.4.  Beyond, the memory's rates
